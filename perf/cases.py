@@ -120,24 +120,24 @@ def _case(name: str, design: str, size: str, requests: int, prompt: int, new: in
 def listed() -> List[dict]:
     return [
         # one person at a small model: a short prompt, then tokens one at a time; latency and launches
-        _case("llama 1b, one request", "llama", "1b", 1, 24, 24),
+        _case("llama 1b - one request", "llama", "1b", 1, 24, 24),
         # the headline of bench.py: eight requests decode after prompts of about 512 tokens
-        _case("llama 8b, 8 requests", "llama", "8b", 8, 512, 32),
+        _case("llama 8b - 8 requests", "llama", "8b", 8, 512, 32),
         # a full serving batch: 64 requests with short prompts of uneven length
-        _case("llama 8b, 64 requests", "llama", "8b", 64, 120, 32),
+        _case("llama 8b - 64 requests", "llama", "8b", 64, 120, 32),
         # a prompt of ordinary length, and the first token (the prefill of bench.py)
-        _case("llama 8b, prompt of 2048", "llama", "8b", 1, 2048, 0),
+        _case("llama 8b - prompt of 2048", "llama", "8b", 1, 2048, 0),
         # a long document in one step
-        _case("llama 8b, prompt of 8192", "llama", "8b", 1, 8192, 0),
+        _case("llama 8b - prompt of 8192", "llama", "8b", 1, 8192, 0),
         # the 32-bit path, as a check of numbers is run: a few odd prompts and a few tokens
         _case("llama 1b in 32 bits", "llama", "1b", 3, 61, 4, "float32"),
         # the further designs, each with prompts and decoding: a long prompt and its answer, or a batch of requests
-        _case("nesilorn 2k, prompt of 2047", "nesilorn", "2k", 1, 2047, 16),
-        _case("rogizen 2k, 8 requests", "rogizen", "2k", 8, 256, 16),
-        _case("malinex 2k, 2 requests", "malinex", "2k", 2, 1000, 8),
-        _case("sikazen 2k, prompt of 3000", "sikazen", "2k", 1, 3000, 8),
-        _case("pamazen 4k, 16 requests", "pamazen", "4k", 16, 128, 16),
-        _case("mirovik 2k, 32 requests", "mirovik", "2k", 32, 64, 16),
+        _case("nesilorn 2k - prompt of 2047", "nesilorn", "2k", 1, 2047, 16),
+        _case("rogizen 2k - 8 requests", "rogizen", "2k", 8, 256, 16),
+        _case("malinex 2k - 2 requests", "malinex", "2k", 2, 1000, 8),
+        _case("sikazen 2k - prompt of 3000", "sikazen", "2k", 1, 3000, 8),
+        _case("pamazen 4k - 16 requests", "pamazen", "4k", 16, 128, 16),
+        _case("mirovik 2k - 32 requests", "mirovik", "2k", 32, 64, 16),
     ]
 
 
