@@ -302,6 +302,25 @@ def test_gemm_generic(M, N, K_):
     assert torch.allclose(outf.double(), wantb, atol=1e-3, rtol=1e-4)
 
 
+# 16 / 17, 32 / 33: the ends of the streaming kernel's one and two groups of rows; 8192: two groups of W's rows a workgroup;
+# 260, 516: a stretch of 256 and a bit; 16, 20: less than a chain more; tiles of 32, 64 and 128 rows and their remainders
+@pytest.mark.parametrize("M,N,K_", [(2, 16, 4), (16, 1000, 2052), (17, 33, 20), (32, 8192, 260), (3, 8200, 4096),
+                                    (33, 97, 516), (65, 4100, 256), (300, 8205, 288), (1030, 8192, 36)])
+def test_gemm_fp32_on_the_matrix_cores_leaves_the_vector_kernels_bits(M, N, K_):
+    padded, w = _rand(M, K_ + 1, seed=1), _rand(N, K_, seed=2)
+    padded[0, :K_] *= 1e-30                                    # products that are subnormal or nothing
+    w[0] *= 1e-10
+    apart = padded[:, :K_]                                     # rows that are not 16-byte aligned: the vector kernel
+    want, got = torch.empty(M, N, device=DEV), torch.empty(M, N, device=DEV)
+    K().gemm_generic(apart, w, want)
+    K().gemm_generic(apart.contiguous(), w, got)
+    assert torch.equal(got, want)
+    # and those are the sums: a chain of 16, 16 of them, K / 256 of those: each level rounds with 2^-24 a term
+    exact = apart.double() @ w.double().T
+    bound = (32 + K_ / 256) * 2.0 ** -24 * (apart.double().abs() @ w.double().abs().T) + 1e-37
+    assert bool(((got.double() - exact).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("M", [1, 2, 8, 16, 17, 33, 64, 65, 81, 100, 128])
 @pytest.mark.parametrize("N,K_", [(250, 96), (384, 176), (4096, 4096), (1000, 14336), (16, 8), (129, 1000)])
 def test_gemm_skinny(M, N, K_):
