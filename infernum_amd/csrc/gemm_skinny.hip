@@ -229,6 +229,81 @@ __global__ __launch_bounds__(256) void gemm_skinny_join_kernel(const float* __re
   store_out<TO>(C + idx, EPI == SK_EPI_SWIGLU ? a / (1.0f + expf(-a)) * b : a);
 }
 
+// ---- up to 16 rows, the parts of K in one workgroup ---------------------------------------------------------------
+// The same sums as the kernel above and its join, in the same order and so the same bits, in one launch: a workgroup
+// takes 16 rows of W (GLU: 16 of each half) and a wave the part of K that a workgroup takes there, chunk after chunk
+// from the same start; the parts meet in LDS and are added in the order of their index.  A wave reads its rows of W and
+// of X straight into registers, a chunk of 256 values in flight at a time.  X comes from the caches once per 16 rows of
+// W instead of once per 64, which is what the rule in whole_k_pays weighs against the join's launch.
+#define SK_MOST_WAVES 16
+
+template <bool GLU, int WAVES, typename TO>
+__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_whole_kernel(const uint16_t* __restrict__ X,
+                                                                       const uint16_t* __restrict__ W,
+                                                                       TO* __restrict__ C, int M, int N, int K,
+                                                                       int chunks_per_split, int splits) {
+  constexpr int NLD = SK_KC / 32;
+  __shared__ f32x4 parts[WAVES][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = lane & 15, q = lane >> 4;
+  const int half = GLU && wave >= splits ? 1 : 0, split = wave - half * splits;
+  const int NO = GLU ? N / 2 : N;
+  const int n0 = blockIdx.x * 16;
+  const int nchunks = (K + SK_KC - 1) / SK_KC;
+  const int c0 = split * chunks_per_split, c1 = min(nchunks, c0 + chunks_per_split), span = c1 - c0;
+  const uint16_t* wrow = W + ((size_t)min(n0 + r, NO - 1) + (size_t)half * NO) * K + q * 8;
+  const uint16_t* xrow = X + (size_t)min(r, M - 1) * K + q * 8;
+  const unsigned tile = (unsigned)(n0 + half * NO) / SK_BN;            // the tile of 64 rows that names the first chunk
+  int at = c0 + (span > 1 ? (int)(((tile * 0x9E3779B1u) >> 8) % (unsigned)span) : 0);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int c = 0; c < span; ++c) {
+    uint4 w[NLD], x[NLD];
+#pragma unroll
+    for (int j = 0; j < NLD; ++j) {
+      const int k = at * SK_KC + 32 * j;
+      const bool in = k + 8 * q < K;
+      w[j] = in ? load_stream_16(wrow + k) : make_uint4(0u, 0u, 0u, 0u);
+      x[j] = in ? *reinterpret_cast<const uint4*>(xrow + k) : make_uint4(0u, 0u, 0u, 0u);
+    }
+    if (++at == c1) at = c0;
+#pragma unroll
+    for (int j = 0; j < NLD; ++j)
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[j]), __builtin_bit_cast(bf16x8, x[j]),
+                                                    acc, 0, 0, 0);
+  }
+  parts[wave][lane] = acc;
+  __syncthreads();
+  // the first waves add the parts: value e of the four that a lane of the products holds, wave by wave
+  const int n = n0 + 4 * q;
+  if (r >= M) return;
+  for (int e = wave; e < 4; e += GLU ? 2 * splits : splits) {
+    float a = 0.f, b = 0.f;
+    for (int v = 0; v < splits; ++v) {
+      a += parts[v][lane][e];
+      if (GLU) b += parts[splits + v][lane][e];
+    }
+    if (n + e < NO) store_out<TO>(C + (size_t)r * NO + n + e, GLU ? a / (1.0f + expf(-a)) * b : a);
+  }
+}
+
+// Whether the kernel above takes a split product whose parts are wanted joined.  Microseconds on an MI355X in a chain of
+// products with cold weights, the split product with its join against this kernel: 2,048 x 2,048 at 1 / 8 / 16 rows 7.9 /
+// 8.6 / 8.9 against 5.3 / 6.1 / 7.1, 4,096 x 4,096 13.0 / 12.7 / 12.8 against 9.8 / 10.5 / 11.9, 8,192 x 2,048 12.7 / 12.6 /
+// 12.8 against 9.4 / 10.1 / 11.6.  It loses where the reads of X weigh more than a launch: 2,048 x 5,504 at 16 rows (13.5
+// against 15.1; 12 rows even), 12,288 x 4,096 and 10,304 x 2,048 at 16 (27.2 against 29.5, 15.2 against 15.9; 8 rows
+// ahead); where the chunks do not deal out evenly over more than four waves, which then wait for the longest
+// (6,144 x 4,096 at 8 rows 15.5 against 15.9); and with few workgroups of many waves (64 x 4,096 at 16 rows 8.2 against
+// 9.5).  With both halves it reads X twice: 5,632 x 2,048 at 8 rows 11.3 against 10.0, 11,008 x 2,048 at 4 rows 15.9
+// against 14.6 and at 8 16.2 against 17.1, 9,472 x 4,096 behind at every number of rows.
+static bool whole_k_pays(int M, int N, int K, int splits, bool glu) {
+  if (M > 16 || (glu ? 2 : 1) * splits > SK_MOST_WAVES) return false;
+  const int nchunks = (K + SK_KC - 1) / SK_KC;
+  if (glu) return N % 32 == 0 && K <= 2048 && (long)M * N <= 65536;
+  if (splits > 4 && nchunks % splits != 0) return false;
+  if (N < 256 && splits > 8 && M > 4) return false;
+  return (long)M * K <= 65536 && (long)M * N <= 131072;
+}
+
 // Shapes whose number of splits was measured (ia_gemm_skinny_set_splits, filled from a table when the library is
 // loaded): few entries, looked up per launch.
 struct KnownSplits { int N, K, splits; };
@@ -344,6 +419,24 @@ static int skinny_product(const void* X, const void* W, void* C, int out_dtype, 
   if (!via_workspace) {
     if (out_dtype == IA_F32) return launch_skinny<false, float, TILED>(x, w, (float*)C, nullptr, M, N, K, 1, stream);
     return launch_skinny<false, uint16_t, TILED>(x, w, (uint16_t*)C, nullptr, M, N, K, 1, stream);
+  }
+  const bool glu = epilogue == SK_EPI_SWIGLU;
+  if (!TILED && C != nullptr && splits > 1 && whole_k_pays(M, N, K, splits, glu)) {
+    const int nchunks = (K + SK_KC - 1) / SK_KC, cps = (nchunks + splits - 1) / splits, NO = glu ? N / 2 : N;
+    const dim3 grid((NO + 15) / 16), block((glu ? 2 : 1) * splits * 64);
+#define SK_WHOLE(G, T)                                                                                              \
+  do {                                                                                                              \
+    if (block.x <= 512) gemm_skinny_whole_kernel<G, 8, T><<<grid, block, 0, stream>>>(x, w, (T*)C, M, N, K, cps, splits); \
+    else gemm_skinny_whole_kernel<G, 16, T><<<grid, block, 0, stream>>>(x, w, (T*)C, M, N, K, cps, splits);          \
+  } while (0)
+    if (glu) {
+      if (out_dtype == IA_F32) SK_WHOLE(true, float); else SK_WHOLE(true, uint16_t);
+    } else {
+      if (out_dtype == IA_F32) SK_WHOLE(false, float); else SK_WHOLE(false, uint16_t);
+    }
+#undef SK_WHOLE
+    IA_LAUNCH_CHECK();
+    return IA_OK;
   }
   const int rc = launch_skinny<false, float, TILED>(x, w, nullptr, workspace, M, N, K, splits, stream);
   if (rc != IA_OK || C == nullptr) return rc;

@@ -370,6 +370,26 @@ def test_gemm_skinny_partial_sums_and_swiglu(M, N, K_):
     assert torch.equal(actb, act.bfloat16())
 
 
+# one workgroup with all of K against the parts and their sum in the order of their index: columns that fill no group of
+# 16, a last chunk that is not full, one to sixteen parts, two chunks and more a part, both halves of [gate | up]
+@pytest.mark.parametrize("M", [1, 5, 16])
+@pytest.mark.parametrize("N,K_,glu", [(250, 520, False), (2049, 776, False), (2048, 4096, False), (200, 5504, False),
+                                      (7000, 2040, False), (5632, 2048, True), (64, 1000, True), (96, 264, True)])
+def test_gemm_skinny_with_all_parts_in_one_workgroup_leaves_the_joined_parts_bits(M, N, K_, glu):
+    api = K()
+    a, w = _rand(M, K_, dtype=torch.bfloat16, seed=11), _rand(N, K_, dtype=torch.bfloat16, scale=0.05, seed=12)
+    kept = api.gemm_skinny(a, w, keep_split=True)
+    total = kept.parts[0].clone()
+    for part in kept.parts[1:]:
+        total += part
+    assert torch.equal(api.gemm_skinny(a, w, out_dtype=torch.float32), total)
+    assert torch.equal(api.gemm_skinny(a, w), total.bfloat16())
+    if glu:
+        got = api.gemm_skinny(a, w, epilogue="swiglu", out_dtype=torch.float32)
+        g, u = total[:, :N // 2].double(), total[:, N // 2:].double()
+        assert torch.allclose(got.double(), g / (1 + torch.exp(-g)) * u, rtol=1e-6, atol=1e-9)     # a few fp32 roundings
+
+
 def test_gemm_skinny_takes_the_measured_number_of_parts_for_the_shapes_of_its_table():
     """The table of measured shapes is in force from the library's load on: its shapes are split as it says (the
     chunks of K dealt out evenly), others by the rule of sizes; a product of such a shape is right and its partial sums
