@@ -1364,3 +1364,45 @@ def test_copy_pages(dtype):
     for s, d in ((0, 1), (2, 3), (7, 8)):              # a pair with a page outside the pool, or onto itself, is left out
         want[d] = before[s]
     assert torch.equal(pool, want)
+
+
+# ---------------------------------------------------------------- routed experts, few pairs
+# one pair, 17 (a second pass over an expert's pairs), 64 (the most); fewer pairs than experts and more; rows that fill no
+# group of 16, K that fills no stretch of 256 or part of a quarter; ids without an expert; the weight on either side
+@pytest.mark.parametrize("gated,weights_on", [(True, "output"), (True, "input"), (False, "output")])
+@pytest.mark.parametrize("N,top,E,W,ff", [(1, 1, 3, 264, 40), (17, 1, 2, 520, 328), (32, 2, 6, 136, 1000), (1, 4, 40, 2048, 1408),
+                                          (5, 3, 300, 72, 2056)])
+def test_routed_experts_of_few_pairs(gated, weights_on, N, top, E, W, ff):
+    api = K()
+    x = _rand(N, W, dtype=torch.bfloat16, seed=1)
+    up = _rand(E, (2 if gated else 1) * ff, W, dtype=torch.bfloat16, scale=2 * W ** -0.5, seed=2)
+    down = _rand(E, W, ff, dtype=torch.bfloat16, scale=ff ** -0.5, seed=3)
+    g = torch.Generator().manual_seed(4)
+    ids = torch.stack([torch.randperm(E + 1, generator=g)[:top] for _ in range(N)]).int().to(DEV)      # E: no expert
+    if N == 17:
+        ids[:] = 1                                              # all of them one expert's
+    wts = torch.rand(N, top, generator=g).to(DEV)
+    assert api.moe_few_tokens(E, top, W, ff, torch.bfloat16) >= N
+    parts = torch.full((top, N, W), 7.0, device=DEV)
+    if gated:
+        api.moe_experts(x, ids, wts, up, down, 7.0, 1.702, 1.0, E + 1, parts, weights_on)
+    else:
+        api.moe_plain_experts(x, ids, wts, up, down, "relu_squared", parts)
+    r = lambda t: t.bfloat16().double()                         # noqa: E731
+    for n in range(N):
+        for c in range(top):
+            e, wt = int(ids[n, c]), float(wts[n, c])
+            if e == E:
+                assert bool((parts[c, n] == 7.0).all())        # left alone
+                continue
+            z = r(up[e].double() @ x[n].double())
+            if gated:
+                z = z * (wt if weights_on == "input" else 1.0)
+                a, b = z[0::2].clamp(max=7.0), z[1::2].clamp(-7.0, 7.0)
+                y = r(a / (1 + torch.exp(-1.702 * a)) * (b + 1.0))
+            else:
+                y = r(z.clamp(min=0) ** 2)
+            want = r(down[e].double() @ y) * (wt if weights_on == "output" else 1.0)
+            # sums in another order flip a rounding to bfloat16 (2^-9) here and there: of the first products (twice in the
+            # activation), of y and of the result
+            assert float((parts[c, n].double() - want).norm() / want.norm()) <= 4 * 2.0 ** -9
