@@ -298,8 +298,8 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
 template <int MT>
 static void launch_f32_stream(const float* A, const float* W, float* C, int M, int N, int K, int lda, int ldw, int ldc,
                               bool wide, hipStream_t stream) {
-  if (N >= GS_TWO_GROUPS_FROM)
-    gemm_f32_stream_kernel<MT, 2><<<(N + 31) / 32, GS_WAVES * 64, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, wide);
+  if (MT == 1 && N >= GS_TWO_GROUPS_FROM)                              // two of both would not fit the registers
+    gemm_f32_stream_kernel<1, 2><<<(N + 31) / 32, GS_WAVES * 64, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, wide);
   else
     gemm_f32_stream_kernel<MT, 1><<<(N + 15) / 16, GS_WAVES * 64, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, wide);
 }
