@@ -37,6 +37,7 @@
 // zeroed (values) or masked (scores): a stale or poisoned page never leaks in.
 // A key that is needed but has no page in the block table gives NaN, not a fault.
 #include "common.h"
+#include "parts_join.h"
 #include <type_traits>
 
 #ifndef IA_HEAD_DIM
@@ -336,7 +337,29 @@ __global__ __launch_bounds__(WAVES * 64, ((WAVES == 4 && IA_MAX_DIM <= 128) ? 3 
   float qa[FUSED ? QPT : 1], qb[FUSED ? QPT : 1];
   const int half = FUSED ? F.rot >> 1 : 0;
   const TS* row = reinterpret_cast<const TS*>(F.src) + (size_t)b * F.row_stride;
+  // what lies behind the rotated part of a head (a latent's row: 224 of 256 values) is copied: eight values an access where
+  // the rows allow it, asked for here too (one value after the other behind the rotation took 7 of 18 us for one token)
+  constexpr int CPT = (16 * HD / 8 + NT - 1) / NT;
+  const bool has_tail = FUSED && F.rot < HD;
+  const int tail8 = (HD - F.rot) >> 3;
+  const bool copy8 = has_tail && sizeof(TS) == 2 && F.gsplits == 1 && (F.rot & 7) == 0 && (F.row_stride & 7) == 0 &&
+                     (reinterpret_cast<uintptr_t>(F.src) & 15) == 0;
+  uint4 qc[FUSED ? CPT : 1];
+  float kc = 0.f;                                           // the new key's value behind its rotated part, one a thread
   if (FUSED) {
+    if (copy8) {
+#pragma unroll
+      for (int u = 0; u < CPT; ++u) {
+        const int idx = tid + u * NT;
+        qc[u] = make_uint4(0u, 0u, 0u, 0u);
+        if (idx < heads_here * tail8) {
+          const int c = idx / tail8, i = F.rot + 8 * (idx - c * tail8);
+          qc[u] = *reinterpret_cast<const uint4*>(row + (size_t)(g * G + ht * 16 + c) * HD + i);
+        }
+      }
+    }
+    if (has_tail && F.slots != nullptr && F.rot + tid < HD)
+      kc = load_split_sum_together(row + (size_t)(nh + g) * HD + F.rot + tid, F.gsplits, F.split_stride);
 #pragma unroll
     for (int u = 0; u < QPT; ++u) {
       const int idx = tid + u * NT;
@@ -441,11 +464,22 @@ __global__ __launch_bounds__(WAVES * 64, ((WAVES == 4 && IA_MAX_DIM <= 128) ? 3 
         s_q[c][i + half] = float_to_bf16_bits(hi);
       }
     }
-    const int tail = HD - F.rot;                             // values beyond the rotated part: copies
-    for (int idx = tid; idx < heads_here * tail; idx += NT) {
-      const int c = idx / tail, i = F.rot + (idx - c * tail);
-      s_q[c][i] = float_to_bf16_bits(
-          load_split_sum(row + (size_t)(g * G + ht * 16 + c) * HD + i, F.gsplits, F.split_stride));
+    if (copy8) {                                             // values beyond the rotated part: copies
+#pragma unroll
+      for (int u = 0; u < CPT; ++u) {
+        const int idx = tid + u * NT;
+        if (idx < heads_here * tail8) {
+          const int c = idx / tail8;
+          *reinterpret_cast<uint4*>(&s_q[c][F.rot + 8 * (idx - c * tail8)]) = qc[u];
+        }
+      }
+    } else if (has_tail) {
+      const int tail = HD - F.rot;
+      for (int idx = tid; idx < heads_here * tail; idx += NT) {
+        const int c = idx / tail, i = F.rot + (idx - c * tail);
+        s_q[c][i] = float_to_bf16_bits(
+            load_split_sum(row + (size_t)(g * G + ht * 16 + c) * HD + i, F.gsplits, F.split_stride));
+      }
     }
     if (own_key) {
       if (tid < half) {
@@ -454,8 +488,7 @@ __global__ __launch_bounds__(WAVES * 64, ((WAVES == 4 && IA_MAX_DIM <= 128) ? 3 
         s_newk[tid] = float_to_bf16_bits(lo);
         s_newk[tid + half] = float_to_bf16_bits(hi);
       }
-      for (int i = F.rot + tid; i < HD; i += NT)
-        s_newk[i] = float_to_bf16_bits(load_split_sum(row + (size_t)(nh + g) * HD + i, F.gsplits, F.split_stride));
+      if (F.rot + tid < HD) s_newk[F.rot + tid] = float_to_bf16_bits(kc);
       if (tid < VD) s_newv[tid] = float_to_bf16_bits(vv);
       geo.patch_key = p;
     }
@@ -546,67 +579,13 @@ extern "C" __global__ __launch_bounds__(64) void attn_decode_reduce_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml, uint16_t* __restrict__ out,
     int out_row_stride, int nh, int num_splits, const float* __restrict__ sinks, const uint16_t* __restrict__ gate,
     int gate_stride) {
-  const int b = blockIdx.x / nh, h = blockIdx.x - b * nh, lane = threadIdx.x;
-  const size_t rec0 = (size_t)blockIdx.x * num_splits;
-  // the first parts' outputs are asked for together with the statistics, not after them
-  constexpr int PRE = 4, NC = (VD + 63) / 64;
-  float pre[PRE][NC];
-#pragma unroll
-  for (int j = 0; j < PRE; ++j)
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const int dim = lane + 64 * c;
-      pre[j][c] = (j < num_splits && dim < VD) ? part_o[(rec0 + j) * VD + dim] : 0.f;
-    }
-  float M = -INFINITY;
-  for (int s = lane; s < num_splits; s += 64) M = fmaxf(M, part_ml[(rec0 + s) * 2]);
-  M = wave_max(M);
-  float acc[NC];
-#pragma unroll
-  for (int c = 0; c < NC; ++c) acc[c] = 0.f;
-  float L = 0.f;
-  for (int s0 = 0; s0 < num_splits; s0 += 64) {
-    const int s = s0 + lane;
-    float wgt = 0.f, wl = 0.f;
-    if (s < num_splits) {
-      const float ms = part_ml[(rec0 + s) * 2];
-      wgt = (ms == -INFINITY) ? 0.f : exp2f(ms - M);
-      wl = wgt * part_ml[(rec0 + s) * 2 + 1];
-    }
-    const int cnt = (num_splits - s0) < 64 ? (num_splits - s0) : 64;
-    int j = 0;
-    if (s0 == 0) {
-#pragma unroll
-      for (; j < PRE; ++j) {
-        if (j >= cnt) break;
-        L += __shfl(wl, j, IA_WAVE);
-        const float wj = __shfl(wgt, j, IA_WAVE);
-#pragma unroll
-        for (int c = 0; c < NC; ++c) acc[c] += (wj != 0.f) ? wj * pre[j][c] : 0.f;
-      }
-    }
-    for (; j < cnt; ++j) {
-      L += __shfl(wl, j, IA_WAVE);
-      const float wj = __shfl(wgt, j, IA_WAVE);
-#pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        const int dim = lane + 64 * c;
-        // every part was written (an empty one holds zeros), so the load needs no guard and does not wait
-        const float v = dim < VD ? part_o[(rec0 + s0 + j) * VD + dim] : 0.f;
-        acc[c] += (wj != 0.f) ? wj * v : 0.f;
-      }
-    }
-  }
-  const float inv = 1.0f / (sinks ? L + exp2f(sinks[h] * 1.4426950408889634f - M) : L);
-#pragma unroll
-  for (int c = 0; c < (VD + 63) / 64; ++c) {
-    const int dim = lane + 64 * c;
-    if (dim >= VD) continue;
-    float v = acc[c] * inv;
-    if (BIAS && gate)
-      v *= 1.0f / (1.0f + __builtin_amdgcn_exp2f(-ATTN_LOG2E * bf16_bits_to_float(gate[(size_t)b * gate_stride + (size_t)h * VD + dim])));
-    out[(size_t)b * out_row_stride + (size_t)h * VD + dim] = float_to_bf16_bits(v);
-  }
+  const int b = blockIdx.x / nh, h = blockIdx.x - b * nh, dim = blockIdx.y * 64 + threadIdx.x;
+  const JoinedParts J = join_parts(part_o, part_ml, (size_t)blockIdx.x * num_splits, num_splits, VD, dim);
+  if (dim >= VD) return;
+  float v = J.sum * (1.0f / (sinks ? J.weight + exp2f(sinks[h] * 1.4426950408889634f - J.top) : J.weight));
+  if (BIAS && gate)
+    v *= 1.0f / (1.0f + __builtin_amdgcn_exp2f(-ATTN_LOG2E * bf16_bits_to_float(gate[(size_t)b * gate_stride + (size_t)h * VD + dim])));
+  out[(size_t)b * out_row_stride + (size_t)h * VD + dim] = float_to_bf16_bits(v);
 }
 
 // ----------------------------------------------------------------------- prefill
@@ -1083,7 +1062,7 @@ extern "C" int ia_attn_decode(const void* q, int q_row_stride, const void* k_pag
 #undef DEC_LAUNCH
   IA_LAUNCH_CHECK();
   if (num_splits > 1) {
-    attn_decode_reduce_kernel<<<B * nh, 64, 0, stream>>>(part_o, part_ml, (uint16_t*)out, out_row_stride, nh,
+    attn_decode_reduce_kernel<<<dim3(B * nh, (VD + 63) / 64), 64, 0, stream>>>(part_o, part_ml, (uint16_t*)out, out_row_stride, nh,
                                                          num_splits, sinks, X.gate, X.gate_stride);
     IA_LAUNCH_CHECK();
   }
@@ -1148,7 +1127,7 @@ extern "C" int ia_attn_decode_fused(const void* src, int src_dtype, int src_spli
 #undef DEC_FUSED_LAUNCH
   IA_LAUNCH_CHECK();
   if (num_splits > 1) {
-    attn_decode_reduce_kernel<<<B * nh, 64, 0, stream>>>(part_o, part_ml, (uint16_t*)out, out_row_stride, nh,
+    attn_decode_reduce_kernel<<<dim3(B * nh, (VD + 63) / 64), 64, 0, stream>>>(part_o, part_ml, (uint16_t*)out, out_row_stride, nh,
                                                          num_splits, sinks, nullptr, 0);
     IA_LAUNCH_CHECK();
   }

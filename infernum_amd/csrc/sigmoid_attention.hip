@@ -20,6 +20,41 @@
 
 #define SA_MAX_D 640
 
+// Bound by trips to memory where tokens are few: grid (N, 2), the queries' norm and the keys' and values' side by side, and
+// up to 8 values a thread (rows of 2,048) with their bias and weight asked for together and kept for the second use (one
+// token of 16 heads of 128: 13.4 us with the loads one after the other, twice, so 7.2).
+#define SQ_KEEP 8
+template <typename T>
+__device__ __forceinline__ float sq_value(const T* __restrict__ row, const float* __restrict__ b, int i) {
+  return to_float(row[i]) + (b ? b[i] : 0.f);
+}
+
+// emit(i, value over the root mean square times factor and w[i]) for every value of one norm of `n` values
+template <typename T, typename Factor, typename Emit>
+__device__ __forceinline__ void sq_norm(const T* __restrict__ row, const float* __restrict__ b, const float* __restrict__ w,
+                                        int n, float eps, float* red, Factor factor, Emit emit) {
+  const int tid = threadIdx.x;
+  float x[SQ_KEEP], wx[SQ_KEEP], ss = 0.f;
+#pragma unroll
+  for (int u = 0; u < SQ_KEEP; ++u) {
+    const int i = min(tid + 256 * u, n - 1);
+    x[u] = sq_value(row, b, i);
+    wx[u] = w[i];
+  }
+#pragma unroll
+  for (int u = 0; u < SQ_KEEP; ++u) ss = tid + 256 * u < n ? fmaf(x[u], x[u], ss) : ss;
+  for (int i = tid + 256 * SQ_KEEP; i < n; i += 256) {
+    const float v = sq_value(row, b, i);
+    ss = fmaf(v, v, ss);
+  }
+  ss = block_sum<256>(ss, red);
+  const float f = factor(1.0f / sqrtf(ss / (float)n + eps));
+#pragma unroll
+  for (int u = 0; u < SQ_KEEP; ++u)
+    if (tid + 256 * u < n) emit(tid + 256 * u, x[u] * f * wx[u]);
+  for (int i = tid + 256 * SQ_KEEP; i < n; i += 256) emit(i, sq_value(row, b, i) * f * w[i]);
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void sigattn_prepare_kernel(
     const T* __restrict__ proj, int proj_stride, const float* __restrict__ bq, const float* __restrict__ bk,
@@ -30,38 +65,24 @@ __global__ __launch_bounds__(256) void sigattn_prepare_kernel(
   const int n = blockIdx.x, tid = threadIdx.x;
   const T* row = proj + (size_t)n * proj_stride;
   const int nq = nh * dim, nk = nkv * dim, nv = nkv * vdim;
-  float ss = 0.f;
-  for (int i = tid; i < nq; i += 256) {
-    const float x = to_float(row[i]) + (bq ? bq[i] : 0.f);
-    ss = fmaf(x, x, ss);
+  if (blockIdx.y == 0) {
+    const int p = temp_every > 0 ? positions[n] : 0;
+    sq_norm(row, bq, wq, nq, eps, red,
+            [&](float f) { return temp_every > 0 ? f * (1.0f + temp_coef * logf((float)((p + 1) / temp_every) + 1.0f)) : f; },
+            [&](int i, float v) { q_out[(size_t)n * nq + i] = from_float<T>(v); });
+    return;
   }
-  ss = block_sum<256>(ss, red);
-  float f = 1.0f / sqrtf(ss / (float)nq + eps);
-  if (temp_every > 0) f *= 1.0f + temp_coef * logf((float)((positions[n] + 1) / temp_every) + 1.0f);
-  for (int i = tid; i < nq; i += 256) {
-    const float x = to_float(row[i]) + (bq ? bq[i] : 0.f);
-    q_out[(size_t)n * nq + i] = from_float<T>(x * f * wq[i]);
-  }
-  if (!slots) return;
   const int slot = slots[n];
   const int page = slot / page_size, off = slot - page * page_size;
   if ((unsigned)page >= (unsigned)num_pages) return;          // a token without a place: nothing is written
-  float sk = 0.f;
-  for (int i = tid; i < nk; i += 256) {
-    const float x = to_float(row[nq + i]) + (bk ? bk[i] : 0.f);
-    sk = fmaf(x, x, sk);
-  }
-  sk = block_sum<256>(sk, red);
-  const float fk = 1.0f / sqrtf(sk / (float)nk + eps);
-  for (int i = tid; i < nk; i += 256) {
-    const int g = i / dim, c = i - g * dim;
-    const float x = to_float(row[nq + i]) + (bk ? bk[i] : 0.f);
-    k_pages[(((size_t)page * nkv + g) * page_size + off) * dim + c] = from_float<T>(x * fk * wk[i]);
-  }
+  sq_norm(row + nq, bk, wk, nk, eps, red, [](float f) { return f; },
+          [&](int i, float v) {
+            const int g = i / dim, c = i - g * dim;
+            k_pages[(((size_t)page * nkv + g) * page_size + off) * dim + c] = from_float<T>(v);
+          });
   for (int i = tid; i < nv; i += 256) {
     const int g = i / vdim, c = i - g * vdim;
-    const float x = to_float(row[nq + nk + i]) + (bv ? bv[i] : 0.f);
-    v_pages[(((size_t)page * nkv + g) * vdim + c) * page_size + off] = from_float<T>(x);
+    v_pages[(((size_t)page * nkv + g) * vdim + c) * page_size + off] = from_float<T>(sq_value(row + nq + nk, bv, i));
   }
 }
 
@@ -79,12 +100,12 @@ extern "C" int ia_sigattn_prepare(const void* proj, int code, int proj_stride, c
   if (!proj || !wq || !q_out || !positions || (slots && (!wk || !k_pages || !v_pages || page_size <= 0 || num_pages <= 0)))
     return IA_ERR_BAD_ARG;
   if (code == IA_F32)
-    sigattn_prepare_kernel<float><<<N, 256, 0, stream>>>((const float*)proj, proj_stride, bq, bk, bv, wq, wk, eps,
+    sigattn_prepare_kernel<float><<<dim3(N, slots ? 2 : 1), 256, 0, stream>>>((const float*)proj, proj_stride, bq, bk, bv, wq, wk, eps,
                                                          temp_coef, temp_every, positions, slots, (float*)q_out,
                                                          (float*)k_pages, (float*)v_pages, nh, nkv, dim, vdim, page_size,
                                                          num_pages);
   else if (code == IA_BF16)
-    sigattn_prepare_kernel<bf16_t><<<N, 256, 0, stream>>>((const bf16_t*)proj, proj_stride, bq, bk, bv, wq, wk, eps,
+    sigattn_prepare_kernel<bf16_t><<<dim3(N, slots ? 2 : 1), 256, 0, stream>>>((const bf16_t*)proj, proj_stride, bq, bk, bv, wq, wk, eps,
                                                           temp_coef, temp_every, positions, slots, (bf16_t*)q_out,
                                                           (bf16_t*)k_pages, (bf16_t*)v_pages, nh, nkv, dim, vdim,
                                                           page_size, num_pages);

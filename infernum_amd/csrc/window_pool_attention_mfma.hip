@@ -23,6 +23,7 @@
 // Values of keys that no column of the tile sees are zeroed after the load and their weights are zero: a page that
 // went back to the pool never leaks in.  A key that is needed but has no page in the block table gives NaN.
 #include "common.h"
+#include "parts_join.h"
 
 #ifndef WP_DIM
 #error "compile with -DWP_DIM=<key size> -DWP_VDIM=<value size>"
@@ -443,7 +444,8 @@ __global__ __launch_bounds__(256) void wpa_decode_kernel(
     const uint16_t* __restrict__ v_pages, const uint16_t* __restrict__ pk_pages, const uint16_t* __restrict__ pv_pages,
     uint16_t* __restrict__ out, const float* __restrict__ sinks, const int* __restrict__ positions,
     const int* __restrict__ bt_tok, int bt_tok_stride, const int* __restrict__ bt_pool, int bt_pool_stride, int nh,
-    int nkv, int ps, int num_pages, int num_pool_pages, float scale_log2, int window, int P) {
+    int nkv, int ps, int num_pages, int num_pool_pages, float scale_log2, int window, int P, int num_parts,
+    float* __restrict__ part_o, float* __restrict__ part_ml) {
   __shared__ f32x4 red[3][NSV][64];
   __shared__ float s_m[4][16], s_l[4][64];
   __shared__ int s_bad;
@@ -472,11 +474,16 @@ __global__ __launch_bounds__(256) void wpa_decode_kernel(
   bool bad = false;
   const int lo = wp_first_key(p, window), nb = wp_blocks_seen(p, window, P);
   const int pos = col_ok ? p : -1, nbc = col_ok ? nb : 0;
-  const int block_tiles = (nb + 15) / 16;
-  for (int i = wave; i < block_tiles; i += 4) wp_tile_blocks<POW2>(G, i * 16, j, qd, nbc, nb, scale_log2, qr, c, o, bad);
+  // this workgroup's part of the tiles: those of blocks, then those of keys
+  const int block_tiles = (nb + 15) / 16, t_lo = lo / 16, tiles = block_tiles + p / 16 - t_lo + 1;
+  const int per = (tiles + num_parts - 1) / num_parts;
+  const int i0 = blockIdx.z * per, i1 = min(tiles, i0 + per), ib = min(i1, block_tiles);
+  for (int i = i0 + wave; i < ib; i += 4) wp_tile_blocks<POW2>(G, i * 16, j, qd, nbc, nb, scale_log2, qr, c, o, bad);
   // the tiles of keys go round the waves from where the tiles of blocks stopped, so that no wave has two more
-  const int turn = (wave + 4 - block_tiles % 4) % 4;
-  wp_walk_keys<POW2, 1, true>(G, (lo / 16 + turn) * 16, 64, j, qd, lo, pos, lo, p, scale_log2, qr1, c1, o1, bad);
+  const int turn = (wave + 4 - max(ib - i0, 0) % 4) % 4;
+  const int tk = t_lo + max(i0, block_tiles) - block_tiles, k_end = min(p, (t_lo + i1 - block_tiles) * 16 - 1);
+  if (i1 > block_tiles && i0 < i1)
+    wp_walk_keys<POW2, 1, true>(G, (tk + turn) * 16, 64, j, qd, lo, pos, lo, k_end, scale_log2, qr1, c1, o1, bad);
   // ---- the waves meet: a common maximum, then sums in the order of the waves
   if (qd == 0) s_m[wave][j] = c.m;
   __syncthreads();
@@ -499,6 +506,16 @@ __global__ __launch_bounds__(256) void wpa_decode_kernel(
   for (int w = 0; w < 4; ++w)
 #pragma unroll
     for (int x = 0; x < 4; ++x) l += s_l[w][x * 16 + j];
+  if (num_parts > 1) {
+    const size_t rec = ((size_t)b * nh + h) * num_parts + blockIdx.z;
+#pragma unroll
+    for (int n = 0; n < NSV; ++n) *reinterpret_cast<f32x4*>(part_o + rec * WP_VDIM + 4 * qd + n * 16) = o[n];
+    if (qd == 0) {
+      part_ml[rec * 2] = M;
+      part_ml[rec * 2 + 1] = s_bad ? __uint_as_float(0x7fc00000u) : l;
+    }
+    return;
+  }
   if (sinks) l += __builtin_amdgcn_exp2f(sinks[h] * WP_LOG2E - M);
   float inv = 1.0f / l;
   if (s_bad) inv = __uint_as_float(0x7fc00000u);
@@ -550,29 +567,47 @@ extern "C" int ia_wpa_prefill(const void* q, int q_stride, const void* k_pages, 
   return IA_OK;
 }
 
+__global__ __launch_bounds__(64) void wpa_join_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
+                                                      uint16_t* __restrict__ out, const float* __restrict__ sinks, int nh,
+                                                      int num_parts) {
+  const int h = blockIdx.x % nh, dim = blockIdx.y * 64 + threadIdx.x;
+  const JoinedParts J = join_parts(part_o, part_ml, (size_t)blockIdx.x * num_parts, num_parts, WP_VDIM, dim);
+  if (dim >= WP_VDIM) return;
+  const float l = sinks ? J.weight + __builtin_amdgcn_exp2f(sinks[h] * WP_LOG2E - J.top) : J.weight;
+  out[(size_t)blockIdx.x * WP_VDIM + dim] = float_to_bf16_bits(J.sum * (1.0f / l));
+}
+
+// num_parts > 1: the tiles of a request's blocks and keys are cut into so many parts, a workgroup each, which leave
+// part_o [B, nh, num_parts, WP_VDIM] and part_ml [B, nh, num_parts, 2] for the join's launch.
 extern "C" int ia_wpa_decode(const void* q, int q_stride, const void* k_pages, const void* v_pages, const void* pk_pages,
                              const void* pv_pages, void* out, const float* sinks, const int* positions, const int* bt_tok,
                              int bt_tok_stride, const int* bt_pool, int bt_pool_stride, int B, int nh, int nkv, int ps,
-                             int num_pages, int num_pool_pages, float scale, int window, int P, hipStream_t stream) {
+                             int num_pages, int num_pool_pages, float scale, int window, int P, int num_parts,
+                             float* part_o, float* part_ml, hipStream_t stream) {
   if (B < 0) return IA_ERR_BAD_ARG;
   const int rc = wp_check(nh, nkv, ps, num_pages, bt_tok_stride, q_stride, window, P, pk_pages, pv_pages, bt_pool,
                           bt_pool_stride, num_pool_pages);
   if (rc != IA_OK) return rc;
   if (B == 0) return IA_OK;
   if (!q || !k_pages || !v_pages || !out || !positions || !bt_tok) return IA_ERR_BAD_ARG;
+  if (num_parts < 1 || num_parts > 64 || (num_parts > 1 && (!part_o || !part_ml))) return IA_ERR_BAD_ARG;
   const int HC = (nh / nkv + 15) / 16;
   if ((long long)nkv * HC > 65535) return IA_ERR_UNSUPPORTED;
   if (!(window > 0 && P > 0)) P = 0;
-  dim3 grid(B, nkv * HC);
+  dim3 grid(B, nkv * HC, num_parts);
 #define WP_DEC(P2)                                                                                                 \
   wpa_decode_kernel<P2><<<grid, 256, 0, stream>>>(                                                                 \
       (const uint16_t*)q, q_stride, (const uint16_t*)k_pages, (const uint16_t*)v_pages, (const uint16_t*)pk_pages, \
       (const uint16_t*)pv_pages, (uint16_t*)out, sinks, positions, bt_tok, bt_tok_stride, bt_pool, bt_pool_stride, \
-      nh, nkv, ps, num_pages, num_pool_pages, scale * WP_LOG2E, window, P)
+      nh, nkv, ps, num_pages, num_pool_pages, scale * WP_LOG2E, window, P, num_parts, part_o, part_ml)
   if ((ps & (ps - 1)) == 0) WP_DEC(true);
   else WP_DEC(false);
 #undef WP_DEC
   IA_LAUNCH_CHECK();
+  if (num_parts > 1) {
+    wpa_join_kernel<<<dim3(B * nh, (WP_VDIM + 63) / 64), 64, 0, stream>>>(part_o, part_ml, (uint16_t*)out, sinks, nh, num_parts);
+    IA_LAUNCH_CHECK();
+  }
   return IA_OK;
 }
 

@@ -2036,22 +2036,50 @@ def _wpa_check(q, k_pages, v_pages, pk_pages, pv_pages, out, sinks, bt_tokens, b
     return pooled, ps, num_pages, d, dv
 
 
+def wpa_decode_parts(batch: int, nh: int, nkv: int, max_len: int, window: int, pool: int,
+                     device: Optional[torch.device] = None) -> int:
+    """Parts that the tiles of a token's keys and blocks are cut into (a workgroup of four waves each): as many as bring
+    the workgroups to the compute units, at most the square root of the tiles (the join grows with the parts as the work of
+    one shrinks: one request on 4 key/value heads, 1,024 keys and 31 blocks, takes 36 us whole and 13 + 6 in 8 parts)
+    and 16."""
+    groups = max(1, batch * nkv * ((nh // nkv + 15) // 16))
+    keys = min(max_len, window + 15) if window > 0 else max_len
+    blocks = max(0, max_len - window) // pool if window > 0 and pool > 0 else 0
+    tiles = (keys + 15) // 16 + (blocks + 15) // 16
+    return max(1, min(compute_units(device) // groups, math.isqrt(max(tiles, 1)), 16))
+
+
+def wpa_decode_part_floats(nh: int, nkv: int, dv: int, device: Optional[torch.device] = None) -> int:
+    """Floats that the parts of any number of tokens take (outputs; a sixteenth of it at the least for their statistics)."""
+    per_group = -(-nh // (nkv * ((nh // nkv + 15) // 16)))        # query heads a workgroup, at the most
+    return compute_units(device) * per_group * dv
+
+
 def wpa_decode(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, pk_pages: Optional[torch.Tensor],
                pv_pages: Optional[torch.Tensor], out: torch.Tensor, sinks: Optional[torch.Tensor],
                positions: torch.Tensor, bt_tokens: torch.Tensor, bt_pool: Optional[torch.Tensor], nh: int, nkv: int,
-               scale: float, window: int, pool: int) -> torch.Tensor:
+               scale: float, window: int, pool: int, max_len: Optional[int] = None,
+               num_parts: Optional[int] = None) -> torch.Tensor:
     """:func:`wpa_attention` of B single tokens on the matrix cores, bf16: row b of q, out and the block tables is
-    token b at positions[b]."""
+    token b at positions[b].  ``max_len`` bounds the positions (default: what the block table holds) and sets into how many
+    parts the keys are cut."""
     pooled, ps, num_pages, d, dv = _wpa_check(q, k_pages, v_pages, pk_pages, pv_pages, out, sinks, bt_tokens, bt_pool,
                                               nh, nkv, window, pool, "wpa_decode")
     B = out.shape[0]
+    parts = num_parts or wpa_decode_parts(B, nh, nkv, max_len or bt_tokens.shape[1] * ps, window, pool if pooled else 0,
+                                          out.device)
+    part_o = part_ml = None
+    if parts > 1:
+        part_o = torch.empty(B * nh * parts * dv, dtype=torch.float32, device=out.device)
+        part_ml = torch.empty(B * nh * parts * 2, dtype=torch.float32, device=out.device)
     _i32(positions, B, "wpa_decode positions")
     _need(bt_tokens.shape[0] >= B and (not pooled or bt_pool.shape[0] >= B), "wpa_decode: a row of the block tables a token")
     _ok(_wpa(d, dv).ia_wpa_decode(_p(q), int(q.stride(0)), _p(k_pages), _p(v_pages), _p(pk_pages if pooled else None),
                                   _p(pv_pages if pooled else None), _p(out), _p(sinks), _p(positions), _p(bt_tokens),
                                   bt_tokens.shape[1], _p(bt_pool if pooled else None), bt_pool.shape[1] if pooled else 0,
                                   B, nh, nkv, ps, num_pages, pk_pages.shape[0] if pooled else 0, ctypes.c_float(scale),
-                                  int(window), int(pool) if pooled else 0, _stream()), "wpa_decode")
+                                  int(window), int(pool) if pooled else 0, parts, _p(part_o), _p(part_ml), _stream()),
+        "wpa_decode")
     return out
 
 

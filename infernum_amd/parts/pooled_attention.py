@@ -141,7 +141,7 @@ class PooledWindowAttention(Mixer):
             nd = ctx.num_decode
             if nd > 0:
                 K.wpa_decode(q[:nd], kp, vp, pk, pv, out[:nd], None, ctx.positions[:nd], bt, bt_pool, nh, nkv, self.scale,
-                             self.window, self.pool)
+                             self.window, self.pool, ctx.max_total_len)
             if ctx.num_seqs > nd:
                 tiles, num_tiles = ctx.row_tiles(K.PREFILL_TILE_ROWS)
                 K.wpa_prefill(q, kp, vp, pk, pv, out, None, ctx.seq_starts, ctx.seq_ctx, bt, bt_pool, tiles, num_tiles,
@@ -183,9 +183,16 @@ class PooledWindowAttention(Mixer):
         if self.use_mfma and ps % 4 == 0:
             lib = K._wpa(d, dv)
             tiles, num_tiles = program.row_tiles(K.PREFILL_TILE_ROWS)
+            pool = self.pool if blocks is not None else 0
+            parts = program.scalar(("wpa parts", nh, nkv, self.window, pool), lambda c: K.wpa_decode_parts(
+                c.num_decode, nh, nkv, c.max_total_len, self.window, pool, rt.device))
+            most = K.wpa_decode_part_floats(nh, nkv, dv, rt.device)
+            part_o = program.buffer("wpa.parts", most * 4)
+            part_ml = program.buffer("wpa.stats", most // dv * 2 * 4)
             program.op(lib, "ia_wpa_decode", [q, nh * d, kp, vp, pk, pv, out, None, program.positions, bt, bt_cols, bt_pool,
                                               pool_cols, program.ND, nh, nkv, ps, num_pages, pool_pages, float(self.scale),
-                                              self.window, self.pool, STREAM], Guard.between(program.ND, 1))
+                                              self.window, self.pool, parts, part_o, part_ml, STREAM],
+                       Guard.between(program.ND, 1))
             program.op(lib, "ia_wpa_prefill", [q, nh * d, kp, vp, pk, pv, out, None, program.seq_starts, program.seq_ctx,
                                                bt, bt_cols, bt_pool, pool_cols, tiles, num_tiles, nh, nkv, ps, num_pages,
                                                pool_pages, float(self.scale), self.window, self.pool, STREAM],

@@ -311,6 +311,31 @@ def test_sinks_in_the_matrix_core_kernels_against_the_plain_kernel(nh, nkv, d, p
     assert rel_err(got, want.double().cpu()) <= 3e-2
 
 
+@pytest.mark.parametrize("parts", [2, 3, 16, 17, 64])
+@pytest.mark.parametrize("nh,nkv,d,dv,ps,window,pool", [(4, 2, 16, 32, 4, 20, 6), (17, 1, 64, 64, 16, 1, 1), (3, 3, 48, 16, 12, 0, 0)])
+def test_window_and_blocks_in_parts(nh, nkv, d, dv, ps, window, pool, parts):
+    """Single tokens whose keys are cut into parts (also more parts than there are tiles) against the same kernel whole.
+    The weights of either are rounded to bfloat16 against maxima of their own, 2^-9 of a weight each, and so is the result:
+    the two differ by at most 2 * 2^-9 of the weighted mean of |v| and one rounding each of the result, at most 2^-7 max |v|."""
+    from infernum_amd.kernels import api as K
+    g = torch.Generator().manual_seed(11)
+    lens = [1, 16, 17, 333]
+    B, MB = len(lens), -(-max(lens) // ps)
+    E = K.wpa_pool_entries(ps, pool) if pool else 1
+    draw = lambda *shape: torch.randn(*shape, generator=g).to(torch.bfloat16).to(DEV)   # noqa: E731
+    pages = B * MB
+    kp, vp, pk, pv = draw(pages, nkv, ps, d), draw(pages, nkv, dv, ps), draw(pages, nkv, E, d), draw(pages, nkv, E, dv)
+    bt = torch.randperm(pages, generator=g).to(torch.int32).view(B, MB).to(DEV)
+    q = draw(B, nh * d)
+    pos = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device=DEV)
+    scale, sinks = 2.0 / math.sqrt(d), torch.randn(nh, generator=g).to(DEV)
+    whole, cut = (torch.empty((B, nh * dv), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    for s in (None, sinks):
+        K.wpa_decode(q, kp, vp, pk, pv, whole, s, pos, bt, bt, nh, nkv, scale, window, pool, num_parts=1)
+        K.wpa_decode(q, kp, vp, pk, pv, cut, s, pos, bt, bt, nh, nkv, scale, window, pool, num_parts=parts)
+        assert (whole.float() - cut.float()).abs().max() <= 2 ** -7 * max(vp.abs().max(), pv.abs().max()).float()
+
+
 @pytest.mark.parametrize("nh,nkv,d,dv,ps,window,pool", [(4, 2, 16, 32, 4, 20, 6), (6, 2, 64, 64, 16, 40, 10), (20, 1, 32, 16, 8, 1, 1),
                                                         (3, 3, 48, 16, 12, 0, 0), (4, 2, 16, 16, 16, 33, 16), (2, 1, 128, 128, 16, 7, 9),
                                                         (17, 1, 16, 16, 4, 40, 5)])
