@@ -108,13 +108,6 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(float* __restrict__ h,
   }
 }
 
-// Four consecutive values of a row as floats.
-__device__ __forceinline__ float4 load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
-__device__ __forceinline__ float4 load4(const bf16_t* p) {
-  const uint2 u = *reinterpret_cast<const uint2*>(p);
-  return make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
-                     __uint_as_float(u.y & 0xffff0000u));
-}
 __device__ __forceinline__ float4 load4_any(const void* p, int dtype, int i) {
   return dtype == IA_F32 ? load4((const float*)p + i) : load4((const bf16_t*)p + i);
 }
@@ -152,30 +145,43 @@ __global__ __launch_bounds__(NT) void add_rmsnorm_vec_kernel(float* __restrict__
   const TD* dr = delta ? delta + (size_t)src * H : nullptr;
   const bool store = (rows == nullptr) && (delta != nullptr);
   float4 v[MAXV], g[MAXV];     // the norm's weights are asked for with the row, not after the sum of squares
+  if (MAXV == 1) {             // one piece a thread: a wave of the row's end reads its last piece where it has none
+    const int il = min((int)threadIdx.x * 4, H - 4);
+    v[0] = g[0] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (((int)__builtin_amdgcn_readfirstlane(threadIdx.x) & ~63) * 4 < H) {
+      v[0] = load4(hr + il);
+      const Raw4 graw = load_raw4(w, w_dtype, il);
+      if (dr) {
+        const float4 d = load_parts4(dr + il, splits, split_stride);
+        v[0].x += d.x; v[0].y += d.y; v[0].z += d.z; v[0].w += d.w;
+      }
+      g[0] = raw4_values(graw, w_dtype);
+    }
+  } else {
 #pragma unroll
-  for (int c = 0; c < MAXV; ++c) {
-    const int i = (threadIdx.x + c * NT) * 4;
-    v[c] = (i < H) ? load4(hr + i) : make_float4(0.f, 0.f, 0.f, 0.f);
-    g[c] = (i < H) ? load4_any(w, w_dtype, i) : make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-  if (dr) {
-    float4 ds[MAXV];
-    constexpr int UNROLL_PARTS = MAXV == 1 ? 8 : 4;
+    for (int c = 0; c < MAXV; ++c) {
+      const int i = (threadIdx.x + c * NT) * 4;
+      v[c] = (i < H) ? load4(hr + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+      g[c] = (i < H) ? load4_any(w, w_dtype, i) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    if (dr) {
+      float4 ds[MAXV];
 #pragma unroll
-    for (int c = 0; c < MAXV; ++c) ds[c] = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma clang loop unroll_count(UNROLL_PARTS)
-    for (int k = 0; k < splits; ++k) {           // unrolled: the loads of several parts are in flight together
+      for (int c = 0; c < MAXV; ++c) ds[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma clang loop unroll_count(4)
+      for (int k = 0; k < splits; ++k) {           // unrolled: the loads of several parts are in flight together
 #pragma unroll
-      for (int c = 0; c < MAXV; ++c) {
-        const int i = (threadIdx.x + c * NT) * 4;
-        if (i < H) {
-          const float4 d = load4(dr + k * split_stride + i);
-          ds[c].x += d.x; ds[c].y += d.y; ds[c].z += d.z; ds[c].w += d.w;
+        for (int c = 0; c < MAXV; ++c) {
+          const int i = (threadIdx.x + c * NT) * 4;
+          if (i < H) {
+            const float4 d = load4(dr + k * split_stride + i);
+            ds[c].x += d.x; ds[c].y += d.y; ds[c].z += d.z; ds[c].w += d.w;
+          }
         }
       }
-    }
 #pragma unroll
-    for (int c = 0; c < MAXV; ++c) { v[c].x += ds[c].x; v[c].y += ds[c].y; v[c].z += ds[c].z; v[c].w += ds[c].w; }
+      for (int c = 0; c < MAXV; ++c) { v[c].x += ds[c].x; v[c].y += ds[c].y; v[c].z += ds[c].z; v[c].w += ds[c].w; }
+    }
   }
   float ss = 0.f;
   if (AS_WIDE) {
@@ -234,13 +240,16 @@ static int launch_add_rmsnorm(float* h, const void* delta, int splits, size_t sp
       add_rmsnorm_vec_kernel<TD, TO, 256, true><<<N, 256, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o,
                                                                         rows, H, eps);
     else if (H >= 2048 && H <= 4096)
-      // one piece a thread: few registers, so the loads of up to eight partial sums are in flight together
+      // one piece a thread: few registers, so the loads of up to sixteen partial sums are in flight together
       // (the sums are the same: the pieces beyond the first are empty at this width)
       add_rmsnorm_vec_kernel<TD, TO, 1024, false, 1><<<N, 1024, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o,
                                                                               rows, H, eps);
     else if (H >= 2048)
       add_rmsnorm_vec_kernel<TD, TO, 1024><<<N, 1024, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, rows,
                                                                     H, eps);
+    else if (H <= 1024)        // as above: one piece a thread
+      add_rmsnorm_vec_kernel<TD, TO, 256, false, 1><<<N, 256, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o,
+                                                                            rows, H, eps);
     else
       add_rmsnorm_vec_kernel<TD, TO, 256><<<N, 256, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, rows, H,
                                                                   eps);

@@ -55,12 +55,6 @@ __global__ __launch_bounds__(NB_NT) void norm_add_kernel(float* __restrict__ h, 
 
 // Rows of a multiple of 4 values up to NT * 4 * NV: every thread keeps its pieces of the row in registers, read 16
 // (or 8) bytes at a time with the loads of all parts of a piece in flight together; one pass over memory.
-__device__ __forceinline__ float4 nb_load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
-__device__ __forceinline__ float4 nb_load4(const bf16_t* p) {
-  const uint2 u = *reinterpret_cast<const uint2*>(p);
-  return make_float4(__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
-                     __uint_as_float(u.y & 0xffff0000u));
-}
 __device__ __forceinline__ void nb_store4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
 __device__ __forceinline__ void nb_store4(bf16_t* p, float4 v) {
   uint2 u;
@@ -79,24 +73,36 @@ __global__ __launch_bounds__(NT) void norm_add_vec_kernel(float* __restrict__ h,
   const TD* dr = delta + (size_t)row * H;
   float* hr = h + (size_t)row * H;
   float4 d[NV], hv[NV], g[NV];
-#pragma unroll
-  for (int c = 0; c < NV; ++c) {
-    const int i = (threadIdx.x + c * NT) * 4;
-    d[c] = hv[c] = g[c] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (i < H) {
-      hv[c] = nb_load4(hr + i);
-      g[c] = w_dtype == IA_F32 ? nb_load4((const float*)w + i) : nb_load4((const bf16_t*)w + i);
-      d[c] = nb_load4(dr + i);
+  if (NV == 1) {                                     // one piece a thread: everything is asked for before the first use
+    const int il = min((int)threadIdx.x * 4, H - 4);
+    d[0] = hv[0] = g[0] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (((int)__builtin_amdgcn_readfirstlane(threadIdx.x) & ~63) * 4 < H) {
+      hv[0] = load4(hr + il);
+      const Raw4 graw = load_raw4(w, w_dtype, il);
+      d[0] = load_parts4(dr + il, splits, split_stride);
+      g[0] = raw4_values(graw, w_dtype);
+      if ((int)threadIdx.x * 4 >= H) d[0] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
-  }
-#pragma clang loop unroll_count(4)
-  for (int k = 1; k < splits; ++k) {                 // the parts in the order of their index
+  } else {
 #pragma unroll
     for (int c = 0; c < NV; ++c) {
       const int i = (threadIdx.x + c * NT) * 4;
+      d[c] = hv[c] = g[c] = make_float4(0.f, 0.f, 0.f, 0.f);
       if (i < H) {
-        const float4 p = nb_load4(dr + k * split_stride + i);
-        d[c].x += p.x; d[c].y += p.y; d[c].z += p.z; d[c].w += p.w;
+        hv[c] = load4(hr + i);
+        g[c] = w_dtype == IA_F32 ? load4((const float*)w + i) : load4((const bf16_t*)w + i);
+        d[c] = load4(dr + i);
+      }
+    }
+#pragma clang loop unroll_count(4)
+    for (int k = 1; k < splits; ++k) {                 // the parts in the order of their index
+#pragma unroll
+      for (int c = 0; c < NV; ++c) {
+        const int i = (threadIdx.x + c * NT) * 4;
+        if (i < H) {
+          const float4 p = load4(dr + k * split_stride + i);
+          d[c].x += p.x; d[c].y += p.y; d[c].z += p.z; d[c].w += p.w;
+        }
       }
     }
   }
@@ -232,7 +238,7 @@ __global__ __launch_bounds__(NB_NT) void gated_norm_add_kernel(float* __restrict
 // a thread keeps its pieces of the row in registers, read 16 (or 8) bytes at a time, the loads of all parts of a piece
 // in flight together; one pass over memory.  The sums of a row are taken in one order whatever the batch holds.
 __device__ __forceinline__ float4 nb_load4_any(const void* p, int dtype, int i) {
-  return dtype == IA_F32 ? nb_load4((const float*)p + i) : nb_load4((const bf16_t*)p + i);
+  return dtype == IA_F32 ? load4((const float*)p + i) : load4((const bf16_t*)p + i);
 }
 
 template <typename TD, typename TG, typename TX, int NT, int NV>
@@ -249,44 +255,67 @@ __global__ __launch_bounds__(NT) void gated_norm_add_vec_kernel(float* __restric
   const TD* dr = delta + (size_t)row * H;
   float* hr = h + (size_t)row * H;
   float4 d[NV], hv[NV];
-#pragma unroll
-  for (int c = 0; c < NV; ++c) {
-    const int i = (threadIdx.x + c * NT) * 4;
-    d[c] = hv[c] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (i < H) {
-      hv[c] = nb_load4(hr + i);
-      d[c] = nb_load4(dr + i);
+  Raw4 wraw, nraw;
+  if (NV == 1) {                                     // one piece a thread: everything is asked for before the first use
+    const int il = min((int)threadIdx.x * 4, H - 4);
+    d[0] = hv[0] = make_float4(0.f, 0.f, 0.f, 0.f);
+    wraw.u = nraw.u = make_uint4(0u, 0u, 0u, 0u);
+    if (((int)__builtin_amdgcn_readfirstlane(threadIdx.x) & ~63) * 4 < H) {
+      hv[0] = load4(hr + il);
+      wraw = load_raw4(w, w_dtype, il);
+      if (w_next) nraw = load_raw4(w_next, w_next_dtype, il);
+      const float4 b = gate_bias ? load4(gate_bias + il) : make_float4(0.f, 0.f, 0.f, 0.f);
+      d[0] = load_parts4(dr + il, splits, split_stride);
+      if (gate) {
+        float4 z = load_parts4(gate + (size_t)row * gate_stride + il, gate_splits, gate_split_stride);
+        z.x += b.x; z.y += b.y; z.z += b.z; z.w += b.w;
+        d[0].x *= 1.0f / (1.0f + expf(-z.x));
+        d[0].y *= 1.0f / (1.0f + expf(-z.y));
+        d[0].z *= 1.0f / (1.0f + expf(-z.z));
+        d[0].w *= 1.0f / (1.0f + expf(-z.w));
+      }
+      if ((int)threadIdx.x * 4 >= H) d[0] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
-  }
-#pragma clang loop unroll_count(4)
-  for (int k = 1; k < splits; ++k) {                 // the parts in the order of their index
+  } else {
 #pragma unroll
     for (int c = 0; c < NV; ++c) {
       const int i = (threadIdx.x + c * NT) * 4;
+      d[c] = hv[c] = make_float4(0.f, 0.f, 0.f, 0.f);
       if (i < H) {
-        const float4 p = nb_load4(dr + k * split_stride + i);
-        d[c].x += p.x; d[c].y += p.y; d[c].z += p.z; d[c].w += p.w;
+        hv[c] = load4(hr + i);
+        d[c] = load4(dr + i);
       }
     }
-  }
-  if (gate) {
+#pragma clang loop unroll_count(4)
+    for (int k = 1; k < splits; ++k) {                 // the parts in the order of their index
 #pragma unroll
-    for (int c = 0; c < NV; ++c) {
-      const int i = (threadIdx.x + c * NT) * 4;
-      if (i < H) {
-        float4 z = nb_load4(gate + (size_t)row * gate_stride + i);
-        for (int k = 1; k < gate_splits; ++k) {        // the logits' parts in the order of their index
-          const float4 q = nb_load4(gate + k * gate_split_stride + (size_t)row * gate_stride + i);
-          z.x += q.x; z.y += q.y; z.z += q.z; z.w += q.w;
+      for (int c = 0; c < NV; ++c) {
+        const int i = (threadIdx.x + c * NT) * 4;
+        if (i < H) {
+          const float4 p = load4(dr + k * split_stride + i);
+          d[c].x += p.x; d[c].y += p.y; d[c].z += p.z; d[c].w += p.w;
         }
-        if (gate_bias) {
-          const float4 b = nb_load4(gate_bias + i);
-          z.x += b.x; z.y += b.y; z.z += b.z; z.w += b.w;
+      }
+    }
+    if (gate) {
+#pragma unroll
+      for (int c = 0; c < NV; ++c) {
+        const int i = (threadIdx.x + c * NT) * 4;
+        if (i < H) {
+          float4 z = load4(gate + (size_t)row * gate_stride + i);
+          for (int k = 1; k < gate_splits; ++k) {        // the logits' parts in the order of their index
+            const float4 q = load4(gate + k * gate_split_stride + (size_t)row * gate_stride + i);
+            z.x += q.x; z.y += q.y; z.z += q.z; z.w += q.w;
+          }
+          if (gate_bias) {
+            const float4 b = load4(gate_bias + i);
+            z.x += b.x; z.y += b.y; z.z += b.z; z.w += b.w;
+          }
+          d[c].x *= 1.0f / (1.0f + expf(-z.x));
+          d[c].y *= 1.0f / (1.0f + expf(-z.y));
+          d[c].z *= 1.0f / (1.0f + expf(-z.z));
+          d[c].w *= 1.0f / (1.0f + expf(-z.w));
         }
-        d[c].x *= 1.0f / (1.0f + expf(-z.x));
-        d[c].y *= 1.0f / (1.0f + expf(-z.y));
-        d[c].z *= 1.0f / (1.0f + expf(-z.z));
-        d[c].w *= 1.0f / (1.0f + expf(-z.w));
       }
     }
   }
@@ -301,7 +330,7 @@ __global__ __launch_bounds__(NT) void gated_norm_add_vec_kernel(float* __restric
   for (int c = 0; c < NV; ++c) {
     const int i = (threadIdx.x + c * NT) * 4;
     if (i < H) {
-      const float4 g = nb_load4_any(w, w_dtype, i);
+      const float4 g = NV == 1 ? raw4_values(wraw, w_dtype) : nb_load4_any(w, w_dtype, i);
       hv[c] = make_float4(hv[c].x + d[c].x * inv * g.x, hv[c].y + d[c].y * inv * g.y, hv[c].z + d[c].z * inv * g.z,
                           hv[c].w + d[c].w * inv * g.w);
       nb_store4(hr + i, hv[c]);
@@ -320,7 +349,7 @@ __global__ __launch_bounds__(NT) void gated_norm_add_vec_kernel(float* __restric
     if (i < H) {
       float4 o = hv[c];
       if (w_next) {
-        const float4 g = nb_load4_any(w_next, w_next_dtype, i);
+        const float4 g = NV == 1 ? raw4_values(nraw, w_next_dtype) : nb_load4_any(w_next, w_next_dtype, i);
         o = make_float4(o.x * inv2 * g.x, o.y * inv2 * g.y, o.z * inv2 * g.z, o.w * inv2 * g.w);
       }
       nb_store4(x + (size_t)row * H + i, o);

@@ -1184,24 +1184,8 @@ extern "C" int ia_stream_add(float* h, const void* delta, int code, int splits, 
 // h += a, then h += b (nullable), each a tensor or a stack of partial sums as in ia_stream_add, the additions in that
 // order; x (nullable) gets the new h in its own type: the two results of sublayers that ran side by side enter the
 // stream in one pass, which also leaves the rounded stream for whoever reads it next.  Four values a thread.
-__device__ __forceinline__ void sa2_load4(const void* p, int code, size_t i, float (&v)[4]) {
-  if (code == IA_F32) {
-    const float4 f = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(p) + i);
-    v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
-  } else {
-    const uint2 u = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(p) + i);
-    v[0] = bf16_bits_to_float((uint16_t)(u.x & 0xffffu)); v[1] = bf16_bits_to_float((uint16_t)(u.x >> 16));
-    v[2] = bf16_bits_to_float((uint16_t)(u.y & 0xffffu)); v[3] = bf16_bits_to_float((uint16_t)(u.y >> 16));
-  }
-}
-__device__ __forceinline__ void sa2_sum4(const void* p, int code, int splits, size_t i, size_t n, float (&v)[4]) {
-  sa2_load4(p, code, i, v);
-  for (int k = 1; k < splits; ++k) {
-    float w[4];
-    sa2_load4(p, code, i + (size_t)k * n, w);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] += w[e];
-  }
+__device__ __forceinline__ float4 sa2_sum4(const void* p, int code, int splits, size_t i, size_t n) {
+  return code == IA_F32 ? load_parts4((const float*)p + i, splits, n) : load_parts4((const bf16_t*)p + i, splits, n);
 }
 template <bool VEC>
 __global__ __launch_bounds__(256) void stream_add2_kernel(float* __restrict__ h, const void* __restrict__ a, int a_code,
@@ -1211,24 +1195,21 @@ __global__ __launch_bounds__(256) void stream_add2_kernel(float* __restrict__ h,
   if (VEC) {
     for (size_t i4 = (size_t)blockIdx.x * 256 + threadIdx.x; i4 < n / 4; i4 += stride) {
       const size_t i = i4 * 4;
-      float hv[4], av[4];
-      sa2_load4(h, IA_F32, i, hv);
-      sa2_sum4(a, a_code, a_splits, i, n, av);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) hv[e] += av[e];
+      float4 hv = load4(h + i);
+      const float4 av = sa2_sum4(a, a_code, a_splits, i, n);
+      hv.x += av.x; hv.y += av.y; hv.z += av.z; hv.w += av.w;
       if (b) {
-        sa2_sum4(b, b_code, b_splits, i, n, av);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) hv[e] += av[e];
+        const float4 bv = sa2_sum4(b, b_code, b_splits, i, n);
+        hv.x += bv.x; hv.y += bv.y; hv.z += bv.z; hv.w += bv.w;
       }
-      *reinterpret_cast<float4*>(h + i) = make_float4(hv[0], hv[1], hv[2], hv[3]);
+      *reinterpret_cast<float4*>(h + i) = hv;
       if (x) {
         if (x_code == IA_F32) {
-          *reinterpret_cast<float4*>(reinterpret_cast<float*>(x) + i) = make_float4(hv[0], hv[1], hv[2], hv[3]);
+          *reinterpret_cast<float4*>(reinterpret_cast<float*>(x) + i) = hv;
         } else {
           uint2 u;
-          u.x = (uint32_t)float_to_bf16_bits(hv[0]) | ((uint32_t)float_to_bf16_bits(hv[1]) << 16);
-          u.y = (uint32_t)float_to_bf16_bits(hv[2]) | ((uint32_t)float_to_bf16_bits(hv[3]) << 16);
+          u.x = (uint32_t)float_to_bf16_bits(hv.x) | ((uint32_t)float_to_bf16_bits(hv.y) << 16);
+          u.y = (uint32_t)float_to_bf16_bits(hv.z) | ((uint32_t)float_to_bf16_bits(hv.w) << 16);
           *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(x) + i) = u;
         }
       }
