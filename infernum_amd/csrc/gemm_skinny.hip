@@ -8,7 +8,12 @@
 // two stages of X still leave room for two workgroups on a compute unit); every wave reads its own 16 rows of W
 // straight from global memory into registers (each byte of W is used by one wave
 // only, so LDS would gain nothing), one chunk ahead of the matrix cores, with
-// plain 16-byte loads.  Products run on v_mfma_f32_16x16x32_bf16 with W as the A
+// plain 16-byte loads.  What bounds it is how much of W is under way: the rounds are
+// written out in pairs and no load has a condition, for with one the compiler waits for
+// everything in every round (the 1B shape's gate+up product, 16,384 x 2,048 at 1 to 16
+// rows, 18.6 us that way and 14.0 so, 11.1 at the rate of a large read; 10,240 x 8,192 at
+// 1 / 64 rows 37.4 / 50.8 and 34.1 / 41.9; a product that fills the chip several times
+// over gains 1 to 7 %).  Products run on v_mfma_f32_16x16x32_bf16 with W as the A
 // operand and X^T as the B operand.  Lane (r, q) = (lane % 16, lane / 16) holds,
 // for load i of a chunk, the 8 values k = chunk*256 + (4 i + q) * 8 .. +7 of row
 // r: the four lanes of a row read 64 contiguous bytes.  X uses the same k for the
@@ -91,26 +96,28 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16
   constexpr int XPIECES = MT * 16 * (KC / 8);
   constexpr int XPT = XPIECES / (SK_WAVES * 64);
   static_assert(XPIECES % (SK_WAVES * 64) == 0, "pieces of X must divide over the threads");
+  // No load stands under a condition: behind one that some lanes, or some rounds, skip the compiler can no longer count
+  // which loads are still under way and waits for all of them.  Pieces beyond K are read from the last valid place and
+  // cleared: X on its way to LDS, W in front of the products of that chunk.
   uint4 xreg[XPT];
   auto load_x = [&](int c) {
 #pragma unroll
     for (int i = 0; i < XPT; ++i) {
       const int pc = tid + i * SK_WAVES * 64;
       const int row = pc / (KC / 8), kk = (pc % (KC / 8)) * 8;
-      const int k = c * KC + kk;
-      const int m = row < M ? row : M - 1;
-      xreg[i] = (k < K) ? *reinterpret_cast<const uint4*>(X + (size_t)m * K + k) : make_uint4(0u, 0u, 0u, 0u);
+      xreg[i] = *reinterpret_cast<const uint4*>(X + (size_t)min(row, M - 1) * K + min(c * KC + kk, K - 8));
     }
   };
-  auto store_x = [&](int buf) {
+  auto store_x = [&](int buf, int c) {
 #pragma unroll
     for (int i = 0; i < XPT; ++i) {
       const int pc = tid + i * SK_WAVES * 64;
       const int row = pc / (KC / 8), kk = (pc % (KC / 8)) * 8;
-      *reinterpret_cast<uint4*>(&xs[buf][row][kk]) = xreg[i];
+      const bool in = c * KC + kk < K;
+      *reinterpret_cast<uint4*>(&xs[buf][row][kk]) =
+          make_uint4(in ? xreg[i].x : 0u, in ? xreg[i].y : 0u, in ? xreg[i].z : 0u, in ? xreg[i].w : 0u);
     }
   };
-  uint4 wcur[NLD], wnext[NLD];
   auto load_w = [&](int c, uint4 (&dst)[NLD]) {
     if (TILED) {
       // piece c of KC values lies in chunk c / PER_CHUNK of 256; the copy is padded with zeros to whole chunks
@@ -120,10 +127,7 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16
       return;
     }
 #pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-      const int k = c * KC + (i * 4 + q) * 8;
-      dst[i] = (k < K) ? load_stream_16(wrow + k) : make_uint4(0u, 0u, 0u, 0u);
-    }
+    for (int i = 0; i < NLD; ++i) dst[i] = load_stream_16(wrow + min(c * KC + (i * 4 + q) * 8, K - 8));
   };
 
   // Workgroups that walk K in step read rows of W one row's length apart at the same moment, and such addresses
@@ -140,36 +144,52 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16
     const int k = c + rot;
     return k >= c1 ? k - span : k;
   };
-  if (c0 < c1) {
-    load_x(ce(c0));
-    load_w(ce(c0), wcur);
-    store_x(0);
-  }
-  __syncthreads();
-  for (int c = c0; c < c1; ++c) {
+  const bool ragged = !TILED && K % KC != 0;
+  auto products = [&](int c, uint4 (&w)[NLD]) {
     const int buf = (c - c0) & 1;
-    const bool more = c + 1 < c1;
-    if (more) {
-      // X first, W after it: the wait for X at the end of the round then leaves the loads of W in flight
-      load_x(ce(c + 1));
-      load_w(ce(c + 1), wnext);
+    if (ragged && ce(c) == nchunks - 1) {
+#pragma unroll
+      for (int i = 0; i < NLD; ++i)
+        if (ce(c) * KC + (i * 4 + q) * 8 >= K) w[i] = make_uint4(0u, 0u, 0u, 0u);
     }
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
         const uint4 xv = *reinterpret_cast<const uint4*>(&xs[buf][mt * 16 + r][(i * 4 + q) * 8]);
-        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wcur[i]),
+        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[i]),
                                                           __builtin_bit_cast(bf16x8, xv), acc[mt], 0, 0, 0);
       }
     }
-    if (more) {
-      store_x(buf ^ 1);
-#pragma unroll
-      for (int i = 0; i < NLD; ++i) wcur[i] = wnext[i];
-    }
+  };
+  uint4 w0[NLD], w1[NLD];
+  // the products of chunk c with its W in `w`, while W of the next chunk comes into `next` and its X to the other stage
+  auto round = [&](int c, uint4 (&w)[NLD], uint4 (&next)[NLD]) {
+    load_x(ce(c + 1));                                 // X first: the wait for it leaves the loads of W under way
+    load_w(ce(c + 1), next);
+    __builtin_amdgcn_sched_barrier(0);                 // all of them in front of the first wait for this chunk's W
+    products(c, w);
+    store_x((c - c0 + 1) & 1, ce(c + 1));
     __syncthreads();
+  };
+  if (c0 < c1) {
+    load_x(ce(c0));
+    load_w(ce(c0), w0);
+    store_x(0, ce(c0));
+    __syncthreads();
+    int c = c0;
+    for (; c + 2 < c1; c += 2) {                       // two rounds a turn: no register of a load under way is copied
+      round(c, w0, w1);
+      round(c + 1, w1, w0);
+    }
+    if (c + 1 < c1) {
+      round(c, w0, w1);
+      products(c + 1, w1);
+    } else {
+      products(c, w0);
+    }
   }
+  if (GLU) __syncthreads();                            // the halves meet in the memory of the stages
   // lane holds D[i = 4 q + e][j = r]: i counts rows of W in the tile, j rows of X
   const int n = n_base + 4 * q;
   if (GLU) {
@@ -221,10 +241,21 @@ __global__ __launch_bounds__(256) void gemm_skinny_join_kernel(const float* __re
   const int m = (int)(idx / NO), n = (int)(idx - (size_t)m * NO);
   const size_t MN = (size_t)M * N;
   const float* p = part + (size_t)m * N + n;
+  constexpr int PRE = 8;                               // so many parts asked for together, added in the order of their index
   float a = 0.f, b = 0.f;
-  for (int s = 0; s < splits; ++s) {
-    a += p[s * MN];
-    if (EPI == SK_EPI_SWIGLU) b += p[s * MN + NO];
+  for (int s0 = 0; s0 < splits; s0 += PRE) {
+    float pa[PRE], pb[PRE];
+#pragma unroll
+    for (int u = 0; u < PRE; ++u) {
+      const size_t at = (size_t)min(s0 + u, splits - 1) * MN;
+      pa[u] = p[at];
+      if (EPI == SK_EPI_SWIGLU) pb[u] = p[at + NO];
+    }
+#pragma unroll
+    for (int u = 0; u < PRE; ++u) {
+      a = s0 + u < splits ? a + pa[u] : a;
+      if (EPI == SK_EPI_SWIGLU) b = s0 + u < splits ? b + pb[u] : b;
+    }
   }
   store_out<TO>(C + idx, EPI == SK_EPI_SWIGLU ? a / (1.0f + expf(-a)) * b : a);
 }
@@ -235,9 +266,8 @@ __global__ __launch_bounds__(256) void gemm_skinny_join_kernel(const float* __re
 // from the same start; the parts meet in LDS and are added in the order of their index.  A wave reads its rows of W and
 // of X straight into registers, a chunk of 256 values in flight at a time.  X comes from the caches once per 16 rows of
 // W instead of once per 64, which is what the rule in whole_k_pays weighs against the join's launch.
-#define SK_MOST_WAVES 16
 
-template <bool GLU, int WAVES, typename TO>
+template <bool GLU, int WAVES, typename TO>            // WAVES: room for so many, GLU ? 2 * splits : splits are launched
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_whole_kernel(const uint16_t* __restrict__ X,
                                                                        const uint16_t* __restrict__ W,
                                                                        TO* __restrict__ C, int M, int N, int K,
@@ -259,11 +289,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_whole_kernel(const uin
   for (int c = 0; c < span; ++c) {
     uint4 w[NLD], x[NLD];
 #pragma unroll
-    for (int j = 0; j < NLD; ++j) {
-      const int k = at * SK_KC + 32 * j;
-      const bool in = k + 8 * q < K;
-      w[j] = in ? load_stream_16(wrow + k) : make_uint4(0u, 0u, 0u, 0u);
-      x[j] = in ? *reinterpret_cast<const uint4*>(xrow + k) : make_uint4(0u, 0u, 0u, 0u);
+    for (int j = 0; j < NLD; ++j) {                    // beyond K the last valid piece is read, and cleared below
+      const int k = min(at * SK_KC + 32 * j + 8 * q, K - 8) - 8 * q;
+      w[j] = load_stream_16(wrow + k);
+      x[j] = *reinterpret_cast<const uint4*>(xrow + k);
+    }
+    if (K % SK_KC != 0 && at == nchunks - 1) {
+#pragma unroll
+      for (int j = 0; j < NLD; ++j)
+        if (at * SK_KC + 32 * j + 8 * q >= K) w[j] = x[j] = make_uint4(0u, 0u, 0u, 0u);
     }
     if (++at == c1) at = c0;
 #pragma unroll
@@ -287,21 +321,22 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_whole_kernel(const uin
 }
 
 // Whether the kernel above takes a split product whose parts are wanted joined.  Microseconds on an MI355X in a chain of
-// products with cold weights, the split product with its join against this kernel: 2,048 x 2,048 at 1 / 8 / 16 rows 7.9 /
-// 8.6 / 8.9 against 5.3 / 6.1 / 7.1, 4,096 x 4,096 13.0 / 12.7 / 12.8 against 9.8 / 10.5 / 11.9, 8,192 x 2,048 12.7 / 12.6 /
-// 12.8 against 9.4 / 10.1 / 11.6.  It loses where the reads of X weigh more than a launch: 2,048 x 5,504 at 16 rows (13.5
-// against 15.1; 12 rows even), 12,288 x 4,096 and 10,304 x 2,048 at 16 (27.2 against 29.5, 15.2 against 15.9; 8 rows
-// ahead); where the chunks do not deal out evenly over more than four waves, which then wait for the longest
-// (6,144 x 4,096 at 8 rows 15.5 against 15.9); and with few workgroups of many waves (64 x 4,096 at 16 rows 8.2 against
-// 9.5).  With both halves it reads X twice: 5,632 x 2,048 at 8 rows 11.3 against 10.0, 11,008 x 2,048 at 4 rows 15.9
-// against 14.6 and at 8 16.2 against 17.1, 9,472 x 4,096 behind at every number of rows.
+// products with cold weights, the split product with its join against this kernel: 2,048 x 2,048 at 1 / 8 / 16 rows 6.2 /
+// 6.4 / 6.7 against 5.4 / 6.1 / 6.9, 3,072 x 2,048 7.3 / 7.4 / 7.9 against 5.7 / 6.3 / 7.2, 4,096 x 4,096 at 1 / 8 / 12 rows
+// 10.6 / 10.4 / 10.6 against 9.2 / 10.0 / 10.6, 12,288 x 4,096 24.1 / 24.7 / 25.3 against 21.3 / 23.2 / 25.4.  It loses where
+// the reads of X weigh more than a launch: 10,304 x 2,048 at 12 rows (13.1 against 13.8; at 8 12.8 and 12.7), 4,096 x 8,192
+// (15.9 against 17.0; at 8 16.0 and 15.6); where the chunks do not deal out evenly over more than four waves, which
+// then wait for the longest (6,144 x 4,096 at 1 row 14.0 against 14.5); with more than eight waves (2,048 x 4,096 at 4 rows
+// 8.0 against 8.6); and with few workgroups (256 x 2,048 at 8 rows 5.1 against 5.4).  With both halves it reads X twice:
+// 5,632 x 2,048 at 8 / 12 rows 9.8 / 10.0 against 9.7 / 10.3, 11,008 x 2,048 at 2 / 8 rows 14.4 / 14.4 against 13.7 / 15.9,
+// 9,472 x 4,096 behind at every number of rows.
 static bool whole_k_pays(int M, int N, int K, int splits, bool glu) {
-  if (M > 16 || (glu ? 2 : 1) * splits > SK_MOST_WAVES) return false;
+  if (M > 16 || splits > 8) return false;
   const int nchunks = (K + SK_KC - 1) / SK_KC;
-  if (glu) return N % 32 == 0 && K <= 2048 && (long)M * N <= 65536;
-  if (splits > 4 && nchunks % splits != 0) return false;
-  if (N < 256 && splits > 8 && M > 4) return false;
-  return (long)M * K <= 65536 && (long)M * N <= 131072;
+  if (glu) return N % 32 == 0 && K <= 2048 && (long)M * N <= 45056;
+  if (N < 512 || (splits > 4 && nchunks % splits != 0)) return false;
+  if (M > 8 && ((long)M * K > 32768 || (K > 1024 && N < 2560))) return false;
+  return (long)M * K <= 65536 && (long)M * N <= 98304;
 }
 
 // Shapes whose number of splits was measured (ia_gemm_skinny_set_splits, filled from a table when the library is
@@ -368,9 +403,19 @@ static int launch_skinny(const uint16_t* x, const uint16_t* w, TO* c, float* par
   const int NO = GLU ? N / 2 : N;
   const int cols = GLU ? SK_BN / 2 : SK_BN;           // columns of the result per workgroup
   dim3 grid((NO + cols - 1) / cols, splits);
+  // Up to 32 rows and with more than one workgroup a compute unit, pieces of 128: less of W under way in each and the first
+  // products sooner (2,048 x 8,192 in 16 parts at 16 / 32 rows 8.4 / 9.4 us with pieces of 256 and 7.9 / 8.7 with 128, the
+  // 8B shape's gate+up from its copy 43.9 / 49.0 and 42.4 / 45.1).  One workgroup a compute unit wants the longer pieces
+  // (the 1B shape's gate+up 14.5 against 15.4), and so do heads of many workgroups (128,256 x 2,048 91.5 against 92.8).
+  const unsigned groups = grid.x * grid.y;
+  const bool shorter = grid.y > 1 || (groups > SK_ENOUGH_BLOCKS && groups <= 4 * SK_ENOUGH_BLOCKS);
   switch ((M + 15) / 16) {
-    case 1: return launch_skinny_one<1, GLU, TO, SK_KC, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
-    case 2: return launch_skinny_one<2, GLU, TO, SK_KC, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
+    case 1:
+      if (shorter) return launch_skinny_one<1, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
+      return launch_skinny_one<1, GLU, TO, SK_KC, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
+    case 2:
+      if (shorter) return launch_skinny_one<2, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
+      return launch_skinny_one<2, GLU, TO, SK_KC, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
     case 3: return launch_skinny_one<3, GLU, TO, SK_KC, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
     case 4: return launch_skinny_one<4, GLU, TO, SK_KC, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
     // above 64 rows: pieces of 128, so that the two stages of X of two workgroups fit a compute unit's LDS
@@ -424,16 +469,16 @@ static int skinny_product(const void* X, const void* W, void* C, int out_dtype, 
   if (!TILED && C != nullptr && splits > 1 && whole_k_pays(M, N, K, splits, glu)) {
     const int nchunks = (K + SK_KC - 1) / SK_KC, cps = (nchunks + splits - 1) / splits, NO = glu ? N / 2 : N;
     const dim3 grid((NO + 15) / 16), block((glu ? 2 : 1) * splits * 64);
-#define SK_WHOLE(G, T)                                                                                              \
-  do {                                                                                                              \
-    if (block.x <= 512) gemm_skinny_whole_kernel<G, 8, T><<<grid, block, 0, stream>>>(x, w, (T*)C, M, N, K, cps, splits); \
-    else gemm_skinny_whole_kernel<G, 16, T><<<grid, block, 0, stream>>>(x, w, (T*)C, M, N, K, cps, splits);          \
+#define SK_WHOLE(G, WAVES)                                                                                            \
+  do {                                                                                                                \
+    if (out_dtype == IA_F32)                                                                                          \
+      gemm_skinny_whole_kernel<G, WAVES, float><<<grid, block, 0, stream>>>(x, w, (float*)C, M, N, K, cps, splits);   \
+    else                                                                                                              \
+      gemm_skinny_whole_kernel<G, WAVES, uint16_t><<<grid, block, 0, stream>>>(x, w, (uint16_t*)C, M, N, K, cps, splits); \
   } while (0)
-    if (glu) {
-      if (out_dtype == IA_F32) SK_WHOLE(true, float); else SK_WHOLE(true, uint16_t);
-    } else {
-      if (out_dtype == IA_F32) SK_WHOLE(false, float); else SK_WHOLE(false, uint16_t);
-    }
+    if (!glu) SK_WHOLE(false, 8);
+    else if (splits <= 4) SK_WHOLE(true, 8);
+    else SK_WHOLE(true, 16);
 #undef SK_WHOLE
     IA_LAUNCH_CHECK();
     return IA_OK;

@@ -370,10 +370,22 @@ def test_gemm_skinny_partial_sums_and_swiglu(M, N, K_):
     assert torch.equal(actb, act.bfloat16())
 
 
+# one, two, three and more chunks of K, a last one that is not full, and both lengths of the pieces (one part of more than
+# 256 workgroups, and several parts); fp32 sums of K exact products: within K * 2^-24 of the sum of their sizes
+@pytest.mark.parametrize("M", [1, 17, 33])
+@pytest.mark.parametrize("N,K_", [(16500, 8), (16500, 136), (16500, 264), (16400, 776), (16385, 1288), (300, 1800), (130, 9000)])
+def test_gemm_skinny_rounds_in_pairs(M, N, K_):
+    api = K()
+    a, w = _rand(M, K_, dtype=torch.bfloat16, seed=21), _rand(N, K_, dtype=torch.bfloat16, seed=22)
+    got = api.gemm_skinny(a, w, out_dtype=torch.float32).double()
+    want, size = a.double() @ w.double().t(), a.double().abs() @ w.double().abs().t()
+    assert ((got - want).abs() <= K_ * 2 ** -24 * size + 1e-30).all()
+
+
 # one workgroup with all of K against the parts and their sum in the order of their index: columns that fill no group of
 # 16, a last chunk that is not full, one to sixteen parts, two chunks and more a part, both halves of [gate | up]
 @pytest.mark.parametrize("M", [1, 5, 16])
-@pytest.mark.parametrize("N,K_,glu", [(250, 520, False), (2049, 776, False), (2048, 4096, False), (200, 5504, False),
+@pytest.mark.parametrize("N,K_,glu", [(650, 520, False), (2049, 776, False), (2048, 4096, False), (200, 5504, False),
                                       (7000, 2040, False), (5632, 2048, True), (64, 1000, True), (96, 264, True)])
 def test_gemm_skinny_with_all_parts_in_one_workgroup_leaves_the_joined_parts_bits(M, N, K_, glu):
     api = K()
