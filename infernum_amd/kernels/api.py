@@ -870,11 +870,16 @@ def decode_splits(batch: int, nh: int, nkv: int, max_len: int, device: Optional[
       against 15.3 in three parts, 32 requests 15.4 against 17.1 in two); at head sizes up to 64 a tile is half the
       bytes and twice as many workgroups are wanted (8 requests with 32,768 keys each: 97 us in eight parts, 138
       in four; 32 requests: 364 in two, 520 whole);
+    * no parts up to 256 keys: eight waves take them in two turns, and the join's launch costs what the parts give (8 key/value
+      heads, one request, whole against two parts: 150 keys of 64 values 7.5 us and 8.8, of 128 values 8.9 and 10.0; 250
+      keys 8.0 and 8.7, 9.8 and 10.2; from 320 keys of 128 values on four parts are 1 us faster);
     * above 128 a compute unit holds one workgroup, and more parts than compute units only cost (head size 256, 32
       requests on 4 key/value heads: 19 us in two parts, 23 in four);
     * the join grows with the parts as the work of a part shrinks with them: the best number of parts for one
       request went with the square root of its tiles (4 parts at 512 keys, 8 at 2,048, 16 at 8,192, 32 at 32,768, for
       head sizes 64, 128 and 256 alike), so that bounds the parts; never more than 64."""
+    if head_dim <= 128 and max_len <= 256:
+        return 1
     cus = compute_units(device)
     fill = cus * (2 if head_dim <= 64 else 1)
     groups = batch * nkv * ((nh // nkv + 15) // 16)
