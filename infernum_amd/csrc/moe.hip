@@ -624,15 +624,15 @@ extern "C" int ia_moe_up(const void* x, const void* Wu, void* y, const int* offs
 //   order of the pairs.
 // Bound by reading the chosen experts' weights once, and with one or two tokens by how many loads are in flight for it.  A
 // workgroup of four waves takes 64 / KS rows of one expert's matrix and finds the expert's pairs among the step's ids
-// itself (one load: at most 64 of them); a wave streams 16 rows over its part of K (all of it, a half or a quarter)
+// itself (one load: at most 32 of them); a wave streams 16 rows over its part of K (all of it, a half or a quarter)
 // straight into registers, two stretches of 256 values in flight, with the pairs' rows of x from the caches beside them.
 // It starts at a stretch of its own and wraps (rows of a power of two would crowd on few memory channels).  The parts'
 // sums meet in LDS and are added in their order.
 // Microseconds for gate, up and down with the tiles and the sort against this, cold weights: 1 token to 4 of 32 experts of
 // 1,408 x 2,048 37.4 against 19.2 (46 MB: 2.4 TB/s, two launches); 2 tokens to 2 of 8 (2,752, no gate) 47 against 28; 1
-// token to 2 of 20 (2,432 x 4,096) 57 against 29, 16 tokens 201 against 180 (5.3 TB/s); 32 tokens to 2 of 16 67.5 against
-// 65.4.  Sixteen pairs a pass of the weights: with more than some tens of pairs the tiles of 32 read them less often.
-#define MOE_FEW_PAIRS 64
+// token to 2 of 20 (2,432 x 4,096) 57 against 29, 16 tokens 201 against 180 (5.3 TB/s).  From 64 pairs on
+// the two are even (32 tokens to 2 of 16 67.5 against 65.4): sixteen pairs a pass of the weights, where the tiles take 32.
+#define MOE_FEW_PAIRS 32
 #define MOE_FEW_WAVES 2048       // waves in the launch that are enough; fewer: K is split over two or four of a workgroup
 
 enum { MOE_GATE_UP = 0, MOE_UP = 1, MOE_DOWN = 2 };

@@ -1379,10 +1379,10 @@ def test_copy_pages(dtype):
 
 
 # ---------------------------------------------------------------- routed experts, few pairs
-# one pair, 17 (a second pass over an expert's pairs), 64 (the most); fewer pairs than experts and more; rows that fill no
+# one pair, 17 (a second pass over an expert's pairs), 32 (the most); fewer pairs than experts and more; rows that fill no
 # group of 16, K that fills no stretch of 256 or part of a quarter; ids without an expert; the weight on either side
 @pytest.mark.parametrize("gated,weights_on", [(True, "output"), (True, "input"), (False, "output")])
-@pytest.mark.parametrize("N,top,E,W,ff", [(1, 1, 3, 264, 40), (17, 1, 2, 520, 328), (32, 2, 6, 136, 1000), (1, 4, 40, 2048, 1408),
+@pytest.mark.parametrize("N,top,E,W,ff", [(1, 1, 3, 264, 40), (17, 1, 2, 520, 328), (16, 2, 6, 136, 1000), (1, 4, 40, 2048, 1408),
                                           (5, 3, 300, 72, 2056)])
 def test_routed_experts_of_few_pairs(gated, weights_on, N, top, E, W, ff):
     api = K()
