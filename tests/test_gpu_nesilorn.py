@@ -173,6 +173,32 @@ def _run_mixer(mixer, steps, x, cuts, rt):
     return torch.cat(out)
 
 
+# one row to the most that few rows are, and one more; columns that fill no group of 16 or 64, K of one piece, of part of a
+# step of 32 and of more than eight steps.  fp32 sums of exact products (K 2^-24 of the sum of their sizes) rounded to
+# bfloat16 (eight significant bits: half a unit is 2^-8 of the value at the most), and with a gate once more, the
+# sigmoid's few fp32 roundings far below
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("N", [1, 16, 17])
+@pytest.mark.parametrize("H,J,Kd", [(3, 37, 8), (2, 64, 72), (4, 130, 264), (1, 16, 520)])
+def test_products_head_by_head_of_few_rows(N, H, J, Kd, gated):
+    from infernum_amd.kernels import api as K
+    g = torch.Generator().manual_seed(N + J)
+    x, w = torch.randn(N, H * Kd + 8, generator=g).bfloat16().cuda(), torch.randn(H, J, Kd, generator=g).bfloat16().cuda()
+    gate = torch.randn(N, H * J + 3, generator=g).bfloat16().cuda() if gated else None
+    out = torch.full((N, H * J + 5), 7.0, dtype=torch.bfloat16, device="cuda")
+    K.gemm_heads(x, 8, Kd, w, out, 2, J, gate, 3)
+    xs, ws = x[:, 8:].double().view(N, H, Kd).cpu(), w.double().cpu()
+    want = (xs[:, :, None, :] * ws[None]).sum(-1).view(N, H * J)
+    size = (xs[:, :, None, :] * ws[None]).abs().sum(-1).view(N, H * J)
+    bound = 2.0 ** -8 * want.abs() + Kd * 2.0 ** -24 * size
+    if gated:
+        s = torch.sigmoid(gate[:, 3:].double().cpu())
+        want, bound = want * s, (bound + 2.0 ** -8 * want.abs()) * s * 1.01
+    got = out[:, 2:2 + H * J].double().cpu()
+    assert ((got - want).abs() <= bound + 1e-30).all()
+    assert (out[:, :2] == 7.0).all() and (out[:, 2 + H * J:] == 7.0).all()
+
+
 @BOTH
 @pytest.mark.parametrize("m,W,T", [
     (NM._mixer(3, 16, 8, 24, 24, 20), 64, 75),                       # head size 32, window inside the prompt

@@ -315,8 +315,8 @@ def test_sinks_in_the_matrix_core_kernels_against_the_plain_kernel(nh, nkv, d, p
 @pytest.mark.parametrize("nh,nkv,d,dv,ps,window,pool", [(4, 2, 16, 32, 4, 20, 6), (17, 1, 64, 64, 16, 1, 1), (3, 3, 48, 16, 12, 0, 0)])
 def test_window_and_blocks_in_parts(nh, nkv, d, dv, ps, window, pool, parts):
     """Single tokens whose keys are cut into parts (also more parts than there are tiles) against the same kernel whole.
-    The weights of either are rounded to bfloat16 against maxima of their own, 2^-9 of a weight each, and so is the result:
-    the two differ by at most 2 * 2^-9 of the weighted mean of |v| and one rounding each of the result, at most 2^-7 max |v|."""
+    The weights of either are rounded to bfloat16 against maxima of their own, 2^-8 of a weight at the most, and so is the
+    result: the two differ by at most 2 * 2^-8 of the weighted mean of |v| and as much for the results, 2^-6 max |v|."""
     from infernum_amd.kernels import api as K
     g = torch.Generator().manual_seed(11)
     lens = [1, 16, 17, 333]
@@ -333,7 +333,7 @@ def test_window_and_blocks_in_parts(nh, nkv, d, dv, ps, window, pool, parts):
     for s in (None, sinks):
         K.wpa_decode(q, kp, vp, pk, pv, whole, s, pos, bt, bt, nh, nkv, scale, window, pool, num_parts=1)
         K.wpa_decode(q, kp, vp, pk, pv, cut, s, pos, bt, bt, nh, nkv, scale, window, pool, num_parts=parts)
-        assert (whole.float() - cut.float()).abs().max() <= 2 ** -7 * max(vp.abs().max(), pv.abs().max()).float()
+        assert (whole.float() - cut.float()).abs().max() <= 2 ** -6 * max(vp.abs().max(), pv.abs().max()).float()
 
 
 @pytest.mark.parametrize("nh,nkv,d,dv,ps,window,pool", [(4, 2, 16, 32, 4, 20, 6), (6, 2, 64, 64, 16, 40, 10), (20, 1, 32, 16, 8, 1, 1),
