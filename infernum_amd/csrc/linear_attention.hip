@@ -24,6 +24,7 @@
 #define GLA_PARTS 16     // the key channels are dealt out over so many groups of threads
 #define GLA_TB 8         // tokens whose rows are staged together
 #define GLA_TILE 64      // rows of a tile of ia_gla_chunked
+#define GLA_PAIRS_FROM 512 // workgroups that are left with two slices each
 
 __host__ __device__ inline int gla_slices(int vdim) { return (vdim + GLA_PW - 1) / GLA_PW; }
 
@@ -31,6 +32,13 @@ __device__ __forceinline__ float gla_log_sigmoid(float z) {
   // log(1 / (1 + exp(-z))): never above zero, no overflow on either side
   return z >= 0.f ? -log1pf(expf(-z)) : z - log1pf(expf(z));
 }
+
+// A value as it lies in memory, and back: what waits in registers is not converted before it is used.
+__device__ __forceinline__ uint32_t gla_bits(float x) { return __float_as_uint(x); }
+__device__ __forceinline__ uint32_t gla_bits(bf16_t x) { return x.bits; }
+template <typename T> __device__ __forceinline__ float gla_value(uint32_t b);
+template <> __device__ __forceinline__ float gla_value<float>(uint32_t b) { return __uint_as_float(b); }
+template <> __device__ __forceinline__ float gla_value<bf16_t>(uint32_t b) { return bf16_bits_to_float((uint16_t)b); }
 
 // The record of the tile that begins at row r0 of request s: the tiles of the requests from ``first_request`` on,
 // counted in the order of the requests and their rows, whatever the order of the list of tiles.
@@ -40,11 +48,14 @@ __device__ __forceinline__ int gla_record(const int* __restrict__ seq_starts, in
   return before + r0 / GLA_TILE;
 }
 
-// grid (heads, requests or tiles, slices), 256 threads: thread (part, p) keeps S[n][p] for n = part, part + 16, ...
-// in registers.  MODE 0: a request's rows from its slot, which is left moved on.  MODE 1: a tile (not a request's
+// grid (heads, requests or tiles, slices / SL), 256 threads: thread (part, p) keeps S[n][p] of SL slices for KMAX channels n
+// of its part in registers.  The tiles are bound by the reads of q, k and the decays, from LDS (16 bytes for four channels of
+// a thread) and from memory into it (once for every workgroup of a head): two slices a workgroup halve both, where the slices
+// are even in number (3,000 rows of 16 heads of 128: 476 us for the whole chain with one slice and every block of rows waited
+// for, 397 with the next block's rows asked for ahead, 299 with two slices).  MODE 0: a request's rows from its slot, which is left moved on.  MODE 1: a tile (not a request's
 // last) from a zero state; no rows are written, the state goes to the tile's record and the product of the decays
 // to ``decay``.  MODE 2: a tile from its record; a request's last tile leaves the state in the slot.
-template <typename T, int KMAX, int MODE>
+template <typename T, int KMAX, int MODE, int SL>
 __global__ __launch_bounds__(256) void gla_scan_kernel(
     const T* __restrict__ proj, int proj_stride, int q_col, int k_col, int v_col, const float* __restrict__ z,
     int z_stride, const float* __restrict__ z_bias, float inv_tau, float q_scale, float* __restrict__ state,
@@ -55,9 +66,9 @@ __global__ __launch_bounds__(256) void gla_scan_kernel(
   float* qs = lds;                                   // [TB][dim]
   float* ks = qs + GLA_TB * dim;                     // [TB][dim]
   float* as = ks + GLA_TB * dim;                     // [TB][dim]  alpha
-  float* vs = as + GLA_TB * dim;                     // [TB][PW]
-  float* ysum = vs + GLA_TB * GLA_PW;                // [TB][PARTS][PW]
-  const int hd = blockIdx.x, slice = blockIdx.z;
+  float* vs = as + GLA_TB * dim;                     // [TB][SL * PW]
+  float* ysum = vs + GLA_TB * SL * GLA_PW;           // [TB][PARTS][SL * PW]
+  const int hd = blockIdx.x, slice = blockIdx.z * SL;
   const int s = MODE == 0 ? blockIdx.y : tiles[2 * blockIdx.y];
   int first = seq_starts[s], count = seq_starts[s + 1] - first;
   bool last = true;
@@ -74,47 +85,87 @@ __global__ __launch_bounds__(256) void gla_scan_kernel(
   const int tid = threadIdx.x;
   const bool vec = (dim & 3) == 0;
   const int p = tid % GLA_PW, part = tid / GLA_PW;
-  const int col = slice * GLA_PW + p;
   const int slices = gla_slices(vdim);
   const size_t within = ((size_t)hd * slices + slice) * dim * GLA_PW;
   float* S = state + (size_t)state_slots[s] * state_stride + within;
   float* R = MODE == 0 ? S : records + (size_t)record * record_stride + within;
+  constexpr int CW = SL * GLA_PW;                                    // value columns of the workgroup
+  const int v_t = tid / CW, v_c = slice * GLA_PW + tid % CW;
+  // Tiles: the next block's rows are asked for before this one is worked on and wait in registers: a thread has the same places of
+  // a block every time, none of its loads a condition (places beyond the rows are read from the last and not kept).
+  constexpr int PLACES = GLA_TB * GLA_PARTS * KMAX / 256;            // of q, k and the decays
+  static_assert(GLA_TB * CW <= 256, "a thread has at most one place of v");
+  int place_t[PLACES], place_n[PLACES];
+#pragma unroll
+  for (int l = 0; l < PLACES; ++l) {
+    place_t[l] = (tid + 256 * l) / dim;
+    place_n[l] = tid + 256 * l - place_t[l] * dim;
+  }
+  T q_next[MODE == 1 ? 1 : PLACES], v_next;
+  uint32_t k_next[PLACES];                                           // form 1: fp32 from z_bias, else T's bits
+  float z_next[PLACES];
+  auto ask = [&](int t0) {
+    // the block's first row is the same for all threads; a thread's place is a short way from it
+    const T* pr = proj + (size_t)(first + t0) * proj_stride;
+    const float* zr = z + (size_t)(first + t0) * z_stride + hd * dim;
+    const int last_t = count - 1 - t0;
+#pragma unroll
+    for (int l = 0; l < PLACES; ++l) {
+      const int t = min(place_t[l], last_t);
+      if (MODE != 1) q_next[l] = pr[(unsigned)(t * proj_stride + q_col + hd * dim + place_n[l])];
+      z_next[l] = zr[(unsigned)(t * z_stride + place_n[l])];
+    }
+    if (form == 1) {
+      const float* kr = z_bias + (size_t)(first + t0) * z_stride + hd * dim;
+#pragma unroll
+      for (int l = 0; l < PLACES; ++l) k_next[l] = __float_as_uint(kr[(unsigned)(min(place_t[l], last_t) * z_stride + place_n[l])]);
+    } else {
+#pragma unroll
+      for (int l = 0; l < PLACES; ++l)
+        k_next[l] = gla_bits(pr[(unsigned)(min(place_t[l], last_t) * proj_stride + k_col + hd * dim + place_n[l])]);
+    }
+    v_next = pr[(unsigned)(min(v_t, last_t) * proj_stride + v_col + hd * vdim + min(v_c, vdim - 1))];
+  };
+  if (MODE != 0) ask(0);
   float dprod[MODE == 1 ? KMAX : 1];
-  float reg[KMAX];
+  float reg[SL][KMAX];
 #pragma unroll
   for (int c = 0; c < KMAX; ++c) {
     const int n = part * KMAX + c;
-    reg[c] = (MODE != 1 && n < dim) ? R[(size_t)n * GLA_PW + p] : 0.f;
+#pragma unroll
+    for (int u = 0; u < SL; ++u) reg[u][c] = (MODE != 1 && n < dim) ? R[(size_t)(u * dim + n) * GLA_PW + p] : 0.f;
     if constexpr (MODE == 1) dprod[c] = 1.f;
   }
   for (int t0 = 0; t0 < count; t0 += GLA_TB) {
     const int nt = count - t0 < GLA_TB ? count - t0 : GLA_TB;
+    if (MODE == 0) ask(t0);
     __syncthreads();                                  // the block before is read to its end
-    for (int i = tid; i < nt * dim; i += 256) {
-      const int t = i / dim, n = i - t * dim;
-      const size_t row = (size_t)(first + t0 + t);
-      const T* pr = proj + row * proj_stride;
-      qs[i] = to_float(pr[q_col + hd * dim + n]) * q_scale;
-      const float zz = z[row * z_stride + hd * dim + n];
+#pragma unroll
+    for (int l = 0; l < PLACES; ++l) {
+      const int i = tid + 256 * l;
+      if (i >= nt * dim) continue;
+      if (MODE != 1) qs[i] = to_float(q_next[l]) * q_scale;
       // the tiles read decays that one kernel made of the logits before them; the walk over a request makes its own.
       // form 1: z holds the decays themselves, and z_bias is no bias but the rows of fp32 keys that go with them
       // (what a channel takes in, 1 - decay, made where the decay was made and not as the difference of a number
       // near one), laid out like z
-      const float a = (MODE != 0 || form == 1) ? zz : expf(gla_log_sigmoid(zz + (z_bias ? z_bias[hd * dim + n] : 0.f)) * inv_tau);
-      as[i] = a;
-      ks[i] = form == 1 ? z_bias[row * z_stride + hd * dim + n] : to_float(pr[k_col + hd * dim + n]);
+      as[i] = (MODE != 0 || form == 1) ? z_next[l]
+                                       : expf(gla_log_sigmoid(z_next[l] + (z_bias ? z_bias[hd * dim + place_n[l]] : 0.f)) * inv_tau);
+      ks[i] = form == 1 ? __uint_as_float(k_next[l]) : gla_value<T>(k_next[l]);
     }
-    for (int i = tid; i < nt * GLA_PW; i += 256) {
-      const int t = i / GLA_PW, c = slice * GLA_PW + (i - t * GLA_PW);
-      vs[i] = c < vdim ? to_float(proj[(size_t)(first + t0 + t) * proj_stride + v_col + hd * vdim + c]) : 0.f;
-    }
+    if (tid < nt * CW) vs[tid] = v_c < vdim ? to_float(v_next) : 0.f;
+    if (MODE != 0 && t0 + GLA_TB < count) ask(t0 + GLA_TB);
     __syncthreads();
     for (int t = 0; t < nt; ++t) {
-      const float v = vs[t * GLA_PW + p];
+      float v[SL], acc[SL];
+#pragma unroll
+      for (int u = 0; u < SL; ++u) {
+        v[u] = vs[t * CW + u * GLA_PW + p];
+        acc[u] = 0.f;
+      }
       const float* qt = qs + t * dim;
       const float* kt = ks + t * dim;
       const float* at = as + t * dim;
-      float acc = 0.f;
 #pragma unroll
       for (int c4 = 0; c4 < KMAX; c4 += 4) {          // a thread's channels lie side by side: 16 bytes a read
         const int n0 = part * KMAX + c4;
@@ -141,22 +192,26 @@ __global__ __launch_bounds__(256) void gla_scan_kernel(
 #pragma unroll
         for (int e = 0; e < 4; ++e) {                  // channels past the head's last stay zero: 0 * 0 + 0 * v
           const int c = c4 + e;
-          reg[c] = __builtin_fmaf(a4[e], reg[c], k4[e] * v);
+#pragma unroll
+          for (int u = 0; u < SL; ++u) {
+            reg[u][c] = __builtin_fmaf(a4[e], reg[u][c], k4[e] * v[u]);
+            if constexpr (MODE != 1) acc[u] = __builtin_fmaf(reg[u][c], q4[e], acc[u]);
+          }
           if constexpr (MODE == 1) dprod[c] *= a4[e];
-          else acc = __builtin_fmaf(reg[c], q4[e], acc);
         }
       }
-      if (MODE != 1) ysum[(t * GLA_PARTS + part) * GLA_PW + p] = acc;
+#pragma unroll
+      for (int u = 0; u < SL; ++u)
+        if (MODE != 1) ysum[(t * GLA_PARTS + part) * CW + u * GLA_PW + p] = acc[u];
     }
     if (MODE == 1) continue;
     __syncthreads();
-    for (int i = tid; i < nt * GLA_PW; i += 256) {
-      const int t = i / GLA_PW, pp = i - t * GLA_PW;
-      const int c = slice * GLA_PW + pp;
-      float y = ysum[(t * GLA_PARTS) * GLA_PW + pp];
+    if (tid < nt * CW) {
+      const int pp = tid % CW;
+      float y = ysum[(v_t * GLA_PARTS) * CW + pp];
 #pragma unroll
-      for (int k = 1; k < GLA_PARTS; ++k) y += ysum[(t * GLA_PARTS + k) * GLA_PW + pp];
-      if (c < vdim) out[(size_t)(first + t0 + t) * ((size_t)nh * vdim) + (size_t)hd * vdim + c] = y;
+      for (int k = 1; k < GLA_PARTS; ++k) y += ysum[(v_t * GLA_PARTS + k) * CW + pp];
+      if (v_c < vdim) out[(size_t)(first + t0 + v_t) * ((size_t)nh * vdim) + (size_t)hd * vdim + v_c] = y;
     }
   }
   if (MODE == 2 && !last) return;
@@ -165,7 +220,8 @@ __global__ __launch_bounds__(256) void gla_scan_kernel(
   for (int c = 0; c < KMAX; ++c) {
     const int n = part * KMAX + c;
     if (n < dim) {
-      W[(size_t)n * GLA_PW + p] = reg[c];
+#pragma unroll
+      for (int u = 0; u < SL; ++u) W[(size_t)(u * dim + n) * GLA_PW + p] = reg[u][c];
       if constexpr (MODE == 1) if (p == 0 && slice == 0) decay[((size_t)record * nh + hd) * dim + n] = dprod[c];
     }
   }
@@ -233,7 +289,7 @@ static int gla_scan_launch(const void* proj, int code, int proj_stride, int q_co
   const size_t lds = sizeof(float) * ((size_t)3 * GLA_TB * dim + GLA_TB * GLA_PW + (size_t)GLA_TB * GLA_PARTS * GLA_PW);
   if (lds > 64 * 1024) return IA_ERR_UNSUPPORTED;
 #define IA_GLA(T, KM)                                                                                                  \
-  gla_scan_kernel<T, KM, 0><<<grid, 256, lds, stream>>>((const T*)proj, proj_stride, q_col, k_col, v_col, z, z_stride, \
+  gla_scan_kernel<T, KM, 0, 1><<<grid, 256, lds, stream>>>((const T*)proj, proj_stride, q_col, k_col, v_col, z, z_stride, \
                                                         z_bias, 1.0f / tau, q_scale, state, state_stride, out,         \
                                                         seq_starts, state_slots, nh, dim, vdim, nullptr, 0, nullptr,   \
                                                         0, nullptr, form)
@@ -305,19 +361,29 @@ static int gla_chunked_launch(const void* proj, int code, int proj_stride, int q
   const int per = (dim + GLA_PARTS - 1) / GLA_PARTS;
   const int slices = gla_slices(vdim);
   if (per > 32 || num_tiles > 65535 || slices > 65535) return IA_ERR_UNSUPPORTED;
-  const dim3 grid((unsigned)nh, (unsigned)num_tiles, (unsigned)slices);
-  const size_t lds = sizeof(float) * ((size_t)3 * GLA_TB * dim + GLA_TB * GLA_PW + (size_t)GLA_TB * GLA_PARTS * GLA_PW);
-  if (lds > 64 * 1024) return IA_ERR_UNSUPPORTED;
-#define IA_GLA(T, KM, MODE)                                                                                        \
-  gla_scan_kernel<T, KM, MODE><<<grid, 256, lds, stream>>>(                                                        \
+  const auto lds_of = [&](int sl) {
+    return sizeof(float) * ((size_t)3 * GLA_TB * dim + (size_t)GLA_TB * sl * GLA_PW + (size_t)GLA_TB * GLA_PARTS * sl * GLA_PW);
+  };
+  if (lds_of(1) > 64 * 1024) return IA_ERR_UNSUPPORTED;
+  // two slices a workgroup while that leaves two workgroups a compute unit (even at 400 rows of 16 heads of 128, 448
+  // workgroups of one slice: 85 us with one), and up to 16 channels a thread (two states of more
+  // leave room for one wave on a SIMD)
+  const bool pairs = slices % 2 == 0 && per <= 16 && (long)nh * num_tiles * (slices / 2) >= GLA_PAIRS_FROM;
+  const dim3 grid((unsigned)nh, (unsigned)num_tiles, (unsigned)(pairs ? slices / 2 : slices));
+  const size_t lds = lds_of(pairs ? 2 : 1);
+#define IA_GLA(T, KM, MODE, SL)                                                                                    \
+  gla_scan_kernel<T, KM, MODE, SL><<<grid, 256, lds, stream>>>(                                                    \
       (const T*)proj, proj_stride, q_col, k_col, v_col, z, z_stride, z_bias, 1.0f / tau, q_scale, state,           \
       state_stride, out, seq_starts, state_slots, nh, dim, vdim, tiles, first_request, records, record_stride, decay, form)
-#define IA_GLA_K(T, MODE)                       \
-  do {                                          \
-    if (per <= 4) IA_GLA(T, 4, MODE);           \
-    else if (per <= 8) IA_GLA(T, 8, MODE);      \
-    else if (per <= 16) IA_GLA(T, 16, MODE);    \
-    else IA_GLA(T, 32, MODE);                   \
+#define IA_GLA_K(T, MODE)                                              \
+  do {                                                                 \
+    if (per <= 4 && pairs) IA_GLA(T, 4, MODE, 2);                      \
+    else if (per <= 4) IA_GLA(T, 4, MODE, 1);                          \
+    else if (per <= 8 && pairs) IA_GLA(T, 8, MODE, 2);                 \
+    else if (per <= 8) IA_GLA(T, 8, MODE, 1);                          \
+    else if (per <= 16 && pairs) IA_GLA(T, 16, MODE, 2);               \
+    else if (per <= 16) IA_GLA(T, 16, MODE, 1);                        \
+    else IA_GLA(T, 32, MODE, 1);                                       \
   } while (0)
 #define IA_GLA_T(MODE)                             \
   do {                                             \
