@@ -1378,6 +1378,18 @@ def test_copy_pages(dtype):
     assert torch.equal(pool, want)
 
 
+# one choice, as many as a wave has lanes, one more and more than twice as many; the weights are quotients of few fp32 roundings
+@pytest.mark.parametrize("softmax_first", [False, True])
+@pytest.mark.parametrize("N,E,top", [(1, 3, 1), (5, 70, 64), (3, 70, 65), (2, 300, 130)])
+def test_choices_wait_in_a_waves_lanes(N, E, top, softmax_first):
+    api = K()
+    z = _rand(N, E, seed=5)
+    ids, w = api.router_softmax_topk(z, None, top) if softmax_first else api.router_topk(z, None, top)
+    v, want = torch.topk(z.double(), top, dim=-1)
+    assert torch.equal(ids.long(), want)
+    assert torch.allclose(w.double(), torch.softmax(v, dim=-1), rtol=(top + 8) * 2.0 ** -23)
+
+
 # ---------------------------------------------------------------- routed experts, few pairs
 # one pair, 17 (a second pass over an expert's pairs), 32 (the most); fewer pairs than experts and more; rows that fill no
 # group of 16, K that fills no stretch of 256 or part of a quarter; ids without an expert; the weight on either side
