@@ -630,210 +630,6 @@ extern "C" int ia_moe_up(const void* x, const void* Wu, void* y, const int* offs
   return IA_OK;
 }
 
-// ---- the experts of a step of few pairs (decoding), without the sort ----------------------------------------------
-//   ia_moe_gate_up_few, ia_moe_up_few, ia_moe_down_few: ia_moe_gate_up, ia_moe_up and ia_moe_down with y's rows in the
-//   order of the pairs.
-// Bound by reading the chosen experts' weights once, and with one or two tokens by how many loads are in flight for it.  A
-// workgroup of four waves takes 64 / KS rows of one expert's matrix and finds the expert's pairs among the step's ids
-// itself (one load: at most 32 of them); a wave streams 16 rows over its part of K (all of it, a half or a quarter)
-// straight into registers, two stretches of 256 values in flight, with the pairs' rows of x from the caches beside them.
-// It starts at a stretch of its own and wraps (rows of a power of two would crowd on few memory channels).  The parts'
-// sums meet in LDS and are added in their order.
-// Microseconds for gate, up and down with the tiles and the sort against this, cold weights: 1 token to 4 of 32 experts of
-// 1,408 x 2,048 37.4 against 19.2 (46 MB: 2.4 TB/s, two launches); 2 tokens to 2 of 8 (2,752, no gate) 47 against 28; 1
-// token to 2 of 20 (2,432 x 4,096) 57 against 29, 16 tokens 201 against 180 (5.3 TB/s).  From 64 pairs on
-// the two are even (32 tokens to 2 of 16 67.5 against 65.4): sixteen pairs a pass of the weights, where the tiles take 32.
-#define MOE_FEW_PAIRS 32
-#define MOE_FEW_WAVES 2048       // waves in the launch that are enough; fewer: K is split over two or four of a workgroup
-
-enum { MOE_GATE_UP = 0, MOE_UP = 1, MOE_DOWN = 2 };
-
-struct MoeFewArgs {
-  const bf16_t* in;          // GATE_UP, UP: x [N, K]; DOWN: y [P, K]
-  const bf16_t* w;           // [E, rows, K]
-  void* out;                 // y [P, ff] bf16; DOWN: parts [top, N, rows] fp32
-  const int* ids;            // [P]
-  const float* weights;      // [P] or null: on the input (GATE_UP) or on the output (DOWN)
-  int P, N, E, top, K, rows, act;
-  float limit, alpha, shift;
-  bool wide;                 // parts can be stored 16 bytes at a time
-};
-
-// 16 pairs (a row of `in` a lane) times this wave's 16 rows over k_first .. k_end - 1: acc[e] is row 4 q + e for pair r
-__device__ __forceinline__ tm_f32x4 moe_few_product(const bf16_t* __restrict__ w_row, const bf16_t* __restrict__ x_row,
-                                                    int k_first, int k_end, int q, unsigned start) {
-  constexpr int PIECE = 8, STRETCH = 32 * PIECE;
-  uint4 w[2][PIECE], x[2][PIECE];
-  tm_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  const int whole = max(k_end - k_first, 0) / STRETCH;
-  int at = whole > 0 ? (int)(start % (unsigned)whole) : 0;
-  // whole stretches without conditions: the waits then count exactly and leave the next stretch in flight
-  auto load = [&](int b) {
-    const int k0 = k_first + at * STRETCH + 8 * q;
-    if (++at == whole) at = 0;
-#pragma unroll
-    for (int j = 0; j < PIECE; ++j) {
-      w[b][j] = *reinterpret_cast<const uint4*>(w_row + k0 + 32 * j);
-      x[b][j] = *reinterpret_cast<const uint4*>(x_row + k0 + 32 * j);
-    }
-  };
-  auto multiply = [&](int b) {
-#pragma unroll
-    for (int j = 0; j < PIECE; ++j)
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(tm_bf16x8, w[b][j]),
-                                                    __builtin_bit_cast(tm_bf16x8, x[b][j]), acc, 0, 0, 0);
-  };
-  if (whole > 0) {
-    load(0);
-    int s = 0;
-    for (; s + 2 < whole; s += 2) {
-      load(1);
-      multiply(0);
-      load(0);
-      multiply(1);
-    }
-    if (s + 1 < whole) {
-      load(1);
-      multiply(0);
-      multiply(1);
-    } else {
-      multiply(0);
-    }
-  }
-  // the rest: 32 values at a time, read from the row's last 8 where a lane's lie past the end, and then not taken
-  for (int k0 = k_first + whole * STRETCH; k0 < k_end; k0 += 32) {
-    const int k = k0 + 8 * q, kc = min(k, k_end - 8);
-    uint4 wt = *reinterpret_cast<const uint4*>(w_row + kc), xt = *reinterpret_cast<const uint4*>(x_row + kc);
-    const uint32_t keep = k < k_end ? 0xffffffffu : 0u;
-    wt.x &= keep; wt.y &= keep; wt.z &= keep; wt.w &= keep;
-    xt.x &= keep; xt.y &= keep; xt.z &= keep; xt.w &= keep;
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(tm_bf16x8, wt), __builtin_bit_cast(tm_bf16x8, xt),
-                                                  acc, 0, 0, 0);
-  }
-  return acc;
-}
-
-// rows c .. c + 3 of the expert's matrix for pair p
-template <int MODE>
-__device__ __forceinline__ void moe_few_emit(const MoeFewArgs& a, int p, int c, const tm_f32x4& v4) {
-  const float wt = MODE != MOE_UP && a.weights ? a.weights[p] : 1.0f;
-  if (MODE == MOE_GATE_UP) {
-    bf16_t* y = reinterpret_cast<bf16_t*>(a.out) + (size_t)p * (a.rows / 2);
-#pragma unroll
-    for (int j = 0; j < 4; j += 2) {
-      if (c + j + 1 >= a.rows) continue;
-      const float g = fminf(wt * to_float(from_float<bf16_t>(v4[j])), a.limit);
-      const float u = fminf(fmaxf(wt * to_float(from_float<bf16_t>(v4[j + 1])), -a.limit), a.limit);
-      y[(c + j) >> 1] = from_float<bf16_t>(g * (1.0f / (1.0f + expf(-a.alpha * g))) * (u + a.shift));
-    }
-  } else if (MODE == MOE_UP) {
-    bf16_t* y = reinterpret_cast<bf16_t*>(a.out) + (size_t)p * a.rows;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (c + j < a.rows) y[c + j] = from_float<bf16_t>(moe_act(to_float(from_float<bf16_t>(v4[j])), a.act));
-  } else {
-    const int token = p / a.top, choice = p - token * a.top;
-    float* o = reinterpret_cast<float*>(a.out) + ((size_t)choice * a.N + token) * a.rows + c;
-    float v[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = to_float(from_float<bf16_t>(v4[j])) * wt;
-    if (a.wide && c + 3 < a.rows) {
-      *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (c + j < a.rows) o[j] = v[j];
-    }
-  }
-}
-
-// grid (64 / KS rows of an expert's matrix, experts: all of them, or with fewer pairs than experts one for each pair that
-// is the first of its expert)
-template <int MODE, int KS>
-__global__ __launch_bounds__(256) void moe_few_kernel(MoeFewArgs a) {
-  __shared__ tm_f32x4 sums[KS > 1 ? 4 : 1][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
-  const bool by_pair = a.P < a.E;
-  const int id = a.ids[min(lane, a.P - 1)];                          // every wave: the step's ids, a lane each
-  const int e = by_pair ? __builtin_amdgcn_readlane(id, (int)blockIdx.y) : (int)blockIdx.y;
-  unsigned long long pairs = __ballot(lane < a.P && id == e);       // the expert's pairs, a bit each
-  if (pairs == 0ull || (unsigned)e >= (unsigned)a.E) return;
-  if (by_pair && __ffsll((long long)pairs) - 1 != (int)blockIdx.y) return;
-  const int part = wave % KS, n0 = blockIdx.x * (64 / KS) + wave / KS * 16;
-  const int per_part = KS == 1 ? a.K : (a.K + 32 * KS - 1) / (32 * KS) * 32;
-  const bf16_t* w_row = a.w + ((size_t)e * a.rows + min(n0 + r, a.rows - 1)) * a.K;
-  while (pairs != 0ull) {                                            // sixteen pairs at a time
-    int p = __ffsll((long long)pairs) - 1;                           // lane r: the r-th of them, or the first
-    unsigned long long left = pairs;
-    int count = 0;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int next = left ? __ffsll((long long)left) - 1 : -1;
-      if (next >= 0) {
-        if (r == i) p = next;
-        left &= left - 1ull;
-        ++count;
-      }
-    }
-    pairs = left;
-    const bf16_t* x_row = a.in + (size_t)(MODE == MOE_DOWN ? p : p / a.top) * a.K;
-    tm_f32x4 acc = moe_few_product(w_row, x_row, part * per_part, min(a.K, (part + 1) * per_part), q,
-                                   ((unsigned)(n0 / 16) * 0x9E3779B1u) >> 8);
-    if (KS > 1) {                                                    // the first part's wave adds the others' sums
-      sums[wave][lane] = acc;
-      __syncthreads();
-      if (part == 0) {
-#pragma unroll
-        for (int k = 1; k < KS; ++k) acc += sums[wave + k][lane];
-      }
-    }
-    if (part == 0 && r < count) moe_few_emit<MODE>(a, p, n0 + 4 * q, acc);
-    if (KS > 1) __syncthreads();
-  }
-}
-
-template <int MODE>
-static int launch_moe_few(const MoeFewArgs& a, hipStream_t stream) {
-  if (a.P < 0 || a.E <= 0 || a.top <= 0 || a.K <= 0 || a.rows <= 0) return IA_ERR_BAD_ARG;
-  if (a.P > MOE_FEW_PAIRS || a.E > 65535 || !tile_rows_aligned(a.in, a.K) || !tile_rows_aligned(a.w, a.K)) return IA_ERR_UNSUPPORTED;
-  if (a.P == 0) return IA_OK;
-  const int experts = a.E < a.P ? a.E : a.P;
-  const long waves = (long)((a.rows + 15) / 16) * experts;           // with all of K a wave
-  const int ks = waves >= MOE_FEW_WAVES ? 1 : 2 * waves >= MOE_FEW_WAVES ? 2 : 4;
-  const dim3 grid((a.rows + 64 / ks - 1) / (64 / ks), experts);
-  if (ks == 1) moe_few_kernel<MODE, 1><<<grid, 256, 0, stream>>>(a);
-  else if (ks == 2) moe_few_kernel<MODE, 2><<<grid, 256, 0, stream>>>(a);
-  else moe_few_kernel<MODE, 4><<<grid, 256, 0, stream>>>(a);
-  IA_LAUNCH_CHECK();
-  return IA_OK;
-}
-
-// The most pairs (tokens times choices) that the three launchers below take.
-extern "C" int ia_moe_few_pairs(void) { return MOE_FEW_PAIRS; }
-
-extern "C" int ia_moe_gate_up_few(const void* x, const void* Wgu, void* y, const int* ids, int P, int E, int top, int W,
-                                  int ff, float limit, float alpha, float shift, const float* in_weights,
-                                  hipStream_t stream) {
-  return launch_moe_few<MOE_GATE_UP>(MoeFewArgs{(const bf16_t*)x, (const bf16_t*)Wgu, y, ids, in_weights, P, 0, E, top, W,
-                                                2 * ff, 0, limit, alpha, shift, false}, stream);
-}
-
-extern "C" int ia_moe_up_few(const void* x, const void* Wu, void* y, const int* ids, int P, int E, int top, int W, int ff,
-                             int act, hipStream_t stream) {
-  if (act < 0 || act > 3) return IA_ERR_BAD_ARG;
-  return launch_moe_few<MOE_UP>(MoeFewArgs{(const bf16_t*)x, (const bf16_t*)Wu, y, ids, nullptr, P, 0, E, top, W, ff, act,
-                                           0.f, 0.f, 0.f, false}, stream);
-}
-
-extern "C" int ia_moe_down_few(const void* y, const void* Wd, float* parts, const float* weights, const int* ids, int N, int E,
-                               int top, int W, int ff, hipStream_t stream) {
-  if (N < 0 || top <= 0) return IA_ERR_BAD_ARG;
-  if (N > MOE_FEW_PAIRS || top > MOE_FEW_PAIRS) return IA_ERR_UNSUPPORTED;
-  const bool wide = ((uintptr_t)parts & 15) == 0 && (W & 3) == 0;
-  return launch_moe_few<MOE_DOWN>(MoeFewArgs{(const bf16_t*)y, (const bf16_t*)Wd, parts, ids, weights, N * top, N, E, top, ff,
-                                             W, 0, 0.f, 0.f, 0.f, wide}, stream);
-}
-
 // ---- what a step adds beside its experts' products ----
 //   ia_moe_extras   for every pair whose expert is one of the last, without tensors (ids >= E: an expert whose result is
 //                   its input): parts[choice, token, :] = weight * x[token, :]; and for every token, with `shared`: its
@@ -928,6 +724,3 @@ IA_OP(ia_moe_glu)
 IA_OP(ia_moe_scatter)
 IA_OP(ia_router_softmax_topk)
 IA_OP(ia_moe_up)
-IA_OP(ia_moe_gate_up_few)
-IA_OP(ia_moe_up_few)
-IA_OP(ia_moe_down_few)

@@ -326,21 +326,6 @@ def moe_grouped_from_tokens(E: int, top: int, W: int, ff: int, dtype: torch.dtyp
     return -(-MOE_GROUPED_ROWS_AN_EXPERT * E // top)
 
 
-def moe_few_tokens(E: int, top: int, W: int, ff: int, dtype: torch.dtype) -> int:
-    """Up to how many tokens of a step the routed experts take the kernels that stream the chosen experts' weights for
-    few pairs and need no sort (decoding); 0: never (32-bit, or rows that cannot be read 16 bytes at a time)."""
-    if dtype != torch.bfloat16 or W % 8 or ff % 8 or top <= 0 or E > 65535:
-        return 0
-    most = int(_core().ia_moe_few_pairs()) // top
-    first = moe_grouped_from_tokens(E, top, W, ff, dtype)
-    return min(most, first - 1) if first > 0 else most
-
-
-def _moe_few(x: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor, E: int, top: int, W: int, ff: int) -> bool:
-    return (1 <= x.shape[0] <= moe_few_tokens(E, top, W, ff, x.dtype)
-            and (x.data_ptr() | w_up.data_ptr() | w_down.data_ptr()) % 16 == 0)
-
-
 def moe_grouped_rows(N: int, E: int, top: int, W: int, ff: int, dtype: torch.dtype) -> bool:
     first = moe_grouped_from_tokens(E, top, W, ff, dtype)
     return first > 0 and N >= first
@@ -373,12 +358,6 @@ def moe_experts(x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, w_gat
     _need(parts.dtype == torch.float32 and parts.dim() == 3 and parts.shape[0] >= top and tuple(parts.shape[1:]) == (N, W),
           "moe: parts fp32 [>= top, N, W]")
     code = DTYPE_CODE[x.dtype]
-    if _moe_few(x, w_gate_up, w_down, E, top, W, ff):
-        _ok(_core().ia_moe_gate_up_few(_p(x), _p(w_gate_up), _p(y), _p(ids), P, E, top, W, ff, ctypes.c_float(limit),
-                                       ctypes.c_float(alpha), ctypes.c_float(shift), _p(in_w), _stream()), "moe_gate_up_few")
-        _ok(_core().ia_moe_down_few(_p(y), _p(w_down), _p(parts), _p(out_w), _p(ids), N, E, top, W, ff, _stream()),
-            "moe_down_few")
-        return SplitSum(parts)
     _ok(_core().ia_moe_sort(_p(ids), _p(offsets), _p(perm), P, total, _stream()), "moe_sort")
     if moe_grouped_rows(N, E, top, W, ff, x.dtype):
         # many rows an expert: the tokens' rows in the order of the sort, the LDS-tiled product expert by expert
@@ -1606,11 +1585,6 @@ def moe_plain_experts(x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
     perm = torch.empty(max(P, 1), dtype=torch.int32, device=x.device)
     y = torch.empty((max(P, 1), ff), dtype=x.dtype, device=x.device)
     code = DTYPE_CODE[x.dtype]
-    if _moe_few(x, w_up, w_down, E, top, W, ff):
-        _ok(_core().ia_moe_up_few(_p(x), _p(w_up), _p(y), _p(ids), P, E, top, W, ff, ACTIVATIONS[act], _stream()), "moe_up_few")
-        _ok(_core().ia_moe_down_few(_p(y), _p(w_down), _p(parts), _p(weights), _p(ids), N, E, top, W, ff, _stream()),
-            "moe_down_few")
-        return parts
     _ok(_core().ia_moe_sort(_p(ids), _p(offsets), _p(perm), P, E, _stream()), "moe_sort")
     if moe_grouped_rows(N, E, top, W, ff, x.dtype):
         xs = torch.empty((P, W), dtype=x.dtype, device=x.device)

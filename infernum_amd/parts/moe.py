@@ -196,19 +196,14 @@ class RoutedExperts(FeedForward):
                                                           int(self.renorm), int(self.sigmoid_scores), STREAM])
         else:
             program.op("core", "ia_router_topk", [z.tensor(), b, b_code, ids, wts, N, total, top, STREAM])
-        from ..engine.program import NEVER, Guard
-        most = K.moe_few_tokens(E, top, H, I, self.rt.dtype)
-        few = Guard.between(N, None, most) if most > 0 else NEVER
-        program.op("core", "ia_moe_sort", [ids, offsets, perm, N * top, total, STREAM], ~few)
+        program.op("core", "ia_moe_sort", [ids, offsets, perm, N * top, total, STREAM])
         if not self.gated:
-            return self._native_plain(program, ids, wts, offsets, perm, y, parts, few)
+            return self._native_plain(program, ids, wts, offsets, perm, y, parts)
+        from ..engine.program import NEVER, Guard
         first = K.moe_grouped_from_tokens(E, top, H, I, self.rt.dtype)
         grouped = Guard.between(N, first) if first > 0 else NEVER
-        tiled = ~grouped & ~few
+        tiled = ~grouped
         in_w, out_w = (wts, None) if self.weights_on == "input" else (None, wts)
-        program.op("core", "ia_moe_gate_up_few", [program.x, self.w_gate_up, y, ids, N * top, E, top, H, I, self.limit,
-                                                  self.alpha, self.up_shift, in_w, STREAM], few)
-        program.op("core", "ia_moe_down_few", [y, self.w_down, parts, out_w, ids, N, E, top, H, I, STREAM], few)
         program.op("core", "ia_moe_gate_up", [program.x, self.w_gate_up, y, offsets, perm, program.act_code, N * top,
                                               E, top, H, I, self.limit, self.alpha, self.up_shift, in_w, STREAM], tiled)
         program.op("core", "ia_moe_down", [y, self.w_down, parts, out_w, offsets, perm, program.act_code, N, E, top, H,
@@ -245,7 +240,7 @@ class RoutedExperts(FeedForward):
                         alt.splits or 1, N, z.at(self.total * 4) if self.shared_gate else None, int(self.w_router.shape[0]), N,
                         E, top, H, STREAM], alt.when)
 
-    def _native_plain(self, program, ids, wts, offsets, perm, y, parts, few) -> None:
+    def _native_plain(self, program, ids, wts, offsets, perm, y, parts) -> None:
         """The launches of ``kernels.api.moe_plain_experts`` and of the shared expert."""
         from ..engine.program import ALWAYS, NEVER, STREAM, Alt, Guard, Value
         from .linear import emit_linear as emit
@@ -253,9 +248,7 @@ class RoutedExperts(FeedForward):
         act, code = K.ACTIVATIONS[self.activation], program.act_code
         first = K.moe_grouped_from_tokens(E, top, H, I, self.rt.dtype)
         grouped = Guard.between(N, first) if 0 < first <= T else NEVER
-        tiled = ~grouped & ~few
-        program.op("core", "ia_moe_up_few", [program.x, self.w_gate_up, y, ids, N * top, E, top, H, I, act, STREAM], few)
-        program.op("core", "ia_moe_down_few", [y, self.w_down, parts, wts, ids, N, E, top, H, I, STREAM], few)
+        tiled = ~grouped
         program.op("core", "ia_moe_up", [program.x, self.w_gate_up, y, offsets, perm, code, N * top, E, top, H, I, act,
                                          STREAM], tiled)
         program.op("core", "ia_moe_down", [y, self.w_down, parts, wts, offsets, perm, code, N, E, top, H, I, STREAM],

@@ -1391,8 +1391,8 @@ def test_choices_wait_in_a_waves_lanes(N, E, top, softmax_first):
 
 
 # ---------------------------------------------------------------- routed experts, few pairs
-# one pair, 17 (a second pass over an expert's pairs), 32 (the most); fewer pairs than experts and more; rows that fill no
-# group of 16, K that fills no stretch of 256 or part of a quarter; ids without an expert; the weight on either side
+# one pair, 17 of one expert, 32; fewer pairs than experts and more; rows and K that fill no tile; ids without an expert; the
+# weight on either side
 @pytest.mark.parametrize("gated,weights_on", [(True, "output"), (True, "input"), (False, "output")])
 @pytest.mark.parametrize("N,top,E,W,ff", [(1, 1, 3, 264, 40), (17, 1, 2, 520, 328), (16, 2, 6, 136, 1000), (1, 4, 40, 2048, 1408),
                                           (5, 3, 300, 72, 2056)])
@@ -1406,7 +1406,6 @@ def test_routed_experts_of_few_pairs(gated, weights_on, N, top, E, W, ff):
     if N == 17:
         ids[:] = 1                                              # all of them one expert's
     wts = torch.rand(N, top, generator=g).to(DEV)
-    assert api.moe_few_tokens(E, top, W, ff, torch.bfloat16) >= N
     parts = torch.full((top, N, W), 7.0, device=DEV)
     if gated:
         api.moe_experts(x, ids, wts, up, down, 7.0, 1.702, 1.0, E + 1, parts, weights_on)
@@ -1430,3 +1429,28 @@ def test_routed_experts_of_few_pairs(gated, weights_on, N, top, E, W, ff):
             # sums in another order flip a rounding to bfloat16 (2^-9) here and there: of the first products (twice in the
             # activation), of y and of the result
             assert float((parts[c, n].double() - want).norm() / want.norm()) <= 4 * 2.0 ** -9
+
+
+# fewer pairs than experts, more, several tiles of 32 pairs of an expert, tiles of 128 (from 48 pairs an expert on)
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("E,top,W,ff,counts", [(32, 4, 2048, 1408, (2, 3, 8, 33)), (8, 2, 520, 328, (2, 5, 65, 200)), (3, 1, 72, 1000, (2, 40))])
+def test_a_pairs_result_does_not_depend_on_the_steps_other_pairs(gated, E, top, W, ff, counts):
+    api = K()
+    most = max(counts)
+    x = _rand(most, W, dtype=torch.bfloat16, seed=1)
+    up = _rand(E, (2 if gated else 1) * ff, W, dtype=torch.bfloat16, scale=2 * W ** -0.5, seed=2)
+    down = _rand(E, W, ff, dtype=torch.bfloat16, scale=ff ** -0.5, seed=3)
+    g = torch.Generator().manual_seed(4)
+    ids = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(most)]).int().to(DEV)
+    wts = torch.rand(most, top, generator=g).to(DEV)
+
+    def parts_of(N):
+        parts = torch.empty(top, N, W, device=DEV)
+        if gated:
+            api.moe_experts(x[:N], ids[:N], wts[:N], up, down, 7.0, 1.702, 1.0, E, parts)
+        else:
+            api.moe_plain_experts(x[:N], ids[:N], wts[:N], up, down, "relu_squared", parts)
+        return parts
+    want = parts_of(most)
+    for N in (1,) + counts:
+        assert torch.equal(parts_of(N), want[:, :N]), N
