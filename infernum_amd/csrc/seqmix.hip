@@ -378,7 +378,7 @@ __global__ __launch_bounds__(256) void qk_prepare_kernel(
   if (is_key) {
     const int slot = slots[t];
     const int page = slot / page_size, off = slot - page * page_size;
-    if (page < 0 || page >= num_pages) return;
+    if (slot < 0 || page >= num_pages) return;
     const int g = hd - nh;
     dst = k_pages + (((size_t)page * nkv + g) * page_size + off) * d;
     // the values: the value head of the row, or the key head as it came in; transposed within the page
@@ -429,7 +429,7 @@ __global__ __launch_bounds__(256) void qk_prepare_vec_kernel(
     const int t = (int)(w / groups) * 16 + (lane & 15), piece = (int)(w % groups) * 4 + (lane >> 4);
     if (t >= N || piece >= pieces) return;
     const int slot = slots[t], page = slot / page_size, off = slot - page * page_size;
-    if (page < 0 || page >= num_pages) return;
+    if (slot < 0 || page >= num_pages) return;
     const int col = piece * 8, g = col / dv, c = col - g * dv;
     const uint4 raw = *(const uint4*)(x + (size_t)t * x_stride + (size_t)(values_are_keys ? nh : heads) * d + col);
     const uint32_t rw[4] = {raw.x, raw.y, raw.z, raw.w};
@@ -478,7 +478,7 @@ __global__ __launch_bounds__(256) void qk_prepare_vec_kernel(
   if (!live || (is_key && !k_pages)) return;
   const int slot = is_key ? slots[t] : 0;
   const int page = slot / page_size, off = slot - page * page_size;
-  if (is_key && (page < 0 || page >= num_pages)) return;
+  if (is_key && (slot < 0 || page >= num_pages)) return;
   const int g = hd - nh;
   if (wn) {
     const float inv = 1.0f / sqrtf(ss / (float)d + eps);

@@ -74,7 +74,7 @@ __global__ __launch_bounds__(256) void sigattn_prepare_kernel(
   }
   const int slot = slots[n];
   const int page = slot / page_size, off = slot - page * page_size;
-  if ((unsigned)page >= (unsigned)num_pages) return;          // a token without a place: nothing is written
+  if (slot < 0 || page >= num_pages) return;                  // a token without a place: nothing is written
   sq_norm(row + nq, bk, wk, nk, eps, red, [](float f) { return f; },
           [&](int i, float v) {
             const int g = i / dim, c = i - g * dim;

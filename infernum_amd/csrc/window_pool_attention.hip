@@ -67,7 +67,7 @@ __global__ __launch_bounds__(64) void wpa_prepare_kernel(
     dst = q_out + (size_t)n * q_stride + (size_t)head * d;
   } else {
     const int slot = slots[n], page = slot / ps, off = slot - page * ps;
-    if ((unsigned)page >= (unsigned)num_pages) return;
+    if (slot < 0 || page >= num_pages) return;
     if (is_k) dst = k_pages + (((size_t)page * nkv + (head - nh)) * ps + off) * d;
     else {
       dst = v_pages + ((size_t)page * nkv + (head - nh - nkv)) * dv * ps + off;

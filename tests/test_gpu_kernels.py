@@ -1390,6 +1390,35 @@ def test_choices_wait_in_a_waves_lanes(N, E, top, softmax_first):
     assert torch.allclose(w.double(), torch.softmax(v, dim=-1), rtol=(top + 8) * 2.0 ** -23)
 
 
+# a token without a place (a slot below zero, or past the pages) leaves pages as they are, and what lies in front of them; vec: 8
+# values an access
+@pytest.mark.parametrize("slot", [-1, -3, -4, -5, 12, 13])
+@pytest.mark.parametrize("dtype,d,dv", [(torch.float32, 24, 12), (torch.bfloat16, 16, 32), (torch.bfloat16, 20, 12)])
+@pytest.mark.parametrize("which", ["rope", "qk", "qk_rows", "sigmoid", "window"])
+def test_a_token_without_a_place_writes_nothing(which, dtype, d, dv, slot):
+    api, N, nh, nkv, ps = K(), 3, 3, 2, 4
+    dv = d if which == "rope" else dv
+    kb, vb = torch.full((4, nkv, ps, d), 7.0, device=DEV, dtype=dtype), torch.full((4, nkv, dv, ps), 7.0, device=DEV, dtype=dtype)
+    kp, vp = kb[1:], vb[1:]
+    x = _rand(N, (nh + nkv) * d + nkv * dv, dtype=dtype)
+    q = torch.empty(N, nh * d, dtype=dtype, device=DEV)
+    pos, slots = torch.arange(N, device=DEV).int(), torch.full((N,), slot, dtype=torch.int32, device=DEV)
+    ones = torch.ones(nh * d, device=DEV)
+    freq = torch.rand(d // 2, dtype=torch.float64, device=DEV)
+    if which == "rope":
+        api.rope_kv_append(x, pos, freq, nh, nkv, d, d, slots, kp, vp, q_out=q)
+    elif which == "qk":
+        api.qk_prepare(x, q, nh, nkv, d, pos, ones[:d], ones[:d], 1e-5, freq, d, "neighbours", 1.0, slots, kp, vp)
+    elif which == "qk_rows":
+        api.qk_rows_prepare(x, q, nh, nkv, d, ones, ones[:nkv * d], 1e-5, slots, kp, vp)
+    elif which == "sigmoid":
+        api.sigattn_prepare(x, None, None, None, ones, ones[:nkv * d], 1e-5, 0.0, 0, pos, slots, q, kp, vp, nh, nkv, d, dv)
+    else:
+        api.wpa_prepare(x, None, q, pos, slots, freq, d, True, 1e-5, kp, vp, nh, nkv, d, dv)
+    assert bool(torch.isfinite(q.float()).all())
+    assert bool((kb == 7.0).all()) and bool((vb == 7.0).all())
+
+
 # ---------------------------------------------------------------- routed experts, few pairs
 # one pair, 17 of one expert, 32; fewer pairs than experts and more; rows and K that fill no tile; ids without an expert; the
 # weight on either side
