@@ -63,7 +63,7 @@ __device__ __forceinline__ void nb_store4(bf16_t* p, float4 v) {
   *reinterpret_cast<uint2*>(p) = u;
 }
 
-template <typename TD, typename TX, int NT, int NV>
+template <typename TD, typename TX, int NT, int NV, bool TOGETHER>          // TOGETHER: rows_are_few
 __global__ __launch_bounds__(NT) void norm_add_vec_kernel(float* __restrict__ h, const TD* __restrict__ delta,
                                                           int splits, size_t split_stride,
                                                           const void* __restrict__ w, int w_dtype,
@@ -73,7 +73,8 @@ __global__ __launch_bounds__(NT) void norm_add_vec_kernel(float* __restrict__ h,
   const TD* dr = delta + (size_t)row * H;
   float* hr = h + (size_t)row * H;
   float4 d[NV], hv[NV], g[NV];
-  if (NV == 1) {                                     // one piece a thread: everything is asked for before the first use
+  static_assert(!TOGETHER || NV == 1, "registers for all parts' loads of one piece");
+  if (TOGETHER) {                                    // everything is asked for before the first use
     const int il = min((int)threadIdx.x * 4, H - 4);
     d[0] = hv[0] = g[0] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (((int)__builtin_amdgcn_readfirstlane(threadIdx.x) & ~63) * 4 < H) {
@@ -132,12 +133,18 @@ static void launch_norm_add(float* h, const void* delta, int splits, size_t stri
   const bool aligned = ((reinterpret_cast<uintptr_t>(h) | reinterpret_cast<uintptr_t>(delta) |
                          reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x)) & 15) == 0 &&
                        (stride & 3) == 0;
-  if ((H & 3) == 0 && aligned && H <= 256 * 4)
-    norm_add_vec_kernel<TD, TX, 256, 1><<<N, 256, 0, stream>>>(h, d, splits, stride, w, w_dtype, xo, H, eps);
-  else if ((H & 3) == 0 && aligned && H <= 1024 * 4)      // the kernel follows from H alone: a row's sums are taken
-    norm_add_vec_kernel<TD, TX, 1024, 1><<<N, 1024, 0, stream>>>(h, d, splits, stride, w, w_dtype, xo, H, eps);   // in one order
-  else if ((H & 3) == 0 && aligned && H <= 1024 * 4 * 4)
-    norm_add_vec_kernel<TD, TX, 1024, 4><<<N, 1024, 0, stream>>>(h, d, splits, stride, w, w_dtype, xo, H, eps);
+#define IA_NA_VEC(NT, NV, TG) \
+  norm_add_vec_kernel<TD, TX, NT, NV, TG><<<N, NT, 0, stream>>>(h, d, splits, stride, w, w_dtype, xo, H, eps)
+  // the threads and pieces follow from H alone: a row's sums are taken in one order
+  if ((H & 3) == 0 && aligned && H <= 256 * 4) {
+    if (rows_are_few(N, 256)) IA_NA_VEC(256, 1, true);
+    else IA_NA_VEC(256, 1, false);
+  } else if ((H & 3) == 0 && aligned && H <= 1024 * 4) {
+    if (rows_are_few(N, 1024)) IA_NA_VEC(1024, 1, true);
+    else IA_NA_VEC(1024, 1, false);
+  } else if ((H & 3) == 0 && aligned && H <= 1024 * 4 * 4)
+    IA_NA_VEC(1024, 4, false);
+#undef IA_NA_VEC
   else
     norm_add_kernel<TD, TX><<<N, NB_NT, 0, stream>>>(h, d, splits, stride, w, w_dtype, xo, H, eps);
 }
@@ -241,7 +248,7 @@ __device__ __forceinline__ float4 nb_load4_any(const void* p, int dtype, int i) 
   return dtype == IA_F32 ? load4((const float*)p + i) : load4((const bf16_t*)p + i);
 }
 
-template <typename TD, typename TG, typename TX, int NT, int NV>
+template <typename TD, typename TG, typename TX, int NT, int NV, bool TOGETHER>
 __global__ __launch_bounds__(NT) void gated_norm_add_vec_kernel(float* __restrict__ h, const TD* __restrict__ delta,
                                                                 int splits, size_t split_stride,
                                                                 const TG* __restrict__ gate, int gate_stride,
@@ -256,7 +263,8 @@ __global__ __launch_bounds__(NT) void gated_norm_add_vec_kernel(float* __restric
   float* hr = h + (size_t)row * H;
   float4 d[NV], hv[NV];
   Raw4 wraw, nraw;
-  if (NV == 1) {                                     // one piece a thread: everything is asked for before the first use
+  static_assert(!TOGETHER || NV == 1, "registers for all parts' loads of one piece");
+  if (TOGETHER) {                                    // everything is asked for before the first use
     const int il = min((int)threadIdx.x * 4, H - 4);
     d[0] = hv[0] = make_float4(0.f, 0.f, 0.f, 0.f);
     wraw.u = nraw.u = make_uint4(0u, 0u, 0u, 0u);
@@ -330,7 +338,7 @@ __global__ __launch_bounds__(NT) void gated_norm_add_vec_kernel(float* __restric
   for (int c = 0; c < NV; ++c) {
     const int i = (threadIdx.x + c * NT) * 4;
     if (i < H) {
-      const float4 g = NV == 1 ? raw4_values(wraw, w_dtype) : nb_load4_any(w, w_dtype, i);
+      const float4 g = TOGETHER ? raw4_values(wraw, w_dtype) : nb_load4_any(w, w_dtype, i);
       hv[c] = make_float4(hv[c].x + d[c].x * inv * g.x, hv[c].y + d[c].y * inv * g.y, hv[c].z + d[c].z * inv * g.z,
                           hv[c].w + d[c].w * inv * g.w);
       nb_store4(hr + i, hv[c]);
@@ -349,7 +357,7 @@ __global__ __launch_bounds__(NT) void gated_norm_add_vec_kernel(float* __restric
     if (i < H) {
       float4 o = hv[c];
       if (w_next) {
-        const float4 g = NV == 1 ? raw4_values(nraw, w_next_dtype) : nb_load4_any(w_next, w_next_dtype, i);
+        const float4 g = TOGETHER ? raw4_values(nraw, w_next_dtype) : nb_load4_any(w_next, w_next_dtype, i);
         o = make_float4(o.x * inv2 * g.x, o.y * inv2 * g.y, o.z * inv2 * g.z, o.w * inv2 * g.w);
       }
       nb_store4(x + (size_t)row * H + i, o);
@@ -367,13 +375,18 @@ static void launch_gated_norm_add_typed(float* h, const TD* delta, int splits, s
                          reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(w_next) |
                          reinterpret_cast<uintptr_t>(x)) & 15) == 0 &&
                        (stride & 3) == 0 && (gate_stride & 3) == 0 && (gate_split_stride & 3) == 0 && (H & 3) == 0;
-#define IA_GNA_VEC(NT, NV)                                                                                          \
-  gated_norm_add_vec_kernel<TD, TG, TX, NT, NV><<<N, NT, 0, stream>>>(                                             \
+#define IA_GNA_VEC(NT, NV, TOGETHER)                                                                                \
+  gated_norm_add_vec_kernel<TD, TG, TX, NT, NV, TOGETHER><<<N, NT, 0, stream>>>(                                             \
       h, delta, splits, stride, gate, gate_stride, gate_splits, gate_split_stride, gate_bias, w, w_dtype, w_next,   \
       w_next_dtype, x, H, eps)
-  if (aligned && H <= 256 * 4) IA_GNA_VEC(256, 1);           // the kernel follows from H alone: a row's sums are taken
-  else if (aligned && H <= 1024 * 4) IA_GNA_VEC(1024, 1);    // in one order
-  else if (aligned && H <= 1024 * 4 * 4) IA_GNA_VEC(1024, 4);
+  // the threads and pieces follow from H alone: a row's sums are taken in one order
+  // (one and two parts are as fast one after the other: 64 rows of 4,096 5.0 / 5.1 us, together 5.1 / 5.3)
+  const bool many_parts = splits > 2 || gate_splits > 2;
+  if (aligned && H <= 256 * 4 && many_parts && rows_are_few(N, 256)) IA_GNA_VEC(256, 1, true);
+  else if (aligned && H <= 256 * 4) IA_GNA_VEC(256, 1, false);
+  else if (aligned && H <= 1024 * 4 && many_parts && rows_are_few(N, 1024)) IA_GNA_VEC(1024, 1, true);
+  else if (aligned && H <= 1024 * 4) IA_GNA_VEC(1024, 1, false);
+  else if (aligned && H <= 1024 * 4 * 4) IA_GNA_VEC(1024, 4, false);
   else
     gated_norm_add_kernel<TD, TG, TX><<<N, NB_NT, 0, stream>>>(h, delta, splits, stride, gate, gate_stride, gate_splits,
                                                                gate_split_stride, gate_bias, w, w_dtype, w_next,

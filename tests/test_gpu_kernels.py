@@ -89,6 +89,32 @@ def test_add_rmsnorm_joins_partial_sums(H, S):
     assert torch.equal(out2, out[rows.long()])
 
 
+# one row more than the few whose loads go out together: the last row and the first of both ways; rows that fill no wave
+@pytest.mark.parametrize("splits", [1, 2, 3, 8, 17])
+@pytest.mark.parametrize("H,few", [(1024, 1024), (500, 1024), (2048, 256), (3100, 256)])
+def test_norms_of_many_rows_equal_those_of_few(H, few, splits):
+    api, N = K(), few + 1
+    h, parts, gates, bias = _rand(N, H, seed=1), _rand(splits, N, H, seed=2), _rand(splits, N, H, seed=3), _rand(H, seed=4)
+    w, w2 = (_rand(H, seed=5).abs() + 0.5).bfloat16(), (_rand(H, seed=6).abs() + 0.5).bfloat16()
+
+    def all_three(rows):
+        hs = [h[rows].clone() for _ in range(3)]
+        xs = [torch.empty(hs[0].shape, dtype=torch.bfloat16, device=DEV) for _ in range(3)]
+        d, g = api.SplitSum(parts[:, rows].contiguous()), api.SplitSum(gates[:, rows].contiguous())
+        api.add_rmsnorm(hs[0], d, w, 1e-5, xs[0])
+        api.norm_add(hs[1], d, w, 1e-5, xs[1])
+        api.gated_norm_add(hs[2], d, g, bias, w, 1e-5, w2, xs[2])
+        return hs + xs
+    many = all_three(slice(0, N))
+    for rows in (slice(0, 3), slice(N - 5, N)):
+        for got, want in zip(all_three(rows), many):
+            assert torch.equal(got, want[rows])
+    d, g = parts.double().sum(0), gates.double().sum(0) + bias.double()
+    d = d / (1 + torch.exp(-g))
+    want = h.double() + d / torch.sqrt((d * d).mean(-1, keepdim=True) + 1e-5) * w.double()
+    assert bool(((many[2].double() - want).abs() <= (splits + 16) * 2.0 ** -22 * (1 + want.abs()) + 1e-6).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("H", [2048, 3000, 4096, 5120, 1000])
 def test_add_rmsnorm_of_many_rows_equals_that_of_few(dtype, H):
