@@ -115,6 +115,19 @@ def test_norms_of_many_rows_equal_those_of_few(H, few, splits):
     assert bool(((many[2].double() - want).abs() <= (splits + 16) * 2.0 ** -22 * (1 + want.abs()) + 1e-6).all())
 
 
+# two results into the stream, by the number of their parts and the values: the loads together (more than six parts, or more than three
+# of two million values) and one after the other; the sums in the order of the parts, so the bits
+@pytest.mark.parametrize("N,H,a_parts,b_parts", [(3, 72, 1, 1), (5, 256, 2, 3), (5, 256, 6, 1), (5, 256, 7, 2), (4, 1000, 1, 17), (3, 256, 8, 0),
+                                                 (1024, 2048, 4, 1), (1023, 2048, 4, 4)])
+def test_two_results_into_the_stream(N, H, a_parts, b_parts):
+    api = K()
+    h, a, b = _rand(N, H, seed=1), _rand(a_parts, N, H, seed=2), _rand(max(b_parts, 1), N, H, seed=3)
+    want = h + sum(a[1:], a[0]) if b_parts == 0 else h + sum(a[1:], a[0]) + sum(b[1:], b[0])
+    x = torch.empty(N, H, dtype=torch.bfloat16, device=DEV)
+    api.stream_add2(h, api.SplitSum(a), api.SplitSum(b) if b_parts else None, x)
+    assert torch.equal(h, want) and torch.equal(x, want.bfloat16())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("H", [2048, 3000, 4096, 5120, 1000])
 def test_add_rmsnorm_of_many_rows_equals_that_of_few(dtype, H):
