@@ -367,12 +367,12 @@ extern "C" int ia_wpa_attention(const void* q, int q_stride, const void* k_pages
 }
 
 // ---- rows divided by their root mean square, a wave a row
-// (rows of up to 1,024 values are asked for at once and kept: one row of 768: 12 us value after value, twice, so 2.9)
-template <typename T>
+// (KEEP values a lane are asked for at once and kept, what lies beyond them is read one after the other, twice: one row of 768:
+// 12 us value after value and 2.9 with sixteen kept)
+template <typename T, int KEEP>
 __global__ __launch_bounds__(256) void rms_rows_kernel(const T* __restrict__ x, int x_stride, const void* __restrict__ w,
                                                        int w_dtype, T* __restrict__ y, int y_stride, int N, int C,
                                                        float eps) {
-  constexpr int KEEP = 16;
   const int n = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (n >= N) return;
   const T* xr = x + (size_t)n * x_stride;
@@ -411,14 +411,26 @@ extern "C" int ia_rms_rows(const void* x, int x_stride, const void* w, int w_dty
   if (N < 0 || C <= 0 || x_stride < C || y_stride < C || !(eps > 0.f)) return IA_ERR_BAD_ARG;
   if (N == 0) return IA_OK;
   if (!x || !y) return IA_ERR_BAD_ARG;
+  if (dtype != IA_F32 && dtype != IA_BF16) return IA_ERR_BAD_ARG;
   const int grid = (N + 3) / 4;
-  if (dtype == IA_F32)
-    rms_rows_kernel<float><<<grid, 256, 0, stream>>>((const float*)x, x_stride, w, w_dtype, (float*)y, y_stride, N, C, eps);
-  else if (dtype == IA_BF16)
-    rms_rows_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)x, x_stride, w, w_dtype, (bf16_t*)y, y_stride, N, C,
-                                                      eps);
-  else
-    return IA_ERR_BAD_ARG;
+#define IA_RMS_ROWS(KEEP)                                                                                            \
+  do {                                                                                                               \
+    if (dtype == IA_F32)                                                                                             \
+      rms_rows_kernel<float, KEEP><<<grid, 256, 0, stream>>>((const float*)x, x_stride, w, w_dtype, (float*)y,       \
+                                                             y_stride, N, C, eps);                                   \
+    else                                                                                                             \
+      rms_rows_kernel<bf16_t, KEEP><<<grid, 256, 0, stream>>>((const bf16_t*)x, x_stride, w, w_dtype, (bf16_t*)y,    \
+                                                              y_stride, N, C, eps);                                  \
+  } while (0)
+  // as many as the row has, for what is asked for twice costs (8,192 rows of 64 / 128 values: with sixteen kept 1.57 / 1.41 times
+  // the time of value after value); and with some thousands of wide rows their second reads come from memory again, where
+  // kept values only cost waves in flight (8,192 rows of 1,536 / 3,072 / 4,096: 0.83 / 1.34 / 1.47 of the time, 4,096 rows 0.62 / 0.77 / 0.83)
+  if (C <= 64 || (C > 2048 && N > 4096)) IA_RMS_ROWS(1);
+  else if (C <= 128) IA_RMS_ROWS(2);
+  else if (C <= 256) IA_RMS_ROWS(4);
+  else if (C <= 512) IA_RMS_ROWS(8);
+  else IA_RMS_ROWS(16);
+#undef IA_RMS_ROWS
   IA_LAUNCH_CHECK();
   return IA_OK;
 }

@@ -101,7 +101,10 @@ CUTS = lambda T: ([T], [1] * T, [T - 9] + [1] * 9, [2] * (T // 2) + [T % 2] * (T
 
 # ------------------------------------------------------------------------------------ small kernels alone
 @BOTH
-@pytest.mark.parametrize("N,C,col,extra", [(1, 8, 0, 0), (37, 80, 5, 9), (200, 24, 0, 40), (3, 300, 2, 1)])
+# 64 .. 1,024: the most values a lane keeps one, two, four, eight and sixteen of, and one more; wide rows, some thousands of them
+@pytest.mark.parametrize("N,C,col,extra", [(1, 8, 0, 0), (37, 80, 5, 9), (200, 24, 0, 40), (3, 300, 2, 1), (5, 64, 0, 0), (6, 65, 1, 0),
+                                           (5, 128, 0, 3), (7, 129, 0, 0), (5, 256, 0, 0), (5, 257, 0, 0), (5, 512, 0, 0), (5, 513, 4, 0),
+                                           (5, 1023, 0, 0), (3, 1024, 0, 0), (3, 1025, 0, 0), (2, 1600, 0, 0), (4098, 1540, 0, 0)])
 def test_rows_divided_by_their_root_mean_square(dtype, N, C, col, extra):
     from infernum_amd.kernels import api as K
     rt = runtime(dtype)
