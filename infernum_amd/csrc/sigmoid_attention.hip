@@ -21,41 +21,41 @@
 #define SA_MAX_D 640
 
 // Bound by trips to memory where tokens are few: grid (N, 2), the queries' norm and the keys' and values' side by side, and
-// up to 8 values a thread (rows of 2,048) with their bias and weight asked for together and kept for the second use (one
-// token of 16 heads of 128: 13.4 us with the loads one after the other, twice, so 7.2).
-#define SQ_KEEP 8
+// up to 8 values a thread (rows of 2,048; KEEP: as many as the row has, what is asked for twice costs) with their bias and
+// weight asked for together and kept for the second use (one token of 16 heads of 128: 13.4 us with the loads one after the
+// other, twice, so 7.2; 3,000 tokens of 4 heads of 64 12.1 one after the other, 13.8 with eight kept).
 template <typename T>
 __device__ __forceinline__ float sq_value(const T* __restrict__ row, const float* __restrict__ b, int i) {
   return to_float(row[i]) + (b ? b[i] : 0.f);
 }
 
 // emit(i, value over the root mean square times factor and w[i]) for every value of one norm of `n` values
-template <typename T, typename Factor, typename Emit>
+template <int KEEP, typename T, typename Factor, typename Emit>
 __device__ __forceinline__ void sq_norm(const T* __restrict__ row, const float* __restrict__ b, const float* __restrict__ w,
                                         int n, float eps, float* red, Factor factor, Emit emit) {
   const int tid = threadIdx.x;
-  float x[SQ_KEEP], wx[SQ_KEEP], ss = 0.f;
+  float x[KEEP], wx[KEEP], ss = 0.f;
 #pragma unroll
-  for (int u = 0; u < SQ_KEEP; ++u) {
+  for (int u = 0; u < KEEP; ++u) {
     const int i = min(tid + 256 * u, n - 1);
     x[u] = sq_value(row, b, i);
     wx[u] = w[i];
   }
 #pragma unroll
-  for (int u = 0; u < SQ_KEEP; ++u) ss = tid + 256 * u < n ? fmaf(x[u], x[u], ss) : ss;
-  for (int i = tid + 256 * SQ_KEEP; i < n; i += 256) {
+  for (int u = 0; u < KEEP; ++u) ss = tid + 256 * u < n ? fmaf(x[u], x[u], ss) : ss;
+  for (int i = tid + 256 * KEEP; i < n; i += 256) {
     const float v = sq_value(row, b, i);
     ss = fmaf(v, v, ss);
   }
   ss = block_sum<256>(ss, red);
   const float f = factor(1.0f / sqrtf(ss / (float)n + eps));
 #pragma unroll
-  for (int u = 0; u < SQ_KEEP; ++u)
+  for (int u = 0; u < KEEP; ++u)
     if (tid + 256 * u < n) emit(tid + 256 * u, x[u] * f * wx[u]);
-  for (int i = tid + 256 * SQ_KEEP; i < n; i += 256) emit(i, sq_value(row, b, i) * f * w[i]);
+  for (int i = tid + 256 * KEEP; i < n; i += 256) emit(i, sq_value(row, b, i) * f * w[i]);
 }
 
-template <typename T>
+template <typename T, int KEEP>
 __global__ __launch_bounds__(256) void sigattn_prepare_kernel(
     const T* __restrict__ proj, int proj_stride, const float* __restrict__ bq, const float* __restrict__ bk,
     const float* __restrict__ bv, const float* __restrict__ wq, const float* __restrict__ wk, float eps, float temp_coef,
@@ -67,7 +67,7 @@ __global__ __launch_bounds__(256) void sigattn_prepare_kernel(
   const int nq = nh * dim, nk = nkv * dim, nv = nkv * vdim;
   if (blockIdx.y == 0) {
     const int p = temp_every > 0 ? positions[n] : 0;
-    sq_norm(row, bq, wq, nq, eps, red,
+    sq_norm<KEEP>(row, bq, wq, nq, eps, red,
             [&](float f) { return temp_every > 0 ? f * (1.0f + temp_coef * logf((float)((p + 1) / temp_every) + 1.0f)) : f; },
             [&](int i, float v) { q_out[(size_t)n * nq + i] = from_float<T>(v); });
     return;
@@ -75,7 +75,7 @@ __global__ __launch_bounds__(256) void sigattn_prepare_kernel(
   const int slot = slots[n];
   const int page = slot / page_size, off = slot - page * page_size;
   if (slot < 0 || page >= num_pages) return;                  // a token without a place: nothing is written
-  sq_norm(row + nq, bk, wk, nk, eps, red, [](float f) { return f; },
+  sq_norm<KEEP>(row + nq, bk, wk, nk, eps, red, [](float f) { return f; },
           [&](int i, float v) {
             const int g = i / dim, c = i - g * dim;
             k_pages[(((size_t)page * nkv + g) * page_size + off) * dim + c] = from_float<T>(v);
@@ -99,18 +99,23 @@ extern "C" int ia_sigattn_prepare(const void* proj, int code, int proj_stride, c
   if (N == 0) return IA_OK;
   if (!proj || !wq || !q_out || !positions || (slots && (!wk || !k_pages || !v_pages || page_size <= 0 || num_pages <= 0)))
     return IA_ERR_BAD_ARG;
-  if (code == IA_F32)
-    sigattn_prepare_kernel<float><<<dim3(N, slots ? 2 : 1), 256, 0, stream>>>((const float*)proj, proj_stride, bq, bk, bv, wq, wk, eps,
-                                                         temp_coef, temp_every, positions, slots, (float*)q_out,
-                                                         (float*)k_pages, (float*)v_pages, nh, nkv, dim, vdim, page_size,
-                                                         num_pages);
-  else if (code == IA_BF16)
-    sigattn_prepare_kernel<bf16_t><<<dim3(N, slots ? 2 : 1), 256, 0, stream>>>((const bf16_t*)proj, proj_stride, bq, bk, bv, wq, wk, eps,
-                                                          temp_coef, temp_every, positions, slots, (bf16_t*)q_out,
-                                                          (bf16_t*)k_pages, (bf16_t*)v_pages, nh, nkv, dim, vdim,
-                                                          page_size, num_pages);
-  else
-    return IA_ERR_BAD_ARG;
+  if (code != IA_F32 && code != IA_BF16) return IA_ERR_BAD_ARG;
+#define IA_SQ(T, KEEP)                                                                                                 \
+  sigattn_prepare_kernel<T, KEEP><<<dim3(N, slots ? 2 : 1), 256, 0, stream>>>(                                        \
+      (const T*)proj, proj_stride, bq, bk, bv, wq, wk, eps, temp_coef, temp_every, positions, slots, (T*)q_out,       \
+      (T*)k_pages, (T*)v_pages, nh, nkv, dim, vdim, page_size, num_pages)
+#define IA_SQ_KEEP(T)                        \
+  do {                                       \
+    if (widest <= 256) IA_SQ(T, 1);          \
+    else if (widest <= 512) IA_SQ(T, 2);     \
+    else if (widest <= 1024) IA_SQ(T, 4);    \
+    else IA_SQ(T, 8);                        \
+  } while (0)
+  const int widest = (slots && nkv > nh ? nkv : nh) * dim;
+  if (code == IA_F32) IA_SQ_KEEP(float);
+  else IA_SQ_KEEP(bf16_t);
+#undef IA_SQ_KEEP
+#undef IA_SQ
   IA_LAUNCH_CHECK();
   return IA_OK;
 }

@@ -73,6 +73,39 @@ def _run_mixer(mixer, steps, x, cuts, rt, request="a"):
 
 
 # ------------------------------------------------------------------------------------ kernels alone
+# queries and keys of one, two, four and eight values a thread and beyond, the ends of each
+@BOTH
+@pytest.mark.parametrize("nh,nkv,dim,vdim", [(2, 1, 128, 16), (1, 2, 136, 16), (4, 2, 128, 32), (3, 1, 176, 16), (8, 2, 128, 16),
+                                             (5, 1, 208, 16), (16, 4, 128, 128), (9, 2, 232, 16)])
+def test_norms_of_queries_and_keys_over_all_heads(dtype, nh, nkv, dim, vdim):
+    from infernum_amd.kernels import api as K
+    rt = runtime(dtype)
+    g = torch.Generator().manual_seed(nh * dim)
+    N, ps, nq, nk, nv = 5, 4, nh * dim, nkv * dim, nkv * vdim
+    proj = torch.randn(N, nq + nk + nv + 8, generator=g).to(DEV).to(rt.dtype)
+    bq, bk, bv = (torch.randn(n, generator=g).to(DEV) for n in (nq, nk, nv))
+    wq, wk = (torch.rand(n, generator=g).to(DEV) + 0.5 for n in (nq, nk))
+    pos = torch.tensor([0, 7, 511, 512, 4000], dtype=torch.int32, device=DEV)
+    slots = torch.tensor([2, 9, -1, 0, 11], dtype=torch.int32, device=DEV)                # a token without a place
+    kp, vp = (torch.full((4, nkv) + rows, 7.0, device=DEV, dtype=rt.dtype)[1:] for rows in ((ps, dim), (vdim, ps)))
+    q = torch.empty(N, nq, device=DEV, dtype=rt.dtype)
+    K.sigattn_prepare(proj, bq, bk, bv, wq, wk, 1e-5, 0.1, 512, pos, slots, q, kp, vp, nh, nkv, dim, vdim)
+    p = proj.double()
+    unit = lambda x: x / torch.sqrt((x * x).mean(-1, keepdim=True) + 1e-5)           # noqa: E731
+    factor = 1 + 0.1 * torch.log(torch.div(pos.double() + 1, 512, rounding_mode="floor") + 1)
+    want_q = unit(p[:, :nq] + bq.double()) * wq.double() * factor[:, None]
+    want_k, want_v = unit(p[:, nq:nq + nk] + bk.double()) * wk.double(), p[:, nq + nk:nq + nk + nv] + bv.double()
+    tol = 2.0 ** -8 if dtype == "bfloat16" else 2.0 ** -19                              # a rounding; sums of up to 2,088 fp32 squares
+    assert bool(((q.double() - want_q).abs() <= tol * want_q.abs() + 1e-6).all())
+    want_kp, want_vp = torch.full(kp.shape, 7.0, dtype=torch.float64, device=DEV), torch.full(vp.shape, 7.0, dtype=torch.float64, device=DEV)
+    for n in (0, 1, 3, 4):
+        page, off = divmod(int(slots[n]), ps)
+        want_kp[page, :, off] = want_k[n].view(nkv, dim)
+        want_vp[page, :, :, off] = want_v[n].view(nkv, vdim)
+    assert bool(((kp.double() - want_kp).abs() <= tol * want_kp.abs() + 1e-6).all())
+    assert bool(((vp.double() - want_vp).abs() <= tol * want_vp.abs() + 1e-6).all())
+
+
 @BOTH
 def test_learned_position_rows(dtype):
     from infernum_amd.kernels import api as K
