@@ -442,17 +442,19 @@ extern "C" int ia_gated_norm_add(float* h, const void* delta, int delta_dtype, i
 
 // h[n, :] += table[index[n], :] (fp32 sums; the table in fp32 or bfloat16): a learned vector per position.  An index
 // outside the table leaves NaN, never a stray read.
-// grid (N, pieces of 1,024 values of a row, at most 65,535): a thread's four values asked for together (two rows of 2,048: 8.4 us with one
-// workgroup a row and one value after the other, 3.3 with everything in the caches; so 2.3 there).
+// grid (N, pieces of VALUES * 256 values of a row, at most 65,535): a thread's values asked for together (two rows of 2,048: 8.4
+// us with one workgroup a row and one value after the other, 3.3 with everything in the caches; so 2.3 there).
+// Rows of up to 256 values give a thread one (8,192 rows of 72: 4.9 us, with four 5.2).
+template <int VALUES>
 __global__ __launch_bounds__(256) void add_rows_kernel(float* __restrict__ h, const void* __restrict__ table, int dtype,
                                                        const int* __restrict__ index, int H, int rows) {
   const int n = blockIdx.x;
   float* hr = h + (size_t)n * H;
-  for (size_t i0 = (size_t)blockIdx.y * 1024 + threadIdx.x; i0 < (size_t)H; i0 += (size_t)gridDim.y * 1024) {
-    size_t i[4];
-    float v[4], t[4];
+  for (size_t i0 = (size_t)blockIdx.y * (VALUES * 256) + threadIdx.x; i0 < (size_t)H; i0 += (size_t)gridDim.y * (VALUES * 256)) {
+    size_t i[VALUES];
+    float v[VALUES], t[VALUES];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < VALUES; ++e) {
       i[e] = i0 + 256 * e < (size_t)H ? i0 + 256 * e : (size_t)H - 1;
       v[e] = hr[i[e]];
     }
@@ -461,13 +463,13 @@ __global__ __launch_bounds__(256) void add_rows_kernel(float* __restrict__ h, co
     const size_t at = (size_t)(in ? r : 0) * H;
     if (dtype == IA_F32) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) t[e] = ((const float*)table)[at + i[e]];
+      for (int e = 0; e < VALUES; ++e) t[e] = ((const float*)table)[at + i[e]];
     } else {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) t[e] = bf16_bits_to_float(((const uint16_t*)table)[at + i[e]]);
+      for (int e = 0; e < VALUES; ++e) t[e] = bf16_bits_to_float(((const uint16_t*)table)[at + i[e]]);
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
+    for (int e = 0; e < VALUES; ++e)
       if (i0 + 256 * e < (size_t)H) hr[i[e]] = in ? v[e] + t[e] : __uint_as_float(0x7fc00000u);
   }
 }
@@ -477,7 +479,10 @@ extern "C" int ia_add_rows(float* h, const void* table, int dtype, const int* in
   if (N < 0 || H <= 0 || rows <= 0 || !h || !table || !index || (dtype != IA_F32 && dtype != IA_BF16)) return IA_ERR_BAD_ARG;
   if (N == 0) return IA_OK;
   const int pieces = (H - 1) / 1024 + 1;
-  add_rows_kernel<<<dim3(N, pieces < 65535 ? pieces : 65535), 256, 0, stream>>>(h, table, dtype, index, H, rows);
+  if (H <= 256)
+    add_rows_kernel<1><<<N, 256, 0, stream>>>(h, table, dtype, index, H, rows);
+  else
+    add_rows_kernel<4><<<dim3(N, pieces < 65535 ? pieces : 65535), 256, 0, stream>>>(h, table, dtype, index, H, rows);
   IA_LAUNCH_CHECK();
   return IA_OK;
 }

@@ -73,6 +73,21 @@ def _run_mixer(mixer, steps, x, cuts, rt, request="a"):
 
 
 # ------------------------------------------------------------------------------------ kernels alone
+# rows of one value a thread, of four, the ends of both, and more than one piece; indices outside the table leave NaN in their rows
+@BOTH
+@pytest.mark.parametrize("H", [255, 256, 257, 1023, 1025, 2050])
+def test_rows_of_a_table_added_by_index(dtype, H):
+    from infernum_amd.kernels import api as K
+    rt = runtime(dtype)
+    g = torch.Generator().manual_seed(H)
+    h, table = torch.randn(7, H, generator=g).to(DEV), torch.randn(5, H, generator=g).to(DEV).to(rt.dtype)
+    index = torch.tensor([4, 0, -1, 2, 5, 2, 1], dtype=torch.int32, device=DEV)
+    want = h + table.float()[index.long().clamp(0, 4)]
+    K.add_rows(h, table, index)
+    ok = torch.tensor([0, 1, 3, 5, 6], device=DEV)
+    assert torch.equal(h[ok], want[ok]) and bool(torch.isnan(h[[2, 4]]).all())
+
+
 # queries and keys of one, two, four and eight values a thread and beyond, the ends of each
 @BOTH
 @pytest.mark.parametrize("nh,nkv,dim,vdim", [(2, 1, 128, 16), (1, 2, 136, 16), (4, 2, 128, 32), (3, 1, 176, 16), (8, 2, 128, 16),
