@@ -567,14 +567,15 @@ extern "C" int ia_wpa_prefill(const void* q, int q_stride, const void* k_pages, 
   return IA_OK;
 }
 
+template <int PRE>
 __global__ __launch_bounds__(64) void wpa_join_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                                       uint16_t* __restrict__ out, const float* __restrict__ sinks, int nh,
                                                       int num_parts) {
   const int h = blockIdx.x % nh, dim = blockIdx.y * 64 + threadIdx.x;
-  const JoinedParts J = join_parts(part_o, part_ml, (size_t)blockIdx.x * num_parts, num_parts, WP_VDIM, dim);
+  const JoinedParts<1> J = join_parts<PRE, 1>(part_o, part_ml, (size_t)blockIdx.x * num_parts, num_parts, WP_VDIM, dim);
   if (dim >= WP_VDIM) return;
   const float l = sinks ? J.weight + __builtin_amdgcn_exp2f(sinks[h] * WP_LOG2E - J.top) : J.weight;
-  out[(size_t)blockIdx.x * WP_VDIM + dim] = float_to_bf16_bits(J.sum * (1.0f / l));
+  out[(size_t)blockIdx.x * WP_VDIM + dim] = float_to_bf16_bits(J.sum[0] * (1.0f / l));
 }
 
 // num_parts > 1: the tiles of a request's blocks and keys are cut into so many parts, a workgroup each, which leave
@@ -605,7 +606,11 @@ extern "C" int ia_wpa_decode(const void* q, int q_stride, const void* k_pages, c
 #undef WP_DEC
   IA_LAUNCH_CHECK();
   if (num_parts > 1) {
-    wpa_join_kernel<<<dim3(B * nh, (WP_VDIM + 63) / 64), 64, 0, stream>>>(part_o, part_ml, (uint16_t*)out, sinks, nh, num_parts);
+    const dim3 heads(B * nh, (WP_VDIM + 63) / 64);
+    const int pre = joined_at_once(num_parts);
+    if (pre == 2) wpa_join_kernel<2><<<heads, 64, 0, stream>>>(part_o, part_ml, (uint16_t*)out, sinks, nh, num_parts);
+    else if (pre == 4) wpa_join_kernel<4><<<heads, 64, 0, stream>>>(part_o, part_ml, (uint16_t*)out, sinks, nh, num_parts);
+    else wpa_join_kernel<16><<<heads, 64, 0, stream>>>(part_o, part_ml, (uint16_t*)out, sinks, nh, num_parts);
     IA_LAUNCH_CHECK();
   }
   return IA_OK;

@@ -1429,6 +1429,22 @@ def test_choices_wait_in_a_waves_lanes(N, E, top, softmax_first):
     assert torch.allclose(w.double(), torch.softmax(v, dim=-1), rtol=(top + 8) * 2.0 ** -23)
 
 
+# the join of a step of 1,024 (token, head) pairs and more, a wave for all channels of one, against that of fewer
+@pytest.mark.parametrize("d,nkv,parts", [(64, 4, 3), (256, 1, 2), (256, 1, 5), (80, 2, 5)])
+def test_join_of_many_heads_equals_that_of_few(d, nkv, parts):
+    api, B, nh, keys = K(), 64, 16, 90
+    pages = -(-keys // 16)
+    kp, vp = _rand(B * pages, nkv, 16, d, dtype=torch.bfloat16, seed=1), _rand(B * pages, nkv, d, 16, dtype=torch.bfloat16, seed=2)
+    bt = torch.randperm(B * pages, generator=torch.Generator().manual_seed(3)).int().view(B, pages).to(DEV)
+    q, pos = _rand(B, nh * d, dtype=torch.bfloat16, seed=4), (torch.arange(B, device=DEV) + keys - B).int()
+    out, few = (torch.empty(B, nh * d, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    api.attention_decode(q, kp, vp, out, pos, bt, nh, nkv, d, d ** -0.5, 0, keys, parts)
+    for b in range(0, B, 32):
+        r = slice(b, b + 32)
+        api.attention_decode(q[r], kp, vp, few[r], pos[r], bt[r], nh, nkv, d, d ** -0.5, 0, keys, parts)
+    assert torch.equal(out, few)
+
+
 # a token without a place (a slot below zero, or past the pages) leaves pages as they are, and what lies in front of them; vec: 8
 # values an access
 @pytest.mark.parametrize("slot", [-1, -3, -4, -5, 12, 13])
