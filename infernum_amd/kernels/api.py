@@ -2020,12 +2020,14 @@ def wpa_decode_parts(batch: int, nh: int, nkv: int, max_len: int, window: int, p
     """Parts that the tiles of a token's keys and blocks are cut into (a workgroup of four waves each): as many as bring
     the workgroups to the compute units, at most the square root of the tiles (the join grows with the parts as the work of
     one shrinks: one request on 4 key/value heads, 1,024 keys and 31 blocks, takes 36 us whole and 13 + 6 in 8 parts)
-    and 16."""
+    and 16.  Two parts of fewer than 16 tiles do not pay for the join's launch (one request, 100 keys 6.4 us whole and 7.0 in two
+    parts, 129 keys 7.2 and in three 7.0; 32 requests 129 keys 7.5 and 8.2 in two, 256 keys 8.8 and 8.6)."""
     groups = max(1, batch * nkv * ((nh // nkv + 15) // 16))
     keys = min(max_len, window + 15) if window > 0 else max_len
     blocks = max(0, max_len - window) // pool if window > 0 and pool > 0 else 0
     tiles = (keys + 15) // 16 + (blocks + 15) // 16
-    return max(1, min(compute_units(device) // groups, math.isqrt(max(tiles, 1)), 16))
+    parts = max(1, min(compute_units(device) // groups, math.isqrt(max(tiles, 1)), 16))
+    return 1 if parts == 2 and tiles < 16 else parts
 
 
 def wpa_decode_part_floats(nh: int, nkv: int, dv: int, device: Optional[torch.device] = None) -> int:
