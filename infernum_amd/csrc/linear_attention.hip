@@ -126,7 +126,8 @@ __global__ __launch_bounds__(256) void gla_scan_kernel(
     }
     v_next = pr[(unsigned)(min(v_t, last_t) * proj_stride + v_col + hd * vdim + min(v_c, vdim - 1))];
   };
-  if (MODE != 0) ask(0);
+  constexpr bool AHEAD = MODE != 0 && KMAX <= 16;  // (32 channels a thread leave no registers for it: 1,000 rows of 2 heads of 512 543 us, 559 with)
+  if (AHEAD) ask(0);
   float dprod[MODE == 1 ? KMAX : 1];
   float reg[SL][KMAX];
 #pragma unroll
@@ -138,7 +139,7 @@ __global__ __launch_bounds__(256) void gla_scan_kernel(
   }
   for (int t0 = 0; t0 < count; t0 += GLA_TB) {
     const int nt = count - t0 < GLA_TB ? count - t0 : GLA_TB;
-    if (MODE == 0) ask(t0);
+    if (!AHEAD) ask(t0);
     __syncthreads();                                  // the block before is read to its end
 #pragma unroll
     for (int l = 0; l < PLACES; ++l) {
@@ -154,7 +155,7 @@ __global__ __launch_bounds__(256) void gla_scan_kernel(
       ks[i] = form == 1 ? __uint_as_float(k_next[l]) : gla_value<T>(k_next[l]);
     }
     if (tid < nt * CW) vs[tid] = v_c < vdim ? to_float(v_next) : 0.f;
-    if (MODE != 0 && t0 + GLA_TB < count) ask(t0 + GLA_TB);
+    if (AHEAD && t0 + GLA_TB < count) ask(t0 + GLA_TB);
     __syncthreads();
     for (int t = 0; t < nt; ++t) {
       float v[SL], acc[SL];
