@@ -58,7 +58,9 @@ template <> __device__ __forceinline__ void store_out<uint16_t>(uint16_t* p, flo
 // TILED: W is the copy that tile_weight_kernel lays out, in which the 64 rows x 256 values that a workgroup
 // multiplies with in one chunk are 32 KB of consecutive memory, chunk after chunk: every workgroup then reads one
 // stretch of memory front to back, where the rows of the matrix as the file holds it lie K values apart.
-template <int MT, bool GLU, typename TO, int KC, bool TILED>
+// PAIRS: the rounds written out in pairs (see the top of the file); else one after the other, with the next chunk's W copied
+// over this one's (rounds_alone says where).  The sums and their order are the same.
+template <int MT, bool GLU, typename TO, int KC, bool TILED, bool PAIRS>
 __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16_t* __restrict__ X,
                                                                     const uint16_t* __restrict__ W,
                                                                     TO* __restrict__ C, float* __restrict__ part,
@@ -96,7 +98,7 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16
   constexpr int XPIECES = MT * 16 * (KC / 8);
   constexpr int XPT = XPIECES / (SK_WAVES * 64);
   static_assert(XPIECES % (SK_WAVES * 64) == 0, "pieces of X must divide over the threads");
-  // No load stands under a condition: behind one that some lanes, or some rounds, skip the compiler can no longer count
+  // With PAIRS no load stands under a condition: behind one that some lanes, or some rounds, skip the compiler can no longer count
   // which loads are still under way and waits for all of them.  Pieces beyond K are read from the last valid place and
   // cleared: X on its way to LDS, W in front of the products of that chunk.
   uint4 xreg[XPT];
@@ -105,7 +107,10 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16
     for (int i = 0; i < XPT; ++i) {
       const int pc = tid + i * SK_WAVES * 64;
       const int row = pc / (KC / 8), kk = (pc % (KC / 8)) * 8;
-      xreg[i] = *reinterpret_cast<const uint4*>(X + (size_t)min(row, M - 1) * K + min(c * KC + kk, K - 8));
+      const int k = c * KC + kk;
+      const uint16_t* x_row = X + (size_t)min(row, M - 1) * K;
+      if (PAIRS) xreg[i] = *reinterpret_cast<const uint4*>(x_row + min(k, K - 8));
+      else xreg[i] = k < K ? *reinterpret_cast<const uint4*>(x_row + k) : make_uint4(0u, 0u, 0u, 0u);
     }
   };
   auto store_x = [&](int buf, int c) {
@@ -113,7 +118,7 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16
     for (int i = 0; i < XPT; ++i) {
       const int pc = tid + i * SK_WAVES * 64;
       const int row = pc / (KC / 8), kk = (pc % (KC / 8)) * 8;
-      const bool in = c * KC + kk < K;
+      const bool in = !PAIRS || c * KC + kk < K;
       *reinterpret_cast<uint4*>(&xs[buf][row][kk]) =
           make_uint4(in ? xreg[i].x : 0u, in ? xreg[i].y : 0u, in ? xreg[i].z : 0u, in ? xreg[i].w : 0u);
     }
@@ -127,7 +132,11 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16
       return;
     }
 #pragma unroll
-    for (int i = 0; i < NLD; ++i) dst[i] = load_stream_16(wrow + min(c * KC + (i * 4 + q) * 8, K - 8));
+    for (int i = 0; i < NLD; ++i) {
+      const int k = c * KC + (i * 4 + q) * 8;
+      if (PAIRS) dst[i] = load_stream_16(wrow + min(k, K - 8));
+      else dst[i] = k < K ? load_stream_16(wrow + k) : make_uint4(0u, 0u, 0u, 0u);
+    }
   };
 
   // Workgroups that walk K in step read rows of W one row's length apart at the same moment, and such addresses
@@ -144,7 +153,7 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16
     const int k = c + rot;
     return k >= c1 ? k - span : k;
   };
-  const bool ragged = !TILED && K % KC != 0;
+  const bool ragged = PAIRS && !TILED && K % KC != 0;
   auto products = [&](int c, uint4 (&w)[NLD]) {
     const int buf = (c - c0) & 1;
     if (ragged && ce(c) == nchunks - 1) {
@@ -172,7 +181,27 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16
     store_x((c - c0 + 1) & 1, ce(c + 1));
     __syncthreads();
   };
-  if (c0 < c1) {
+  if (!PAIRS && c0 < c1) {
+    load_x(ce(c0));
+    load_w(ce(c0), w0);
+    store_x(0, ce(c0));
+    __syncthreads();
+    for (int c = c0; c < c1; ++c) {
+      const bool more = c + 1 < c1;
+      if (more) {
+        load_x(ce(c + 1));
+        load_w(ce(c + 1), w1);
+      }
+      products(c, w0);
+      if (more) {
+        store_x((c - c0 + 1) & 1, ce(c + 1));
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) w0[i] = w1[i];
+      }
+      __syncthreads();
+    }
+  }
+  if (PAIRS && c0 < c1) {
     load_x(ce(c0));
     load_w(ce(c0), w0);
     store_x(0, ce(c0));
@@ -379,20 +408,40 @@ extern "C" int ia_gemm_skinny_set_splits(int N, int K, int splits) {
 // Number of K splits the kernel uses for a weight [N, K] (a function of N and K only).
 extern "C" int ia_gemm_skinny_splits(int N, int K) { return (N > 0 && K > 0) ? skinny_splits(N, K) : 0; }
 
-template <int MT, bool GLU, typename TO, int KC, bool TILED>
+template <int MT, bool GLU, typename TO, int KC, bool TILED, bool PAIRS = true>
 static int launch_skinny_one(dim3 grid, const uint16_t* x, const uint16_t* w, TO* c, float* part, int M, int N, int K,
                              int cps, hipStream_t stream) {
   constexpr size_t lds = (size_t)2 * MT * 16 * (KC + SK_XPAD) * sizeof(uint16_t);
   static bool allowed = false;      // more than 64 KB of LDS has to be asked for, once per kernel
   if (lds > 65536 && !allowed) {
-    hipError_t e = hipFuncSetAttribute((const void*)gemm_skinny_kernel<MT, GLU, TO, KC, TILED>,
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_skinny_kernel<MT, GLU, TO, KC, TILED, PAIRS>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return (int)e;
     allowed = true;
   }
-  gemm_skinny_kernel<MT, GLU, TO, KC, TILED><<<grid, SK_WAVES * 64, lds, stream>>>(x, w, c, part, M, N, K, cps);
+  gemm_skinny_kernel<MT, GLU, TO, KC, TILED, PAIRS><<<grid, SK_WAVES * 64, lds, stream>>>(x, w, c, part, M, N, K, cps);
   IA_LAUNCH_CHECK();
   return IA_OK;
+}
+
+// Whether the rounds run one after the other instead of in pairs.  Where one workgroup has a compute unit to itself pairs are 15
+// to 30 % faster from 33 rows on, and with many in turn 0 to 13; with two side by side and no third, each covers the other's waits,
+// and the registers and selects of the unconditional loads cost more than they give at some numbers of tiles of 16 rows (MT).
+// Microseconds one after the other / in pairs: 28,672 x 4,096 with the activation from its copy, 33 / 48 / 64 / 128 rows 47.6 /
+// 50.8 / 54.3 / 73.3 against 51.1 / 53.0 / 55.4 / 75.5; 32,000 x 2,048 at 33 / 64 rows 27.8 / 32.1 against 29.3 / 33.6; at 112 rows
+// every shape without a copy (24,000 x 2,048, 20,480 x 2,560, 28,672 x 4,096 with the activation) 1.03 to 1.05 of the time in pairs.
+// Not so: 20,480 x 2,560 (320 workgroups) at 33 to 64 rows 0.93 to 0.97, copies at 65 to 80 rows 0.86 to 0.92.  With more
+// workgroups: short walks over K at 49 to 64 rows (50,257 x 2,048 55 against 57.5, 65,536 x 2,048 1.03; 36,864 x 4,096 0.92); and at 81
+// to 96 rows, where the rounds alone leave a compute unit the registers for a third workgroup and pairs do not, up to three
+// workgroups a unit of a few chunks each (12,288 / 13,312 / 14,336 x 4,096 in three parts 36.2 / 36.7 / 37.2 against 38.0 / 39.9 /
+// 40.5; with eight chunks and more 0.94 to 0.96, with two or three 0.95 to 0.99).
+static bool rounds_alone(int MT, bool tiled, unsigned groups, unsigned splits, int chunks) {
+  if (MT == 4 && splits == 1 && chunks <= 8 && groups > 360) return true;
+  if (MT == 6) return splits > 1 && groups > 560 && groups <= 3 * SK_ENOUGH_BLOCKS && chunks >= 4 && chunks <= 6;
+  if (groups <= SK_ENOUGH_BLOCKS || groups > 2 * SK_ENOUGH_BLOCKS) return false;
+  if (MT == 3) return splits == 1 ? tiled || groups > 360 : splits >= 4 && chunks >= 8;  // (8,192 x 8,192: 1.03; 15,360 x 5,120 in two parts 0.97)
+  if (MT == 4) return splits == 1 && groups > 360;
+  return (MT == 7 && !tiled) || (MT == 8 && tiled);
 }
 
 template <bool GLU, typename TO, bool TILED = false>
@@ -409,6 +458,7 @@ static int launch_skinny(const uint16_t* x, const uint16_t* w, TO* c, float* par
   // (the 1B shape's gate+up 14.5 against 15.4), and so do heads of many workgroups (128,256 x 2,048 91.5 against 92.8).
   const unsigned groups = grid.x * grid.y;
   const bool shorter = grid.y > 1 || (groups > SK_ENOUGH_BLOCKS && groups <= 4 * SK_ENOUGH_BLOCKS);
+  const bool alone = rounds_alone((M + 15) / 16, TILED, groups, grid.y, cps);
   switch ((M + 15) / 16) {
     case 1:
       if (shorter) return launch_skinny_one<1, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
@@ -416,13 +466,23 @@ static int launch_skinny(const uint16_t* x, const uint16_t* w, TO* c, float* par
     case 2:
       if (shorter) return launch_skinny_one<2, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
       return launch_skinny_one<2, GLU, TO, SK_KC, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
-    case 3: return launch_skinny_one<3, GLU, TO, SK_KC, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
-    case 4: return launch_skinny_one<4, GLU, TO, SK_KC, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
+    case 3:
+      if (alone) return launch_skinny_one<3, GLU, TO, SK_KC, TILED, false>(grid, x, w, c, part, M, N, K, cps, stream);
+      return launch_skinny_one<3, GLU, TO, SK_KC, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
+    case 4:
+      if (alone) return launch_skinny_one<4, GLU, TO, SK_KC, TILED, false>(grid, x, w, c, part, M, N, K, cps, stream);
+      return launch_skinny_one<4, GLU, TO, SK_KC, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
     // above 64 rows: pieces of 128, so that the two stages of X of two workgroups fit a compute unit's LDS
     case 5: return launch_skinny_one<5, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
-    case 6: return launch_skinny_one<6, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
-    case 7: return launch_skinny_one<7, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
-    case 8: return launch_skinny_one<8, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
+    case 6:
+      if (alone) return launch_skinny_one<6, GLU, TO, SK_KC / 2, TILED, false>(grid, x, w, c, part, M, N, K, cps, stream);
+      return launch_skinny_one<6, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
+    case 7:
+      if (alone) return launch_skinny_one<7, GLU, TO, SK_KC / 2, TILED, false>(grid, x, w, c, part, M, N, K, cps, stream);
+      return launch_skinny_one<7, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
+    case 8:
+      if (alone) return launch_skinny_one<8, GLU, TO, SK_KC / 2, TILED, false>(grid, x, w, c, part, M, N, K, cps, stream);
+      return launch_skinny_one<8, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
     default: return IA_ERR_UNSUPPORTED;
   }
 }

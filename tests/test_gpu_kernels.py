@@ -421,6 +421,25 @@ def test_gemm_skinny_rounds_in_pairs(M, N, K_):
     assert ((got - want).abs() <= K_ * 2 ** -24 * size + 1e-30).all()
 
 
+# rounds one after the other (257 to 512 workgroups: 361 and more without a copy up to 64 rows, all copies at 33 to 48 and from 113
+# rows on, all without a copy at 97 to 112; parts of eight chunks and more at 33 to 48 rows) leave the bits that a row has alone;
+# a last chunk that is not full
+@pytest.mark.parametrize("M", [33, 48, 49, 64, 97, 112, 113, 128])
+@pytest.mark.parametrize("N,K_,tiled", [(23200, 520, False), (16500, 776, False), (19300, 776, True), (28670, 264, True), (8190, 7944, False)])
+def test_gemm_skinny_rounds_one_after_the_other(M, N, K_, tiled):
+    api = K()
+    a, w = _rand(M, K_, dtype=torch.bfloat16, seed=23), _rand(N, K_, dtype=torch.bfloat16, scale=0.05, seed=24)
+    kw = dict(epilogue="swiglu", tiled=api.tile_weight(w, "swiglu")) if tiled else dict(out_dtype=torch.float32)
+    if not tiled and api.gemm_skinny_splits(N, K_) > 1:
+        got = api.gemm_skinny(a, w, keep_split=True).parts
+        for m in (0, 31, 32, M - 1):
+            assert torch.equal(got[:, m:m + 1], api.gemm_skinny(a[m:m + 1], w, keep_split=True).parts)
+    else:
+        got = api.gemm_skinny(a, w, **kw)
+        for m in (0, 31, 32, M - 1):
+            assert torch.equal(got[m:m + 1], api.gemm_skinny(a[m:m + 1], w, **kw))
+
+
 # one workgroup with all of K against the parts and their sum in the order of their index: columns that fill no group of
 # 16, a last chunk that is not full, one to sixteen parts, two chunks and more a part, both halves of [gate | up]
 @pytest.mark.parametrize("M", [1, 5, 16])
