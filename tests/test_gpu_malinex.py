@@ -265,7 +265,9 @@ def test_gated_linear_attention_alone(dtype, m, W, T):
 
 
 @BOTH
-@pytest.mark.parametrize("nh,dim,vdim,tau", [(2, 16, 32, 8.0), (3, 10, 24, 1.0), (1, 128, 128, 16.0), (2, 40, 16, 0.25)])
+# the last four: 512 workgroups and more of two slices each, by the key channels a thread keeps (4, 8, 16), a last slice not full; 32
+@pytest.mark.parametrize("nh,dim,vdim,tau", [(2, 16, 32, 8.0), (3, 10, 24, 1.0), (1, 128, 128, 16.0), (2, 40, 16, 0.25), (16, 40, 120, 0.25),
+                                             (16, 128, 128, 16.0), (8, 200, 120, 1.0), (1, 300, 32, 4.0)])
 def test_the_recurrence_in_tiles_against_the_recurrence_token_after_token(dtype, nh, dim, vdim, tau):
     """Requests of 1 to 300 rows whose ends fall on, before and behind the edges of the tiles, through slots out of
     order that hold earlier states, the tiles listed in any order: the tiles side by side give the rows and the final states of the walk token after

@@ -404,6 +404,30 @@ def test_window_and_blocks_on_the_matrix_cores_against_the_plain_kernel(nh, nkv,
         assert rel_err(got, want.double().cpu()) <= 3e-2
 
 
+# decays and keys given: two slices a workgroup (512 of them and more) by the key channels a thread keeps, a last slice not full
+@BOTH
+@pytest.mark.parametrize("nh,dim,vdim", [(16, 40, 120), (16, 128, 128), (8, 200, 120)])
+def test_hgrn2_in_tiles_against_token_after_token(dtype, nh, dim, vdim):
+    from infernum_amd.kernels import api as K
+    rt = runtime(dtype)
+    g = torch.Generator().manual_seed(dim)
+    lens = [63, 64, 65, 1, 128, 129, 300, 2]
+    N, B, floats = sum(lens), len(lens), K.gla_state_floats(nh, dim, vdim)
+    proj = torch.randn(N, nh * (dim + vdim), generator=g).to(DEV).to(rt.dtype)
+    k = torch.sigmoid(torch.randn(N, nh * dim, generator=g) - 3).to(DEV)
+    f = 1 - k
+    slots = torch.tensor([5, 0, 7, 2, 9, 1, 3, 8], dtype=torch.int32, device=DEV)
+    starts = torch.tensor([sum(lens[:i]) for i in range(B + 1)], dtype=torch.int32, device=DEV)
+    tiles = torch.tensor([(b, r) for b, n in enumerate(lens) for r in range(0, n, K.PREFILL_TILE_ROWS)], dtype=torch.int32).to(DEV)
+    state = torch.randn(10, floats, generator=g).to(DEV)
+    s_want, s_got = state.clone(), state.clone()
+    want, got = torch.empty(N, nh * vdim, device=DEV), torch.full((N, nh * vdim), 7.0, device=DEV)
+    K.hgrn2_scan(proj, 0, nh * dim, f, k, s_want, want, starts, slots, nh, dim, vdim)
+    K.hgrn2_chunked(proj, 0, nh * dim, f, k, s_got, got, starts, slots, tiles, tiles.shape[0], 0, nh, dim, vdim)
+    assert rel_err(got, want.cpu()) <= 2e-5 and rel_err(s_got, s_want.cpu()) <= 2e-5
+    assert torch.equal(s_got[4], state[4]) and torch.equal(s_got[6], state[6])           # slots of no request
+
+
 HGRN_CASES = [(SM.S1["layers"][2]["mixer"], 64, 150), (SM.S2["layers"][3]["mixer"], 100, 70), (SM.S3["layers"][1]["mixer"], 128, 131),
               (SM.S4["layers"][1]["mixer"], 80, 64)]
 
