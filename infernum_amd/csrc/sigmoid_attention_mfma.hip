@@ -21,6 +21,7 @@
 // Values of keys that no column of the tile sees are zeroed after the load and their weights are zero: a stale or
 // poisoned page never leaks in.  A key that is needed but has no page in the block table gives NaN, not a fault.
 #include "common.h"
+#include "parts_join.h"
 
 #ifndef SA_DIM
 #error "compile with -DSA_DIM=<key size> -DSA_VDIM=<value size>"
@@ -206,8 +207,10 @@ __global__ __launch_bounds__(256) void sigattn_decode_kernel(
   }
 }
 
-// grid (B, nh), 64 threads: the parts of a token's head added in their order, gated, rounded once.
-// grid (B, nh, 64 channels each); sixteen parts' loads in flight (one after the other: 17 us for 32 parts, so 4.1)
+// grid (B, nh, channels / 64), 64 threads: the parts of a token's head added in their order, gated, rounded once.
+// PRE parts' loads in flight, as joined_at_once says (one after the other: 17 us for 32 parts, with sixteen 4.1; sixteen loads
+// for two parts cost 64 tokens of 16 heads of 128 with 65 keys 0.7 of 7.1 us).
+template <int PRE>
 __global__ __launch_bounds__(64) void sigattn_join_kernel(const float* __restrict__ part, const uint16_t* __restrict__ gate,
                                                           int gate_stride, uint16_t* __restrict__ out, int nh, int parts) {
   const int b = blockIdx.x, h = blockIdx.y, c = blockIdx.z * 64 + threadIdx.x, cc = min(c, SA_VDIM - 1);
@@ -215,12 +218,12 @@ __global__ __launch_bounds__(64) void sigattn_join_kernel(const float* __restric
   const float* from = part + ((size_t)b * parts * nh + h) * SA_VDIM + cc;
   const size_t step = (size_t)nh * SA_VDIM;
   float acc = 0.f;
-  for (int z0 = 0; z0 < parts; z0 += 16) {
-    float v[16];
+  for (int z0 = 0; z0 < parts; z0 += PRE) {
+    float v[PRE];
 #pragma unroll
-    for (int z = 0; z < 16; ++z) v[z] = from[min(z0 + z, parts - 1) * step];
+    for (int z = 0; z < PRE; ++z) v[z] = from[min(z0 + z, parts - 1) * step];
 #pragma unroll
-    for (int z = 0; z < 16; ++z) acc = z0 + z < parts ? acc + v[z] : acc;
+    for (int z = 0; z < PRE; ++z) acc = z0 + z < parts ? acc + v[z] : acc;
   }
   if (c < SA_VDIM) out[((size_t)b * nh + h) * SA_VDIM + c] = float_to_bf16_bits(acc * gt);
 }
@@ -314,8 +317,14 @@ extern "C" int ia_sigattn_decode(const void* q, int q_stride, const void* k_page
 #undef SA_DEC
   IA_LAUNCH_CHECK();
   if (parts > 1) {
-    sigattn_join_kernel<<<dim3(B, nh, (SA_VDIM + 63) / 64), 64, 0, stream>>>(part, (const uint16_t*)gate, gate_stride, (uint16_t*)out, nh,
-                                                        parts);
+    const dim3 heads(B, nh, (SA_VDIM + 63) / 64);
+    const int pre = joined_at_once(parts);
+    if (pre == 2)
+      sigattn_join_kernel<2><<<heads, 64, 0, stream>>>(part, (const uint16_t*)gate, gate_stride, (uint16_t*)out, nh, parts);
+    else if (pre == 4)
+      sigattn_join_kernel<4><<<heads, 64, 0, stream>>>(part, (const uint16_t*)gate, gate_stride, (uint16_t*)out, nh, parts);
+    else
+      sigattn_join_kernel<16><<<heads, 64, 0, stream>>>(part, (const uint16_t*)gate, gate_stride, (uint16_t*)out, nh, parts);
     IA_LAUNCH_CHECK();
   }
   return IA_OK;

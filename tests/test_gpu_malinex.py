@@ -379,7 +379,7 @@ def test_sigmoid_attention_alone(dtype, m, W, T, ps):
 @pytest.mark.parametrize("nh,nkv,dim,vdim,ps", [(4, 2, 16, 32, 4), (20, 1, 32, 64, 12), (3, 3, 48, 16, 16), (8, 2, 128, 64, 8),
                                                 (2, 1, 128, 128, 20)])
 def test_sigmoid_attention_on_the_matrix_cores_against_the_plain_kernel(nh, nkv, dim, vdim, ps):
-    """The kernels for single tokens (whole, and with the keys cut into 2, 5 and 64 parts) and for portions of
+    """The kernels for single tokens (whole, and with the keys cut into 2, 3, 5 and 64 parts) and for portions of
     prompts (rows of 1 to 150 behind 0 to 130 keys) give what the plain kernel gives on the same pages, of sizes that
     are and are not powers of two; places of the pages that no request holds are NaN."""
     from infernum_amd.kernels import api as K
@@ -416,7 +416,7 @@ def test_sigmoid_attention_on_the_matrix_cores_against_the_plain_kernel(nh, nkv,
     k32, v32 = k.float(), v.float()                          # the plain kernel on the same values, in 32-bit throughout
     K.sigattn_generic(q.float(), k32, v32, gate.float(), want, seq, pos, bt, r1, r2, pb, nh, nkv, dim, vdim, scale)
     assert torch.isfinite(want).all()
-    for parts in (1, 2, 5, 64, None):
+    for parts in (1, 2, 3, 5, 64, None):
         got.fill_(7.0)
         K.sigattn_decode(q, k, v, gate, got, pos, bt, r1, r2, pb, nh, nkv, dim, vdim, scale, max(lens), parts)
         assert rel_err(got, want.float().cpu()) <= PART_TOL["bfloat16"], parts
