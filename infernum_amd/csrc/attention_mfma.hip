@@ -307,7 +307,8 @@ struct DecFused {
 // FUSED: q is not read; every workgroup rotates the queries of its heads into LDS, the workgroups whose keys
 // include the token's own also make its key and value, use them from LDS (the loads from the page are replaced
 // in registers) and one of them (the first tile of heads) writes them to the page.
-template <bool FUSED, typename TS, bool POW2, int WAVES>
+// EARLY (FUSED): what lies behind a head's rotated part is asked for before the rotation, see below.
+template <bool FUSED, typename TS, bool POW2, int WAVES, bool EARLY = true>
 __global__ __launch_bounds__(WAVES * 64, ((WAVES == 4 && IA_MAX_DIM <= 128) ? 3 : 1)) void attn_decode_kernel(
     const uint16_t* __restrict__ q, int q_row_stride, uint16_t* k_pages, uint16_t* v_pages,
     uint16_t* __restrict__ out, int out_row_stride, float* __restrict__ part_o, float* __restrict__ part_ml,
@@ -338,9 +339,11 @@ __global__ __launch_bounds__(WAVES * 64, ((WAVES == 4 && IA_MAX_DIM <= 128) ? 3 
   const int half = FUSED ? F.rot >> 1 : 0;
   const TS* row = reinterpret_cast<const TS*>(F.src) + (size_t)b * F.row_stride;
   // what lies behind the rotated part of a head (a latent's row: 224 of 256 values) is copied: eight values an access where
-  // the rows allow it, asked for here too (one value after the other behind the rotation took 7 of 18 us for one token)
+  // the rows allow it, asked for here too (one value after the other behind the rotation took 7 of 18 us for one token);
+  // where that is one value for some of the threads, as it is needed (8 heads of 96 with 48 rotated, each on its own
+  // keys, 8 / 64 tokens 7.9 / 8.8 us, early 8.3 / 9.3)
   constexpr int CPT = (16 * HD / 8 + NT - 1) / NT;
-  const bool has_tail = FUSED && F.rot < HD;
+  const bool has_tail = FUSED && EARLY && F.rot < HD;
   const int tail8 = (HD - F.rot) >> 3;
   const bool copy8 = has_tail && sizeof(TS) == 2 && F.gsplits == 1 && (F.rot & 7) == 0 && (F.row_stride & 7) == 0 &&
                      (reinterpret_cast<uintptr_t>(F.src) & 15) == 0;
@@ -473,7 +476,7 @@ __global__ __launch_bounds__(WAVES * 64, ((WAVES == 4 && IA_MAX_DIM <= 128) ? 3 
           *reinterpret_cast<uint4*>(&s_q[c][F.rot + 8 * (idx - c * tail8)]) = qc[u];
         }
       }
-    } else if (has_tail) {
+    } else if (has_tail || !EARLY) {
       const int tail = HD - F.rot;
       for (int idx = tid; idx < heads_here * tail; idx += NT) {
         const int c = idx / tail, i = F.rot + (idx - c * tail);
@@ -488,7 +491,12 @@ __global__ __launch_bounds__(WAVES * 64, ((WAVES == 4 && IA_MAX_DIM <= 128) ? 3 
         s_newk[tid] = float_to_bf16_bits(lo);
         s_newk[tid + half] = float_to_bf16_bits(hi);
       }
-      if (F.rot + tid < HD) s_newk[F.rot + tid] = float_to_bf16_bits(kc);
+      if constexpr (EARLY) {
+        if (F.rot + tid < HD) s_newk[F.rot + tid] = float_to_bf16_bits(kc);
+      } else {
+        for (int i = F.rot + tid; i < HD; i += NT)
+          s_newk[i] = float_to_bf16_bits(load_split_sum(row + (size_t)(nh + g) * HD + i, F.gsplits, F.split_stride));
+      }
       if (tid < VD) s_newv[tid] = float_to_bf16_bits(vv);
       geo.patch_key = p;
     }
@@ -1130,22 +1138,25 @@ extern "C" int ia_attn_decode_fused(const void* src, int src_dtype, int src_spli
   F.freq_f64 = freq_f64;
   F.rot = rot;
   dim3 grid(B, nkv * HT, num_splits);
-#define DEC_FUSED_LAUNCH(TS, P2, W)                                                                                 \
-  attn_decode_kernel<true, TS, P2, W><<<grid, W * 64, 0, stream>>>(                                                 \
+#define DEC_FUSED_LAUNCH(TS, P2, W, EARLY)                                                                          \
+  attn_decode_kernel<true, TS, P2, W, EARLY><<<grid, W * 64, 0, stream>>>(                                                 \
       nullptr, 0, (uint16_t*)k_pages, (uint16_t*)v_pages, (uint16_t*)out, out_row_stride, part_o, part_ml, positions, \
       block_tables, bt_stride, nh, nkv, ps, num_pages, scale_log2, window, num_splits, F, sinks, X)
-#define DEC_FUSED_WAVES(TS, P2)                       \
-  do {                                                \
-    if (wide) DEC_FUSED_LAUNCH(TS, P2, DEC_WAVES_FEW); \
-    else DEC_FUSED_LAUNCH(TS, P2, DEC_WAVES);         \
+#define DEC_FUSED_WAVES(TS, P2, EARLY)                       \
+  do {                                                       \
+    if (wide) DEC_FUSED_LAUNCH(TS, P2, DEC_WAVES_FEW, EARLY); \
+    else DEC_FUSED_LAUNCH(TS, P2, DEC_WAVES, EARLY);         \
   } while (0)
   const bool pow2 = (ps & (ps - 1)) == 0, wide = dec_wide(B, nkv * HT, num_splits);
   if (src_dtype == IA_F32) {
-    if (pow2) DEC_FUSED_WAVES(float, true);
-    else DEC_FUSED_WAVES(float, false);
+    if (pow2) DEC_FUSED_WAVES(float, true, true);
+    else DEC_FUSED_WAVES(float, false, true);
+  } else if (rot < HD && G * (HD - rot) <= 64) {
+    if (pow2) DEC_FUSED_WAVES(bf16_t, true, false);
+    else DEC_FUSED_WAVES(bf16_t, false, false);
   } else {
-    if (pow2) DEC_FUSED_WAVES(bf16_t, true);
-    else DEC_FUSED_WAVES(bf16_t, false);
+    if (pow2) DEC_FUSED_WAVES(bf16_t, true, true);
+    else DEC_FUSED_WAVES(bf16_t, false, true);
   }
 #undef DEC_FUSED_WAVES
 #undef DEC_FUSED_LAUNCH

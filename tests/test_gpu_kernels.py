@@ -1157,7 +1157,10 @@ def test_attention_mfma_decode(nh, nkv, d, ps, window, splits):
 @pytest.mark.parametrize("nh,nkv,d,ps,window,rot", [(8, 2, 128, 16, 0, 128), (6, 3, 48, 4, 0, 48), (32, 8, 128, 16, 0, 128),
                                                     (40, 2, 64, 8, 0, 32), (5, 5, 16, 16, 0, 0), (2, 1, 256, 64, 0, 256),
                                                     (8, 2, 128, 16, 100, 128), (4, 1, 96, 4, 17, 96),
-                                                    (3, 1, 80, 12, 0, 80), (6, 2, 64, 20, 33, 64)])   # pages: no power of two
+                                                    (3, 1, 80, 12, 0, 80), (6, 2, 64, 20, 33, 64),    # pages: no power of two
+                                                    # behind the rotated part: 48 and 64 values in all, more, many heads of many
+                                                    (3, 3, 96, 16, 0, 48), (2, 2, 64, 4, 0, 0), (4, 1, 80, 16, 0, 62),
+                                                    (6, 1, 256, 4, 0, 30), (16, 1, 256, 16, 0, 32)])
 def test_attention_decode_rotating_equals_rotation_then_attention(nh, nkv, d, ps, window, rot, splits, gemm_splits):
     """One launch for rotation, write to the pages and attention against the two kernels one after the other:
     the same attention output and the same pages, bit for bit.  The QKV product comes as bf16 rows
