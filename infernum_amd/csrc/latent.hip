@@ -133,7 +133,7 @@ __global__ __launch_bounds__(256) void gemm_heads_big_kernel(const bf16_t* __res
 // The same for few rows (decoding), without LDS: bound by one trip to memory.  A wave takes 16 columns of one head for up to
 // 16 rows of x and asks for eight steps of 32 values of K of both at once, none under a condition (pieces beyond K are read
 // from the last place and cleared); the sums are those of the tiles above, step by step in the same order.  Grid (tiles of
-// 64 of Nout, tiles of 16 of N, H).  One row, 16 heads: 224 x 64 3.9 us with the tiles and 2.4 so, 64 x 224 with
+// 64 of Nout, 1, H).  One row, 16 heads: 224 x 64 3.9 us with the tiles and 2.4 so, 64 x 224 with
 // a gate 6.7 and 4.4, 128 x 512 with a gate 9.8 and 7.5; 16 rows 3.9 and 2.6, 6.8 and 4.0, 8.7 and 7.8.
 #define GH_FEW_ROWS 16
 __global__ __launch_bounds__(256) void gemm_heads_few_kernel(const bf16_t* __restrict__ x, int x_row, int x_head,
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(256) void gemm_heads_few_kernel(const bf16_t* __res
                                                              int g_row, int N, int Nout, int K) {
   constexpr int PIECE = 8;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
-  const int h = blockIdx.z, n0 = (blockIdx.x * 4 + wave) * 16, m = blockIdx.y * GH_FEW_ROWS + r, mc = min(m, N - 1);
+  const int h = blockIdx.z, n0 = (blockIdx.x * 4 + wave) * 16, m = r, mc = min(m, N - 1);
   if (n0 >= Nout) return;
   const bf16_t* w_row = W + ((size_t)h * Nout + min(n0 + r, Nout - 1)) * K;
   const bf16_t* x_row_ = x + (size_t)mc * x_row + (size_t)h * x_head;

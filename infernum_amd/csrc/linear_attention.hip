@@ -366,8 +366,8 @@ static int gla_chunked_launch(const void* proj, int code, int proj_stride, int q
     return sizeof(float) * ((size_t)3 * GLA_TB * dim + (size_t)GLA_TB * sl * GLA_PW + (size_t)GLA_TB * GLA_PARTS * sl * GLA_PW);
   };
   if (lds_of(1) > 64 * 1024) return IA_ERR_UNSUPPORTED;
-  // two slices a workgroup while that leaves two workgroups a compute unit (even at 400 rows of 16 heads of 128, 448
-  // workgroups of one slice: 85 us with one), and up to 16 channels a thread (two states of more
+  // two slices a workgroup while that leaves two workgroups a compute unit (400 rows of 16 heads of 128, 896 workgroups of one
+  // slice and 448 of two, take 84 us with one; 700 rows, 704 of two, 92 against 130 before either change), and up to 16 channels a thread (two states of more
   // leave room for one wave on a SIMD)
   const bool pairs = slices % 2 == 0 && per <= 16 && (long)nh * num_tiles * (slices / 2) >= GLA_PAIRS_FROM;
   const dim3 grid((unsigned)nh, (unsigned)num_tiles, (unsigned)(pairs ? slices / 2 : slices));

@@ -53,6 +53,9 @@ SKINNY_WIDE = 16384
 # that go to the library, for 17 to 128 rows.  Measured with ``measure_route`` on an MI355X, three times over, a
 # bit kept where most runs agreed; the shapes are those of the Llama 1B, 8B, 13B and 70B layers.  The library's
 # kernels are ahead for some shapes already at 32 rows and behind for others at 128, and no rule of sizes tells.
+# (Measured before the weight-streaming kernel asked for a chunk ahead without conditions; it has gained since, most where
+# its workgroups have a compute unit each: 16,384 x 2,048 with the activation at 32 / 64 / 128 rows 20 / 23 / 32 us then and
+# 16 / 18 / 25 now.)
 KNOWN_ROUTES: Dict[Tuple[int, int, Optional[str], bool], int] = {
     (3072, 2048, None, True): 0, (2048, 2048, None, True): 0, (16384, 2048, "swiglu", False): 0b11110010,
     (2048, 8192, None, True): 0,
@@ -76,8 +79,9 @@ KNOWN_ROUTES: Dict[Tuple[int, int, Optional[str], bool], int] = {
 # against 34.  The 8B shape's decode step at 160 / 192 / 256 requests: 19.8k / 21.4k / 24.3k tokens/s against 15.7k /
 # 16.3k / 21.7k with the library's products.
 # Up to 128 rows, against the weight-streaming kernel (or the library where KNOWN_ROUTES has it), at 32 / 64 / 128
-# rows: the 8B shape's down projection 25 / 26 / 30 against 29 / 32 / 40, its QKV product 13 / 14 / 17 against 15 / 17 /
-# 24, its output projection 10.5 / 11.5 / 14 against 10 / 12 / 15.5; the 13B shape's down projection 28 / 30 / 34
+# rows: the 8B shape's down projection 25 / 26 / 30 against 29 / 32 / 40 (since that kernel asks for a chunk ahead without
+# conditions 25 / 30 / 37), its QKV product 13 / 14 / 17 against 15 / 17 / 24 (14 / 16 / 21), its output projection 10.5 / 11.5 / 14
+# against 10 / 12 / 15.5 (9.3 / 11.4 / 15); the 13B shape's down projection 28 / 30 / 34
 # against 33 / 37 / 46, its output projection 14 / 16 / 19 against 16 / 19 / 23; the 70B shape's down projection 84 /
 # 90 / 105 against 94 / 111 / 139, its QKV product 36 / 35 / 39 against 38 / 41 / 52.  The 8B shape's decode step at 32 / 64 / 128 requests: 7.34k / 11.93k / 17.84k tokens/s
 # against 7.08k / 11.52k / 17.03k.  A band begins where the tiled kernel was ahead; a shape whose product came out
