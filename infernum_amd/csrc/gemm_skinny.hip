@@ -349,23 +349,28 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_whole_kernel(const uin
   }
 }
 
-// Whether the kernel above takes a split product whose parts are wanted joined.  Microseconds on an MI355X in a chain of
-// products with cold weights, the split product with its join against this kernel: 2,048 x 2,048 at 1 / 8 / 16 rows 6.2 /
-// 6.4 / 6.7 against 5.4 / 6.1 / 6.9, 3,072 x 2,048 7.3 / 7.4 / 7.9 against 5.7 / 6.3 / 7.2, 4,096 x 4,096 at 1 / 8 / 12 rows
-// 10.6 / 10.4 / 10.6 against 9.2 / 10.0 / 10.6, 12,288 x 4,096 24.1 / 24.7 / 25.3 against 21.3 / 23.2 / 25.4.  It loses where
-// the reads of X weigh more than a launch: 10,304 x 2,048 at 12 rows (13.1 against 13.8; at 8 12.8 and 12.7), 4,096 x 8,192
-// (15.9 against 17.0; at 8 16.0 and 15.6); where the chunks do not deal out evenly over more than four waves, which
-// then wait for the longest (6,144 x 4,096 at 1 row 14.0 against 14.5); with more than eight waves (2,048 x 4,096 at 4 rows
-// 8.0 against 8.6); and with few workgroups (256 x 2,048 at 8 rows 5.1 against 5.4).  With both halves it reads X twice:
-// 5,632 x 2,048 at 8 / 12 rows 9.8 / 10.0 against 9.7 / 10.3, 11,008 x 2,048 at 2 / 8 rows 14.4 / 14.4 against 13.7 / 15.9,
-// 9,472 x 4,096 behind at every number of rows.
+// Whether the kernel above takes a split product whose parts are wanted joined.  Measured on an MI355X in a chain of products
+// with cold weights over N of 512 to 15,360 and K of 1,024 to 13,824, at 1 to 16 rows: the time of this kernel over that of the
+// split product with its join.  It gains a launch (2,048 x 2,048 at 1 / 8 rows 0.88 / 0.96, 4,096 x 4,096 0.85 / 0.96, 12,288 x 4,096
+// 0.89 / 0.93) and loses
+// - where the last turn of workgroups leaves compute units idle: 5,120 rows of W are 320 workgroups, 1.25 a unit (5,120 x 5,120
+//   at 1 / 8 rows 1.12 / 1.31, 5,120 x 13,824 1.38 / 1.63), 10,240 are 2.5 (10,240 x 8,192 1.14 / 1.27, x 4,096 0.89 / 1.05);
+// - where the reads of X weigh more than a launch: 4,096 x 8,192 at 4 / 12 rows 0.94 / 1.14, 8,192 x 6,144 at 4 / 8 0.97 / 1.05;
+// - with few workgroups and more than a chunk a wave (2,048 x 8,192 1.19 / 1.39), or many rows (512 x 2,048 at 4 / 8 0.97 / 1.03);
+// - where the chunks do not deal out evenly over more than four waves, which then wait for the longest;
+// - with both halves, whose X it reads twice, from nine rows on, with more than six parts (4,096 x 2,048 in eight 1.05 / 1.14) and
+//   with few workgroups (2,048 x 2,048 1.31; 5,632 x 2,048 0.88 / 0.99, 13,824 x 2,048 at 1 / 4 0.92 / 0.97).
 static bool whole_k_pays(int M, int N, int K, int splits, bool glu) {
   if (M > 16 || splits > 8) return false;
-  const int nchunks = (K + SK_KC - 1) / SK_KC;
-  if (glu) return N % 32 == 0 && K <= 2048 && (long)M * N <= 45056;
-  if (N < 512 || (splits > 4 && nchunks % splits != 0)) return false;
-  if (M > 8 && ((long)M * K > 32768 || (K > 1024 && N < 2560))) return false;
-  return (long)M * K <= 65536 && (long)M * N <= 98304;
+  const int nchunks = (K + SK_KC - 1) / SK_KC, cps = (nchunks + splits - 1) / splits;
+  const int groups = ((glu ? N / 2 : N) + 15) / 16, turns = (groups + 255) / 256;
+  const int full = groups <= 256 ? 100 : groups * 100 / (turns * 256);     // how much of the chip the turns fill, in per cent
+  if (glu) return N % 32 == 0 && K <= 2048 && M <= 8 && splits <= 6 && groups >= 128 && (long)M * N <= 45056;
+  if (N < 512 || (splits > 4 && nchunks % splits != 0) || (long)M * N > 98304) return false;
+  if (groups < 160) return cps == 1 && (K <= 1024 || M <= (N >= 2048 ? 12 : splits <= 6 ? 8 : 4));
+  if (full < 70 && K > 2048) return false;
+  if (full < 99 && ((splits >= 5 && cps >= 4) || (splits == 3 && cps > 8))) return false;
+  return (long)M * K <= (full < 70 ? 8192 : full < 99 ? 16384 : groups < 768 ? 32768 : 65536);
 }
 
 // Shapes whose number of splits was measured (ia_gemm_skinny_set_splits, filled from a table when the library is
