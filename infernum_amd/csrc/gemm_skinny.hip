@@ -261,7 +261,9 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16
 
 // C[m, n] = sum_s part[s, m, n]                                       (SK_EPI_NONE,   n < N)
 // C[m, n] = silu(sum_s part[s, m, n]) * sum_s part[s, m, N/2 + n]      (SK_EPI_SWIGLU, n < N/2)
-template <typename TO, int EPI>
+// PRE parts are asked for together and added in the order of their index (eight loads for two parts cost 128 rows of 15,360 x 5,120
+// 1.5 of 58 us).
+template <typename TO, int EPI, int PRE>
 __global__ __launch_bounds__(256) void gemm_skinny_join_kernel(const float* __restrict__ part, TO* __restrict__ C,
                                                                int M, int N, int splits) {
   const int NO = EPI == SK_EPI_SWIGLU ? N / 2 : N;
@@ -270,7 +272,6 @@ __global__ __launch_bounds__(256) void gemm_skinny_join_kernel(const float* __re
   const int m = (int)(idx / NO), n = (int)(idx - (size_t)m * NO);
   const size_t MN = (size_t)M * N;
   const float* p = part + (size_t)m * N + n;
-  constexpr int PRE = 8;                               // so many parts asked for together, added in the order of their index
   float a = 0.f, b = 0.f;
   for (int s0 = 0; s0 < splits; s0 += PRE) {
     float pa[PRE], pb[PRE];
@@ -432,20 +433,25 @@ static int launch_skinny_one(dim3 grid, const uint16_t* x, const uint16_t* w, TO
 // Whether the rounds run one after the other instead of in pairs.  Where one workgroup has a compute unit to itself pairs are 15
 // to 30 % faster from 33 rows on, and with many in turn 0 to 13; with two side by side and no third, each covers the other's waits,
 // and the registers and selects of the unconditional loads cost more than they give at some numbers of tiles of 16 rows (MT).
-// Microseconds one after the other / in pairs: 28,672 x 4,096 with the activation from its copy, 33 / 48 / 64 / 128 rows 47.6 /
-// 50.8 / 54.3 / 73.3 against 51.1 / 53.0 / 55.4 / 75.5; 32,000 x 2,048 at 33 / 64 rows 27.8 / 32.1 against 29.3 / 33.6; at 112 rows
-// every shape without a copy (24,000 x 2,048, 20,480 x 2,560, 28,672 x 4,096 with the activation) 1.03 to 1.05 of the time in pairs.
-// Not so: 20,480 x 2,560 (320 workgroups) at 33 to 64 rows 0.93 to 0.97, copies at 65 to 80 rows 0.86 to 0.92.  With more
-// workgroups: short walks over K at 49 to 64 rows (50,257 x 2,048 55 against 57.5, 65,536 x 2,048 1.03; 36,864 x 4,096 0.92); and at 81
-// to 96 rows, where the rounds alone leave a compute unit the registers for a third workgroup and pairs do not, up to three
-// workgroups a unit of a few chunks each (12,288 / 13,312 / 14,336 x 4,096 in three parts 36.2 / 36.7 / 37.2 against 38.0 / 39.9 /
-// 40.5; with eight chunks and more 0.94 to 0.96, with two or three 0.95 to 0.99).
-static bool rounds_alone(int MT, bool tiled, unsigned groups, unsigned splits, int chunks) {
+// The time one after the other over that in pairs, with 257 to 512 workgroups:
+// - K a power of two, without a copy: 32,000 x 2,048 at 40 / 64 rows 0.95 / 0.97, 28,672 x 4,096 with the activation 0.98 / 0.98;
+//   not so other K (27,648 x 5,120 1.05 / 1.07, 20,480 x 2,560 1.04);
+// - copies at 33 to 64 and 113 to 128 rows (28,672 x 4,096 0.95 / 0.99 and 0.97), not at 65 to 112 (1.09, 0.99, 1.09);
+// - rows that do not lie on whole lines of 128 bytes (K % 64): 21,056 x 3,680 at 40 / 72 / 96 / 128 rows 0.96 / 0.96 / 0.94 / 0.93,
+//   24,000 x 1,480 0.97 / 0.93 / 0.92 / 0.90; walks of many chunks from 65 rows on only (24,000 x 7,400 1.01 / 0.95 / 0.95 / 0.92);
+// - at 97 to 112 rows all without a copy, 0.92 to 0.97.
+// With more workgroups: short walks at 49 to 64 rows (50,257 x 592 / 2,048 0.92 / 0.99; 36,864 x 4,608 1.10); and at 81 to 96 rows,
+// where the rounds alone leave a compute unit the registers for a third workgroup and pairs do not, up to three workgroups a unit
+// of a few chunks each (12,288 / 13,312 / 14,336 x 4,096 in three parts 36.2 / 36.7 / 37.2 us against 38.0 / 39.9 / 40.5; with eight
+// chunks and more 0.94 to 0.96 in pairs, with two or three 0.95 to 0.99).
+static bool rounds_alone(int MT, bool tiled, int K, unsigned groups, unsigned splits, int chunks) {
+  const bool whole_lines = tiled || K % 64 == 0, power_of_two = (K & (K - 1)) == 0;
   if (MT == 4 && splits == 1 && chunks <= 8 && groups > 360) return true;
-  if (MT == 6) return splits > 1 && groups > 560 && groups <= 3 * SK_ENOUGH_BLOCKS && chunks >= 4 && chunks <= 6;
+  if (MT == 6 && splits > 1 && groups > 560 && groups <= 3 * SK_ENOUGH_BLOCKS && chunks >= 4 && chunks <= 6) return true;
   if (groups <= SK_ENOUGH_BLOCKS || groups > 2 * SK_ENOUGH_BLOCKS) return false;
-  if (MT == 3) return splits == 1 ? tiled || groups > 360 : splits >= 4 && chunks >= 8;  // (8,192 x 8,192: 1.03; 15,360 x 5,120 in two parts 0.97)
-  if (MT == 4) return splits == 1 && groups > 360;
+  if (!whole_lines && chunks >= 2 && MT >= 3) return MT >= 5 || chunks <= (MT == 3 ? 20 : 8);
+  if (MT == 3) return splits == 1 ? tiled || (power_of_two && groups > 360) : power_of_two && splits >= 4 && chunks >= 8;
+  if (MT == 4) return splits == 1 && (tiled || power_of_two) && groups > 360;
   return (MT == 7 && !tiled) || (MT == 8 && tiled);
 }
 
@@ -461,9 +467,15 @@ static int launch_skinny(const uint16_t* x, const uint16_t* w, TO* c, float* par
   // products sooner (2,048 x 8,192 in 16 parts at 16 / 32 rows 8.4 / 9.4 us with pieces of 256 and 7.9 / 8.7 with 128, the
   // 8B shape's gate+up from its copy 43.9 / 49.0 and 42.4 / 45.1).  One workgroup a compute unit wants the longer pieces
   // (the 1B shape's gate+up 14.5 against 15.4), and so do heads of many workgroups (128,256 x 2,048 91.5 against 92.8).
+  // Rows off the lines of 128 bytes want the longer pieces too, once the walk has some chunks (21,056 x 1,480 / 3,680 / 7,400 at 1 row
+  // 9 / 3 / 10 % and at 32 rows 11 / 10 / 15 % longer in pieces of 128); a single chunk is done sooner in two (2,176 x 128 with
+  // the activation 3.6 us and 3.2; from a copy only if the second holds nothing: 2,848 x 224 3.6 and 3.8).
   const unsigned groups = grid.x * grid.y;
-  const bool shorter = grid.y > 1 || (groups > SK_ENOUGH_BLOCKS && groups <= 4 * SK_ENOUGH_BLOCKS);
-  const bool alone = rounds_alone((M + 15) / 16, TILED, groups, grid.y, cps);
+  const bool off_lines = !TILED && K % 64 != 0;
+  const bool shorter = (cps == 1 && (!TILED || K <= SK_KC / 2)) || (grid.y > 1 ? !off_lines
+                                               : groups > SK_ENOUGH_BLOCKS && groups <= 4 * SK_ENOUGH_BLOCKS &&
+                                                     !(off_lines && cps >= 4 && groups > SK_ENOUGH_BLOCKS + 8));
+  const bool alone = rounds_alone((M + 15) / 16, TILED, K, groups, grid.y, cps);
   switch ((M + 15) / 16) {
     case 1:
       if (shorter) return launch_skinny_one<1, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
@@ -478,7 +490,9 @@ static int launch_skinny(const uint16_t* x, const uint16_t* w, TO* c, float* par
       if (alone) return launch_skinny_one<4, GLU, TO, SK_KC, TILED, false>(grid, x, w, c, part, M, N, K, cps, stream);
       return launch_skinny_one<4, GLU, TO, SK_KC, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
     // above 64 rows: pieces of 128, so that the two stages of X of two workgroups fit a compute unit's LDS
-    case 5: return launch_skinny_one<5, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
+    case 5:
+      if (alone) return launch_skinny_one<5, GLU, TO, SK_KC / 2, TILED, false>(grid, x, w, c, part, M, N, K, cps, stream);
+      return launch_skinny_one<5, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
     case 6:
       if (alone) return launch_skinny_one<6, GLU, TO, SK_KC / 2, TILED, false>(grid, x, w, c, part, M, N, K, cps, stream);
       return launch_skinny_one<6, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
@@ -496,10 +510,15 @@ template <typename TO>
 static int launch_join(const float* part, TO* c, int M, int N, int splits, int epilogue, hipStream_t stream) {
   const int NO = epilogue == SK_EPI_SWIGLU ? N / 2 : N;
   const unsigned grid = (unsigned)(((size_t)M * NO + 255) / 256);
-  if (epilogue == SK_EPI_SWIGLU)
-    gemm_skinny_join_kernel<TO, SK_EPI_SWIGLU><<<grid, 256, 0, stream>>>(part, c, M, N, splits);
-  else
-    gemm_skinny_join_kernel<TO, SK_EPI_NONE><<<grid, 256, 0, stream>>>(part, c, M, N, splits);
+#define SK_JOIN(EPI)                                                                                          \
+  do {                                                                                                        \
+    if (splits <= 2) gemm_skinny_join_kernel<TO, EPI, 2><<<grid, 256, 0, stream>>>(part, c, M, N, splits);    \
+    else if (splits <= 4) gemm_skinny_join_kernel<TO, EPI, 4><<<grid, 256, 0, stream>>>(part, c, M, N, splits); \
+    else gemm_skinny_join_kernel<TO, EPI, 8><<<grid, 256, 0, stream>>>(part, c, M, N, splits);                \
+  } while (0)
+  if (epilogue == SK_EPI_SWIGLU) SK_JOIN(SK_EPI_SWIGLU);
+  else SK_JOIN(SK_EPI_NONE);
+#undef SK_JOIN
   IA_LAUNCH_CHECK();
   return IA_OK;
 }

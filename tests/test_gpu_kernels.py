@@ -421,11 +421,12 @@ def test_gemm_skinny_rounds_in_pairs(M, N, K_):
     assert ((got - want).abs() <= K_ * 2 ** -24 * size + 1e-30).all()
 
 
-# rounds one after the other (257 to 512 workgroups: 361 and more without a copy up to 64 rows, all copies at 33 to 48 and from 113
-# rows on, all without a copy at 97 to 112; parts of eight chunks and more at 33 to 48 rows) leave the bits that a row has alone;
-# a last chunk that is not full
-@pytest.mark.parametrize("M", [33, 48, 49, 64, 97, 112, 113, 128])
-@pytest.mark.parametrize("N,K_,tiled", [(23200, 520, False), (16500, 776, False), (19300, 776, True), (28670, 264, True), (8190, 7944, False)])
+# rounds one after the other (by rows, workgroups, K's lines and chunks: rounds_alone) leave the bits that a row has alone: rows off
+# the lines of 128 bytes with three chunks, and eight in parts; K a power of two, whole and in parts; copies; three parts of four
+# chunks; a last chunk that is not full
+@pytest.mark.parametrize("M", [33, 48, 49, 64, 72, 90, 97, 112, 113, 128])
+@pytest.mark.parametrize("N,K_,tiled", [(23200, 520, False), (16500, 776, False), (19300, 776, True), (28670, 264, True), (8190, 7944, False),
+                                        (23200, 512, False), (8190, 8192, False), (12290, 2816, False)])
 def test_gemm_skinny_rounds_one_after_the_other(M, N, K_, tiled):
     api = K()
     a, w = _rand(M, K_, dtype=torch.bfloat16, seed=23), _rand(N, K_, dtype=torch.bfloat16, scale=0.05, seed=24)
