@@ -136,6 +136,16 @@ __global__ __launch_bounds__(256) void gemm_heads_big_kernel(const bf16_t* __res
 // 64 of Nout, 1, H).  One row, 16 heads: 224 x 64 3.9 us with the tiles and 2.4 so, 64 x 224 with
 // a gate 6.7 and 4.4, 128 x 512 with a gate 9.8 and 7.5; 16 rows 3.9 and 2.6, 6.8 and 4.0, 8.7 and 7.8.
 #define GH_FEW_ROWS 16
+// The reads of x, once for every 16 columns of W, make it lose with long rows and many workgroups.  Its time over that of the
+// tiles at 1 / 8 / 16 rows, by K and workgroups: 64 and up to 512 0.67 to 0.85; 128 x 512 0.81 / 0.85 / 0.92, 128 x 1,024 0.87 /
+// 0.95 / 1.04; 192 x 1,024 1.00 / 1.08 / 1.18; 256 x 512 0.95 / 1.02 / 1.09; 512 x 128 0.89 / 0.97 / 1.04, 512 x 256 (16 heads of
+// 1,024) 1.03 / 1.13 / 1.16; 1,024 x 64 0.98 / 1.07 / 1.14, x 128 1.16 / 1.33 / 1.39.
+static bool heads_few_pays(int N, int H, int Nout, int K) {
+  const long work = (long)K * H * ((Nout + 63) / 64);
+  if (K > 256) return N <= GH_FEW_ROWS && work <= (K <= 512 && N <= 8 ? 65536 : 16384);
+  return N <= GH_FEW_ROWS && work <= (N <= 4 ? 131072 : N <= 8 ? 98304 : 65536);
+}
+
 __global__ __launch_bounds__(256) void gemm_heads_few_kernel(const bf16_t* __restrict__ x, int x_row, int x_head,
                                                              const bf16_t* __restrict__ W, bf16_t* __restrict__ out,
                                                              int o_row, int o_head, const bf16_t* __restrict__ gate,
@@ -195,7 +205,7 @@ extern "C" int ia_gemm_heads(const void* x, int x_row, int x_head, const void* W
                                                               (float*)out, o_row, o_head, (const float*)gate, g_row,
                                                               N, Nout, K);
   else if (dtype == IA_BF16 && (K & 7) == 0 && tile_rows_aligned(x, x_row, x_head) && tile_rows_aligned(W, K)) {
-    if (N <= GH_FEW_ROWS) {
+    if (heads_few_pays(N, H, Nout, K)) {
       gemm_heads_few_kernel<<<dim3((Nout + 63) / 64, 1, H), 256, 0, stream>>>((const bf16_t*)x, x_row, x_head, (const bf16_t*)W,
                                                                               (bf16_t*)out, o_row, o_head, (const bf16_t*)gate,
                                                                               g_row, N, Nout, K);

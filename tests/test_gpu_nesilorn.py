@@ -179,7 +179,7 @@ def _run_mixer(mixer, steps, x, cuts, rt):
 # sigmoid's few fp32 roundings far below
 @pytest.mark.parametrize("gated", [False, True])
 @pytest.mark.parametrize("N", [1, 16, 17])
-@pytest.mark.parametrize("H,J,Kd", [(3, 37, 8), (2, 64, 72), (4, 130, 264), (1, 16, 520)])
+@pytest.mark.parametrize("H,J,Kd", [(3, 37, 8), (2, 64, 72), (4, 130, 264), (1, 16, 504), (1, 16, 520)])
 def test_products_head_by_head_of_few_rows(N, H, J, Kd, gated):
     from infernum_amd.kernels import api as K
     g = torch.Generator().manual_seed(N + J)
