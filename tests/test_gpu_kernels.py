@@ -344,7 +344,9 @@ def test_gemm_generic(M, N, K_):
 # 16 / 17, 32 / 33: the ends of the streaming kernel's one and two groups of rows; 8192: two groups of W's rows a workgroup;
 # 260, 516: a stretch of 256 and a bit; 16, 20: less than a chain more; tiles of 32, 64 and 128 rows and their remainders
 @pytest.mark.parametrize("M,N,K_", [(2, 16, 4), (16, 1000, 2052), (17, 33, 20), (32, 8192, 260), (3, 8200, 4096),
-                                    (33, 97, 516), (65, 4100, 256), (300, 8205, 288), (1030, 8192, 36)])
+                                    (33, 97, 516), (65, 4100, 256), (300, 8205, 288), (1030, 8192, 36),
+                                    # short rows: the vector kernel's, and the first that are not
+                                    (5, 300, 16), (5, 4100, 48), (5, 4100, 52), (20, 4100, 96), (20, 4100, 100)])
 def test_gemm_fp32_on_the_matrix_cores_leaves_the_vector_kernels_bits(M, N, K_):
     padded, w = _rand(M, K_ + 1, seed=1), _rand(N, K_, seed=2)
     padded[0, :K_] *= 1e-30                                    # products that are subnormal or nothing
