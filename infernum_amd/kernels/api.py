@@ -2019,7 +2019,7 @@ def wpa_decode_parts(batch: int, nh: int, nkv: int, max_len: int, window: int, p
                      device: Optional[torch.device] = None) -> int:
     """Parts that the tiles of a token's keys and blocks are cut into (a workgroup of four waves each): as many as bring
     the workgroups to the compute units, at most the square root of the tiles (the join grows with the parts as the work of
-    one shrinks: one request on 4 key/value heads, 1,024 keys and 31 blocks, takes 36 us whole and 13 + 6 in 8 parts)
+    one shrinks: one request on 4 key/value heads, 1,024 / 3,000 keys, takes 19.0 / 21.7 us whole and 8.5 / 10.8 in parts)
     and 16.  Two parts of fewer than 16 tiles do not pay for the join's launch (one request, 100 keys 6.4 us whole and 7.0 in two
     parts, 129 keys 7.2 and in three 7.0; 32 requests 129 keys 7.5 and 8.2 in two, 256 keys 8.8 and 8.6)."""
     groups = max(1, batch * nkv * ((nh // nkv + 15) // 16))
