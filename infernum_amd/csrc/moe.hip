@@ -134,25 +134,42 @@ extern "C" int ia_moe_sort(const int* ids, int* offsets, int* perm, int P, int E
 }
 
 // Tile t of the launch (`rows` pairs a tile, expert by expert): its expert and its first place in perm; false when
-// the launch has more tiles than the step needs.
+// the launch has more tiles than the step needs.  A wave's lanes take an expert each and a prefix sum says whose tile it is:
+// walking the experts one after the other took 2 us for 32 of them, in front of every workgroup's first load.
 __device__ __forceinline__ bool moe_tile(const int* __restrict__ offsets, int E, int t, int& expert, int& first,
                                          int& last, int rows = TF_T) {
+  const int lane = threadIdx.x & 63;
   int seen = 0;
-  for (int e = 0; e < E; ++e) {
-    const int lo = offsets[e], hi = offsets[e + 1];
-    const int tiles = (hi - lo + rows - 1) / rows;
-    if (t < seen + tiles) {
-      expert = e;
-      first = lo + (t - seen) * rows;
-      last = hi;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int e = e0 + lane;
+    const int lo = offsets[min(e, E)], hi = offsets[min(e + 1, E)];
+    const int tiles = (hi - lo + rows - 1) / rows;           // none beyond the last expert
+    int upto = tiles;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(upto, o, IA_WAVE);
+      upto += lane >= o ? v : 0;
+    }
+    const unsigned long long reach = __ballot(t < seen + upto);
+    if (reach) {
+      const int l = __ffsll(reach) - 1;
+      expert = e0 + l;
+      first = __builtin_amdgcn_readlane(lo, l) + (t - seen - __builtin_amdgcn_readlane(upto - tiles, l)) * rows;
+      last = __builtin_amdgcn_readlane(hi, l);
       return true;
     }
-    seen += tiles;
+    seen += __builtin_amdgcn_readlane(upto, 63);
   }
   return false;
 }
+// Tiles of `rows` pairs that P pairs of E experts can need: an expert that has any starts one, and every further `rows` of its
+// pairs another.
+static inline long moe_most_tiles(int P, int E, int rows) {
+  const int some = P < E ? P : E;
+  return some + (P - some) / rows;
+}
 
-// grid: (tiles of 2 * ff columns, ceil(P / 64) + E).  Wgu [E, 2 ff, W]: row 2 j the gate's row j, row 2 j + 1 up's.
+// grid: (tiles of 2 * ff columns, moe_most_tiles).  Wgu [E, 2 ff, W]: row 2 j the gate's row j, row 2 j + 1 up's.
 // On the vector ALUs in fp32: the 32-bit path, and bfloat16 rows that cannot be read 16 bytes at a time.
 template <typename T>
 __global__ __launch_bounds__(256) void moe_gate_up_kernel(const T* __restrict__ x, const T* __restrict__ Wgu,
@@ -183,59 +200,225 @@ __global__ __launch_bounds__(256) void moe_gate_up_kernel(const T* __restrict__ 
   });
 }
 
-// The same on tiles of BM x BN (tile_mfma_big): grid (tiles of BN of the 2 ff columns, ceil(P / BM) + E).
-template <int BM, int BN>
-__global__ __launch_bounds__(BN == 256 ? 512 : 256) void moe_gate_up_big_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ Wgu,
+// ---- tiles of up to 64 pairs ------------------------------------------------------------------------------------------
+// What bounds a step of few pairs is the stream of the chosen experts' weights.  A workgroup of WAVES waves takes 16 rows of
+// W a wave and walks K in chunks of 256: W straight from memory to registers, one chunk ahead (each byte of it is used by one
+// wave only), the chunk of the pairs' rows through LDS, two stages.  No load stands under a condition; chunks are written
+// out in pairs so that no register of a load under way is copied; what lies beyond K is read from the row's end and cleared.
+// v_mfma_f32_16x16x32_bf16 with W's rows as its first operand: lane (r = lane % 16, q = lane / 16) ends with four
+// consecutive columns 4 q .. 4 q + 3 of row r of the result.
+// All workgroups walking K in step read places one row's length apart at the same moment, and where that length is a power
+// of two those lie on few memory channels, so every 256 columns start their walk at a chunk of their own (moe_first_chunk) and
+// wrap around.  The tile of 128 pairs starts there too: an element is one chain over K in an order that
+// depends on K and its column alone.
+// Before, tiles of 32 x 128 in steps of 64 through one LDS stage and all walks from the same start (cold weights,
+// gate and up / down, microseconds before and now): 4 of 32 experts of 1,408 x 2,048 22.0 / 15.9 and 12.4 / 7.2; 16 of 16, 32
+// tokens, 44.7 / 20.3 and 35.3 / 19.3 (184 MB: 5.2 TB/s); 16 of 20 of 2,432 x 4,096 136 / 56.6 and 108.6 / 56.4 (5.9 and 5.7 TB/s).
+#define MS_KC 256
+#define MS_LD (MS_KC + 8)     // bf16 of a row in LDS (the padding spreads the banks)
+
+__device__ __forceinline__ int moe_first_chunk(int column, int K) {
+  const unsigned chunks = (unsigned)(K + MS_KC - 1) / MS_KC;
+  return (int)((((unsigned)(column / 256) * 0x9E3779B1u) >> 8) % chunks);
+}
+
+// `x_row(r)`: row r of the tile's pairs, 0 <= r < rows; Wm: the expert's matrix [w_rows, K]; this workgroup's columns
+// of the result begin at n0.  Rows of 16-byte alignment, K a multiple of 8.
+template <int MT, int ROWS, int WAVES, typename XRow, typename Emit>
+__device__ __forceinline__ void moe_stream_tile(const bf16_t* __restrict__ Wm, int w_rows, int n0, int K, int rows,
+                                                XRow x_row, uint16_t (*xs)[ROWS][MS_LD], Emit emit) {
+  constexpr int T = WAVES * 64, NLD = MS_KC / 32, PIECES = MS_KC / 8;
+  constexpr int XPT = MT * 16 * PIECES / T;                  // 16-byte pieces of the pairs' rows a thread brings in
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
+  const int n = n0 + (tid >> 6) * 16;
+  const bf16_t* wrow = Wm + (size_t)min(n + r, w_rows - 1) * K;
+  const int chunks = (K + MS_KC - 1) / MS_KC, rot = moe_first_chunk(n0, K);
+  auto at = [&](int c) {                                     // where chunk c of the walk begins
+    const int k = c + rot;
+    return (k >= chunks ? k - chunks : k) * MS_KC;
+  };
+  const bf16_t* xp[XPT];
+#pragma unroll
+  for (int i = 0; i < XPT; ++i) xp[i] = x_row(min((tid + i * T) / PIECES, rows - 1));
+  const int xk = (tid % PIECES) * 8;                         // T is a multiple of PIECES: the same place of every row
+  uint4 xr[XPT], w0[NLD], w1[NLD];
+  tm_f32x4 acc[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) acc[m] = tm_f32x4{0.f, 0.f, 0.f, 0.f};
+  auto load_x = [&](int c) {
+    const int k = min(at(c) + xk, K - 8);
+#pragma unroll
+    for (int i = 0; i < XPT; ++i) xr[i] = *reinterpret_cast<const uint4*>(xp[i] + k);
+  };
+  auto store_x = [&](int c) {
+    const bool in = at(c) + xk < K;
+#pragma unroll
+    for (int i = 0; i < XPT; ++i)
+      *reinterpret_cast<uint4*>(&xs[c & 1][(tid + i * T) / PIECES][xk]) =
+          make_uint4(in ? xr[i].x : 0u, in ? xr[i].y : 0u, in ? xr[i].z : 0u, in ? xr[i].w : 0u);
+  };
+  auto load_w = [&](int c, uint4 (&w)[NLD]) {
+    const int k0 = at(c) + 8 * q;
+#pragma unroll
+    for (int j = 0; j < NLD; ++j) w[j] = *reinterpret_cast<const uint4*>(wrow + min(k0 + 32 * j, K - 8));
+  };
+  auto products = [&](int c, uint4 (&w)[NLD]) {
+    if (K % MS_KC != 0 && at(c) + MS_KC > K) {
+#pragma unroll
+      for (int j = 0; j < NLD; ++j)
+        if (at(c) + 32 * j + 8 * q >= K) w[j] = make_uint4(0u, 0u, 0u, 0u);
+    }
+#pragma unroll
+    for (int j = 0; j < NLD; ++j)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const uint4 xv = *reinterpret_cast<const uint4*>(&xs[c & 1][16 * m + r][32 * j + 8 * q]);
+        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(tm_bf16x8, w[j]),
+                                                         __builtin_bit_cast(tm_bf16x8, xv), acc[m], 0, 0, 0);
+      }
+  };
+  auto round = [&](int c, uint4 (&w)[NLD], uint4 (&next)[NLD]) {
+    load_x(c + 1);
+    load_w(c + 1, next);
+    __builtin_amdgcn_sched_barrier(0);                       // all of them in front of the first wait for this chunk's W
+    products(c, w);
+    store_x(c + 1);
+    __syncthreads();
+  };
+  load_x(0);
+  load_w(0, w0);
+  store_x(0);
+  __syncthreads();
+  int c = 0;
+  for (; c + 2 < chunks; c += 2) {
+    round(c, w0, w1);
+    round(c + 1, w1, w0);
+  }
+  if (c + 1 < chunks) {
+    round(c, w0, w1);
+    products(c + 1, w1);
+  } else {
+    products(c, w0);
+  }
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const float v[4] = {acc[m][0], acc[m][1], acc[m][2], acc[m][3]};
+    emit(16 * m + r, n + 4 * q, v);
+  }
+}
+
+// The tile with as many groups of 16 rows as it has pairs.
+template <int ROWS, int WAVES, typename XRow, typename Emit>
+__device__ __forceinline__ void moe_stream(const bf16_t* __restrict__ Wm, int w_rows, int n0, int K, int rows, XRow x_row,
+                                           uint16_t (*xs)[ROWS][MS_LD], Emit emit) {
+  if (rows <= 16) return moe_stream_tile<1, ROWS, WAVES>(Wm, w_rows, n0, K, rows, x_row, xs, emit);
+  if (rows <= 32) return moe_stream_tile<2, ROWS, WAVES>(Wm, w_rows, n0, K, rows, x_row, xs, emit);
+  if constexpr (ROWS > 32) {
+    if (rows <= 48) return moe_stream_tile<3, ROWS, WAVES>(Wm, w_rows, n0, K, rows, x_row, xs, emit);
+    moe_stream_tile<4, ROWS, WAVES>(Wm, w_rows, n0, K, rows, x_row, xs, emit);
+  }
+}
+
+// Which tiles (pairs x columns) take a launch.  Measured with cold weights at 1 to 400 pairs an expert on average, microseconds
+// of gate and up / down:
+// - up to 10 pairs an expert, tiles of 32: with 64 columns, or with 32 where those make few workgroups, so that more compute
+//   units read (4 of 32 experts of 1,408 x 2,048 12.4 / 9.3 with 64 columns and 12.7 / 7.2 with 32, 7 of 32 22.2 / 10.5
+//   and 18.4 / 10.5; 16 of 16 with 64 pairs 35.3 / 19.4 and 40.0 / 19.1; 20 of 2,432 x 4,096 with 128 pairs 135 / 73 and 137 / 79);
+// - above, tiles of 64, so that an expert's weights are read once again (32 experts of 1,408 x 2,048 at 12 pairs 67.4 / 41.0
+//   with 32 and 67.1 / 37.0 with 64);
+// - from 24 pairs on with 128 columns, which read the pairs' rows half as often, unless that leaves compute units idle (20 experts of
+//   2,432 x 4,096 at 37 pairs 160 / 106 with 64 columns and 148 / 97 with 128; 8 of 2,752 x 2,048 at 47 pairs, 286 and 208
+//   workgroups, 31.7 / 26.4 and 29.1 / 37.3);
+// - from 56 on tiles of 128 x 256 that share both operands, if they fill the chip (32 experts of 1,408 x 2,048 at 64 pairs
+//   109 / 67 with 64 x 128 and 108 / 53 with these; 8 of 2,752 x 2,048, at most 100 workgroups, 35 / 42 and 54 / 66).
+enum MoeTile { MOE_32_32, MOE_32_64, MOE_64_64, MOE_64_128, MOE_128_256 };
+static inline int moe_tile_rows(MoeTile t) { return t == MOE_128_256 ? 128 : t >= MOE_64_64 ? 64 : 32; }
+static inline MoeTile moe_tile_for(int P, int E, int columns) {
+  auto groups = [&](int rows, int width) { return (columns + width - 1) / width * moe_most_tiles(P, E, rows); };
+  if (P >= 56L * E && groups(128, 256) >= 224) return MOE_128_256;
+  if (P >= 24L * E && groups(64, 128) >= 224) return MOE_64_128;
+  if (P >= 10L * E) return MOE_64_64;
+  return groups(32, 64) > 512 ? MOE_32_64 : MOE_32_32;
+}
+
+// Gate and up of one row of the result: four consecutive columns are two of each.  Both products are rounded as a stored tensor
+// would be, then the activation in fp32.
+__device__ __forceinline__ void moe_gate_up_store(bf16_t* __restrict__ y, int ff, int p, int c0, const float* v, float wt, float limit,
+                                                  float alpha, float shift) {
+#pragma unroll
+  for (int j = 0; j < 4; j += 2) {
+    const int c = c0 + j;
+    if (c + 1 >= 2 * ff) continue;
+    const float g = fminf(wt * to_float(from_float<bf16_t>(v[j])), limit);
+    const float u = fminf(fmaxf(wt * to_float(from_float<bf16_t>(v[j + 1])), -limit), limit);
+    y[(size_t)p * ff + (c >> 1)] = from_float<bf16_t>(g * (1.0f / (1.0f + expf(-alpha * g))) * (u + shift));
+  }
+}
+
+// Tiles of 128 pairs x 256 columns (tile_mfma_big): grid (tiles of the 2 ff columns, moe_most_tiles).
+__global__ __launch_bounds__(512) void moe_gate_up_big_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ Wgu,
                                                               bf16_t* __restrict__ y, const int* __restrict__ offsets,
                                                               const int* __restrict__ perm, int E, int top, int W,
                                                               int ff, float limit, float alpha, float shift,
                                                               const float* __restrict__ in_w) {
-  __shared__ TileBigLds<BM, BN> lds;
+  __shared__ TileBigLds<128, 256> lds;
   int e, first, last;
-  if (!moe_tile(offsets, E, blockIdx.y, e, first, last, BM)) return;
-  const int n0 = blockIdx.x * BN;
-  tile_mfma_big<BM, BN>(
+  if (!moe_tile(offsets, E, blockIdx.y, e, first, last, 128)) return;
+  const int n0 = blockIdx.x * 256;
+  tile_mfma_big<128, 256>(
       [&](int r) { return x + (size_t)(perm[first + r] / top) * W; },
       [&](int r) { return Wgu + ((size_t)e * 2 * ff + n0 + r) * W; }, last - first, 2 * ff - n0, W, lds,
       [&](int i, int j0, const float* v) {
         const int p = first + i;
-        if (p >= last) return;
-        const float wt = in_w ? in_w[perm[p]] : 1.0f;
-#pragma unroll
-        for (int j = 0; j < 4; j += 2) {
-          const int c = n0 + j0 + j;
-          if (c + 1 >= 2 * ff) continue;
-          const float g = fminf(wt * to_float(from_float<bf16_t>(v[j])), limit);
-          const float u = fminf(fmaxf(wt * to_float(from_float<bf16_t>(v[j + 1])), -limit), limit);
-          y[(size_t)p * ff + (c >> 1)] = from_float<bf16_t>(g * (1.0f / (1.0f + expf(-alpha * g))) * (u + shift));
-        }
-      });
+        if (p < last) moe_gate_up_store(y, ff, p, n0 + j0, v, in_w ? in_w[perm[p]] : 1.0f, limit, alpha, shift);
+      }, moe_first_chunk(n0, W) * (MS_KC / TB_KS));
 }
 
-// Rows a tile of the experts' products takes: 128 where an expert has some tens of pairs on average, else 32.
-static inline int moe_tile_rows(int P, int E) { return (long)P >= 48L * E ? 128 : 32; }
+// Tiles of up to ROWS pairs x 16 columns a wave (moe_stream_tile): grid (tiles of the 2 ff columns, moe_most_tiles).
+template <int ROWS, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void moe_gate_up_stream_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ Wgu,
+                                                                        bf16_t* __restrict__ y, const int* __restrict__ offsets,
+                                                                        const int* __restrict__ perm, int E, int top, int W,
+                                                                        int ff, float limit, float alpha, float shift,
+                                                                        const float* __restrict__ in_w) {
+  __shared__ __attribute__((aligned(16))) uint16_t xs[2][ROWS][MS_LD];
+  int e, first, last;
+  if (!moe_tile(offsets, E, blockIdx.y, e, first, last, ROWS)) return;
+  const int rows = min(last - first, ROWS), n0 = blockIdx.x * WAVES * 16;
+  const bf16_t* Wm = Wgu + (size_t)e * 2 * ff * W;
+  auto x_row = [&](int r) { return x + (size_t)(perm[first + r] / top) * W; };
+  auto emit = [&](int i, int c0, const float* v) {
+    if (i < rows) moe_gate_up_store(y, ff, first + i, c0, v, in_w ? in_w[perm[first + i]] : 1.0f, limit, alpha, shift);
+  };
+  moe_stream<ROWS, WAVES>(Wm, 2 * ff, n0, W, rows, x_row, xs, emit);
+}
 
 extern "C" int ia_moe_gate_up(const void* x, const void* Wgu, void* y, const int* offsets, const int* perm, int dtype,
                               int P, int E, int top, int W, int ff, float limit, float alpha, float shift,
                               const float* in_weights, hipStream_t stream) {
   if (P < 0 || E <= 0 || top <= 0 || W <= 0 || ff <= 0) return IA_ERR_BAD_ARG;
   if (P == 0) return IA_OK;
-  dim3 grid((2 * ff + TF_T - 1) / TF_T, (P + TF_T - 1) / TF_T + E);
-  if (grid.y > 65535u) return IA_ERR_UNSUPPORTED;
+  const long tiles = moe_most_tiles(P, E, TF_T);
+  const dim3 grid((2 * ff + TF_T - 1) / TF_T, (unsigned)tiles);
+  if (tiles > 65535) return IA_ERR_UNSUPPORTED;
   if (dtype == IA_F32)
     moe_gate_up_kernel<float><<<grid, 256, 0, stream>>>((const float*)x, (const float*)Wgu, (float*)y, offsets,
                                                                perm, E, top, W, ff, limit, alpha, shift, in_weights);
   else if (dtype == IA_BF16 && tile_rows_aligned(x, W) && tile_rows_aligned(Wgu, W)) {
-    const int bm = moe_tile_rows(P, E);
-    const int bn = bm == 128 ? 256 : TB_N;
-    dim3 big((2 * ff + bn - 1) / bn, (P + bm - 1) / bm + E);
-    if (big.y > 65535u) return IA_ERR_UNSUPPORTED;
-    if (bm == 128)
-      moe_gate_up_big_kernel<128, 256><<<big, 512, 0, stream>>>((const bf16_t*)x, (const bf16_t*)Wgu, (bf16_t*)y, offsets,
-                                                           perm, E, top, W, ff, limit, alpha, shift, in_weights);
-    else
-      moe_gate_up_big_kernel<32, TB_N><<<big, 256, 0, stream>>>((const bf16_t*)x, (const bf16_t*)Wgu, (bf16_t*)y, offsets,
-                                                          perm, E, top, W, ff, limit, alpha, shift, in_weights);
+    const MoeTile tile = moe_tile_for(P, E, 2 * ff);
+    const long most = moe_most_tiles(P, E, moe_tile_rows(tile));
+    if (most > 65535) return IA_ERR_UNSUPPORTED;
+#define IA_GU(kernel, columns, threads)                                                                                \
+  kernel<<<dim3((2 * ff + (columns) - 1) / (columns), (unsigned)most), threads, 0, stream>>>(                          \
+      (const bf16_t*)x, (const bf16_t*)Wgu, (bf16_t*)y, offsets, perm, E, top, W, ff, limit, alpha, shift, in_weights)
+    switch (tile) {
+      case MOE_32_32: IA_GU((moe_gate_up_stream_kernel<32, 2>), 32, 128); break;
+      case MOE_32_64: IA_GU((moe_gate_up_stream_kernel<32, 4>), 64, 256); break;
+      case MOE_64_64: IA_GU((moe_gate_up_stream_kernel<64, 4>), 64, 256); break;
+      case MOE_64_128: IA_GU((moe_gate_up_stream_kernel<64, 8>), 128, 512); break;
+      case MOE_128_256: IA_GU(moe_gate_up_big_kernel, 256, 512); break;
+    }
+#undef IA_GU
   }
   else if (dtype == IA_BF16)
     moe_gate_up_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)x, (const bf16_t*)Wgu, (bf16_t*)y,
@@ -246,7 +429,7 @@ extern "C" int ia_moe_gate_up(const void* x, const void* Wgu, void* y, const int
   return IA_OK;
 }
 
-// grid: (tiles of W columns, ceil(P / 64) + E).  Wd [E, W, ff]; parts [top, N, W] fp32.
+// grid: (tiles of W columns, moe_most_tiles).  Wd [E, W, ff]; parts [top, N, W] fp32.
 template <typename T>
 __global__ __launch_bounds__(256) void moe_down_kernel(const T* __restrict__ y, const T* __restrict__ Wd,
                                                        float* __restrict__ parts, const float* __restrict__ weights,
@@ -274,31 +457,48 @@ __global__ __launch_bounds__(256) void moe_down_kernel(const T* __restrict__ y, 
   });
 }
 
-template <int BM, int BN>
-__global__ __launch_bounds__(BN == 256 ? 512 : 256) void moe_down_big_kernel(const bf16_t* __restrict__ y, const bf16_t* __restrict__ Wd,
+// One row of the result times the pair's weight, the product rounded as a stored tensor would be.
+__device__ __forceinline__ void moe_down_store(float* __restrict__ parts, const float* __restrict__ weights, int pair, int top, int N,
+                                               int W, int c0, const float* v) {
+  const int token = pair / top, choice = pair - token * top;
+  const float wt = weights ? weights[pair] : 1.0f;
+  float* o = parts + ((size_t)choice * N + token) * W;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (c0 + j < W) o[c0 + j] = to_float(from_float<bf16_t>(v[j])) * wt;
+}
+
+__global__ __launch_bounds__(512) void moe_down_big_kernel(const bf16_t* __restrict__ y, const bf16_t* __restrict__ Wd,
                                                            float* __restrict__ parts, const float* __restrict__ weights,
                                                            const int* __restrict__ offsets, const int* __restrict__ perm,
                                                            int E, int top, int N, int W, int ff) {
-  __shared__ TileBigLds<BM, BN> lds;
+  __shared__ TileBigLds<128, 256> lds;
   int e, first, last;
-  if (!moe_tile(offsets, E, blockIdx.y, e, first, last, BM)) return;
-  const int n0 = blockIdx.x * BN;
-  tile_mfma_big<BM, BN>(
+  if (!moe_tile(offsets, E, blockIdx.y, e, first, last, 128)) return;
+  const int n0 = blockIdx.x * 256;
+  tile_mfma_big<128, 256>(
       [&](int r) { return y + (size_t)(first + r) * ff; },
       [&](int r) { return Wd + ((size_t)e * W + n0 + r) * ff; }, last - first, W - n0, ff, lds,
       [&](int i, int j0, const float* v) {
-        const int p = first + i;
-        if (p >= last) return;
-        const int pair = perm[p];
-        const int token = pair / top, choice = pair - token * top;
-        const float wt = weights ? weights[pair] : 1.0f;
-        float* o = parts + ((size_t)choice * N + token) * W;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int c = n0 + j0 + j;
-          if (c < W) o[c] = to_float(from_float<bf16_t>(v[j])) * wt;
-        }
-      });
+        if (first + i < last) moe_down_store(parts, weights, perm[first + i], top, N, W, n0 + j0, v);
+      }, moe_first_chunk(n0, ff) * (MS_KC / TB_KS));
+}
+
+template <int ROWS, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void moe_down_stream_kernel(const bf16_t* __restrict__ y, const bf16_t* __restrict__ Wd,
+                                                                     float* __restrict__ parts, const float* __restrict__ weights,
+                                                                     const int* __restrict__ offsets, const int* __restrict__ perm,
+                                                                     int E, int top, int N, int W, int ff) {
+  __shared__ __attribute__((aligned(16))) uint16_t xs[2][ROWS][MS_LD];
+  int e, first, last;
+  if (!moe_tile(offsets, E, blockIdx.y, e, first, last, ROWS)) return;
+  const int rows = min(last - first, ROWS), n0 = blockIdx.x * WAVES * 16;
+  const bf16_t* Wm = Wd + (size_t)e * W * ff;
+  auto y_row = [&](int r) { return y + (size_t)(first + r) * ff; };
+  auto emit = [&](int i, int c0, const float* v) {
+    if (i < rows) moe_down_store(parts, weights, perm[first + i], top, N, W, c0, v);
+  };
+  moe_stream<ROWS, WAVES>(Wm, W, n0, ff, rows, y_row, xs, emit);
 }
 
 extern "C" int ia_moe_down(const void* y, const void* Wd, float* parts, const float* weights, const int* offsets,
@@ -306,22 +506,27 @@ extern "C" int ia_moe_down(const void* y, const void* Wd, float* parts, const fl
   if (N < 0 || E <= 0 || top <= 0 || W <= 0 || ff <= 0) return IA_ERR_BAD_ARG;
   if (N == 0) return IA_OK;
   const int P = N * top;
-  dim3 grid((W + TF_T - 1) / TF_T, (P + TF_T - 1) / TF_T + E);
-  if (grid.y > 65535u) return IA_ERR_UNSUPPORTED;
+  const long tiles = moe_most_tiles(P, E, TF_T);
+  const dim3 grid((W + TF_T - 1) / TF_T, (unsigned)tiles);
+  if (tiles > 65535) return IA_ERR_UNSUPPORTED;
   if (dtype == IA_F32)
     moe_down_kernel<float><<<grid, 256, 0, stream>>>((const float*)y, (const float*)Wd, parts, weights, offsets,
                                                             perm, E, top, N, W, ff);
   else if (dtype == IA_BF16 && tile_rows_aligned(y, ff) && tile_rows_aligned(Wd, ff)) {
-    const int bm = moe_tile_rows(P, E);
-    const int bn = bm == 128 ? 256 : TB_N;
-    dim3 big((W + bn - 1) / bn, (P + bm - 1) / bm + E);
-    if (big.y > 65535u) return IA_ERR_UNSUPPORTED;
-    if (bm == 128)
-      moe_down_big_kernel<128, 256><<<big, 512, 0, stream>>>((const bf16_t*)y, (const bf16_t*)Wd, parts, weights, offsets,
-                                                        perm, E, top, N, W, ff);
-    else
-      moe_down_big_kernel<32, TB_N><<<big, 256, 0, stream>>>((const bf16_t*)y, (const bf16_t*)Wd, parts, weights, offsets,
-                                                       perm, E, top, N, W, ff);
+    const MoeTile tile = moe_tile_for(P, E, W);
+    const long most = moe_most_tiles(P, E, moe_tile_rows(tile));
+    if (most > 65535) return IA_ERR_UNSUPPORTED;
+#define IA_DN(kernel, columns, threads)                                                                                     \
+  kernel<<<dim3((W + (columns) - 1) / (columns), (unsigned)most), threads, 0, stream>>>(                                    \
+      (const bf16_t*)y, (const bf16_t*)Wd, parts, weights, offsets, perm, E, top, N, W, ff)
+    switch (tile) {
+      case MOE_32_32: IA_DN((moe_down_stream_kernel<32, 2>), 32, 128); break;
+      case MOE_32_64: IA_DN((moe_down_stream_kernel<32, 4>), 64, 256); break;
+      case MOE_64_64: IA_DN((moe_down_stream_kernel<64, 4>), 64, 256); break;
+      case MOE_64_128: IA_DN((moe_down_stream_kernel<64, 8>), 128, 512); break;
+      case MOE_128_256: IA_DN(moe_down_big_kernel, 256, 512); break;
+    }
+#undef IA_DN
   }
   else if (dtype == IA_BF16)
     moe_down_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)y, (const bf16_t*)Wd, parts, weights,
@@ -578,49 +783,69 @@ __global__ __launch_bounds__(256) void moe_up_kernel(const T* __restrict__ x, co
   });
 }
 
-template <int BM, int BN>
-__global__ __launch_bounds__(BN == 256 ? 512 : 256) void moe_up_big_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ Wu,
-                                                              bf16_t* __restrict__ y, const int* __restrict__ offsets,
-                                                              const int* __restrict__ perm, int E, int top, int W,
-                                                              int ff, int act) {
-  __shared__ TileBigLds<BM, BN> lds;
+__device__ __forceinline__ void moe_up_store(bf16_t* __restrict__ y, int ff, int p, int c0, const float* v, int act) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (c0 + j < ff) y[(size_t)p * ff + c0 + j] = from_float<bf16_t>(moe_act(to_float(from_float<bf16_t>(v[j])), act));
+}
+
+__global__ __launch_bounds__(512) void moe_up_big_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ Wu,
+                                                         bf16_t* __restrict__ y, const int* __restrict__ offsets,
+                                                         const int* __restrict__ perm, int E, int top, int W, int ff, int act) {
+  __shared__ TileBigLds<128, 256> lds;
   int e, first, last;
-  if (!moe_tile(offsets, E, blockIdx.y, e, first, last, BM)) return;
-  const int n0 = blockIdx.x * BN;
-  tile_mfma_big<BM, BN>(
+  if (!moe_tile(offsets, E, blockIdx.y, e, first, last, 128)) return;
+  const int n0 = blockIdx.x * 256;
+  tile_mfma_big<128, 256>(
       [&](int r) { return x + (size_t)(perm[first + r] / top) * W; },
       [&](int r) { return Wu + ((size_t)e * ff + n0 + r) * W; }, last - first, ff - n0, W, lds,
       [&](int i, int j0, const float* v) {
-        const int p = first + i;
-        if (p >= last) return;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int c = n0 + j0 + j;
-          if (c < ff) y[(size_t)p * ff + c] = from_float<bf16_t>(moe_act(to_float(from_float<bf16_t>(v[j])), act));
-        }
-      });
+        if (first + i < last) moe_up_store(y, ff, first + i, n0 + j0, v, act);
+      }, moe_first_chunk(n0, W) * (MS_KC / TB_KS));
+}
+
+template <int ROWS, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void moe_up_stream_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ Wu,
+                                                                   bf16_t* __restrict__ y, const int* __restrict__ offsets,
+                                                                   const int* __restrict__ perm, int E, int top, int W, int ff,
+                                                                   int act) {
+  __shared__ __attribute__((aligned(16))) uint16_t xs[2][ROWS][MS_LD];
+  int e, first, last;
+  if (!moe_tile(offsets, E, blockIdx.y, e, first, last, ROWS)) return;
+  const int rows = min(last - first, ROWS), n0 = blockIdx.x * WAVES * 16;
+  const bf16_t* Wm = Wu + (size_t)e * ff * W;
+  auto x_row = [&](int r) { return x + (size_t)(perm[first + r] / top) * W; };
+  auto emit = [&](int i, int c0, const float* v) {
+    if (i < rows) moe_up_store(y, ff, first + i, c0, v, act);
+  };
+  moe_stream<ROWS, WAVES>(Wm, ff, n0, W, rows, x_row, xs, emit);
 }
 
 extern "C" int ia_moe_up(const void* x, const void* Wu, void* y, const int* offsets, const int* perm, int dtype, int P,
                          int E, int top, int W, int ff, int act, hipStream_t stream) {
   if (P < 0 || E <= 0 || top <= 0 || W <= 0 || ff <= 0 || act < 0 || act > 3) return IA_ERR_BAD_ARG;
   if (P == 0) return IA_OK;
-  dim3 grid((ff + TF_T - 1) / TF_T, (P + TF_T - 1) / TF_T + E);
-  if (grid.y > 65535u) return IA_ERR_UNSUPPORTED;
+  const long tiles = moe_most_tiles(P, E, TF_T);
+  const dim3 grid((ff + TF_T - 1) / TF_T, (unsigned)tiles);
+  if (tiles > 65535) return IA_ERR_UNSUPPORTED;
   if (dtype == IA_F32)
     moe_up_kernel<float><<<grid, 256, 0, stream>>>((const float*)x, (const float*)Wu, (float*)y, offsets, perm, E, top,
                                                    W, ff, act);
   else if (dtype == IA_BF16 && tile_rows_aligned(x, W) && tile_rows_aligned(Wu, W)) {
-    const int bm = moe_tile_rows(P, E);
-    const int bn = bm == 128 ? 256 : TB_N;
-    dim3 big((ff + bn - 1) / bn, (P + bm - 1) / bm + E);
-    if (big.y > 65535u) return IA_ERR_UNSUPPORTED;
-    if (bm == 128)
-      moe_up_big_kernel<128, 256><<<big, 512, 0, stream>>>((const bf16_t*)x, (const bf16_t*)Wu, (bf16_t*)y, offsets, perm,
-                                                           E, top, W, ff, act);
-    else
-      moe_up_big_kernel<32, TB_N><<<big, 256, 0, stream>>>((const bf16_t*)x, (const bf16_t*)Wu, (bf16_t*)y, offsets, perm,
-                                                          E, top, W, ff, act);
+    const MoeTile tile = moe_tile_for(P, E, ff);
+    const long most = moe_most_tiles(P, E, moe_tile_rows(tile));
+    if (most > 65535) return IA_ERR_UNSUPPORTED;
+#define IA_UP(kernel, columns, threads)                                                                                     \
+  kernel<<<dim3((ff + (columns) - 1) / (columns), (unsigned)most), threads, 0, stream>>>(                                   \
+      (const bf16_t*)x, (const bf16_t*)Wu, (bf16_t*)y, offsets, perm, E, top, W, ff, act)
+    switch (tile) {
+      case MOE_32_32: IA_UP((moe_up_stream_kernel<32, 2>), 32, 128); break;
+      case MOE_32_64: IA_UP((moe_up_stream_kernel<32, 4>), 64, 256); break;
+      case MOE_64_64: IA_UP((moe_up_stream_kernel<64, 4>), 64, 256); break;
+      case MOE_64_128: IA_UP((moe_up_stream_kernel<64, 8>), 128, 512); break;
+      case MOE_128_256: IA_UP(moe_up_big_kernel, 256, 512); break;
+    }
+#undef IA_UP
   } else if (dtype == IA_BF16)
     moe_up_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)x, (const bf16_t*)Wu, (bf16_t*)y, offsets, perm, E,
                                                     top, W, ff, act);

@@ -101,7 +101,7 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float tm_f32x4;
 // four consecutive columns of one row of the result, as a thread of the fp32 tile above does.  Every element is
 // summed in an order that depends on K alone.
 // `a_row(r)` / `w_row(r)`: row r of the tile's A / W (16-byte aligned, K a multiple of 8 and at least 8); row 0
-// always exists.
+// always exists.  `first_step`: the step of K, below their number, at which the walk begins (it wraps around).
 #define TB_KS 64
 #define TB_LD 72
 #define TB_N 128
@@ -119,7 +119,7 @@ constexpr int tile_big_threads() { return BN == 256 ? 512 : 256; }
 
 template <int BM, int BN = TB_N, typename ARow, typename WRow, typename Emit>
 __device__ __forceinline__ void tile_mfma_big(ARow a_row, WRow w_row, int a_rows, int w_rows, int K,
-                                              TileBigLds<BM, BN>& lds, Emit emit) {
+                                              TileBigLds<BM, BN>& lds, Emit emit, int first_step = 0) {
   static_assert((BM == 128 || BM == 32) && (BN == 128 || (BN == 256 && BM == 128)), "tiles of 128 x 128, 32 x 128, 128 x 256");
   constexpr int WAVES = tile_big_threads<BM, BN>() / 64;
   constexpr int WM = BM == 128 ? 2 : 1, WN = WAVES / WM;       // waves along the rows and the columns
@@ -143,8 +143,10 @@ __device__ __forceinline__ void tile_mfma_big(ARow a_row, WRow w_row, int a_rows
     for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = tm_f32x4{0.f, 0.f, 0.f, 0.f};
   const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
   uint4 ra[2][AR], rw[2][WR];
-  auto fetch = [&](int k0, uint4 (&xa)[AR], uint4 (&xw)[WR]) {
-    const int k = k0 + lk;
+  const int steps = (K + TB_KS - 1) / TB_KS;
+  auto fetch = [&](int i, uint4 (&xa)[AR], uint4 (&xw)[WR]) {
+    const int at = i + first_step;
+    const int k = i < steps ? (at < steps ? at : at - steps) * TB_KS + lk : K;      // past the last step: never multiplied with
     const int kc = k < K ? k : K - 8;                          // stays inside the row
 #pragma unroll
     for (int s = 0; s < AR; ++s) xa[s] = *reinterpret_cast<const uint4*>(ap[s] + kc);
@@ -179,21 +181,20 @@ __device__ __forceinline__ void tile_mfma_big(ARow a_row, WRow w_row, int a_rows
       }
     }
   };
-  const int steps = (K + TB_KS - 1) / TB_KS;
   fetch(0, ra[0], rw[0]);
-  fetch(TB_KS, ra[1], rw[1]);                                  // past K: zeros
+  fetch(1, ra[1], rw[1]);
   stage(ra[0], rw[0]);
   __syncthreads();
   for (int i = 0; i < steps; i += 2) {
     // step i: LDS holds it; set 0 is free for step i + 2, set 1 holds step i + 1
-    fetch((i + 2) * TB_KS, ra[0], rw[0]);
+    fetch(i + 2, ra[0], rw[0]);
     multiply();
     __syncthreads();
     if (i + 1 >= steps) break;
     stage(ra[1], rw[1]);
     __syncthreads();
     // step i + 1
-    fetch((i + 3) * TB_KS, ra[1], rw[1]);
+    fetch(i + 3, ra[1], rw[1]);
     multiply();
     __syncthreads();
     if (i + 2 >= steps) break;

@@ -314,20 +314,25 @@ def gemm_mfma_grouped(x: torch.Tensor, w: torch.Tensor, rows_at: torch.Tensor, o
     return out
 
 
-MOE_GROUPED_ROWS_AN_EXPERT = 48
+# From how many rows an expert on average the grouped form is ahead of the tiles behind the sort: sort to scatter, microseconds of
+# grouped / tiles with cold weights.  Gated: 32 experts of 1,408 x 2,048 at 48 / 96 / 128 rows 182 / 137, 201 / 178, 255 / 257; of
+# 2,432 x 4,096 445 / 398, 499 / 482, 625 / 631; 16 of 2,432 x 4,096 268 / 225, 291 / 288, 313 / 345.  Without a gate: 8 of
+# 4,800 x 4,096 at 48 / 56 / 64 rows 186 / 161, 189 / 167, 193 / 216.
+MOE_GROUPED_ROWS_AN_EXPERT = 112
+MOE_GROUPED_ROWS_A_PLAIN_EXPERT = 56
 
 
-def moe_grouped_from_tokens(E: int, top: int, W: int, ff: int, dtype: torch.dtype) -> int:
+def moe_grouped_from_tokens(E: int, top: int, W: int, ff: int, dtype: torch.dtype, gated: bool = True) -> int:
     """From how many tokens of a step on the routed experts take the grouped form of the LDS-tiled product (an
     expert then has some tens of rows on average); 0: never (32-bit, or sizes that product does not take: its
     inner dimensions W and ff must be multiples of 64)."""
     if dtype != torch.bfloat16 or W % 64 or ff % 64:
         return 0
-    return -(-MOE_GROUPED_ROWS_AN_EXPERT * E // top)
+    return -(-(MOE_GROUPED_ROWS_AN_EXPERT if gated else MOE_GROUPED_ROWS_A_PLAIN_EXPERT) * E // top)
 
 
-def moe_grouped_rows(N: int, E: int, top: int, W: int, ff: int, dtype: torch.dtype) -> bool:
-    first = moe_grouped_from_tokens(E, top, W, ff, dtype)
+def moe_grouped_rows(N: int, E: int, top: int, W: int, ff: int, dtype: torch.dtype, gated: bool = True) -> bool:
+    first = moe_grouped_from_tokens(E, top, W, ff, dtype, gated)
     return first > 0 and N >= first
 
 
@@ -1586,7 +1591,7 @@ def moe_plain_experts(x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
     y = torch.empty((max(P, 1), ff), dtype=x.dtype, device=x.device)
     code = DTYPE_CODE[x.dtype]
     _ok(_core().ia_moe_sort(_p(ids), _p(offsets), _p(perm), P, E, _stream()), "moe_sort")
-    if moe_grouped_rows(N, E, top, W, ff, x.dtype):
+    if moe_grouped_rows(N, E, top, W, ff, x.dtype, False):
         xs = torch.empty((P, W), dtype=x.dtype, device=x.device)
         _ok(_core().ia_moe_gather(_p(x), _p(perm), _p(xs), P, top, W, _stream()), "moe_gather")
         gemm_mfma_grouped(xs, w_up, offsets, y)

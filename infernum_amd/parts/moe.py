@@ -246,7 +246,7 @@ class RoutedExperts(FeedForward):
         from .linear import emit_linear as emit
         H, I, E, top, T, N = self.hidden_size, self.ff, self.num_experts, self.top, program.T, program.N
         act, code = K.ACTIVATIONS[self.activation], program.act_code
-        first = K.moe_grouped_from_tokens(E, top, H, I, self.rt.dtype)
+        first = K.moe_grouped_from_tokens(E, top, H, I, self.rt.dtype, False)
         grouped = Guard.between(N, first) if 0 < first <= T else NEVER
         tiled = ~grouped
         program.op("core", "ia_moe_up", [program.x, self.w_gate_up, y, offsets, perm, code, N * top, E, top, H, I, act,

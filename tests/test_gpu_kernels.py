@@ -1564,3 +1564,41 @@ def test_a_pairs_result_does_not_depend_on_the_steps_other_pairs(gated, E, top, 
     want = parts_of(most)
     for N in (1,) + counts:
         assert torch.equal(parts_of(N), want[:, :N]), N
+
+
+# every tile behind the sort, with as many pairs of an expert as fill its groups of sixteen rows or are one more or one less:
+# tiles of 32 x 32 and 32 x 64, of 64 x 64, of 64 x 128, and of 128 x 256 for the first and for the second product; K that
+# ends within a chunk of 256 and within a step of 64; an expert without pairs
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("counts,W,ff", [((1, 16, 0, 17), 136, 208), ((9, 0, 11, 3, 1, 2, 5, 7), 4616, 4624), ((1, 16, 17, 32, 33), 520, 336),
+                                         ((65, 64, 49, 48, 33, 17, 1, 0), 2440, 2448), ((129, 65, 17), 136, 14352),
+                                         ((129, 65, 17), 14344, 144)])
+def test_routed_experts_tile_by_tile(gated, counts, W, ff):
+    api = K()
+    E, N = len(counts), sum(counts)
+    ff //= 2 if gated else 1
+    x = _rand(N, W, dtype=torch.bfloat16, seed=1)
+    up = _rand(E, (2 if gated else 1) * ff, W, dtype=torch.bfloat16, scale=2 * W ** -0.5, seed=2)
+    down = _rand(E, W, ff, dtype=torch.bfloat16, scale=ff ** -0.5, seed=3)
+    expert = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(N, generator=torch.Generator().manual_seed(4))]
+    ids = expert.int()[:, None].to(DEV)
+    wts = torch.rand(N, 1, generator=torch.Generator().manual_seed(5)).to(DEV)
+
+    def parts_of(rows):
+        parts = torch.full((1, len(rows), W), 7.0, device=DEV)
+        if gated:
+            api.moe_experts(x[rows], ids[rows], wts[rows], up, down, 7.0, 1.702, 1.0, E, parts)
+        else:
+            api.moe_plain_experts(x[rows], ids[rows], wts[rows], up, down, "relu_squared", parts)
+        return parts[0]
+    got = parts_of(list(range(N)))
+    z = torch.einsum("nw,nfw->nf", x[:4].double(), up[expert[:4]].double()).bfloat16().double()
+    y = z[:, 0::2].clamp(max=7.0), (z[:, 1::2].clamp(-7.0, 7.0) + 1.0) if gated else None
+    y = y[0] * torch.sigmoid(1.702 * y[0]) * y[1] if gated else z.clamp(min=0.0) ** 2
+    want = torch.einsum("nf,nwf->nw", y.bfloat16().double(), down[expert[:4]].double()).bfloat16().double() * wts[:4].double()
+    # as above: roundings to bfloat16 (2^-9) that fall the other way
+    assert float((got[:4].double() - want).norm() / want.norm()) <= 4 * 2.0 ** -9
+    for e in range(E):
+        mine = torch.nonzero(expert == e).flatten().tolist()
+        for n in mine[:1] + mine[len(mine) // 2:len(mine) // 2 + 1] + mine[-1:]:
+            assert torch.equal(parts_of([n])[0], got[n]), (e, n)          # alone: tiles of 32 x 32
