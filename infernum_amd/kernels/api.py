@@ -858,10 +858,14 @@ def decode_splits(batch: int, nh: int, nkv: int, max_len: int, device: Optional[
       heads, one request, whole against two parts: 150 keys of 64 values 7.5 us and 8.8, of 128 values 8.9 and 10.0; 250
       keys 8.0 and 8.7, 9.8 and 10.2; from 320 keys of 128 values on four parts are 1 us faster);
     * above 128 a compute unit holds one workgroup, and more parts than compute units only cost (head size 256, 32
-      requests on 4 key/value heads: 19 us in two parts, 23 in four);
-    * the join grows with the parts as the work of a part shrinks with them: the best number of parts for one
-      request went with the square root of its tiles (4 parts at 512 keys, 8 at 2,048, 16 at 8,192, 32 at 32,768, for
-      head sizes 64, 128 and 256 alike), so that bounds the parts; never more than 64."""
+      requests on 4 key/value heads: 19 us in two parts, 23 in four); at 65 to 128, where eight waves take a part,
+      three quarters of the compute units do better than all from eight parts on (4 requests on 8 key/value heads of 128,
+      2,048 / 4,096 keys: 16.3 / 22.6 us in six parts, 17.8 / 22.9 in eight);
+    * the join, which asks for sixteen parts' results at once, costs little, so a wave should have a tile or two: up to
+      a part for four tiles (six, up to a head size of 128), and for long requests with the square root of the tiles (one
+      request of 16 heads of 256 on one key/value head, 1,024 / 2,048 / 4,096 / 16,384 keys: 18.2 / 21.6 / 24.1 / 35.9 us in
+      5 / 8 / 11 / 24 parts, 15.3 / 16.5 / 19.5 / 26.2 in 16 / 22 / 32 / 64; of 8 key/value heads of 128 at 1,000 / 2,048 /
+      4,096: 13.1 / 14.3 / 15.0 in 5 / 8 / 11, 11.4 / 12.5 / 13.9 in 10 / 17 / 24); never more than 64."""
     if head_dim <= 128 and max_len <= 256:
         return 1
     cus = compute_units(device)
@@ -871,10 +875,13 @@ def decode_splits(batch: int, nh: int, nkv: int, max_len: int, device: Optional[
     if 8 * groups >= 5 * fill:
         return 1
     if head_dim > 128:
-        wanted = fill // groups
+        wanted, most = fill // groups, min(tiles // 4, math.isqrt(4 * tiles))
     else:
         wanted = fill // groups if 4 * groups <= fill else 2 * fill // groups
-    return max(1, min(wanted, math.isqrt(tiles // 2), 64))
+        if head_dim > 64 and wanted >= 8:
+            wanted = 3 * fill // (4 * groups)
+        most = min(tiles // 6, math.isqrt(9 * tiles // 4))
+    return max(1, min(wanted, most, 64))
 
 
 def attention_decode(qkv: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, out: torch.Tensor,
