@@ -396,6 +396,20 @@ static int skinny_splits(int N, int K) {
   return split_count(nchunks, (SK_TARGET_BLOCKS + nb - 1) / nb);
 }
 
+// Whether both halves of [gate | up] take all of K in every workgroup, activation included, although K of a weight [N, K] is split:
+// a split product with this use has to be joined in a launch of its own, which is worth more than full compute units from some
+// 150 workgroups on (168 with longer K).  Both sides with cold weights, whole / in parts and the join, us at 1, 16, 64 and 128 rows:
+// 11,008 x 2,048 12.7 / 13.9, 13.6 / 15.2, 16.7 / 20.9, 23.7 / 27.7; 9,600 x 2,048 (150 workgroups) 12.8 / 13.5, 13.2 / 13.9, 16.5 / 18.8,
+// 23.8 / 25.5; 11,008 x 4,096 (172) 21.1 / 23.8, 22.9 / 25.1, 28.4 / 30.9, 39.8 / 41.7; 15,360 x 4,096 25.2 / 26.9, 25.3 / 29.1, 30.1 / 35.5,
+// 41.0 / 47.2.  Below: 10,240 x 4,096 (160) 21.2 / 21.0, 22.7 / 22.1, 28.0 / 28.0, 39.9 / 37.0; 7,168 x 2,048 (112) 12.2 / 9.0, 12.1 / 11.1.
+static bool glu_whole(int N, int K) {
+  const int nb = (N + SK_BN - 1) / SK_BN;
+  if (skinny_splits(N, K) == 1) return true;
+  for (int i = 0; i < g_known_count; ++i)
+    if (g_known_splits[i].N == N && g_known_splits[i].K == K) return false;
+  return nb >= (K <= 2048 ? 150 : 168);
+}
+
 // Says into how many parts (about: the chunks of K are dealt out evenly) the inner dimension of a weight [N, K] is
 // split from now on, in place of the rule of sizes.  To be called before the first product of that shape (the
 // partial sums' layout follows the number).  Returns 0, or 10001 for bad arguments or a full table.
@@ -538,7 +552,8 @@ static int skinny_product(const void* X, const void* W, void* C, int out_dtype, 
   if (splits > 65535) return IA_ERR_UNSUPPORTED;
   const uint16_t* x = (const uint16_t*)X;
   const uint16_t* w = (const uint16_t*)W;
-  if (splits == 1 && epilogue == SK_EPI_SWIGLU && C != nullptr) {
+  if (splits > 1 && (!workspace || workspace_floats < (size_t)splits * M * N)) return IA_ERR_BAD_ARG;
+  if (epilogue == SK_EPI_SWIGLU && C != nullptr && glu_whole(N, K)) {
     // one pass: both halves of W in the same wave, the activation in the epilogue
     if (out_dtype == IA_F32) return launch_skinny<true, float, TILED>(x, w, (float*)C, nullptr, M, N, K, 1, stream);
     return launch_skinny<true, uint16_t, TILED>(x, w, (uint16_t*)C, nullptr, M, N, K, 1, stream);
@@ -581,7 +596,7 @@ extern "C" int ia_gemm_skinny(const void* X, const void* W, void* C, int out_dty
 // ---- the weight laid out for the kernel: every workgroup's 64 rows x 256 values of a chunk consecutive ----------
 // Whether the copy for this weight and use is laid out for the kernel that multiplies with both halves of
 // [gate | up] at once (a workgroup then takes 32 rows of each half).
-static bool tiled_glu(int N, int K, int epilogue) { return epilogue == SK_EPI_SWIGLU && skinny_splits(N, K) == 1; }
+static bool tiled_glu(int N, int K, int epilogue) { return epilogue == SK_EPI_SWIGLU && glu_whole(N, K); }
 
 // Elements (bf16) of the copy: rows padded to whole workgroups, K to whole chunks.
 extern "C" size_t ia_gemm_skinny_tiled_elements(int N, int K, int epilogue) {

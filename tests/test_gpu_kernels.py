@@ -443,6 +443,26 @@ def test_gemm_skinny_rounds_one_after_the_other(M, N, K_, tiled):
             assert torch.equal(got[m:m + 1], api.gemm_skinny(a[m:m + 1], w, **kw))
 
 
+# both halves whole in a workgroup although the weight is split (glu_whole): the smallest and largest of either range of K, columns
+# that fill no group of 16, a last chunk that is not full; the copy leaves the same bits, and a row those it has alone
+@pytest.mark.parametrize("M", [1, 16, 33, 128])
+@pytest.mark.parametrize("N,K_", [(9538, 2048), (9602, 520), (16320, 776), (10690, 2056), (16318, 4096)])
+def test_gemm_skinny_glu_whole_where_the_weight_is_split(M, N, K_):
+    api = K()
+    assert api.gemm_skinny_splits(N, K_) > 1
+    a, w = _rand(M, K_, dtype=torch.bfloat16, seed=31), _rand(N, K_, dtype=torch.bfloat16, scale=0.05, seed=32)
+    got = api.gemm_skinny(a, w, epilogue="swiglu", out_dtype=torch.float32)
+    y = a.double() @ w.double().t()
+    g, u = y[:, :N // 2], y[:, N // 2:]
+    # fp32 sums of K exact products: each within K 2^-24 of the sum of their sizes; silu has a slope of at most 1.1
+    e = K_ * 2.0 ** -24 * (a.double().abs() @ w.double().abs().t())
+    eg, eu = e[:, :N // 2], e[:, N // 2:]
+    assert bool(((got.double() - g / (1 + torch.exp(-g)) * u).abs() <= eg * 1.1 * (u.abs() + eu) + (g.abs() + eg) * eu + 1e-6 * (g * u).abs()).all())
+    assert torch.equal(api.gemm_skinny(a, w, epilogue="swiglu", out_dtype=torch.float32, tiled=api.tile_weight(w, "swiglu")), got)
+    assert torch.equal(api.gemm_skinny(a[M - 1:], w, epilogue="swiglu", out_dtype=torch.float32)[0], got[M - 1])
+    assert torch.equal(api.gemm_skinny(a, w, epilogue="swiglu"), got.bfloat16())
+
+
 # one workgroup with all of K against the parts and their sum in the order of their index: columns that fill no group of
 # 16, a last chunk that is not full, one to sixteen parts, two chunks and more a part, both halves of [gate | up]
 @pytest.mark.parametrize("M", [1, 5, 16])
