@@ -36,23 +36,49 @@ __device__ __forceinline__ void router_finish(int mine_e, float mine_w, int top,
   weights[last] = mine_w * factor;
 }
 
-// PL: experts a lane holds (32 experts, one token: 4.4 us with one a lane, 9.0 with sixteen)
+// Up to 64 experts, one a lane: the place of this lane's expert among all, largest first and the lowest index among equals (64 for
+// an expert that cannot be chosen).  Every lane compares with every expert, whose values come as scalars: no step waits
+// for the one before, where `top` rounds of a maximum over the wave are chains of twelve exchanges each (1 / 64 tokens to 4 of 32 with
+// join and sort 7.3 / 8.5 us in rounds, 6.2 / 7.3 so; to 8 of 64 10.5 / 12.0 and 9.0 / 9.8).
+__device__ __forceinline__ int expert_rank(float x, bool can, int E, int lane) {
+  const int b = __float_as_int(x + 0.0f);                  // -0 counts as 0
+  const int key = can ? b ^ ((b >> 31) & 0x7fffffff) : (int)0x80000000;      // in the order of the values
+  int rank = 0;
+#pragma unroll 8
+  for (int i = 0; i < E; ++i) {
+    const int other = __builtin_amdgcn_readlane(key, i);
+    rank += (other > key || (other == key && i < lane)) ? 1 : 0;
+  }
+  return can ? rank : 64;
+}
+// The value of the lane with rank k, for all lanes.
+__device__ __forceinline__ float value_of_rank(float v, int rank, int k) {
+  const unsigned long long who = __ballot(rank == k);
+  return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), who ? __ffsll(who) - 1 : 0));
+}
+
+// PL: experts a lane holds (32 experts, one token: 4.4 us with one a lane, 9.0 with sixteen).  v: this lane's logits with their
+// biases; leaves the token's choices and weights at ids and weights, and with one expert a lane its place among them in mine_rank.
 template <int PL>
-__global__ __launch_bounds__(256) void router_topk_kernel(const float* __restrict__ logits,
-                                                          const void* __restrict__ bias, int bias_dtype,
-                                                          int* __restrict__ ids, float* __restrict__ weights, int N,
-                                                          int E, int top) {
-  const int n = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (n >= N) return;
-  const float* z = logits + (size_t)n * E;
-  float v[PL];
+__device__ __forceinline__ void choose_then_softmax(const float (&v)[PL], int E, int top, int lane, int* ids, float* weights, int& mine_rank) {
+  if constexpr (PL == 1) {
+    // a value that compares with nothing (NaN) counts as the smallest
+    const float x = (v[0] == v[0]) ? v[0] : -INFINITY;
+    const int rank = expert_rank(x, lane < E, E, lane);
+    const float w = expf(x - value_of_rank(x, rank, 0));
+    float sum = 0.f;
+    for (int k = 0; k < top; ++k) sum += value_of_rank(w, rank, k);
+    if (rank < top) {
+      ids[rank] = lane;
+      weights[rank] = w * (1.0f / sum);
+    }
+    mine_rank = rank;
+    return;
+  }
   unsigned taken = 0u;
 #pragma unroll
-  for (int c = 0; c < PL; ++c) {
-    const int e = lane + 64 * c;
-    v[c] = e < E ? z[e] + (bias ? load_as_float(bias, bias_dtype, e) : 0.f) : -INFINITY;
-    if (e >= E) taken |= 1u << c;
-  }
+  for (int c = 0; c < PL; ++c)
+    if (lane + 64 * c >= E) taken |= 1u << c;
   float first_v = 0.f, sum = 0.f, mine_w = 0.f;
   int mine_e = 0;
   for (int k = 0; k < top; ++k) {
@@ -78,9 +104,27 @@ __global__ __launch_bounds__(256) void router_topk_kernel(const float* __restric
     if (k == 0) first_v = best_v;
     const float w = expf(best_v - first_v);
     sum += w;
-    router_keep(mine_e, mine_w, k, lane, best_e, w, ids + (size_t)n * top, weights + (size_t)n * top);
+    router_keep(mine_e, mine_w, k, lane, best_e, w, ids, weights);
   }
-  router_finish(mine_e, mine_w, top, lane, 1.0f / sum, ids + (size_t)n * top, weights + (size_t)n * top);
+  router_finish(mine_e, mine_w, top, lane, 1.0f / sum, ids, weights);
+}
+
+template <int PL>
+__global__ __launch_bounds__(256) void router_topk_kernel(const float* __restrict__ logits,
+                                                          const void* __restrict__ bias, int bias_dtype,
+                                                          int* __restrict__ ids, float* __restrict__ weights, int N,
+                                                          int E, int top) {
+  const int n = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (n >= N) return;
+  const float* z = logits + (size_t)n * E;
+  float v[PL];
+#pragma unroll
+  for (int c = 0; c < PL; ++c) {
+    const int e = lane + 64 * c;
+    v[c] = e < E ? z[e] + (bias ? load_as_float(bias, bias_dtype, e) : 0.f) : -INFINITY;
+  }
+  int rank;
+  choose_then_softmax<PL>(v, E, top, lane, ids + (size_t)n * top, weights + (size_t)n * top, rank);
 }
 
 extern "C" int ia_router_topk(const float* logits, const void* bias, int bias_dtype, int* ids, float* weights, int N,
@@ -641,24 +685,19 @@ __device__ __forceinline__ float moe_act(float z, int act) {
   return z;
 }
 
-// PL: experts a lane holds (lane, lane + 64, ...)
+// PL: experts a lane holds (lane, lane + 64, ...).  zv: this lane's logits; scores: 64 PL floats of LDS, this wave's own (read
+// with groups only); the rest as for choose_then_softmax.
 template <int PL>
-__global__ __launch_bounds__(256) void router_softmax_topk_kernel(const float* __restrict__ logits,
-                                                                  const void* __restrict__ corr, int corr_dtype,
-                                                                  int* __restrict__ ids, float* __restrict__ weights,
-                                                                  int N, int E, int top, int z_stride, int groups,
-                                                                  int keep, int renorm, int sigmoid) {
-  __shared__ float s_v[4][64 * PL];       // a wave's choice scores, then (in place) its groups' scores
-  const int n = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (n >= N) return;
-  const float* z = logits + (size_t)n * z_stride;
+__device__ __forceinline__ void softmax_then_choose(const float (&zv)[PL], const void* __restrict__ corr, int corr_dtype, int E, int top,
+                                                    int groups, int keep, int renorm, int sigmoid, int lane, float* scores,
+                                                    int* ids, float* weights, int& mine_rank) {
   float s[PL], v[PL];
   unsigned taken = 0u;
   float zmax = -INFINITY;
 #pragma unroll
   for (int c = 0; c < PL; ++c) {
     const int e = lane + 64 * c;
-    s[c] = e < E ? z[e] : -INFINITY;
+    s[c] = e < E ? zv[c] : -INFINITY;
     zmax = fmaxf(zmax, s[c]);
     if (e >= E) taken |= 1u << c;
   }
@@ -675,7 +714,7 @@ __global__ __launch_bounds__(256) void router_softmax_topk_kernel(const float* _
   for (int c = 0; c < PL; ++c) {
     const int e = lane + 64 * c;
     if (sigmoid) {
-      const float x = e < E ? z[e] : -INFINITY;
+      const float x = e < E ? zv[c] : -INFINITY;
       s[c] = 1.0f / (1.0f + expf(-x));
       v[c] = e < E ? (corr ? s[c] + load_as_float(corr, corr_dtype, e) : x) : -INFINITY;
     } else {
@@ -685,7 +724,7 @@ __global__ __launch_bounds__(256) void router_softmax_topk_kernel(const float* _
   }
   if (groups > 1) {
     // each wave works on its own part of LDS: a wave's accesses are in order, no barrier is needed between them
-    volatile float* mine = s_v[threadIdx.x >> 6];
+    volatile float* mine = scores;
     const int size = E / groups;
 #pragma unroll
     for (int c = 0; c < PL; ++c)
@@ -714,6 +753,17 @@ __global__ __launch_bounds__(256) void router_softmax_topk_kernel(const float* _
       if (better >= keep) taken |= 1u << c;
     }
   }
+  if constexpr (PL == 1) {
+    const int rank = expert_rank((v[0] == v[0]) ? v[0] : -INFINITY, !(taken & 1u), E, lane);
+    float chosen = 0.f;
+    for (int k = 0; k < top; ++k) chosen += value_of_rank(s[0], rank, k);
+    if (rank < top) {
+      ids[rank] = lane;
+      weights[rank] = s[0] * (renorm ? 1.0f / (chosen + 1e-20f) : 1.0f);
+    }
+    mine_rank = rank;
+    return;
+  }
   float sum = 0.f, mine_w = 0.f;
   int mine_e = 0;
   for (int k = 0; k < top; ++k) {
@@ -737,9 +787,27 @@ __global__ __launch_bounds__(256) void router_softmax_topk_kernel(const float* _
     }
     if ((best_e & 63) == lane) taken |= 1u << (best_e >> 6);
     sum += best_s;
-    router_keep(mine_e, mine_w, k, lane, best_e, best_s, ids + (size_t)n * top, weights + (size_t)n * top);
+    router_keep(mine_e, mine_w, k, lane, best_e, best_s, ids, weights);
   }
-  router_finish(mine_e, mine_w, top, lane, renorm ? 1.0f / (sum + 1e-20f) : 1.0f, ids + (size_t)n * top, weights + (size_t)n * top);
+  router_finish(mine_e, mine_w, top, lane, renorm ? 1.0f / (sum + 1e-20f) : 1.0f, ids, weights);
+}
+
+template <int PL>
+__global__ __launch_bounds__(256) void router_softmax_topk_kernel(const float* __restrict__ logits,
+                                                                  const void* __restrict__ corr, int corr_dtype,
+                                                                  int* __restrict__ ids, float* __restrict__ weights,
+                                                                  int N, int E, int top, int z_stride, int groups,
+                                                                  int keep, int renorm, int sigmoid) {
+  __shared__ float s_v[4][64 * PL];       // a wave's choice scores, then (in place) its groups' scores
+  const int n = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (n >= N) return;
+  const float* z = logits + (size_t)n * z_stride;
+  float zv[PL];
+#pragma unroll
+  for (int c = 0; c < PL; ++c) zv[c] = lane + 64 * c < E ? z[lane + 64 * c] : -INFINITY;
+  int rank;
+  softmax_then_choose<PL>(zv, corr, corr_dtype, E, top, groups, keep, renorm, sigmoid, lane, s_v[threadIdx.x >> 6],
+                          ids + (size_t)n * top, weights + (size_t)n * top, rank);
 }
 
 extern "C" int ia_router_softmax_topk(const float* logits, const void* corr, int corr_dtype, int* ids, float* weights,
@@ -758,6 +826,129 @@ extern "C" int ia_router_softmax_topk(const float* logits, const void* corr, int
 #undef IA_RT
   IA_LAUNCH_CHECK();
   return IA_OK;
+}
+
+// ---- a step of few tokens: the parts of the router's product joined, the choices and the sort ---------------------------
+// The join of the logits' parts, ia_router_topk or ia_router_softmax_topk and ia_moe_sort are three launches and a few trips to
+// memory for some kilobytes.  Up to 16 tokens one workgroup does the lot: all threads join the logits into LDS (the
+// parts in the order of their index), a wave a token chooses, and the ids go into the sort from LDS.  With more tokens one compute unit
+// takes longer than the launches it saves, and the parts are joined where a wave a token chooses, the sort behind it.  The same
+// ids, weights and offsets.  Behind the product's parts, us with a launch each and so: 1 / 16 / 32 / 64 / 128 tokens to 4 of 32 experts
+// 6.2 / 6.9 / 7.1 / 7.3 / 7.5 and 3.9 / 5.1 / 5.5 / 5.6 / 5.7 (one workgroup for all of 32 / 64 / 128: 8.4 / 14.5 / 26.4).
+#define ROUTE_ONE 16
+#define ROUTE_TOKENS 128
+#define ROUTE_EXPERTS 64
+#define ROUTE_TOP 16
+struct RouteArgs {
+  const float* parts;        // [splits, N, row]: the logits of the experts (and, with gate, one more per token)
+  int splits, row;
+  const void* bias;          // the choice's bias or correction (nullable)
+  int bias_dtype;
+  int* ids;                  // [N, top]
+  float* weights;            // [N, top]
+  int* offsets;              // [E + 1]
+  int* perm;                 // [N * top]
+  float* gate;               // nullable: gate[n] = the logit behind the experts'
+  int N, E, top, softmax_first, groups, keep, renorm, sigmoid;
+};
+
+// Value i of [N, row], its parts added in the order of their index, eight asked for together.
+__device__ __forceinline__ float route_logit(const RouteArgs& A, int i) {
+  const int values = A.N * A.row;
+  float sum = 0.f;
+  for (int s0 = 0; s0 < A.splits; s0 += 8) {
+    float p[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) p[u] = A.parts[(size_t)min(s0 + u, A.splits - 1) * values + i];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) sum = s0 + u < A.splits ? sum + p[u] : sum;
+  }
+  return sum;
+}
+
+// Token n's choices; z: this lane's logit (any number beyond the experts).  Returns this lane's expert's place among them.
+__device__ __forceinline__ int route_token(const RouteArgs& A, int n, float z, int lane, float* scores) {
+  int* ids = A.ids + (size_t)n * A.top;
+  float* weights = A.weights + (size_t)n * A.top;
+  int rank;
+  if (A.softmax_first) {
+    const float zv[1] = {lane < A.E ? z : -INFINITY};
+    softmax_then_choose<1>(zv, A.bias, A.bias_dtype, A.E, A.top, A.groups, A.keep, A.renorm, A.sigmoid, lane, scores, ids, weights, rank);
+  } else {
+    const float v[1] = {lane < A.E ? z + (A.bias ? load_as_float(A.bias, A.bias_dtype, lane) : 0.f) : -INFINITY};
+    choose_then_softmax<1>(v, A.E, A.top, lane, ids, weights, rank);
+  }
+  return rank;
+}
+
+__global__ __launch_bounds__(1024) void moe_route_kernel(RouteArgs A) {
+  __shared__ float z[ROUTE_ONE * (ROUTE_EXPERTS + 1)];
+  __shared__ float scores[ROUTE_ONE][ROUTE_EXPERTS];
+  __shared__ int chosen[ROUTE_ONE * ROUTE_TOP];
+  __shared__ int cnt[ROUTE_EXPERTS], cur[ROUTE_EXPERTS];
+  const int tid = threadIdx.x, lane = tid & 63, n = tid >> 6;
+  if (tid < A.E) cnt[tid] = 0;
+  for (int i = tid; i < A.N * A.row; i += 1024) z[i] = route_logit(A, i);
+  __syncthreads();
+  if (n < A.N) {
+    const float* zn = z + n * A.row;
+    const int rank = route_token(A, n, zn[min(lane, A.E - 1)], lane, scores[n]);
+    if (rank < A.top) {
+      chosen[n * A.top + rank] = lane;
+      atomicAdd(&cnt[lane], 1);
+    }
+    if (A.gate && lane == 0) A.gate[n] = zn[A.E];
+  }
+  __syncthreads();
+  if (n == 0) {
+    const int own = lane < A.E ? cnt[lane] : 0;
+    int upto = own;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(upto, o, IA_WAVE);
+      upto += lane >= o ? v : 0;
+    }
+    if (lane < A.E) {
+      cur[lane] = upto - own;
+      A.offsets[lane] = upto - own;
+    }
+    if (lane == A.E - 1) A.offsets[A.E] = upto;
+  }
+  __syncthreads();
+  for (int p = tid; p < A.N * A.top; p += 1024) A.perm[atomicAdd(&cur[chosen[p]], 1)] = p;
+}
+
+__global__ __launch_bounds__(256) void moe_choose_kernel(RouteArgs A) {
+  __shared__ float scores[4][ROUTE_EXPERTS];
+  const int lane = threadIdx.x & 63, n = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (n >= A.N) return;
+  const float z = route_logit(A, n * A.row + min(lane, A.row - 1));
+  route_token(A, n, z, lane, scores[threadIdx.x >> 6]);
+  if (A.gate && A.E < 64 && lane == A.E) A.gate[n] = z;
+  if (A.gate && A.E == 64 && lane == 0) A.gate[n] = route_logit(A, n * A.row + 64);
+}
+
+// Whether ia_moe_route takes a step of N tokens.
+extern "C" int ia_moe_route_takes(int N, int E, int top) {
+  return N >= 1 && N <= ROUTE_TOKENS && E >= 1 && E <= ROUTE_EXPERTS && top >= 1 && top <= ROUTE_TOP && top <= E;
+}
+
+// parts: fp32 [splits, N, row], row E, or E + 1 with gate (fp32 [N], nullable): the logit behind the experts' goes there.
+// softmax_first != 0: as ia_router_softmax_topk chooses, with bias its correction (nullable); else as ia_router_topk (groups
+// 1, keep 1).  ids, weights [N, top], offsets [E + 1], perm [N * top].
+extern "C" int ia_moe_route(const float* parts, int splits, int row, const void* bias, int bias_dtype, int* ids, float* weights,
+                            int* offsets, int* perm, float* gate, int N, int E, int top, int softmax_first, int groups, int keep,
+                            int renorm, int sigmoid, hipStream_t stream) {
+  if (N < 0 || E <= 0 || top <= 0 || top > E || splits < 1 || row != E + (gate ? 1 : 0) || groups < 1 || E % groups || keep < 1 ||
+      keep > groups || top > keep * (E / groups) || !parts || !ids || !weights || !offsets || !perm) return IA_ERR_BAD_ARG;
+  if (N == 0) return IA_OK;
+  if (!ia_moe_route_takes(N, E, top)) return IA_ERR_UNSUPPORTED;
+  const RouteArgs A{parts, splits, row, bias, bias_dtype, ids, weights, offsets, perm, gate, N, E, top, softmax_first, groups,
+                    keep, renorm, sigmoid};
+  if (N <= ROUTE_ONE) moe_route_kernel<<<1, 1024, 0, stream>>>(A);
+  else moe_choose_kernel<<<(N + 3) / 4, 256, 0, stream>>>(A);
+  IA_LAUNCH_CHECK();
+  return N <= ROUTE_ONE ? IA_OK : ia_moe_sort(ids, offsets, perm, N * top, E, stream);
 }
 
 template <typename T>
@@ -942,6 +1133,7 @@ extern "C" int ia_moe_extras(const void* x, int dtype, const int* ids, const flo
 IA_OP(ia_moe_extras)
 IA_OP(ia_router_topk)
 IA_OP(ia_moe_sort)
+IA_OP(ia_moe_route)
 IA_OP(ia_moe_gate_up)
 IA_OP(ia_moe_down)
 IA_OP(ia_moe_gather)

@@ -314,6 +314,38 @@ def gemm_mfma_grouped(x: torch.Tensor, w: torch.Tensor, rows_at: torch.Tensor, o
     return out
 
 
+ROUTE_MOST_TOKENS = 128
+
+
+def moe_route_takes(N: int, E: int, top: int) -> bool:
+    """Whether :func:`moe_route` takes a step of N tokens (up to 128) to ``top`` (16) of E (64) experts."""
+    return bool(_core().ia_moe_route_takes(int(N), int(E), int(top)))
+
+
+def moe_route(logits, bias: Optional[torch.Tensor], top: int, experts: int, softmax_first: bool = False, groups: int = 1,
+              keep: int = 1, renorm: bool = True, sigmoid: bool = False):
+    """The choices of :func:`router_softmax_topk` (``softmax_first``) or :func:`router_topk` and the sort of the pairs by
+    expert, for few tokens in one launch.  ``logits``: fp32 [N, experts], or a :class:`SplitSum` of it; with one column more
+    that column's values come back too.  Returns (ids [N, top], weights [N, top], offsets [experts + 1], perm [N top],
+    the column behind the experts' or None)."""
+    src = logits.parts if isinstance(logits, SplitSum) else logits[None]
+    _dev(src, bias)
+    splits, N, row = src.shape
+    _need(src.dtype == torch.float32 and src.is_contiguous() and row in (experts, experts + 1), "moe_route: fp32 logits [N, experts (+ 1)]")
+    _need(moe_route_takes(N, experts, top), f"moe_route: {N} tokens to {top} of {experts} experts")
+    _need(bias is None or (bias.dtype in DTYPE_CODE and bias.numel() == experts), "moe_route: bias [experts]")
+    dev = src.device
+    ids = torch.empty((N, top), dtype=torch.int32, device=dev)
+    weights = torch.empty((N, top), dtype=torch.float32, device=dev)
+    offsets = torch.empty(experts + 1, dtype=torch.int32, device=dev)
+    perm = torch.empty(N * top, dtype=torch.int32, device=dev)
+    gate = torch.empty(N, dtype=torch.float32, device=dev) if row > experts else None
+    _ok(_core().ia_moe_route(_p(src), splits, row, _p(bias), DTYPE_CODE[bias.dtype] if bias is not None else 0, _p(ids), _p(weights),
+                             _p(offsets), _p(perm), _p(gate), N, experts, top, int(softmax_first), groups, keep, int(renorm),
+                             int(sigmoid), _stream()), "moe_route")
+    return ids, weights, offsets, perm, gate
+
+
 # From how many rows an expert on average the grouped form is ahead of the tiles behind the sort: sort to scatter, microseconds of
 # grouped / tiles with cold weights.  Gated: 32 experts of 1,408 x 2,048 at 48 / 96 / 128 rows 182 / 137, 201 / 178, 255 / 257; of
 # 2,432 x 4,096 445 / 398, 499 / 482, 625 / 631; 16 of 2,432 x 4,096 268 / 225, 291 / 288, 313 / 345.  Without a gate: 8 of

@@ -177,11 +177,13 @@ class RoutedExperts(FeedForward):
     def native(self, program, view=None) -> None:
         if type(self).forward is not RoutedExperts.forward:
             return super().native(program, view)
-        from ..engine.program import ALWAYS, STREAM, Alt, Value
+        from ..engine.program import ALWAYS, NEVER, STREAM, Alt, Guard, Value
         H, I, E, top, T, N = self.hidden_size, self.ff, self.num_experts, self.top, program.T, program.N
         total = self.total
         program.keep(self.w_router, self.b_router, self.w_gate_up, self.w_down)
-        z = emit_linear(program, program.x, N, self.w_router, torch.float32, None, False, "moe.logits", "moe.router")
+        # few tokens: parts of the logits, choices and sort in one launch (kernels.api.moe_route); else one after the other
+        route = K.moe_route_takes(1, total, top)
+        z = emit_linear(program, program.x, N, self.w_router, torch.float32, None, route, "moe.logits", "moe.router")
         ids = program.buffer("moe.ids", T * top * 4)
         wts = program.buffer("moe.weights", T * top * 4)
         offsets = program.buffer("moe.offsets", (total + 1) * 4)
@@ -190,16 +192,30 @@ class RoutedExperts(FeedForward):
         parts = program.buffer("moe.parts", (top + bool(self.gated and self.shared_ff)) * T * H * 4)
         b = self.b_router
         b_code = K.DTYPE_CODE[b.dtype] if b is not None else 0
-        if self.router == "softmax_top":
-            program.op("core", "ia_router_softmax_topk", [z.tensor(), b, b_code, ids, wts, N, total, top,
-                                                          int(self.w_router.shape[0]), self.groups, self.keep_groups,
-                                                          int(self.renorm), int(self.sigmoid_scores), STREAM])
-        else:
-            program.op("core", "ia_router_topk", [z.tensor(), b, b_code, ids, wts, N, total, top, STREAM])
-        program.op("core", "ia_moe_sort", [ids, offsets, perm, N * top, total, STREAM])
+        first_softmax, rows = self.router == "softmax_top", int(self.w_router.shape[0])
+        few = Guard.between(N, 1, K.ROUTE_MOST_TOKENS) if route else NEVER
+        gate = program.buffer("moe.gate", T * 4) if self.shared_gate else None
+        gates = []                                        # where the shared expert's gates lie, and how far apart
+        for alt in z.alts:
+            program.op("core", "ia_moe_route",
+                       [alt.where, alt.splits or 1, rows, b, b_code, ids, wts, offsets, perm, gate, N, total, top,
+                        int(first_softmax), self.groups, self.keep_groups, int(self.renorm), int(self.sigmoid_scores), STREAM],
+                       alt.when & few)
+            many = alt.when & ~few
+            if many.never or alt.splits:                  # parts are left for few tokens only
+                continue
+            if first_softmax:
+                program.op("core", "ia_router_softmax_topk", [alt.where, b, b_code, ids, wts, N, total, top, rows, self.groups,
+                                                              self.keep_groups, int(self.renorm), int(self.sigmoid_scores),
+                                                              STREAM], many)
+            else:
+                program.op("core", "ia_router_topk", [alt.where, b, b_code, ids, wts, N, total, top, STREAM], many)
+            program.op("core", "ia_moe_sort", [ids, offsets, perm, N * top, total, STREAM], many)
+            if self.shared_gate:
+                gates.append((many, alt.where.at(total * 4), rows))
+        gates.append((few, gate, 1) if self.shared_gate else (ALWAYS, None, 1))
         if not self.gated:
             return self._native_plain(program, ids, wts, offsets, perm, y, parts)
-        from ..engine.program import NEVER, Guard
         first = K.moe_grouped_from_tokens(E, top, H, I, self.rt.dtype)
         grouped = Guard.between(N, first) if first > 0 else NEVER
         tiled = ~grouped
@@ -221,11 +237,12 @@ class RoutedExperts(FeedForward):
             program.op("core", "ia_moe_scatter", [xs, perm, out_w, parts, offsets.at(E * 4) if self.identity else None, N, top, H,
                                                   STREAM], grouped)
         if self.identity or self.shared_ff:
-            self._native_extras(program, z.tensor(), ids, wts, parts)
+            self._native_extras(program, gates, ids, wts, parts)
         program.pending = Value(H, [Alt(ALWAYS, parts, top + bool(self.shared_ff), torch.float32)])
 
-    def _native_extras(self, program, z, ids, wts, parts) -> None:
-        """Identity experts' pairs and the shared expert of gated experts."""
+    def _native_extras(self, program, gates, ids, wts, parts) -> None:
+        """Identity experts' pairs and the shared expert of gated experts; ``gates``: (for which steps, the logits of the
+        shared expert's gate, from a token's to the next)."""
         from ..engine.program import ALWAYS, STREAM, Alt
         H, E, top, N, code = self.hidden_size, self.num_experts, self.top, program.N, program.act_code
         alts = [Alt(ALWAYS, None, 0, self.rt.dtype)]
@@ -235,10 +252,10 @@ class RoutedExperts(FeedForward):
             alts = emit_linear(program, act, N, self.w_shared_down, self.rt.dtype, None, True, "moe.shared.out",
                                "moe.shared.down").alts
         for alt in alts:
-            program.op("core", "ia_moe_extras",
-                       [program.x, code, ids, wts, parts, alt.where, K.DTYPE_CODE[torch.float32 if alt.splits else alt.dtype],
-                        alt.splits or 1, N, z.at(self.total * 4) if self.shared_gate else None, int(self.w_router.shape[0]), N,
-                        E, top, H, STREAM], alt.when)
+            for when, gate, stride in gates:
+                program.op("core", "ia_moe_extras",
+                           [program.x, code, ids, wts, parts, alt.where, K.DTYPE_CODE[torch.float32 if alt.splits else alt.dtype],
+                            alt.splits or 1, N, gate, stride, N, E, top, H, STREAM], alt.when & when)
 
     def _native_plain(self, program, ids, wts, offsets, perm, y, parts) -> None:
         """The launches of ``kernels.api.moe_plain_experts`` and of the shared expert."""

@@ -1622,3 +1622,37 @@ def test_routed_experts_tile_by_tile(gated, counts, W, ff):
         mine = torch.nonzero(expert == e).flatten().tolist()
         for n in mine[:1] + mine[len(mine) // 2:len(mine) // 2 + 1] + mine[-1:]:
             assert torch.equal(parts_of([n])[0], got[n]), (e, n)          # alone: tiles of 32 x 32
+
+
+# ---------------------------------------------------------------- the router and the sort of few tokens in one launch
+# one token, a token more than the waves, the most; one expert, 64; parts that are no multiple of the loads asked for together; the
+# column behind the experts' logits; groups; ties, infinities and NaN among the logits
+@pytest.mark.parametrize("N,E,top,splits,kind", [(1, 32, 4, 8, "top"), (17, 8, 2, 1, "top"), (128, 64, 16, 9, "top"), (3, 1, 1, 3, "softmax"),
+                                                 (16, 24, 2, 16, "groups"), (128, 63, 7, 2, "softmax"), (33, 20, 3, 5, "sigmoid"),
+                                                 (64, 64, 8, 7, "groups")])
+def test_route_of_few_tokens_in_one_launch(N, E, top, splits, kind):
+    api = K()
+    row = E + (kind in ("groups", "sigmoid"))
+    parts = torch.randint(-6, 7, (splits, N, row), generator=torch.Generator().manual_seed(7)).float().to(DEV) / 4     # many ties
+    if E >= 8:
+        parts[0, N // 2, 3], parts[0, 0, 5], parts[0, N - 1, 1] = float("inf"), float("nan"), float("-inf")
+    z = parts[0].clone()
+    for p in parts[1:]:
+        z += p
+    bias = _rand(E, seed=8) if kind != "softmax" else None
+    if kind == "top":
+        want = api.router_topk(z, bias, top)
+        got = api.moe_route(api.SplitSum(parts), bias, top, E)
+    else:
+        kw = dict(groups=4, keep=3) if kind == "groups" else dict(renorm=False, sigmoid=kind == "sigmoid")
+        want = api.router_softmax_topk(z, bias, top, experts=E, **kw)
+        got = api.moe_route(api.SplitSum(parts), bias, top, E, True, **kw)
+    ids, weights, offsets, perm, gate = got
+    assert torch.equal(ids, want[0]) and torch.equal(weights.nan_to_num(-1.0), want[1].nan_to_num(-1.0))
+    assert (gate is None) == (row == E) and (gate is None or torch.equal(gate, z[:, E]))
+    counts = torch.bincount(ids.flatten().long(), minlength=E)
+    assert torch.equal(offsets.long(), torch.cat([counts.new_zeros(1), counts.cumsum(0)]))
+    assert torch.equal(perm.long().sort().values, torch.arange(N * top, device=DEV))
+    assert torch.equal(ids.flatten()[perm.long()].long(), torch.repeat_interleave(torch.arange(E, device=DEV), counts))
+    one = api.moe_route(z, bias, top, E, kind != "top", **({} if kind == "top" else kw))
+    assert torch.equal(one[0], ids) and torch.equal(one[2], offsets)
