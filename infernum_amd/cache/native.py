@@ -57,6 +57,7 @@ _SIGNATURES = {
     "ia_program_add_op": (c_int, [c_void_p, c_void_p, c_char_p, POINTER(c_int64), c_int, POINTER(c_int64), c_int, c_int]),
     "ia_program_finish": (c_int, [c_void_p, c_int, c_int]),
     "ia_program_run": (c_int, [c_void_p, POINTER(c_int64), c_int, POINTER(c_void_p), c_int, c_void_p]),
+    "ia_program_run_part": (c_int, [c_void_p, POINTER(c_int64), c_int, POINTER(c_void_p), c_int, c_void_p, c_int, c_int]),
     "ia_cache_token_slots": (c_int, [c_void_p, c_int, c_int64, c_int64, c_int, POINTER(c_int32)]),
     "ia_cache_pack_step": (c_int, [c_void_p, c_int, POINTER(c_int64), POINTER(c_int), POINTER(c_int32), POINTER(c_int),
                                    POINTER(c_int32), c_int, c_int, POINTER(c_int32), c_int]),

@@ -147,15 +147,20 @@ int ia_program_finish(void* h, int n_vars, int n_ptrs) {
   return 0;
 }
 
-// One step: its numbers, its arrays, the stream.  Operations run in the program's order.
-int ia_program_run(void* h, const int64_t* vars, int n_vars, void* const* ptrs, int n_ptrs, void* stream) {
+// One step, or a part of it: its numbers, its arrays, the stream.  Operations `first` to `last` - 1 run in the program's order
+// (last < 0: to the end); an operation that stands in for the one before it cannot be the first.
+int ia_program_run_part(void* h, const int64_t* vars, int n_vars, void* const* ptrs, int n_ptrs, void* stream, int first, int last) {
   Program* p = static_cast<Program*>(h);
   if (p->n_vars < 0) return fail(p, ERR_PROGRAM, "the program is not finished");
   if (n_vars != p->n_vars || n_ptrs != p->n_ptrs || (n_vars && !vars) || (n_ptrs && !ptrs)) return fail(p, ERR_BAD_ARG, "run");
+  const size_t end = last < 0 ? p->ops.size() : (size_t)last;
+  if (first < 0 || end > p->ops.size() || (size_t)first > end ||
+      ((size_t)first < end && (p->ops[(size_t)first].flags & FLAG_IF_UNSUPPORTED)))
+    return fail(p, ERR_BAD_ARG, "run: the part");
   uint64_t slots[MAX_ARGS];
   p->launches = 0;
   bool unsupported = false;          // the operation before this one ran and found its size unsupported
-  for (size_t i = 0; i < p->ops.size(); ++i) {
+  for (size_t i = (size_t)first; i < end; ++i) {
     const Op& op = p->ops[i];
     if (op.flags & FLAG_IF_UNSUPPORTED) {
       if (!unsupported) continue;
@@ -181,13 +186,17 @@ int ia_program_run(void* h, const int64_t* vars, int n_vars, void* const* ptrs, 
     }
     const int rc = op.fn(slots, n);
     ++p->launches;
-    if (rc == ERR_UNSUPPORTED && i + 1 < p->ops.size() && (p->ops[i + 1].flags & FLAG_IF_UNSUPPORTED)) {
+    if (rc == ERR_UNSUPPORTED && i + 1 < end && (p->ops[i + 1].flags & FLAG_IF_UNSUPPORTED)) {
       unsupported = true;
       continue;
     }
     if (rc) return fail(p, rc, "operation #" + std::to_string(i) + " (" + op.name + ")");
   }
   return 0;
+}
+
+int ia_program_run(void* h, const int64_t* vars, int n_vars, void* const* ptrs, int n_ptrs, void* stream) {
+  return ia_program_run_part(h, vars, n_vars, ptrs, n_ptrs, stream, 0, -1);
 }
 
 }  // extern "C"

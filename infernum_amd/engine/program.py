@@ -284,6 +284,8 @@ class StepProgram:
         self._logits: Optional[torch.Tensor] = None
         self._numbers: List[int] = []
         self._python_error: Optional[BaseException] = None
+        self._head_at = -1                                       # the first operation of the head, once it is written
+        self.head_runs_alone = False
         # the step's numbers
         self._vars: List[Var] = []
         self._var_fns: List[Callable[[StepContext], int]] = []
@@ -472,6 +474,7 @@ class StepProgram:
         self.num_ops = len(self._ops)
         self.op_names = [op[1] for op in self._ops]              # the launchers, in the program's order
         self.num_python_ops = sum(1 for op in self._ops if op[1].startswith("python:"))   # parts called back into
+        self.head_runs_alone = self._head_at >= 0 and not any(op[1].startswith("python:") for op in self._ops[self._head_at:])
         self._ops = []
         self._finished = True
         self._var_array = (ctypes.c_int64 * len(self._vars))()
@@ -512,24 +515,39 @@ class StepProgram:
             raise (K.KernelUnsupported if rc == 10002 else ProgramError)(msg)
 
     # ---- one step ------------------------------------------------------------------------------
-    def run(self, ctx: StepContext) -> torch.Tensor:
-        """The launches of the model's forward pass for this step; fp32 logits [R, V] at ctx.logit_rows."""
+    def begin_head(self) -> None:
+        """What is written from here on makes the logits from the normalised rows in ``x``: it can run as a part of its own
+        (:class:`HeadRun`) if none of it is written in Python."""
+        self._not_finished()
+        self._head_at = len(self._ops)
+
+    def _fill(self, ctx: StepContext, va, pa) -> List[int]:
+        numbers = self._numbers = [int(fn(ctx)) for fn in self._var_fns]
+        for i, x in enumerate(numbers):
+            va[i] = x
+        for i, fn in enumerate(self._ptr_fns):
+            t = fn(ctx)
+            pa[i] = t.data_ptr() if t is not None else None
+        return numbers
+
+    def _run_part(self, va, pa, first: int, last: int) -> None:
+        self._check(self._lib.ia_program_run_part(self._h, va, len(self._vars), pa, len(self._ptr_fns), K._stream(), first, last))
+
+    def run(self, ctx: StepContext, but_the_head: bool = False) -> Optional[torch.Tensor]:
+        """The launches of the model's forward pass for this step; fp32 logits [R, V] at ctx.logit_rows.
+        ``but_the_head``: the launches in front of the head's only, no logits."""
         if not self._finished:
             raise ProgramError("the program is not finished")
         if ctx.num_tokens > self.T:
             raise ProgramError(f"a step of {ctx.num_tokens} tokens; the program's intermediates hold {self.T}")
+        if but_the_head and not self.head_runs_alone:
+            raise ProgramError("the head of this program is no part of its own")
         R = int(ctx.logit_rows.numel())
-        self._logits = torch.empty((R, self.logits_cols), dtype=torch.float32, device=self.rt.device)
+        self._logits = None if but_the_head else torch.empty((R, self.logits_cols), dtype=torch.float32, device=self.rt.device)
         self._ctx = ctx
         try:
-            numbers = self._numbers = [int(fn(ctx)) for fn in self._var_fns]
-            va, pa = self._var_array, self._ptr_array
-            for i, x in enumerate(numbers):
-                va[i] = x
-            for i, fn in enumerate(self._ptr_fns):
-                t = fn(ctx)
-                pa[i] = t.data_ptr() if t is not None else None
-            self._check(self._lib.ia_program_run(self._h, va, len(numbers), pa, len(self._ptr_fns), K._stream()))
+            self._fill(ctx, self._var_array, self._ptr_array)
+            self._run_part(self._var_array, self._ptr_array, 0, self._head_at if but_the_head else -1)
             return self._logits
         finally:
             self._ctx = None
@@ -548,6 +566,26 @@ class StepProgram:
 
     def last_launches(self) -> int:
         return int(self._lib.ia_program_last_launches(self._h))
+
+
+class HeadRun:
+    """The head's launches for steps of the shape of ``ctx``, whose other launches a recording repeats: every run leaves its
+    logits in a tensor of its own (what a recording's launches write is written again by its next replay)."""
+
+    def __init__(self, program: StepProgram, ctx: StepContext):
+        if not program.head_runs_alone:
+            raise ProgramError("the head of this program is no part of its own")
+        self.program, self.rows, self._ctx = program, int(ctx.logit_rows.numel()), ctx       # the step's arrays stay where they are
+        self._vars = (ctypes.c_int64 * len(program._vars))()
+        self._ptrs = (ctypes.c_void_p * len(program._ptrs))()
+        program._fill(ctx, self._vars, self._ptrs)
+
+    def __call__(self) -> torch.Tensor:
+        program = self.program
+        logits = torch.empty((self.rows, program.logits_cols), dtype=torch.float32, device=program.rt.device)
+        self._ptrs[program.logits.index] = logits.data_ptr()
+        program._run_part(self._vars, self._ptrs, program._head_at, -1)
+        return logits
 
 
 def build(model, views: Sequence[CacheView], num_groups: int, max_tokens: int) -> Optional[StepProgram]:

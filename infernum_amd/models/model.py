@@ -149,6 +149,7 @@ class DecoderModel:
                 program.x.view(dt, rows.numel(), H).copy_(h.index_select(0, rows.long()))
             program.python(wanted_rows, "wanted rows")
             program.pending = None
+        program.begin_head()
         self.head.native(program, None)
 
     # ---- one step --------------------------------------------------------------

@@ -295,6 +295,29 @@ def test_recorded_decode_steps_equal_eager_ones(models, name, dtype):
            every_place=False)
 
 
+@pytest.mark.parametrize("executor", ["native", "parts"])          # the head behind the recording; within it
+def test_a_recorded_steps_logits_stay(models, executor):
+    """Logits that a caller keeps are those of their own step after further replays, on a stream of the caller's own too; a
+    step without wanted rows between them."""
+    from infernum_amd import CacheConfig, Engine, StepEntry
+    d, cfg, reqs, ref = models[("B", "bfloat16")]
+    cache = CacheConfig(page_size=PAGE["B"], num_pages=128, num_state_slots=8)
+    eager = Engine.from_pretrained(d, dtype="bfloat16", use_graphs=False, cache_config=cache)
+    graphed = Engine.from_pretrained(d, dtype="bfloat16", executor=executor, cache_config=cache)
+    names = sorted(reqs, key=lambda r: -len(reqs[r]))[:2]
+    kept, want = [], []
+    for eng, out in ((eager, want), (graphed, kept)):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for r in names:
+                eng.step([StepEntry(r, reqs[r][:20], [])])
+            for t in range(20, 32):
+                out.append(eng.step([StepEntry(r, reqs[r][t:t + 1], [] if t == 27 else [0]) for r in names]))
+            torch.cuda.synchronize()
+    assert graphed.graph_replays >= 8 and (graphed.program is not None) == (executor == "native")
+    for a, b in zip(want, kept):
+        assert a.shape == b.shape and torch.equal(a, b)
+
+
 def test_time_per_kernel_switch(models):
     """INFERNUM_PROFILE=1 / set_profile: every kernel call is timed on the device and summed by function; an
     engine made meanwhile records no graphs; the logits are those of an engine without it."""
