@@ -130,83 +130,103 @@ __device__ __forceinline__ void store_four(float* __restrict__ C, int m, int n, 
   }
 }
 
-// Few rows (a decode step): bound by reading W once (3 rows x 128,256 x 2,048: 275 us, 3.8 TB/s, against 1,021 with the
-// vector kernel; 4,096 x 14,336 at 1 row 52 against 2,263 us, 4.5 TB/s; 2,048 x 2,048 9 against 298 us).  A workgroup of 8 waves takes RT * 16 rows of W and all of K; a
-// wave takes every eighth stretch of 256 values, whose loads are all in flight at once (16 KB of W a wave and 16 rows),
-// straight into registers: each byte of W is used by one wave.  The stretches' sums meet in LDS, where they are added
-// in the order of k.  A's rows come from the caches (MT * 16 of them, RT * 16 rows of W share a load).
-#define GS_WAVES 8
-#define GS_MOST_ROWS 32             // rows of A that the streaming kernel takes (3,072 x 2,048: 20 us at 32 rows, the tiles 36 at 33)
-#define GS_TWO_GROUPS_FROM 8192     // rows of W from which a workgroup takes 32 of them: one workgroup a compute unit
-#define GS_ENOUGH_TILES 512         // the largest tile that still gives so many workgroups
-
-template <int MT, int RT>
-__global__ __launch_bounds__(GS_WAVES * 64) void gemm_f32_stream_kernel(const float* __restrict__ A,
-                                                                        const float* __restrict__ W,
-                                                                        float* __restrict__ C, int M, int N, int K,
-                                                                        int lda, int ldw, int ldc, bool wide) {
-  constexpr int TILES = MT * RT;
-  constexpr int PIECE = TILES >= 4 ? 4 : TILES == 2 ? 8 : 16;          // chains whose loads are in flight together
-  __shared__ gf32x4 mids[2][GS_WAVES][TILES][64];
+// Few rows (a decode step, a short prompt): bound by reading W once.  A workgroup takes RT * 16 rows of W, MT * 16 rows of A and
+// all of K; a wave takes every WAVES-th stretch of 256 values, straight into registers (each byte of W is used by one wave of a
+// row of workgroups), PIECE chains of 16 at a time in two sets of registers: the next piece is asked for before this one is worked
+// on, and no load has a condition (what lies beyond K is read from the row's end and cleared), so that the wait for one piece
+// leaves the other under way.  The stretches' sums meet in LDS, where they are added in the order of k.
+// Cold weights, us before (all of half a stretch's loads, then its products, eight waves) and now: 128,256 x 2,048 at 1 / 4 / 16
+// rows 250 / 274 / 303 and 173 / 191 / 249 (1.05 GB: 6.1 to 4.2 TB/s); 16,384 x 2,048 37.6 / 39.8 / 41.7 and 26.6 / 28.7 / 34.1; 2,048 x 8,192
+// 28.8 / 31.5 / 44.3 and 24.3 / 27.1 / 38.8; 4,096 x 14,336 at 1 row 50.9 and 44.5; 16,384 x 2,048 at 17 / 32 rows 82.4 / 87.1 and 41.3 / 45.0;
+// 2,048 x 8,192 at 64 / 142 rows 166 / 173 (the tiles below) and 52.6 / 100.
+template <int MT, int RT, int WAVES, int PIECE>
+__global__ __launch_bounds__(WAVES * 64) void gemm_f32_stream_kernel(const float* __restrict__ A,
+                                                                     const float* __restrict__ W,
+                                                                     float* __restrict__ C, int M, int N, int K,
+                                                                     int lda, int ldw, int ldc, bool wide) {
+  constexpr int TILES = MT * RT, OWN = (TILES + WAVES - 1) / WAVES;    // tiles whose stretches a wave adds up
+  static_assert(16 % (2 * PIECE) == 0, "a stretch is a whole number of pairs of pieces");
+  __shared__ gf32x4 mids[2][WAVES][TILES][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, q = lane >> 4;
-  const int n0 = blockIdx.x * (16 * RT);
+  const int n0 = blockIdx.x * (16 * RT), m0 = blockIdx.y * (16 * MT);
   const float* wrow[RT];
   const float* arow[MT];
 #pragma unroll
-  for (int i = 0; i < RT; ++i) wrow[i] = W + (size_t)min(n0 + 16 * i + r, N - 1) * ldw + 4 * q;
+  for (int i = 0; i < RT; ++i) wrow[i] = W + (size_t)min(n0 + 16 * i + r, N - 1) * ldw;
 #pragma unroll
-  for (int i = 0; i < MT; ++i) arow[i] = A + (size_t)min(16 * i + r, M - 1) * lda + 4 * q;
+  for (int i = 0; i < MT; ++i) arow[i] = A + (size_t)min(m0 + 16 * i + r, M - 1) * lda;
   const int stretches = (K + 255) / 256;
-  gf32x4 acc = {0.f, 0.f, 0.f, 0.f};                                   // wave t: tile t
-  float4 w[PIECE][RT], x[PIECE][MT];
-  auto load = [&](int k0) {                                            // PIECE chains from k0 on; past K zeros
+  float4 w0[PIECE][RT], x0[PIECE][MT], w1[PIECE][RT], x1[PIECE][MT];
+  auto load = [&](int k0, float4 (&w)[PIECE][RT], float4 (&x)[PIECE][MT]) {
 #pragma unroll
     for (int c = 0; c < PIECE; ++c) {
-      const bool in = k0 + 16 * c + 4 * q < K;
+      const int k = min(k0 + 16 * c + 4 * q, K - 4);
 #pragma unroll
-      for (int i = 0; i < RT; ++i)
-        w[c][i] = in ? *reinterpret_cast<const float4*>(wrow[i] + k0 + 16 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int i = 0; i < RT; ++i) w[c][i] = *reinterpret_cast<const float4*>(wrow[i] + k);
 #pragma unroll
-      for (int i = 0; i < MT; ++i)
-        x[c][i] = in ? *reinterpret_cast<const float4*>(arow[i] + k0 + 16 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int i = 0; i < MT; ++i) x[c][i] = *reinterpret_cast<const float4*>(arow[i] + k);
     }
   };
+  gf32x4 mid[TILES];
+  auto work = [&](int k0, float4 (&w)[PIECE][RT], float4 (&x)[PIECE][MT]) {
+    if (k0 + 16 * PIECE > K) {                                         // the row's end
+#pragma unroll
+      for (int c = 0; c < PIECE; ++c)
+        if (k0 + 16 * c + 4 * q >= K) {
+#pragma unroll
+          for (int i = 0; i < RT; ++i) w[c][i] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+          for (int i = 0; i < MT; ++i) x[c][i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < PIECE; ++c) {
+#pragma unroll
+      for (int i = 0; i < RT; ++i) w[c][i] = quarters_turned(w[c][i]);
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+        const float4 xt = quarters_turned(x[c][j]);
+#pragma unroll
+        for (int i = 0; i < RT; ++i) mid[i * MT + j] += chain_of_16(w[c][i], xt);
+      }
+    }
+  };
+  gf32x4 acc[OWN];                                                     // wave t: tiles t, t + WAVES, ...
+#pragma unroll
+  for (int o = 0; o < OWN; ++o) acc[o] = gf32x4{0.f, 0.f, 0.f, 0.f};
   int buf = 0;
-  if (wave < stretches) load(wave * 256);
-  for (int s0 = 0; s0 < stretches; s0 += GS_WAVES, buf ^= 1) {
-    const int s = s0 + wave;
+  if (wave < stretches) load(wave * 256, w0, x0);
+  for (int s0 = 0; s0 < stretches; s0 += WAVES, buf ^= 1) {
+    const int s = s0 + wave, k0 = s * 256;
     if (s < stretches) {
-      gf32x4 mid[TILES];
 #pragma unroll
       for (int t = 0; t < TILES; ++t) mid[t] = gf32x4{0.f, 0.f, 0.f, 0.f};
+      const int next = s + WAVES < stretches ? k0 + WAVES * 256 : k0;  // behind the wave's last stretch anything that can be read
 #pragma unroll
-      for (int piece = 0; piece < 16; piece += PIECE) {
-#pragma unroll
-        for (int c = 0; c < PIECE; ++c) {
-#pragma unroll
-          for (int i = 0; i < RT; ++i) w[c][i] = quarters_turned(w[c][i]);
-#pragma unroll
-          for (int j = 0; j < MT; ++j) {
-            const float4 xt = quarters_turned(x[c][j]);
-#pragma unroll
-            for (int i = 0; i < RT; ++i) mid[i * MT + j] += chain_of_16(w[c][i], xt);
-          }
-        }
-        // the next chains: of this stretch, or of the wave's next one
-        if (piece + PIECE < 16) load(s * 256 + (piece + PIECE) * 16);
-        else if (s + GS_WAVES < stretches) load((s + GS_WAVES) * 256);
+      for (int c = 0; c < 16; c += 2 * PIECE) {
+        load(k0 + 16 * (c + PIECE), w1, x1);
+        __builtin_amdgcn_sched_barrier(0);                             // all of them in front of the first wait
+        work(k0 + 16 * c, w0, x0);
+        load(c + 2 * PIECE < 16 ? k0 + 16 * (c + 2 * PIECE) : next, w0, x0);
+        __builtin_amdgcn_sched_barrier(0);
+        work(k0 + 16 * (c + PIECE), w1, x1);
       }
 #pragma unroll
       for (int t = 0; t < TILES; ++t) mids[buf][wave][t][lane] = mid[t];
     }
     __syncthreads();                 // the other buffer is written next, and this one only after the next barrier
-    if (wave < TILES) {
-      const int have = min(GS_WAVES, stretches - s0);
-      for (int i = 0; i < have; ++i) acc += mids[buf][i][wave][lane];
-    }
+    const int have = min(WAVES, stretches - s0);
+#pragma unroll
+    for (int o = 0; o < OWN; ++o)
+      if (wave + o * WAVES < TILES)
+        for (int i = 0; i < have; ++i) acc[o] += mids[buf][i][wave + o * WAVES][lane];
   }
-  if (wave < TILES) store_four(C, 16 * (wave % MT) + r, n0 + 16 * (wave / MT) + 4 * q, M, N, ldc, wide, acc);
+#pragma unroll
+  for (int o = 0; o < OWN; ++o) {
+    const int t = wave + o * WAVES;
+    if (t < TILES) store_four(C, m0 + 16 * (t % MT) + r, n0 + 16 * (t / MT) + 4 * q, M, N, ldc, wide, acc[o]);
+  }
 }
 
 // Many rows: bound by the matrix instructions (157 TFLOP/s): 2,048 rows x 28,672 x 4,096 at 102 TFLOP/s, 4.7 against
@@ -295,15 +315,16 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
       store_four(C, m0 + 16 * (wm + i) + r, n0 + 16 * (wn + j) + 4 * q, M, N, ldc, wide, acc[i][j] + mid[i][j]);
 }
 
-template <int MT>
+template <int MT, int RT, int WAVES, int PIECE>
 static void launch_f32_stream(const float* A, const float* W, float* C, int M, int N, int K, int lda, int ldw, int ldc,
                               bool wide, hipStream_t stream) {
-  if (MT == 1 && N >= GS_TWO_GROUPS_FROM)                              // two of both would not fit the registers
-    gemm_f32_stream_kernel<1, 2><<<(N + 31) / 32, GS_WAVES * 64, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, wide);
-  else
-    gemm_f32_stream_kernel<MT, 1><<<(N + 15) / 16, GS_WAVES * 64, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, wide);
+  gemm_f32_stream_kernel<MT, RT, WAVES, PIECE><<<dim3((N + 16 * RT - 1) / (16 * RT), (M + 16 * MT - 1) / (16 * MT)), WAVES * 64,
+                                                 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, wide);
 }
 
+#define GS_MOST_ROWS 32             // rows of A that the streaming kernel takes whatever the shape
+#define GS_UNITS 256                // compute units
+#define GS_ENOUGH_TILES 512         // the largest tile that still gives so many workgroups
 template <int WM, int WN>
 static long f32_tiles(int M, int N) { return (long)((M + 32 * WM - 1) / (32 * WM)) * ((N + 32 * WN - 1) / (32 * WN)); }
 
@@ -322,9 +343,35 @@ static bool gemm_f32(const float* A, const float* W, float* C, int M, int N, int
   // the vector kernel 4.7 / 7.0 / 10.9, at 20 rows 17 / 17 / 18 and 5.2 / 7.8 / 12.5; 1,000 x 16 / 32 at 20 rows 6.9 and 5.0 / 7.5)
   if (M <= GS_MOST_ROWS && (K <= 16 || (N > 4096 && K <= (M > 16 ? 96 : 48)))) return false;
   const bool wide = ((uintptr_t)C & 15) == 0 && (ldc & 3) == 0;
-  if (M <= 16) launch_f32_stream<1>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
-  else if (M <= GS_MOST_ROWS) launch_f32_stream<2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
-  else if (f32_tiles<4, 4>(M, N) >= GS_ENOUGH_TILES) launch_f32_tile<4, 4>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
+  // Up to 16 rows: 16 rows of W a workgroup, of 16 waves where those are at most one a compute unit and each wave has a stretch
+  // (4,096 x 4,096 at 1 row 15.7 us, with four waves 19.6; 6,144 x 4,096 26.5 and 25.2), of four otherwise; from nine rows on, whose
+  // reads then weigh as much as W's, 64 rows of W share them (16 rows x 128,256 x 2,048 249 us, with 16 rows of W 295; 8,192 x 2,048, which
+  // that leaves 128 workgroups, 28.6 and 20.2).
+  if (M <= 16) {
+    if (N <= 16 * GS_UNITS && K > 1024) launch_f32_stream<1, 1, 16, 2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
+    else if (M > 8 && N >= 64 * GS_UNITS) launch_f32_stream<1, 4, 4, 2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
+    else launch_f32_stream<1, 1, 4, 2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
+    return true;
+  }
+  // Above: the matrix instructions of a compute unit are what its one workgroup of four waves has, so a shape costs its
+  // workgroups in turns of the compute units, and the tiles below, which share both operands but walk K in step with two
+  // barriers every 32 values, as much as some 2.7 turns of theirs at the least.  Per turn, us with K of 8,192: 32 x 16 of the result 50,
+  // 32 x 32 70, 48 x 32 100, tiles of 32 x 32 62 (166 at the least).  Three stretches of K and fewer leave waves without one (4,099 x 516
+  // at 33 rows 15.2 us, the tiles 12.5; 1,000 x 1,000 7.8 and 18.0).
+  auto turns = [&](int rows, int cols) {
+    const long groups = (long)((M + rows - 1) / rows) * ((N + cols - 1) / cols);
+    return (groups + GS_UNITS - 1) / GS_UNITS;
+  };
+  const long c21 = 50 * turns(32, 16), c22 = 70 * turns(32, 32), c32 = 100 * turns(48, 32);
+  const long tiles = 62L * ((M + 31) / 32) * ((N + 31) / 32) / GS_UNITS, least = tiles < 166 ? 166 : tiles;
+  const long best = c21 < c22 ? (c21 < c32 ? c21 : c32) : (c22 < c32 ? c22 : c32);
+  if (M <= GS_MOST_ROWS || (K > 768 && 10 * best < 9 * least)) {
+    if (c21 <= best) launch_f32_stream<2, 1, 4, 2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
+    else if (c22 <= best || M <= GS_MOST_ROWS) launch_f32_stream<2, 2, 4, 2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
+    else launch_f32_stream<3, 2, 4, 1>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
+    return true;
+  }
+  if (f32_tiles<4, 4>(M, N) >= GS_ENOUGH_TILES) launch_f32_tile<4, 4>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
   else if (f32_tiles<2, 2>(M, N) >= GS_ENOUGH_TILES) launch_f32_tile<2, 2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
   else launch_f32_tile<1, 1>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
   return true;
