@@ -1044,6 +1044,30 @@ def test_attention_generic_far_key_and_first_row():
     assert torch.allclose(out[1].reshape(nh, d), case["vd"][1][0, 0].expand(nh, d), atol=1e-6)
 
 
+# rows of keys read 16 bytes at a time, or value by value where they begin elsewhere: the same bits; one piece of 64 channels, two,
+# four and ten, and a channel more than fills them; 64 keys, one more, and fewer than are asked for together
+@pytest.mark.parametrize("d,dv", [(64, 64), (4, 65), (68, 128), (132, 129), (256, 256), (640, 257)])
+def test_attention_generic_by_how_rows_can_be_read(d, dv):
+    nh, nkv, ps, lens = 4, 2, 16, [65, 64, 5]
+    case = _paged_case(nh, nkv, max(d, dv), ps, lens, [3, 2, 5], torch.float32)
+    q = case["q"].view(case["N"], nh, -1)[:, :, :d].reshape(case["N"], nh * d).contiguous()
+    kp, vp = case["kp"][:, :, :, :d].contiguous(), case["vp"][:, :, :dv].contiguous()
+    room = torch.empty(kp.numel() + 1, device=DEV)
+    room[1:] = kp.flatten()
+    outs = []
+    for pages in (kp, room[1:].view(kp.shape)):
+        outs.append(torch.full((case["N"], nh * dv), float("nan"), device=DEV))
+        K().attention_generic(q, pages, vp, outs[-1], case["token_seq"], case["positions"], case["bt"], nh, nkv, d, d ** -0.5, 0)
+    assert torch.equal(outs[0], outs[1])
+    for n in (0, 4, case["N"] - 1):
+        b, pos = int(case["token_seq"][n]), int(case["positions"][n])
+        k, v = (case[x][b].double()[:pos + 1].repeat_interleave(2, dim=1) for x in ("kd", "vd"))
+        w = torch.softmax((k[:, :, :d] * q[n].view(nh, d).double()).sum(-1) * d ** -0.5, dim=0)
+        want = (w[:, :, None] * v[:, :, :dv]).sum(0)
+        # fp32 chains of d products and of 65 keys: 2^-24 a term, values of order one
+        assert float((outs[0][n].view(nh, dv).double() - want).abs().max()) <= (4 * d + 65) * 2.0 ** -24 * 8
+
+
 def test_attention_generic_missing_page_poisons():
     nh, nkv, d, ps = 1, 1, 16, 4
     case = _paged_case(nh, nkv, d, ps, [20], [1], torch.float32)
