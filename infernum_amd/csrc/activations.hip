@@ -12,17 +12,8 @@ __global__ __launch_bounds__(256) void activation_kernel(const T* __restrict__ i
                                                          int kind) {
   const size_t stride = (size_t)gridDim.x * 256;
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) {
-    const float z = to_float(in[i]);
-    float y = z;
-    if (kind == IA_ACT_GELU_TANH) y = 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));   // gelu_tanh_f below, same roundings
-    else if (kind == IA_ACT_GELU_ERF) y = 0.5f * z * (1.0f + erff(z * 0.7071067811865476f));
-    else if (kind == IA_ACT_RELU_SQUARED) { const float r = fmaxf(z, 0.f); y = r * r; }
-    out[i] = from_float<T>(y);
+    out[i] = from_float<T>(ia_activate(to_float(in[i]), kind));
   }
-}
-
-__device__ __forceinline__ float gelu_tanh_f(float z) {
-  return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
 }
 
 // Eight bfloat16 values (16 bytes) a thread and pass.
@@ -35,7 +26,7 @@ __global__ __launch_bounds__(256) void gelu_tanh_bf16x8_kernel(const uint4* __re
     uint32_t o[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const float lo = gelu_tanh_f(__uint_as_float(w[k] << 16)), hi = gelu_tanh_f(__uint_as_float(w[k] & 0xffff0000u));
+      const float lo = ia_activate(__uint_as_float(w[k] << 16), IA_ACT_GELU_TANH), hi = ia_activate(__uint_as_float(w[k] & 0xffff0000u), IA_ACT_GELU_TANH);
       o[k] = (uint32_t)float_to_bf16_bits(lo) | ((uint32_t)float_to_bf16_bits(hi) << 16);
     }
     out[i] = make_uint4(o[0], o[1], o[2], o[3]);

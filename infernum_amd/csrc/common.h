@@ -189,6 +189,14 @@ __device__ __forceinline__ void rope_pair(float a, float b, float cs, float sn, 
   hi = __builtin_fmaf(a, sn, b * cs);
 }
 
+// The activations between two products, by code (0: none): 1 the tanh form of GELU, 2 GELU, 3 the square of relu.
+__device__ __forceinline__ float ia_activate(float z, int kind) {
+  if (kind == 3) { const float r = fmaxf(z, 0.f); return r * r; }
+  if (kind == 2) return 0.5f * z * (1.0f + erff(z * 0.7071067811865476f));
+  if (kind == 1) return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+  return z;
+}
+
 // The first key that a query at position p sees, from the mask's code: 0 all keys from 0; w > 0 a sliding
 // window, the last w keys (p - w + 1 .. p); w < 0 chunks of -w positions counted from the request's start,
 // the keys of the query's own chunk (floor(p / c) c .. p).  Never decreases with p.

@@ -51,6 +51,25 @@ template <typename TO> __device__ __forceinline__ void store_out(TO* p, float v)
 template <> __device__ __forceinline__ void store_out<float>(float* p, float v) { *p = v; }
 template <> __device__ __forceinline__ void store_out<uint16_t>(uint16_t* p, float v) { *p = float_to_bf16_bits(v); }
 
+// What becomes of a product's values on their way to memory in place of a launch of its own behind it, 2 us each in a step:
+// bf16 results get a bias (fp32, by column) and an activation (ia_activate), fp32 results a factor and a softcap c > 0,
+// c tanh(v / c).  Every one of them rounds as the launch that stores in between would.
+struct SkFinish {
+  const float* bias;
+  int act;
+  float scale, cap;
+};
+__device__ __forceinline__ void store_finished(uint16_t* p, float v, int n, const SkFinish& f) {
+  float x = bf16_bits_to_float(float_to_bf16_bits(v));
+  if (f.bias) x = bf16_bits_to_float(float_to_bf16_bits(x + f.bias[n]));
+  *p = float_to_bf16_bits(ia_activate(x, f.act));
+}
+__device__ __forceinline__ void store_finished(float* p, float v, int, const SkFinish& f) {
+  if (f.scale != 1.0f) v *= f.scale;
+  if (f.cap > 0.f) v = f.cap * tanhf(v * (1.0f / f.cap));
+  *p = v;
+}
+
 // part != nullptr: fp32 partial tiles go to part[split, m, n]; else the result goes to C (one split only).
 // GLU (one split only): a workgroup takes 32 columns n of the result; waves 0 and 1 multiply with the rows n
 // of the first half of W, waves 2 and 3 with the rows N/2 + n of the second half; the halves meet in LDS and
@@ -60,11 +79,13 @@ template <> __device__ __forceinline__ void store_out<uint16_t>(uint16_t* p, flo
 // stretch of memory front to back, where the rows of the matrix as the file holds it lie K values apart.
 // PAIRS: the rounds written out in pairs (see the top of the file); else one after the other, with the next chunk's W copied
 // over this one's (rounds_alone says where).  The sums and their order are the same.
-template <int MT, bool GLU, typename TO, int KC, bool TILED, bool PAIRS>
+// FIN: the values are finished on their way to C (SkFinish).
+template <int MT, bool GLU, typename TO, int KC, bool TILED, bool PAIRS, bool FIN>
 __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16_t* __restrict__ X,
                                                                     const uint16_t* __restrict__ W,
                                                                     TO* __restrict__ C, float* __restrict__ part,
-                                                                    int M, int N, int K, int chunks_per_split) {
+                                                                    int M, int N, int K, int chunks_per_split,
+                                                                    SkFinish finish) {
   // chunks_per_split counts chunks of SK_KC; the kernel walks them in pieces of KC (the sums are the same in
   // the same order either way: a piece is a run of the chunk's matrix instructions)
   constexpr int XROW = KC + SK_XPAD;
@@ -253,8 +274,11 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16
     } else {
       TO* o = C + (size_t)m * N + n;
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (n + e < N) store_out<TO>(o + e, acc[mt][e]);
+      for (int e = 0; e < 4; ++e) {
+        if (n + e >= N) continue;
+        if constexpr (FIN) store_finished(o + e, acc[mt][e], n + e, finish);
+        else store_out<TO>(o + e, acc[mt][e]);
+      }
     }
   }
 }
@@ -265,7 +289,7 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16
 // 1.5 of 58 us).
 template <typename TO, int EPI, int PRE>
 __global__ __launch_bounds__(256) void gemm_skinny_join_kernel(const float* __restrict__ part, TO* __restrict__ C,
-                                                               int M, int N, int splits) {
+                                                               int M, int N, int splits, SkFinish finish) {
   const int NO = EPI == SK_EPI_SWIGLU ? N / 2 : N;
   const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (idx >= (size_t)M * NO) return;
@@ -287,7 +311,8 @@ __global__ __launch_bounds__(256) void gemm_skinny_join_kernel(const float* __re
       if (EPI == SK_EPI_SWIGLU) b = s0 + u < splits ? b + pb[u] : b;
     }
   }
-  store_out<TO>(C + idx, EPI == SK_EPI_SWIGLU ? a / (1.0f + expf(-a)) * b : a);
+  if (EPI == SK_EPI_SWIGLU) store_out<TO>(C + idx, a / (1.0f + expf(-a)) * b);
+  else store_finished(C + idx, a, n, finish);
 }
 
 // ---- up to 16 rows, the parts of K in one workgroup ---------------------------------------------------------------
@@ -301,7 +326,7 @@ template <bool GLU, int WAVES, typename TO>            // WAVES: room for so man
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_whole_kernel(const uint16_t* __restrict__ X,
                                                                        const uint16_t* __restrict__ W,
                                                                        TO* __restrict__ C, int M, int N, int K,
-                                                                       int chunks_per_split, int splits) {
+                                                                       int chunks_per_split, int splits, SkFinish finish) {
   constexpr int NLD = SK_KC / 32;
   __shared__ f32x4 parts[WAVES][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -346,7 +371,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_whole_kernel(const uin
       a += parts[v][lane][e];
       if (GLU) b += parts[splits + v][lane][e];
     }
-    if (n + e < NO) store_out<TO>(C + (size_t)r * NO + n + e, GLU ? a / (1.0f + expf(-a)) * b : a);
+    if (n + e >= NO) continue;
+    if (GLU) store_out<TO>(C + (size_t)r * NO + n + e, a / (1.0f + expf(-a)) * b);
+    else store_finished(C + (size_t)r * NO + n + e, a, n + e, finish);
   }
 }
 
@@ -428,18 +455,18 @@ extern "C" int ia_gemm_skinny_set_splits(int N, int K, int splits) {
 // Number of K splits the kernel uses for a weight [N, K] (a function of N and K only).
 extern "C" int ia_gemm_skinny_splits(int N, int K) { return (N > 0 && K > 0) ? skinny_splits(N, K) : 0; }
 
-template <int MT, bool GLU, typename TO, int KC, bool TILED, bool PAIRS = true>
+template <int MT, bool GLU, typename TO, int KC, bool TILED, bool PAIRS, bool FIN>
 static int launch_skinny_one(dim3 grid, const uint16_t* x, const uint16_t* w, TO* c, float* part, int M, int N, int K,
-                             int cps, hipStream_t stream) {
+                             int cps, const SkFinish& finish, hipStream_t stream) {
   constexpr size_t lds = (size_t)2 * MT * 16 * (KC + SK_XPAD) * sizeof(uint16_t);
   static bool allowed = false;      // more than 64 KB of LDS has to be asked for, once per kernel
   if (lds > 65536 && !allowed) {
-    hipError_t e = hipFuncSetAttribute((const void*)gemm_skinny_kernel<MT, GLU, TO, KC, TILED, PAIRS>,
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_skinny_kernel<MT, GLU, TO, KC, TILED, PAIRS, FIN>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return (int)e;
     allowed = true;
   }
-  gemm_skinny_kernel<MT, GLU, TO, KC, TILED, PAIRS><<<grid, SK_WAVES * 64, lds, stream>>>(x, w, c, part, M, N, K, cps);
+  gemm_skinny_kernel<MT, GLU, TO, KC, TILED, PAIRS, FIN><<<grid, SK_WAVES * 64, lds, stream>>>(x, w, c, part, M, N, K, cps, finish);
   IA_LAUNCH_CHECK();
   return IA_OK;
 }
@@ -469,9 +496,9 @@ static bool rounds_alone(int MT, bool tiled, int K, unsigned groups, unsigned sp
   return (MT == 7 && !tiled) || (MT == 8 && tiled);
 }
 
-template <bool GLU, typename TO, bool TILED = false>
+template <bool GLU, typename TO, bool TILED = false, bool FIN = false>
 static int launch_skinny(const uint16_t* x, const uint16_t* w, TO* c, float* part, int M, int N, int K, int splits,
-                         hipStream_t stream) {
+                         hipStream_t stream, const SkFinish& finish = SkFinish{nullptr, 0, 1.0f, 0.0f}) {
   const int nchunks = (K + SK_KC - 1) / SK_KC;
   const int cps = (nchunks + splits - 1) / splits;
   const int NO = GLU ? N / 2 : N;
@@ -492,43 +519,43 @@ static int launch_skinny(const uint16_t* x, const uint16_t* w, TO* c, float* par
   const bool alone = rounds_alone((M + 15) / 16, TILED, K, groups, grid.y, cps);
   switch ((M + 15) / 16) {
     case 1:
-      if (shorter) return launch_skinny_one<1, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
-      return launch_skinny_one<1, GLU, TO, SK_KC, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
+      if (shorter) return launch_skinny_one<1, GLU, TO, SK_KC / 2, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
+      return launch_skinny_one<1, GLU, TO, SK_KC, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
     case 2:
-      if (shorter) return launch_skinny_one<2, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
-      return launch_skinny_one<2, GLU, TO, SK_KC, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
+      if (shorter) return launch_skinny_one<2, GLU, TO, SK_KC / 2, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
+      return launch_skinny_one<2, GLU, TO, SK_KC, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
     case 3:
-      if (alone) return launch_skinny_one<3, GLU, TO, SK_KC, TILED, false>(grid, x, w, c, part, M, N, K, cps, stream);
-      return launch_skinny_one<3, GLU, TO, SK_KC, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
+      if (alone) return launch_skinny_one<3, GLU, TO, SK_KC, TILED, false, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
+      return launch_skinny_one<3, GLU, TO, SK_KC, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
     case 4:
-      if (alone) return launch_skinny_one<4, GLU, TO, SK_KC, TILED, false>(grid, x, w, c, part, M, N, K, cps, stream);
-      return launch_skinny_one<4, GLU, TO, SK_KC, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
+      if (alone) return launch_skinny_one<4, GLU, TO, SK_KC, TILED, false, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
+      return launch_skinny_one<4, GLU, TO, SK_KC, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
     // above 64 rows: pieces of 128, so that the two stages of X of two workgroups fit a compute unit's LDS
     case 5:
-      if (alone) return launch_skinny_one<5, GLU, TO, SK_KC / 2, TILED, false>(grid, x, w, c, part, M, N, K, cps, stream);
-      return launch_skinny_one<5, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
+      if (alone) return launch_skinny_one<5, GLU, TO, SK_KC / 2, TILED, false, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
+      return launch_skinny_one<5, GLU, TO, SK_KC / 2, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
     case 6:
-      if (alone) return launch_skinny_one<6, GLU, TO, SK_KC / 2, TILED, false>(grid, x, w, c, part, M, N, K, cps, stream);
-      return launch_skinny_one<6, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
+      if (alone) return launch_skinny_one<6, GLU, TO, SK_KC / 2, TILED, false, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
+      return launch_skinny_one<6, GLU, TO, SK_KC / 2, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
     case 7:
-      if (alone) return launch_skinny_one<7, GLU, TO, SK_KC / 2, TILED, false>(grid, x, w, c, part, M, N, K, cps, stream);
-      return launch_skinny_one<7, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
+      if (alone) return launch_skinny_one<7, GLU, TO, SK_KC / 2, TILED, false, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
+      return launch_skinny_one<7, GLU, TO, SK_KC / 2, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
     case 8:
-      if (alone) return launch_skinny_one<8, GLU, TO, SK_KC / 2, TILED, false>(grid, x, w, c, part, M, N, K, cps, stream);
-      return launch_skinny_one<8, GLU, TO, SK_KC / 2, TILED>(grid, x, w, c, part, M, N, K, cps, stream);
+      if (alone) return launch_skinny_one<8, GLU, TO, SK_KC / 2, TILED, false, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
+      return launch_skinny_one<8, GLU, TO, SK_KC / 2, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
     default: return IA_ERR_UNSUPPORTED;
   }
 }
 
 template <typename TO>
-static int launch_join(const float* part, TO* c, int M, int N, int splits, int epilogue, hipStream_t stream) {
+static int launch_join(const float* part, TO* c, int M, int N, int splits, int epilogue, const SkFinish& finish, hipStream_t stream) {
   const int NO = epilogue == SK_EPI_SWIGLU ? N / 2 : N;
   const unsigned grid = (unsigned)(((size_t)M * NO + 255) / 256);
 #define SK_JOIN(EPI)                                                                                          \
   do {                                                                                                        \
-    if (splits <= 2) gemm_skinny_join_kernel<TO, EPI, 2><<<grid, 256, 0, stream>>>(part, c, M, N, splits);    \
-    else if (splits <= 4) gemm_skinny_join_kernel<TO, EPI, 4><<<grid, 256, 0, stream>>>(part, c, M, N, splits); \
-    else gemm_skinny_join_kernel<TO, EPI, 8><<<grid, 256, 0, stream>>>(part, c, M, N, splits);                \
+    if (splits <= 2) gemm_skinny_join_kernel<TO, EPI, 2><<<grid, 256, 0, stream>>>(part, c, M, N, splits, finish);    \
+    else if (splits <= 4) gemm_skinny_join_kernel<TO, EPI, 4><<<grid, 256, 0, stream>>>(part, c, M, N, splits, finish); \
+    else gemm_skinny_join_kernel<TO, EPI, 8><<<grid, 256, 0, stream>>>(part, c, M, N, splits, finish);                \
   } while (0)
   if (epilogue == SK_EPI_SWIGLU) SK_JOIN(SK_EPI_SWIGLU);
   else SK_JOIN(SK_EPI_NONE);
@@ -543,7 +570,8 @@ static int launch_join(const float* part, TO* c, int M, int N, int splits, int e
 // as [splits, M, N] for a later kernel to join.
 template <bool TILED>
 static int skinny_product(const void* X, const void* W, void* C, int out_dtype, int M, int N, int K, int epilogue,
-                          float* workspace, size_t workspace_floats, hipStream_t stream) {
+                          float* workspace, size_t workspace_floats, hipStream_t stream,
+                          const SkFinish& finish = SkFinish{nullptr, 0, 1.0f, 0.0f}) {
   if (M <= 0 || M > 128 || N <= 0 || K <= 0 || (K % 8) != 0) return IA_ERR_UNSUPPORTED;
   if (epilogue != SK_EPI_NONE && epilogue != SK_EPI_SWIGLU) return IA_ERR_BAD_ARG;
   if (epilogue == SK_EPI_SWIGLU && (N & 1)) return IA_ERR_BAD_ARG;
@@ -571,9 +599,9 @@ static int skinny_product(const void* X, const void* W, void* C, int out_dtype, 
 #define SK_WHOLE(G, WAVES)                                                                                            \
   do {                                                                                                                \
     if (out_dtype == IA_F32)                                                                                          \
-      gemm_skinny_whole_kernel<G, WAVES, float><<<grid, block, 0, stream>>>(x, w, (float*)C, M, N, K, cps, splits);   \
+      gemm_skinny_whole_kernel<G, WAVES, float><<<grid, block, 0, stream>>>(x, w, (float*)C, M, N, K, cps, splits, finish);   \
     else                                                                                                              \
-      gemm_skinny_whole_kernel<G, WAVES, uint16_t><<<grid, block, 0, stream>>>(x, w, (uint16_t*)C, M, N, K, cps, splits); \
+      gemm_skinny_whole_kernel<G, WAVES, uint16_t><<<grid, block, 0, stream>>>(x, w, (uint16_t*)C, M, N, K, cps, splits, finish); \
   } while (0)
     if (!glu) SK_WHOLE(false, 8);
     else if (splits <= 4) SK_WHOLE(true, 8);
@@ -584,13 +612,35 @@ static int skinny_product(const void* X, const void* W, void* C, int out_dtype, 
   }
   const int rc = launch_skinny<false, float, TILED>(x, w, nullptr, workspace, M, N, K, splits, stream);
   if (rc != IA_OK || C == nullptr) return rc;
-  if (out_dtype == IA_F32) return launch_join<float>(workspace, (float*)C, M, N, splits, epilogue, stream);
-  return launch_join<uint16_t>(workspace, (uint16_t*)C, M, N, splits, epilogue, stream);
+  if (out_dtype == IA_F32) return launch_join<float>(workspace, (float*)C, M, N, splits, epilogue, finish, stream);
+  return launch_join<uint16_t>(workspace, (uint16_t*)C, M, N, splits, epilogue, finish, stream);
 }
 
 extern "C" int ia_gemm_skinny(const void* X, const void* W, void* C, int out_dtype, int M, int N, int K,
                               int epilogue, float* workspace, size_t workspace_floats, hipStream_t stream) {
   return skinny_product<false>(X, W, C, out_dtype, M, N, K, epilogue, workspace, workspace_floats, stream);
+}
+
+// ia_gemm_skinny without an epilogue whose values are finished on their way to C (SkFinish): a bf16 result by bias (nullable)
+// and act, an fp32 one by scale and cap (0: none).  The same bits as the launches behind it (ia_add_bias, ia_activation, ia_scale,
+// ia_softcap); a bf16 product in one part is followed by them.
+extern "C" int ia_add_bias(void* y, int code, const float* bias, int N, int C, hipStream_t stream);
+extern "C" int ia_activation(const void* in, void* out, int dtype, size_t n, int kind, hipStream_t stream);
+extern "C" int ia_gemm_skinny_finished(const void* X, const void* W, void* C, int out_dtype, int M, int N, int K, const float* bias,
+                                       int act, float scale, float cap, float* workspace, size_t workspace_floats,
+                                       hipStream_t stream) {
+  if (C == nullptr || act < 0 || act > 3 || !(cap >= 0.f) || (out_dtype == IA_F32 ? bias != nullptr || act != 0 : scale != 1.0f || cap > 0.f))
+    return IA_ERR_BAD_ARG;
+  const SkFinish finish{bias, act, scale, cap};
+  if (M <= 0 || M > 128 || N <= 0 || K <= 0 || (K % 8) != 0) return IA_ERR_UNSUPPORTED;
+  if (skinny_splits(N, K) > 1)
+    return skinny_product<false>(X, W, C, out_dtype, M, N, K, SK_EPI_NONE, workspace, workspace_floats, stream, finish);
+  if (out_dtype == IA_F32)
+    return launch_skinny<false, float, false, true>((const uint16_t*)X, (const uint16_t*)W, (float*)C, nullptr, M, N, K, 1, stream, finish);
+  int rc = skinny_product<false>(X, W, C, out_dtype, M, N, K, SK_EPI_NONE, workspace, workspace_floats, stream);
+  if (rc == IA_OK && bias) rc = ia_add_bias(C, IA_BF16, bias, M, N, stream);
+  if (rc == IA_OK && act) rc = ia_activation(C, C, IA_BF16, (size_t)M * N, act, stream);
+  return rc;
 }
 
 // ---- the weight laid out for the kernel: every workgroup's 64 rows x 256 values of a chunk consecutive ----------
@@ -723,5 +773,6 @@ extern "C" int ia_gemm_skinny_no_alloc(const void* X, const void* W, void* C, in
 // ---- the launchers of this file as operations of a step's program (see op_call.h) ----
 #include "op_call.h"
 IA_OP(ia_gemm_skinny)
+IA_OP(ia_gemm_skinny_finished)
 IA_OP(ia_gemm_skinny_tiled)
 IA_OP(ia_gemm_skinny_rows)

@@ -678,13 +678,6 @@ extern "C" int ia_moe_scatter(const void* o, const int* perm, const float* weigh
 //                            lowest index among equals) can be chosen;
 //   ia_moe_up                per expert, over its pairs' tokens: y = act(Wu x), Wu [E, ff, W]; act by the codes of
 //                            ia_activation (2: the erf GELU, 3: the square of relu).
-__device__ __forceinline__ float moe_act(float z, int act) {
-  if (act == 3) { const float r = fmaxf(z, 0.f); return r * r; }
-  if (act == 2) return 0.5f * z * (1.0f + erff(z * 0.7071067811865476f));
-  if (act == 1) return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
-  return z;
-}
-
 // PL: experts a lane holds (lane, lane + 64, ...).  zv: this lane's logits; scores: 64 PL floats of LDS, this wave's own (read
 // with groups only); the rest as for choose_then_softmax.
 template <int PL>
@@ -969,7 +962,7 @@ __global__ __launch_bounds__(256) void moe_up_kernel(const T* __restrict__ x, co
     for (int j = 0; j < 4; ++j) {
       const int c = n0 + j0 + j;
       // the product is rounded as a stored tensor would be, then the activation in fp32
-      if (c < ff) y[(size_t)p * ff + c] = from_float<T>(moe_act(to_float(from_float<T>(v[j])), act));
+      if (c < ff) y[(size_t)p * ff + c] = from_float<T>(ia_activate(to_float(from_float<T>(v[j])), act));
     }
   });
 }
@@ -977,7 +970,7 @@ __global__ __launch_bounds__(256) void moe_up_kernel(const T* __restrict__ x, co
 __device__ __forceinline__ void moe_up_store(bf16_t* __restrict__ y, int ff, int p, int c0, const float* v, int act) {
 #pragma unroll
   for (int j = 0; j < 4; ++j)
-    if (c0 + j < ff) y[(size_t)p * ff + c0 + j] = from_float<bf16_t>(moe_act(to_float(from_float<bf16_t>(v[j])), act));
+    if (c0 + j < ff) y[(size_t)p * ff + c0 + j] = from_float<bf16_t>(ia_activate(to_float(from_float<bf16_t>(v[j])), act));
 }
 
 __global__ __launch_bounds__(512) void moe_up_big_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ Wu,

@@ -759,6 +759,28 @@ def gemm_skinny(a: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = 
     return out
 
 
+def gemm_skinny_finished(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                         act: Optional[str] = None, scale: float = 1.0, cap: float = 0.0) -> torch.Tensor:
+    """:func:`gemm_skinny` whose values are finished on their way to ``out``: bf16 ones by ``bias`` (fp32 [N]) and then ``act``
+    (ACTIVATIONS), fp32 ones by a factor and a softcap.  The same bits as :func:`add_bias`, :func:`activation`, :func:`scale_` and
+    :func:`softcap` behind it."""
+    _dev(a, w, out, bias)
+    M, K = a.shape
+    N = w.shape[0]
+    _need(a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and w.dim() == 2 and w.shape[1] == K, "gemm_skinny_finished: shapes")
+    _need(gemm_skinny_supported(M, N, K), f"gemm_skinny_finished: M={M} N={N} K={K} not supported (M <= 128, K % 8 == 0)")
+    _need(out.dtype in DTYPE_CODE and tuple(out.shape) == (M, N) and out.is_contiguous(), f"gemm_skinny_finished: out [{M}, {N}]")
+    _need(act is None or act in ACTIVATIONS, f"gemm_skinny_finished: unknown activation {act!r}")
+    if bias is not None:
+        _f32(bias, N, "gemm_skinny_finished bias")
+    splits = gemm_skinny_splits(N, K)
+    ws = torch.empty((splits, M, N), dtype=torch.float32, device=a.device) if splits > 1 else None
+    _ok(_core().ia_gemm_skinny_finished(_p(a), _p(w), _p(out), DTYPE_CODE[out.dtype], M, N, K, _p(bias),
+                                        ACTIVATIONS[act] if act else 0, ctypes.c_float(scale), ctypes.c_float(cap), _p(ws),
+                                        ctypes.c_size_t(ws.numel() if ws is not None else 0), _stream()), "gemm_skinny_finished")
+    return out
+
+
 def gemm_skinny_rows(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, tiled: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out[M, N] = a[M, K] @ w[N, K]^T for any M through :func:`gemm_skinny`'s kernel, 128 rows at a time (an fp32
     result from bf16 operands has no other kernel: the head of a step that wants the logits of many places)."""

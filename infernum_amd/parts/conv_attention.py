@@ -21,7 +21,7 @@ import torch
 from ..kernels import api as K
 from .attention import Attention
 from .base import CacheView, Runtime, StateSpec, StepContext, WeightSpec, register_part
-from .linear import emit_linear, linear, prepare_weights
+from .linear import Finish, emit_linear, linear, prepare_weights
 
 
 class ConvAttention(Attention):
@@ -99,7 +99,7 @@ class ConvAttention(Attention):
                      cache.k_pages, cache.v_pages, values_are_keys=True)
         out = torch.empty((n, nh * d), dtype=self.rt.dtype, device=dev)
         self.attend(q, out, ctx, cache)
-        return K.add_bias(linear(out, self.w_o, kernels=self.rt.kernels), self.b_o)
+        return linear(out, self.w_o, kernels=self.rt.kernels, finish=Finish(bias=self.b_o))
 
     def native(self, program, view: CacheView) -> None:
         if type(self).forward is not ConvAttention.forward:
@@ -134,9 +134,8 @@ class ConvAttention(Attention):
                     float(pos.magnitude), k, v, N, nh, nkv, d, d, int(k.shape[2]), int(k.shape[0]), 1,
                     1.0, None, 0, 0.0, STREAM])
         out = self.emit_attend(program, view, q, nh * d, ALWAYS)
-        o = emit_linear(program, out, N, self.w_o, rt.dtype, None, False, "conv_attention.out", "conv_attention.o")
-        program.op("core", "ia_add_bias", [o.tensor(), act, self.b_o, N, self.hidden_size, STREAM])
-        program.pending = o
+        program.pending = emit_linear(program, out, N, self.w_o, rt.dtype, None, False, "conv_attention.out", "conv_attention.o",
+                                      finish=Finish(bias=self.b_o))
 
 
 register_part("mixer", "conv_attention", ConvAttention)

@@ -15,7 +15,7 @@ import torch
 
 from ..kernels import api as K
 from .base import Embedding, Head, Runtime, StepContext, WeightSpec, register_part
-from .linear import emit_linear, linear
+from .linear import Finish, emit_linear, linear
 
 
 EMBEDDING_OUTPUT = "embedding.out"
@@ -118,22 +118,16 @@ class LinearHead(Head):
         self.weight = tensors[self.name]
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        logits = linear(x, self.weight, out_dtype=torch.float32, kernels=self.rt.kernels)
-        if self.scale != 1.0 and logits.shape[0]:
-            logits = K.scale_(logits if logits.is_contiguous() else logits.contiguous(), self.scale)
-        if self.softcap and logits.shape[0]:
-            logits = K.softcap(logits if logits.is_contiguous() else logits.contiguous(), self.softcap)
-        return logits
+        return linear(x, self.weight, out_dtype=torch.float32, kernels=self.rt.kernels, finish=self._finish())
+
+    def _finish(self) -> Finish:
+        return Finish(scale=self.scale, cap=self.softcap)
 
     def native(self, program, view=None) -> None:
         if type(self).forward is not LinearHead.forward:
             return super().native(program, view)
-        emit_linear(program, program.x, program.R, self.weight, torch.float32, None, False, program.logits, "head")
-        from ..engine.program import STREAM
-        if self.scale != 1.0:
-            program.op("core", "ia_scale", [program.logits, program.R, self.vocab_size, float(self.scale), STREAM])
-        if self.softcap:
-            program.op("core", "ia_softcap", [program.logits, program.R, self.vocab_size, float(self.softcap), STREAM])
+        emit_linear(program, program.x, program.R, self.weight, torch.float32, None, False, program.logits, "head",
+                    finish=self._finish())
 
 
 register_part("embedding", "token", TokenEmbedding)

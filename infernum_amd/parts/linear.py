@@ -390,10 +390,61 @@ def _run(kind: str, x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, ep
     raise K.KernelError(f"linear: unknown route {kind!r}")
 
 
+@dataclass(frozen=True)
+class Finish:
+    """What becomes of a product's values: the compute type's get ``bias`` (fp32, by column) and ``act`` (K.ACTIVATIONS), an fp32
+    result ``scale`` and a softcap ``cap``.  The weight-streaming kernel does it on the way to memory; behind the
+    other products it is a launch or two of its own, with the same bits."""
+
+    bias: Optional[torch.Tensor] = None
+    act: Optional[str] = None
+    scale: float = 1.0
+    cap: float = 0.0
+
+    def __bool__(self) -> bool:
+        return self.bias is not None or bool(self.act) or self.scale != 1.0 or self.cap > 0.0
+
+    def fused(self, w: torch.Tensor, dtype: torch.dtype, out_dtype: torch.dtype) -> bool:
+        """Whether the weight-streaming kernel takes it with this weight."""
+        fits = out_dtype == torch.float32 and self.bias is None and not self.act or \
+            out_dtype == torch.bfloat16 and self.scale == 1.0 and not self.cap
+        return bool(self) and fits and dtype == torch.bfloat16 and tiled_copy(w, None) is None
+
+    def apply(self, y: torch.Tensor) -> torch.Tensor:
+        if self.bias is not None:
+            K.add_bias(y, self.bias)
+        if self.act:
+            K.activation(y, self.act)
+        if self.scale != 1.0:
+            K.scale_(y, self.scale)
+        if self.cap:
+            K.softcap(y, self.cap)
+        return y
+
+    def emit(self, program, y: Any, M: Any, cols: int, code: int, when: Any) -> None:
+        """The launches of :meth:`apply` on the [M, cols] values at ``y``."""
+        from ..engine.program import STREAM
+        if self.bias is not None:
+            program.keep(self.bias)
+            program.op("core", "ia_add_bias", [y, code, self.bias, M, cols, STREAM], when)
+        if self.act:
+            program.op("core", "ia_activation", [y, y, code, M * cols, K.ACTIVATIONS[self.act], STREAM], when)
+        if self.scale != 1.0:
+            program.op("core", "ia_scale", [y, M, cols, float(self.scale), STREAM], when)
+        if self.cap:
+            program.op("core", "ia_softcap", [y, M, cols, float(self.cap), STREAM], when)
+
+
+NO_FINISH = Finish()
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
            epilogue: Optional[str] = None, keep_split: bool = False,
-           kernels: str = "auto") -> Union[torch.Tensor, SplitSum]:
-    """``kernels="generic"``: the plain product (fp32 multiply-adds in a fixed order) for every size and type."""
+           kernels: str = "auto", finish: Finish = NO_FINISH) -> Union[torch.Tensor, SplitSum]:
+    """``kernels="generic"``: the plain product (fp32 multiply-adds in a fixed order) for every size and type.  ``finish``
+    goes with neither ``epilogue`` nor ``keep_split``."""
+    if finish and (epilogue or keep_split):
+        raise K.KernelError("linear: a product is finished, or activated, or left in parts")
     M, Kdim = x.shape
     N = w.shape[0]
     out_dtype = out_dtype or x.dtype
@@ -402,6 +453,11 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
     if not x.is_contiguous():
         x = x.contiguous()
     route = route_of(plan(N, Kdim, x.dtype, out_dtype, epilogue, keep_split, kernels), M)
+    if finish:
+        if route.kind == "skinny" and finish.fused(w, x.dtype, out_dtype):
+            return K.gemm_skinny_finished(x, w, torch.empty((M, N), dtype=out_dtype, device=x.device), finish.bias, finish.act,
+                                          finish.scale, finish.cap)
+        return finish.apply(_run(route.kind, x, w, out_dtype, None, route.fallback, route.parts)[0])
     y, activated = _run(route.kind, x, w, out_dtype, epilogue, route.fallback, route.parts)
     if epilogue == "swiglu" and not activated:
         return K.swiglu(y, torch.empty((M, N // 2), dtype=y.dtype, device=y.device))
@@ -410,12 +466,14 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
 
 # ------------------------------------------------------------------- the same routes, written into a program
 def emit_linear(program, x: Any, M: Any, w: torch.Tensor, out_dtype: torch.dtype, epilogue: Optional[str],
-                keep_split: bool, out: Any, key: str, when: Any = None):
+                keep_split: bool, out: Any, key: str, when: Any = None, finish: Finish = NO_FINISH):
     """Writes the launches of :func:`linear` for ``x`` (an address: a Buffer, a tensor, a StepPtr) of ``M`` rows
     (a number of the step) into ``program``, one route after the other, each for its rows.  ``out``: a key (the
     result gets a buffer of that name) or a StepPtr (the step's logits); ``key`` names the scratch memory.
     Returns the ``Value`` that stands for the result."""
     from ..engine import program as P
+    if finish and (epilogue or keep_split):
+        raise K.KernelError("linear: a product is finished, or activated, or left in parts")
     rt = program.rt
     when = P.ALWAYS if when is None else when
     N, Kdim = w.shape
@@ -467,6 +525,7 @@ def emit_linear(program, x: Any, M: Any, w: torch.Tensor, out_dtype: torch.dtype
             continue
         if r.kind == "mfma_f32":                # one part: the fp32 matrix itself
             program.op("core", "ia_gemm_mfma_split", [x, w, out, M, N, Kdim, 1, P.STREAM], g)
+            finish.emit(program, out, M, N, code, g)
             alts.append(P.Alt(g, out, 0, out_dtype))
             continue
         if r.kind == "skinny_split":
@@ -475,12 +534,20 @@ def emit_linear(program, x: Any, M: Any, w: torch.Tensor, out_dtype: torch.dtype
             continue
         if r.kind == "skinny":
             ws = program.buffer(key + ".parts", splits * small * N * 4) if splits > 1 else None
-            program.op("core", skinny, [x, wk, out, code, M, N, Kdim, K.EPILOGUE[epilogue], ws,
-                                        M * (splits * N) if splits > 1 else 0, P.STREAM], g)
+            if finish.fused(w, rt.dtype, out_dtype):
+                program.keep(finish.bias)
+                program.op("core", "ia_gemm_skinny_finished",
+                           [x, w, out, code, M, N, Kdim, finish.bias, K.ACTIVATIONS[finish.act] if finish.act else 0,
+                            float(finish.scale), float(finish.cap), ws, M * (splits * N) if splits > 1 else 0, P.STREAM], g)
+            else:
+                program.op("core", skinny, [x, wk, out, code, M, N, Kdim, K.EPILOGUE[epilogue], ws,
+                                            M * (splits * N) if splits > 1 else 0, P.STREAM], g)
+                finish.emit(program, out, M, N, code, g)
         elif r.kind == "skinny_rows":
             ws = program.buffer(key + ".parts", splits * small * N * 4) if splits > 1 else None
             program.op("core", "ia_gemm_skinny_rows", [x, wk, int(tiled is not None), out, code, M, N, Kdim, ws,
                                                         splits * small * N if splits > 1 else 0, P.STREAM], g)
+            finish.emit(program, out, M, N, code, g)
         else:
             # a product that leaves the whole matrix: into scratch first when an activation follows
             y = program.buffer(key + ".product", T * N * out_bytes) if epilogue == "swiglu" else out
@@ -489,6 +556,7 @@ def emit_linear(program, x: Any, M: Any, w: torch.Tensor, out_dtype: torch.dtype
                 _emit_whole(program, r.fallback, x, w, y, M, N, Kdim, in_code, code, g, True)
             if epilogue == "swiglu":
                 program.op("core", "ia_swiglu", [y, out, code, M, N // 2, P.STREAM], g)
+            finish.emit(program, out, M, N, code, g)
         alts.append(P.Alt(g, out, 0, out_dtype))
     return P.Value(n_out, alts)
 

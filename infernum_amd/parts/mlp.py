@@ -14,7 +14,7 @@ import torch
 
 from ..kernels import api as K
 from .base import FeedForward, Runtime, StepContext, WeightSpec, register_part
-from .linear import emit_linear, linear, prepare_weights
+from .linear import Finish, emit_linear, linear, prepare_weights
 
 
 class SwiGLUFeedForward(FeedForward):
@@ -81,17 +81,15 @@ class DenseFeedForward(FeedForward):
         prepare_weights(self.rt, [(self.w_up, None, False), (self.w_down, None, True)])
 
     def forward(self, x: torch.Tensor, ctx: Optional[StepContext] = None):
-        act = K.activation(linear(x, self.w_up, kernels=self.rt.kernels), self.activation)
+        act = linear(x, self.w_up, kernels=self.rt.kernels, finish=Finish(act=self.activation))
         return linear(act, self.w_down, keep_split=True, kernels=self.rt.kernels)
 
     def native(self, program, view=None) -> None:
         if type(self).forward is not DenseFeedForward.forward:
             return super().native(program, view)
-        from ..engine.program import STREAM
         dt = self.rt.dtype
-        up = emit_linear(program, program.x, program.N, self.w_up, dt, None, False, "dense.act", "dense.up").tensor()
-        program.op("core", "ia_activation", [up, up, program.act_code, program.N * self.intermediate_size,
-                                             K.ACTIVATIONS[self.activation], STREAM])
+        up = emit_linear(program, program.x, program.N, self.w_up, dt, None, False, "dense.act", "dense.up",
+                         finish=Finish(act=self.activation)).tensor()
         program.pending = emit_linear(program, up, program.N, self.w_down, dt, None, True, "dense.out", "dense.down")
 
 

@@ -38,7 +38,7 @@ import torch
 
 from ..kernels import api as K
 from .base import FeedForward, Runtime, StepContext, WeightSpec, register_part
-from .linear import emit_linear, linear
+from .linear import Finish, emit_linear, linear
 
 
 class RoutedExperts(FeedForward):
@@ -170,7 +170,7 @@ class RoutedExperts(FeedForward):
             return K.moe_extras(x, ids, weights, parts, self.num_experts, shared, z[:, self.total] if self.shared_gate else None)
         parts = K.moe_plain_experts(x, ids, weights, self.w_gate_up, self.w_down, self.activation)
         if self.shared_ff:
-            u = K.activation(linear(x, self.w_shared_up, kernels=self.rt.kernels), self.activation)
+            u = linear(x, self.w_shared_up, kernels=self.rt.kernels, finish=Finish(act=self.activation))
             K.stream_add(parts[0], linear(u, self.w_shared_down, out_dtype=torch.float32, kernels=self.rt.kernels))
         return K.SplitSum(parts)
 
@@ -280,8 +280,7 @@ class RoutedExperts(FeedForward):
         if self.shared_ff:
             program.keep(self.w_shared_up, self.w_shared_down)
             u = emit(program, program.x, N, self.w_shared_up, self.rt.dtype, None, False, "moe.shared.act",
-                     "moe.shared.up").tensor()
-            program.op("core", "ia_activation", [u, u, code, N * self.shared_ff, act, STREAM])
+                     "moe.shared.up", finish=Finish(act=self.activation)).tensor()
             down = emit(program, u, N, self.w_shared_down, torch.float32, None, True, "moe.shared.out", "moe.shared.down")
             f32 = K.DTYPE_CODE[torch.float32]
             for alt in down.alts:

@@ -452,6 +452,34 @@ def test_gemm_skinny_rounds_one_after_the_other(M, N, K_, tiled):
             assert torch.equal(got[m:m + 1], api.gemm_skinny(a[m:m + 1], w, **kw))
 
 
+# a product finished on its way to memory leaves the bits of the launches behind it: all parts of K in one workgroup, parts joined (two
+# and more loads at once), one part (fp32: finished in the product, pieces of 128 and 256, in pairs and one after the other)
+@pytest.mark.parametrize("M", [1, 16, 33, 64, 128])
+@pytest.mark.parametrize("N,K_", [(2048, 2048), (650, 520), (4100, 264), (9000, 1288), (16390, 264), (32000, 512), (70000, 72)])
+def test_gemm_skinny_finished_leaves_the_bits_of_separate_launches(M, N, K_):
+    api = K()
+    a, w = _rand(M, K_, dtype=torch.bfloat16, seed=41), _rand(N, K_, dtype=torch.bfloat16, scale=0.05, seed=42)
+    bias = _rand(N, seed=43)
+    for kw in (dict(bias=bias), dict(act="gelu_tanh"), dict(act="gelu"), dict(act="relu_squared", bias=bias)):
+        want = api.gemm_skinny(a, w)
+        if "bias" in kw:
+            api.add_bias(want, bias)
+        if "act" in kw:
+            api.activation(want, kw["act"])
+        assert torch.equal(api.gemm_skinny_finished(a, w, torch.empty_like(want), **kw), want), kw
+    for kw in (dict(scale=0.25), dict(cap=2.5), dict(scale=3.0, cap=1.5)):
+        want = api.gemm_skinny(a, w, out_dtype=torch.float32)
+        if "scale" in kw:
+            api.scale_(want, kw["scale"])
+        if "cap" in kw:
+            api.softcap(want, kw["cap"])
+        assert torch.equal(api.gemm_skinny_finished(a, w, torch.empty_like(want), **kw), want), kw
+    with pytest.raises(api.KernelError):
+        api.gemm_skinny_finished(a, w, torch.empty(M, N, device=DEV), bias=bias)
+    with pytest.raises(api.KernelError):
+        api.gemm_skinny_finished(a, w, torch.empty(M, N, dtype=torch.bfloat16, device=DEV), scale=2.0)
+
+
 # both halves whole in a workgroup although the weight is split (glu_whole): the smallest and largest of either range of K, columns
 # that fill no group of 16, a last chunk that is not full; the copy leaves the same bits, and a row those it has alone
 @pytest.mark.parametrize("M", [1, 16, 33, 128])
