@@ -75,7 +75,8 @@ template <typename TD, typename TO>
 __global__ __launch_bounds__(256) void add_rmsnorm_kernel(float* __restrict__ h, const TD* __restrict__ delta,
                                                           int splits, size_t split_stride,
                                                           const void* __restrict__ w, int w_dtype,
-                                                          TO* __restrict__ out, const int* __restrict__ rows, int H,
+                                                          TO* __restrict__ out, const void* __restrict__ w2, int w2_dtype,
+                                                          TO* __restrict__ out2, const int* __restrict__ rows, int H,
                                                           float eps) {
   __shared__ float red[4];
   const int row = blockIdx.x;
@@ -105,6 +106,7 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(float* __restrict__ h,
       s += d;
     }
     o[i] = from_float<TO>(s * inv * load_as_float(w, w_dtype, i));
+    if (out2) out2[(size_t)row * H + i] = from_float<TO>(s * inv * load_as_float(w2, w2_dtype, i));
   }
 }
 
@@ -119,15 +121,104 @@ __device__ __forceinline__ void store4(bf16_t* p, float4 v) {
   *reinterpret_cast<uint2*>(p) = u;
 }
 
-// Vector kernel: H a multiple of 4 and at most NT * 4 * RN_MAXV.  Every thread keeps its part of the row in
-// registers (16-byte loads, all issued before the first use), so the row is read once and no load waits for
-// another.  Sums are taken in the same order whatever the batch: a row's result depends on the row alone.
 #define RN_MAXV 4
 // x^2 + y^2 + z^2 + w^2 with its roundings written out (two products, two fused multiply-adds, one addition), so
-// that every instantiation of the kernel below gives the same bits for the same row.
+// that every instantiation of the kernels below gives the same bits for the same row.
 __device__ __forceinline__ float sum_of_squares4(const float4 v) {
   return __builtin_fmaf(v.x, v.x, v.y * v.y) + __builtin_fmaf(v.z, v.z, v.w * v.w);
 }
+
+// ------------------------------------------------------- embedding + norm
+// The launches of a step's front as one, for few rows: h[n] = table[ids[n]] * scale (+ pos_table[positions[n]]), kept[n] = h[n] in
+// the activations' type (nullable), h[n] += vector (nullable), x[n] = norm(h[n]) * w (without w: h[n] itself), x2[n] the
+// same norm with w2 (nullable).  One workgroup a row, four values a thread, every row that does not wait for another asked
+// for at once; roundings and the order of the sum of squares are those of the single launches.  Each of them is two trips
+// to memory and a launch, about 4 us in a decoded step: embedding, cast and norm of one row of 2,048 took 11.9 us there.
+template <typename TO, int NT>
+__global__ __launch_bounds__(NT) void embed_norm_kernel(const char* __restrict__ table, int table_dtype, const int* __restrict__ ids,
+                                                        const char* __restrict__ pos_table, int pos_dtype,
+                                                        const int* __restrict__ positions, int pos_rows,
+                                                        const void* __restrict__ vector, int vector_dtype, float* __restrict__ h,
+                                                        TO* __restrict__ kept, const void* __restrict__ w, int w_dtype,
+                                                        TO* __restrict__ x, const void* __restrict__ w2, int w2_dtype,
+                                                        TO* __restrict__ x2, int H, int V, float scale, float eps) {
+#pragma clang fp contract(off)
+  __shared__ float red[NT / 64];
+  const int row = blockIdx.x, i = threadIdx.x * 4, il = min(i, H - 4);
+  const int id = ids[row], at = positions ? positions[row] : 0;
+  const bool known = (unsigned)id < (unsigned)V, placed = (unsigned)at < (unsigned)pos_rows;
+  Raw4 wr, w2r, vr, pr;
+  wr.u = w2r.u = vr.u = pr.u = make_uint4(0u, 0u, 0u, 0u);
+  const size_t width = table_dtype == IA_F32 ? 4 : 2, pwidth = pos_dtype == IA_F32 ? 4 : 2;
+  const Raw4 tr = load_raw4(table + (size_t)(known ? id : 0) * H * width, table_dtype, il);
+  if (pos_table) pr = load_raw4(pos_table + (size_t)(placed ? at : 0) * H * pwidth, pos_dtype, il);
+  if (vector) vr = load_raw4(vector, vector_dtype, il);
+  if (w) wr = load_raw4(w, w_dtype, il);
+  if (w2) w2r = load_raw4(w2, w2_dtype, il);
+  const float nan = __uint_as_float(0x7fc00000u);
+  float4 v = raw4_values(tr, table_dtype);
+  v = known ? make_float4(v.x * scale, v.y * scale, v.z * scale, v.w * scale) : make_float4(nan, nan, nan, nan);
+  if (pos_table) {
+    const float4 p = raw4_values(pr, pos_dtype);
+    v = placed ? make_float4(v.x + p.x, v.y + p.y, v.z + p.z, v.w + p.w) : make_float4(nan, nan, nan, nan);
+  }
+  const size_t o = (size_t)row * H + i;
+  if (kept && i < H) store4(kept + o, v);
+  if (vector) {
+    const float4 p = raw4_values(vr, vector_dtype);
+    v = make_float4(v.x + p.x, v.y + p.y, v.z + p.z, v.w + p.w);
+  }
+  if (i < H) store4(h + o, v);
+  if (!w) {
+    if (i < H) store4(x + o, v);
+    return;
+  }
+  const float ss = block_sum<NT>(i < H ? sum_of_squares4(v) : 0.f, red);
+  const float inv = 1.0f / sqrtf(ss / (float)H + eps);
+  if (i >= H) return;
+  const float4 g = raw4_values(wr, w_dtype);
+  store4(x + o, make_float4(v.x * inv * g.x, v.y * inv * g.y, v.z * inv * g.z, v.w * inv * g.w));
+  if (x2) {
+    const float4 k = raw4_values(w2r, w2_dtype);
+    store4(x2 + o, make_float4(v.x * inv * k.x, v.y * inv * k.y, v.z * inv * k.z, v.w * inv * k.w));
+  }
+}
+
+// table [V, H] and pos_table (nullable, with positions) [pos_rows, H] and vector (nullable) [H] in either type; w (nullable) without w2.
+// H a multiple of 4, at most 1,024 or 2,048 to 4,096 (the norm's launch sums other rows in other orders); every pointer on 16 bytes.
+extern "C" int ia_embed_norm(const void* table, int table_dtype, const int* ids, const void* pos_table, int pos_dtype,
+                             const int* positions, int pos_rows, const void* vector, int vector_dtype, float* h, void* kept,
+                             const void* w, int w_dtype, void* x, const void* w2, int w2_dtype, void* x2, int act_dtype, int N,
+                             int H, int V, float scale, float eps, hipStream_t stream) {
+  auto known = [](int t) { return t == IA_F32 || t == IA_BF16; };
+  const uintptr_t all = reinterpret_cast<uintptr_t>(table) | reinterpret_cast<uintptr_t>(pos_table) | reinterpret_cast<uintptr_t>(vector) |
+                        reinterpret_cast<uintptr_t>(h) | reinterpret_cast<uintptr_t>(kept) | reinterpret_cast<uintptr_t>(w) |
+                        reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w2) | reinterpret_cast<uintptr_t>(x2);
+  if (N < 0 || V <= 0 || !(scale == scale) || !(eps > 0.f) || !table || !ids || !h || !x || H <= 0 || (H & 7) || (all & 15) ||
+      !(H <= 1024 || (H >= 2048 && H <= 4096)) || (!pos_table) != (!positions) || (pos_table && pos_rows <= 0) || (!w2) != (!x2) ||
+      (w2 && !w) || !known(table_dtype) || (pos_table && !known(pos_dtype)) || (vector && !known(vector_dtype)) ||
+      (w && !known(w_dtype)) || (w2 && !known(w2_dtype)) || !known(act_dtype))
+    return IA_ERR_BAD_ARG;
+  if (N == 0) return IA_OK;
+#define IA_EMBED_NORM(TO, NT)                                                                                                       \
+  embed_norm_kernel<TO, NT><<<N, NT, 0, stream>>>((const char*)table, table_dtype, ids, (const char*)pos_table, pos_dtype, positions, \
+                                                  pos_rows, vector, vector_dtype, h, (TO*)kept, w, w_dtype, (TO*)x, w2, w2_dtype,   \
+                                                  (TO*)x2, H, V, scale, eps)
+  if (act_dtype == IA_F32) {
+    if (H <= 1024) IA_EMBED_NORM(float, 256);
+    else IA_EMBED_NORM(float, 1024);
+  } else {
+    if (H <= 1024) IA_EMBED_NORM(bf16_t, 256);
+    else IA_EMBED_NORM(bf16_t, 1024);
+  }
+#undef IA_EMBED_NORM
+  IA_LAUNCH_CHECK();
+  return IA_OK;
+}
+
+// Vector kernel: H a multiple of 4 and at most NT * 4 * RN_MAXV.  Every thread keeps its part of the row in
+// registers (16-byte loads, all issued before the first use), so the row is read once and no load waits for
+// another.  Sums are taken in the same order whatever the batch: a row's result depends on the row alone.
 // AS_WIDE (NT = 256, H <= 4096): the sum of squares is taken in the very order of the kernel of 1024 threads
 // (piece c of this thread is the piece of thread threadIdx.x + 256 c there: 16 sums over 64 lanes, added in the
 // order of their index), so that a row's result has the same bits from either; with many rows 256 threads
@@ -136,8 +227,9 @@ template <typename TD, typename TO, int NT, bool AS_WIDE = false, int MAXV = RN_
 __global__ __launch_bounds__(NT) void add_rmsnorm_vec_kernel(float* __restrict__ h, const TD* __restrict__ delta,
                                                              int splits, size_t split_stride,
                                                              const void* __restrict__ w, int w_dtype,
-                                                             TO* __restrict__ out, const int* __restrict__ rows,
-                                                             int H, float eps) {
+                                                             TO* __restrict__ out, const void* __restrict__ w2,
+                                                             int w2_dtype, TO* __restrict__ out2,
+                                                             const int* __restrict__ rows, int H, float eps) {
   __shared__ float red[NT / 64];
   const int row = blockIdx.x;
   const int src = rows ? rows[row] : row;
@@ -145,6 +237,8 @@ __global__ __launch_bounds__(NT) void add_rmsnorm_vec_kernel(float* __restrict__
   const TD* dr = delta ? delta + (size_t)src * H : nullptr;
   const bool store = (rows == nullptr) && (delta != nullptr);
   float4 v[MAXV], g[MAXV];     // the norm's weights are asked for with the row, not after the sum of squares
+  Raw4 g2raw;                  // (one piece a thread: the second norm's weights too)
+  g2raw.u = make_uint4(0u, 0u, 0u, 0u);
   static_assert(!TOGETHER || MAXV == 1, "registers for all parts' loads of one piece");
   if (TOGETHER) {              // a wave of the row's end reads its last piece where it has none
     const int il = min((int)threadIdx.x * 4, H - 4);
@@ -152,6 +246,7 @@ __global__ __launch_bounds__(NT) void add_rmsnorm_vec_kernel(float* __restrict__
     if (((int)__builtin_amdgcn_readfirstlane(threadIdx.x) & ~63) * 4 < H) {
       v[0] = load4(hr + il);
       const Raw4 graw = load_raw4(w, w_dtype, il);
+      if (w2) g2raw = load_raw4(w2, w2_dtype, il);
       if (dr) {
         const float4 d = load_parts4(dr + il, splits, split_stride);
         v[0].x += d.x; v[0].y += d.y; v[0].z += d.z; v[0].w += d.w;
@@ -227,61 +322,63 @@ __global__ __launch_bounds__(NT) void add_rmsnorm_vec_kernel(float* __restrict__
     if (i < H)
       store4(o + i, make_float4(v[c].x * inv * g[c].x, v[c].y * inv * g[c].y, v[c].z * inv * g[c].z,
                                 v[c].w * inv * g[c].w));
+    if (i < H && out2) {
+      const float4 k = TOGETHER ? raw4_values(g2raw, w2_dtype) : load4_any(w2, w2_dtype, i);
+      store4(out2 + (size_t)row * H + i, make_float4(v[c].x * inv * k.x, v[c].y * inv * k.y, v[c].z * inv * k.z,
+                                                     v[c].w * inv * k.w));
+    }
   }
 }
 
 template <typename TD, typename TO>
 static int launch_add_rmsnorm(float* h, const void* delta, int splits, size_t split_stride, const void* w, int w_dtype,
-                              void* out, const int* rows, int N, int H, float eps, hipStream_t stream) {
+                              void* out, const void* w2, int w2_dtype, void* out2, const int* rows, int N, int H,
+                              float eps, hipStream_t stream) {
   const TD* d = (const TD*)delta;
-  TO* o = (TO*)out;
+  TO *o = (TO*)out, *o2 = (TO*)out2;
   if ((H & 3) == 0 && H <= 1024 * 4 * RN_MAXV) {
     // wide rows: 1024 threads, one to four 16-byte pieces each; with many rows of up to 4096 values, 256 threads
     // that take the sums in the same order.  A row's sums are taken in the same order whatever the batch holds.
     if (H >= 2048 && H <= 4096 && N >= 1024)   // measured: from about 1,000 rows on the narrow workgroups win
-      add_rmsnorm_vec_kernel<TD, TO, 256, true><<<N, 256, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o,
-                                                                        rows, H, eps);
+      add_rmsnorm_vec_kernel<TD, TO, 256, true><<<N, 256, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows, H, eps);
     else if (H >= 2048 && H <= 4096 && rows_are_few(N, 1024))
       // one piece a thread: few registers, so the loads of up to sixteen partial sums are in flight together
       // (the sums are the same: the pieces beyond the first are empty at this width)
-      add_rmsnorm_vec_kernel<TD, TO, 1024, false, 1, true><<<N, 1024, 0, stream>>>(h, d, splits, split_stride, w, w_dtype,
-                                                                                    o, rows, H, eps);
+      add_rmsnorm_vec_kernel<TD, TO, 1024, false, 1, true><<<N, 1024, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows, H, eps);
     else if (H >= 2048 && H <= 4096)
-      add_rmsnorm_vec_kernel<TD, TO, 1024, false, 1><<<N, 1024, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o,
-                                                                              rows, H, eps);
+      add_rmsnorm_vec_kernel<TD, TO, 1024, false, 1><<<N, 1024, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows, H, eps);
     else if (H >= 2048)
-      add_rmsnorm_vec_kernel<TD, TO, 1024><<<N, 1024, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, rows,
+      add_rmsnorm_vec_kernel<TD, TO, 1024><<<N, 1024, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows,
                                                                     H, eps);
     else if (H <= 1024)        // one piece a thread, and few threads a row: together whatever the rows (0.6 to 0.95 of the
                                // time with four pieces at 1 to 4,096 rows of 512 and 1,024)
-      add_rmsnorm_vec_kernel<TD, TO, 256, false, 1, true><<<N, 256, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o,
-                                                                                  rows, H, eps);
+      add_rmsnorm_vec_kernel<TD, TO, 256, false, 1, true><<<N, 256, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows, H, eps);
     else
-      add_rmsnorm_vec_kernel<TD, TO, 256><<<N, 256, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, rows, H,
+      add_rmsnorm_vec_kernel<TD, TO, 256><<<N, 256, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows, H,
                                                                   eps);
   } else {
-    add_rmsnorm_kernel<TD, TO><<<N, 256, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, rows, H, eps);
+    add_rmsnorm_kernel<TD, TO><<<N, 256, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows, H, eps);
   }
   IA_LAUNCH_CHECK();
   return IA_OK;
 }
 
 // delta_dtype: dtype of delta (IA_F32 for a stack of partial sums in the bf16 path); act_dtype: dtype of out.
-// delta is [splits, delta_rows, H].
+// delta is [splits, delta_rows, H].  w2 with out2 (nullable): a second norm of the same rows.
 extern "C" int ia_add_rmsnorm(float* h, const void* delta, int delta_dtype, int splits, int delta_rows,
-                              int act_dtype, const void* w, int w_dtype, void* out, const int* rows, int N, int H,
-                              float eps, hipStream_t stream) {
+                              int act_dtype, const void* w, int w_dtype, void* out, const void* w2, int w2_dtype, void* out2,
+                              const int* rows, int N, int H, float eps, hipStream_t stream) {
   if (N < 0 || H <= 0 || !(eps > 0.f)) return IA_ERR_BAD_ARG;
-  if (delta && (splits < 1 || delta_rows < 0)) return IA_ERR_BAD_ARG;
+  if ((delta && (splits < 1 || delta_rows < 0)) || (!w2) != (!out2)) return IA_ERR_BAD_ARG;
   if (N == 0) return IA_OK;
   const size_t stride = (size_t)delta_rows * H;
   if (!delta) delta_dtype = act_dtype;
   if (act_dtype == IA_F32 && delta_dtype == IA_F32)
-    return launch_add_rmsnorm<float, float>(h, delta, splits, stride, w, w_dtype, out, rows, N, H, eps, stream);
+    return launch_add_rmsnorm<float, float>(h, delta, splits, stride, w, w_dtype, out, w2, w2_dtype, out2, rows, N, H, eps, stream);
   if (act_dtype == IA_BF16 && delta_dtype == IA_BF16)
-    return launch_add_rmsnorm<bf16_t, bf16_t>(h, delta, splits, stride, w, w_dtype, out, rows, N, H, eps, stream);
+    return launch_add_rmsnorm<bf16_t, bf16_t>(h, delta, splits, stride, w, w_dtype, out, w2, w2_dtype, out2, rows, N, H, eps, stream);
   if (act_dtype == IA_BF16 && delta_dtype == IA_F32)
-    return launch_add_rmsnorm<float, bf16_t>(h, delta, splits, stride, w, w_dtype, out, rows, N, H, eps, stream);
+    return launch_add_rmsnorm<float, bf16_t>(h, delta, splits, stride, w, w_dtype, out, w2, w2_dtype, out2, rows, N, H, eps, stream);
   return IA_ERR_BAD_ARG;
 }
 
@@ -718,6 +815,7 @@ extern "C" int ia_words_to_host(void* host_dst, const void* src, int n, hipStrea
 #include "op_call.h"
 IA_OP(ia_embed)
 IA_OP(ia_add_rmsnorm)
+IA_OP(ia_embed_norm)
 IA_OP(ia_residual_add)
 IA_OP(ia_rope_kv_append)
 IA_OP(ia_swiglu)

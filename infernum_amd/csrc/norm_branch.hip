@@ -170,7 +170,8 @@ extern "C" int ia_norm_add(float* h, const void* delta, int delta_dtype, int spl
 // ---- the same with a gate on the branch, and optionally the next sublayer's norm behind the add ----
 //   d = sum_k delta[k][n] * sigmoid(gate[n] + gate_bias)   (fp32; the gate's logits in fp32 or the activations' type)
 //   h[n] += d / sqrt(mean(d^2) + eps) * w
-//   x[n] = h[n] / sqrt(mean(h[n]^2) + eps) * w_next   (with w_next; without it x[n] = h[n]; x may be absent)
+//   x[n] = h[n] / sqrt(mean(h[n]^2) + eps) * w_next   (with w_next; without it x[n] = h[n]; x may be absent;
+//   x_side the same with w_side)
 // One workgroup a row, the row's values in registers (rows above NB_NT * NB_KEEP values are read again).
 template <typename TD, typename TG, typename TX>
 __global__ __launch_bounds__(NB_NT) void gated_norm_add_kernel(float* __restrict__ h, const TD* __restrict__ delta,
@@ -180,7 +181,8 @@ __global__ __launch_bounds__(NB_NT) void gated_norm_add_kernel(float* __restrict
                                                                const float* __restrict__ gate_bias,
                                                                const void* __restrict__ w, int w_dtype,
                                                                const void* __restrict__ w_next, int w_next_dtype,
-                                                               TX* __restrict__ x, int H, float eps) {
+                                                               TX* __restrict__ x, const void* __restrict__ w_side,
+                                                               int w_side_dtype, TX* __restrict__ x_side, int H, float eps) {
   __shared__ float red[NB_NT / 64];
   const int row = blockIdx.x;
   const TD* dr = delta + (size_t)row * H;
@@ -235,10 +237,15 @@ __global__ __launch_bounds__(NB_NT) void gated_norm_add_kernel(float* __restrict
 #pragma unroll
   for (int c = 0; c < NB_KEEP; ++c) {
     const int i = threadIdx.x + c * NB_NT;
-    if (i < H) x[(size_t)row * H + i] = from_float<TX>(w_next ? keep[c] * inv2 * load_as_float(w_next, w_next_dtype, i) : keep[c]);
+    if (i < H) {
+      x[(size_t)row * H + i] = from_float<TX>(w_next ? keep[c] * inv2 * load_as_float(w_next, w_next_dtype, i) : keep[c]);
+      if (x_side) x_side[(size_t)row * H + i] = from_float<TX>(keep[c] * inv2 * load_as_float(w_side, w_side_dtype, i));
+    }
   }
-  for (int i = threadIdx.x + NB_KEEP * NB_NT; i < H; i += NB_NT)
+  for (int i = threadIdx.x + NB_KEEP * NB_NT; i < H; i += NB_NT) {
     x[(size_t)row * H + i] = from_float<TX>(w_next ? hr[i] * inv2 * load_as_float(w_next, w_next_dtype, i) : hr[i]);
+    if (x_side) x_side[(size_t)row * H + i] = from_float<TX>(hr[i] * inv2 * load_as_float(w_side, w_side_dtype, i));
+  }
 }
 
 // The same for rows of a multiple of 4 values up to NT * 4 * NV, with every pointer and stride a multiple of 16 bytes:
@@ -256,22 +263,24 @@ __global__ __launch_bounds__(NT) void gated_norm_add_vec_kernel(float* __restric
                                                                 const float* __restrict__ gate_bias,
                                                                 const void* __restrict__ w, int w_dtype,
                                                                 const void* __restrict__ w_next, int w_next_dtype,
-                                                                TX* __restrict__ x, int H, float eps) {
+                                                                TX* __restrict__ x, const void* __restrict__ w_side,
+                                                                int w_side_dtype, TX* __restrict__ x_side, int H, float eps) {
   __shared__ float red[NT / 64];
   const int row = blockIdx.x;
   const TD* dr = delta + (size_t)row * H;
   float* hr = h + (size_t)row * H;
   float4 d[NV], hv[NV];
-  Raw4 wraw, nraw;
+  Raw4 wraw, nraw, sraw;
   static_assert(!TOGETHER || NV == 1, "registers for all parts' loads of one piece");
   if (TOGETHER) {                                    // everything is asked for before the first use
     const int il = min((int)threadIdx.x * 4, H - 4);
     d[0] = hv[0] = make_float4(0.f, 0.f, 0.f, 0.f);
-    wraw.u = nraw.u = make_uint4(0u, 0u, 0u, 0u);
+    wraw.u = nraw.u = sraw.u = make_uint4(0u, 0u, 0u, 0u);
     if (((int)__builtin_amdgcn_readfirstlane(threadIdx.x) & ~63) * 4 < H) {
       hv[0] = load4(hr + il);
       wraw = load_raw4(w, w_dtype, il);
       if (w_next) nraw = load_raw4(w_next, w_next_dtype, il);
+      if (w_side) sraw = load_raw4(w_side, w_side_dtype, il);
       const float4 b = gate_bias ? load4(gate_bias + il) : make_float4(0.f, 0.f, 0.f, 0.f);
       d[0] = load_parts4(dr + il, splits, split_stride);
       if (gate) {
@@ -361,6 +370,11 @@ __global__ __launch_bounds__(NT) void gated_norm_add_vec_kernel(float* __restric
         o = make_float4(o.x * inv2 * g.x, o.y * inv2 * g.y, o.z * inv2 * g.z, o.w * inv2 * g.w);
       }
       nb_store4(x + (size_t)row * H + i, o);
+      if (x_side) {
+        const float4 g = TOGETHER ? raw4_values(sraw, w_side_dtype) : nb_load4_any(w_side, w_side_dtype, i);
+        nb_store4(x_side + (size_t)row * H + i, make_float4(hv[c].x * inv2 * g.x, hv[c].y * inv2 * g.y,
+                                                            hv[c].z * inv2 * g.z, hv[c].w * inv2 * g.w));
+      }
     }
   }
 }
@@ -368,17 +382,18 @@ __global__ __launch_bounds__(NT) void gated_norm_add_vec_kernel(float* __restric
 template <typename TD, typename TG, typename TX>
 static void launch_gated_norm_add_typed(float* h, const TD* delta, int splits, size_t stride, const TG* gate,
                                         int gate_stride, int gate_splits, size_t gate_split_stride, const float* gate_bias, const void* w, int w_dtype,
-                                        const void* w_next, int w_next_dtype, TX* x, int N, int H, float eps,
-                                        hipStream_t stream) {
+                                        const void* w_next, int w_next_dtype, TX* x, const void* w_side, int w_side_dtype,
+                                        TX* x_side, int N, int H, float eps, hipStream_t stream) {
   const bool aligned = ((reinterpret_cast<uintptr_t>(h) | reinterpret_cast<uintptr_t>(delta) |
                          reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(gate_bias) |
                          reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(w_next) |
-                         reinterpret_cast<uintptr_t>(x)) & 15) == 0 &&
+                         reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w_side) |
+                         reinterpret_cast<uintptr_t>(x_side)) & 15) == 0 &&
                        (stride & 3) == 0 && (gate_stride & 3) == 0 && (gate_split_stride & 3) == 0 && (H & 3) == 0;
 #define IA_GNA_VEC(NT, NV, TOGETHER)                                                                                \
   gated_norm_add_vec_kernel<TD, TG, TX, NT, NV, TOGETHER><<<N, NT, 0, stream>>>(                                             \
       h, delta, splits, stride, gate, gate_stride, gate_splits, gate_split_stride, gate_bias, w, w_dtype, w_next,   \
-      w_next_dtype, x, H, eps)
+      w_next_dtype, x, w_side, w_side_dtype, x_side, H, eps)
   // the threads and pieces follow from H alone: a row's sums are taken in one order
   // (one and two parts are as fast one after the other: 64 rows of 4,096 5.0 / 5.1 us, together 5.1 / 5.3)
   const bool many_parts = splits > 2 || gate_splits > 2;
@@ -390,20 +405,20 @@ static void launch_gated_norm_add_typed(float* h, const TD* delta, int splits, s
   else
     gated_norm_add_kernel<TD, TG, TX><<<N, NB_NT, 0, stream>>>(h, delta, splits, stride, gate, gate_stride, gate_splits,
                                                                gate_split_stride, gate_bias, w, w_dtype, w_next,
-                                                               w_next_dtype, x, H, eps);
+                                                               w_next_dtype, x, w_side, w_side_dtype, x_side, H, eps);
 #undef IA_GNA_VEC
 }
 
 template <typename TD, typename TX>
 static int launch_gated_norm_add(float* h, const void* delta, int splits, size_t stride, const void* gate, int gate_dtype,
                                  int gate_stride, int gate_splits, size_t gate_split_stride, const float* gate_bias, const void* w, int w_dtype, const void* w_next,
-                                 int w_next_dtype, void* x, int N, int H, float eps, hipStream_t stream) {
+                                 int w_next_dtype, void* x, const void* w_side, int w_side_dtype, void* x_side, int N, int H, float eps, hipStream_t stream) {
   if (gate_dtype == IA_F32)
     launch_gated_norm_add_typed<TD, float, TX>(h, (const TD*)delta, splits, stride, (const float*)gate, gate_stride,
-                                               gate_splits, gate_split_stride, gate_bias, w, w_dtype, w_next, w_next_dtype, (TX*)x, N, H, eps, stream);
+                                               gate_splits, gate_split_stride, gate_bias, w, w_dtype, w_next, w_next_dtype, (TX*)x, w_side, w_side_dtype, (TX*)x_side, N, H, eps, stream);
   else if (gate_dtype == IA_BF16)
     launch_gated_norm_add_typed<TD, bf16_t, TX>(h, (const TD*)delta, splits, stride, (const bf16_t*)gate, gate_stride,
-                                                gate_splits, gate_split_stride, gate_bias, w, w_dtype, w_next, w_next_dtype, (TX*)x, N, H, eps, stream);
+                                                gate_splits, gate_split_stride, gate_bias, w, w_dtype, w_next, w_next_dtype, (TX*)x, w_side, w_side_dtype, (TX*)x_side, N, H, eps, stream);
   else
     return IA_ERR_BAD_ARG;
   return IA_OK;
@@ -412,12 +427,14 @@ static int launch_gated_norm_add(float* h, const void* delta, int splits, size_t
 // delta [splits, delta_rows, H] of delta_dtype; gate (nullable) [gate_splits, gate_rows, >= H] rows of gate_stride
 // values of gate_dtype (parts of the logits, added in the order of their index; more than one part: fp32);
 // gate_bias (nullable) fp32 [H]; w_next (nullable): the weight of the norm that follows the add; x (nullable) of act_dtype.
+// w_side with x_side (nullable, next to w_next): another norm of the same row, for a sublayer beside the next one.
 extern "C" int ia_gated_norm_add(float* h, const void* delta, int delta_dtype, int splits, int delta_rows, const void* gate,
                                  int gate_dtype, int gate_stride, int gate_splits, int gate_rows, const float* gate_bias, const void* w, int w_dtype,
-                                 const void* w_next, int w_next_dtype, void* x, int act_dtype, int N, int H, float eps,
-                                 hipStream_t stream) {
+                                 const void* w_next, int w_next_dtype, void* x, const void* w_side, int w_side_dtype, void* x_side,
+                                 int act_dtype, int N, int H, float eps, hipStream_t stream) {
   if (N < 0 || H <= 0 || !(eps > 0.f) || !delta || !h || !w || splits < 1 || delta_rows < N ||
-      (gate && (gate_stride < H || gate_splits < 1 || gate_rows < N || (gate_splits > 1 && gate_dtype != IA_F32))))
+      (gate && (gate_stride < H || gate_splits < 1 || gate_rows < N || (gate_splits > 1 && gate_dtype != IA_F32))) ||
+      (!x_side) != (!w_side) || (x_side && (!x || !w_next)))
     return IA_ERR_BAD_ARG;
   if (N == 0) return IA_OK;
   const size_t stride = (size_t)delta_rows * H;
@@ -426,13 +443,13 @@ extern "C" int ia_gated_norm_add(float* h, const void* delta, int delta_dtype, i
   int rc;
   if (delta_dtype == IA_F32 && act_dtype == IA_F32)
     rc = launch_gated_norm_add<float, float>(h, delta, splits, stride, gate, gate_dtype, gate_stride, gate_splits, gstride, gate_bias, w, w_dtype,
-                                             w_next, w_next_dtype, x, N, H, eps, stream);
+                                             w_next, w_next_dtype, x, w_side, w_side_dtype, x_side, N, H, eps, stream);
   else if (delta_dtype == IA_BF16 && act_dtype == IA_BF16)
     rc = launch_gated_norm_add<bf16_t, bf16_t>(h, delta, splits, stride, gate, gate_dtype, gate_stride, gate_splits, gstride, gate_bias, w,
-                                               w_dtype, w_next, w_next_dtype, x, N, H, eps, stream);
+                                               w_dtype, w_next, w_next_dtype, x, w_side, w_side_dtype, x_side, N, H, eps, stream);
   else if (delta_dtype == IA_F32 && act_dtype == IA_BF16)
     rc = launch_gated_norm_add<float, bf16_t>(h, delta, splits, stride, gate, gate_dtype, gate_stride, gate_splits, gstride, gate_bias, w,
-                                              w_dtype, w_next, w_next_dtype, x, N, H, eps, stream);
+                                              w_dtype, w_next, w_next_dtype, x, w_side, w_side_dtype, x_side, N, H, eps, stream);
   else
     return IA_ERR_BAD_ARG;
   if (rc != IA_OK) return rc;

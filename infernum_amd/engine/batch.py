@@ -53,6 +53,13 @@ class PackedStep:
     tile_rows: int = 0                   # height of the row tiles that were packed (0: none)
     order: Sequence[int] = ()            # row r of the batch is entry order[r] of the step
 
+    @property
+    def rows_are_tokens(self) -> bool:
+        """The wanted rows are all rows, in their order (as in a step in which every request brings one token)."""
+        n = self.num_logit_rows
+        first = self.offsets[6]
+        return n == self.sizes[0] and self.host[first:first + n].tolist() == list(range(n))
+
     def context(self, dev: torch.Tensor) -> StepContext:
         """The step as the parts see it, over ``dev``, the device copy of ``host``."""
         def seg(i: int) -> torch.Tensor:
@@ -66,6 +73,7 @@ class PackedStep:
             slots=[seg(8 + 2 * g) for g in range(n_groups)],
             q_lens=self.q_lens, ctx_lens=self.ctx_lens, max_q_len=max(self.q_lens),
             max_total_len=max(c + q for c, q in zip(self.ctx_lens, self.q_lens)),
+            rows_are_tokens=self.rows_are_tokens,
             packed_row_tiles={self.tile_rows: (seg(7).view(-1, 2), self.num_tiles)} if self.tile_rows else {},
         )
 

@@ -238,7 +238,7 @@ class Engine:
         packed = pack_step(cache, entries, bt_width=POW2_WIDTH, tile_rows=self._tile_rows)
         widths = tuple(shape[1] for shape in packed.bt_shapes)           # one width per group of the cache
         limit = max(widths, default=0) * cache.page_size
-        key = (len(entries), widths, packed.num_logit_rows)
+        key = (len(entries), widths, packed.num_logit_rows, packed.rows_are_tokens)
         g = self._graphs.get(key)
         if g is not None:
             self._graphs[key] = self._graphs.pop(key)       # most recently used last

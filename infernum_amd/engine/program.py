@@ -261,6 +261,15 @@ class Value:
         return self.alts[0].where
 
 
+class _Writer:
+    """The operations that completed the stream, as the last ones written (``StepProgram.stream_written``)."""
+
+    __slots__ = ("first", "end", "write", "when", "eps", "add_vector")
+
+    def __init__(self, first: int, end: int, write, when: Guard, eps, add_vector):
+        self.first, self.end, self.write, self.when, self.eps, self.add_vector = first, end, write, when, eps, add_vector
+
+
 _CALLBACK = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.POINTER(ctypes.c_uint64), ctypes.c_int)
 
 
@@ -297,6 +306,7 @@ class StepProgram:
         self.MAX_LEN = self._var("longest request", lambda c: c.max_total_len)
         self.NP = self._var("requests with a portion", lambda c: c.num_seqs - c.num_decode)
         self.NPT = self._var("tokens of portions", lambda c: c.num_tokens - c.num_decode)
+        self.ALL_ROWS = self._var("the wanted rows are the tokens", lambda c: int(c.rows_are_tokens))
         self._bt_cols = [self._var(f"block-table width {g}", (lambda c, g=g: int(c.block_tables[g].shape[1])))
                          for g in range(num_groups)]
         # the step's arrays
@@ -318,6 +328,7 @@ class StepProgram:
         self.h = self.buffer("h", self.T * self.hidden_size * 4)
         self.x = self.buffer("x", self.T * self.hidden_size * self.act_bytes)
         self.pending: Optional[Value] = None
+        self._writer: Optional["_Writer"] = None                 # see stream_written
 
     def __del__(self):
         if getattr(self, "_h", None):
@@ -421,6 +432,51 @@ class StepProgram:
         cb = _CALLBACK(call)
         self._keep.append(cb)
         self._ops.append((ctypes.cast(cb, ctypes.c_void_p), "python:" + name, [], when, False))
+
+    # ---- a norm on the launch that completes the stream ---------------------------------------
+    def stream_written(self, first: int, write: Callable[..., None], when: Guard = ALWAYS, eps: Optional[float] = None,
+                       add_vector: Optional[Callable[[torch.Tensor], None]] = None) -> None:
+        """The operations from number ``first`` on complete the stream in ``h``, and their launcher can go on with the
+        norm of its rows for the steps of ``when`` (with the root's ``eps``, or with any): ``write(when, norm, side)``
+        writes them again, with ``norm`` into ``x`` and ``side`` (None, or another norm and its buffer) or without (None).
+        ``add_vector(v)`` writes them again with v added to all rows; a launcher that has it also takes the norm "cast",
+        the rows themselves rounded into ``x``."""
+        self._writer = _Writer(first, len(self._ops), write, when, eps, add_vector)
+
+    def _last_writer(self) -> Optional["_Writer"]:
+        w, self._writer = self._writer, None
+        return w if w is not None and w.end == len(self._ops) and self.pending is None else None
+
+    def _write_again(self, w: "_Writer", when: Guard, norm: Any, side: Optional[tuple]) -> Guard:
+        del self._ops[w.first:]
+        if not (~when).never:
+            w.write(~when, None, None)
+        w.write(when, norm, side)
+        return when
+
+    def vector_rides(self, vector: torch.Tensor) -> bool:
+        """True when the launch that completed the stream adds ``vector`` to its rows as well."""
+        w = self._last_writer()
+        if w is None or w.add_vector is None:
+            return False
+        del self._ops[w.first:]
+        w.add_vector(vector)
+        return True
+
+    def cast_rides(self) -> Guard:
+        """For which steps the launch that completed the stream leaves its rows in ``x`` as well, rounded."""
+        w = self._last_writer()
+        return NEVER if w is None or w.add_vector is None else self._write_again(w, w.when, "cast", None)
+
+    def norm_rides(self, norm: Any, rows: bool = False, side: Optional[tuple] = None) -> Guard:
+        """For which steps the launches just written, that completed the stream, leave its norm behind as well: no launch
+        for it is needed then.  ``rows``: the norm is wanted of the wanted rows, which have to be all rows in their order.
+        The norms' kernels sum a row's squares in one order up to 1,024 values and from 2,048 on (between, and off
+        multiples of four, in another each), so that the row's bits are those of the norm's own launch."""
+        w, H = self._last_writer(), self.hidden_size
+        if w is None or H % 4 or not (H <= 1024 or 2048 <= H <= 16384) or (w.eps is not None and w.eps != norm.eps):
+            return NEVER
+        return self._write_again(w, w.when & Guard.between(self.ALL_ROWS, 1) if rows else w.when, norm, side)
 
     # ---- values between Python operations and launches ----------------------------------------
     def read(self, value: Optional[Value], rows: int):

@@ -140,6 +140,34 @@ def embed(table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor, scale: floa
     return out
 
 
+def embed_norm(table: torch.Tensor, ids: torch.Tensor, h: torch.Tensor, weight: Optional[torch.Tensor], eps: float,
+               out: torch.Tensor, scale: float = 1.0, position_table: Optional[torch.Tensor] = None,
+               positions: Optional[torch.Tensor] = None, vector: Optional[torch.Tensor] = None,
+               kept: Optional[torch.Tensor] = None, side_weight: Optional[torch.Tensor] = None,
+               out_side: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``embed`` (+ ``add_rows``, a cast into ``kept``, ``add_vector``) into h, and its norm into ``out`` (without ``weight`` h itself,
+    rounded), with ``side_weight`` another into ``out_side``: one launch for few rows of up to 1,024 or 2,048 to 4,096 values."""
+    _dev(table, ids, h, weight, out, position_table, positions, vector, kept, side_weight, out_side)
+    V, H = table.shape
+    N = ids.numel()
+    _need(table.dtype in DTYPE_CODE and h.dtype == torch.float32 and tuple(h.shape) == (N, H), f"embed_norm: h must be fp32 [{N}, {H}]")
+    _i32(ids, N, "embed_norm ids")
+    for t in (out, kept, out_side):
+        _need(t is None or (t.dtype == out.dtype and t.dtype in DTYPE_CODE and tuple(t.shape) == (N, H)), f"embed_norm: outputs [{N}, {H}] of one type")
+    for t in (weight, side_weight, vector):
+        _need(t is None or (t.dtype in DTYPE_CODE and t.numel() == H), f"embed_norm: weights of {H} values")
+    _need((position_table is None) == (positions is None), "embed_norm: a table of positions and the positions")
+    if positions is not None:
+        _i32(positions, N, "embed_norm positions")
+        _need(position_table.dtype in DTYPE_CODE and position_table.dim() == 2 and position_table.shape[1] == H, "embed_norm: a row per position")
+    code = lambda t: DTYPE_CODE[t.dtype] if t is not None else 0         # noqa: E731
+    _ok(_core().ia_embed_norm(_p(table), code(table), _p(ids), _p(position_table), code(position_table), _p(positions),
+                              position_table.shape[0] if positions is not None else 0, _p(vector), code(vector), _p(h), _p(kept),
+                              _p(weight), code(weight), _p(out), _p(side_weight), code(side_weight), _p(out_side), code(out), N, H,
+                              V, ctypes.c_float(scale), ctypes.c_float(eps), _stream()), "embed_norm")
+    return out
+
+
 class SplitSum:
     """A matrix [M, N] given as a stack of fp32 partial sums ``parts`` [S, M, N]: what a matrix product
     whose inner dimension was split over workgroups leaves.  The kernels that take the product next
@@ -162,15 +190,17 @@ class SplitSum:
 
 
 def add_rmsnorm(h: torch.Tensor, delta, weight: torch.Tensor, eps: float,
-                out: torch.Tensor, rows: Optional[torch.Tensor] = None) -> torch.Tensor:
+                out: torch.Tensor, rows: Optional[torch.Tensor] = None, side_weight: Optional[torch.Tensor] = None,
+                out_side: Optional[torch.Tensor] = None) -> torch.Tensor:
     """h += delta (fp32, in place); out = h * rsqrt(mean(h^2) + eps) * weight.
 
     ``delta`` is None, a tensor of h's shape in out's dtype, or a :class:`SplitSum`.
-    With ``rows`` the norm is taken of the selected rows only and h stays as it is.
+    With ``rows`` the norm is taken of the selected rows only and h stays as it is.  ``out_side``, like ``out``: the same
+    norm with ``side_weight``.
     """
     split = isinstance(delta, SplitSum)
     d = delta.parts if split else delta
-    _dev(h, d, weight, out, rows)
+    _dev(h, d, weight, out, rows, side_weight, out_side)
     _need(h.dtype == torch.float32 and h.dim() == 2, "add_rmsnorm: h must be fp32 [N, H]")
     H = h.shape[1]
     n_out = rows.numel() if rows is not None else h.shape[0]
@@ -182,11 +212,15 @@ def add_rmsnorm(h: torch.Tensor, delta, weight: torch.Tensor, eps: float,
     elif d is not None:
         _need(d.dtype == out.dtype and tuple(d.shape) == tuple(h.shape),
               "add_rmsnorm: delta must have h's shape and out's dtype")
-    _need(weight.dtype in DTYPE_CODE and weight.numel() == H, f"add_rmsnorm: weight must hold {H} values")
+    for wt in (weight, side_weight):
+        _need(wt is None or (wt.dtype in DTYPE_CODE and wt.numel() == H), f"add_rmsnorm: weight must hold {H} values")
+    _need((out_side is None) == (side_weight is None) and (out_side is None or (
+        out_side.dtype == out.dtype and out_side.shape == out.shape)), "add_rmsnorm: out_side like out, with a weight of its own")
     if rows is not None:
         _i32(rows, n_out, "add_rmsnorm rows")
     _ok(_core().ia_add_rmsnorm(_p(h), _p(d), d_code, splits, d_rows, DTYPE_CODE[out.dtype], _p(weight),
-                               DTYPE_CODE[weight.dtype], _p(out), _p(rows), n_out, H, ctypes.c_float(eps),
+                               DTYPE_CODE[weight.dtype], _p(out), _p(side_weight),
+                               DTYPE_CODE[side_weight.dtype] if side_weight is not None else 0, _p(out_side), _p(rows), n_out, H, ctypes.c_float(eps),
                                _stream()), "add_rmsnorm")
     return out
 
@@ -1565,14 +1599,15 @@ def add_rows(h: torch.Tensor, table: torch.Tensor, index: torch.Tensor) -> torch
 
 def gated_norm_add(h: torch.Tensor, delta, gate, gate_bias: Optional[torch.Tensor],
                    weight: torch.Tensor, eps: float, next_weight: Optional[torch.Tensor] = None,
-                   x: Optional[torch.Tensor] = None) -> torch.Tensor:
+                   x: Optional[torch.Tensor] = None, side_weight: Optional[torch.Tensor] = None,
+                   x_side: Optional[torch.Tensor] = None) -> torch.Tensor:
     """d = delta * sigmoid(gate + gate_bias);  h += d * rsqrt(mean(d^2) + eps) * weight  (fp32, in place).  ``delta``: a
     tensor of h's shape in the activations' dtype or a :class:`SplitSum`; ``gate``: rows of at least H values (fp32 or
     the activations' dtype), a :class:`SplitSum` of the logits, or None for no gate; ``x`` (optional, h's shape in the activations' dtype) receives
-    rms_norm(h) * next_weight, or the new h itself without ``next_weight``."""
+    rms_norm(h) * next_weight, or the new h itself without ``next_weight``; ``x_side`` (next to ``x`` and ``next_weight``) rms_norm(h) * side_weight."""
     split = isinstance(delta, SplitSum)
     d = delta.parts if split else delta
-    _dev(h, d, weight, x, gate_bias, next_weight)
+    _dev(h, d, weight, x, gate_bias, next_weight, side_weight, x_side)
     _need(h.dtype == torch.float32 and h.dim() == 2, "gated_norm_add: h must be fp32 [N, H]")
     N, H = h.shape
     splits, d_rows = 1, N
@@ -1591,16 +1626,20 @@ def gated_norm_add(h: torch.Tensor, delta, gate, gate_bias: Optional[torch.Tenso
         _need(gate.shape[0] >= N, "gated_norm_add: a gate row per row of h")
         g_rows, g_stride = gate.shape[0], int(gate.stride(0))
     _f32(gate_bias, H, "gated_norm_add gate bias")
-    for wt in (weight, next_weight):
+    for wt in (weight, next_weight, side_weight):
         _need(wt is None or (wt.dtype in DTYPE_CODE and wt.numel() == H), f"gated_norm_add: weights of {H} values")
     act = x.dtype if x is not None else (torch.bfloat16 if d.dtype == torch.bfloat16 else torch.float32)
     if x is not None:
         _need(x.dtype in DTYPE_CODE and tuple(x.shape) == (N, H) and (split or x.dtype == d.dtype),
               "gated_norm_add: x of h's shape in the activations' dtype")
+    _need((x_side is None) == (side_weight is None) and (x_side is None or (
+        x is not None and next_weight is not None and x_side.dtype == x.dtype and tuple(x_side.shape) == (N, H))),
+          "gated_norm_add: x_side like x, beside the next norm's weight, with a weight of its own")
     _ok(_core().ia_gated_norm_add(
         _p(h), _p(d), DTYPE_CODE[d.dtype], splits, d_rows, _p(gate), DTYPE_CODE[gate.dtype] if gate is not None else 0,
         g_stride if gate is not None else 0, g_splits, g_rows, _p(gate_bias), _p(weight), DTYPE_CODE[weight.dtype],
-        _p(next_weight), DTYPE_CODE[next_weight.dtype] if next_weight is not None else 0, _p(x), DTYPE_CODE[act], N, H,
+        _p(next_weight), DTYPE_CODE[next_weight.dtype] if next_weight is not None else 0, _p(x), _p(side_weight),
+        DTYPE_CODE[side_weight.dtype] if side_weight is not None else 0, _p(x_side), DTYPE_CODE[act], N, H,
         ctypes.c_float(eps), _stream()), "gated_norm_add")
     return h
 

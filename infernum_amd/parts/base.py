@@ -227,6 +227,7 @@ class StepContext:
     ctx_lens: Sequence[int] = ()
     max_q_len: int = 0
     max_total_len: int = 0                  # largest ctx + q over the batch
+    rows_are_tokens: bool = False           # logit_rows is 0 .. N-1: every token's logits are wanted, in the rows' order
     # lists of row tiles by tile height, as far as the step's packing made them (see ``row_tiles``)
     packed_row_tiles: Dict[int, Tuple[torch.Tensor, int]] = field(default_factory=dict)
     extras: Dict[str, Any] = field(default_factory=dict)

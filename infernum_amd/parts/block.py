@@ -106,7 +106,7 @@ class BranchNormBlock(Block):
                 raise K.KernelError("branchnorm after an arrangement that leaves its delta unadded is not written "
                                     "as launches")
             program.op("core", "ia_cast", [program.h, K.DTYPE_CODE[torch.float32], program.x, program.act_code,
-                                           program.N * H, STREAM])
+                                           program.N * H, STREAM], ~program.cast_rides())
         self.mixer.native(program, view)
         self.mixer_norm.native_branch(program)
         if self.feed_forward is not None:
@@ -154,7 +154,7 @@ class SandwichBlock(Block):
 
     def _emit_branch(self, program, gate, post, key: str, next_norm=None) -> None:
         """``program.x`` holds what the sublayer read, ``program.pending`` its result."""
-        from ..engine.program import STREAM
+        from ..engine.program import ALWAYS, STREAM
         from ..kernels import api as K
         H = program.hidden_size
         logits = gate.emit_logits(program, key) if gate is not None else None
@@ -162,22 +162,28 @@ class SandwichBlock(Block):
         program.keep(post.weight, next_norm.weight if next_norm is not None else None,
                      gate.bias if gate is not None else None)
         galts = logits.alts if logits is not None else [None]
-        for alt in program.pending.alts:
-            if not alt.splits and alt.dtype != self.rt.dtype:
-                raise K.KernelError("gated_norm_add: the delta must have the activations' dtype")
-            code = f32 if alt.splits else program.act_code
-            for galt in galts:                      # the gate's logits whole or as the parts of a split product
-                if galt is not None and galt.dtype != torch.float32:
-                    raise K.KernelError("gated_norm_add: the gate's logits must be fp32")
-                program.op("core", "ia_gated_norm_add",
-                           [program.h, alt.where, code, alt.splits or 1, program.N,
-                            galt.where if galt is not None else None, f32, H, (galt.splits or 1) if galt is not None else 1,
-                            program.N, gate.bias if gate is not None else None, post.weight,
-                            K.DTYPE_CODE[post.weight.dtype], next_norm.weight if next_norm is not None else None,
-                            K.DTYPE_CODE[next_norm.weight.dtype] if next_norm is not None else 0,
-                            program.x if next_norm is not None else None, program.act_code, program.N, H,
-                            float(post.eps), STREAM], alt.when & galt.when if galt is not None else alt.when)
+        branch, first = program.pending, len(program._ops)
+
+        def write(when, norm, side) -> None:
+            behind = norm.next_operands(program, side) if norm is not None else [None, 0, None, None, 0, None]
+            for alt in branch.alts:
+                if not alt.splits and alt.dtype != self.rt.dtype:
+                    raise K.KernelError("gated_norm_add: the delta must have the activations' dtype")
+                code = f32 if alt.splits else program.act_code
+                for galt in galts:                      # the gate's logits whole or as the parts of a split product
+                    if galt is not None and galt.dtype != torch.float32:
+                        raise K.KernelError("gated_norm_add: the gate's logits must be fp32")
+                    program.op("core", "ia_gated_norm_add",
+                               [program.h, alt.where, code, alt.splits or 1, program.N,
+                                galt.where if galt is not None else None, f32, H, (galt.splits or 1) if galt is not None else 1,
+                                program.N, gate.bias if gate is not None else None, post.weight,
+                                K.DTYPE_CODE[post.weight.dtype]] + behind +
+                               [program.act_code, program.N, H, float(post.eps), STREAM],
+                               alt.when & when & galt.when if galt is not None else alt.when & when)
+        write(ALWAYS, next_norm, None)
         program.pending = None
+        if next_norm is None:
+            program.stream_written(first, write, eps=post.eps)
 
     def native(self, program, view: CacheView) -> None:
         if type(self).forward is not SandwichBlock.forward:
@@ -240,13 +246,28 @@ class ParallelBlock(Block):
     def native(self, program, view: CacheView) -> None:
         if type(self).forward is not ParallelBlock.forward:
             return super().native(program, view)
+        from .mlp import DenseFeedForward, SwiGLUFeedForward
+        from .rmsnorm import RMSNorm
         if self.extra.get("stream_in") is not None and view.pass_index > 0:
             self.extra["stream_in"].native(program, view)
-        self.mixer_norm.native(program, None)
+        # the feed-forward's norm is of the same rows as the mixer's: one launch for both, each into a buffer of its own, where both
+        # are the stock norm and the feed-forward's launches name what they read when they are written (one written in
+        # Python looks at ``program.x`` as it runs)
+        both = (self.feed_forward is not None and type(self.mixer_norm) is RMSNorm and type(self.feed_forward_norm) is RMSNorm
+                and self.mixer_norm.eps == self.feed_forward_norm.eps and type(self.feed_forward) in (SwiGLUFeedForward, DenseFeedForward))
+        if both:
+            beside = program.buffer("parallel.x", program.T * program.hidden_size * program.act_bytes)
+            self.mixer_norm.native(program, None, side=(self.feed_forward_norm, beside))
+        else:
+            self.mixer_norm.native(program, None)
         self.mixer.native(program, view)
         a, program.pending = program.pending, None
         f = None
-        if self.feed_forward is not None:
+        if both:
+            kept, program.x = program.x, beside
+            self.feed_forward.native(program, None)
+            f, program.pending, program.x = program.pending, None, kept
+        elif self.feed_forward is not None:
             self.feed_forward_norm.native(program, None)          # nothing pending: the norm of the same stream
             self.feed_forward.native(program, None)
             f, program.pending = program.pending, None

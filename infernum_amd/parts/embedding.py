@@ -18,6 +18,7 @@ from .base import Embedding, Head, Runtime, StepContext, WeightSpec, register_pa
 from .linear import Finish, emit_linear, linear
 
 
+FEW_ROWS = 256          # rows whose embedding and norm are one launch: a workgroup a row, on a compute unit of its own
 EMBEDDING_OUTPUT = "embedding.out"
 EMBEDDING_OUTPUT_F32 = "embedding.out.f32"      # with keep_output="fp32": the rows as they entered the stream, unrounded
 
@@ -75,22 +76,41 @@ class TokenEmbedding(Embedding):
     def native(self, program, view=None) -> None:
         if type(self).forward is not TokenEmbedding.forward:
             return super().native(program, view)
-        from ..engine.program import STREAM
-        program.op("core", "ia_embed", [self.table, K.DTYPE_CODE[self.table.dtype], program.token_ids, program.h,
-                                        program.N, self.hidden_size, self.vocab_size, float(self.scale), STREAM])
-        if self.pos_rows is not None:
-            program.op("core", "ia_add_rows", [program.h, self.pos_rows, K.DTYPE_CODE[self.pos_rows.dtype],
-                                               program.positions, program.N, self.hidden_size,
-                                               int(self.pos_rows.shape[0]), STREAM])
-        if self.keep_output:
-            kept = program.buffer(EMBEDDING_OUTPUT, program.T * self.hidden_size * program.act_bytes)
-            program.op("core", "ia_cast", [program.h, K.DTYPE_CODE[torch.float32], kept, program.act_code,
-                                           program.N * self.hidden_size, STREAM])
+        from ..engine.program import ALWAYS, STREAM, Guard
+        H, N, f32 = self.hidden_size, program.N, K.DTYPE_CODE[torch.float32]
+        code = lambda t: K.DTYPE_CODE[t.dtype] if t is not None else 0          # noqa: E731
+        kept = program.buffer(EMBEDDING_OUTPUT, program.T * H * program.act_bytes) if self.keep_output else None
+        pos, pos_rows = self.pos_rows, int(self.pos_rows.shape[0]) if self.pos_rows is not None else 0
+
+        def begin(vector: Optional[torch.Tensor]) -> None:
+            def write(when, norm, side) -> None:
+                if norm is not None:
+                    behind = [None, 0, program.x, None, 0, None] if norm == "cast" else norm.next_operands(program, side)
+                    program.op("core", "ia_embed_norm",
+                               [self.table, code(self.table), program.token_ids, pos, code(pos), program.positions if pos is not None else None,
+                                pos_rows, vector, code(vector), program.h, kept] + behind +
+                               [program.act_code, N, H, self.vocab_size, float(self.scale),
+                                float(norm.eps) if norm != "cast" else 1.0, STREAM], when)
+                    return
+                program.op("core", "ia_embed", [self.table, code(self.table), program.token_ids, program.h, N, H, self.vocab_size,
+                                                float(self.scale), STREAM], when)
+                if pos is not None:
+                    program.op("core", "ia_add_rows", [program.h, pos, code(pos), program.positions, N, H, pos_rows, STREAM], when)
+                if kept is not None:
+                    program.op("core", "ia_cast", [program.h, f32, kept, program.act_code, N * H, STREAM], when)
+                if vector is not None:
+                    program.op("core", "ia_add_vector", [program.h, vector, code(vector), N, H, STREAM], when)
+            first = len(program._ops)
+            write(ALWAYS, None, None)
+            program.pending = None
+            # one launch for a few rows' embedding and the norm behind it; with many each pass runs at the rate of a copy
+            aligned = all(t is None or t.data_ptr() % 16 == 0 for t in (self.table, pos, vector))
+            if H % 8 == 0 and (H <= 1024 or 2048 <= H <= 4096) and aligned:
+                program.stream_written(first, write, Guard.between(N, None, FEW_ROWS), add_vector=begin if vector is None else None)
+        begin(None)
         if self.keep_f32:
-            kept = program.buffer(EMBEDDING_OUTPUT_F32, program.T * self.hidden_size * 4)
-            f32 = K.DTYPE_CODE[torch.float32]
-            program.op("core", "ia_cast", [program.h, f32, kept, f32, program.N * self.hidden_size, STREAM])
-        program.pending = None
+            whole = program.buffer(EMBEDDING_OUTPUT_F32, program.T * H * 4)
+            program.op("core", "ia_cast", [program.h, f32, whole, f32, N * H, STREAM])
 
 
 class LinearHead(Head):

@@ -55,18 +55,38 @@ class RMSNorm(Norm):
 
     def native_branch(self, program, x_out: bool = True) -> None:
         """:meth:`add_normed` of ``program.pending`` into ``program.h``; the new h, rounded, goes to ``program.x``."""
-        from ..engine.program import STREAM
+        from ..engine.program import ALWAYS, STREAM
         if program.pending is None:
             raise K.KernelError("norm on a branch: there is no branch output to normalise")
-        for alt in program.pending.alts:
-            if not alt.splits and alt.dtype != self.rt.dtype:
-                raise K.KernelError("norm_add: the delta must have the activations' dtype")
-            code = K.DTYPE_CODE[torch.float32] if alt.splits else program.act_code
-            program.op("core", "ia_norm_add",
-                       [program.h, alt.where, code, alt.splits or 1, program.N, self.weight,
-                        K.DTYPE_CODE[self.weight.dtype], program.x if x_out else None, program.act_code, program.N,
-                        self.size, float(self.eps), STREAM], alt.when)
+        branch, f32, first = program.pending, K.DTYPE_CODE[torch.float32], len(program._ops)
+
+        def write(when, norm, side) -> None:
+            for alt in branch.alts:
+                if not alt.splits and alt.dtype != self.rt.dtype:
+                    raise K.KernelError("norm_add: the delta must have the activations' dtype")
+                code, head = f32 if alt.splits else program.act_code, [program.h, alt.where]
+                weight = [self.weight, K.DTYPE_CODE[self.weight.dtype]]
+                if norm is None:
+                    program.op("core", "ia_norm_add",
+                               head + [code, alt.splits or 1, program.N] + weight +
+                               [program.x if x_out else None, program.act_code, program.N, self.size, float(self.eps),
+                                STREAM], alt.when & when)
+                else:
+                    program.op("core", "ia_gated_norm_add",
+                               head + [code, alt.splits or 1, program.N, None, f32, self.size, 1, program.N, None] + weight +
+                               norm.next_operands(program, side) +
+                               [program.act_code, program.N, self.size, float(self.eps), STREAM], alt.when & when)
+        write(ALWAYS, None, None)
         program.pending = None
+        program.stream_written(first, write, eps=self.eps)
+
+    def next_operands(self, program, side) -> list:
+        """This norm's weight and ``program.x``, and the norm beside it with its buffer (or None), as the launchers that
+        complete the stream take them."""
+        other, where = side or (None, None)
+        program.keep(self.weight, other.weight if other is not None else None)
+        return [self.weight, K.DTYPE_CODE[self.weight.dtype], program.x, other.weight if other is not None else None,
+                K.DTYPE_CODE[other.weight.dtype] if other is not None else 0, where]
 
     def forward(self, h: torch.Tensor, delta, out: Optional[torch.Tensor] = None,
                 rows: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -76,12 +96,14 @@ class RMSNorm(Norm):
         return K.add_rmsnorm(h, delta, self.weight, self.eps, out, rows)
 
 
-    def native(self, program, view=None, rows: bool = False) -> None:
-        """One launch per form the pending delta can have (none, a tensor, partial sums of a split product)."""
+    def native(self, program, view=None, rows: bool = False, side: Optional[tuple] = None) -> None:
+        """One launch per form the pending delta can have (none, a tensor, partial sums of a split product); none where
+        the launch that completed the stream takes the norm along (``StepProgram.norm_rides``).  ``side``: another
+        norm of the same rows and root, and the buffer for it."""
         if type(self).forward is not RMSNorm.forward:
             return super().native(program, view, rows)          # a subclass that computes something else
         from ..engine.program import ALWAYS, STREAM, Guard
-        base = Guard.between(program.R, 1) if rows else ALWAYS
+        base = (Guard.between(program.R, 1) if rows else ALWAYS) & ~program.norm_rides(self, rows, side)
         for alt in (program.pending.alts if program.pending is not None else [None]):
             delta, code, splits, when = None, program.act_code, 1, base
             if alt is not None:
@@ -91,7 +113,8 @@ class RMSNorm(Norm):
                 code, splits = (K.DTYPE_CODE[torch.float32], alt.splits) if alt.splits else (program.act_code, 1)
             program.op("core", "ia_add_rmsnorm",
                        [program.h, delta, code, splits, program.N, program.act_code, self.weight,
-                        K.DTYPE_CODE[self.weight.dtype], program.x, program.logit_rows if rows else None,
+                        K.DTYPE_CODE[self.weight.dtype], program.x] + self.next_operands(program, side)[3:] +
+                       [program.logit_rows if rows else None,
                         program.R if rows else program.N, self.size, float(self.eps), STREAM], when)
         program.pending = None
 

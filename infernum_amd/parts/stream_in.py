@@ -128,6 +128,8 @@ class PassVectorStreamIn(Part):
         program.pending = None
         program.keep(self.table)
         vector = self.table[view.pass_index if view is not None else 0]
+        if program.vector_rides(vector):
+            return
         program.op("core", "ia_add_vector", [program.h, vector, K.DTYPE_CODE[vector.dtype], N, H, STREAM])
 
 

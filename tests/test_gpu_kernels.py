@@ -40,6 +40,69 @@ def test_embed_bad_id_gives_nan_not_a_fault():
     assert torch.equal(out[0], table[3]) and out[1].isnan().all() and out[2].isnan().all()
 
 
+# rows shorter than a wave's piece and than a workgroup's, the longest of either kernel; ids and positions outside their tables; the
+# bits of embedding, positions, cast, vector and norm as launches of their own
+@pytest.mark.parametrize("act", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N,H", [(1, 8), (3, 264), (2, 1024), (5, 2048), (2, 2056), (256, 4096)])
+def test_embedding_and_norm_in_one_launch_leave_the_bits_of_separate_launches(N, H, act):
+    api = K()
+    V, P = 61, 37
+    table, pos = _rand(V, H, dtype=act, seed=1), _rand(P, H, dtype=torch.bfloat16, seed=2)
+    vector, w, w2 = _rand(H, seed=3), _rand(H, dtype=torch.bfloat16, seed=4), _rand(H, seed=5)
+    ids = torch.randint(0, V, (N,), dtype=torch.int32, device=DEV)
+    at = torch.randint(0, P, (N,), dtype=torch.int32, device=DEV)
+    if N > 2:
+        ids[1], at[2] = V, P
+    full = lambda: torch.full((N, H), 7.0, dtype=act, device=DEV)          # noqa: E731
+    for with_pos, with_vector, scale in ((False, False, 1.0), (True, True, 45.3), (True, False, 1.0), (False, True, 0.3)):
+        h = torch.empty(N, H, device=DEV)
+        api.embed(table, ids, h, scale)
+        if with_pos:
+            api.add_rows(h, pos, at)
+        kept = api.cast(h, act).clone()
+        if with_vector:
+            api.add_vector(h, vector)
+        x, x2 = full(), full()
+        api.add_rmsnorm(h, None, w, 1e-6, x)
+        api.add_rmsnorm(h, None, w2, 1e-6, x2)
+        gh, gk, gx, gx2 = torch.empty_like(h), full(), full(), full()
+        kw = dict(scale=scale, position_table=pos if with_pos else None, positions=at if with_pos else None,
+                  vector=vector if with_vector else None)
+        api.embed_norm(table, ids, gh, w, 1e-6, gx, kept=gk, side_weight=w2, out_side=gx2, **kw)
+        for a, b in ((h, gh), (kept, gk), (x, gx), (x2, gx2)):
+            assert torch.equal(a.nan_to_num(123.0), b.nan_to_num(123.0))
+        gx.fill_(7.0)
+        api.embed_norm(table, ids, gh, None, 1e-6, gx, **kw)
+        assert torch.equal(gx.nan_to_num(123.0), api.cast(h, act).nan_to_num(123.0))
+
+
+@pytest.mark.parametrize("splits", [0, 1, 3, 8])
+@pytest.mark.parametrize("N,H", [(1, 60), (3, 1024), (2, 1100), (1, 2048), (300, 2048), (2, 4096), (3, 6000), (2, 77)])
+def test_norms_of_a_sublayer_beside_the_next_one(N, H, splits):
+    """A second norm of the same rows equals a launch of its own: behind the add, and behind a branch."""
+    api, bf = K(), torch.bfloat16
+    h0, w, w2, wb = _rand(N, H, seed=1), _rand(H, dtype=bf, seed=2), _rand(H, seed=3), _rand(H, seed=4)
+    d = api.SplitSum(_rand(splits, N, H, seed=5)) if splits else _rand(N, H, dtype=bf, seed=5)
+    new = lambda: torch.full((N, H), 7.0, dtype=bf, device=DEV)            # noqa: E731
+    h, a, a2, b2 = h0.clone(), new(), new(), new()
+    api.add_rmsnorm(h, d, w, 1e-5, a, None, w2, a2)
+    hb, b = h0.clone(), new()
+    api.add_rmsnorm(hb, d, w, 1e-5, b)
+    api.add_rmsnorm(hb, None, w2, 1e-5, b2)
+    assert torch.equal(h, hb) and torch.equal(a, b) and torch.equal(a2, b2)
+    h, a, a2 = h0.clone(), new(), new()
+    api.gated_norm_add(h, d, None, None, wb, 1e-5, w, a, w2, a2)
+    hb, b, b2 = h0.clone(), new(), new()
+    api.norm_add(hb, d, wb, 1e-5)
+    api.add_rmsnorm(hb, None, w, 1e-5, b)
+    api.add_rmsnorm(hb, None, w2, 1e-5, b2)
+    assert torch.equal(h, hb)
+    if H % 4 == 0 and (H <= 1024 or H >= 2048):        # where one order of the sums of squares is promised
+        assert torch.equal(a, b) and torch.equal(a2, b2)
+    else:                                              # another order: the root's error, then one rounding to bf16
+        assert torch.allclose(a.float(), b.float(), rtol=2 ** -7) and torch.allclose(a2.float(), b2.float(), rtol=2 ** -7)
+
+
 @pytest.mark.parametrize("dtype,wdtype", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16),
                                           (torch.bfloat16, torch.float32)])
 @pytest.mark.parametrize("H", [4, 100, 2048, 5120])
