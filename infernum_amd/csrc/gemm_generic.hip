@@ -135,10 +135,8 @@ __device__ __forceinline__ void store_four(float* __restrict__ C, int m, int n, 
 // row of workgroups), PIECE chains of 16 at a time in two sets of registers: the next piece is asked for before this one is worked
 // on, and no load has a condition (what lies beyond K is read from the row's end and cleared), so that the wait for one piece
 // leaves the other under way.  The stretches' sums meet in LDS, where they are added in the order of k.
-// Cold weights, us before (all of half a stretch's loads, then its products, eight waves) and now: 128,256 x 2,048 at 1 / 4 / 16
-// rows 250 / 274 / 303 and 173 / 191 / 249 (1.05 GB: 6.1 to 4.2 TB/s); 16,384 x 2,048 37.6 / 39.8 / 41.7 and 26.6 / 28.7 / 34.1; 2,048 x 8,192
-// 28.8 / 31.5 / 44.3 and 24.3 / 27.1 / 38.8; 4,096 x 14,336 at 1 row 50.9 and 44.5; 16,384 x 2,048 at 17 / 32 rows 82.4 / 87.1 and 41.3 / 45.0;
-// 2,048 x 8,192 at 64 / 142 rows 166 / 173 (the tiles below) and 52.6 / 100.
+// Cold weights, us: 128,256 x 2,048 at 1 / 4 / 12 rows 178 / 195 / 229 (1.05 GB: 5.9 to 4.6 TB/s); 16,384 x 2,048 27.5 / 29.3 / 33.1;
+// 2,048 x 8,192 24.1 / 26.8 / 34.3; 28,672 x 4,096 87.9 / 93.7 / 108; shapes of more rows beside the rule below.
 template <int MT, int RT, int WAVES, int PIECE>
 __global__ __launch_bounds__(WAVES * 64) void gemm_f32_stream_kernel(const float* __restrict__ A,
                                                                      const float* __restrict__ W,
@@ -146,26 +144,31 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_stream_kernel(const float
                                                                      int lda, int ldw, int ldc, bool wide) {
   constexpr int TILES = MT * RT, OWN = (TILES + WAVES - 1) / WAVES;    // tiles whose stretches a wave adds up
   static_assert(16 % (2 * PIECE) == 0, "a stretch is a whole number of pairs of pieces");
+  // written out for the smallest tile only: of the others, a whole stretch at once kept twice the registers and more (48 x 32 all
+  // 512), one wave a SIMD for two or three (142 rows x 2,048 x 8,192 107 us, as a loop 91; 40 x 6,144 x 4,096 57.8 and 50.4)
+  constexpr int ROUNDS = TILES == 1 ? 16 / (2 * PIECE) : 1;
   __shared__ gf32x4 mids[2][WAVES][TILES][64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 15, q = lane >> 4;
   const int n0 = blockIdx.x * (16 * RT), m0 = blockIdx.y * (16 * MT);
-  const float* wrow[RT];
-  const float* arow[MT];
+  // the workgroup's first rows as scalars, a lane's place behind them in 32 bits (the host looks after that)
+  const char* const wbase = (const char*)(W + (size_t)n0 * ldw);
+  const char* const abase = (const char*)(A + (size_t)m0 * lda);
+  uint32_t wrow[RT], arow[MT];
 #pragma unroll
-  for (int i = 0; i < RT; ++i) wrow[i] = W + (size_t)min(n0 + 16 * i + r, N - 1) * ldw;
+  for (int i = 0; i < RT; ++i) wrow[i] = (uint32_t)min(16 * i + r, N - 1 - n0) * (uint32_t)ldw * 4u;
 #pragma unroll
-  for (int i = 0; i < MT; ++i) arow[i] = A + (size_t)min(m0 + 16 * i + r, M - 1) * lda;
+  for (int i = 0; i < MT; ++i) arow[i] = (uint32_t)min(16 * i + r, M - 1 - m0) * (uint32_t)lda * 4u;
   const int stretches = (K + 255) / 256;
   float4 w0[PIECE][RT], x0[PIECE][MT], w1[PIECE][RT], x1[PIECE][MT];
   auto load = [&](int k0, float4 (&w)[PIECE][RT], float4 (&x)[PIECE][MT]) {
 #pragma unroll
     for (int c = 0; c < PIECE; ++c) {
-      const int k = min(k0 + 16 * c + 4 * q, K - 4);
+      const uint32_t k = (uint32_t)min(k0 + 16 * c + 4 * q, K - 4) * 4u;
 #pragma unroll
-      for (int i = 0; i < RT; ++i) w[c][i] = *reinterpret_cast<const float4*>(wrow[i] + k);
+      for (int i = 0; i < RT; ++i) w[c][i] = *reinterpret_cast<const float4*>(wbase + (wrow[i] + k));
 #pragma unroll
-      for (int i = 0; i < MT; ++i) x[c][i] = *reinterpret_cast<const float4*>(arow[i] + k);
+      for (int i = 0; i < MT; ++i) x[c][i] = *reinterpret_cast<const float4*>(abase + (arow[i] + k));
     }
   };
   gf32x4 mid[TILES];
@@ -203,7 +206,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_stream_kernel(const float
 #pragma unroll
       for (int t = 0; t < TILES; ++t) mid[t] = gf32x4{0.f, 0.f, 0.f, 0.f};
       const int next = s + WAVES < stretches ? k0 + WAVES * 256 : k0;  // behind the wave's last stretch anything that can be read
-#pragma unroll
+#pragma clang loop unroll_count(ROUNDS)
       for (int c = 0; c < 16; c += 2 * PIECE) {
         load(k0 + 16 * (c + PIECE), w1, x1);
         __builtin_amdgcn_sched_barrier(0);                             // all of them in front of the first wait
@@ -230,7 +233,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_stream_kernel(const float
 }
 
 // Many rows: bound by the matrix instructions (157 TFLOP/s): 2,048 rows x 28,672 x 4,096 at 102 TFLOP/s, 4.7 against
-// 12.7 ms with the vector kernel; 142 rows x 2,048 x 8,192 178 against 1,315 us (320 workgroups, a chain of K).  Tiles of 32 WM rows of A x 32 WN rows of W, four waves, 16 WM x 16 WN of the result each.  K is walked 32
+// 12.7 ms with the vector kernel.  Tiles of 32 WM rows of A x 32 WN rows of W, four waves, 16 WM x 16 WN of the result each.  K is walked 32
 // values (two chains) at a time through two LDS stages, written as the matrix instructions read them; the loads of the
 // stage after next are in flight meanwhile.
 template <int WM, int WN>
@@ -344,35 +347,47 @@ static bool gemm_f32(const float* A, const float* W, float* C, int M, int N, int
   if (M <= GS_MOST_ROWS && (K <= 16 || (N > 4096 && K <= (M > 16 ? 96 : 48)))) return false;
   const bool wide = ((uintptr_t)C & 15) == 0 && (ldc & 3) == 0;
   // Up to 16 rows: 16 rows of W a workgroup, of 16 waves where those are at most one a compute unit and each wave has a stretch
-  // (4,096 x 4,096 at 1 row 15.7 us, with four waves 19.6; 6,144 x 4,096 26.5 and 25.2), of four otherwise; from nine rows on, whose
-  // reads then weigh as much as W's, 64 rows of W share them (16 rows x 128,256 x 2,048 249 us, with 16 rows of W 295; 8,192 x 2,048, which
-  // that leaves 128 workgroups, 28.6 and 20.2).
-  if (M <= 16) {
+  // (4,096 x 4,096 at 1 row 15.7 us, with four waves 19.6; 6,144 x 4,096 26.5 and 25.2), of eight where each has two (28,672 x 4,096
+  // at 1 / 4 rows 87.9 / 93.7, with four 94.7 / 98.4; with one each 16,384 x 2,048 29.7, with four 27.5), of four otherwise; from nine
+  // rows on, whose reads then weigh as much as W's, 64 rows of W share them (16 rows x 128,256 x 2,048 249 us, with 16 rows
+  // of W 295; 8,192 x 2,048, which that leaves 128 workgroups, 28.6 and 20.2).
+  const bool near = lda < 1 << 24 && ldw < 1 << 24;                    // 64 rows within 32 bits of the first
+  if (M <= 16 && near) {
     if (N <= 16 * GS_UNITS && K > 1024) launch_f32_stream<1, 1, 16, 2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
     else if (M > 8 && N >= 64 * GS_UNITS) launch_f32_stream<1, 4, 4, 2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
+    else if (M <= 8 && K >= 4096) launch_f32_stream<1, 1, 8, 2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
     else launch_f32_stream<1, 1, 4, 2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
     return true;
   }
-  // Above: the matrix instructions of a compute unit are what its one workgroup of four waves has, so a shape costs its
-  // workgroups in turns of the compute units, and the tiles below, which share both operands but walk K in step with two
-  // barriers every 32 values, as much as some 2.7 turns of theirs at the least.  Per turn, us with K of 8,192: 32 x 16 of the result 50,
-  // 32 x 32 70, 48 x 32 100, tiles of 32 x 32 62 (166 at the least).  Three stretches of K and fewer leave waves without one (4,099 x 516
-  // at 33 rows 15.2 us, the tiles 12.5; 1,000 x 1,000 7.8 and 18.0).
-  auto turns = [&](int rows, int cols) {
-    const long groups = (long)((M + rows - 1) / rows) * ((N + cols - 1) / cols);
-    return (groups + GS_UNITS - 1) / GS_UNITS;
-  };
-  const long c21 = 50 * turns(32, 16), c22 = 70 * turns(32, 32), c32 = 100 * turns(48, 32);
-  const long tiles = 62L * ((M + 31) / 32) * ((N + 31) / 32) / GS_UNITS, least = tiles < 166 ? 166 : tiles;
-  const long best = c21 < c22 ? (c21 < c32 ? c21 : c32) : (c22 < c32 ? c22 : c32);
-  if (M <= GS_MOST_ROWS || (K > 768 && 10 * best < 9 * least)) {
-    if (c21 <= best) launch_f32_stream<2, 1, 4, 2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
-    else if (c22 <= best || M <= GS_MOST_ROWS) launch_f32_stream<2, 2, 4, 2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
-    else launch_f32_stream<3, 2, 4, 1>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
+  // Above: the matrix instructions of a compute unit are what its workgroup has, so a shape costs its workgroups in turns of
+  // the compute units, and the tile that wastes least of the last turn and of the last rows wins.  A turn, us with K of 8,192: 16
+  // x 16 of the result 35, 32 x 16 50, 32 x 32 69, 48 x 32 84, 64 x 32 100, 48 x 48 112, 48 x 64 155, 64 x 64 198 (from 64 x 32 on 12.4 to 12.9 a
+  // tile of 16 x 16; the matrix instructions alone 6.8).  The tiles below share both operands but walk K in step with two barriers
+  // every 32 values; several of them on a compute unit make up for that, so they cost by the share of a turn: 128 x 128 of many rows
+  // 680, 64 x 64 190, 32 x 32 62 and 166 at the least.  Cold weights, us with 32 x 16, 32 x 32 and 48 x 32 alone and now: 16,384 x 2,048 at 40 / 96 /
+  // 142 rows 61.8 / 110 / 157 and 45.1 / 85.4 / 126, 6,144 x 4,096 at 64 / 96 / 142 76.8 / 116 / 155 and 57.4 / 59.2 / 107, 4,096 x 14,336 at
+  // 142 / 220 372 / 452 and 264 / 349, 2,048 x 8,192 at 24 / 142 / 300 48.3 / 107 / 219 and 35.2 / 84.0 / 154, 128,256 x 2,048 at 142 1,373 and 1,012.
+  // (300 x 128,256 x 2,048, where both cost the same by this rule: 2,053 in tiles, 2,236 in 64 x 64: the tiles unless 2 % are won.)
+  // Three stretches of K and fewer leave waves without one (4,099 x 516 at 33 rows 15.2 us, the tiles 12.5; 1,000 x 1,000 7.8 and 18.0).
+  typedef void (*Launch)(const float*, const float*, float*, int, int, int, int, int, int, bool, hipStream_t);
+  static const struct { int rows, cols, turn; Launch launch; } shapes[] = {
+      {16, 16, 35, launch_f32_stream<1, 1, 16, 2>}, {32, 16, 50, launch_f32_stream<2, 1, 4, 2>}, {32, 32, 69, launch_f32_stream<2, 2, 4, 2>},
+      {48, 32, 84, launch_f32_stream<3, 2, 8, 1>},  {64, 32, 100, launch_f32_stream<4, 2, 8, 1>}, {48, 48, 112, launch_f32_stream<3, 3, 8, 1>},
+      {48, 64, 155, launch_f32_stream<3, 4, 4, 1>}, {64, 64, 198, launch_f32_stream<4, 4, 4, 1>}};
+  long best = 0;
+  Launch launch = nullptr;
+  for (const auto& s : shapes) {
+    const long groups = (long)((M + s.rows - 1) / s.rows) * ((N + s.cols - 1) / s.cols), cost = s.turn * ((groups + GS_UNITS - 1) / GS_UNITS);
+    if (!launch || cost < best) { best = cost; launch = s.launch; }
+  }
+  const long t44 = f32_tiles<4, 4>(M, N), t22 = f32_tiles<2, 2>(M, N), t11 = 62 * f32_tiles<1, 1>(M, N) / GS_UNITS;
+  const long tiles = t44 >= GS_ENOUGH_TILES ? 680 * t44 / GS_UNITS : t22 >= GS_ENOUGH_TILES ? 190 * t22 / GS_UNITS : t11 < 166 ? 166 : t11;
+  if (near && (M <= GS_MOST_ROWS || (K > 768 && 50 * best < 49 * tiles))) {
+    launch(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
     return true;
   }
-  if (f32_tiles<4, 4>(M, N) >= GS_ENOUGH_TILES) launch_f32_tile<4, 4>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
-  else if (f32_tiles<2, 2>(M, N) >= GS_ENOUGH_TILES) launch_f32_tile<2, 2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
+  if (t44 >= GS_ENOUGH_TILES) launch_f32_tile<4, 4>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
+  else if (t22 >= GS_ENOUGH_TILES) launch_f32_tile<2, 2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
   else launch_f32_tile<1, 1>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
   return true;
 }

@@ -425,11 +425,14 @@ def test_gemm_fp32_on_the_matrix_cores_leaves_the_vector_kernels_bits(M, N, K_):
     assert bool(((got.double() - exact).abs() <= bound).all())
 
 
-# the streaming kernel's shapes: 16 rows of A x 16 of W in sixteen waves, in four, x 64; 32 x 16, 32 x 32, 48 x 32; each with rows that
-# fill no group and a last stretch of one piece, of a part of one, and of all; more waves than stretches, and a stretch more
+# the streaming kernel's shapes: 16 rows of A x 16 of W in sixteen waves, in four, in eight, x 64; 32 x 16, 32 x 32, 48 x 32, 64 x 32, 48 x 48,
+# 48 x 64, 64 x 64; each with rows that fill no group and a last stretch of one piece, of a part of one, and of all; more waves than
+# stretches, and a stretch more
 @pytest.mark.parametrize("M,N,K_", [(3, 100, 1028), (16, 4096, 4096), (1, 4090, 4360), (5, 5000, 1284), (2, 1000, 1024), (1, 70, 264),
                                     (9, 16400, 264), (16, 16385, 1028), (17, 70, 2052), (64, 2040, 1284), (96, 2050, 1316),
-                                    (32, 16390, 260), (142, 2050, 1284), (130, 1990, 1024)])
+                                    (32, 16390, 260), (142, 2050, 1284), (130, 1990, 1024), (7, 4100, 4100), (19, 1990, 2052),
+                                    (200, 2040, 1028), (250, 2047, 2308), (95, 6130, 1284), (140, 6143, 1028), (47, 16380, 2052),
+                                    (142, 16383, 1028), (63, 16384, 1284), (301, 3070, 1028)])
 def test_gemm_fp32_streamed_leaves_the_vector_kernels_bits(M, N, K_):
     test_gemm_fp32_on_the_matrix_cores_leaves_the_vector_kernels_bits(M, N, K_)
 
