@@ -332,8 +332,6 @@ __global__ __launch_bounds__(WAVES * 64, ((WAVES == 4 && IA_MAX_DIM <= 128) ? 3 
   const int h = g * G + hj;
   const int heads_here = (G - ht * 16) < 16 ? (G - ht * 16) : 16;
 
-  // FUSED: the sums of the queries' pairs are asked for first of all (they need nothing but the token's row),
-  // so that they come in while the position, the block table and the angles are worked out
   constexpr int QPT = (16 * (HD / 2) + NT - 1) / NT;        // pairs of query values a thread may have to rotate
   float qa[FUSED ? QPT : 1], qb[FUSED ? QPT : 1];
   const int half = FUSED ? F.rot >> 1 : 0;
@@ -363,17 +361,6 @@ __global__ __launch_bounds__(WAVES * 64, ((WAVES == 4 && IA_MAX_DIM <= 128) ? 3 
     }
     if (has_tail && F.slots != nullptr && F.rot + tid < HD)
       kc = load_split_sum_together(row + (size_t)(nh + g) * HD + F.rot + tid, F.gsplits, F.split_stride);
-#pragma unroll
-    for (int u = 0; u < QPT; ++u) {
-      const int idx = tid + u * NT;
-      qa[u] = qb[u] = 0.f;
-      if (idx < heads_here * half) {
-        const int c = idx / half, i = idx - c * half;
-        const TS* x = row + (size_t)(g * G + ht * 16 + c) * HD + i;
-        qa[u] = load_split_sum_together(x, F.gsplits, F.split_stride);
-        qb[u] = load_split_sum_together(x + half, F.gsplits, F.split_stride);
-      }
-    }
   }
 
   // the start of the request's block table is asked for together with its position, not after it: a request of
@@ -381,6 +368,41 @@ __global__ __launch_bounds__(WAVES * 64, ((WAVES == 4 && IA_MAX_DIM <= 128) ? 3 
   const int* bt = block_tables + (size_t)b * bt_stride;
   const int bt_ahead = tid < bt_stride ? bt[tid] : -1;
   const int p = positions[b];
+  // and so is this thread's frequency, and behind them the parts of the queries' pairs, of the key's pair and of the value, all in
+  // one go, the latter two also by workgroups that turn out not to own the token's key: with the key and the value asked for once the
+  // position was there, the frequency behind that, and every part under a condition, one token of the 1B shape (8 parts, 45 keys)
+  // took 8.6 us in a decoded step, so 6.4
+  double freq64 = 0.0;
+  float freq32 = 0.f, ka = 0.f, kb = 0.f, vv = 0.f;
+  if (FUSED) {
+    if (tid < half) {
+      if (F.freq_f64) freq64 = reinterpret_cast<const double*>(F.inv_freq)[tid];
+      else freq32 = reinterpret_cast<const float*>(F.inv_freq)[tid];
+    }
+    auto query = [&](int idx) {                              // the pair's first value; without rotation, or beyond the pairs, any
+      const int at = min(idx, max(heads_here * half, 1) - 1), c = half > 0 ? at / half : 0;
+      return row + (size_t)(g * G + ht * 16 + c) * HD + (at - c * half);
+    };
+    {
+      const TS* x = query(tid);
+      const TS* k = F.slots != nullptr ? row + (size_t)(nh + g) * HD + min(tid, max(half, 1) - 1) : x;
+      const TS* const from[5] = {x, x + half, k, k + half, F.slots != nullptr ? row + (size_t)(nh + nkv) * HD + (size_t)g * VD + min(tid, VD - 1) : x};
+      float v[5];
+      load_split_sums<5>(from, F.gsplits, F.split_stride, v);
+      qa[0] = v[0]; qb[0] = v[1]; ka = v[2]; kb = v[3]; vv = v[4];
+    }
+#pragma unroll
+    for (int u = 1; u < QPT; ++u) {
+      qa[u] = qb[u] = 0.f;
+      if (u * NT < heads_here * half) {
+        const TS* x = query(tid + u * NT);
+        const TS* const from[2] = {x, x + half};
+        float v[2];
+        load_split_sums<2>(from, F.gsplits, F.split_stride, v);
+        qa[u] = v[0]; qb[u] = v[1];
+      }
+    }
+  }
   const int lo0 = ia_first_visible_key(p, window);
   // EXT: tiles are counted from t_first - n_keep on; the n_keep tiles before t_first stand for the request's first
   const int n_keep = EXT ? attn_keep_tiles(X.keep, lo0, 16) : 0;
@@ -440,17 +462,10 @@ __global__ __launch_bounds__(WAVES * 64, ((WAVES == 4 && IA_MAX_DIM <= 128) ? 3 
   // this workgroup's keys end with the token's own, which it makes itself
   const bool own_key = FUSED && F.slots != nullptr && ta < tb && t_last < tb;
   if (FUSED) {
-    // the key's pair and the value of this thread, and the angles (one a thread)
-    float ka = 0.f, kb = 0.f, vv = 0.f;
-    if (own_key) {
-      if (tid < half) {
-        const TS* x = row + (size_t)(nh + g) * HD + tid;
-        ka = load_split_sum_together(x, F.gsplits, F.split_stride);
-        kb = load_split_sum_together(x + half, F.gsplits, F.split_stride);
-      }
-      if (tid < VD) vv = load_split_sum_together(row + (size_t)(nh + nkv) * HD + (size_t)g * VD + tid, F.gsplits, F.split_stride);
+    if (tid < half) {                                        // one angle a thread
+      if (F.freq_f64) rope_sincos(p, &freq64, 1, 0, s_sin[tid], s_cos[tid]);
+      else rope_sincos(p, &freq32, 0, 0, s_sin[tid], s_cos[tid]);
     }
-    for (int i = tid; i < half; i += NT) rope_sincos(p, F.inv_freq, F.freq_f64, i, s_sin[i], s_cos[i]);
     // barriers without the fence of __syncthreads(), which would wait for every load in flight: only LDS
     // traffic has to be through
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

@@ -100,6 +100,36 @@ __device__ __forceinline__ float load_split_sum_together(const TS* p, int splits
   return v;
 }
 
+// The sums of several values whose parts lie alike: all parts of all of them are asked for before the first addition, and no load
+// has a condition (the last part is read again in place of those there are not).  The same order of additions, the same bits.
+template <int PRE, int NV, typename TS>
+__device__ __forceinline__ void load_split_sums_by(const TS* const (&p)[NV], int splits, size_t split_stride, float (&v)[NV]) {
+  TS x[NV][PRE];
+#pragma unroll
+  for (int k = 0; k < PRE; ++k)
+#pragma unroll
+    for (int i = 0; i < NV; ++i) x[i][k] = p[i][(size_t)min(k, splits - 1) * split_stride];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    v[i] = to_float(x[i][0]);
+#pragma unroll
+    for (int k = 1; k < PRE; ++k) v[i] = k < splits ? v[i] + to_float(x[i][k]) : v[i];
+  }
+}
+template <int NV, typename TS>
+__device__ __forceinline__ void load_split_sums(const TS* const (&p)[NV], int splits, size_t split_stride, float (&v)[NV]) {
+  if (splits == 1) {
+    load_split_sums_by<1>(p, splits, split_stride, v);
+  } else if (splits <= 4) {
+    load_split_sums_by<4>(p, splits, split_stride, v);
+  } else if (splits <= 8) {
+    load_split_sums_by<8>(p, splits, split_stride, v);
+  } else {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) v[i] = load_split_sum(p[i], splits, split_stride);
+  }
+}
+
 // Four consecutive values as floats.
 __device__ __forceinline__ float4 load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
 __device__ __forceinline__ float4 load4(const bf16_t* p) {
