@@ -359,8 +359,12 @@ __global__ __launch_bounds__(WAVES * 64, ((WAVES == 4 && IA_MAX_DIM <= 128) ? 3 
         }
       }
     }
-    if (has_tail && F.slots != nullptr && F.rot + tid < HD)
-      kc = load_split_sum_together(row + (size_t)(nh + g) * HD + F.rot + tid, F.gsplits, F.split_stride);
+    if (has_tail && F.slots != nullptr && F.rot + tid < HD) {
+      const TS* const from[1] = {row + (size_t)(nh + g) * HD + F.rot + tid};
+      float v[1];
+      load_split_sums<1>(from, F.gsplits, F.split_stride, v);
+      kc = v[0];
+    }
   }
 
   // the start of the request's block table is asked for together with its position, not after it: a request of

@@ -86,22 +86,8 @@ __device__ __forceinline__ float load_split_sum(const TS* p, int splits, size_t 
   return v;
 }
 
-// The same sum with the loads of up to eight parts asked for together, before the first is added (more parts:
-// the loop above).  Same order of additions, so the same bits.
-template <typename TS>
-__device__ __forceinline__ float load_split_sum_together(const TS* p, int splits, size_t split_stride) {
-  if (splits > 8) return load_split_sum(p, splits, split_stride);
-  float x[8];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) x[k] = k < splits ? to_float(p[k * split_stride]) : 0.f;
-  float v = x[0];
-#pragma unroll
-  for (int k = 1; k < 8; ++k) v = k < splits ? v + x[k] : v;
-  return v;
-}
-
 // The sums of several values whose parts lie alike: all parts of all of them are asked for before the first addition, and no load
-// has a condition (the last part is read again in place of those there are not).  The same order of additions, the same bits.
+// has a condition (the last part is read again in place of those there are not; more than eight parts: the loop above).  The same order of additions, the same bits.
 template <int PRE, int NV, typename TS>
 __device__ __forceinline__ void load_split_sums_by(const TS* const (&p)[NV], int splits, size_t split_stride, float (&v)[NV]) {
   TS x[NV][PRE];
