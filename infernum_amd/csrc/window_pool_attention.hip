@@ -440,8 +440,10 @@ __device__ __forceinline__ float wpa_gelu_tanh(float z) {
   return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void gelu_mul_rows_kernel(const T* __restrict__ u, T* __restrict__ y,
+// u may lie there as the fp32 parts of a split product: they are added in the order of their index and rounded as the join of
+// such a product does, whose launch (4.7 us in a decoded step, three a step with three layers) is not needed then.
+template <typename T, typename TU>
+__global__ __launch_bounds__(256) void gelu_mul_rows_kernel(const TU* __restrict__ u, int splits, size_t split_stride, T* __restrict__ y,
                                                             const void* __restrict__ table, int t_dtype, int t_stride,
                                                             int col0, const int* __restrict__ ids, int vocab, long total,
                                                             int C) {
@@ -452,22 +454,30 @@ __global__ __launch_bounds__(256) void gelu_mul_rows_kernel(const T* __restrict_
   const int id = ids[n];
   const float e = (unsigned)id < (unsigned)vocab ? load_as_float(table, t_dtype, (size_t)id * t_stride + col0 + j)
                                                  : __uint_as_float(0x7fc00000u);
-  y[i] = from_float<T>(wpa_gelu_tanh(to_float(u[i])) * e);
+  const TU* const from[1] = {u + i};
+  float v[1];
+  load_split_sums<1>(from, splits, split_stride, v);
+  y[i] = from_float<T>(wpa_gelu_tanh(to_float(from_float<T>(v[0]))) * e);
 }
 
-extern "C" int ia_gelu_mul_rows(const void* u, void* y, int dtype, const void* table, int t_dtype, int t_stride,
-                                int col0, const int* ids, int vocab, int N, int C, hipStream_t stream) {
-  if (N < 0 || C <= 0 || col0 < 0 || t_stride < col0 + C || vocab <= 0) return IA_ERR_BAD_ARG;
+// u [splits, u_rows, C] of u_dtype (y's dtype, or fp32), y [N, C]
+extern "C" int ia_gelu_mul_rows(const void* u, int u_dtype, int splits, int u_rows, void* y, int dtype, const void* table, int t_dtype,
+                                int t_stride, int col0, const int* ids, int vocab, int N, int C, hipStream_t stream) {
+  if (N < 0 || C <= 0 || col0 < 0 || t_stride < col0 + C || vocab <= 0 || splits < 1 || u_rows < N) return IA_ERR_BAD_ARG;
   if (N == 0) return IA_OK;
   if (!u || !y || !table || !ids) return IA_ERR_BAD_ARG;
   const long total = (long)N * C;
   const int grid = (int)((total + 255) / 256);
-  if (dtype == IA_F32)
-    gelu_mul_rows_kernel<float><<<grid, 256, 0, stream>>>((const float*)u, (float*)y, table, t_dtype, t_stride, col0,
-                                                          ids, vocab, total, C);
-  else if (dtype == IA_BF16)
-    gelu_mul_rows_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)u, (bf16_t*)y, table, t_dtype, t_stride, col0,
-                                                           ids, vocab, total, C);
+  const size_t stride = (size_t)u_rows * C;
+  if (dtype == IA_F32 && u_dtype == IA_F32)
+    gelu_mul_rows_kernel<float, float><<<grid, 256, 0, stream>>>((const float*)u, splits, stride, (float*)y, table, t_dtype,
+                                                                 t_stride, col0, ids, vocab, total, C);
+  else if (dtype == IA_BF16 && u_dtype == IA_F32)
+    gelu_mul_rows_kernel<bf16_t, float><<<grid, 256, 0, stream>>>((const float*)u, splits, stride, (bf16_t*)y, table, t_dtype,
+                                                                  t_stride, col0, ids, vocab, total, C);
+  else if (dtype == IA_BF16 && u_dtype == IA_BF16)
+    gelu_mul_rows_kernel<bf16_t, bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)u, splits, stride, (bf16_t*)y, table, t_dtype,
+                                                                   t_stride, col0, ids, vocab, total, C);
   else
     return IA_ERR_BAD_ARG;
   IA_LAUNCH_CHECK();

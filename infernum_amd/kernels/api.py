@@ -2208,19 +2208,23 @@ def rms_rows(x: torch.Tensor, col: int, cols: int, weight: Optional[torch.Tensor
     return out
 
 
-def gelu_mul_rows(u: torch.Tensor, table: torch.Tensor, col: int, ids: torch.Tensor,
-                  out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """out[n, j] = gelu_tanh(u[n, j]) * table[ids[n], col + j]."""
-    N, C = u.shape
-    _need(u.is_cuda and u.is_contiguous() and u.dtype in DTYPE_CODE, "gelu_mul_rows: u [N, C]")
+def gelu_mul_rows(u, table: torch.Tensor, col: int, ids: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """out[n, j] = gelu_tanh(u[n, j]) * table[ids[n], col + j].  ``u``: a tensor, or with ``out`` the :class:`SplitSum` of a product,
+    joined in out's dtype."""
+    split = isinstance(u, SplitSum)
+    u = u.parts if split else u
+    N, C = u.shape[-2:]
+    _need(u.is_cuda and u.is_contiguous() and u.dtype in DTYPE_CODE and (not split or out is not None), "gelu_mul_rows: u [N, C]")
     _need(table.is_cuda and table.dim() == 2 and table.is_contiguous() and table.dtype in DTYPE_CODE
           and 0 <= col and col + C <= table.shape[1], "gelu_mul_rows: the table's rows are too short")
     _i32(ids, N, "gelu_mul_rows ids")
     if out is None:
         out = torch.empty_like(u)
-    _need(out.is_cuda and out.is_contiguous() and out.dtype == u.dtype and out.shape == u.shape, "gelu_mul_rows: out like u")
-    _ok(_core().ia_gelu_mul_rows(_p(u), _p(out), DTYPE_CODE[u.dtype], _p(table), DTYPE_CODE[table.dtype], table.shape[1],
-                                 int(col), _p(ids), table.shape[0], N, C, _stream()), "gelu_mul_rows")
+    _need(out.is_cuda and out.is_contiguous() and (out.dtype == u.dtype or split) and out.shape == (N, C) and out.dtype in DTYPE_CODE,
+          "gelu_mul_rows: out like u")
+    _ok(_core().ia_gelu_mul_rows(_p(u), DTYPE_CODE[u.dtype], u.shape[0] if split else 1, N, _p(out), DTYPE_CODE[out.dtype],
+                                 _p(table), DTYPE_CODE[table.dtype], table.shape[1], int(col), _p(ids), table.shape[0], N, C, _stream()),
+        "gelu_mul_rows")
     return out
 
 

@@ -86,11 +86,14 @@ class GatedTableInput(Part):
         x = self.stream_buffer(program)
         if not x_ready:
             program.op("core", "ia_cast", [program.h, K.DTYPE_CODE[torch.float32], x, program.act_code, N * H, STREAM])
-        u = emit_linear(program, x, N, self.w_gate, rt.dtype, None, False, "token_input.u", "token_input.gate").tensor()
-        program.op("core", "ia_gelu_mul_rows", [u, u, program.act_code, self.table, K.DTYPE_CODE[self.table.dtype],
-                                                self.columns, self.column, program.token_ids, self.vocab_size, N,
-                                                self.dim, STREAM])
-        program.pending = emit_linear(program, u, N, self.w_proj, rt.dtype, None, True, "token_input.y", "token_input.proj")
+        u = emit_linear(program, x, N, self.w_gate, rt.dtype, None, True, "token_input.u", "token_input.gate")
+        g = program.buffer("token_input.g", T * self.dim * program.act_bytes)
+        for alt in u.alts:                                  # whole, or the parts of a split product, which the launch joins
+            code = K.DTYPE_CODE[torch.float32] if alt.splits else K.DTYPE_CODE[alt.dtype]
+            program.op("core", "ia_gelu_mul_rows", [alt.where, code, alt.splits or 1, N, g, program.act_code, self.table,
+                                                    K.DTYPE_CODE[self.table.dtype], self.columns, self.column,
+                                                    program.token_ids, self.vocab_size, N, self.dim, STREAM], alt.when)
+        program.pending = emit_linear(program, g, N, self.w_proj, rt.dtype, None, True, "token_input.y", "token_input.proj")
         self.norm.native_branch(program, x_out=False)
 
 

@@ -76,6 +76,20 @@ def test_embedding_and_norm_in_one_launch_leave_the_bits_of_separate_launches(N,
         assert torch.equal(gx.nan_to_num(123.0), api.cast(h, act).nan_to_num(123.0))
 
 
+@pytest.mark.parametrize("act", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N,C,splits", [(1, 256, 8), (3, 70, 1), (5, 33, 4), (128, 256, 5), (2, 300, 11)])
+def test_gelu_times_a_tables_rows_joins_partial_sums(N, C, splits, act):
+    """The parts of a split product equal the product joined and rounded first."""
+    api = K()
+    table, ids = _rand(19, C + 40, dtype=torch.bfloat16, seed=1), torch.randint(0, 19, (N,), dtype=torch.int32, device=DEV)
+    parts, out = _rand(splits, N, C, seed=2), torch.empty(N, C, dtype=act, device=DEV)
+    whole = parts[0].clone()
+    for k in range(1, splits):
+        whole += parts[k]
+    api.gelu_mul_rows(api.SplitSum(parts), table, 24, ids, out)
+    assert torch.equal(out, api.gelu_mul_rows(whole.to(act), table, 24, ids))
+
+
 @pytest.mark.parametrize("splits", [0, 1, 3, 8])
 @pytest.mark.parametrize("N,H", [(1, 60), (3, 1024), (2, 1100), (1, 2048), (300, 2048), (2, 4096), (3, 6000), (2, 77)])
 def test_norms_of_a_sublayer_beside_the_next_one(N, H, splits):
