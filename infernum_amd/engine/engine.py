@@ -54,7 +54,8 @@ class _DecodeGraph:
 
 class Engine:
     """``use_graphs``: steps in which every request brings one token are recorded into a HIP graph per shape
-    (number of requests, width of the block tables, number of wanted rows) the second time the shape comes,
+    (number of requests, width of the block tables, number of wanted rows and whether they are the
+    requests in their order) the second time the shape comes,
     and replayed from then on: one launch instead of some hundred.  The step's int32 arrays are copied into
     the graph's own input buffer first; pages, state and weights are where they always are.  Models with a
     part that is not marked ``graph_safe`` (one that reads device memory on the host, say) run without."""
