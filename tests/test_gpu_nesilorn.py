@@ -390,6 +390,27 @@ def test_one_request_at_a_time(models, name, dtype, how):
 
 
 @BOTH
+@pytest.mark.parametrize("name", NAMES[:2])
+def test_final_norm_of_all_rows_of_some_and_of_some_twice(models, name, dtype):
+    """The final norm rides on the last branch where the wanted rows are all rows in their order; as many wanted rows otherwise
+    (one twice, one not at all), or fewer, take its own launch.  Repeated until each shape is recorded, against the parts' own forward."""
+    from infernum_amd.engine import StepEntry
+    d, cfg, w, reqs, ref, *_ = models[name]
+    toks = max(reqs.values(), key=len)
+    a, b = _engine(d, dtype, PAGE[name], 64), _engine(d, dtype, PAGE[name], 64, executor="parts", use_graphs=False)
+    for eng in (a, b):
+        eng.step([StepEntry(r, toks[:5 + i], [4]) for i, r in enumerate("xyz")])
+    wants = [[[0], [0], [0]], [[0, 0], [], [0]], [[0], [], []], [[], [], []]]
+    for k in range(12):
+        step = [StepEntry(r, [toks[6 + (k + i) % 3]], wants[k % 4][i]) for i, r in enumerate("xyz")]
+        got, want = a.step(step), b.step(step)
+        assert torch.equal(got, want), k
+    assert a.graph_replays >= 4
+    if a.program is not None:
+        a.program.check_guards()
+
+
+@BOTH
 @pytest.mark.parametrize("name", NAMES)
 def test_mixed_batches_with_pages_used_again(models, name, dtype):
     d, cfg, w, _, _, reqs, ref = models[name]
