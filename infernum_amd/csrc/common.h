@@ -213,6 +213,15 @@ __device__ __forceinline__ float ia_activate(float z, int kind) {
   return z;
 }
 
+// Where the routed experts' products begin their walk over K, by the column of the result: every 256 columns at a chunk of 256 values of
+// their own (a hash of the columns' number), from which they wrap around (moe.hip says why).  The tiles of few pairs and the grouped
+// product of many both start there, so that a pair's result does not depend on how many share the step.
+#define IA_EXPERT_CHUNK 256
+__device__ __forceinline__ int ia_expert_first_chunk(int column, int K) {
+  const unsigned chunks = (unsigned)(K + IA_EXPERT_CHUNK - 1) / IA_EXPERT_CHUNK;
+  return (int)((((unsigned)(column / 256) * 0x9E3779B1u) >> 8) % chunks);
+}
+
 // The first key that a query at position p sees, from the mask's code: 0 all keys from 0; w > 0 a sliding
 // window, the last w keys (p - w + 1 .. p); w < 0 chunks of -w positions counted from the request's start,
 // the keys of the query's own chunk (floor(p / c) c .. p).  Never decreases with p.

@@ -185,8 +185,11 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_mfma_kernel(const
   // own (a hash of its number) and wraps: 46.7 against 57.2 us for the 8B shape's gate+up product at 64 rows, 25.7
   // against 27.8 for its down projection in eight parts.  The start depends on the tile of columns alone, so a row's
   // sums depend neither on the rows beside it nor on the number of rows.
-  constexpr bool ROTATE = SPLIT || GLU;
-  const int rot = ROTATE ? (int)((((unsigned)tn * 0x9E3779B1u) >> 8) % (unsigned)ksteps) : 0;
+  // The grouped product starts where the tiles of few pairs do (ia_expert_first_chunk): the same bits from either.
+  constexpr bool ROTATE = SPLIT || GLU || GROUPED;
+  static_assert(!GROUPED || BN == 256, "the grouped product's tile is the 256 columns that share a start");
+  const int rot = GROUPED ? ia_expert_first_chunk(n0, K) * (IA_EXPERT_CHUNK / GM_BK)
+                  : ROTATE ? (int)((((unsigned)tn * 0x9E3779B1u) >> 8) % (unsigned)ksteps) : 0;
   auto krot = [&](int kt) {
     const int k = kt + rot;
     return (ROTATE && k >= ksteps) ? k - ksteps : k;

@@ -252,19 +252,14 @@ __global__ __launch_bounds__(256) void moe_gate_up_kernel(const T* __restrict__ 
 // v_mfma_f32_16x16x32_bf16 with W's rows as its first operand: lane (r = lane % 16, q = lane / 16) ends with four
 // consecutive columns 4 q .. 4 q + 3 of row r of the result.
 // All workgroups walking K in step read places one row's length apart at the same moment, and where that length is a power
-// of two those lie on few memory channels, so every 256 columns start their walk at a chunk of their own (moe_first_chunk) and
-// wrap around.  The tile of 128 pairs starts there too: an element is one chain over K in an order that
-// depends on K and its column alone.
+// of two those lie on few memory channels, so every 256 columns start their walk at a chunk of their own (ia_expert_first_chunk) and
+// wrap around.  The tile of 128 pairs and the grouped product of gemm_mfma.hip start there too: an element is one chain over K in
+// an order that depends on K and its column alone.
 // Before, tiles of 32 x 128 in steps of 64 through one LDS stage and all walks from the same start (cold weights,
 // gate and up / down, microseconds before and now): 4 of 32 experts of 1,408 x 2,048 22.0 / 15.9 and 12.4 / 7.2; 16 of 16, 32
 // tokens, 44.7 / 20.3 and 35.3 / 19.3 (184 MB: 5.2 TB/s); 16 of 20 of 2,432 x 4,096 136 / 56.6 and 108.6 / 56.4 (5.9 and 5.7 TB/s).
-#define MS_KC 256
+#define MS_KC IA_EXPERT_CHUNK
 #define MS_LD (MS_KC + 8)     // bf16 of a row in LDS (the padding spreads the banks)
-
-__device__ __forceinline__ int moe_first_chunk(int column, int K) {
-  const unsigned chunks = (unsigned)(K + MS_KC - 1) / MS_KC;
-  return (int)((((unsigned)(column / 256) * 0x9E3779B1u) >> 8) % chunks);
-}
 
 // `x_row(r)`: row r of the tile's pairs, 0 <= r < rows; Wm: the expert's matrix [w_rows, K]; this workgroup's columns
 // of the result begin at n0.  Rows of 16-byte alignment, K a multiple of 8.
@@ -276,7 +271,7 @@ __device__ __forceinline__ void moe_stream_tile(const bf16_t* __restrict__ Wm, i
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
   const int n = n0 + (tid >> 6) * 16;
   const bf16_t* wrow = Wm + (size_t)min(n + r, w_rows - 1) * K;
-  const int chunks = (K + MS_KC - 1) / MS_KC, rot = moe_first_chunk(n0, K);
+  const int chunks = (K + MS_KC - 1) / MS_KC, rot = ia_expert_first_chunk(n0, K);
   auto at = [&](int c) {                                     // where chunk c of the walk begins
     const int k = c + rot;
     return (k >= chunks ? k - chunks : k) * MS_KC;
@@ -415,7 +410,7 @@ __global__ __launch_bounds__(512) void moe_gate_up_big_kernel(const bf16_t* __re
       [&](int i, int j0, const float* v) {
         const int p = first + i;
         if (p < last) moe_gate_up_store(y, ff, p, n0 + j0, v, in_w ? in_w[perm[p]] : 1.0f, limit, alpha, shift);
-      }, moe_first_chunk(n0, W) * (MS_KC / TB_KS));
+      }, ia_expert_first_chunk(n0, W) * (MS_KC / TB_KS));
 }
 
 // Tiles of up to ROWS pairs x 16 columns a wave (moe_stream_tile): grid (tiles of the 2 ff columns, moe_most_tiles).
@@ -525,7 +520,7 @@ __global__ __launch_bounds__(512) void moe_down_big_kernel(const bf16_t* __restr
       [&](int r) { return Wd + ((size_t)e * W + n0 + r) * ff; }, last - first, W - n0, ff, lds,
       [&](int i, int j0, const float* v) {
         if (first + i < last) moe_down_store(parts, weights, perm[first + i], top, N, W, n0 + j0, v);
-      }, moe_first_chunk(n0, ff) * (MS_KC / TB_KS));
+      }, ia_expert_first_chunk(n0, ff) * (MS_KC / TB_KS));
 }
 
 template <int ROWS, int WAVES>
@@ -985,7 +980,7 @@ __global__ __launch_bounds__(512) void moe_up_big_kernel(const bf16_t* __restric
       [&](int r) { return Wu + ((size_t)e * ff + n0 + r) * W; }, last - first, ff - n0, W, lds,
       [&](int i, int j0, const float* v) {
         if (first + i < last) moe_up_store(y, ff, first + i, n0 + j0, v, act);
-      }, moe_first_chunk(n0, W) * (MS_KC / TB_KS));
+      }, ia_expert_first_chunk(n0, W) * (MS_KC / TB_KS));
 }
 
 template <int ROWS, int WAVES>

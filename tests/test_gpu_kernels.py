@@ -1727,6 +1727,34 @@ def test_a_pairs_result_does_not_depend_on_the_steps_other_pairs(gated, E, top, 
         assert torch.equal(parts_of(N), want[:, :N]), N
 
 
+# the grouped product that many pairs of an expert take from some number on: a step of so many tokens, one of a token less (the tiles),
+# and one of three; columns of several starts of the walk over K, a last chunk of 256 that is not full
+@pytest.mark.parametrize("gated,weights_on", [(True, "output"), (True, "input"), (False, "output")])
+@pytest.mark.parametrize("E,top,W,ff", [(4, 1, 832, 704), (5, 3, 512, 1344)])
+def test_a_pairs_result_is_the_same_from_the_tiles_and_from_the_grouped_product(gated, weights_on, E, top, W, ff):
+    api = K()
+    most = api.moe_grouped_from_tokens(E, top, W, ff, torch.bfloat16, gated)
+    assert most > 3 and api.moe_grouped_rows(most, E, top, W, ff, torch.bfloat16, gated)
+    assert not api.moe_grouped_rows(most - 1, E, top, W, ff, torch.bfloat16, gated)
+    x = _rand(most, W, dtype=torch.bfloat16, seed=1)
+    up = _rand(E, (2 if gated else 1) * ff, W, dtype=torch.bfloat16, scale=2 * W ** -0.5, seed=2)
+    down = _rand(E, W, ff, dtype=torch.bfloat16, scale=ff ** -0.5, seed=3)
+    g = torch.Generator().manual_seed(4)
+    ids = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(most)]).int().to(DEV)
+    wts = torch.rand(most, top, generator=g).to(DEV)
+
+    def parts_of(N):
+        parts = torch.empty(top, N, W, device=DEV)
+        if gated:
+            api.moe_experts(x[:N], ids[:N], wts[:N], up, down, 7.0, 1.702, 1.0, E, parts, weights_on)
+        else:
+            api.moe_plain_experts(x[:N], ids[:N], wts[:N], up, down, "relu_squared", parts)
+        return parts
+    want = parts_of(most)
+    for N in (most - 1, 3):
+        assert torch.equal(parts_of(N), want[:, :N]), N
+
+
 # every tile behind the sort, with as many pairs of an expert as fill its groups of sixteen rows or are one more or one less:
 # tiles of 32 x 32 and 32 x 64, of 64 x 64, of 64 x 128, and of 128 x 256 for the first and for the second product; K that
 # ends within a chunk of 256 and within a step of 64; an expert without pairs
