@@ -79,18 +79,21 @@ __device__ __forceinline__ void store_finished(float* p, float v, int, const SkF
 // stretch of memory front to back, where the rows of the matrix as the file holds it lie K values apart.
 // PAIRS: the rounds written out in pairs (see the top of the file); else one after the other, with the next chunk's W copied
 // over this one's (rounds_alone says where).  The sums and their order are the same.
-// FIN: the values are finished on their way to C (SkFinish).
+// FIN: without GLU the values are finished on their way to C (SkFinish).  With it, for a weight whose K is split elsewhere (glu_whole),
+// the sums join a total after every sum_chunks chunks of SK_KC and begin again, so that they are no longer chains than the parts that
+// they stand in for: one chain over K is twice as far from 64 bits (9,600 x 2,048 4.1e-7 of the result, the parts and so 2.0e-7).
 template <int MT, bool GLU, typename TO, int KC, bool TILED, bool PAIRS, bool FIN>
 __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16_t* __restrict__ X,
                                                                     const uint16_t* __restrict__ W,
                                                                     TO* __restrict__ C, float* __restrict__ part,
                                                                     int M, int N, int K, int chunks_per_split,
-                                                                    SkFinish finish) {
+                                                                    int sum_chunks, SkFinish finish) {
   // chunks_per_split counts chunks of SK_KC; the kernel walks them in pieces of KC (the sums are the same in
   // the same order either way: a piece is a run of the chunk's matrix instructions)
   constexpr int XROW = KC + SK_XPAD;
   constexpr int NLD = KC / 32;                         // 16-byte loads of W per lane and piece
   constexpr int PER_CHUNK = SK_KC / KC;
+  constexpr bool SUMS = GLU && FIN;
   extern __shared__ __attribute__((aligned(16))) char skinny_lds[];
   uint16_t (*xs)[MT * 16][XROW] = reinterpret_cast<uint16_t (*)[MT * 16][XROW]>(skinny_lds);      // two stages
   // the second halves' sums meet the first halves' in the same memory, once the last stage has been read
@@ -111,9 +114,12 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16
   // TILED: this lane's row within the workgroup's tiles, which follow each other chunk by chunk
   const int chunks256 = (K + SK_KC - 1) / SK_KC;
   const uint16_t* wtile = W + ((size_t)blockIdx.x * chunks256 * SK_BN + (size_t)(wave * 16 + r)) * SK_KC;
-  f32x4 acc[MT];
+  f32x4 acc[MT], total[SUMS ? MT : 1];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) acc[mt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int mt = 0; mt < (SUMS ? MT : 1); ++mt) total[mt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  int until_total = sum_chunks;
 
   // the chunk of X is MT*16 rows of KC values = MT*2*KC/16 pieces of 16 bytes, spread over the 256 threads
   constexpr int XPIECES = MT * 16 * (KC / 8);
@@ -192,6 +198,20 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16
       }
     }
   };
+  // behind everything else that a round does, whose instructions a branch among them would keep from mixing
+  auto to_total = [&](int c) {
+    if constexpr (SUMS) {
+      if ((ce(c) + 1) % PER_CHUNK == 0 || ce(c) == nchunks - 1) --until_total;       // a chunk of SK_KC is done (K may end within one)
+      if (until_total == 0) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+          total[mt] += acc[mt];
+          acc[mt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        }
+        until_total = sum_chunks;
+      }
+    }
+  };
   uint4 w0[NLD], w1[NLD];
   // the products of chunk c with its W in `w`, while W of the next chunk comes into `next` and its X to the other stage
   auto round = [&](int c, uint4 (&w)[NLD], uint4 (&next)[NLD]) {
@@ -200,6 +220,7 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16
     __builtin_amdgcn_sched_barrier(0);                 // all of them in front of the first wait for this chunk's W
     products(c, w);
     store_x((c - c0 + 1) & 1, ce(c + 1));
+    to_total(c);
     __syncthreads();
   };
   if (!PAIRS && c0 < c1) {
@@ -219,6 +240,7 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16
 #pragma unroll
         for (int i = 0; i < NLD; ++i) w0[i] = w1[i];
       }
+      to_total(c);
       __syncthreads();
     }
   }
@@ -242,6 +264,10 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(const uint16
   if (GLU) __syncthreads();                            // the halves meet in the memory of the stages
   // lane holds D[i = 4 q + e][j = r]: i counts rows of W in the tile, j rows of X
   const int n = n_base + 4 * q;
+  if constexpr (SUMS) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[mt] = total[mt] + acc[mt];
+  }
   if (GLU) {
     if (half == 1) {
 #pragma unroll
@@ -425,16 +451,22 @@ static int skinny_splits(int N, int K) {
 
 // Whether both halves of [gate | up] take all of K in every workgroup, activation included, although K of a weight [N, K] is split:
 // a split product with this use has to be joined in a launch of its own, which is worth more than full compute units from some
-// 150 workgroups on (168 with longer K).  Both sides with cold weights, whole / in parts and the join, us at 1, 16, 64 and 128 rows:
-// 11,008 x 2,048 12.7 / 13.9, 13.6 / 15.2, 16.7 / 20.9, 23.7 / 27.7; 9,600 x 2,048 (150 workgroups) 12.8 / 13.5, 13.2 / 13.9, 16.5 / 18.8,
-// 23.8 / 25.5; 11,008 x 4,096 (172) 21.1 / 23.8, 22.9 / 25.1, 28.4 / 30.9, 39.8 / 41.7; 15,360 x 4,096 25.2 / 26.9, 25.3 / 29.1, 30.1 / 35.5,
-// 41.0 / 47.2.  Below: 10,240 x 4,096 (160) 21.2 / 21.0, 22.7 / 22.1, 28.0 / 28.0, 39.9 / 37.0; 7,168 x 2,048 (112) 12.2 / 9.0, 12.1 / 11.1.
+// 150 workgroups on, unless the parts fill two turns of the compute units and no more: 150 in three parts (K of 1,025 to 1,536), and, with
+// longer K, 160 and 170 in three and four.  From 171 on three parts of each spill into a third turn.  Both sides with cold weights, whole /
+// in parts and the join, us at 1, 16, 64 and 128 rows:
+//   9,600 x 512 (150 workgroups) 4.9 / 5.4, 4.7 / 6.8, 7.0 / 10.1, 11.4 / 15.2; x 1,024 7.2 / 8.2, 7.4 / 9.1, 10.6 / 14.2, 16.6 / 19.3;
+//   x 1,536 10.6 / 11.2, 9.8 / 10.5, 13.7 / 14.5, 20.8 / 19.4 (in parts: 72 and 96 rows lose too); x 2,048 11.3 / 13.1, 11.8 / 13.4, 16.6 / 18.8, 25.5 / 25.3;
+//   11,008 x 2,048 12.2 / 13.7, 12.0 / 15.2, 16.8 / 21.2, 25.3 / 27.6; x 4,096 21.0 / 24.3, 23.4 / 25.7, 30.9 / 32.3, 43.6 / 42.8;
+//   16,320 x 4,096 26.6 / 28.5, 26.4 / 30.7, 32.7 / 38.5, 47.4 / 52.6; 14,336 x 8,192 46.5 / 49.7, 45.5 / 51.6, 58.0 / 60.9, 83.7 / 81.5.
+// Below the line for longer K: 10,752 x 5,120 (168) 28.7 / 26.9, 32.1 / 28.5, 36.5 / 35.3, 51.4 / 47.2; x 14,336 68 / 65, 78 / 67, 97 / 83, 131 / 106.
+// What it costs at the line: 171 and 172 workgroups at 128 rows 1.02 to 1.05 of the time in parts (80 rows of 11,008 x 8,192 1.04).
 static bool glu_whole(int N, int K) {
-  const int nb = (N + SK_BN - 1) / SK_BN;
-  if (skinny_splits(N, K) == 1) return true;
+  const int nb = (N + SK_BN - 1) / SK_BN, splits = skinny_splits(N, K);
+  if (splits == 1) return true;
   for (int i = 0; i < g_known_count; ++i)
     if (g_known_splits[i].N == N && g_known_splits[i].K == K) return false;
-  return nb >= (K <= 2048 ? 150 : 168);
+  if (K > 2048) return nb >= 171;
+  return nb >= 150 && (K <= 1024 || nb * splits > 2 * SK_ENOUGH_BLOCKS);
 }
 
 // Says into how many parts (about: the chunks of K are dealt out evenly) the inner dimension of a weight [N, K] is
@@ -457,7 +489,7 @@ extern "C" int ia_gemm_skinny_splits(int N, int K) { return (N > 0 && K > 0) ? s
 
 template <int MT, bool GLU, typename TO, int KC, bool TILED, bool PAIRS, bool FIN>
 static int launch_skinny_one(dim3 grid, const uint16_t* x, const uint16_t* w, TO* c, float* part, int M, int N, int K,
-                             int cps, const SkFinish& finish, hipStream_t stream) {
+                             int cps, int sums, const SkFinish& finish, hipStream_t stream) {
   constexpr size_t lds = (size_t)2 * MT * 16 * (KC + SK_XPAD) * sizeof(uint16_t);
   static bool allowed = false;      // more than 64 KB of LDS has to be asked for, once per kernel
   if (lds > 65536 && !allowed) {
@@ -466,7 +498,7 @@ static int launch_skinny_one(dim3 grid, const uint16_t* x, const uint16_t* w, TO
     if (e != hipSuccess) return (int)e;
     allowed = true;
   }
-  gemm_skinny_kernel<MT, GLU, TO, KC, TILED, PAIRS, FIN><<<grid, SK_WAVES * 64, lds, stream>>>(x, w, c, part, M, N, K, cps, finish);
+  gemm_skinny_kernel<MT, GLU, TO, KC, TILED, PAIRS, FIN><<<grid, SK_WAVES * 64, lds, stream>>>(x, w, c, part, M, N, K, cps, sums, finish);
   IA_LAUNCH_CHECK();
   return IA_OK;
 }
@@ -501,6 +533,7 @@ static int launch_skinny(const uint16_t* x, const uint16_t* w, TO* c, float* par
                          hipStream_t stream, const SkFinish& finish = SkFinish{nullptr, 0, 1.0f, 0.0f}) {
   const int nchunks = (K + SK_KC - 1) / SK_KC;
   const int cps = (nchunks + splits - 1) / splits;
+  const int sum_parts = GLU && FIN ? skinny_splits(N, K) : 1, sums = (nchunks + sum_parts - 1) / sum_parts;
   const int NO = GLU ? N / 2 : N;
   const int cols = GLU ? SK_BN / 2 : SK_BN;           // columns of the result per workgroup
   dim3 grid((NO + cols - 1) / cols, splits);
@@ -519,30 +552,30 @@ static int launch_skinny(const uint16_t* x, const uint16_t* w, TO* c, float* par
   const bool alone = rounds_alone((M + 15) / 16, TILED, K, groups, grid.y, cps);
   switch ((M + 15) / 16) {
     case 1:
-      if (shorter) return launch_skinny_one<1, GLU, TO, SK_KC / 2, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
-      return launch_skinny_one<1, GLU, TO, SK_KC, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
+      if (shorter) return launch_skinny_one<1, GLU, TO, SK_KC / 2, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, sums, finish, stream);
+      return launch_skinny_one<1, GLU, TO, SK_KC, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, sums, finish, stream);
     case 2:
-      if (shorter) return launch_skinny_one<2, GLU, TO, SK_KC / 2, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
-      return launch_skinny_one<2, GLU, TO, SK_KC, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
+      if (shorter) return launch_skinny_one<2, GLU, TO, SK_KC / 2, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, sums, finish, stream);
+      return launch_skinny_one<2, GLU, TO, SK_KC, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, sums, finish, stream);
     case 3:
-      if (alone) return launch_skinny_one<3, GLU, TO, SK_KC, TILED, false, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
-      return launch_skinny_one<3, GLU, TO, SK_KC, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
+      if (alone) return launch_skinny_one<3, GLU, TO, SK_KC, TILED, false, FIN>(grid, x, w, c, part, M, N, K, cps, sums, finish, stream);
+      return launch_skinny_one<3, GLU, TO, SK_KC, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, sums, finish, stream);
     case 4:
-      if (alone) return launch_skinny_one<4, GLU, TO, SK_KC, TILED, false, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
-      return launch_skinny_one<4, GLU, TO, SK_KC, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
+      if (alone) return launch_skinny_one<4, GLU, TO, SK_KC, TILED, false, FIN>(grid, x, w, c, part, M, N, K, cps, sums, finish, stream);
+      return launch_skinny_one<4, GLU, TO, SK_KC, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, sums, finish, stream);
     // above 64 rows: pieces of 128, so that the two stages of X of two workgroups fit a compute unit's LDS
     case 5:
-      if (alone) return launch_skinny_one<5, GLU, TO, SK_KC / 2, TILED, false, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
-      return launch_skinny_one<5, GLU, TO, SK_KC / 2, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
+      if (alone) return launch_skinny_one<5, GLU, TO, SK_KC / 2, TILED, false, FIN>(grid, x, w, c, part, M, N, K, cps, sums, finish, stream);
+      return launch_skinny_one<5, GLU, TO, SK_KC / 2, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, sums, finish, stream);
     case 6:
-      if (alone) return launch_skinny_one<6, GLU, TO, SK_KC / 2, TILED, false, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
-      return launch_skinny_one<6, GLU, TO, SK_KC / 2, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
+      if (alone) return launch_skinny_one<6, GLU, TO, SK_KC / 2, TILED, false, FIN>(grid, x, w, c, part, M, N, K, cps, sums, finish, stream);
+      return launch_skinny_one<6, GLU, TO, SK_KC / 2, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, sums, finish, stream);
     case 7:
-      if (alone) return launch_skinny_one<7, GLU, TO, SK_KC / 2, TILED, false, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
-      return launch_skinny_one<7, GLU, TO, SK_KC / 2, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
+      if (alone) return launch_skinny_one<7, GLU, TO, SK_KC / 2, TILED, false, FIN>(grid, x, w, c, part, M, N, K, cps, sums, finish, stream);
+      return launch_skinny_one<7, GLU, TO, SK_KC / 2, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, sums, finish, stream);
     case 8:
-      if (alone) return launch_skinny_one<8, GLU, TO, SK_KC / 2, TILED, false, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
-      return launch_skinny_one<8, GLU, TO, SK_KC / 2, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, finish, stream);
+      if (alone) return launch_skinny_one<8, GLU, TO, SK_KC / 2, TILED, false, FIN>(grid, x, w, c, part, M, N, K, cps, sums, finish, stream);
+      return launch_skinny_one<8, GLU, TO, SK_KC / 2, TILED, true, FIN>(grid, x, w, c, part, M, N, K, cps, sums, finish, stream);
     default: return IA_ERR_UNSUPPORTED;
   }
 }
@@ -583,6 +616,10 @@ static int skinny_product(const void* X, const void* W, void* C, int out_dtype, 
   if (splits > 1 && (!workspace || workspace_floats < (size_t)splits * M * N)) return IA_ERR_BAD_ARG;
   if (epilogue == SK_EPI_SWIGLU && C != nullptr && glu_whole(N, K)) {
     // one pass: both halves of W in the same wave, the activation in the epilogue
+    if (splits > 1) {                                  // the sums in as many pieces as K has parts
+      if (out_dtype == IA_F32) return launch_skinny<true, float, TILED, true>(x, w, (float*)C, nullptr, M, N, K, 1, stream);
+      return launch_skinny<true, uint16_t, TILED, true>(x, w, (uint16_t*)C, nullptr, M, N, K, 1, stream);
+    }
     if (out_dtype == IA_F32) return launch_skinny<true, float, TILED>(x, w, (float*)C, nullptr, M, N, K, 1, stream);
     return launch_skinny<true, uint16_t, TILED>(x, w, (uint16_t*)C, nullptr, M, N, K, 1, stream);
   }

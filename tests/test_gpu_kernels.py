@@ -560,10 +560,10 @@ def test_gemm_skinny_finished_leaves_the_bits_of_separate_launches(M, N, K_):
         api.gemm_skinny_finished(a, w, torch.empty(M, N, dtype=torch.bfloat16, device=DEV), scale=2.0)
 
 
-# both halves whole in a workgroup although the weight is split (glu_whole): the smallest and largest of either range of K, columns
-# that fill no group of 16, a last chunk that is not full; the copy leaves the same bits, and a row those it has alone
+# both halves whole in a workgroup although the weight is split (glu_whole): the smallest and largest of either range of K and the
+# largest below it, columns that fill no group of 16, a last chunk that is not full; the copy leaves the same bits, and a row those it has alone
 @pytest.mark.parametrize("M", [1, 16, 33, 128])
-@pytest.mark.parametrize("N,K_", [(9538, 2048), (9602, 520), (16320, 776), (10690, 2056), (16318, 4096)])
+@pytest.mark.parametrize("N,K_", [(9538, 2048), (9602, 520), (16320, 776), (10690, 2056), (10882, 2056), (16318, 4096)])
 def test_gemm_skinny_glu_whole_where_the_weight_is_split(M, N, K_):
     api = K()
     assert api.gemm_skinny_splits(N, K_) > 1
@@ -578,6 +578,26 @@ def test_gemm_skinny_glu_whole_where_the_weight_is_split(M, N, K_):
     assert torch.equal(api.gemm_skinny(a, w, epilogue="swiglu", out_dtype=torch.float32, tiled=api.tile_weight(w, "swiglu")), got)
     assert torch.equal(api.gemm_skinny(a[M - 1:], w, epilogue="swiglu", out_dtype=torch.float32)[0], got[M - 1])
     assert torch.equal(api.gemm_skinny(a, w, epilogue="swiglu"), got.bfloat16())
+
+
+# ... and their sums are chains no longer than a part's: as near to 64 bits as the parts added in the order of their index.  The
+# activation in fp32 adds its own roundings (a few 2^-24)
+@pytest.mark.parametrize("M", [1, 33, 128])
+@pytest.mark.parametrize("N,K_", [(9602, 2048), (11008, 4096), (13824, 5120)])
+def test_gemm_skinny_glu_whole_is_as_near_to_64_bits_as_the_parts_joined(M, N, K_):
+    api = K()
+    a, w = _rand(M, K_, dtype=torch.bfloat16, seed=33), _rand(N, K_, dtype=torch.bfloat16, scale=K_ ** -0.5, seed=34)
+
+    def activated(y):
+        return y[:, :N // 2] / (1 + torch.exp(-y[:, :N // 2])) * y[:, N // 2:]
+    kept = api.gemm_skinny(a, w, keep_split=True)
+    total = kept.parts[0].clone()
+    for part in kept.parts[1:]:
+        total += part
+    want = activated(a.double() @ w.double().t())
+    joined = float((activated(total.double()) - want).norm() / want.norm())
+    whole = float((api.gemm_skinny(a, w, epilogue="swiglu", out_dtype=torch.float32).double() - want).norm() / want.norm())
+    assert whole <= ((1.1 * joined) ** 2 + (2 * 2.0 ** -24) ** 2) ** 0.5
 
 
 # one workgroup with all of K against the parts and their sum in the order of their index: columns that fill no group of
