@@ -381,10 +381,16 @@ def moe_route(logits, bias: Optional[torch.Tensor], top: int, experts: int, soft
 
 
 # From how many rows an expert on average the grouped form is ahead of the tiles behind the sort: sort to scatter, microseconds of
-# grouped / tiles with cold weights.  Gated: 32 experts of 1,408 x 2,048 at 48 / 96 / 128 rows 182 / 137, 201 / 178, 255 / 257; of
-# 2,432 x 4,096 445 / 398, 499 / 482, 625 / 631; 16 of 2,432 x 4,096 268 / 225, 291 / 288, 313 / 345.  Without a gate: 8 of
-# 4,800 x 4,096 at 48 / 56 / 64 rows 186 / 161, 189 / 167, 193 / 216.
+# grouped / tiles with cold weights.  Gated: 32 experts of 1,408 x 2,048 at 64 / 112 / 128 rows 171 / 172, 192 / 191, 245 / 278; 64 of them
+# 314 / 306, 391 / 372, 458 / 452; 8 of 2,752 x 2,048 106 / 99, 116 / 103, 160 / 169; 4 of 4,800 x 4,096 162 / 162, 178 / 164, 182 / 205.
+# Without a gate: 8 of 4,800 x 4,096 at 48 / 56 / 64 rows 172 / 163, 175 / 169, 178 / 218.
+# The passes around the grouped products (rows in the order of the sort, activation, scatter) take rows times (W + ff), the products rows
+# times W ff; where those weigh little and the tiles of 128 x 256 that the experts then have fill the chip, gated ones change over sooner: at
+# 48 / 56 / 64 / 112 rows 20 of 2,432 x 4,096 298 / 272, 315 / 334, 313 / 342, 343 / 393; 8 of 4,800 x 4,096 255 / 211, 258 / 264, 263 / 304,
+# 289 / 320; 8 of 14,336 x 4,096 603 / 552, 616 / 628, 626 / 729, 688 / 726; 8 of 8,192 x 5,120 413 / 446, 418 / 475, 428 / 468, 466 / 515.
+# Either way a pair's result has the same bits.
 MOE_GROUPED_ROWS_AN_EXPERT = 112
+MOE_GROUPED_ROWS_A_WIDE_EXPERT = 56
 MOE_GROUPED_ROWS_A_PLAIN_EXPERT = 56
 
 
@@ -394,7 +400,9 @@ def moe_grouped_from_tokens(E: int, top: int, W: int, ff: int, dtype: torch.dtyp
     inner dimensions W and ff must be multiples of 64)."""
     if dtype != torch.bfloat16 or W % 64 or ff % 64:
         return 0
-    return -(-(MOE_GROUPED_ROWS_AN_EXPERT if gated else MOE_GROUPED_ROWS_A_PLAIN_EXPERT) * E // top)
+    wide = W * ff >= 1500 * (W + ff) and E * -(-2 * ff // 256) >= 224
+    rows = (MOE_GROUPED_ROWS_A_WIDE_EXPERT if wide else MOE_GROUPED_ROWS_AN_EXPERT) if gated else MOE_GROUPED_ROWS_A_PLAIN_EXPERT
+    return -(-rows * E // top)
 
 
 def moe_grouped_rows(N: int, E: int, top: int, W: int, ff: int, dtype: torch.dtype, gated: bool = True) -> bool:
