@@ -223,7 +223,9 @@ extern "C" int ia_embed_norm(const void* table, int table_dtype, const int* ids,
 // (piece c of this thread is the piece of thread threadIdx.x + 256 c there: 16 sums over 64 lanes, added in the
 // order of their index), so that a row's result has the same bits from either; with many rows 256 threads
 // per row keep more rows on a compute unit and are a sixth faster.
-template <typename TD, typename TO, int NT, bool AS_WIDE = false, int MAXV = RN_MAXV, bool TOGETHER = false>
+// SIDE: a second norm of the same rows (w2, out2).  A form of its own, as its condition and its registers cost the others: 4,096 rows of
+// 256 / 512 / 1,024 values 5.1 / 6.5 / 8.2 us without it in the kernel, 6.3 / 7.6 / 8.5 with it there and not asked for.
+template <bool SIDE, typename TD, typename TO, int NT, bool AS_WIDE = false, int MAXV = RN_MAXV, bool TOGETHER = false>
 __global__ __launch_bounds__(NT) void add_rmsnorm_vec_kernel(float* __restrict__ h, const TD* __restrict__ delta,
                                                              int splits, size_t split_stride,
                                                              const void* __restrict__ w, int w_dtype,
@@ -246,7 +248,7 @@ __global__ __launch_bounds__(NT) void add_rmsnorm_vec_kernel(float* __restrict__
     if (((int)__builtin_amdgcn_readfirstlane(threadIdx.x) & ~63) * 4 < H) {
       v[0] = load4(hr + il);
       const Raw4 graw = load_raw4(w, w_dtype, il);
-      if (w2) g2raw = load_raw4(w2, w2_dtype, il);
+      if (SIDE) g2raw = load_raw4(w2, w2_dtype, il);
       if (dr) {
         const float4 d = load_parts4(dr + il, splits, split_stride);
         v[0].x += d.x; v[0].y += d.y; v[0].z += d.z; v[0].w += d.w;
@@ -322,7 +324,7 @@ __global__ __launch_bounds__(NT) void add_rmsnorm_vec_kernel(float* __restrict__
     if (i < H)
       store4(o + i, make_float4(v[c].x * inv * g[c].x, v[c].y * inv * g[c].y, v[c].z * inv * g[c].z,
                                 v[c].w * inv * g[c].w));
-    if (i < H && out2) {
+    if (SIDE && i < H) {
       const float4 k = TOGETHER ? raw4_values(g2raw, w2_dtype) : load4_any(w2, w2_dtype, i);
       store4(out2 + (size_t)row * H + i, make_float4(v[c].x * inv * k.x, v[c].y * inv * k.y, v[c].z * inv * k.z,
                                                      v[c].w * inv * k.w));
@@ -330,37 +332,45 @@ __global__ __launch_bounds__(NT) void add_rmsnorm_vec_kernel(float* __restrict__
   }
 }
 
-template <typename TD, typename TO>
-static int launch_add_rmsnorm(float* h, const void* delta, int splits, size_t split_stride, const void* w, int w_dtype,
-                              void* out, const void* w2, int w2_dtype, void* out2, const int* rows, int N, int H,
-                              float eps, hipStream_t stream) {
+template <bool SIDE, typename TD, typename TO>
+static int launch_add_rmsnorm_as(float* h, const void* delta, int splits, size_t split_stride, const void* w, int w_dtype,
+                                 void* out, const void* w2, int w2_dtype, void* out2, const int* rows, int N, int H,
+                                 float eps, hipStream_t stream) {
   const TD* d = (const TD*)delta;
   TO *o = (TO*)out, *o2 = (TO*)out2;
   if ((H & 3) == 0 && H <= 1024 * 4 * RN_MAXV) {
     // wide rows: 1024 threads, one to four 16-byte pieces each; with many rows of up to 4096 values, 256 threads
     // that take the sums in the same order.  A row's sums are taken in the same order whatever the batch holds.
     if (H >= 2048 && H <= 4096 && N >= 1024)   // measured: from about 1,000 rows on the narrow workgroups win
-      add_rmsnorm_vec_kernel<TD, TO, 256, true><<<N, 256, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows, H, eps);
+      add_rmsnorm_vec_kernel<SIDE, TD, TO, 256, true><<<N, 256, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows, H, eps);
     else if (H >= 2048 && H <= 4096 && rows_are_few(N, 1024))
       // one piece a thread: few registers, so the loads of up to sixteen partial sums are in flight together
       // (the sums are the same: the pieces beyond the first are empty at this width)
-      add_rmsnorm_vec_kernel<TD, TO, 1024, false, 1, true><<<N, 1024, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows, H, eps);
+      add_rmsnorm_vec_kernel<SIDE, TD, TO, 1024, false, 1, true><<<N, 1024, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows, H, eps);
     else if (H >= 2048 && H <= 4096)
-      add_rmsnorm_vec_kernel<TD, TO, 1024, false, 1><<<N, 1024, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows, H, eps);
+      add_rmsnorm_vec_kernel<SIDE, TD, TO, 1024, false, 1><<<N, 1024, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows, H, eps);
     else if (H >= 2048)
-      add_rmsnorm_vec_kernel<TD, TO, 1024><<<N, 1024, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows,
+      add_rmsnorm_vec_kernel<SIDE, TD, TO, 1024><<<N, 1024, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows,
                                                                     H, eps);
     else if (H <= 1024)        // one piece a thread, and few threads a row: together whatever the rows (0.6 to 0.95 of the
                                // time with four pieces at 1 to 4,096 rows of 512 and 1,024)
-      add_rmsnorm_vec_kernel<TD, TO, 256, false, 1, true><<<N, 256, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows, H, eps);
+      add_rmsnorm_vec_kernel<SIDE, TD, TO, 256, false, 1, true><<<N, 256, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows, H, eps);
     else
-      add_rmsnorm_vec_kernel<TD, TO, 256><<<N, 256, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows, H,
+      add_rmsnorm_vec_kernel<SIDE, TD, TO, 256><<<N, 256, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows, H,
                                                                   eps);
   } else {
     add_rmsnorm_kernel<TD, TO><<<N, 256, 0, stream>>>(h, d, splits, split_stride, w, w_dtype, o, w2, w2_dtype, o2, rows, H, eps);
   }
   IA_LAUNCH_CHECK();
   return IA_OK;
+}
+
+template <typename TD, typename TO>
+static int launch_add_rmsnorm(float* h, const void* delta, int splits, size_t split_stride, const void* w, int w_dtype,
+                              void* out, const void* w2, int w2_dtype, void* out2, const int* rows, int N, int H,
+                              float eps, hipStream_t stream) {
+  return w2 ? launch_add_rmsnorm_as<true, TD, TO>(h, delta, splits, split_stride, w, w_dtype, out, w2, w2_dtype, out2, rows, N, H, eps, stream)
+            : launch_add_rmsnorm_as<false, TD, TO>(h, delta, splits, split_stride, w, w_dtype, out, w2, w2_dtype, out2, rows, N, H, eps, stream);
 }
 
 // delta_dtype: dtype of delta (IA_F32 for a stack of partial sums in the bf16 path); act_dtype: dtype of out.
