@@ -39,7 +39,11 @@ __device__ __forceinline__ void router_finish(int mine_e, float mine_w, int top,
 // Up to 64 experts, one a lane: the place of this lane's expert among all, largest first and the lowest index among equals (64 for
 // an expert that cannot be chosen).  Every lane compares with every expert, whose values come as scalars: no step waits
 // for the one before, where `top` rounds of a maximum over the wave are chains of twelve exchanges each (1 / 64 tokens to 4 of 32 with
-// join and sort 7.3 / 8.5 us in rounds, 6.2 / 7.3 so; to 8 of 64 10.5 / 12.0 and 9.0 / 9.8).
+// join and sort 7.3 / 8.5 us in rounds, 6.2 / 7.3 so; to 8 of 64 10.5 / 12.0 and 9.0 / 9.8).  The comparisons grow with the experts and
+// the rounds with the choices, so few choices of many experts stay with the rounds (1 / 512 / 8,192 tokens to 1 of 64 2.3 / 2.8 / 3.9 us in
+// rounds and 4.1 / 4.6 / 9.2 by rank, to 2 of 32 2.9 / 3.4 / 5.5 and 3.0 / 3.5 / 5.9, to 4 of 64 4.2 / 4.5 / 8.6 and 4.2 / 4.6 / 9.2, to 4 of 32
+// 4.2 / 4.5 / 8.3 and 3.0 / 3.5 / 6.1).
+__device__ __forceinline__ bool choose_by_rank(int E, int top) { return 12 * top >= E; }
 __device__ __forceinline__ int expert_rank(float x, bool can, int E, int lane) {
   const int b = __float_as_int(x + 0.0f);                  // -0 counts as 0
   const int key = can ? b ^ ((b >> 31) & 0x7fffffff) : (int)0x80000000;      // in the order of the values
@@ -61,7 +65,7 @@ __device__ __forceinline__ float value_of_rank(float v, int rank, int k) {
 // biases; leaves the token's choices and weights at ids and weights, and with one expert a lane its place among them in mine_rank.
 template <int PL>
 __device__ __forceinline__ void choose_then_softmax(const float (&v)[PL], int E, int top, int lane, int* ids, float* weights, int& mine_rank) {
-  if constexpr (PL == 1) {
+  if (PL == 1 && choose_by_rank(E, top)) {
     // a value that compares with nothing (NaN) counts as the smallest
     const float x = (v[0] == v[0]) ? v[0] : -INFINITY;
     const int rank = expert_rank(x, lane < E, E, lane);
@@ -75,6 +79,7 @@ __device__ __forceinline__ void choose_then_softmax(const float (&v)[PL], int E,
     mine_rank = rank;
     return;
   }
+  mine_rank = 64;
   unsigned taken = 0u;
 #pragma unroll
   for (int c = 0; c < PL; ++c)
@@ -100,7 +105,10 @@ __device__ __forceinline__ void choose_then_softmax(const float (&v)[PL], int E,
         best_e = oe;
       }
     }
-    if ((best_e & 63) == lane) taken |= 1u << (best_e >> 6);
+    if ((best_e & 63) == lane) {
+      taken |= 1u << (best_e >> 6);
+      if (PL == 1) mine_rank = k;
+    }
     if (k == 0) first_v = best_v;
     const float w = expf(best_v - first_v);
     sum += w;
@@ -741,7 +749,7 @@ __device__ __forceinline__ void softmax_then_choose(const float (&zv)[PL], const
       if (better >= keep) taken |= 1u << c;
     }
   }
-  if constexpr (PL == 1) {
+  if (PL == 1 && choose_by_rank(E, top)) {
     const int rank = expert_rank((v[0] == v[0]) ? v[0] : -INFINITY, !(taken & 1u), E, lane);
     float chosen = 0.f;
     for (int k = 0; k < top; ++k) chosen += value_of_rank(s[0], rank, k);
@@ -752,6 +760,7 @@ __device__ __forceinline__ void softmax_then_choose(const float (&zv)[PL], const
     mine_rank = rank;
     return;
   }
+  mine_rank = 64;
   float sum = 0.f, mine_w = 0.f;
   int mine_e = 0;
   for (int k = 0; k < top; ++k) {
@@ -773,7 +782,10 @@ __device__ __forceinline__ void softmax_then_choose(const float (&zv)[PL], const
         best_s = os;
       }
     }
-    if ((best_e & 63) == lane) taken |= 1u << (best_e >> 6);
+    if ((best_e & 63) == lane) {
+      taken |= 1u << (best_e >> 6);
+      if (PL == 1) mine_rank = k;
+    }
     sum += best_s;
     router_keep(mine_e, mine_w, k, lane, best_e, best_s, ids, weights);
   }

@@ -1813,6 +1813,72 @@ def test_routed_experts_tile_by_tile(gated, counts, W, ff):
             assert torch.equal(parts_of([n])[0], got[n]), (e, n)          # alone: tiles of 32 x 32
 
 
+# ---------------------------------------------------------------- the router
+# what a router chooses and how much, from the definition: NaN counts as the smallest, the lowest index among equals (+0 and -0 are), the
+# groups with the largest members first.  Few choices of many experts (rounds of a maximum) and the others (by rank), one expert a lane;
+# rows of equal logits, of both zeros, with infinities and NaN, of nothing else
+def _router_choice(z, add, top, softmax, groups=1, keep=1, renorm=True, sigmoid=False):
+    z, add = z.float().cpu(), None if add is None else add.float().cpu()
+    if not softmax:
+        v = z if add is None else z + add
+    else:
+        zmax = torch.where(z.isnan(), torch.tensor(-math.inf), z).max(1, keepdim=True).values
+        e = torch.exp(z.double() - zmax.double())
+        s = 1 / (1 + torch.exp(-z.double())) if sigmoid else e / e.sum(1, keepdim=True)
+        v = (z.double() if sigmoid else s) if add is None else s + add.double()
+    v = torch.where(v.isnan(), torch.tensor(-math.inf, dtype=v.dtype), v)
+    free = torch.ones_like(v, dtype=torch.bool)
+    if groups > 1:
+        best = v.view(len(v), groups, -1).max(2).values
+        kept = best.sort(dim=1, descending=True, stable=True).indices[:, :keep]
+        free = torch.zeros_like(best, dtype=torch.bool).scatter(1, kept, True).repeat_interleave(z.shape[1] // groups, 1)
+    order = torch.where(free, v, torch.tensor(-math.inf, dtype=v.dtype)).sort(dim=1, descending=True, stable=True).indices
+    # among values of minus infinity those that can be chosen come first
+    order = torch.stack([torch.tensor([i for i in row.tolist() if f[i]] + [i for i in row.tolist() if not f[i]]) for row, f in zip(order, free)])
+    ids = order[:, :top]
+    if not softmax:
+        x = v.double().gather(1, ids)
+        w = torch.exp(x - x[:, :1])
+        return ids, w / w.sum(1, keepdim=True)
+    w = s.gather(1, ids)
+    return ids, w / (w.sum(1, keepdim=True) + 1e-20) if renorm else w
+
+
+@pytest.mark.parametrize("kind", ["top", "softmax", "groups", "sigmoid"])
+@pytest.mark.parametrize("E,top", [(1, 1), (4, 4), (12, 1), (16, 1), (16, 2), (24, 2), (32, 2), (32, 4), (60, 4), (60, 5), (64, 1), (64, 5), (64, 6), (64, 16)])
+def test_a_router_chooses_as_it_is_defined(kind, E, top):
+    api = K()
+    g = torch.Generator().manual_seed(E + top)
+    # quarters and eighths: sums are exact, equal ones are equal, and the others lie further apart than roundings reach
+    z = torch.randint(-12, 13, (40, E), generator=g).float() / 4
+    z[1] = 0.75
+    z[2] = torch.where(torch.arange(E) % 2 == 0, 0.0, -0.0)
+    z[3] = -math.inf
+    z[4] = math.nan
+    z[5, E // 2] = math.inf
+    z[6, E - 1], z[6, 0] = math.inf, math.inf
+    z[7, ::2] = -math.inf
+    z[8, E // 3] = math.nan
+    z[9] = torch.where(torch.arange(E) % 3 == 0, math.nan, -math.inf)
+    add = (torch.randint(-8, 9, (E,), generator=g).float() / 8) if kind != "softmax" else None
+    zd, ad = z.to(DEV), None if add is None else add.to(DEV)
+    if kind == "top":
+        want = _router_choice(z, add, top, False)
+        got = api.router_topk(zd, ad, top)
+        routed = api.moe_route(zd, ad, top, E)
+    else:
+        kw = dict(groups=4, keep=-(-4 * top // E)) if kind == "groups" and E % 4 == 0 else \
+            dict(renorm=kind == "softmax", sigmoid=kind == "sigmoid")
+        want = _router_choice(z, add, top, True, **kw)
+        got = api.router_softmax_topk(zd, ad, top, **kw)
+        routed = api.moe_route(zd, ad, top, E, True, **kw)
+    few = api.moe_route(api.SplitSum(torch.stack([zd[:16], torch.zeros_like(zd[:16])])), ad, top, E, kind != "top", **({} if kind == "top" else kw))
+    assert torch.equal(got[0].cpu().long(), want[0])
+    assert torch.allclose(got[1].cpu().double(), want[1], rtol=2e-6, atol=1e-30, equal_nan=True)      # a few fp32 roundings
+    for r, n in ((routed, 40), (few, 16)):
+        assert torch.equal(r[0], got[0][:n]) and torch.equal(r[1].nan_to_num(-1.0), got[1][:n].nan_to_num(-1.0))
+
+
 # ---------------------------------------------------------------- the router and the sort of few tokens in one launch
 # one token, a token more than the waves, the most; one expert, 64; parts that are no multiple of the loads asked for together; the
 # column behind the experts' logits; groups; ties, infinities and NaN among the logits
