@@ -137,7 +137,10 @@ __device__ __forceinline__ void store_four(float* __restrict__ C, int m, int n, 
 // leaves the other under way.  The stretches' sums meet in LDS, where they are added in the order of k.
 // Cold weights, us: 128,256 x 2,048 at 1 / 4 / 12 rows 178 / 195 / 229 (1.05 GB: 5.9 to 4.6 TB/s); 16,384 x 2,048 27.5 / 29.3 / 33.1;
 // 2,048 x 8,192 24.1 / 26.8 / 34.3; 28,672 x 4,096 87.9 / 93.7 / 108; shapes of more rows beside the rule below.
-template <int MT, int RT, int WAVES, int PIECE>
+// SHORT: a wave is done where K ends within its stretch.  The branches cost what they leave out where stretches are full (16,384 x
+// 1,024 at 8 rows 19.8 us without and 21.1 with them), so only K of few stretches takes it: 2,048 x 64 / 300 / 516 / 900 at 8 rows 4.9 / 5.4 / 5.5 /
+// 5.6 without and 2.6 / 4.8 / 5.0 / 5.1 with them.
+template <int MT, int RT, int WAVES, int PIECE, bool SHORT>
 __global__ __launch_bounds__(WAVES * 64) void gemm_f32_stream_kernel(const float* __restrict__ A,
                                                                      const float* __restrict__ W,
                                                                      float* __restrict__ C, int M, int N, int K,
@@ -207,7 +210,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_stream_kernel(const float
       for (int t = 0; t < TILES; ++t) mid[t] = gf32x4{0.f, 0.f, 0.f, 0.f};
       const int next = s + WAVES < stretches ? k0 + WAVES * 256 : k0;  // behind the wave's last stretch anything that can be read
 #pragma clang loop unroll_count(ROUNDS)
-      for (int c = 0; c < 16; c += 2 * PIECE) {
+      for (int c = 0; c < 16 && (!SHORT || k0 + 16 * c < K); c += 2 * PIECE) {
         load(k0 + 16 * (c + PIECE), w1, x1);
         __builtin_amdgcn_sched_barrier(0);                             // all of them in front of the first wait
         work(k0 + 16 * c, w0, x0);
@@ -318,10 +321,10 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
       store_four(C, m0 + 16 * (wm + i) + r, n0 + 16 * (wn + j) + 4 * q, M, N, ldc, wide, acc[i][j] + mid[i][j]);
 }
 
-template <int MT, int RT, int WAVES, int PIECE>
+template <int MT, int RT, int WAVES, int PIECE, bool SHORT = false>
 static void launch_f32_stream(const float* A, const float* W, float* C, int M, int N, int K, int lda, int ldw, int ldc,
                               bool wide, hipStream_t stream) {
-  gemm_f32_stream_kernel<MT, RT, WAVES, PIECE><<<dim3((N + 16 * RT - 1) / (16 * RT), (M + 16 * MT - 1) / (16 * MT)), WAVES * 64,
+  gemm_f32_stream_kernel<MT, RT, WAVES, PIECE, SHORT><<<dim3((N + 16 * RT - 1) / (16 * RT), (M + 16 * MT - 1) / (16 * MT)), WAVES * 64,
                                                  0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc, wide);
 }
 
@@ -346,8 +349,9 @@ static bool gemm_f32(const float* A, const float* W, float* C, int M, int N, int
   // the vector kernel 4.7 / 7.0 / 10.9, at 20 rows 17 / 17 / 18 and 5.2 / 7.8 / 12.5; 1,000 x 16 / 32 at 20 rows 6.9 and 5.0 / 7.5)
   if (M <= GS_MOST_ROWS && (K <= 16 || (N > 4096 && K <= (M > 16 ? 96 : 48)))) return false;
   const bool wide = ((uintptr_t)C & 15) == 0 && (ldc & 3) == 0;
-  // Up to 16 rows: 16 rows of W a workgroup, of 16 waves where those are at most one a compute unit and each wave has a stretch
-  // (4,096 x 4,096 at 1 row 15.7 us, with four waves 19.6; 6,144 x 4,096 26.5 and 25.2), of eight where each has two (28,672 x 4,096
+  // Up to 16 rows: 16 rows of W a workgroup, of 16 waves where those are at most one a compute unit and there are more stretches
+  // than four waves take at once, although some waves have none until K is 3,841 (4,096 x 4,096 at 1 row 15.7 us, with four waves
+  // 21.6; x 1,028 / 2,048 8.4 / 10.0 and 10.4 / 12.6; with eight, where four of sixteen or fewer have one, the same; 6,144 x 4,096, more than one a unit, 26.5 and 25.2), of eight where each has two (28,672 x 4,096
   // at 1 / 4 rows 87.9 / 93.7, with four 94.7 / 98.4; with one each 16,384 x 2,048 29.7, with four 27.5), of four otherwise; from nine
   // rows on, whose reads then weigh as much as W's, 64 rows of W share them (16 rows x 128,256 x 2,048 249 us, with 16 rows
   // of W 295; 8,192 x 2,048, which that leaves 128 workgroups, 28.6 and 20.2).
@@ -355,6 +359,7 @@ static bool gemm_f32(const float* A, const float* W, float* C, int M, int N, int
   if (M <= 16 && near) {
     if (N <= 16 * GS_UNITS && K > 1024) launch_f32_stream<1, 1, 16, 2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
     else if (M > 8 && N >= 64 * GS_UNITS) launch_f32_stream<1, 4, 4, 2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
+    else if (K < 1024 && K % 256 != 0) launch_f32_stream<1, 1, 4, 2, true>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
     else if (M <= 8 && K >= 4096) launch_f32_stream<1, 1, 8, 2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
     else launch_f32_stream<1, 1, 4, 2>(A, W, C, M, N, K, lda, ldw, ldc, wide, stream);
     return true;
@@ -367,6 +372,10 @@ static bool gemm_f32(const float* A, const float* W, float* C, int M, int N, int
   // 680, 64 x 64 190, 32 x 32 62 and 166 at the least.  Cold weights, us with 32 x 16, 32 x 32 and 48 x 32 alone and now: 16,384 x 2,048 at 40 / 96 /
   // 142 rows 61.8 / 110 / 157 and 45.1 / 85.4 / 126, 6,144 x 4,096 at 64 / 96 / 142 76.8 / 116 / 155 and 57.4 / 59.2 / 107, 4,096 x 14,336 at
   // 142 / 220 372 / 452 and 264 / 349, 2,048 x 8,192 at 24 / 142 / 300 48.3 / 107 / 219 and 35.2 / 84.0 / 154, 128,256 x 2,048 at 142 1,373 and 1,012.
+  // Those turns are of 32 stretches, eight on each of a unit's four matrix units.  Against the tiles several turns cost as many stretches as
+  // the fullest one has: K of 1,280 is two stretches for one of them and one for the others (300 x 4,096 x 1,280 72.6 us, in tiles 54.8; 142 x
+  // 16,384 x 1,280 118 and 93.9; x 3,072, three on each, 221 and 238).  A single turn is mostly the way there and back and stays as it is (96 x
+  // 6,144 x 1,280 29.2 us, in tiles 37.9; 33 x 1,000 x 1,280 7.8 and 27.0; left behind: 200 x 4,096 x 1,280 51.9 and 44.7, 64 x 16,384 x 1,280 53.5 and 47.3).
   // (300 x 128,256 x 2,048, where both cost the same by this rule: 2,053 in tiles, 2,236 in 64 x 64: the tiles unless 2 % are won.)
   // Three stretches of K and fewer leave waves without one (4,099 x 516 at 33 rows 15.2 us, the tiles 12.5; 1,000 x 1,000 7.8 and 18.0).
   typedef void (*Launch)(const float*, const float*, float*, int, int, int, int, int, int, bool, hipStream_t);
@@ -374,12 +383,13 @@ static bool gemm_f32(const float* A, const float* W, float* C, int M, int N, int
       {16, 16, 35, launch_f32_stream<1, 1, 16, 2>}, {32, 16, 50, launch_f32_stream<2, 1, 4, 2>}, {32, 32, 69, launch_f32_stream<2, 2, 4, 2>},
       {48, 32, 84, launch_f32_stream<3, 2, 8, 1>},  {64, 32, 100, launch_f32_stream<4, 2, 8, 1>}, {48, 48, 112, launch_f32_stream<3, 3, 8, 1>},
       {48, 64, 155, launch_f32_stream<3, 4, 4, 1>}, {64, 64, 198, launch_f32_stream<4, 4, 4, 1>}};
-  long best = 0;
+  long best = 0, best_turns = 0;
   Launch launch = nullptr;
   for (const auto& s : shapes) {
-    const long groups = (long)((M + s.rows - 1) / s.rows) * ((N + s.cols - 1) / s.cols), cost = s.turn * ((groups + GS_UNITS - 1) / GS_UNITS);
-    if (!launch || cost < best) { best = cost; launch = s.launch; }
+    const long groups = (long)((M + s.rows - 1) / s.rows) * ((N + s.cols - 1) / s.cols), turns = (groups + GS_UNITS - 1) / GS_UNITS, cost = s.turn * turns;
+    if (!launch || cost < best) { best = cost; best_turns = turns; launch = s.launch; }
   }
+  if (best_turns > 1) best = best * ((K + 1023) / 1024 * 1024) / K;
   const long t44 = f32_tiles<4, 4>(M, N), t22 = f32_tiles<2, 2>(M, N), t11 = 62 * f32_tiles<1, 1>(M, N) / GS_UNITS;
   const long tiles = t44 >= GS_ENOUGH_TILES ? 680 * t44 / GS_UNITS : t22 >= GS_ENOUGH_TILES ? 190 * t22 / GS_UNITS : t11 < 166 ? 166 : t11;
   if (near && (M <= GS_MOST_ROWS || (K > 768 && 50 * best < 49 * tiles))) {

@@ -423,7 +423,12 @@ def test_gemm_generic(M, N, K_):
 @pytest.mark.parametrize("M,N,K_", [(2, 16, 4), (16, 1000, 2052), (17, 33, 20), (32, 8192, 260), (3, 8200, 4096),
                                     (33, 97, 516), (65, 4100, 256), (300, 8205, 288), (1030, 8192, 36),
                                     # short rows: the vector kernel's, and the first that are not
-                                    (5, 300, 16), (5, 4100, 48), (5, 4100, 52), (20, 4100, 96), (20, 4100, 100)])
+                                    (5, 300, 16), (5, 4100, 48), (5, 4100, 52), (20, 4100, 96), (20, 4100, 100),
+                                    # up to 16 rows: a last stretch that is not full, of one to four; full ones; one more than four
+                                    (1, 300, 20), (8, 1000, 252), (16, 2050, 260), (7, 130, 772), (8, 16500, 900), (9, 70, 1020),
+                                    (4, 300, 1024), (1, 300, 1028),
+                                    # shapes against tiles by the fullest of four: five stretches, twelve
+                                    (300, 4100, 1280), (142, 6150, 3072)])
 def test_gemm_fp32_on_the_matrix_cores_leaves_the_vector_kernels_bits(M, N, K_):
     padded, w = _rand(M, K_ + 1, seed=1), _rand(N, K_, seed=2)
     padded[0, :K_] *= 1e-30                                    # products that are subnormal or nothing
