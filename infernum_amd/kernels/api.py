@@ -954,9 +954,15 @@ def decode_splits(batch: int, nh: int, nkv: int, max_len: int, device: Optional[
       heads, one request, whole against two parts: 150 keys of 64 values 7.5 us and 8.8, of 128 values 8.9 and 10.0; 250
       keys 8.0 and 8.7, 9.8 and 10.2; from 320 keys of 128 values on four parts are 1 us faster);
     * above 128 a compute unit holds one workgroup, and more parts than compute units only cost (head size 256, 32
-      requests on 4 key/value heads: 19 us in two parts, 23 in four); at 65 to 128, where eight waves take a part,
-      three quarters of the compute units do better than all from eight parts on (4 requests on 8 key/value heads of 128,
-      2,048 / 4,096 keys: 16.3 / 22.6 us in six parts, 17.8 / 22.9 in eight);
+      requests on 4 key/value heads: 19 us in two parts, 23 in four); at 97 to 128, where eight waves take a part,
+      three quarters of the compute units do better than all of them from eight parts on (4 requests on 8 key/value heads of
+      128, 2,048 / 8,192 / 32,768 keys: 13.8 / 31.3 / 96 us in six parts, 15.2 / 33.3 / 112 in eight), but not better than nearly all
+      (3 requests, 4,096 / 8,192 / 32,768 keys: 17.3 / 25.0 / 78.4 us in eight parts, 192 workgroups, and 16.9 / 24.7 / 75.5 in ten, 240; 3 on 4 key/value
+      heads with 32,768: 46.5 in sixteen, 42.6 in 21);
+    * at head sizes up to 64 and up to 8,192 keys the second workgroup on a compute unit costs the join more than it gives,
+      where the first alone cuts a request into four parts or more, and more than 32 parts of one never pay (one request on 8 key/value
+      heads, 8,192 / 32,768 keys: 12.3 / 22.0 us in 32 parts, 14.2 / 25.5 in 40 / 64; two with 4,096: 11.1 in 16, 12.4 in 24; four with 1,024: 8.4
+      in 8, 9.6 in 10; eight with 528: 9.2 in four, 9.4 in five);
     * the join, which asks for sixteen parts' results at once, costs little, so a wave should have a tile or two: up to
       a part for four tiles (six, up to a head size of 128), and for long requests with the square root of the tiles (one
       request of 16 heads of 256 on one key/value head, 1,024 / 2,048 / 4,096 / 16,384 keys: 18.2 / 21.6 / 24.1 / 35.9 us in
@@ -973,10 +979,13 @@ def decode_splits(batch: int, nh: int, nkv: int, max_len: int, device: Optional[
     if head_dim > 128:
         wanted, most = fill // groups, min(tiles // 4, math.isqrt(4 * tiles))
     else:
-        wanted = fill // groups if 4 * groups <= fill else 2 * fill // groups
-        if head_dim > 64 and wanted >= 8:
-            wanted = 3 * fill // (4 * groups)
-        most = min(tiles // 6, math.isqrt(9 * tiles // 4))
+        if head_dim <= 64 and max_len <= 8192 and 4 * groups <= cus:
+            wanted = cus // groups
+        else:
+            wanted = fill // groups if 4 * groups <= fill else 2 * fill // groups
+        if head_dim > 96 and wanted >= 8 and fill % groups == 0:
+            wanted = 3 * wanted // 4
+        most = min(tiles // 6, math.isqrt(9 * tiles // 4), 32 if head_dim <= 64 else 64)
     return max(1, min(wanted, most, 64))
 
 
