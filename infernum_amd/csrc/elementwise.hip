@@ -185,7 +185,7 @@ __global__ __launch_bounds__(NT) void embed_norm_kernel(const char* __restrict__
 }
 
 // table [V, H] and pos_table (nullable, with positions) [pos_rows, H] and vector (nullable) [H] in either type; w (nullable) without w2.
-// H a multiple of 4, at most 1,024 or 2,048 to 4,096 (the norm's launch sums other rows in other orders); every pointer on 16 bytes.
+// H a multiple of 8, at most 1,024 or 2,048 to 4,096 (the norm's launch sums other rows in other orders); every pointer on 16 bytes.
 extern "C" int ia_embed_norm(const void* table, int table_dtype, const int* ids, const void* pos_table, int pos_dtype,
                              const int* positions, int pos_rows, const void* vector, int vector_dtype, float* h, void* kept,
                              const void* w, int w_dtype, void* x, const void* w2, int w2_dtype, void* x2, int act_dtype, int N,

@@ -264,10 +264,10 @@ class Value:
 class _Writer:
     """The operations that completed the stream, as the last ones written (``StepProgram.stream_written``)."""
 
-    __slots__ = ("first", "end", "write", "when", "eps", "add_vector")
+    __slots__ = ("first", "end", "write", "when", "eps", "add_vector", "reads")
 
-    def __init__(self, first: int, end: int, write, when: Guard, eps, add_vector):
-        self.first, self.end, self.write, self.when, self.eps, self.add_vector = first, end, write, when, eps, add_vector
+    def __init__(self, first: int, end: int, write, when: Guard, eps, add_vector, reads):
+        self.first, self.end, self.write, self.when, self.eps, self.add_vector, self.reads = first, end, write, when, eps, add_vector, reads
 
 
 _CALLBACK = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.POINTER(ctypes.c_uint64), ctypes.c_int)
@@ -435,13 +435,14 @@ class StepProgram:
 
     # ---- a norm on the launch that completes the stream ---------------------------------------
     def stream_written(self, first: int, write: Callable[..., None], when: Guard = ALWAYS, eps: Optional[float] = None,
-                       add_vector: Optional[Callable[[torch.Tensor], None]] = None) -> None:
+                       add_vector: Optional[Callable[[torch.Tensor], None]] = None,
+                       reads: Sequence[Optional[torch.Tensor]] = ()) -> None:
         """The operations from number ``first`` on complete the stream in ``h``, and their launcher can go on with the
         norm of its rows for the steps of ``when`` (with the root's ``eps``, or with any): ``write(when, norm, side)``
         writes them again, with ``norm`` into ``x`` and ``side`` (None, or another norm and its buffer) or without (None).
         ``add_vector(v)`` writes them again with v added to all rows; a launcher that has it also takes the norm "cast",
-        the rows themselves rounded into ``x``."""
-        self._writer = _Writer(first, len(self._ops), write, when, eps, add_vector)
+        the rows themselves rounded into ``x``.  ``reads``: the model's tensors that the launcher reads."""
+        self._writer = _Writer(first, len(self._ops), write, when, eps, add_vector, tuple(reads))
 
     def _last_writer(self) -> Optional["_Writer"]:
         w, self._writer = self._writer, None
@@ -472,9 +473,12 @@ class StepProgram:
         """For which steps the launches just written, that completed the stream, leave its norm behind as well: no launch
         for it is needed then.  ``rows``: the norm is wanted of the wanted rows, which have to be all rows in their order.
         The norms' kernels sum a row's squares in one order up to 1,024 values and from 2,048 on (between, and off
-        multiples of four, in another each), so that the row's bits are those of the norm's own launch."""
+        multiples of four, in another each), so that the row's bits are those of the norm's own launch.  That launch reads a weight
+        from any address, those that go on with a norm 16 bytes at a time (a model may be loaded with views into larger tensors)."""
         w, H = self._last_writer(), self.hidden_size
         if w is None or H % 4 or not (H <= 1024 or 2048 <= H <= 16384) or (w.eps is not None and w.eps != norm.eps):
+            return NEVER
+        if any(t is not None and t.data_ptr() % 16 for t in (norm.weight, side[0].weight if side is not None else None, *w.reads)):
             return NEVER
         return self._write_again(w, w.when & Guard.between(self.ALL_ROWS, 1) if rows else w.when, norm, side)
 

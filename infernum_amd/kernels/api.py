@@ -146,7 +146,8 @@ def embed_norm(table: torch.Tensor, ids: torch.Tensor, h: torch.Tensor, weight: 
                kept: Optional[torch.Tensor] = None, side_weight: Optional[torch.Tensor] = None,
                out_side: Optional[torch.Tensor] = None) -> torch.Tensor:
     """``embed`` (+ ``add_rows``, a cast into ``kept``, ``add_vector``) into h, and its norm into ``out`` (without ``weight`` h itself,
-    rounded), with ``side_weight`` another into ``out_side``: one launch for few rows of up to 1,024 or 2,048 to 4,096 values."""
+    rounded), with ``side_weight`` another into ``out_side``: one launch for few rows of up to 1,024 or 2,048 to 4,096 values, a multiple
+    of 8; every tensor on 16 bytes."""
     _dev(table, ids, h, weight, out, position_table, positions, vector, kept, side_weight, out_side)
     V, H = table.shape
     N = ids.numel()

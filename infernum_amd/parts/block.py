@@ -183,7 +183,7 @@ class SandwichBlock(Block):
         write(ALWAYS, next_norm, None)
         program.pending = None
         if next_norm is None:
-            program.stream_written(first, write, eps=post.eps)
+            program.stream_written(first, write, eps=post.eps, reads=[post.weight, gate.bias if gate is not None else None])
 
     def native(self, program, view: CacheView) -> None:
         if type(self).forward is not SandwichBlock.forward:

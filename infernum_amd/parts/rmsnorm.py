@@ -78,7 +78,7 @@ class RMSNorm(Norm):
                                [program.act_code, program.N, self.size, float(self.eps), STREAM], alt.when & when)
         write(ALWAYS, None, None)
         program.pending = None
-        program.stream_written(first, write, eps=self.eps)
+        program.stream_written(first, write, eps=self.eps, reads=[self.weight])
 
     def next_operands(self, program, side) -> list:
         """This norm's weight and ``program.x``, and the norm beside it with its buffer (or None), as the launchers that

@@ -370,6 +370,22 @@ def test_native_program_makes_the_launches_of_the_parts(models, name, dtype):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("name", ["A", "B"])
+def test_norm_weights_off_16_bytes(models, name, dtype, monkeypatch):
+    """A model loaded with norm weights that are views 8 bytes into larger tensors: the norms' own launches read them from there, so
+    none may ride on a launch that does not (behind the embedding), and every step gives the bits of the parts' own forward."""
+    from infernum_amd.models.model import DecoderModel
+    d, cfg, reqs, ref = models[(name, dtype)]
+    TT.off_16_bytes(monkeypatch, DecoderModel, lambda n: "norm" in n)
+    native = _engine(d, dtype, PAGE[name], 64)
+    parts = _engine(d, dtype, PAGE[name], 64, executor="parts")
+    for steps in (TT.trace_whole(reqs), TT.trace_tail_one_by_one(reqs, 5)):
+        a, b = TT.run_steps(native, steps), TT.run_steps(parts, steps)
+        assert a.keys() == b.keys() and all(torch.equal(a[k], b[k]) for k in a)
+        _check({k: t for k, t in a.items()}, {r: t for r, t in ref.items()}, dtype, f"{name} {dtype} off 16 bytes", every_place=False)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("limit", [7, 64, 129, 300])
 def test_intermediates_of_the_program_are_large_enough_for_steps_of_every_shape(models, dtype, limit):
     """An engine whose steps take at most ``limit`` tokens has intermediates for exactly that many: steps that fill

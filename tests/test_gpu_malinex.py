@@ -628,6 +628,22 @@ def test_one_request_at_a_time(models, name, dtype, how):
 
 
 @BOTH
+@pytest.mark.parametrize("which", ["norm1b", "norm2b", "norm1", "norm2", "final.norm", "rg", "pos"])
+def test_weights_off_16_bytes(models, which, dtype, monkeypatch):
+    """Weights of the branches' norms, of the norms behind them, the gates' biases and the positions' rows as views 8 bytes into larger tensors, one kind at
+    a time: a step of the program gives the bits of the parts' own forward, whose norms are launches of their own."""
+    from infernum_amd.engine import StepEntry
+    from infernum_amd.models.model import DecoderModel
+    d, cfg, w, reqs, ref, *_ = models["X1"]
+    TT.off_16_bytes(monkeypatch, DecoderModel, lambda n: n == which or n.endswith("." + which) or (which == "rg" and ".rg" in n and n.endswith(".b")))
+    a, b = _engine(d, dtype, PAGE["X1"], 64), _engine(d, dtype, PAGE["X1"], 64, executor="parts")
+    toks = max(reqs.values(), key=len)
+    for step in ([StepEntry("a", toks[:40], [39]), StepEntry("b", toks[3:20], [16])], [StepEntry(r, [toks[50]], [0]) for r in "ab"],
+                 [StepEntry(r, [toks[51]], [0]) for r in "ab"], [StepEntry(r, [toks[52]], [0]) for r in "ab"]):
+        assert torch.equal(a.step(step), b.step(step))
+
+
+@BOTH
 @pytest.mark.parametrize("name", NAMES)
 def test_mixed_batches_with_pages_and_slots_used_again(models, name, dtype):
     d, cfg, w, _, _, reqs, ref = models[name]

@@ -147,3 +147,24 @@ def rms_error_against(got: Dict[Tuple[str, int], torch.Tensor], want: Dict[str, 
         sq_w += float((ref * ref).sum())
         n += ref.numel()
     return (sq_d / max(sq_w, 1e-300)) ** 0.5
+
+
+def off_16_bytes(monkeypatch, model, which) -> None:
+    """Models loaded from now on get the tensors whose name ``which`` accepts as views 8 bytes into tensors of their own."""
+    load = model.load_weights
+
+    def moved(t):
+        room = torch.empty(t.numel() + 16 // t.element_size(), dtype=t.dtype, device=t.device)
+        view = room[8 // t.element_size():][:t.numel()].view(t.shape)
+        view.copy_(t)
+        assert view.data_ptr() % 16 == 8
+        return view
+
+    class Moved:
+        def __init__(self, tensors):
+            self.tensors = tensors
+
+        def __getitem__(self, name):
+            t = self.tensors[name]
+            return moved(t) if which(name) else t
+    monkeypatch.setattr(model, "load_weights", lambda self, tensors: load(self, Moved(tensors)))
