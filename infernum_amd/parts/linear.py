@@ -402,7 +402,7 @@ class Finish:
     cap: float = 0.0
 
     def __bool__(self) -> bool:
-        return self.bias is not None or bool(self.act) or self.scale != 1.0 or self.cap > 0.0
+        return self.bias is not None or bool(self.act) or self.scale != 1.0 or self.cap != 0.0     # (one that is not positive is refused below)
 
     def fused(self, w: torch.Tensor, dtype: torch.dtype, out_dtype: torch.dtype) -> bool:
         """Whether the weight-streaming kernel takes it with this weight."""

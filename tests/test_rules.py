@@ -33,3 +33,12 @@ def test_tokens_from_which_experts_take_the_grouped_product(E, top, W, ff, gated
 def test_parts_of_the_keys_in_decode_attention(monkeypatch, batch, nkv, head, keys, parts):
     monkeypatch.setattr(K, "compute_units", lambda device=None: 256)
     assert K.decode_splits(batch, 4 * nkv, nkv, keys, None, head) == parts
+
+
+@pytest.mark.parametrize("cap", [-30.0, float("nan")])
+def test_a_softcap_that_is_not_positive_is_no_empty_finish(cap):
+    """... so that the launch or the function that applies it refuses it, as before it was applied on the way to memory."""
+    from infernum_amd.parts.linear import Finish
+    assert Finish(cap=cap) and not Finish() and Finish(cap=2.0) and Finish(scale=0.5)
+    with pytest.raises(K.KernelError):
+        Finish(cap=cap).apply(torch.zeros(2, 8))
