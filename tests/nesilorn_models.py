@@ -8,7 +8,7 @@ N2: sizes that no fast kernel takes (latent head size 26, width 100, odd vocabul
 N4: see below.
 N3: twenty heads on the one cached head (more than one tile of sixteen heads); plain query size equal to the
     latent's; rotated part partly rotated (rot.dims below rot_dim); four experts, three chosen, of sizes that
-    send portions of 64 tokens and more to the grouped product and shorter ones to the tiles.
+    send portions of 150 tokens and more (kernels.api.moe_grouped_from_tokens) to the grouped product and shorter ones to the tiles.
 """
 import json
 import os

@@ -1727,9 +1727,11 @@ def test_routed_experts_of_few_pairs(gated, weights_on, N, top, E, W, ff):
             assert float((parts[c, n].double() - want).norm() / want.norm()) <= 4 * 2.0 ** -9
 
 
-# fewer pairs than experts, more, several tiles of 32 pairs of an expert, tiles of 128 (from 48 pairs an expert on)
+# fewer pairs than experts, more, several tiles of 32 pairs of an expert, tiles of 64 x 128; tiles of 128 x 256, which steps of 56 pairs an
+# expert and 224 such tiles take (the last for its first product alone)
 @pytest.mark.parametrize("gated", [True, False])
-@pytest.mark.parametrize("E,top,W,ff,counts", [(32, 4, 2048, 1408, (2, 3, 8, 33)), (8, 2, 520, 328, (2, 5, 65, 200)), (3, 1, 72, 1000, (2, 40))])
+@pytest.mark.parametrize("E,top,W,ff,counts", [(32, 4, 2048, 1408, (2, 3, 8, 33)), (8, 2, 520, 328, (2, 5, 65, 200)), (3, 1, 72, 1000, (2, 40)),
+                                               (40, 2, 1288, 1000, (3, 300, 1130))])
 def test_a_pairs_result_does_not_depend_on_the_steps_other_pairs(gated, E, top, W, ff, counts):
     api = K()
     most = max(counts)

@@ -676,6 +676,29 @@ def test_the_stream_after_every_layer(models, tmp_path, name, dtype):
         assert torch.equal(parts, logits)
 
 
+def test_routed_layers_by_the_tiles_and_by_the_grouped_product(models):
+    """Prompts of a token less than the routed layers take the grouped product from, of as many, and of more: the step's program against
+    the plain model and, bit for bit, the parts' own forward, with the launches of either route."""
+    from infernum_amd.engine import StepEntry
+    from infernum_amd.kernels import api as K
+    m, layers = models["V3"], (1,)
+    f = m.cfg["layers"][layers[0]]["mlp"]
+    first = K.moe_grouped_from_tokens(f["router"]["experts"], f["router"]["top"], m.cfg["width"], f["expert"]["ff"], torch.bfloat16)
+    a, b = (_engine(m.dir["bfloat16"], "bfloat16", PAGE["V3"], 64, **kw) for kw in ({}, {"executor": "parts"}))
+    launches = []
+    for r, toks in TT.make_requests(m.cfg["vocab"], (first - 1, first, first + 43), seed=31).items():
+        step = [StepEntry(r, toks, list(range(len(toks))))]
+        logits = a.step(step).cpu()
+        launches.append(a.program.last_launches())
+        assert torch.equal(logits, b.step(step).cpu()), r
+        _check({(r, p): logits[p] for p in range(len(toks))}, {r: MP.forward(m.cfg, m.w["bfloat16"], toks)}, "bfloat16", f"V3 {len(toks)} tokens", "V3")
+        a.end(r), b.end(r)
+    a.program.check_guards()
+    # two products with their sort's order inside; rows gathered, product, activation, product, scatter
+    passes = sum(e.layer in layers for e in a.model.spec.schedule)
+    assert launches[1] - launches[0] == 3 * passes and launches[2] == launches[1]
+
+
 @BOTH
 @pytest.mark.parametrize("name", NAMES)
 @pytest.mark.parametrize("how", ["whole", "tail", "portions", "one_by_one"])

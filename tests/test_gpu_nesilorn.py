@@ -389,6 +389,28 @@ def test_one_request_at_a_time(models, name, dtype, how):
         assert eng.program.num_python_ops == 0             # every part wrote its own launches
 
 
+def test_routed_layers_by_the_tiles_and_by_the_grouped_product(models):
+    """Prompts of a token less than the routed layers take the grouped product from, of as many, and of more: the step's program against
+    the plain model and, bit for bit, the parts' own forward, with the launches of either route."""
+    from infernum_amd.engine import StepEntry
+    from infernum_amd.kernels import api as K
+    d, cfg, w, *_ = models["N3"]
+    f = cfg["layers"][0]["mlp"]
+    first = K.moe_grouped_from_tokens(f["router"]["experts"], f["router"]["top"], cfg["width"], f["expert"]["ff"], torch.bfloat16)
+    a, b = _engine(d, "bfloat16", PAGE["N3"], 64), _engine(d, "bfloat16", PAGE["N3"], 64, executor="parts")
+    launches = []
+    for r, toks in TT.make_requests(cfg["vocab"], (first - 1, first, first + 43), seed=32).items():
+        step = [StepEntry(r, toks, list(range(len(toks))))]
+        logits = a.step(step).cpu()
+        launches.append(a.program.last_launches())
+        assert torch.equal(logits, b.step(step).cpu()), r
+        _check({(r, p): logits[p] for p in range(len(toks))}, {r: _plain(cfg, w, toks)}, "bfloat16", f"N3 {len(toks)} tokens", "N3")
+        a.end(r), b.end(r)
+    a.program.check_guards()
+    # two products with their sort's order inside; rows gathered, product, activation, product, scatter
+    assert launches[1] - launches[0] == 3 and launches[2] == launches[1]
+
+
 @BOTH
 @pytest.mark.parametrize("name", NAMES[:2])
 def test_final_norm_of_all_rows_of_some_and_of_some_twice(models, name, dtype):

@@ -548,7 +548,7 @@ def test_values_mixed_with_an_earlier_layers(dtype):
 @BOTH
 @pytest.mark.parametrize("mlp,W,N", [(PM.P1["layers"][0]["mlp"], 64, 60), (PM.P2["layers"][0]["mlp"], 100, 9), (PM.P2["layers"][2]["mlp"], 100, 40),
                                      (PM.P3["layers"][1]["mlp"], 128, 1), (PM.P3["layers"][2]["mlp"], 128, 70), (PM.P5["layers"][1]["mlp"], 48, 30),
-                                     (PM._moe(64, 4, 2, 4, (2, 1), 64), 64, 300), (PM._moe(64, 6, 3, 3, (3, 2)), 128, 200)])
+                                     (PM._moe(64, 4, 2, 4, (2, 1), 64), 64, 300), (PM._moe(64, 6, 3, 3, (3, 2)), 128, 230)])
 def test_routed_experts_alone(dtype, mlp, W, N):
     """Groups, a correction, identity experts and the gated shared expert; by natural routers (where no choice is a
     close call) and by corrections that decide alone; few tokens and so many that the grouped product takes them."""
@@ -678,6 +678,29 @@ def test_the_stream_after_every_layer(models, tmp_path, name, dtype):
                f"{name} {dtype} first {k} layers", name)
         parts = _engine(sd, dtype, PAGE[name], 64, executor="parts").step([StepEntry("a", toks, list(range(len(toks))))]).cpu()
         assert torch.equal(parts, logits)
+
+
+def test_routed_layers_by_the_tiles_and_by_the_grouped_product(models):
+    """Prompts of a token less than the routed layers take the grouped product from, of as many, and of more: the step's program against
+    the plain model and, bit for bit, the parts' own forward, with the launches of either route."""
+    from infernum_amd.engine import StepEntry
+    from infernum_amd.kernels import api as K
+    m, layers = models["P3"], (0, 2)
+    f = m.cfg["layers"][layers[0]]["mlp"]
+    first = K.moe_grouped_from_tokens(f["router"]["experts"], f["router"]["top"], m.cfg["width"], f["expert"]["ff"], torch.bfloat16)
+    a, b = (_engine(m.dir["bfloat16"], "bfloat16", PAGE["P3"], 64, **kw) for kw in ({}, {"executor": "parts"}))
+    launches = []
+    for r, toks in TT.make_requests(m.cfg["vocab"], (first - 1, first, first + 43), seed=31).items():
+        step = [StepEntry(r, toks, list(range(len(toks))))]
+        logits = a.step(step).cpu()
+        launches.append(a.program.last_launches())
+        assert torch.equal(logits, b.step(step).cpu()), r
+        _check({(r, p): logits[p] for p in range(len(toks))}, {r: PP.forward(m.cfg, m.w["bfloat16"], toks)}, "bfloat16", f"P3 {len(toks)} tokens", "P3")
+        a.end(r), b.end(r)
+    a.program.check_guards()
+    # two products with their sort's order inside; rows gathered, product, activation, product, scatter
+    passes = sum(e.layer in layers for e in a.model.spec.schedule)
+    assert launches[1] - launches[0] == 3 * passes and launches[2] == launches[1]
 
 
 @BOTH
