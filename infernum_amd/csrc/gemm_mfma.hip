@@ -187,7 +187,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_mfma_kernel(const
   // sums depend neither on the rows beside it nor on the number of rows.
   // The grouped product starts where the tiles of few pairs do (ia_expert_first_chunk): the same bits from either.
   constexpr bool ROTATE = SPLIT || GLU || GROUPED;
-  static_assert(!GROUPED || BN == 256, "the grouped product's tile is the 256 columns that share a start");
+  static_assert(!GROUPED || 512 % BN == 0, "a tile lies in the columns that share a start");
   const int rot = GROUPED ? ia_expert_first_chunk(n0, K) * (IA_EXPERT_CHUNK / GM_BK)
                   : ROTATE ? (int)((((unsigned)tn * 0x9E3779B1u) >> 8) % (unsigned)ksteps) : 0;
   auto krot = [&](int kt) {

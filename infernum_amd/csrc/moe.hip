@@ -260,7 +260,7 @@ __global__ __launch_bounds__(256) void moe_gate_up_kernel(const T* __restrict__ 
 // v_mfma_f32_16x16x32_bf16 with W's rows as its first operand: lane (r = lane % 16, q = lane / 16) ends with four
 // consecutive columns 4 q .. 4 q + 3 of row r of the result.
 // All workgroups walking K in step read places one row's length apart at the same moment, and where that length is a power
-// of two those lie on few memory channels, so every 256 columns start their walk at a chunk of their own (ia_expert_first_chunk) and
+// of two those lie on few memory channels, so every 512 columns start their walk at a chunk of their own (ia_expert_first_chunk) and
 // wrap around.  The tile of 128 pairs and the grouped product of gemm_mfma.hip start there too: an element is one chain over K in
 // an order that depends on K and its column alone.
 // Before, tiles of 32 x 128 in steps of 64 through one LDS stage and all walks from the same start (cold weights,
