@@ -382,13 +382,13 @@ def moe_route(logits, bias: Optional[torch.Tensor], top: int, experts: int, soft
 
 
 # From how many rows an expert on average the grouped form is ahead of the tiles behind the sort: sort to scatter, microseconds of
-# grouped / tiles with cold weights.  Gated: 32 experts of 1,408 x 2,048 at 64 / 112 / 128 rows 171 / 172, 192 / 191, 245 / 278; 64 of them
-# 314 / 306, 391 / 372, 458 / 452; 8 of 2,752 x 2,048 106 / 99, 116 / 103, 160 / 169; 4 of 4,800 x 4,096 162 / 162, 178 / 164, 182 / 205.
-# Without a gate: 8 of 4,800 x 4,096 at 48 / 56 / 64 rows 172 / 163, 175 / 169, 178 / 218.
+# grouped / tiles with cold weights.  Gated: 32 experts of 1,408 x 2,048 at 64 / 112 / 128 rows 173 / 173, 193 / 192, 233 / 276; 64 of them
+# 319 / 308, 392 / 372, 446 / 450; 8 of 2,752 x 2,048 104 / 100, 116 / 104, 149 / 173; 4 of 4,800 x 4,096 161 / 163, 175 / 163, 179 / 204.
+# Without a gate: 8 of 4,800 x 4,096 at 48 / 56 / 64 rows 172 / 164, 174 / 169, 177 / 220.
 # The passes around the grouped products (rows in the order of the sort, activation, scatter) take rows times (W + ff), the products rows
 # times W ff; where those weigh little and the tiles of 128 x 256 that the experts then have fill the chip, gated ones change over sooner: at
-# 48 / 56 / 64 / 112 rows 20 of 2,432 x 4,096 298 / 272, 315 / 334, 313 / 342, 343 / 393; 8 of 4,800 x 4,096 255 / 211, 258 / 264, 263 / 304,
-# 289 / 320; 8 of 14,336 x 4,096 603 / 552, 616 / 628, 626 / 729, 688 / 726; 8 of 8,192 x 5,120 413 / 446, 418 / 475, 428 / 468, 466 / 515.
+# 48 / 56 / 64 / 112 rows 20 of 2,432 x 4,096 297 / 274, 306 / 335, 310 / 342, 333 / 381; 8 of 4,800 x 4,096 253 / 207, 257 / 260, 260 / 307,
+# 281 / 318; 8 of 14,336 x 4,096 621 / 536, 627 / 617, 635 / 726, 684 / 735; 8 of 8,192 x 5,120 412 / 448, 415 / 466, 423 / 467, 452 / 504.
 # Either way a pair's result has the same bits.
 MOE_GROUPED_ROWS_AN_EXPERT = 112
 MOE_GROUPED_ROWS_A_WIDE_EXPERT = 56
