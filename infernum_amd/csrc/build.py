@@ -40,6 +40,7 @@ CORE_SOURCES = [
     "gemm_generic.hip",
     "gemm_skinny.hip",
     "gemm_mfma.hip",
+    "gemm_tiles.hip",
     "attention_generic.hip",
     "norm_branch.hip",
     "activations.hip",

@@ -652,6 +652,45 @@ def gemm_mfma(a: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = No
     return out
 
 
+GEMM_TILES = ((256, 256), (256, 224), (256, 192), (256, 160), (256, 128), (224, 256), (192, 256), (192, 192), (192, 128),
+              (160, 256), (160, 192), (160, 128), (128, 256), (128, 192), (128, 128))
+
+
+def gemm_tiles_supported(M: int, N: int, K: int) -> bool:
+    """Sizes :func:`gemm_tiles` takes: K in steps of 64, rows addressed with 32-bit byte offsets."""
+    return M >= 1 and N >= 1 and K >= 64 and K % 64 == 0 and max(M, N) * K * 2 < 2 ** 32 - 3072
+
+
+def gemm_tiles_pays(M: int, N: int, K: int) -> bool:
+    """Whether a whole product of many rows goes to :func:`gemm_tiles` rather than to the vendor's library."""
+    return bool(_core().ia_gemm_tiles_pays(int(M), int(N), int(K)))
+
+
+def gemm_tiles(a: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None, swiglu: bool = False,
+               tile: Optional[Tuple[int, int]] = None) -> torch.Tensor:
+    """a[M, K] @ w[N, K]^T in bf16 with fp32 accumulation for a prompt's rows; with ``swiglu`` silu(a @ w[:N/2]^T) *
+    (a @ w[N/2:]^T), [M, N/2], the activation on the fp32 sums.  ``tile``: rows of a and of w a workgroup takes, of GEMM_TILES
+    (default: chosen by the sizes).  A row's result depends neither on the tile nor on the rows beside it."""
+    _dev(a, w, out)
+    _need(a.dim() == 2 and w.dim() == 2 and a.shape[1] == w.shape[1], "gemm_tiles: shapes")
+    M, K = a.shape
+    N = w.shape[0]
+    _need(a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16, "gemm_tiles: bf16 operands")
+    _need(a.is_contiguous() and w.is_contiguous() and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0,
+          "gemm_tiles: contiguous operands on 16 bytes")
+    _need(gemm_tiles_supported(M, N, K) and not (swiglu and N % 2),
+          f"gemm_tiles: M={M} N={N} K={K} not supported (K % 64 == 0, below 4 GiB, N even with the activation)")
+    _need(tile is None or (tuple(tile) in GEMM_TILES and not (swiglu and tile[1] in (224, 160))), f"gemm_tiles: no tile {tile!r}")
+    cols = N // 2 if swiglu else N
+    if out is None:
+        out = torch.empty((M, cols), dtype=torch.bfloat16, device=a.device)
+    _need(out.dtype == torch.bfloat16 and out.is_contiguous() and tuple(out.shape) == (M, cols) and out.data_ptr() % 16 == 0,
+          f"gemm_tiles: out must be contiguous bf16 [{M}, {cols}] on 16 bytes")
+    rows_, cols_ = tile if tile is not None else (0, 0)
+    _ok(_core().ia_gemm_tiles(_p(a), _p(w), _p(out), M, N, K, int(swiglu), rows_, cols_, _stream()), "gemm_tiles")
+    return out
+
+
 def gemm_mfma_swiglu(a: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
                      tiled: Optional[torch.Tensor] = None) -> torch.Tensor:
     """silu(a @ w[:N/2]^T) * (a @ w[N/2:]^T) as bf16 [M, N/2]: the LDS-tiled MFMA product (tiles of 128 x 128) with
@@ -2427,7 +2466,7 @@ def attention_mfma_available(d: int, dv: Optional[int] = None) -> bool:
 # standard error when the process ends (``profile_report`` gives it at any time).  The reference's switch of the
 # same name prints the time per operation of its graph executor (infernum-cpu/src/executor.rs:24-71).  Steps
 # are not recorded into HIP graphs meanwhile (a replayed launch has no call to bracket).
-_PROFILED = ("sigattn_decode", "sigattn_prefill", "gemm_mfma_grouped", "norm_add", "activation", "latent_prepare", "gemm_heads", "router_topk", "moe_experts", "cast", "copy_pages", "gather_tokens", "words_from_host", "words_to_host", "embed", "add_rmsnorm", "residual_add", "rope_kv_append", "swiglu", "gemm_generic", "gemm_mfma",
+_PROFILED = ("sigattn_decode", "sigattn_prefill", "gemm_mfma_grouped", "norm_add", "activation", "latent_prepare", "gemm_heads", "router_topk", "moe_experts", "cast", "copy_pages", "gather_tokens", "words_from_host", "words_to_host", "embed", "add_rmsnorm", "residual_add", "rope_kv_append", "swiglu", "gemm_generic", "gemm_mfma", "gemm_tiles",
              "gemm_library", "gemm_skinny", "gemm_skinny_rows", "attention_generic", "attention_decode", "attention_decode_rotating",
              "attention_prefill", "argmax", "repetition_penalty", "sample")
 _profile_on = False

@@ -17,7 +17,8 @@ the same launches; ``INFERNUM_GEMM_ROUTE=measured`` times both when a model load
 the rule of sizes); for the bands of rows of :data:`KNOWN_MID_ROWS` (up to a few hundred rows) the LDS-tiled MFMA
 kernel with K split over workgroups, for products whose partial sums the next kernel takes (the library's kernels
 for so few rows leave most of the GPU idle, and from some tens of rows on the tiled kernel streams a weight faster
-than the weight-streaming one); above that the library, as the reference uses its library there; an fp32 result of more
+than the weight-streaming one); above that the library, as the reference uses its library there, or where it is the faster (a rule
+of sizes, and always with the activation in its epilogue) the kernel of ``csrc/gemm_tiles.hip``, the same bits on the shapes tried; an fp32 result of more
 than 128 rows comes from the LDS-tiled kernel's fp32 sums (128 rows at a time from the weight-streaming kernel where
 the tiled one does not take the size).  ``set_prefill_gemm("mfma")`` (or
 INFERNUM_PREFILL_GEMM=mfma) sends the many-row bf16 products to the hand-written LDS-tiled MFMA kernel instead,
@@ -253,15 +254,14 @@ def measure_route(w: torch.Tensor, epilogue: Optional[str], keep_split: bool, ma
             for block in range(1, K.SKINNY_MAX_M // 16):
                 M = 16 * (block + 1)
                 x = torch.zeros((M, Kdim), dtype=torch.bfloat16, device=w.device)
-                y = torch.empty((M, N), dtype=torch.bfloat16, device=w.device)
                 act = torch.empty((M, N // 2), dtype=torch.bfloat16, device=w.device) if epilogue == "swiglu" else None
 
                 def own():
                     K.gemm_skinny(x, w, epilogue=epilogue, keep_split=keep_split)
 
                 def library():
-                    K.gemm_library(x, w, out=y)
-                    if act is not None:
+                    y, activated = _run("library", x, w, torch.bfloat16, epilogue, "mfma")
+                    if act is not None and not activated:
                         K.swiglu(y, act)
                 own(), library()                      # the first call of a shape asks the library for its plan
                 if timed(library) < margin * timed(own):
@@ -363,6 +363,14 @@ def route_of(routes: List[Route], M: int) -> Route:
     raise K.KernelError(f"linear: no route for {M} rows")
 
 
+def on_16_bytes(t: Any) -> bool:
+    """Whether an operand (a tensor, or a place in a program's arena, whose buffers begin on 256 bytes) is known to lie on 16 bytes."""
+    if isinstance(t, torch.Tensor):
+        return t.data_ptr() % 16 == 0
+    from ..engine.program import Buffer, BufferAt
+    return isinstance(t, Buffer) or (isinstance(t, BufferAt) and t.nbytes % 16 == 0)
+
+
 def _run(kind: str, x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, epilogue: Optional[str],
          fallback: Optional[str] = None, parts: int = 0):
     M, N = x.shape[0], w.shape[0]
@@ -383,6 +391,11 @@ def _run(kind: str, x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, ep
     if kind == "mfma":
         return K.gemm_mfma(x, w), False
     if kind == "library":
+        if x.dtype == torch.bfloat16 and K.gemm_tiles_supported(M, N, x.shape[1]) and on_16_bytes(x) and on_16_bytes(w):
+            if epilogue == "swiglu":
+                return K.gemm_tiles(x, w, swiglu=True), True
+            if K.gemm_tiles_pays(M, N, x.shape[1]):
+                return K.gemm_tiles(x, w), False
         try:
             return K.gemm_library(x, w), False
         except K.KernelUnsupported:             # the library has no algorithm for this shape
@@ -548,6 +561,9 @@ def emit_linear(program, x: Any, M: Any, w: torch.Tensor, out_dtype: torch.dtype
             program.op("core", "ia_gemm_skinny_rows", [x, wk, int(tiled is not None), out, code, M, N, Kdim, ws,
                                                         splits * small * N if splits > 1 else 0, P.STREAM], g)
             finish.emit(program, out, M, N, code, g)
+        elif r.kind == "library" and epilogue == "swiglu" and rt.dtype == torch.bfloat16 and K.gemm_tiles_supported(T, N, Kdim) and \
+                on_16_bytes(x) and on_16_bytes(w) and on_16_bytes(out):
+            program.op("core", "ia_gemm_tiles", [x, w, out, M, N, Kdim, 1, 0, 0, P.STREAM], g)
         else:
             # a product that leaves the whole matrix: into scratch first when an activation follows
             y = program.buffer(key + ".product", T * N * out_bytes) if epilogue == "swiglu" else out
@@ -569,7 +585,10 @@ def _emit_whole(program, kind, x, w, y, M, N, Kdim, in_code, out_code, when, if_
     elif kind == "mfma":
         program.op("core", "ia_gemm_mfma", [x, w, y, M, N, Kdim, 0, P.STREAM], when, if_unsupported)
     elif kind == "library":
+        tiles = in_code == out_code == K.DTYPE_CODE[torch.bfloat16] and K.gemm_tiles_supported(program.T, N, Kdim)
+        if tiles:                              # it refuses what the library is faster for, and what does not lie on 16 bytes
+            program.op("core", "ia_gemm_tiles", [x, w, y, M, N, Kdim, 0, -1, 0, P.STREAM], when, if_unsupported)
         ws = K.library_workspace(program.rt.device)
-        program.op("blaslt", "ia_gemm_lt", [x, w, y, M, N, Kdim, in_code, ws, ws.numel(), P.STREAM], when, if_unsupported)
+        program.op("blaslt", "ia_gemm_lt", [x, w, y, M, N, Kdim, in_code, ws, ws.numel(), P.STREAM], when, if_unsupported or tiles)
     else:
         raise K.KernelError(f"linear: {kind!r} does not leave a whole matrix")

@@ -1,0 +1,135 @@
+"""The products of a prompt's rows in quadrants (csrc/gemm_tiles.hip) against plain products in 64 bits, at the edges of their tiles."""
+import importlib
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def K():
+    from infernum_amd.kernels import api
+    return api
+
+
+def _rand(*shape, scale=1.0, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return (torch.randn(*shape, device=DEV, generator=g) * scale).to(torch.bfloat16)
+
+
+TILES = K().GEMM_TILES
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("M,N,K_", [(1, 8, 64), (257, 516, 128), (300, 1003, 192), (515, 771, 448), (129, 250, 576)])
+def test_whole_products_at_sizes_that_fill_no_tile(tile, M, N, K_):
+    """One row and one step of K; an odd and an even number of steps; edges in M and N; columns off 16 bytes."""
+    api = K()
+    a, w = _rand(M, K_, seed=1), _rand(N, K_, scale=0.1, seed=2)
+    want = a.double() @ w.double().t()
+    out = torch.full((M + 1, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    api.gemm_tiles(a, w, out[:M], tile=tile)
+    # fp32 sums of K_ products (each addition within 2^-24 of the running sum, of the order of 0.1 sqrt(K)), one rounding to bf16
+    bound = 2e-5 * math.sqrt(K_) * 0.1 + 2.0 ** -8 * want.abs()
+    assert bool(((out[:M].double() - want).abs() <= bound).all())
+    assert bool(out[M].isnan().all())                                   # nothing behind the last row
+    # a row's result depends neither on the rows beside it nor on the tile: the sums run over K in its order
+    assert torch.equal(api.gemm_tiles(a[M - 1:M].clone(), w, tile=tile)[0], out[M - 1])
+    assert torch.equal(api.gemm_tiles(a, w), out[:M])
+    assert torch.equal(api.gemm_mfma(a, w, tile="128x128"), out[:M])
+
+
+@pytest.mark.parametrize("tile", [t for t in TILES if t[1] not in (224, 160)])
+@pytest.mark.parametrize("M,N,K_", [(1, 16, 64), (300, 1004, 192), (515, 770, 448)])
+def test_products_with_the_activation(tile, M, N, K_):
+    api = K()
+    a, w = _rand(M, K_, seed=3), _rand(N, K_, scale=0.2, seed=4)
+    g, u = (a.double() @ w.double().t()).split(N // 2, dim=1)
+    want = g * torch.sigmoid(g) * u
+    out = api.gemm_tiles(a, w, swiglu=True, tile=tile)
+    # the sums' errors e through silu' <= 1.1 and the other factor, the activation's few 2^-24, one rounding to bf16
+    e = 2e-5 * math.sqrt(K_) * 0.2
+    bound = e * (1.1 * u.abs() + g.abs()) + 1e-6 * want.abs() + 2.0 ** -8 * want.abs() + 1e-6
+    assert bool(((out.double() - want).abs() <= bound).all())
+    assert torch.equal(api.gemm_tiles(a[M - 1:M].clone(), w, swiglu=True)[0], out[M - 1])
+
+
+def test_the_activation_at_its_ends():
+    """Gates that saturate to either side and infinite sums give what silu(g) u gives in fp32 (0 and u g; NaN for -inf)."""
+    api = K()
+    gates = torch.tensor([-3e4, -200.0, -90.0, -20.0, 0.0, 20.0, 200.0, 3e4], device=DEV)
+    a = torch.zeros(8, 64, dtype=torch.bfloat16, device=DEV)
+    a[:, 0], a[:, 1] = gates.to(torch.bfloat16), 1.0
+    w = torch.zeros(32, 64, dtype=torch.bfloat16, device=DEV)
+    w[:16, 0], w[16:, 1] = 1.0, 2.0
+    out = api.gemm_tiles(a, w, swiglu=True)
+    g = a[:, :1].double()
+    want = (g * torch.sigmoid(g) * 2.0).expand(8, 16)
+    assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-7).all())
+
+
+def test_one_product_is_picked_out():
+    """Single entries at the ends of rows, columns and K: a wrong place in LDS, half-tile or step would move or lose one."""
+    api = K()
+    M, N, K_ = 515, 771, 448
+    a = torch.zeros(M, K_, dtype=torch.bfloat16, device=DEV)
+    w = torch.zeros(N, K_, dtype=torch.bfloat16, device=DEV)
+    for i, (m, n, k) in enumerate([(0, 0, 0), (M - 1, N - 1, K_ - 1), (256, 255, 64), (129, 513, 71), (300, 2, 447), (63, 127, 320)]):
+        a[m, k] = 1 + i
+        w[n, k] = 2
+    want = a.float() @ w.float().t()
+    for tile in TILES:
+        assert torch.equal(api.gemm_tiles(a, w, tile=tile).float(), want), tile
+
+
+def test_what_it_refuses():
+    api = K()
+    a, w = _rand(70, 96), _rand(32, 96)
+    with pytest.raises(api.KernelError):
+        api.gemm_tiles(a, w)                                                            # K % 64
+    a, w = _rand(70, 128), _rand(33, 128)
+    with pytest.raises(api.KernelError):
+        api.gemm_tiles(a, w, swiglu=True)                                               # halves of an odd number
+    with pytest.raises(api.KernelError):
+        api.gemm_tiles(a, w, tile=(64, 64))
+    off = torch.zeros(33 * 128 + 4, dtype=torch.bfloat16, device=DEV)[4:].view(33, 128)
+    with pytest.raises(api.KernelError):
+        api.gemm_tiles(a, off)                                                          # off 16 bytes
+
+
+@pytest.mark.parametrize("off", [False, True])
+@pytest.mark.parametrize("M,N,K_", [(300, 512, 256), (2304, 2048, 2048), (2304, 2304, 4096)])
+def test_many_rows_take_it_where_it_is_the_faster(M, N, K_, off):
+    """The many-row route, plain and with the activation, for weights on 16 bytes and off them (the library's then)."""
+    L = importlib.import_module("infernum_amd.parts.linear")   # the package exports the function under this name
+    api = K()
+    x = _rand(M, K_, seed=5)
+    raw = torch.empty(N * K_ + 8, dtype=torch.bfloat16, device=DEV)
+    w = raw[4:4 + N * K_].view(N, K_) if off else raw[:N * K_].view(N, K_)
+    w.copy_(_rand(N, K_, scale=0.1, seed=6))
+    for epilogue in (None, "swiglu"):
+        assert L.route_of(L.plan(N, K_, torch.bfloat16, torch.bfloat16, epilogue, False), M).kind == "library"
+        y = L.linear(x, w, epilogue=epilogue)
+        want = x.double() @ w.double().t()
+        if epilogue:
+            g, u = want.split(N // 2, dim=1)
+            want = g * torch.sigmoid(g) * u
+        # with the activation behind the library's product gate, up and result are rounded to bf16
+        assert float((y.double() - want).norm() / want.norm()) < (6e-3 if epilogue else 3e-3)
+        if not off and (epilogue or api.gemm_tiles_pays(M, N, K_)):
+            assert torch.equal(y, api.gemm_tiles(x, w.clone(), swiglu=bool(epilogue)))
+
+
+@pytest.mark.parametrize("M,N,K_", [(2048, 4096, 14336), (8192, 4096, 14336), (7650, 4096, 14336), (512, 4096, 14336), (1500, 6144, 4096),
+                                   (300, 4096, 4096), (5700, 2048, 2048), (2300, 2048, 8192), (3000, 2048, 2048), (2048, 4096, 1984),
+                                   (2048, 4096, 4100), (70000, 4096, 32768)])
+def test_where_whole_products_take_it(M, N, K_):
+    """The rule of sizes against itself written plainly."""
+    api = K()
+    large, small = math.ceil(M / 256) * math.ceil(N / 256), math.ceil(M / 128) * math.ceil(N / 128)
+    empty = math.ceil(large / 256) * 256 / large
+    want = (K_ % 64 == 0 and max(M, N) * K_ * 2 < 2 ** 32 - 3072 and small >= 200 and K_ >= 2048 and (K_ >= 4096 or large <= 140)
+            and empty >= (1.06 if K_ >= 8192 and large > 256 else 1.2))
+    assert api.gemm_tiles_pays(M, N, K_) == want
