@@ -1048,6 +1048,13 @@ __global__ __launch_bounds__(4 * HGW * 64) void attn_prefill_kernel(
   }
 }
 
+#if IA_ATTN_EXT == 0 && IA_HEAD_DIM == 128 && IA_VALUE_DIM == 128
+#define IA_PREFILL_WIDE 1
+#include "attention_prefill.h"
+#else
+#define IA_PREFILL_WIDE 0
+#endif
+
 // ------------------------------------------------------------------ C interface
 extern "C" int ia_attn_head_dim() { return HD; }
 
@@ -1228,6 +1235,17 @@ extern "C" int ia_attn_prefill(const void* q, int q_row_stride, const void* k_pa
   const int xrc = attn_ext(window, keep, softcap, scale, bias, span, gate, gate_stride, nh, X, scale_log2);
   if (xrc != IA_OK) return xrc;
   dim3 grid(num_tiles, nkv * HC);
+#if IA_PREFILL_WIDE
+  if (G >= 2 && (ps & (ps - 1)) == 0 && ps >= 8 && bt_stride <= PW_BT) {
+#define PW_LAUNCH(W)                                                                                                          \
+  return launch_prefill_wide<W>(grid, q, q_row_stride, k_pages, v_pages, out, out_row_stride, seq_starts, seq_ctx, block_tables, \
+                                bt_stride, tiles, nh, nkv, ps, num_pages, scale_log2, window, paired, sinks, stream)
+    if (HGW == 1) PW_LAUNCH(1);
+    if (HGW == 2) PW_LAUNCH(2);
+    PW_LAUNCH(4);
+#undef PW_LAUNCH
+  }
+#endif
 #define PF_LAUNCH_P(C, W, P2)                                                                                     \
   attn_prefill_kernel<C, W, P2><<<grid, 4 * W * 64, 0, stream>>>(                                                 \
       (const uint16_t*)q, q_row_stride, (const uint16_t*)k_pages, (const uint16_t*)v_pages, (uint16_t*)out,       \

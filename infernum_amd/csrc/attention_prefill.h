@@ -1,0 +1,391 @@
+// Prompt attention with 32 rows of a query head a wave (part of attention_mfma.hip, for a head size of 128 and two or more query heads
+// to a key/value head).
+//
+// A workgroup takes 64 rows (or, paired, 32 from each end of the request's new tokens) of up to HGW query heads of one key/value
+// head: two waves a head, 32 rows each as two tiles of 16 columns.  Keys and values come in tiles of 64 keys, by loads straight into LDS,
+// into rings of four stages: the keys of tile i + 3 and the values of tile i + 2 are asked for while tile i is worked on, half by
+// half, with one bare barrier a tile.
+//   S^T[key, col] = K[key, :] . Q[col, :]       v_mfma_f32_16x16x32_bf16 over 32 head dims a step
+//   O^T[dim, col] += V^T[dim, key] P^T[key, col] the same over 32 keys a step
+// Row r of the S^T tile t (of a half's two) stands for the key 8 (r / 4) + r % 4 + 4 t of the half, so that the accumulators leave
+// lane (col, q) with the keys 8 q .. 8 q + 7: what the second product wants of the probabilities, and 16 contiguous bytes of a row
+// of V^T, as pages hold it.
+//
+// What bounds it: a SIMD has two such waves, whose matrix instructions take 2,176 cycles a tile, their exponentials and what goes with
+// them some 1,700, and whose reads of LDS (256 KB a tile and compute unit, half of what waves of 16 rows need) 2,048.  These have to run
+// beside each other: a piece of a pair of exponentials of 32 keys' scores stands behind every product of the next 32's scores and every one of the
+// probabilities of the 32 before.  The 8B shape's heads (32 over 8), waves of 16 rows / this kernel, us: 2,048 tokens 69 / 62, 4,096
+// 203 / 162, 8,192 666 / 553 (0.99 PFLOP/s), 2,048 after 6,144 cached 294 / 244; 64 prompts of 120 60 / 68, under a window of
+// 1,024 2,047 tokens of 16 heads over 4 41 / 44 (few tiles a workgroup: its start is longer).  With the products in a row and the exponentials behind them 8,192 tokens
+// took 590.  Heads of 64 gained nothing (2,048 tokens 48 / 54, 8,192 438 / 418), one query head to a key/value head lost (2,000 tokens of 8 heads 53 / 67).
+//
+// In LDS the 16-byte piece c of row r (a key's values; a dim's 64 keys) lies at position c ^ s(r), s(key) = key % 4 + 4 (key / 8 % 2),
+// s(dim) = dim % 8: the 8 lanes that read together find 8 different places.
+#pragma once
+
+#define PW_KT 64                        // keys a tile
+#define PW_STAGES 4
+#define PW_BT 4096                      // block-table entries kept in LDS
+
+typedef const __attribute__((address_space(1))) void* pw_global_ptr;
+typedef __attribute__((address_space(3))) void* pw_lds_ptr;
+
+constexpr int PW_K_BYTES = PW_KT * HD * 2, PW_V_BYTES = VD * PW_KT * 2;
+constexpr int PW_LDS = PW_STAGES * (PW_K_BYTES + PW_V_BYTES) + PW_BT * 4;
+
+typedef f32x4 pw_scores[2][2];          // of 32 keys: [tile of 16][column]
+
+template <int HGW>
+__global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
+    const uint16_t* __restrict__ q, int q_row_stride, const uint16_t* __restrict__ k_pages, const uint16_t* __restrict__ v_pages,
+    uint16_t* __restrict__ out, int out_row_stride, const int* __restrict__ seq_starts, const int* __restrict__ seq_ctx,
+    const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ tiles, int nh, int nkv, int ps_shift, int num_pages,
+    float scale_log2, int window, int paired, const float* __restrict__ sinks) {
+  constexpr int NW = 2 * HGW, THREADS = NW * 64;
+  constexpr int KS = HD / 32;                                           // steps of the scores' product
+  constexpr int KF = PW_K_BYTES / 1024 / NW, VF = PW_V_BYTES / 1024 / NW, LOADS = KF + VF;      // a wave's loads a tile
+  static_assert(HD % 64 == 0 && VD % 64 == 0 && KF >= 1 && VF >= 1, "whole loads for every wave");
+  extern __shared__ __attribute__((aligned(1024))) char pw_lds[];
+  char* const k_lds = pw_lds;
+  char* const v_lds = pw_lds + PW_STAGES * PW_K_BYTES;
+  int* const s_bt = reinterpret_cast<int*>(v_lds + PW_STAGES * PW_V_BYTES);
+  __shared__ int s_poison;
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane & 15, qd = lane >> 4;
+  // waves go to the SIMDs in turn: the row blocks are turned from the fourth wave on, so that every SIMD has waves of both
+  // and those that run out of keys early leave none empty
+  const int hgw = wave >> 1, rblock = (wave ^ (wave >> 2)) & 1;
+  // all heads of the first tile, then of the next (the host lists the tiles with the most keys first)
+  const int lin = blockIdx.y * gridDim.x + blockIdx.x;
+  const int tile = lin / gridDim.y, by = lin - tile * gridDim.y;
+  const int sidx = tiles[2 * tile], row0 = tiles[2 * tile + 1];
+  const int G = nh / nkv, HC = (G + HGW - 1) / HGW;
+  const int g = by / HC, h_in = (by - g * HC) * HGW + hgw;
+  const int h = g * G + (h_in < G ? h_in : 0);
+  const int qstart = seq_starts[sidx], qlen = seq_starts[sidx + 1] - qstart, ctx = seq_ctx[sidx];
+  int rb, first_row, last_row;
+  bool wave_live;
+  if (paired) {
+    const int halves = (qlen + 31) >> 5, ha = row0 >> 6, hb = halves - 1 - ha;      // hb >= ha
+    rb = (rblock == 0 ? ha : hb) * 32;
+    wave_live = rb < qlen && (rblock == 0 || hb > ha);
+    first_row = ha * 32;
+    last_row = (hb * 32 + 32 < qlen ? hb * 32 + 32 : qlen) - 1;
+  } else {
+    rb = row0 + rblock * 32;
+    wave_live = rb < qlen;
+    first_row = row0;
+    last_row = (row0 + 64 < qlen ? row0 + 64 : qlen) - 1;
+  }
+  wave_live = wave_live && h_in < G;
+  if (tid == 0) s_poison = 0;
+
+  // ---- keys: those that the workgroup's rows may see, those that this wave's may
+  const int key_hi = ctx + last_row, key_lo = ia_first_visible_key(ctx + first_row, window);
+  const int wave_last = rb + 31 < qlen ? rb + 31 : qlen - 1;
+  const int wave_hi = ctx + wave_last;
+  const int wave_lo_last = ia_first_visible_key(wave_hi, window);
+  const int t_begin = key_lo / PW_KT, t_end = key_hi / PW_KT;
+  const int w_end = wave_live ? wave_hi / 32 : -1;                      // the wave's last half of a tile
+  {
+    const int* bt = block_tables + (size_t)sidx * bt_stride;
+    const int first = key_lo >> ps_shift, count = (key_hi >> ps_shift) - first + 1;
+    for (int i = tid; i < count; i += THREADS) s_bt[i] = bt[first + i];
+  }
+  const int bt_first = key_lo >> ps_shift, ps = 1 << ps_shift;
+
+  // ---- queries as B operands; columns c = 0, 1 are rows rb + j and rb + 16 + j
+  bf16x8_t qreg[2][KS];
+  float m[2];
+  f32x4 o[NSV][2], lacc[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int row = rb + 16 * c + j;
+    const bool ok = wave_live && row < qlen;
+    const uint16_t* qrow = q + (size_t)(qstart + (ok ? row : first_row)) * q_row_stride + (size_t)h * HD;
+#pragma unroll
+    for (int st = 0; st < KS; ++st) {
+      const uint4 v = *reinterpret_cast<const uint4*>(qrow + st * 32 + qd * 8);
+      qreg[c][st] = __builtin_bit_cast(bf16x8_t, ok ? v : make_uint4(0u, 0u, 0u, 0u));
+    }
+    m[c] = ok ? -INFINITY : 0.f;         // a column without a row never asks for a reference point
+    lacc[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int n = 0; n < NSV; ++n) o[n][c] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  }
+  const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+  const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
+
+  // ---- loads.  A wave brings KG groups of eight keys, KF / KG loads each, and VF loads of 8 dims' 64 keys each, of which a lane
+  // has the same eight every time: eight keys lie in one page.  Groups beyond the range come from the page at its end (scores of theirs are
+  // masked, values zeroed).
+  constexpr int KG = PW_KT / 8 / NW >= 1 ? PW_KT / 8 / NW : 1, KL = KF / KG;
+  static_assert(KG * KL == KF && KG * NW == PW_KT / 8, "whole groups");
+  const uint32_t k_page = (uint32_t)nkv * (uint32_t)ps * (HD * 2), v_page = (uint32_t)nkv * (uint32_t)ps * (VD * 2);     // bytes
+  const char* const k_base = reinterpret_cast<const char*>(k_pages) + (size_t)g * ps * (HD * 2);
+  const char* const v_base = reinterpret_cast<const char*>(v_pages) + (size_t)g * VD * (ps * 2);
+  const int k_row = lane / (HD / 8);
+  // s(key) of the rows of a load: bit 2 is the group's number's lowest bit
+  const uint32_t k_lane_at = (uint32_t)(k_row * HD * 2 + (((lane & (HD / 8 - 1)) ^ (k_row & 3)) * 16));
+  const int v_key = 8 * ((lane & 7) ^ (lane >> 3));
+  const uint32_t v_lane_at = (uint32_t)(8 * wave * VF + (lane >> 3)) * (uint32_t)(ps * 2), v_step = (uint32_t)(16 * ps);
+  const int last_page = (key_hi >> ps_shift) - bt_first;
+  bool bad = false;
+  int k_pg[KG], v_pg;
+  auto page_of = [&](int key) { return s_bt[min(max((key >> ps_shift) - bt_first, 0), last_page)]; };
+  auto pages_of_k = [&](int t) {
+#pragma unroll
+    for (int f = 0; f < KG; ++f) k_pg[f] = page_of(t * PW_KT + 8 * (wave * KG + f));
+  };
+  auto pages_of_v = [&](int t) { v_pg = page_of(t * PW_KT + v_key); };
+  auto load_k = [&](int t, int slot) {
+#pragma unroll
+    for (int f = 0; f < KG; ++f) {
+      const bool ok = (unsigned)k_pg[f] < (unsigned)num_pages;
+      bad |= !ok;
+      const uint32_t in_page = (uint32_t)((t * PW_KT + 8 * (wave * KG + f)) & (ps - 1)) * (HD * 2);
+      const char* src = k_base + ((uint64_t)(uint32_t)(ok ? k_pg[f] : 0) * k_page + (in_page + (k_lane_at ^ (((wave * KG + f) & 1) * 64u))));
+      // a group's loads follow each other in the page and in LDS alike: the instruction's offset moves both
+      char* const dst = k_lds + slot * PW_K_BYTES + 1024 * KL * (wave * KG + f);
+      __builtin_amdgcn_global_load_lds((pw_global_ptr)src, (pw_lds_ptr)dst, 16, 0, 0);
+      if constexpr (KL > 1) __builtin_amdgcn_global_load_lds((pw_global_ptr)src, (pw_lds_ptr)dst, 16, 1024, 0);
+      static_assert(KL <= 2, "a group's loads");
+    }
+  };
+  auto load_v = [&](int t, int slot) {
+    const bool ok = (unsigned)v_pg < (unsigned)num_pages;
+    bad |= !ok;
+    const uint32_t in_page = (uint32_t)((t * PW_KT + v_key) & (ps - 1)) * 2u;
+    const char* src = v_base + ((uint64_t)(uint32_t)(ok ? v_pg : 0) * v_page + (v_lane_at + in_page));
+#pragma unroll
+    for (int f = 0; f < VF; ++f)
+      __builtin_amdgcn_global_load_lds((pw_global_ptr)(src + (uint64_t)(f * v_step)),
+                                       (pw_lds_ptr)(v_lds + slot * PW_V_BYTES + 1024 * (wave * VF + f)), 16, 0, 0);
+  };
+
+  // ---- reads: this lane's row and pieces
+  const int k_lane = (8 * (j >> 2) + (j & 3)) * (HD * 2), v_lane = j * (PW_KT * 2);
+  const int piece0 = (qd ^ (j & 7)) * 16, piece1 = ((4 + qd) ^ (j & 7)) * 16;
+  auto read_k = [&](const char* half, int t, int st) {        // tile t of the half's two, step st of the head dims
+    return *reinterpret_cast<const bf16x8_t*>(half + k_lane + t * (4 * HD * 2) + (st >> 1) * 128 + ((st & 1) ? piece1 : piece0));
+  };
+  // `values`: the stage of the half's tile, with this lane's place in it
+  auto read_v = [&](const char* values, int n) { return *reinterpret_cast<const bf16x8_t*>(values + n * (16 * PW_KT * 2)); };
+
+  typedef uint32_t packed[2][4];        // probabilities as B operands: [column][pairs of keys]
+  float emax[2];
+  // the two exponentials of pair i (of four) of column c of 32 keys' scores, packed
+  auto pair_of = [&](const pw_scores& s, packed& pk, int c, int i, float neg_m) {
+    const int t = i >> 1, r = 2 * (i & 1);
+    const f32x2_t e = {__builtin_amdgcn_exp2f(fmaf(s[t][c][r], scale_log2, neg_m)), __builtin_amdgcn_exp2f(fmaf(s[t][c][r + 1], scale_log2, neg_m))};
+    emax[c] = fmaxf(emax[c], fmaxf(e[0], e[1]));
+    pk[c][i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(e, bf16x2_t));
+  };
+  // keys that a column does not see
+  auto mask = [&](pw_scores& s, int t0) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int row = rb + 16 * c + j, last = row < qlen ? ctx + row : -1, first = ia_first_visible_key(ctx + row, window);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int key = t0 + 8 * qd + 4 * t + r;
+          s[t][c][r] = (key <= last && key >= first) ? s[t][c][r] : -INFINITY;
+        }
+    }
+  };
+  // The reference point of the exponentials follows the running maximum lazily, as in the kernel above: only when an exponential against
+  // it comes out above 2^PF_LAZY, or a column has none yet, it moves, the accumulators are rescaled and the exponentials taken again.
+  auto settle = [&](const pw_scores& s, packed& pk) {
+    if (!__any(emax[0] > PF_LAZY_EXP || emax[1] > PF_LAZY_EXP || m[0] == -INFINITY || m[1] == -INFINITY)) return;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      float top = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) top = fmaxf(top, fmaxf(fmaxf(s[t][c][0], s[t][c][1]), fmaxf(s[t][c][2], s[t][c][3])));
+      top *= scale_log2;                 // (the scale is positive)
+      top = fmaxf(top, __shfl_xor(top, 16, IA_WAVE));
+      top = fmaxf(top, __shfl_xor(top, 32, IA_WAVE));
+      const float m_new = (top > m[c] + PF_LAZY) ? top : m[c];          // never moves to -inf
+      const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
+      const float corr = __builtin_amdgcn_exp2f(m[c] - m_safe);         // 1 where nothing moved, 0 at the start
+      lacc[c] *= corr;
+#pragma unroll
+      for (int n = 0; n < NSV; ++n) o[n][c] *= corr;
+      m[c] = m_new;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) pair_of(s, pk, c, i, -m_safe);
+    }
+  };
+  auto scores = [&](pw_scores& s, const char* half) {
+#pragma unroll
+    for (int x = 0; x < 2 * KS; ++x) {
+      const bf16x8_t a = read_k(half, x & 1, x >> 1);
+      s[x & 1][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qreg[0][x >> 1], x < 2 ? none : s[x & 1][0], 0, 0, 0);
+      s[x & 1][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qreg[1][x >> 1], x < 2 ? none : s[x & 1][1], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);                     // one read's registers at a time
+    }
+  };
+
+  // half x of the keys: its scores `cur` become probabilities `pk`, while the scores of half x + 1 (keys at `half`) come into `next` and
+  // the probabilities `before` of half x - 1 weigh its `values` into the accumulators: three halves' work, none of
+  // which waits for another's.  One path for every half: a wave's first has no probabilities before it (zeros, against values that it
+  // multiplies with anyway), its last no scores behind it (of keys that are there; nobody looks at them), and the one behind that
+  // only probabilities before it.
+  auto part = [&](int x, pw_scores& cur, pw_scores& next, packed& pk, const packed& before, const char* half, const char* values) {
+    if (x > w_end + 1) return;                               // the same for the wave, as all that follows
+    const int t0 = x * 32;
+    if (x <= w_end && ((t0 + 31 > ctx + rb) || (window != 0 && t0 < wave_lo_last) || rb + 31 >= qlen)) mask(cur, t0);
+    const float neg[2] = {(m[0] == -INFINITY) ? 0.f : -m[0], (m[1] == -INFINITY) ? 0.f : -m[1]};
+    emax[0] = emax[1] = 0.f;
+    constexpr int NY = NSV;                                  // turns: a read of keys and one of values, two products each
+    static_assert(2 * KS == NSV, "as many reads of keys as of values");
+    bf16x8_t ak[3], av[3], p[2];
+#pragma unroll
+    for (int y = 0; y < 2; ++y) {
+      ak[y] = read_k(half, y & 1, y >> 1);
+      av[y] = read_v(values, y);
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) p[c] = __builtin_bit_cast(bf16x8_t, make_uint4(before[c][0], before[c][1], before[c][2], before[c][3]));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) lacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, p[c], lacc[c], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int y = 0; y < NY; ++y) {
+      if (y + 2 < NY) {
+        ak[(y + 2) % 3] = read_k(half, (y + 2) & 1, (y + 2) >> 1);
+        av[(y + 2) % 3] = read_v(values, y + 2);
+      }
+      // the turn's pairs of exponentials, a piece behind each of its four products
+      constexpr int PAIRS = 8 / NY;
+      f32x2_t e[PAIRS];
+      auto piece = [&](int stage) {
+#pragma unroll
+        for (int k = 0; k < PAIRS; ++k) {
+          const int i = y * PAIRS + k, c = i >> 2, t = (i >> 1) & 1, r = 2 * (i & 1);
+          if (stage == 0) e[k] = (f32x2_t){fmaf(cur[t][c][r], scale_log2, neg[c]), fmaf(cur[t][c][r + 1], scale_log2, neg[c])};
+          if (stage == 1) e[k][0] = __builtin_amdgcn_exp2f(e[k][0]);
+          if (stage == 2) e[k][1] = __builtin_amdgcn_exp2f(e[k][1]);
+          if (stage == 3) {
+            pk[c][i & 3] = __builtin_bit_cast(uint32_t, __builtin_convertvector(e[k], bf16x2_t));
+            emax[c] = fmaxf(emax[c], fmaxf(e[k][0], e[k][1]));
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        next[y & 1][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ak[y % 3], qreg[c][y >> 1], y < 2 ? none : next[y & 1][c], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        piece(2 * c);
+        o[y][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[y % 3], p[c], o[y][c], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        piece(2 * c + 1);
+      }
+    }
+    if (x <= w_end) settle(cur, pk);
+  };
+  auto barrier = [&] {                  // behind all loads but those of the round before
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LOADS) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
+  // asked for as if by the rounds before: keys of t_begin; keys of the next tile and values of t_begin; keys and values behind those
+  __syncthreads();
+  pages_of_k(t_begin);
+  load_k(t_begin, 0);
+  pages_of_k(t_begin + 1);
+  pages_of_v(t_begin);
+  load_k(t_begin + 1, 1);
+  load_v(t_begin, 0);
+  barrier();
+  pages_of_k(t_begin + 2);
+  pages_of_v(t_begin + 1);
+  load_k(t_begin + 2, 2);
+  load_v(t_begin + 1, 1);
+  pages_of_k(t_begin + 3);
+  pages_of_v(t_begin + 2);
+  pw_scores sa, sb;
+  packed pa, pb;
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    sa[0][c] = sa[1][c] = sb[0][c] = sb[1][c] = none;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) pa[c][i] = pb[c][i] = 0u;
+  }
+  if (wave_live) scores(sa, k_lds);
+  // (one round more where the last keys lie in the second half of their tile: its probabilities weigh in then)
+  const int t_last = t_end + ((key_hi >> 5) & 1);
+  for (int i = t_begin; i <= t_last; ++i) {
+    const int slot = (i - t_begin) & 3;
+    if (i <= t_end) {
+      barrier();                        // keys up to tile i + 1 and values up to tile i are there; nobody reads keys of tile i - 1 or values of i - 2 any more
+      load_k(i + 3, (slot + 3) & 3);    // (past the range: of its last page, for nobody, so that every round has as many loads under way)
+      load_v(i + 2, (slot + 2) & 3);
+      pages_of_k(i + 4);
+      pages_of_v(i + 3);
+    }
+    // values of keys that no row sees are not the request's: zero them in LDS (the tiles at the ends of the range)
+    const int t0 = i * PW_KT;
+    if (i <= t_end && (t0 < key_lo || t0 + PW_KT - 1 > key_hi)) {
+      for (int at = tid; at < VD * 8; at += THREADS) {
+        const int dim = at >> 3, key = t0 + 8 * ((at & 7) ^ (dim & 7));
+        if (key >= key_lo && key + 7 <= key_hi) continue;
+        uint16_t* const v = reinterpret_cast<uint16_t*>(v_lds + slot * PW_V_BYTES + at * 16);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (key + e < key_lo || key + e > key_hi) v[e] = 0;
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
+    const char* const here = v_lds + slot * PW_V_BYTES + v_lane + piece0;
+    part(2 * i, sa, sb, pa, pb, k_lds + slot * PW_K_BYTES + 32 * HD * 2,
+         i == t_begin ? here : v_lds + ((slot + 3) & 3) * PW_V_BYTES + v_lane + piece1);
+    part(2 * i + 1, sb, sa, pb, pa, k_lds + ((slot + 1) & 3) * PW_K_BYTES, here);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the loads asked for past the end
+  if (bad) s_poison = 1;      // a key that is needed has no page in the block table: the result is NaN
+  __syncthreads();
+  const bool poison = s_poison != 0;
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    if (!wave_live || rb + 16 * c + j >= qlen) continue;
+    float lsum = lacc[c][0];
+    if (sinks) lsum += exp2f(sinks[h] * 1.4426950408889634f - m[c]);
+    const float inv = poison ? __uint_as_float(0x7fc00000u) : 1.0f / lsum;
+    uint16_t* const orow = out + (size_t)(qstart + rb + 16 * c + j) * out_row_stride + (size_t)h * VD + 4 * qd;
+#pragma unroll
+    for (int n = 0; n < NSV; ++n) {
+      uint2 w;
+      w.x = (uint32_t)float_to_bf16_bits(o[n][c][0] * inv) | ((uint32_t)float_to_bf16_bits(o[n][c][1] * inv) << 16);
+      w.y = (uint32_t)float_to_bf16_bits(o[n][c][2] * inv) | ((uint32_t)float_to_bf16_bits(o[n][c][3] * inv) << 16);
+      *reinterpret_cast<uint2*>(orow + n * 16) = w;
+    }
+  }
+}
+
+template <int HGW>
+static int launch_prefill_wide(dim3 grid, const void* q, int q_row_stride, const void* k_pages, const void* v_pages, void* out,
+                               int out_row_stride, const int* seq_starts, const int* seq_ctx, const int* block_tables, int bt_stride,
+                               const int* tiles, int nh, int nkv, int ps, int num_pages, float scale_log2, int window, int paired,
+                               const float* sinks, hipStream_t stream) {
+  static bool configured = false;
+  if (!configured) {
+    const hipError_t e = hipFuncSetAttribute((const void*)attn_prefill_wide_kernel<HGW>, hipFuncAttributeMaxDynamicSharedMemorySize, PW_LDS);
+    if (e != hipSuccess) return (int)e;
+    configured = true;
+  }
+  int shift = 0;
+  while ((1 << shift) < ps) ++shift;
+  attn_prefill_wide_kernel<HGW><<<grid, HGW * 128, PW_LDS, stream>>>(
+      (const uint16_t*)q, q_row_stride, (const uint16_t*)k_pages, (const uint16_t*)v_pages, (uint16_t*)out, out_row_stride, seq_starts,
+      seq_ctx, block_tables, bt_stride, tiles, nh, nkv, shift, num_pages, scale_log2, window, paired, sinks);
+  IA_LAUNCH_CHECK();
+  return IA_OK;
+}

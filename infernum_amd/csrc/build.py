@@ -57,7 +57,7 @@ CORE_SOURCES = [
     "sampling.hip",
     "peaks.hip",
 ]
-HEADERS = ["common.h", "no_alloc.h", "op_call.h", "parts_join.h", "tile_fma.h"]
+HEADERS = ["attention_prefill.h", "common.h", "no_alloc.h", "op_call.h", "parts_join.h", "tile_fma.h"]
 # The host library: plain C++ (cache bookkeeping, packing of a step), built with the C++ compiler.
 HOST_SOURCES = ["host_core.cpp", "step_program.cpp"]
 CXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall"]

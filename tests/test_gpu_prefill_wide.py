@@ -1,0 +1,119 @@
+"""Prompt attention with 32 rows of a head a wave (csrc/attention_prefill.h) at the edges of its tiles, against the plain kernel and
+plain attention in 64 bits."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+D = 128
+
+
+def K():
+    from infernum_amd.kernels import api
+    return api
+
+
+def _case(nh, nkv, ps, lens, q_lens, seed, cols=None, poison=True):
+    """Requests of lens keys whose last q_lens tokens are new, pages in a shuffled order; what no request holds is NaN."""
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    rnd = lambda *s: torch.randn(*s, device=DEV, generator=g).to(torch.bfloat16)                     # noqa: E731
+    counts = [-(-n // ps) for n in lens]
+    P = sum(counts) + 2
+    order = torch.randperm(P - 1, device=DEV, generator=g).int() + 1
+    bt = torch.full((len(lens), cols or max(counts)), 0, dtype=torch.int32, device=DEV)
+    kp = torch.full((P, nkv, ps, D), float("nan") if poison else 0.0, dtype=torch.bfloat16, device=DEV)
+    vp = torch.full((P, nkv, D, ps), float("nan") if poison else 0.0, dtype=torch.bfloat16, device=DEV)
+    k = [rnd(n, nkv, D) for n in lens]
+    v = [rnd(n, nkv, D) for n in lens]
+    at = 0
+    for i, n in enumerate(lens):
+        bt[i, :counts[i]] = order[at:at + counts[i]]
+        at += counts[i]
+        for p in range(counts[i]):
+            page, a, b = int(bt[i, p]), p * ps, min(n, p * ps + ps)
+            kp[page, :, :b - a] = k[i][a:b].transpose(0, 1)
+            vp[page, :, :, :b - a] = v[i][a:b].permute(1, 2, 0)
+    q = rnd(sum(q_lens), nh * D)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)                                   # noqa: E731
+    starts = i32([sum(q_lens[:i]) for i in range(len(q_lens) + 1)])
+    ctx = i32([a - b for a, b in zip(lens, q_lens)])
+    tiles = i32([(s, r) for s in range(len(lens)) for r in range(0, q_lens[s], 64)]).reshape(-1, 2)
+    return dict(q=q, k=k, v=v, kp=kp, vp=vp, bt=bt, starts=starts, ctx=ctx, tiles=tiles, lens=lens, q_lens=q_lens)
+
+
+def _run(c, nh, nkv, window=0, **kw):
+    out = torch.full_like(c["q"], float("nan"))
+    K().attention_prefill(c["q"], c["kp"], c["vp"], out, c["starts"], c["ctx"], c["bt"], c["tiles"], c["tiles"].shape[0], nh, nkv, D,
+                          D ** -0.5, window, **kw)
+    return out
+
+
+def _want(c, nh, nkv, window):
+    rows, at = [], 0
+    for k, v, n, m in zip(c["k"], c["v"], c["lens"], c["q_lens"]):
+        q = c["q"][at:at + m].view(m, nh, D).double()
+        at += m
+        pos, key = torch.arange(n - m, n, device=DEV)[:, None], torch.arange(n, device=DEV)[None, :]
+        seen = (key <= pos) & ((key > pos - window) if window else (key >= 0))
+        for_heads = lambda t: t.double().repeat_interleave(nh // nkv, dim=1)                         # noqa: E731
+        s = torch.einsum("qhd,khd->hqk", q, for_heads(k)) * D ** -0.5
+        p = torch.softmax(s.masked_fill(~seen, -math.inf), dim=-1)
+        rows.append(torch.einsum("hqk,khd->qhd", p, for_heads(v)).reshape(m, nh * D))
+    return torch.cat(rows)
+
+
+@pytest.mark.parametrize("nh,nkv,ps", [(4, 1, 16), (6, 2, 8), (4, 2, 64), (14, 2, 32), (8, 2, 128)])
+@pytest.mark.parametrize("lens,q_lens", [([1, 2, 31, 32, 33], [1, 2, 31, 32, 33]), ([63, 64, 65, 127, 129], [63, 64, 65, 127, 129]),
+                                         ([95, 96, 97, 200, 161], [1, 33, 65, 64, 7]), ([300, 449], [300, 100])])
+@pytest.mark.parametrize("window", [0, 1, 40, 100])
+def test_edges_of_tiles(nh, nkv, ps, lens, q_lens, window):
+    c = _case(nh, nkv, ps, lens, q_lens, seed=nh * ps + len(lens) + window)
+    out = _run(c, nh, nkv, window)
+    # probabilities within 2^-9 of themselves (their sum is taken of the rounded ones), values of order one, one rounding to bf16
+    err = (out.double() - _want(c, nh, nkv, window)).abs().max().item()
+    assert err <= 2.5e-2, err
+    for hpw in (1, 2, 4):
+        for paired in (False, True):
+            assert torch.equal(_run(c, nh, nkv, window, heads_per_workgroup=hpw, paired=paired), out), (hpw, paired)
+    # a wide block table takes the kernel with 16 rows a wave: as near
+    wide = _case(nh, nkv, ps, lens, q_lens, seed=nh * ps + len(lens) + window, cols=4097)
+    assert ((_run(wide, nh, nkv, window).double() - out.double()).abs().max().item()) <= 2.5e-2
+
+
+def test_whole_and_in_portions_the_same_bits():
+    nh, nkv, ps, n = 8, 2, 16, 333
+    whole = _case(nh, nkv, ps, [n], [n], seed=3)
+    want = _run(whole, nh, nkv)
+    for a, b in ((0, 64), (64, 100), (100, 333), (31, 32), (200, 333)):
+        part = dict(whole, q=whole["q"][a:b].clone(), lens=[b], q_lens=[b - a], ctx=torch.tensor([a], dtype=torch.int32, device=DEV),
+                    starts=torch.tensor([0, b - a], dtype=torch.int32, device=DEV),
+                    tiles=torch.tensor([(0, r) for r in range(0, b - a, 64)], dtype=torch.int32, device=DEV).reshape(-1, 2))
+        assert torch.equal(_run(part, nh, nkv), want[a:b]), (a, b)
+
+
+def test_a_later_token_that_is_not_finite_stays_out_of_the_rows_before_it():
+    """Keys and values of a token are read by workgroups whose earlier rows do not see it."""
+    nh, nkv, ps, n = 4, 1, 16, 200
+    for bad in (float("inf"), float("nan")):
+        c = _case(nh, nkv, ps, [n], [n], seed=4)
+        want = _run(c, nh, nkv)
+        t = 170                                                         # its half of a tile begins at key 160
+        page = int(c["bt"][0, t // ps])
+        c["kp"][page, :, t % ps] = bad
+        got = _run(c, nh, nkv)
+        assert torch.equal(got[:t], want[:t])
+        c["vp"][page, :, :, t % ps] = bad
+        got = _run(c, nh, nkv)
+        assert torch.equal(got[:160], want[:160]) and not bool(got[t:].isfinite().all())
+
+
+def test_a_key_without_a_page_gives_nan():
+    nh, nkv, ps = 4, 1, 16
+    c = _case(nh, nkv, ps, [100, 64], [100, 64], seed=5)
+    c["bt"][0, 2] = -1
+    out = _run(c, nh, nkv)
+    assert bool(out[64:100].isnan().all()) and bool(out[100:].isfinite().all())
+    c["bt"][0, 2] = 10 ** 6
+    assert bool(_run(c, nh, nkv)[64:100].isnan().all())
