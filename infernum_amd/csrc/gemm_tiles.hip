@@ -40,6 +40,7 @@
 // keep: operands come from LDS reads, for which the compiler waits, and from nothing else (no vector instruction writes one: tests
 // read the loop's assembly for moves), and the accumulators are written before and read after with a wait between.
 #include "common.h"
+#include <cmath>
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -67,8 +68,11 @@ typedef __attribute__((address_space(3))) void* gt_lds_ptr;
     else GT_FETCH_AT(rsrc, lds, at, step, 3072);                    \
   } while (0)
 
-template <int TX0, int TX1, int TW0, int TW1, bool GLU>
+enum { GT_PLAIN, GT_GLU, GT_GROUPED };
+
+template <int TX0, int TX1, int TW0, int TW1, int MODE>
 struct GemmTile {
+  static constexpr bool GLU = MODE == GT_GLU;
   static constexpr int BM = 32 * (TX0 + TX1), BN = 32 * (TW0 + TW1);      // rows of X and of W
   static constexpr int COLS = GLU ? BN / 2 : BN;                          // columns of the result
   static constexpr int STAGE = (BM + BN) * GT_ROW;
@@ -106,10 +110,12 @@ struct GemmTile {
     __builtin_amdgcn_sched_barrier(0);                                                                         \
   }
 
-template <int TX0, int TX1, int TW0, int TW1, bool GLU>
+template <int TX0, int TX1, int TW0, int TW1, int MODE>
 __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W,
-                                                            uint16_t* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n) {
-  using T = GemmTile<TX0, TX1, TW0, TW1, GLU>;
+                                                            uint16_t* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n,
+                                                            const int* __restrict__ rows_at, int groups) {
+  using T = GemmTile<TX0, TX1, TW0, TW1, MODE>;
+  constexpr bool GLU = T::GLU, GROUPED = MODE == GT_GROUPED;
   constexpr int BM = T::BM, BN = T::BN, WM = BM / 2, WN = BN / 2, STAGE = T::STAGE;
   constexpr int RX0 = 0, RX1 = 32 * TX0, RW0 = BM, RW1 = BM + 32 * TW0;       // a step's half-tiles, in rows of its stage
   constexpr int ALL = TX0 + TX1 + TW0 + TW1;                                  // a wave's loads a step
@@ -117,24 +123,51 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const uint16_t* __re
 
   // workgroups go to the 8 dies in turn (workgroup i to die i % 8), and each die has an L2 of its own: every die gets one
   // contiguous run of tiles, four tiles of M under one tile of N at a time
+  if constexpr (GROUPED) {
+    // the tiles of rows that the groups have in this step (the launch has one for every case): the dies share those evenly,
+    // and the workgroups beyond them leave
+    tiles_m = 0;
+    for (int g = 0; g < groups; ++g) tiles_m += (rows_at[g + 1] - rows_at[g] + BM - 1) / BM;
+  }
   const int total = tiles_m * tiles_n, xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
+  if (GROUPED && idx >= (total >> 3) + (xcd < (total & 7) ? 1 : 0)) return;
   const int bid = xcd * (total >> 3) + min(xcd, total & 7) + idx;
   constexpr int GROUP = 4;
   const int group = bid / (GROUP * tiles_n), in_group = bid - group * (GROUP * tiles_n);
   const int group_rows = min(GROUP, tiles_m - group * GROUP);
-  const int m0 = (group * GROUP + in_group % group_rows) * BM, tn = in_group / group_rows;
+  const int tm = group * GROUP + in_group % group_rows, tn = in_group / group_rows;
+  const int m0 = GROUPED ? 0 : tm * BM;
   const int NO = GLU ? N / 2 : N, n0 = tn * T::COLS;                          // columns of the result
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1, r16 = lane & 15, q4 = lane >> 4;
 
+  // GROUPED: the tile's group, its first row among the sorted ones; from here on M is what the group has from there on
+  int rot = 0;
+  if constexpr (GROUPED) {
+    int g = 0, seen = 0;
+    for (; g < groups - 1; ++g) {
+      const int t = (rows_at[g + 1] - rows_at[g] + BM - 1) / BM;
+      if (tm < seen + t) break;
+      seen += t;
+    }
+    const int first = rows_at[g] + (tm - seen) * BM;
+    M = rows_at[g + 1] - first;
+    W += ((size_t)g * N + n0) * K;
+    X += (size_t)first * K;
+    C += (size_t)first * N;
+    static_assert(!GROUPED || 512 % BN == 0, "a tile lies in the columns that share a start");
+    rot = ia_expert_first_chunk(n0, K) * (IA_EXPERT_CHUNK / GT_BK);
+  }
+
   // ---- loads: load f of a half-tile of 32 T rows fills its rows 8 (T wave + f) .. + 7, this lane position lane % 8 of row
   // lane / 8 of them.  The half-tile's first 16 T rows belong to the waves with wm (wn) 0, the others to those with 1.
-  const auto x_all = GT_BUFFER(reinterpret_cast<const char*>(X) - GT_AHEAD, (unsigned)M * (unsigned)K * 2u + GT_AHEAD);
-  const auto w_all = GT_BUFFER(reinterpret_cast<const char*>(W) - GT_AHEAD, (unsigned)N * (unsigned)K * 2u + GT_AHEAD);
-  auto place = [&](int t, int f, int first, int apart, int rows, int behind) {
+  const int x_rows = GROUPED ? min(M, BM) : M, w_rows = GROUPED ? min(N - n0, BN) : N;
+  const auto x_all = GT_BUFFER(reinterpret_cast<const char*>(X) - GT_AHEAD, (unsigned)x_rows * (unsigned)K * 2u + GT_AHEAD);
+  const auto w_all = GT_BUFFER(reinterpret_cast<const char*>(W) - GT_AHEAD, (unsigned)w_rows * (unsigned)K * 2u + GT_AHEAD);
+  auto place = [&](int t, int f, int from, int apart, int rows, int behind) {
     const int row = 8 * (t * wave + f) + (lane >> 3), of = row / (16 * t), in = row - of * (16 * t);
-    const uint32_t r = (uint32_t)(min(first + of * apart + in, rows - 1) + behind);
+    const uint32_t r = (uint32_t)(min(from + of * apart + in, rows - 1) + behind);
     return GT_AHEAD - 1024u * (uint32_t)f + (r * (uint32_t)K + (uint32_t)(((lane & 7) ^ (row & 7)) * 8)) * 2u;
   };
   uint32_t sx0[TX0], sx1[TX1], sw0[TW0], sw1[TW1];
@@ -144,15 +177,22 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const uint16_t* __re
   for (int f = 0; f < TX1; ++f) sx1[f] = place(TX1, f, m0 + 16 * TX0, WM, M, 0);
   // GLU: the first half of a wave's rows of W is of the first half of the matrix, the second of the second, for the same columns
 #pragma unroll
-  for (int f = 0; f < TW0; ++f) sw0[f] = place(TW0, f, n0, GLU ? WN / 2 : WN, NO, 0);
+  for (int f = 0; f < TW0; ++f) sw0[f] = place(TW0, f, GROUPED ? 0 : n0, GLU ? WN / 2 : WN, GROUPED ? w_rows : NO, 0);
 #pragma unroll
-  for (int f = 0; f < TW1; ++f) sw1[f] = GLU ? place(TW1, f, n0, WN / 2, NO, NO) : place(TW1, f, n0 + 16 * TW0, WN, NO, 0);
+  for (int f = 0; f < TW1; ++f)
+    sw1[f] = GLU ? place(TW1, f, n0, WN / 2, NO, NO)
+                 : place(TW1, f, (GROUPED ? 0 : n0) + 16 * TW0, WN, GROUPED ? w_rows : NO, 0);
   const int steps = K / GT_BK;
-  // past the end the last step is fetched again, into memory that is not read any more
-#define GT_X0(t, f) GT_FETCH(x_all, lds + ((t) & 1) * STAGE + RX0 * GT_ROW + 1024 * (TX0 * wave), sx0[f], min(t, steps - 1) * GT_ROW, f)
-#define GT_X1(t, f) GT_FETCH(x_all, lds + ((t) & 1) * STAGE + RX1 * GT_ROW + 1024 * (TX1 * wave), sx1[f], min(t, steps - 1) * GT_ROW, f)
-#define GT_W0(t, f) GT_FETCH(w_all, lds + ((t) & 1) * STAGE + RW0 * GT_ROW + 1024 * (TW0 * wave), sw0[f], min(t, steps - 1) * GT_ROW, f)
-#define GT_W1(t, f) GT_FETCH(w_all, lds + ((t) & 1) * STAGE + RW1 * GT_ROW + 1024 * (TW1 * wave), sw1[f], min(t, steps - 1) * GT_ROW, f)
+  // past the end the last step is fetched again, into memory that is not read any more; GROUPED: the walk begins at step
+  // rot and wraps around
+  auto step_at = [&](int t) {
+    const int k = min(t, steps - 1) + rot;
+    return (GROUPED && k >= steps ? k - steps : k) * GT_ROW;
+  };
+#define GT_X0(t, f) GT_FETCH(x_all, lds + ((t) & 1) * STAGE + RX0 * GT_ROW + 1024 * (TX0 * wave), sx0[f], step_at(t), f)
+#define GT_X1(t, f) GT_FETCH(x_all, lds + ((t) & 1) * STAGE + RX1 * GT_ROW + 1024 * (TX1 * wave), sx1[f], step_at(t), f)
+#define GT_W0(t, f) GT_FETCH(w_all, lds + ((t) & 1) * STAGE + RW0 * GT_ROW + 1024 * (TW0 * wave), sw0[f], step_at(t), f)
+#define GT_W1(t, f) GT_FETCH(w_all, lds + ((t) & 1) * STAGE + RW1 * GT_ROW + 1024 * (TW1 * wave), sw1[f], step_at(t), f)
 
   // ---- accumulators of the quadrants, W the first operand: register e of lane (r, q) of tile [i][j] is the product for
   // n = 16 i + 4 q + e and m = 16 j + r, four neighbours in a row of C
@@ -220,10 +260,14 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const uint16_t* __re
     step(t + 1, wb, wa);
   }
   if (t < steps) step(t, wa, wb);
-  // the loads asked for past the end write LDS too; and the last products are through
+  // the loads asked for past the end write LDS too; and the last products are through before an accumulator is read
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#define GT_KEEP(a, I, J)                        \
+  _Pragma("unroll") for (int i = 0; i < I; ++i) \
+  _Pragma("unroll") for (int j = 0; j < J; ++j) asm volatile("" : "+a"(a[i][j]));
+  GT_KEEP(a00, TW0, TX0) GT_KEEP(a10, TW1, TX0) GT_KEEP(a11, TW1, TX1) GT_KEEP(a01, TW0, TX1)
 
   // ---- C through LDS, a region of its own for every wave, so that rows leave as consecutive 16-byte pieces
   char* const region = lds + wave * (WM * T::OUT_ROW);
@@ -279,19 +323,22 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const uint16_t* __re
   }
 }
 
-template <int TX0, int TX1, int TW0, int TW1, bool GLU>
-static int launch_gemm_tiles(const uint16_t* x, const uint16_t* w, uint16_t* c, int M, int N, int K, hipStream_t stream) {
-  using T = GemmTile<TX0, TX1, TW0, TW1, GLU>;
+template <int TX0, int TX1, int TW0, int TW1, int MODE>
+static int launch_gemm_tiles(const uint16_t* x, const uint16_t* w, uint16_t* c, int M, int N, int K, const int* rows_at,
+                             int groups, hipStream_t stream) {
+  using T = GemmTile<TX0, TX1, TW0, TW1, MODE>;
   static bool configured = false;
   if (!configured) {
-    const hipError_t e = hipFuncSetAttribute((const void*)gemm_tiles_kernel<TX0, TX1, TW0, TW1, GLU>,
+    const hipError_t e = hipFuncSetAttribute((const void*)gemm_tiles_kernel<TX0, TX1, TW0, TW1, MODE>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS);
     if (e != hipSuccess) return (int)e;
     configured = true;
   }
-  const int tiles_m = (M + T::BM - 1) / T::BM, tiles_n = ((GLU ? N / 2 : N) + T::COLS - 1) / T::COLS;
+  // grouped: a tile for every way the rows can fall into groups
+  const int tiles_m = MODE == GT_GROUPED ? M / T::BM + (M < groups ? M : groups) : (M + T::BM - 1) / T::BM;
+  const int tiles_n = ((T::GLU ? N / 2 : N) + T::COLS - 1) / T::COLS;
   if ((long long)tiles_m * tiles_n > 0x7fffffffLL) return IA_ERR_UNSUPPORTED;
-  gemm_tiles_kernel<TX0, TX1, TW0, TW1, GLU><<<tiles_m * tiles_n, 256, T::LDS, stream>>>(x, w, c, M, N, K, tiles_m, tiles_n);
+  gemm_tiles_kernel<TX0, TX1, TW0, TW1, MODE><<<tiles_m * tiles_n, 256, T::LDS, stream>>>(x, w, c, M, N, K, tiles_m, tiles_n, rows_at, groups);
   IA_LAUNCH_CHECK();
   return IA_OK;
 }
@@ -363,14 +410,64 @@ extern "C" int ia_gemm_tiles(const void* X, const void* W, void* C, int M, int N
   if (rows <= 0) choose_tile(M, N, K, glu != 0, rows, cols);
 #define GT_ONE(BM, BN, TX0, TX1, TW0, TW1)                                                                        \
   if (rows == BM && cols == BN) {                                                                                 \
-    if (!glu) return launch_gemm_tiles<TX0, TX1, TW0, TW1, false>(x, w, c, M, N, K, stream);                      \
-    if constexpr (TW0 == TW1) return launch_gemm_tiles<TX0, TX1, TW0, TW1, true>(x, w, c, M, N, K, stream);       \
+    if (!glu) return launch_gemm_tiles<TX0, TX1, TW0, TW1, GT_PLAIN>(x, w, c, M, N, K, nullptr, 0, stream);                      \
+    if constexpr (TW0 == TW1) return launch_gemm_tiles<TX0, TX1, TW0, TW1, GT_GLU>(x, w, c, M, N, K, nullptr, 0, stream);       \
   }
   GT_TILES(GT_ONE)
 #undef GT_ONE
   return IA_ERR_BAD_ARG;
 }
 
+// ---- rows in groups, each with a matrix of its own: the routed experts' products of many tokens ----
+// Rows rows_at[g] .. rows_at[g + 1] - 1 of X (sorted by group) times matrix g of W [groups, N, K]; rows_at [groups + 1] lies on the device
+// and nothing is read back: the launch has a workgroup for every way the rows can fall into groups, and those to spare leave.  The walk
+// over K starts where the tiles of few pairs do (ia_expert_first_chunk) and wraps: the same bits from either.  among: how many groups the
+// rows are spread over, with those that have no matrix and lie behind the others (the choice of a tile goes by it).
+//
+// What bounds it: between the stream of the experts' weights and the matrix cores, and the turns of the compute units that tiles fill in
+// part.  First / second products, us, with the tiles of 128 x 256 of 32 x 32 x 16 instructions before and now:
+//   20 experts of 2,432 x 4,096, 161 rows each 243 -> 219 / 140 -> 111   32 of 1,408 x 2,048, 255 rows 165 -> 136 / 97 -> 73
+//   16 of 1,408 x 2,048, 256 rows 79 -> 71 / 53 -> 33                    8 of 2,752 x 2,048 without a gate, 500 rows 66 -> 61 / 81 -> 52
+
+// How many rows the tiles of `rows` rows multiply for groups whose sizes differ as those of a random choice do.
+static long grouped_rows(int groups, int mean, int rows) {
+  const double spread = std::sqrt((double)mean);
+  long tiles = 0;
+  for (const double d : {-1.2, -0.5, 0.0, 0.5, 1.2}) {
+    const int n = (int)(mean + d * spread);
+    tiles += ((n < 1 ? 1 : n) + rows - 1) / rows;
+  }
+  return tiles * groups * rows;
+}
+
+// Which tile: of 160 x 128 and 192 x 128, two of which share a compute unit, the one that multiplies fewer rows in all (255 rows of
+// 1,408 x 2,048 136 / 140 us, 340 of 2,432 x 4,096 400 / 290, 512 of 1,408 x 2,048 262 / 220).  96 x 128 up to 90 rows (75 rows of
+// 1,408 x 2,048 90 us, 94 with 160 x 128; 100 rows of 2,432 x 4,096 233 / 164) and where 160 x 128 would not give every unit one
+// (16 of 1,408 x 2,048 with 150 rows 25 / 33), and of these 96 x 256 where that turns more tiles than units into fewer (16 of 1,408 x 2,048
+// with 75 rows 48 / 43).  Over 38 products of 49 to 1,024 rows this takes 2.6 % longer than the fastest of ten tiles.
+extern "C" int ia_gemm_tiles_grouped(const void* X, const void* W, void* C, const int* rows_at, int groups, int among, int rows, int N, int K,
+                                     hipStream_t stream) {
+  if (groups <= 0 || among < groups || !rows_at) return IA_ERR_BAD_ARG;
+  if (rows == 0) return IA_OK;
+  if (rows < 0 || N <= 0 || K <= 0 || K % GT_BK != 0) return IA_ERR_UNSUPPORTED;
+  // rows are addressed with 32 bits from the tile's first on, whose GT_AHEAD bytes in front are within reach of 256 rows
+  if ((unsigned long long)rows * K * 2 > 0xffffffffULL || (unsigned long long)N * K * 2 > 0xffffffffULL) return IA_ERR_UNSUPPORTED;
+  if (256ULL * K * 2 > 0xffffffffULL - GT_AHEAD) return IA_ERR_UNSUPPORTED;
+  const uint16_t *x = (const uint16_t*)X, *w = (const uint16_t*)W;
+  uint16_t* c = (uint16_t*)C;
+  const int mean = rows / among;
+  const long long strips = (N + 127) / 128, of_96 = (mean + 95) / 96, of_160 = (mean + 159) / 160;
+  if (mean <= 90 || groups * of_160 * strips <= 256) {
+    if (groups * of_96 * strips > 256 && groups * of_96 * ((N + 255) / 256) <= 256)
+      return launch_gemm_tiles<2, 1, 4, 4, GT_GROUPED>(x, w, c, rows, N, K, rows_at, groups, stream);
+    return launch_gemm_tiles<2, 1, 2, 2, GT_GROUPED>(x, w, c, rows, N, K, rows_at, groups, stream);
+  }
+  if (grouped_rows(groups, mean, 160) < grouped_rows(groups, mean, 192))
+    return launch_gemm_tiles<3, 2, 2, 2, GT_GROUPED>(x, w, c, rows, N, K, rows_at, groups, stream);
+  return launch_gemm_tiles<3, 3, 2, 2, GT_GROUPED>(x, w, c, rows, N, K, rows_at, groups, stream);
+}
+
 // ---- the launchers of this file as operations of a step's program (see op_call.h) ----
 #include "op_call.h"
 IA_OP(ia_gemm_tiles)
+IA_OP(ia_gemm_tiles_grouped)

@@ -261,7 +261,7 @@ __global__ __launch_bounds__(256) void moe_gate_up_kernel(const T* __restrict__ 
 // consecutive columns 4 q .. 4 q + 3 of row r of the result.
 // All workgroups walking K in step read places one row's length apart at the same moment, and where that length is a power
 // of two those lie on few memory channels, so every 512 columns start their walk at a chunk of their own (ia_expert_first_chunk) and
-// wrap around.  The tile of 128 pairs and the grouped product of gemm_mfma.hip start there too: an element is one chain over K in
+// wrap around.  The tile of 128 pairs and the grouped product of gemm_tiles.hip start there too: an element is one chain over K in
 // an order that depends on K and its column alone.
 // Before, tiles of 32 x 128 in steps of 64 through one LDS stage and all walks from the same start (cold weights,
 // gate and up / down, microseconds before and now): 4 of 32 experts of 1,408 x 2,048 22.0 / 15.9 and 12.4 / 7.2; 16 of 16, 32
@@ -584,7 +584,7 @@ extern "C" int ia_moe_down(const void* y, const void* Wd, float* parts, const fl
   return IA_OK;
 }
 
-// ---- the experts of a step of many rows by the grouped form of the LDS-tiled product (ia_gemm_mfma_grouped) ----------
+// ---- the experts of a step of many rows by the grouped form of the LDS-tiled product (ia_gemm_tiles_grouped) ----------
 // The tokens' rows are first brought into the order of the sort (an expert's rows one after the other), the two
 // products run expert by expert over those rows, and the activation and the routing weight are passes of their own:
 //   ia_moe_gather   xs[p, :] = x[perm[p] / top, :]

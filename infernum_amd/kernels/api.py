@@ -332,10 +332,12 @@ def router_topk(logits: torch.Tensor, bias: Optional[torch.Tensor], top: int):
     return ids, weights
 
 
-def gemm_mfma_grouped(x: torch.Tensor, w: torch.Tensor, rows_at: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+def gemm_mfma_grouped(x: torch.Tensor, w: torch.Tensor, rows_at: torch.Tensor, out: Optional[torch.Tensor] = None,
+                      among: int = 0) -> torch.Tensor:
     """out[rows_at[g] : rows_at[g + 1]] = x[rows_at[g] : rows_at[g + 1]] @ w[g]^T for every group g: x [rows, K] and
     w [groups, N, K] in bf16, rows_at int32 [groups + 1] on the device, rising from 0 to at most rows (nothing of it
-    is read on the host; rows past rows_at[-1] are left as they are).  K must be a multiple of 64."""
+    is read on the host; rows past rows_at[-1] are left as they are).  K must be a multiple of 64.  ``among``: how many groups the
+    rows are spread over, with those behind the last of w (the choice of a tile goes by it; 0: those of w)."""
     _dev(x, w, rows_at, out)
     _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == 2 and w.dim() == 3
           and w.shape[2] == x.shape[1], "gemm_mfma_grouped: x [rows, K] and w [groups, N, K] in bf16")
@@ -344,7 +346,7 @@ def gemm_mfma_grouped(x: torch.Tensor, w: torch.Tensor, rows_at: torch.Tensor, o
     if out is None:
         out = torch.empty((x.shape[0], N), dtype=torch.bfloat16, device=x.device)
     _need(out.dtype == torch.bfloat16 and tuple(out.shape) == (x.shape[0], N), "gemm_mfma_grouped: out [rows, N] in bf16")
-    _ok(_core().ia_gemm_mfma_grouped(_p(x), _p(w), _p(out), _p(rows_at), G, x.shape[0], N, Kd, _stream()),
+    _ok(_core().ia_gemm_tiles_grouped(_p(x), _p(w), _p(out), _p(rows_at), G, max(int(among), G), x.shape[0], N, Kd, _stream()),
         "gemm_mfma_grouped")
     return out
 
@@ -382,13 +384,12 @@ def moe_route(logits, bias: Optional[torch.Tensor], top: int, experts: int, soft
 
 
 # From how many rows an expert on average the grouped form is ahead of the tiles behind the sort: sort to scatter, microseconds of
-# grouped / tiles with cold weights.  Gated: 32 experts of 1,408 x 2,048 at 64 / 112 / 128 rows 173 / 173, 193 / 192, 233 / 276; 64 of them
-# 319 / 308, 392 / 372, 446 / 450; 8 of 2,752 x 2,048 104 / 100, 116 / 104, 149 / 173; 4 of 4,800 x 4,096 161 / 163, 175 / 163, 179 / 204.
-# Without a gate: 8 of 4,800 x 4,096 at 48 / 56 / 64 rows 172 / 164, 174 / 169, 177 / 220.
+# grouped / tiles with cold weights.  Gated: 32 experts of 1,408 x 2,048 at 48 / 64 / 96 / 112 / 128 rows 150 / 142, 158 / 173, 177 / 183,
+# 187 / 221, 190 / 269; 64 of them 289 / 277, 305 / 301, 345 / 337, 356 / 360, 366 / 420.  Without a gate, at 48 / 64 / 96 rows: 8 of
+# 2,752 x 2,048 72 / 61, 74 / 86, 86 / 92; 16 of 1,408 x 2,048 70 / 62, 71 / 81, 97 / 104.
 # The passes around the grouped products (rows in the order of the sort, activation, scatter) take rows times (W + ff), the products rows
-# times W ff; where those weigh little and the tiles of 128 x 256 that the experts then have fill the chip, gated ones change over sooner: at
-# 48 / 56 / 64 / 112 rows 20 of 2,432 x 4,096 297 / 274, 306 / 335, 310 / 342, 333 / 381; 8 of 4,800 x 4,096 253 / 207, 257 / 260, 260 / 307,
-# 281 / 318; 8 of 14,336 x 4,096 621 / 536, 627 / 617, 635 / 726, 684 / 735; 8 of 8,192 x 5,120 412 / 448, 415 / 466, 423 / 467, 452 / 504.
+# times W ff; where those weigh little and the experts' columns fill the chip, gated ones change over sooner: at 32 / 48 / 64 / 96 rows 20 of
+# 2,432 x 4,096 259 / 247, 268 / 267, 277 / 341, 310 / 355.
 # Either way a pair's result has the same bits.
 MOE_GROUPED_ROWS_AN_EXPERT = 112
 MOE_GROUPED_ROWS_A_WIDE_EXPERT = 56
@@ -444,10 +445,10 @@ def moe_experts(x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, w_gat
         xs = torch.empty((P, W), dtype=x.dtype, device=x.device)
         gu = torch.empty((P, 2 * ff), dtype=x.dtype, device=x.device)
         _ok(_core().ia_moe_gather(_p(x), _p(perm), _p(xs), P, top, W, _stream()), "moe_gather")
-        gemm_mfma_grouped(xs, w_gate_up, offsets, gu)
+        gemm_mfma_grouped(xs, w_gate_up, offsets, gu, total)
         _ok(_core().ia_moe_glu(_p(gu), _p(y), P, ff, ctypes.c_float(limit), ctypes.c_float(alpha),
                                ctypes.c_float(shift), _p(perm), _p(in_w), _stream()), "moe_glu")
-        gemm_mfma_grouped(y, w_down, offsets, xs)
+        gemm_mfma_grouped(y, w_down, offsets, xs, total)
         _ok(_core().ia_moe_scatter(_p(xs), _p(perm), _p(out_w), _p(parts), _p(offsets[E:] if total > E else None), N, top,
                                    W, _stream()), "moe_scatter")
         return SplitSum(parts)

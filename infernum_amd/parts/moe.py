@@ -229,11 +229,11 @@ class RoutedExperts(FeedForward):
             xs = program.buffer("moe.sorted", T * top * H * program.act_bytes)
             gu = program.buffer("moe.gate_up", T * top * 2 * I * program.act_bytes)
             program.op("core", "ia_moe_gather", [program.x, perm, xs, N * top, top, H, STREAM], grouped)
-            program.op("core", "ia_gemm_mfma_grouped", [xs, self.w_gate_up, gu, offsets, E, N * top, 2 * I, H, STREAM],
+            program.op("core", "ia_gemm_tiles_grouped", [xs, self.w_gate_up, gu, offsets, E, total, N * top, 2 * I, H, STREAM],
                        grouped)
             program.op("core", "ia_moe_glu", [gu, y, N * top, I, self.limit, self.alpha, self.up_shift, perm, in_w, STREAM],
                        grouped)
-            program.op("core", "ia_gemm_mfma_grouped", [y, self.w_down, xs, offsets, E, N * top, H, I, STREAM], grouped)
+            program.op("core", "ia_gemm_tiles_grouped", [y, self.w_down, xs, offsets, E, total, N * top, H, I, STREAM], grouped)
             program.op("core", "ia_moe_scatter", [xs, perm, out_w, parts, offsets.at(E * 4) if self.identity else None, N, top, H,
                                                   STREAM], grouped)
         if self.identity or self.shared_ff:
@@ -273,9 +273,9 @@ class RoutedExperts(FeedForward):
         if 0 < first <= T:
             xs = program.buffer("moe.sorted", T * top * H * program.act_bytes)
             program.op("core", "ia_moe_gather", [program.x, perm, xs, N * top, top, H, STREAM], grouped)
-            program.op("core", "ia_gemm_mfma_grouped", [xs, self.w_gate_up, y, offsets, E, N * top, I, H, STREAM], grouped)
+            program.op("core", "ia_gemm_tiles_grouped", [xs, self.w_gate_up, y, offsets, E, E, N * top, I, H, STREAM], grouped)
             program.op("core", "ia_activation", [y, y, code, N * (top * I), act, STREAM], grouped)
-            program.op("core", "ia_gemm_mfma_grouped", [y, self.w_down, xs, offsets, E, N * top, H, I, STREAM], grouped)
+            program.op("core", "ia_gemm_tiles_grouped", [y, self.w_down, xs, offsets, E, E, N * top, H, I, STREAM], grouped)
             program.op("core", "ia_moe_scatter", [xs, perm, wts, parts, None, N, top, H, STREAM], grouped)
         if self.shared_ff:
             program.keep(self.w_shared_up, self.w_shared_down)

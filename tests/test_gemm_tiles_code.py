@@ -67,3 +67,14 @@ def test_the_tiles_of_the_kernel_are_those_of_its_callers():
     for bm, bn, *t in listed:
         x0, x1, w0, w1 = map(int, t)
         assert int(bm) == 32 * (x0 + x1) and int(bn) == 32 * (w0 + w1) and x0 >= x1 and w0 >= w1
+
+
+def test_accumulators_are_read_behind_the_wait_for_the_last_products(assembly):
+    for name, body in re.findall(r"^(_Z\w*gemm_tiles_kernel\w+):(.*?)\.end_amdhsa_kernel", assembly, re.S | re.M):
+        lines = body.split("\n")
+        last = 0
+        for i, line in enumerate(lines):
+            if "v_mfma" in line:
+                last = i
+            elif "v_accvgpr_read" in line:
+                assert any("s_nop 15" in other for other in lines[last:i]), (name, line)

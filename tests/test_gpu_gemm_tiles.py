@@ -133,3 +133,26 @@ def test_where_whole_products_take_it(M, N, K_):
     want = (K_ % 64 == 0 and max(M, N) * K_ * 2 < 2 ** 32 - 3072 and small >= 200 and K_ >= 2048 and (K_ >= 4096 or large <= 140)
             and empty >= (1.06 if K_ >= 8192 and large > 256 else 1.2))
     assert api.gemm_tiles_pays(M, N, K_) == want
+
+
+# rows of the groups (and how often these repeat), columns, K; which tile they lead to: 96 x 128 as few workgroups, 96 x 256, 160 x 128,
+# 192 x 128; a tile's last row and one more, one row, none; columns that fill no tile, of two starts of the walk, off 16 bytes
+@pytest.mark.parametrize("counts,times,N,K_", [((96, 97, 0, 1, 95, 192), 1, 200, 64), ((3,), 1, 130, 320), ((96, 97, 0, 1, 95, 64), 6, 1032, 192),
+                                               ((160, 161, 0, 1, 159, 300), 6, 1032, 320), ((192, 193, 0, 1, 191, 500), 6, 1032, 448)])
+def test_rows_in_groups_at_the_edges_of_each_tile(counts, times, N, K_):
+    api = K()
+    counts = list(counts) * times
+    rows, G = sum(counts) + 2, len(counts)
+    x, w = _rand(rows, K_, seed=5), _rand(G, N, K_, scale=0.1, seed=6)
+    at = torch.tensor([0] + counts, device=DEV).cumsum(0).int()
+    out = torch.full((rows, N), 7.0, dtype=torch.bfloat16, device=DEV)
+    api.gemm_mfma_grouped(x, w, at, out)
+    lo = 0
+    for g, n in enumerate(counts):
+        want = x[lo:lo + n].double() @ w[g].double().t()
+        # as for whole products above
+        assert bool(((out[lo:lo + n].double() - want).abs() <= 2e-5 * math.sqrt(K_) * 0.1 + 2.0 ** -8 * want.abs()).all()), g
+        if n:                                                            # the first 512 columns begin their walk over K at 0
+            assert torch.equal(out[lo:lo + n, :512], api.gemm_tiles(x[lo:lo + n].clone(), w[g])[:, :512]), g
+        lo += n
+    assert bool((out[lo:] == 7.0).all())
