@@ -417,6 +417,13 @@ extern "C" int ia_gemm_mfma_split(const void* X, const void* W, float* parts, in
                                   hipStream_t stream) {
   if (!gemm_mfma_takes(M, N, K)) return IA_ERR_UNSUPPORTED;
   if (splits < 1 || splits > K / GM_BK || !parts) return IA_ERR_BAD_ARG;
+  // Up to 64 rows half of a tile of 128 is padding, and its four waves hold sums of 64 x 64 that never come to anything: tiles of
+  // 64 x 128 by eight waves, two workgroups of which fit a compute unit, keep more loads under way.  The same bits (the start of
+  // the walk goes by the tile's columns).  N x K in parts, us at 64 rows, 128 x 128 / 64 x 128: 6,144 x 4,096 in 5 14.7 / 13.6,
+  // 4,096 x 14,336 in 8 25.9 / 24.9, 9,216 x 2,048 in 3 12.7 / 11.8, 2,048 x 2,048 in 8 7.4 / 6.6, 128,256 x 4,096 whole 206 / 202; at 17
+  // rows 12.9 / 12.2, 26.2 / 24.4, 11.1 / 10.3, 6.3 / 5.5, 194 / 190.
+  if (M <= 64)
+    return launch_gemm_mfma<64, 128, 2, 4, 3, 2, true>((const uint16_t*)X, (const uint16_t*)W, nullptr, parts, M, N, K, splits, stream);
   return launch_gemm_mfma<128, 128, 2, 2, 4, 1, true>((const uint16_t*)X, (const uint16_t*)W, nullptr, parts, M, N, K,
                                                       splits, stream);
 }
@@ -432,14 +439,22 @@ extern "C" int ia_gemm_mfma_swiglu(const void* X, const void* W, int w_tiled, vo
                                    hipStream_t stream) {
   if (!gemm_mfma_takes(M, N, K)) return IA_ERR_UNSUPPORTED;
   if (N & 1) return IA_ERR_BAD_ARG;
+  // up to 64 rows tiles of 64 x 128, as for the split product: N x K at 17 / 64 rows, us, 128 x 128 and 64 x 128: 28,672 x 4,096
+  // 44.2 / 44.9 and 43.2 / 42.6, 11,008 x 2,048 19.6 / 22.3 and 17.3 / 19.5, 57,344 x 8,192 181 / 178 and 160 / 164
   if (w_tiled) {
     if (ia_gemm_skinny_splits(N, K) != 1) return IA_ERR_BAD_ARG;
     // the copy is addressed with 32 bits too: rows padded to blocks of 32 columns, K to chunks of 256
     const unsigned long long blocks = (N / 2 + 31) / 32, chunks = (K + 255) / 256;
     if (blocks * chunks * 64 * 256 * 2 > 0xffffffffULL) return IA_ERR_UNSUPPORTED;
+    if (M <= 64)
+      return launch_gemm_mfma<64, 128, 2, 2, 4, 1, false, true, true>((const uint16_t*)X, (const uint16_t*)W, (uint16_t*)C, nullptr, M, N,
+                                                                      K, 1, stream);
     return launch_gemm_mfma<128, 128, 2, 2, 4, 1, false, true, true>((const uint16_t*)X, (const uint16_t*)W,
                                                                      (uint16_t*)C, nullptr, M, N, K, 1, stream);
   }
+  if (M <= 64)
+    return launch_gemm_mfma<64, 128, 2, 2, 4, 1, false, true>((const uint16_t*)X, (const uint16_t*)W, (uint16_t*)C, nullptr, M, N, K, 1,
+                                                              stream);
   return launch_gemm_mfma<128, 128, 2, 2, 4, 1, false, true>((const uint16_t*)X, (const uint16_t*)W, (uint16_t*)C,
                                                              nullptr, M, N, K, 1, stream);
 }

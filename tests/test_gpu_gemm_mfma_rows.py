@@ -1,0 +1,33 @@
+"""The split product and the one with the activation on either side of 64 rows, from where on their tiles are larger: the same bits."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _rand(*shape, scale=1.0, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return (torch.randn(*shape, device=DEV, generator=g) * scale).to(torch.bfloat16)
+
+
+# columns of one tile, of one and some; one step of K, fewer steps than stages, more; parts of unequal length
+@pytest.mark.parametrize("N,K_,S", [(96, 64, 1), (130, 128, 2), (770, 704, 3), (256, 1024, 1)])
+def test_up_to_64_rows_as_with_more(N, K_, S):
+    from infernum_amd.kernels import api
+    a, w = _rand(65, K_, seed=1), _rand(N, K_, scale=0.1, seed=2)
+    want = a.double() @ w.double().t()
+    of_65 = api.gemm_mfma_split(a, w, S).parts
+    # fp32 sums of K_ products, each addition within 2^-24 of the running sum, of the order of 0.1 sqrt(K)
+    assert bool(((of_65.double().sum(0) - want).abs() <= 2e-5 * math.sqrt(K_) * 0.1).all())
+    act = api.gemm_mfma_swiglu(a, w)
+    tiled = api.tile_weight(w, "swiglu") if api.gemm_skinny_splits(N, K_) == 1 else None
+    for M in (64, 63, 33, 32, 1):
+        parts = torch.full((S + 1, M, N), 7.0, device=DEV)
+        assert torch.equal(api.gemm_mfma_split(a[:M].contiguous(), w, S, parts[:S]).parts, of_65[:, :M]), M
+        assert bool((parts[S] == 7.0).all())                             # nothing behind the last part
+        assert torch.equal(api.gemm_mfma_swiglu(a[:M].contiguous(), w), act[:M]), M
+        if tiled is not None:
+            assert torch.equal(api.gemm_mfma_swiglu(a[:M].contiguous(), w, tiled=tiled), act[:M]), M
