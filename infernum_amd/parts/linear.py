@@ -312,6 +312,7 @@ class Route:
 
 
 FP32_TILED_FROM_ROWS = (49, 81)     # an fp32 result goes to the tiled kernel from so many rows on: K >= 4,096; shorter K
+FP32_TILED_WIDE, FP32_TILED_WIDE_FROM_ROWS = 24576, 17     # and with so many columns (192 tiles) from so many rows, whatever K
 _MANY_ROWS = 65536         # the LDS-tiled kernel addresses rows with 32 bits: its fitness is judged at this many
 
 
@@ -336,11 +337,14 @@ def plan(N: int, Kdim: int, dtype: torch.dtype, out_dtype: torch.dtype, epilogue
         # many rows (the head of a step that wants the logits of many places): the LDS-tiled kernel leaving its fp32
         # sums (one part), which reads the weight once per 128 x 128 tile of the result where the weight-streaming
         # kernel reads all of it for every 128 rows (the head of 128,256 x 4,096 on an MI355X: 371 against 649 us at
-        # 256 rows, 2.6 against 4.9 ms at 2,048) and all of X for every 64 rows of the weight (201 against 229 us at
-        # 64 rows, 226 against 314 at 128; with K of 2,048 even at 64 rows, 150 against 181 at 128).  The same bits.
+        # 256 rows, 2.6 against 4.9 ms at 2,048) and all of X for every 64 rows of the weight (226 against 314 us at
+        # 128 rows; with K of 2,048 150 against 181).  A head whose tiles occupy three quarters of the compute units goes there
+        # from 17 rows on, tiled / weight-streaming at 17, 32, 48 and 64 rows: 128,256 x 4,096 187, 190, 195, 202 / 196, 205, 229, 251;
+        # 32,000 x 2,048 26, 27, 27, 27 / 27, 29, 33, 36; 50,304 x 1,024 23, 24, 26, 27 / 28, 31, 34, 38 (16,384 x 4,096 39, 36, 37, 38 /
+        # 28, 28, 30, 33: not so).
         routes = [Route(_UP_TO_128, own), Route(ALL_BLOCKS & ~_UP_TO_128, "skinny_rows")]
         if tiled_fits:
-            first = FP32_TILED_FROM_ROWS[0] if Kdim >= 4096 else FP32_TILED_FROM_ROWS[1]
+            first = FP32_TILED_WIDE_FROM_ROWS if N >= FP32_TILED_WIDE else FP32_TILED_FROM_ROWS[0] if Kdim >= 4096 else FP32_TILED_FROM_ROWS[1]
             routes.insert(0, Route(ALL_BLOCKS, "mfma_f32", rows=(first, (2 ** 32 - 1) // (2 * Kdim) - 1)))
         return routes
     to_library = library_rows(N, Kdim, epilogue, keep_split) if _prefill_gemm == "library" else \

@@ -31,3 +31,22 @@ def test_up_to_64_rows_as_with_more(N, K_, S):
         assert torch.equal(api.gemm_mfma_swiglu(a[:M].contiguous(), w), act[:M]), M
         if tiled is not None:
             assert torch.equal(api.gemm_mfma_swiglu(a[:M].contiguous(), w, tiled=tiled), act[:M]), M
+
+
+def test_the_head_of_many_columns_from_17_rows_on():
+    """An fp32 result as wide as fills the chip by the tiled kernel from 17 rows on, in the plan and in what linear gives; each row as
+    near to 64 bits as by the weight-streaming kernel, and the same whatever stands beside it."""
+    import importlib
+    from infernum_amd.kernels import api
+    L = importlib.import_module("infernum_amd.parts.linear")
+    N, K_ = L.FP32_TILED_WIDE, 1088
+    kinds = [L.route_of(L.plan(n, K_, torch.bfloat16, torch.float32, None, False), m).kind for n, m in ((N, 16), (N, 17), (N - 1, 17))]
+    assert kinds == ["skinny", "mfma_f32", "skinny"]
+    x, w = _rand(33, K_, seed=3), _rand(N, K_, scale=0.1, seed=4)
+    want = x.double() @ w.double().t()
+    y = L.linear(x, w, out_dtype=torch.float32)
+    few = api.gemm_skinny(x, w, out_dtype=torch.float32)
+    assert y.dtype == torch.float32 and bool(((y.double() - want).abs() <= 2e-5 * math.sqrt(K_) * 0.1).all())
+    a, b = ((t.double() - want).pow(2).mean().sqrt().item() for t in (y, few))
+    assert a <= 1.25 * b, (a, b)
+    assert torch.equal(L.linear(x[:17].contiguous(), w, out_dtype=torch.float32), y[:17])
