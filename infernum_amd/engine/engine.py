@@ -176,8 +176,8 @@ class Engine:
         cache = self.cache
         reqs, q_lens = [e.request for e in entries], [len(e.tokens) for e in entries]
         fresh = [r for r in reqs if not cache.has(r)]
-        for r in fresh:
-            cache.admit(r)
+        if fresh:
+            cache.admit_many(fresh)
         reserved = False
         try:
             arrays = cache.step_arrays(reqs, q_lens)        # once for the reservation and the commit
