@@ -148,7 +148,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_mfma_kernel(const
   // against 27.8 for its down projection in eight parts.  The start depends on the tile of columns alone, so a row's
   // sums depend neither on the rows beside it nor on the number of rows.
   constexpr bool ROTATE = SPLIT || GLU;
-  const int rot = ROTATE ? (int)((((unsigned)tn * 0x9E3779B1u) >> 8) % (unsigned)ksteps) : 0;
+  const int rot = ROTATE ? (int)((((unsigned)(n0 / 128) * 0x9E3779B1u) >> 8) % (unsigned)ksteps) : 0;
   auto krot = [&](int kt) {
     const int k = kt + rot;
     return (ROTATE && k >= ksteps) ? k - ksteps : k;
@@ -424,6 +424,13 @@ extern "C" int ia_gemm_mfma_split(const void* X, const void* W, float* parts, in
   // rows 12.9 / 12.2, 26.2 / 24.4, 11.1 / 10.3, 6.3 / 5.5, 194 / 190.
   if (M <= 64)
     return launch_gemm_mfma<64, 128, 2, 4, 3, 2, true>((const uint16_t*)X, (const uint16_t*)W, nullptr, parts, M, N, K, splits, stream);
+  // Few columns (a router's) or few rows of them: a workgroup's walk over K is one chain of steps, each as long as its loads and its
+  // barrier, and tiles of 128 x 128 leave most units without one.  Tiles of 32 x 64 have shorter steps and four times the rows in
+  // parallel, as long as there are no more of them than two a compute unit.  The same bits.  M x N x K, us, 128 x 128 / 32 x 64:
+  // 1,934 x 24 x 4,096 33 / 19, 2,047 x 32 x 2,048 20 / 12, 8,192 x 32 x 2,048 20 / 12, 1,000 x 256 x 8,192 59 / 33, 1,000 x 768 x 2,048
+  // (384 of them) 20 / 15; 2,000 x 2,048 x 2,048 has 2,016 and stays at 24.
+  if ((long long)((M + 31) / 32) * ((N + 63) / 64) * splits <= 512)
+    return launch_gemm_mfma<32, 64, 1, 2, 6, 1, true>((const uint16_t*)X, (const uint16_t*)W, nullptr, parts, M, N, K, splits, stream);
   return launch_gemm_mfma<128, 128, 2, 2, 4, 1, true>((const uint16_t*)X, (const uint16_t*)W, nullptr, parts, M, N, K,
                                                       splits, stream);
 }

@@ -50,3 +50,19 @@ def test_the_head_of_many_columns_from_17_rows_on():
     a, b = ((t.double() - want).pow(2).mean().sqrt().item() for t in (y, few))
     assert a <= 1.25 * b, (a, b)
     assert torch.equal(L.linear(x[:17].contiguous(), w, out_dtype=torch.float32), y[:17])
+
+
+# as many tiles of 32 x 64 as the rule takes (a row more of tiles: tiles of 128 x 128), rows and columns that fill no tile, fewer steps of
+# K than stages
+@pytest.mark.parametrize("M,N,K_,S", [(65, 5, 64, 1), (1248, 770, 448, 1), (8192, 120, 192, 1), (607, 770, 320, 2)])
+def test_few_columns_as_with_more_rows(M, N, K_, S):
+    from infernum_amd.kernels import api
+    tiles = -(-M // 32) * -(-N // 64) * S
+    more = M + 32 * (-(-(513 - tiles) // (-(-N // 64) * S)))
+    assert tiles <= 512 < -(-more // 32) * -(-N // 64) * S
+    a, w = _rand(more, K_, seed=7), _rand(N, K_, scale=0.1, seed=8)
+    want = a[:M].double() @ w.double().t()
+    parts = torch.full((S + 1, M, N), 7.0, device=DEV)
+    got = api.gemm_mfma_split(a[:M].contiguous(), w, S, parts[:S]).parts
+    assert bool(((got.double().sum(0) - want).abs() <= 2e-5 * math.sqrt(K_) * 0.1).all()) and bool((parts[S] == 7.0).all())
+    assert torch.equal(api.gemm_mfma_split(a, w, S).parts[:, :M], got)
