@@ -25,7 +25,7 @@
 // place of 32 x 32 x 16 (the same cycles, 5 to 10 % more clock for the power), a barrier for two phases in place of one (2,384), one value
 // of m0 for all loads of a half-tile (2,314).  Whole products, M x N x K, us (library / this; of 4,096 x 4,096 x 4,096 1.42 PFLOP/s):
 //   2,048 x 28,672 x 4,096 374 / 371   2,048 x 4,096 x 14,336 199 / 184   1,934 x 9,472 x 4,096 253 / 110   2,003 x 9,216 x 2,048 85 / 70
-//   4,096 x 4,096 x 4,096 95 / 97      8,192 x 28,672 x 4,096 1,276 / 1,312 (with the activation's launch 1,428 / 1,330)
+//   4,096 x 4,096 x 4,096 95 / 97      8,192 x 28,672 x 4,096 1,276 / 1,312 (with the activation 1,428, a launch of its own / 1,271)
 //
 // Both matrices have K contiguous.  Lane (r, q) = (lane % 16, lane / 16) of an operand holds the 8 values k = 32 s + 8 q .. + 7 of
 // row r, one 16-byte LDS read.  A load instruction of a wave fills 1,024 consecutive bytes of LDS, lane by lane: 8 rows of 128

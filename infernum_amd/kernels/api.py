@@ -1158,13 +1158,13 @@ def prefill_launch_shape(nh: int, nkv: int, d: int, q_lens: Sequence[int], ctx_l
 
     Four heads a workgroup (the default at head sizes 80 to 160 with three or more query heads to a key/value
     head) read the keys least often but make few workgroups: when they would fill fewer than three quarters of
-    the compute units, two heads are taken (1,024 tokens: 34 against 49 us).  When the launch has no more
+    the compute units, two heads are taken (1,024 tokens: 33 against 43 us).  When the launch has no more
     workgroups than compute units, every workgroup runs from start to end and the longest sets the time: under
     the causal mask that is the last block of a prompt, with twice the rounds of the average one.  Paired rows
-    give all workgroups of a request the same work then (2,048 tokens: 66 against 89 us with four heads, 71 with
-    two unpaired; 2,048 after 2,048: 147 against 171).  With more workgroups than compute units the rounds of a
+    give all workgroups of a request the same work then (2,048 tokens: 61 against 77 us with four heads, 66 with
+    two unpaired; 2,048 after 2,048: 125 against 141).  With more workgroups than compute units the rounds of a
     paired workgroup in which half its waves have run out of keys cost more than the balance gains (4,096
-    tokens: 220 against 192 us), and under a window the rows of the two ends share no keys: not paired then.
+    tokens: 194 against 168 us), and under a window the rows of the two ends share no keys: not paired then.
     """
     G = nh // nkv
     widest = 4 if 80 <= d <= 160 else 2
