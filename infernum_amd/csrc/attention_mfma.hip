@@ -659,6 +659,9 @@ static void launch_decode_reduce(const float* part_o, const float* part_ml, void
 // The accumulators of the two S^T tiles of 16 keys leave lane (col, qd) with the keys 4 qd .. 4 qd + 3 and
 // 16 + 4 qd .. 16 + 4 qd + 3; the values are laid into LDS in that order of keys, so the probabilities go
 // from registers to registers.
+// EIGHTS: row r of the S^T tile kt stands for the key 8 (r / 4) + r % 4 + 4 kt (the keys' rows are laid into LDS so), and lane (col, qd)
+// has the keys 8 qd .. 8 qd + 7: the order of the kernel of attention_prefill.h, whose sums these then are to the bit.  Where a launch
+// may go to either, this is the form: which one it goes to (by the width of the step's block tables, say) leaves a request's bits alone.
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 #define PF_KT (IA_MAX_DIM <= 128 ? 64 : 32)   // keys per round of the main loop (one barrier), in parts of 32
 #define PF_SUBS (PF_KT / 32)
@@ -668,7 +671,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 #define PF_LAZY 6.0f            // log2 of how far the running maximum may run ahead of the reference point
 #define PF_LAZY_EXP 64.0f       // 2^PF_LAZY
 
-template <int CT, int HGW, bool POW2>
+template <int CT, int HGW, bool POW2, bool EIGHTS = false>
 __global__ __launch_bounds__(4 * HGW * 64) void attn_prefill_kernel(
     const uint16_t* __restrict__ q, int q_row_stride, const uint16_t* __restrict__ k_pages,
     const uint16_t* __restrict__ v_pages, uint16_t* __restrict__ out, int out_row_stride,
@@ -874,18 +877,21 @@ __global__ __launch_bounds__(4 * HGW * 64) void attn_prefill_kernel(
     for (int i = 0; i < KPT; ++i) {
       const int pc = tid + i * PF_THREADS;
       const int kr = pc / (HD / 8), dp = pc - kr * (HD / 8);
-      if (pc < KPIECES) *reinterpret_cast<uint4*>(&ks[buf][kr][dp * 8]) = kreg[i];
+      const int at = EIGHTS ? (kr & ~31) + 16 * ((kr >> 2) & 1) + 4 * ((kr >> 3) & 3) + (kr & 3) : kr;
+      if (pc < KPIECES) *reinterpret_cast<uint4*>(&ks[buf][at][dp * 8]) = kreg[i];
     }
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
       const int pc = tid + i * PF_THREADS;
       const int dim = pc / PF_QPT, quad = pc & (PF_QPT - 1), sub = quad >> 3, q8 = quad & 7;
       // within a part of 32 keys, quad q8 = 4 kt + qd holds the keys 16 kt + 4 qd .. + 3: they go to the places
-      // 8 qd + 4 kt .. + 3
-      if (pc < VPIECES) *reinterpret_cast<uint2*>(&vs[buf][sub][dim][(q8 & 3) * 8 + (q8 >> 2) * 4]) = vreg[i];
+      // 8 qd + 4 kt .. + 3 (EIGHTS: in their order)
+      if (pc < VPIECES) *reinterpret_cast<uint2*>(&vs[buf][sub][dim][EIGHTS ? q8 * 4 : (q8 & 3) * 8 + (q8 >> 2) * 4]) = vreg[i];
     }
   };
 
+  // the key of this lane's score r of the S^T tile kt
+  auto key_in = [&](int kt, int r) { return EIGHTS ? 8 * qd + 4 * kt + r : 16 * kt + 4 * qd + r; };
   // Tile t lies in register set and LDS buffer (t - t_begin) & 1.
   using set0 = std::integral_constant<int, 0>;
   using set1 = std::integral_constant<int, 1>;
@@ -916,7 +922,7 @@ __global__ __launch_bounds__(4 * HGW * 64) void attn_prefill_kernel(
 #pragma unroll
         for (int c = 0; c < CT; ++c)
 #pragma unroll
-          for (int i = 0; i < 8; ++i) bv[c][i] = brow[c][t0 + (i >> 2) * 16 + 4 * qd + (i & 3)];
+          for (int i = 0; i < 8; ++i) bv[c][i] = brow[c][t0 + key_in(i >> 2, i & 3)];
       }
       // ---- S^T = K Q^T for the two tiles of 16 keys
       f32x4 sc[CT][2];
@@ -962,7 +968,7 @@ __global__ __launch_bounds__(4 * HGW * 64) void attn_prefill_kernel(
           for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              const int kr = t0 + kt * 16 + 4 * qd + r;
+              const int kr = t0 + key_in(kt, r);
               const bool ok = pos[c] >= 0 && kr <= pos[c] && (kr >= lo[c] || (EXT && kr < X.keep));
               sv[kt * 4 + r] = ok ? sv[kt * 4 + r] : -INFINITY;
             }
@@ -1235,8 +1241,11 @@ extern "C" int ia_attn_prefill(const void* q, int q_row_stride, const void* k_pa
   const int xrc = attn_ext(window, keep, softcap, scale, bias, span, gate, gate_stride, nh, X, scale_log2);
   if (xrc != IA_OK) return xrc;
   dim3 grid(num_tiles, nkv * HC);
+  // where a wave may take 32 rows (attention_prefill.h): by the model's heads and the pages' size alone, so that all of a request's
+  // launches sum in one order; which of the two kernels a launch goes to is free then
+  const bool eights = IA_PREFILL_WIDE && G >= 2 && (ps & (ps - 1)) == 0 && ps >= 8;
 #if IA_PREFILL_WIDE
-  if (G >= 2 && (ps & (ps - 1)) == 0 && ps >= 8 && bt_stride <= PW_BT) {
+  if (eights && bt_stride <= PW_BT) {
 #define PW_LAUNCH(W)                                                                                                          \
   return launch_prefill_wide<W>(grid, q, q_row_stride, k_pages, v_pages, out, out_row_stride, seq_starts, seq_ctx, block_tables, \
                                 bt_stride, tiles, nh, nkv, ps, num_pages, scale_log2, window, paired, sinks, stream)
@@ -1246,14 +1255,15 @@ extern "C" int ia_attn_prefill(const void* q, int q_row_stride, const void* k_pa
 #undef PW_LAUNCH
   }
 #endif
-#define PF_LAUNCH_P(C, W, P2)                                                                                     \
-  attn_prefill_kernel<C, W, P2><<<grid, 4 * W * 64, 0, stream>>>(                                                 \
+#define PF_LAUNCH_P(C, W, ...)                                                                                    \
+  attn_prefill_kernel<C, W, __VA_ARGS__><<<grid, 4 * W * 64, 0, stream>>>(                                        \
       (const uint16_t*)q, q_row_stride, (const uint16_t*)k_pages, (const uint16_t*)v_pages, (uint16_t*)out,       \
       out_row_stride, seq_starts, seq_ctx, block_tables, bt_stride, tiles, nh, nkv, ps, num_pages, scale_log2, window, \
       paired, sinks, X)
 #define PF_LAUNCH(C, W)                      \
   do {                                       \
-    if ((ps & (ps - 1)) == 0) PF_LAUNCH_P(C, W, true); \
+    if (eights) PF_LAUNCH_P(C, W, true, IA_PREFILL_WIDE != 0); \
+    else if ((ps & (ps - 1)) == 0) PF_LAUNCH_P(C, W, true); \
     else PF_LAUNCH_P(C, W, false);           \
   } while (0)
   if (HGW == 1) PF_LAUNCH(1, 1);

@@ -117,3 +117,16 @@ def test_a_key_without_a_page_gives_nan():
     assert bool(out[64:100].isnan().all()) and bool(out[100:].isfinite().all())
     c["bt"][0, 2] = 10 ** 6
     assert bool(_run(c, nh, nkv)[64:100].isnan().all())
+
+
+@pytest.mark.parametrize("nh,nkv,ps", [(4, 1, 16), (6, 2, 8), (4, 2, 64)])
+@pytest.mark.parametrize("lens,q_lens", [([1, 31, 33, 64, 129], [1, 31, 33, 64, 129]), ([300, 449], [300, 100])])
+@pytest.mark.parametrize("window", [0, 40, -96])
+def test_the_block_tables_width_leaves_the_bits_alone(nh, nkv, ps, lens, q_lens, window):
+    """A neighbour's length makes a step's tables wider than the kernel keeps in LDS: the other kernel, the same order of sums."""
+    c = _case(nh, nkv, ps, lens, q_lens, seed=nh + ps + len(lens))
+    out = _run(c, nh, nkv, window)
+    c["bt"] = torch.cat([c["bt"], torch.zeros(len(lens), 4097, dtype=torch.int32, device=DEV)], dim=1).contiguous()
+    for hpw in (1, 2, 4):
+        for paired in (False, True):
+            assert torch.equal(_run(c, nh, nkv, window, heads_per_workgroup=hpw, paired=paired), out), (hpw, paired)
