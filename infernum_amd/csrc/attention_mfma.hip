@@ -1247,8 +1247,9 @@ extern "C" int ia_attn_prefill(const void* q, int q_row_stride, const void* k_pa
 #if IA_PREFILL_WIDE
   if (eights && bt_stride <= PW_BT) {
 #define PW_LAUNCH(W)                                                                                                          \
-  return launch_prefill_wide<W>(grid, q, q_row_stride, k_pages, v_pages, out, out_row_stride, seq_starts, seq_ctx, block_tables, \
-                                bt_stride, tiles, nh, nkv, ps, num_pages, scale_log2, window, paired, sinks, stream)
+  return (window != 0 ? launch_prefill_wide<W, true> : launch_prefill_wide<W, false>)(                                        \
+      grid, q, q_row_stride, k_pages, v_pages, out, out_row_stride, seq_starts, seq_ctx, block_tables, bt_stride, tiles, nh, nkv, \
+      ps, num_pages, scale_log2, window, paired, sinks, stream)
     if (HGW == 1) PW_LAUNCH(1);
     if (HGW == 2) PW_LAUNCH(2);
     PW_LAUNCH(4);

@@ -14,10 +14,11 @@
 // What bounds it: a SIMD has two such waves, whose matrix instructions take 2,176 cycles a tile, their exponentials and what goes with
 // them some 1,700, and whose reads of LDS (256 KB a tile and compute unit, half of what waves of 16 rows need) 2,048.  These have to run
 // beside each other: a piece of a pair of exponentials of 32 keys' scores stands behind every product of the next 32's scores and every one of the
-// probabilities of the 32 before.  The 8B shape's heads (32 over 8), waves of 16 rows / this kernel, us: 2,048 tokens 69 / 62, 4,096
-// 203 / 162, 8,192 666 / 553 (0.99 PFLOP/s), 2,048 after 6,144 cached 294 / 244; 64 prompts of 120 60 / 68, under a window of
-// 1,024 2,047 tokens of 16 heads over 4 41 / 44 (few tiles a workgroup: its start is longer).  With the products in a row and the exponentials behind them 8,192 tokens
-// took 590.  Heads of 64 gained nothing (2,048 tokens 48 / 54, 8,192 438 / 418), one query head to a key/value head lost (2,000 tokens of 8 heads 53 / 67).
+// probabilities of the 32 before.  The 8B shape's heads (32 over 8), waves of 16 rows / this kernel, us: 2,048 tokens 70 / 55, 4,096
+// 191 / 148, 8,192 662 / 508 (1.08 PFLOP/s), 2,048 after 6,144 cached 293 / 226; under a window of 4,096 8,192 tokens 512 / 412; 64 prompts of
+// 120 59 / 63, under a window of 1,024 2,047 tokens of 16 heads over 4 41 / 42 (few tiles a workgroup: its start is longer).  With the products
+// in a row and the exponentials behind them 8,192 tokens took 590, with tests for a wave's first and last half inside the loop 587.
+// Heads of 64 gained nothing (2,048 tokens 48 / 54, 8,192 438 / 418), one query head to a key/value head lost (2,000 tokens of 8 heads 53 / 67).
 //
 // In LDS the 16-byte piece c of row r (a key's values; a dim's 64 keys) lies at position c ^ s(r), s(key) = key % 4 + 4 (key / 8 % 2),
 // s(dim) = dim % 8: the 8 lanes that read together find 8 different places.
@@ -25,6 +26,7 @@
 
 #define PW_KT 64                        // keys a tile
 #define PW_STAGES 4
+#define PW_INLINE __attribute__((always_inline))
 #define PW_BT 4096                      // block-table entries kept in LDS
 
 typedef const __attribute__((address_space(1))) void* pw_global_ptr;
@@ -35,7 +37,7 @@ constexpr int PW_LDS = PW_STAGES * (PW_K_BYTES + PW_V_BYTES) + PW_BT * 4;
 
 typedef f32x4 pw_scores[2][2];          // of 32 keys: [tile of 16][column]
 
-template <int HGW>
+template <int HGW, bool WINDOW>
 __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
     const uint16_t* __restrict__ q, int q_row_stride, const uint16_t* __restrict__ k_pages, const uint16_t* __restrict__ v_pages,
     uint16_t* __restrict__ out, int out_row_stride, const int* __restrict__ seq_starts, const int* __restrict__ seq_ctx,
@@ -86,7 +88,9 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
   const int wave_hi = ctx + wave_last;
   const int wave_lo_last = ia_first_visible_key(wave_hi, window);
   const int t_begin = key_lo / PW_KT, t_end = key_hi / PW_KT;
-  const int w_end = wave_live ? wave_hi / 32 : -1;                      // the wave's last half of a tile
+  // halves of tiles (32 keys): the wave's first and last, the last of its first 16 rows, the first of the others
+  const int w_end = wave_live ? wave_hi / 32 : -2, w_begin = wave_live ? ia_first_visible_key(ctx + rb, window) / 32 : 0;
+  const int end0 = (ctx + (rb + 15 < qlen ? rb + 15 : qlen - 1)) / 32, begin1 = WINDOW ? ia_first_visible_key(ctx + rb + 16, window) / 32 : 0;
   {
     const int* bt = block_tables + (size_t)sidx * bt_stride;
     const int first = key_lo >> ps_shift, count = (key_hi >> ps_shift) - first + 1;
@@ -132,13 +136,13 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
   const int last_page = (key_hi >> ps_shift) - bt_first;
   bool bad = false;
   int k_pg[KG], v_pg;
-  auto page_of = [&](int key) { return s_bt[min(max((key >> ps_shift) - bt_first, 0), last_page)]; };
-  auto pages_of_k = [&](int t) {
+  auto page_of = [&](int key) PW_INLINE { return s_bt[min(max((key >> ps_shift) - bt_first, 0), last_page)]; };
+  auto pages_of_k = [&](int t) PW_INLINE {
 #pragma unroll
     for (int f = 0; f < KG; ++f) k_pg[f] = page_of(t * PW_KT + 8 * (wave * KG + f));
   };
-  auto pages_of_v = [&](int t) { v_pg = page_of(t * PW_KT + v_key); };
-  auto load_k = [&](int t, int slot) {
+  auto pages_of_v = [&](int t) PW_INLINE { v_pg = page_of(t * PW_KT + v_key); };
+  auto load_k = [&](int t, int slot) PW_INLINE {
 #pragma unroll
     for (int f = 0; f < KG; ++f) {
       const bool ok = (unsigned)k_pg[f] < (unsigned)num_pages;
@@ -152,7 +156,7 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
       static_assert(KL <= 2, "a group's loads");
     }
   };
-  auto load_v = [&](int t, int slot) {
+  auto load_v = [&](int t, int slot) PW_INLINE {
     const bool ok = (unsigned)v_pg < (unsigned)num_pages;
     bad |= !ok;
     const uint32_t in_page = (uint32_t)((t * PW_KT + v_key) & (ps - 1)) * 2u;
@@ -166,23 +170,23 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
   // ---- reads: this lane's row and pieces
   const int k_lane = (8 * (j >> 2) + (j & 3)) * (HD * 2), v_lane = j * (PW_KT * 2);
   const int piece0 = (qd ^ (j & 7)) * 16, piece1 = ((4 + qd) ^ (j & 7)) * 16;
-  auto read_k = [&](const char* half, int t, int st) {        // tile t of the half's two, step st of the head dims
+  auto read_k = [&](const char* half, int t, int st) PW_INLINE {        // tile t of the half's two, step st of the head dims
     return *reinterpret_cast<const bf16x8_t*>(half + k_lane + t * (4 * HD * 2) + (st >> 1) * 128 + ((st & 1) ? piece1 : piece0));
   };
   // `values`: the stage of the half's tile, with this lane's place in it
-  auto read_v = [&](const char* values, int n) { return *reinterpret_cast<const bf16x8_t*>(values + n * (16 * PW_KT * 2)); };
+  auto read_v = [&](const char* values, int n) PW_INLINE { return *reinterpret_cast<const bf16x8_t*>(values + n * (16 * PW_KT * 2)); };
 
   typedef uint32_t packed[2][4];        // probabilities as B operands: [column][pairs of keys]
   float emax[2];
   // the two exponentials of pair i (of four) of column c of 32 keys' scores, packed
-  auto pair_of = [&](const pw_scores& s, packed& pk, int c, int i, float neg_m) {
+  auto pair_of = [&](const pw_scores& s, packed& pk, int c, int i, float neg_m) PW_INLINE {
     const int t = i >> 1, r = 2 * (i & 1);
     const f32x2_t e = {__builtin_amdgcn_exp2f(fmaf(s[t][c][r], scale_log2, neg_m)), __builtin_amdgcn_exp2f(fmaf(s[t][c][r + 1], scale_log2, neg_m))};
     emax[c] = fmaxf(emax[c], fmaxf(e[0], e[1]));
     pk[c][i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(e, bf16x2_t));
   };
   // keys that a column does not see
-  auto mask = [&](pw_scores& s, int t0) {
+  auto mask = [&](pw_scores& s, int t0) PW_INLINE {
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const int row = rb + 16 * c + j, last = row < qlen ? ctx + row : -1, first = ia_first_visible_key(ctx + row, window);
@@ -197,7 +201,7 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
   };
   // The reference point of the exponentials follows the running maximum lazily, as in the kernel above: only when an exponential against
   // it comes out above 2^PF_LAZY, or a column has none yet, it moves, the accumulators are rescaled and the exponentials taken again.
-  auto settle = [&](const pw_scores& s, packed& pk) {
+  auto settle = [&](const pw_scores& s, packed& pk) PW_INLINE {
     if (!__any(emax[0] > PF_LAZY_EXP || emax[1] > PF_LAZY_EXP || m[0] == -INFINITY || m[1] == -INFINITY)) return;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
@@ -218,7 +222,7 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
       for (int i = 0; i < 4; ++i) pair_of(s, pk, c, i, -m_safe);
     }
   };
-  auto scores = [&](pw_scores& s, const char* half) {
+  auto scores = [&](pw_scores& s, const char* half) PW_INLINE {
 #pragma unroll
     for (int x = 0; x < 2 * KS; ++x) {
       const bf16x8_t a = read_k(half, x & 1, x >> 1);
@@ -231,12 +235,13 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
   // half x of the keys: its scores `cur` become probabilities `pk`, while the scores of half x + 1 (keys at `half`) come into `next` and
   // the probabilities `before` of half x - 1 weigh its `values` into the accumulators: three halves' work, none of
   // which waits for another's.  One path for every half: a wave's first has no probabilities before it (zeros, against values that it
-  // multiplies with anyway), its last no scores behind it (of keys that are there; nobody looks at them), and the one behind that
-  // only probabilities before it.
-  auto part = [&](int x, pw_scores& cur, pw_scores& next, packed& pk, const packed& before, const char* half, const char* values) {
-    if (x > w_end + 1) return;                               // the same for the wave, as all that follows
+  // multiplies with anyway), its last no scores behind it (of keys that are there; nobody looks at them).
+  // 16 rows meet the halves that hold a key some of them may see, and no other: 0 times a value that is not finite is NaN.  So what a column
+  // has gathered when its first half's scores are weighed (the values of halves in front of its window or chunk, times 0: nothing, or
+  // NaN) is cleared, and the last half's values, which can be beyond the first 16 rows, come in behind the loop.
+  auto part = [&](int x, pw_scores& cur, pw_scores& next, packed& pk, const packed& before, const char* half, const char* values) PW_INLINE {
     const int t0 = x * 32;
-    if (x <= w_end && ((t0 + 31 > ctx + rb) || (window != 0 && t0 < wave_lo_last) || rb + 31 >= qlen)) mask(cur, t0);
+    if ((t0 + 31 > ctx + rb) || (WINDOW && t0 < wave_lo_last) || rb + 31 >= qlen) mask(cur, t0);
     const float neg[2] = {(m[0] == -INFINITY) ? 0.f : -m[0], (m[1] == -INFINITY) ? 0.f : -m[1]};
     emax[0] = emax[1] = 0.f;
     constexpr int NY = NSV;                                  // turns: a read of keys and one of values, two products each
@@ -286,7 +291,17 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
         piece(2 * c + 1);
       }
     }
-    if (x <= w_end) settle(cur, pk);
+    settle(cur, pk);
+    if constexpr (WINDOW) {
+      if (x == w_begin) {
+#pragma unroll
+        for (int n = 0; n < NSV; ++n) o[n][0] = none;
+      }
+      if (x == begin1) {
+#pragma unroll
+        for (int n = 0; n < NSV; ++n) o[n][1] = none;
+      }
+    }
   };
   auto barrier = [&] {                  // behind all loads but those of the round before
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LOADS) : "memory");
@@ -317,21 +332,17 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
 #pragma unroll
     for (int i = 0; i < 4; ++i) pa[c][i] = pb[c][i] = 0u;
   }
-  if (wave_live) scores(sa, k_lds);
-  // (one round more where the last keys lie in the second half of their tile: its probabilities weigh in then)
-  const int t_last = t_end + ((key_hi >> 5) & 1);
-  for (int i = t_begin; i <= t_last; ++i) {
+  // A round: everybody's loads and barrier, for every tile of the workgroup's range.  A wave has work in those of its own range.
+  auto round = [&](int i) PW_INLINE {
     const int slot = (i - t_begin) & 3;
-    if (i <= t_end) {
-      barrier();                        // keys up to tile i + 1 and values up to tile i are there; nobody reads keys of tile i - 1 or values of i - 2 any more
-      load_k(i + 3, (slot + 3) & 3);    // (past the range: of its last page, for nobody, so that every round has as many loads under way)
-      load_v(i + 2, (slot + 2) & 3);
-      pages_of_k(i + 4);
-      pages_of_v(i + 3);
-    }
+    barrier();                          // keys up to tile i + 1 and values up to tile i are there; nobody reads keys of tile i - 1 or values of i - 2 any more
+    load_k(i + 3, (slot + 3) & 3);      // (past the range: of its last page, for nobody, so that every round has as many loads under way)
+    load_v(i + 2, (slot + 2) & 3);
+    pages_of_k(i + 4);
+    pages_of_v(i + 3);
     // values of keys that no row sees are not the request's: zero them in LDS (the tiles at the ends of the range)
     const int t0 = i * PW_KT;
-    if (i <= t_end && (t0 < key_lo || t0 + PW_KT - 1 > key_hi)) {
+    if (t0 < key_lo || t0 + PW_KT - 1 > key_hi) {
       for (int at = tid; at < VD * 8; at += THREADS) {
         const int dim = at >> 3, key = t0 + 8 * ((at & 7) ^ (dim & 7));
         if (key >= key_lo && key + 7 <= key_hi) continue;
@@ -344,11 +355,49 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
     }
-    const char* const here = v_lds + slot * PW_V_BYTES + v_lane + piece0;
-    part(2 * i, sa, sb, pa, pb, k_lds + slot * PW_K_BYTES + 32 * HD * 2,
-         i == t_begin ? here : v_lds + ((slot + 3) & 3) * PW_V_BYTES + v_lane + piece1);
-    part(2 * i + 1, sb, sa, pb, pa, k_lds + ((slot + 1) & 3) * PW_K_BYTES, here);
+  };
+  int i = t_begin;
+  if (WINDOW) {
+    for (; i < w_begin >> 1; ++i) round(i);
   }
+  const int first = i;
+  if (wave_live) scores(sa, k_lds + ((i - t_begin) & 3) * PW_K_BYTES);
+  auto even = [&]() PW_INLINE {
+    const int slot = (i - t_begin) & 3;
+    const char* const here = v_lds + slot * PW_V_BYTES + v_lane;
+    part(2 * i, sa, sb, pa, pb, k_lds + slot * PW_K_BYTES + 32 * HD * 2,
+         i == first ? here + piece0 : v_lds + ((slot + 3) & 3) * PW_V_BYTES + v_lane + piece1);
+    return here;
+  };
+  for (; 2 * i < w_end; ++i) {
+    round(i);
+    const char* const here = even();
+    part(2 * i + 1, sb, sa, pb, pa, k_lds + (((i - t_begin) + 1) & 3) * PW_K_BYTES, here + piece0);
+  }
+  if (wave_live) {
+    // the last half's values: of a tile that is there until the next round
+    const bool in_first = 2 * i == w_end;
+    if (in_first) {
+      round(i);
+      even();
+      ++i;
+    }
+    const char* const values = v_lds + ((i - 1 - t_begin) & 3) * PW_V_BYTES + v_lane + (in_first ? piece0 : piece1);
+    bf16x8_t p[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const uint4 a = make_uint4(pa[c][0], pa[c][1], pa[c][2], pa[c][3]), b = make_uint4(pb[c][0], pb[c][1], pb[c][2], pb[c][3]);
+      p[c] = __builtin_bit_cast(bf16x8_t, in_first ? a : b);
+      lacc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, p[c], lacc[c], 0, 0, 0);
+    }
+#pragma unroll
+    for (int n = 0; n < NSV; ++n) {
+      const bf16x8_t av = read_v(values, n);
+      o[n][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, p[1], o[n][1], 0, 0, 0);
+      if (end0 == w_end) o[n][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, p[0], o[n][0], 0, 0, 0);
+    }
+  }
+  for (; i <= t_end; ++i) round(i);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // the loads asked for past the end
   if (bad) s_poison = 1;      // a key that is needed has no page in the block table: the result is NaN
   __syncthreads();
@@ -370,20 +419,20 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
   }
 }
 
-template <int HGW>
+template <int HGW, bool WINDOW>
 static int launch_prefill_wide(dim3 grid, const void* q, int q_row_stride, const void* k_pages, const void* v_pages, void* out,
                                int out_row_stride, const int* seq_starts, const int* seq_ctx, const int* block_tables, int bt_stride,
                                const int* tiles, int nh, int nkv, int ps, int num_pages, float scale_log2, int window, int paired,
                                const float* sinks, hipStream_t stream) {
   static bool configured = false;
   if (!configured) {
-    const hipError_t e = hipFuncSetAttribute((const void*)attn_prefill_wide_kernel<HGW>, hipFuncAttributeMaxDynamicSharedMemorySize, PW_LDS);
+    const hipError_t e = hipFuncSetAttribute((const void*)attn_prefill_wide_kernel<HGW, WINDOW>, hipFuncAttributeMaxDynamicSharedMemorySize, PW_LDS);
     if (e != hipSuccess) return (int)e;
     configured = true;
   }
   int shift = 0;
   while ((1 << shift) < ps) ++shift;
-  attn_prefill_wide_kernel<HGW><<<grid, HGW * 128, PW_LDS, stream>>>(
+  attn_prefill_wide_kernel<HGW, WINDOW><<<grid, HGW * 128, PW_LDS, stream>>>(
       (const uint16_t*)q, q_row_stride, (const uint16_t*)k_pages, (const uint16_t*)v_pages, (uint16_t*)out, out_row_stride, seq_starts,
       seq_ctx, block_tables, bt_stride, tiles, nh, nkv, shift, num_pages, scale_log2, window, paired, sinks);
   IA_LAUNCH_CHECK();

@@ -130,3 +130,34 @@ def test_the_block_tables_width_leaves_the_bits_alone(nh, nkv, ps, lens, q_lens,
     for hpw in (1, 2, 4):
         for paired in (False, True):
             assert torch.equal(_run(c, nh, nkv, window, heads_per_workgroup=hpw, paired=paired), out), (hpw, paired)
+
+
+def _first_visible(pos, window):
+    return 0 if window == 0 else max(0, pos - window + 1) if window > 0 else pos // -window * -window
+
+
+@pytest.mark.parametrize("ctx,n,window", [(16, 100, 0), (1, 64, 0), (15, 97, 0), (17, 97, 0), (0, 200, 40), (16, 200, 33), (5, 150, 1),
+                                          (40, 130, 100), (0, 200, -48), (30, 170, -128), (0, 257, -16)])
+def test_a_value_that_is_not_finite_reaches_the_16_rows_that_meet_its_32_keys(ctx, n, window):
+    """A key's half of a tile is weighed in for a block of 16 rows if one of them may see a key of it; no other row may change."""
+    nh, nkv, ps, total = 4, 1, 16, ctx + n
+    c = _case(nh, nkv, ps, [total], [n], seed=9)
+    wide = dict(c, bt=torch.cat([c["bt"], torch.zeros(1, 4097, dtype=torch.int32, device=DEV)], dim=1).contiguous())
+    want = _run(c, nh, nkv, window)
+    assert bool(want.isfinite().all())
+    for t in sorted({0, 15, 31, 32, 40, 63, 64, 95, 100, ctx, total - 1}):
+        if t >= total:
+            continue
+        page = int(c["bt"][0, t // ps])
+        was = c["vp"][page, :, :, t % ps].clone()
+        c["vp"][page, :, :, t % ps] = float("inf")
+        meets = torch.zeros(n, dtype=torch.bool, device=DEV)
+        for first in range(0, n, 16):
+            lo, hi = _first_visible(ctx + first, window), ctx + min(first + 15, n - 1)
+            meets[first:first + 16] = lo // 32 <= t // 32 <= hi // 32
+        sees = torch.tensor([_first_visible(ctx + r, window) <= t <= ctx + r for r in range(n)], device=DEV)
+        for case, paired in ((c, False), (c, True), (wide, False)):
+            got = _run(case, nh, nkv, window, paired=paired)
+            assert torch.equal(got[~meets], want[~meets]), (t, paired)
+            assert not bool(got[sees].isfinite().any()), (t, paired)
+        c["vp"][page, :, :, t % ps] = was
