@@ -1204,14 +1204,16 @@ extern "C" int ia_attn_decode_fused(const void* src, int src_dtype, int src_spli
 // groups of four waves, one query head each, that share the tiles of keys and values a workgroup brings in.
 // Bit 8 (IA_PREFILL_PAIRED): a workgroup takes 32 rows from each end of its request's new tokens in place of 64
 // consecutive ones (see the kernel); tiles must then list every block of 64 rows of every request, as the
-// engine's do.  Without effect under a window.  The result has the same bits whatever the shape.
+// engine's do.  Without effect under a window.  Bit 9 (IA_PREFILL_NARROW): waves of 16 rows where they could have 32 (the
+// kernel of attention_prefill.h); without effect elsewhere.  The result has the same bits whatever the shape.
 #define IA_PREFILL_PAIRED 0x100
+#define IA_PREFILL_NARROW 0x200
 extern "C" int ia_attn_prefill(const void* q, int q_row_stride, const void* k_pages, const void* v_pages, void* out,
                                int out_row_stride, const int* seq_starts, const int* seq_ctx, const int* block_tables,
                                int bt_stride, const int* tiles, int num_tiles, int nh, int nkv, int ps, int num_pages,
                                float scale, int window, int launch_shape, const float* sinks, int keep, float softcap,
                                const float* bias, int span, const void* gate, int gate_stride, hipStream_t stream) {
-  if (launch_shape < 0 || (launch_shape & ~(0xff | IA_PREFILL_PAIRED))) return IA_ERR_BAD_ARG;
+  if (launch_shape < 0 || (launch_shape & ~(0xff | IA_PREFILL_PAIRED | IA_PREFILL_NARROW))) return IA_ERR_BAD_ARG;
   // under a window the rows of the two ends share no keys, and the keys between them may have no page any more:
   // rows are not paired then, whatever was asked for
   const int heads_per_workgroup = launch_shape & 0xff, paired = ((launch_shape & IA_PREFILL_PAIRED) && window == 0) ? 1 : 0;
@@ -1245,7 +1247,7 @@ extern "C" int ia_attn_prefill(const void* q, int q_row_stride, const void* k_pa
   // launches sum in one order; which of the two kernels a launch goes to is free then
   const bool eights = IA_PREFILL_WIDE && G >= 2 && (ps & (ps - 1)) == 0 && ps >= 8;
 #if IA_PREFILL_WIDE
-  if (eights && bt_stride <= PW_BT) {
+  if (eights && bt_stride <= PW_BT && !(launch_shape & IA_PREFILL_NARROW)) {
 #define PW_LAUNCH(W)                                                                                                          \
   return (window != 0 ? launch_prefill_wide<W, true> : launch_prefill_wide<W, false>)(                                        \
       grid, q, q_row_stride, k_pages, v_pages, out, out_row_stride, seq_starts, seq_ctx, block_tables, bt_stride, tiles, nh, nkv, \

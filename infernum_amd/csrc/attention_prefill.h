@@ -15,9 +15,11 @@
 // them some 1,700, and whose reads of LDS (256 KB a tile and compute unit, half of what waves of 16 rows need) 2,048.  These have to run
 // beside each other: a piece of a pair of exponentials of 32 keys' scores stands behind every product of the next 32's scores and every one of the
 // probabilities of the 32 before.  The 8B shape's heads (32 over 8), waves of 16 rows / this kernel, us: 2,048 tokens 70 / 55, 4,096
-// 191 / 148, 8,192 662 / 508 (1.08 PFLOP/s), 2,048 after 6,144 cached 293 / 226; under a window of 4,096 8,192 tokens 512 / 412; 64 prompts of
-// 120 59 / 63, under a window of 1,024 2,047 tokens of 16 heads over 4 41 / 42 (few tiles a workgroup: its start is longer).  With the products
-// in a row and the exponentials behind them 8,192 tokens took 590, with tests for a wave's first and last half inside the loop 587.
+// 191 / 148, 8,192 662 / 508 (1.08 PFLOP/s), 2,048 after 6,144 cached 293 / 226; under a window of 4,096 8,192 tokens 512 / 412.  Short ranges
+// of keys are the other kernel's, by the same order of sums (a prompt of 20 tokens 5.9 / 8.9, of 257 13.9 / 15.5: a longer start, and a
+// wave's work one after the other); the line is drawn where launches are shaped.  With the products in a row and the exponentials behind them
+// 8,192 tokens took 590; with tests for a wave's first and last half inside the loop 587; with a mask in every half of a wave that has
+// rows to spare 4,016 tokens of 4 heads took 111, 80 without.
 // Heads of 64 gained nothing (2,048 tokens 48 / 54, 8,192 438 / 418), one query head to a key/value head lost (2,000 tokens of 8 heads 53 / 67).
 //
 // In LDS the 16-byte piece c of row r (a key's values; a dim's 64 keys) lies at position c ^ s(r), s(key) = key % 4 + 4 (key / 8 % 2),
@@ -91,11 +93,6 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
   // halves of tiles (32 keys): the wave's first and last, the last of its first 16 rows, the first of the others
   const int w_end = wave_live ? wave_hi / 32 : -2, w_begin = wave_live ? ia_first_visible_key(ctx + rb, window) / 32 : 0;
   const int end0 = (ctx + (rb + 15 < qlen ? rb + 15 : qlen - 1)) / 32, begin1 = WINDOW ? ia_first_visible_key(ctx + rb + 16, window) / 32 : 0;
-  {
-    const int* bt = block_tables + (size_t)sidx * bt_stride;
-    const int first = key_lo >> ps_shift, count = (key_hi >> ps_shift) - first + 1;
-    for (int i = tid; i < count; i += THREADS) s_bt[i] = bt[first + i];
-  }
   const int bt_first = key_lo >> ps_shift, ps = 1 << ps_shift;
 
   // ---- queries as B operands; columns c = 0, 1 are rows rb + j and rb + 16 + j
@@ -108,15 +105,26 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
     const bool ok = wave_live && row < qlen;
     const uint16_t* qrow = q + (size_t)(qstart + (ok ? row : first_row)) * q_row_stride + (size_t)h * HD;
 #pragma unroll
-    for (int st = 0; st < KS; ++st) {
-      const uint4 v = *reinterpret_cast<const uint4*>(qrow + st * 32 + qd * 8);
-      qreg[c][st] = __builtin_bit_cast(bf16x8_t, ok ? v : make_uint4(0u, 0u, 0u, 0u));
-    }
+    for (int st = 0; st < KS; ++st) qreg[c][st] = *reinterpret_cast<const bf16x8_t*>(qrow + st * 32 + qd * 8);
     m[c] = ok ? -INFINITY : 0.f;         // a column without a row never asks for a reference point
     lacc[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int n = 0; n < NSV; ++n) o[n][c] = (f32x4){0.f, 0.f, 0.f, 0.f};
   }
+  {
+    const int* bt = block_tables + (size_t)sidx * bt_stride;
+    const int first = key_lo >> ps_shift, count = (key_hi >> ps_shift) - first + 1;
+    for (int i = tid; i < count; i += THREADS) s_bt[i] = bt[first + i];
+  }
+  // the queries are here before the first load into LDS: waiting for them behind it would wait for all of these too
+  static_assert(KS == 4, "all queries of a lane");
+  asm volatile("" : "+v"(qreg[0][0]), "+v"(qreg[0][1]), "+v"(qreg[0][2]), "+v"(qreg[0][3]), "+v"(qreg[1][0]), "+v"(qreg[1][1]),
+               "+v"(qreg[1][2]), "+v"(qreg[1][3]));
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int st = 0; st < KS; ++st)
+      if (!(wave_live && rb + 16 * c + j < qlen)) qreg[c][st] = __builtin_bit_cast(bf16x8_t, make_uint4(0u, 0u, 0u, 0u));
   const f32x4 none = {0.f, 0.f, 0.f, 0.f};
   const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
 
@@ -189,7 +197,7 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
   auto mask = [&](pw_scores& s, int t0) PW_INLINE {
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-      const int row = rb + 16 * c + j, last = row < qlen ? ctx + row : -1, first = ia_first_visible_key(ctx + row, window);
+      const int row = rb + 16 * c + j, last = ctx + row, first = ia_first_visible_key(last, window);
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -241,7 +249,8 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
   // NaN) is cleared, and the last half's values, which can be beyond the first 16 rows, come in behind the loop.
   auto part = [&](int x, pw_scores& cur, pw_scores& next, packed& pk, const packed& before, const char* half, const char* values) PW_INLINE {
     const int t0 = x * 32;
-    if ((t0 + 31 > ctx + rb) || (WINDOW && t0 < wave_lo_last) || rb + 31 >= qlen) mask(cur, t0);
+    // (columns without a row need no mask: their queries are zero, and what they gather goes nowhere)
+    if ((t0 + 31 > ctx + rb) || (WINDOW && t0 < wave_lo_last)) mask(cur, t0);
     const float neg[2] = {(m[0] == -INFINITY) ? 0.f : -m[0], (m[1] == -INFINITY) ? 0.f : -m[1]};
     emax[0] = emax[1] = 0.f;
     constexpr int NY = NSV;                                  // turns: a read of keys and one of values, two products each

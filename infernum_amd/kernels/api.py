@@ -1115,6 +1115,7 @@ def attention_decode_rotating(qkv, positions: torch.Tensor, inv_freq: Optional[t
 
 PREFILL_TILE_ROWS = 64      # query rows of a workgroup's tile in attention_prefill
 PREFILL_PAIRED = 0x100      # in a launch shape: 32 rows from each end of a request in place of 64 consecutive ones
+PREFILL_NARROW = 0x200      # in a launch shape: waves of 16 rows where the kernel with 32 would be taken
 
 
 def attention_prefill(qkv: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor, out: torch.Tensor,
@@ -1129,7 +1130,7 @@ def attention_prefill(qkv: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.T
     before; tiles[i] = (s, first row of a block of PREFILL_TILE_ROWS among the request's rows).  ``heads_per_workgroup``:
     0 for the kernel's own choice, or 1, 2, 4; ``paired``: a workgroup takes half a block of rows from each end of
     its request's new tokens, so that all workgroups of a request have the same work under the causal mask (every
-    block of every request must be listed then; without effect under a window).  A value of :func:`prefill_launch_shape` may stand in
+    block of every request must be listed then; without effect under a window).  A value of :func:`prefill_shape` may stand in
     ``heads_per_workgroup`` for both.  The result has the same bits whatever the shape.  ``keep``, ``softcap``, ``bias``
     and ``gate``: see :func:`attention_generic`.
     """
@@ -1158,13 +1159,13 @@ def prefill_launch_shape(nh: int, nkv: int, d: int, q_lens: Sequence[int], ctx_l
 
     Four heads a workgroup (the default at head sizes 80 to 160 with three or more query heads to a key/value
     head) read the keys least often but make few workgroups: when they would fill fewer than three quarters of
-    the compute units, two heads are taken (1,024 tokens: 33 against 43 us).  When the launch has no more
+    the compute units, two heads are taken (1,024 tokens: 30 against 38 us).  When the launch has no more
     workgroups than compute units, every workgroup runs from start to end and the longest sets the time: under
     the causal mask that is the last block of a prompt, with twice the rounds of the average one.  Paired rows
-    give all workgroups of a request the same work then (2,048 tokens: 61 against 77 us with four heads, 66 with
-    two unpaired; 2,048 after 2,048: 125 against 141).  With more workgroups than compute units the rounds of a
+    give all workgroups of a request the same work then (2,048 tokens: 54 against 66 us with four heads, 59 with
+    two unpaired; 2,048 after 2,048: 113 against 122).  With more workgroups than compute units the rounds of a
     paired workgroup in which half its waves have run out of keys cost more than the balance gains (4,096
-    tokens: 194 against 168 us), and under a window the rows of the two ends share no keys: not paired then.
+    tokens: 168 against 153 us), and under a window the rows of the two ends share no keys: not paired then.
     """
     G = nh // nkv
     widest = 4 if 80 <= d <= 160 else 2
@@ -1191,6 +1192,32 @@ def prefill_launch_shape(nh: int, nkv: int, d: int, q_lens: Sequence[int], ctx_l
     if hpw == 4 and workgroups <= cus and longest * tiles >= 1.5 * total:
         hpw = 2
     return hpw
+
+
+# Up to how many keys of the longest block of rows waves of 16 rows are ahead of those of 32 (two heads a workgroup; four): the
+# latter's workgroups take longer to start and walk twice the work one after the other.  Microseconds of 16 / 32 rows: one prompt of 20
+# tokens 5.9 / 8.9, of 257 (32 heads over 8) 13.9 / 15.5, of 478 19.8 / 18.0, of 1,024 31.6 / 29.0; 64 of 122 58.2 / 59.8, 32 of 266 82.7 / 76.7,
+# 7 of 512 40.8 / 38.8; three of 570 under a window of 512 25.1 / 25.9, 2,811 (8 over 1) under one of 512 25.3 / 23.4.  Over 395 launches of
+# 9 to 14,000 rows without chunks what this picks takes 0.3 % longer than the faster of the two, and never longer than 16 rows do.
+# A wave of 32 rows that two chunks share walks both, which all others wait for (4,096 tokens of 16 heads over 8 in chunks of 1,024 from a chunk's
+# start on 58.8 / 53.4, from 16 tokens on 60.7 / 76.5): where a request's rows do not begin on a multiple of 32 and chunks are no longer than
+# PREFILL_NARROW_CHUNK, 16 rows (183 launches under chunks: 1.3 % longer than the faster, at most 5 % longer than 16 rows).
+PREFILL_NARROW_KEYS = (600, 448)
+PREFILL_NARROW_CHUNK = 2048
+
+
+def prefill_shape(nh: int, nkv: int, d: int, q_lens: Sequence[int], ctx_lens: Sequence[int], window: int, device: torch.device) -> int:
+    """:func:`prefill_launch_shape`, with :data:`PREFILL_NARROW` added where waves of 16 rows are the faster (a head size of 128 with two and
+    more query heads to a key/value head has both; elsewhere it is without effect).  The bits of the result do not depend on it."""
+    shape = prefill_launch_shape(nh, nkv, d, q_lens, ctx_lens, window, device)
+    if shape == 0 or d != 128 or nh < 2 * nkv:
+        return shape
+    longest = max(q + c for q, c in zip(q_lens, ctx_lens))
+    if window:
+        longest = min(longest, abs(window) + 64)
+    shared = 0 < -window <= PREFILL_NARROW_CHUNK and any(c % 32 for c in ctx_lens)
+    narrow = shared or longest <= PREFILL_NARROW_KEYS[shape & 0xff == 4]
+    return shape | (PREFILL_NARROW if narrow else 0)
 
 
 # ------------------------------------------------------------- mixers with a little state from token to token

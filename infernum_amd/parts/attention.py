@@ -300,7 +300,7 @@ class Attention(Mixer):
             nd = ctx.num_decode
             if ctx.num_seqs == nd:
                 return 0
-            return K.prefill_launch_shape(nh, nkv, big, ctx.q_lens[nd:], ctx.ctx_lens[nd:], window, dev)
+            return K.prefill_shape(nh, nkv, big, ctx.q_lens[nd:], ctx.ctx_lens[nd:], window, dev)
         return (program.scalar(("attention: parts of the keys", nh, nkv, big, g, ps, self._span(1 << 60)), parts_of_the_keys),
                 program.scalar(("attention: launch shape", nh, nkv, big, window), launch_shape))
 
@@ -374,11 +374,10 @@ class Attention(Mixer):
                                gate=gate[:nd] if gate is not None else None)
         if ctx.num_seqs > nd:
             big = max(d, self.vd)
-            key = ("prefill_launch_shape", nh, nkv, big, self.mask)
+            key = ("prefill_shape", nh, nkv, big, self.mask)
             hpw = ctx.extras.get(key)
             if hpw is None:             # once per step for all layers of this shape
-                hpw = ctx.extras[key] = K.prefill_launch_shape(nh, nkv, big, ctx.q_lens[nd:], ctx.ctx_lens[nd:],
-                                                               self.mask, qkv.device)
+                hpw = ctx.extras[key] = K.prefill_shape(nh, nkv, big, ctx.q_lens[nd:], ctx.ctx_lens[nd:], self.mask, qkv.device)
             tiles, num_tiles = ctx.row_tiles(K.PREFILL_TILE_ROWS)
             K.attention_prefill(qkv, cache.k_pages, cache.v_pages, out, ctx.seq_starts, ctx.seq_ctx, bt,
                                 tiles, num_tiles, nh, nkv, d, self.scale, self.mask, hpw, sinks=self.sinks,

@@ -161,3 +161,28 @@ def test_a_value_that_is_not_finite_reaches_the_16_rows_that_meet_its_32_keys(ct
             assert torch.equal(got[~meets], want[~meets]), (t, paired)
             assert not bool(got[sees].isfinite().any()), (t, paired)
         c["vp"][page, :, :, t % ps] = was
+
+
+def test_short_ranges_of_keys_go_to_waves_of_16_rows():
+    """Where the line lies, and the same bits on both sides of it, through the shape that a step's launch is given."""
+    api = K()
+    dev = torch.device(DEV)
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    of_two, of_four = api.PREFILL_NARROW_KEYS
+    narrow = lambda q, c, nh=32, nkv=8, w=0, d=128: bool(api.prefill_shape(nh, nkv, d, q, c, w, dev) & api.PREFILL_NARROW)    # noqa: E731
+    assert narrow([20], [0]) and narrow([64], [of_two - 64]) and not narrow([64], [of_two - 63])
+    assert narrow([64] * cus, [of_four - 64] * cus) and not narrow([64] * cus, [of_four - 63] * cus)
+    assert narrow([64], [5000], w=500) and not narrow([64], [5000], w=2000)
+    chunk = api.PREFILL_NARROW_CHUNK
+    assert narrow([64], [5000], w=-chunk) and not narrow([64], [5000], w=-chunk - 1) and not narrow([64], [5024], w=-chunk)
+    assert narrow([64], [5024], w=-500)
+    assert not narrow([20], [0], nh=8) and not narrow([20], [0], d=64) and not narrow([], [])
+    for window in (0, 100, -64):
+        c = _case(8, 2, 16, [200, 33], [120, 33], seed=11)
+        shape = api.prefill_shape(8, 2, D, c["q_lens"], [80, 0], window, dev)
+        assert shape & api.PREFILL_NARROW
+        want = _run(c, 8, 2, window)
+        assert torch.equal(_run(c, 8, 2, window, heads_per_workgroup=shape), want)
+        assert torch.equal(_run(c, 8, 2, window, heads_per_workgroup=shape & ~api.PREFILL_NARROW), want)
+    with pytest.raises(api.KernelError):
+        _run(c, 8, 2, heads_per_workgroup=0x402)
