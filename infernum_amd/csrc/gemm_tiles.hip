@@ -381,8 +381,9 @@ static void choose_tile(int M, int N, int K, bool glu, int& rows, int& cols) {
 #undef GT_COST
 }
 
-// Whether this kernel or the vendor library's takes a whole product of many rows (with the activation it is this one always: 80
-// products of 130 to 4,600 rows 1.01 to 1.5 times as fast as the library's with a launch for the activation).  The library's large tile runs
+// Whether this kernel or the vendor library's takes a whole product of many rows (with the activation there is a rule of its own where the
+// routes are planned: 260 products of 129 to 8,192 rows 1.16 times as fast as the library's with a launch for the activation, up to half as fast
+// where few tiles walk a long K).  The library's large tile runs
 // 5 to 10 % faster than this kernel's (8,192 x 4,096 x 4,096 184 / 205 us, 4,096 x 4,096 x 14,336 313 / 325), so where tiles of 256 x 256
 // fill their turns of the compute units it is ahead, and for few tiles it splits K (512 x 4,096 x 14,336 85 / 110, 1,000 x 2,048 x 5,504
 // 40 / 50).  Between them, where such tiles leave a fifth of their turns empty and tiles of 128 x 128 occupy 200 units,

@@ -17,8 +17,8 @@ the same launches; ``INFERNUM_GEMM_ROUTE=measured`` times both when a model load
 the rule of sizes); for the bands of rows of :data:`KNOWN_MID_ROWS` (up to a few hundred rows) the LDS-tiled MFMA
 kernel with K split over workgroups, for products whose partial sums the next kernel takes (the library's kernels
 for so few rows leave most of the GPU idle, and from some tens of rows on the tiled kernel streams a weight faster
-than the weight-streaming one); above that the library, as the reference uses its library there, or where it is the faster (a rule
-of sizes, and always with the activation in its epilogue) the kernel of ``csrc/gemm_tiles.hip``, the same bits on the shapes tried; an fp32 result of more
+than the weight-streaming one); above that the library, as the reference uses its library there, or where it is the faster (rules
+of sizes, with the activation in its epilogue and without) the kernel of ``csrc/gemm_tiles.hip``, the same bits on the shapes tried; an fp32 result of more
 than 128 rows comes from the LDS-tiled kernel's fp32 sums (128 rows at a time from the weight-streaming kernel where
 the tiled one does not take the size).  ``set_prefill_gemm("mfma")`` (or
 INFERNUM_PREFILL_GEMM=mfma) sends the many-row bf16 products to the hand-written LDS-tiled MFMA kernel instead,
@@ -54,18 +54,18 @@ SKINNY_WIDE = 16384
 # that go to the library, for 17 to 128 rows.  Measured with ``measure_route`` on an MI355X, three times over, a
 # bit kept where most runs agreed; the shapes are those of the Llama 1B, 8B, 13B and 70B layers.  The library's
 # kernels are ahead for some shapes already at 32 rows and behind for others at 128, and no rule of sizes tells.
-# (Measured before the weight-streaming kernel asked for a chunk ahead without conditions; it has gained since, most where
-# its workgroups have a compute unit each: 16,384 x 2,048 with the activation at 32 / 64 / 128 rows 20 / 23 / 32 us then and
-# 16 / 18 / 25 now.)
+# (Measured before the weight-streaming kernel asked for a chunk ahead without conditions, but for those with the activation: the
+# weight-streaming kernel / the library's product with the activation's launch for 16,384 x 2,048 at 24, 64, 65, 96 and 128 rows 16.0, 18.5,
+# 22.1, 23.7, 28.9 / 19.6, 20.7, 21.6, 22.1, 24.0 us; the others' rows are all KNOWN_GLU_ROWS'.)
 KNOWN_ROUTES: Dict[Tuple[int, int, Optional[str], bool], int] = {
-    (3072, 2048, None, True): 0, (2048, 2048, None, True): 0, (16384, 2048, "swiglu", False): 0b11110010,
+    (3072, 2048, None, True): 0, (2048, 2048, None, True): 0, (16384, 2048, "swiglu", False): 0b11110000,
     (2048, 8192, None, True): 0,
-    (6144, 4096, None, True): 0, (4096, 4096, None, True): 0, (28672, 4096, "swiglu", False): 0b11110000,
+    (6144, 4096, None, True): 0, (4096, 4096, None, True): 0, (28672, 4096, "swiglu", False): 0,
     (4096, 14336, None, True): 0,
     (15360, 5120, None, True): 0b11111110, (5120, 5120, None, True): 0,
-    (27648, 5120, "swiglu", False): 0b11111010, (5120, 13824, None, True): 0,
+    (27648, 5120, "swiglu", False): 0, (5120, 13824, None, True): 0,
     (10240, 8192, None, True): 0, (8192, 8192, None, True): 0,
-    (57344, 8192, "swiglu", False): 0b11111110, (8192, 28672, None, True): 0,
+    (57344, 8192, "swiglu", False): 0, (8192, 28672, None, True): 0,
 }
 
 # (N, K) of a weight whose product leaves partial sums for the next kernel -> bands (first row, last row, parts): for
@@ -99,12 +99,12 @@ KNOWN_MID_ROWS: Dict[Tuple[int, int], Tuple[Tuple[int, int, int], ...]] = {
 }
 
 # (N, K) of a gate+up weight -> bands (first row, last row) in which the LDS-tiled kernel with the activation in
-# its epilogue takes the product (the 8B shape's at 32 / 64 / 128 rows: 43 / 45 / 51 us against the weight-streaming
-# kernel's 47 / 56 / 73 and the library's with the activation's launch 54 / 54 / 57).  No rule of sizes stands behind
-# this table: 22,016 x 4,096 gains as the 8B shape does (38 / 42 / 48 us against 45 / 53 / 71 and 46 / 48 / 50), while for
-# 16,384 x 3,072 and 37,888 x 3,584 the library's product with the activation's launch is ahead from 32 rows on.
+# its epilogue takes the product.  At 24 / 64 / 128 rows, us, this / weight-streaming / gemm_tiles / the library's with the activation's launch:
+# 28,672 x 4,096 46, 44, 52 / 47, 56, 74 / 53, 52, 54 / 55, 54, 57; 27,648 x 5,120 54, 56, 67 / 59, 69, 91 / 60, 60, 67 / 56, 60, 70;
+# 57,344 x 8,192 163, 162, 194 / 182, 198, 275 / 192, 185, 191 / 188, 194, 205; 22,016 x 4,096 37, 41, 49 / 42, 55, 71 / 47, 49, 49 / 45, 48, 49.
+# No rule of sizes stands behind this table: 16,384 x 3,072 29, 30, 38 / 23, 25, 40 / 34, 33, 37 / 26, 26, 31.
 KNOWN_GLU_ROWS: Dict[Tuple[int, int], Tuple[Tuple[int, int], ...]] = {
-    (28672, 4096): ((17, 128),), (27648, 5120): ((33, 128),), (57344, 8192): ((17, 128),), (16384, 2048): ((129, 256),),
+    (28672, 4096): ((17, 128),), (27648, 5120): ((17, 128),), (57344, 8192): ((17, 128),), (16384, 2048): ((129, 256),),
     (22016, 4096): ((17, 128),),
 }
 
@@ -313,6 +313,26 @@ class Route:
 
 FP32_TILED_FROM_ROWS = (49, 81)     # an fp32 result goes to the tiled kernel from so many rows on: K >= 4,096; shorter K
 FP32_TILED_WIDE, FP32_TILED_WIDE_FROM_ROWS = 24576, 17     # and with so many columns (192 tiles) from so many rows, whatever K
+GLU_TILES_TURNS = 2 ** 18
+COMPUTE_UNITS = 256        # an MI355X's
+
+
+def glu_tiles_from(N: int, Kdim: int) -> int:
+    """From how many rows on the many-row product with the activation goes to ``gemm_tiles`` and not to the library's product and a launch
+    for the activation.  Where tiles of 128 x 128 leave many compute units without one, each of which walks all of K, the library's kernels,
+    which split K or have smaller tiles, make up for their launch: from K (256 - tiles) of 2^18 on.  At most 2,048 values of K and
+    more than 64 tiles of more than 128 rows stay.  This / library and launch, us: 16,384 x 2,048 at 65 / 128 rows (128 tiles) 23.5 / 21.6 and
+    25.5 / 24.0, 16,384 x 5,120 at 128 62.7 / 46.8, 16,512 x 2,048 at 65 23.4 / 30.2, 10,752 x 5,120 at 129 / 256 rows 46.9 / 40.6 and 56.1 / 64.4,
+    2,816 x 8,192 at 150 64.9 / 30.8, 9,472 x 4,096 at 129 38.2 / 33.2, 6,144 x 2,048 at 256 16.4 / 23.4.  Over 650 products of 65
+    to 8,192 rows what this picks takes 0.5 % longer than the faster of the two, and 6 % at most than the library's."""
+    cols, first = -(-N // 128), []
+    tiles = COMPUTE_UNITS - (GLU_TILES_TURNS - 1) // Kdim          # so many 128 x 128 tiles at least
+    first.append(128 * max(0, -(-tiles // cols) - 1) + 1)
+    if Kdim <= 2048:
+        first.append(128 * max(1, 64 // cols) + 1)
+    return min(first)
+
+
 _MANY_ROWS = 65536         # the LDS-tiled kernel addresses rows with 32 bits: its fitness is judged at this many
 
 
@@ -396,7 +416,7 @@ def _run(kind: str, x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype, ep
         return K.gemm_mfma(x, w), False
     if kind == "library":
         if x.dtype == torch.bfloat16 and K.gemm_tiles_supported(M, N, x.shape[1]) and on_16_bytes(x) and on_16_bytes(w):
-            if epilogue == "swiglu":
+            if epilogue == "swiglu" and M >= glu_tiles_from(N, x.shape[1]):
                 return K.gemm_tiles(x, w, swiglu=True), True
             if K.gemm_tiles_pays(M, N, x.shape[1]):
                 return K.gemm_tiles(x, w), False
@@ -565,10 +585,16 @@ def emit_linear(program, x: Any, M: Any, w: torch.Tensor, out_dtype: torch.dtype
             program.op("core", "ia_gemm_skinny_rows", [x, wk, int(tiled is not None), out, code, M, N, Kdim, ws,
                                                         splits * small * N if splits > 1 else 0, P.STREAM], g)
             finish.emit(program, out, M, N, code, g)
-        elif r.kind == "library" and epilogue == "swiglu" and rt.dtype == torch.bfloat16 and K.gemm_tiles_supported(T, N, Kdim) and \
-                on_16_bytes(x) and on_16_bytes(w) and on_16_bytes(out):
-            program.op("core", "ia_gemm_tiles", [x, w, out, M, N, Kdim, 1, 0, 0, P.STREAM], g)
         else:
+            if r.kind == "library" and epilogue == "swiglu" and rt.dtype == torch.bfloat16 and K.gemm_tiles_supported(T, N, Kdim) and \
+                    on_16_bytes(x) and on_16_bytes(w) and on_16_bytes(out):
+                first = glu_tiles_from(N, Kdim)
+                on_tiles, g = g & P.Guard.between(M, first), g & P.Guard.between(M, None, first - 1)
+                if not on_tiles.never:
+                    program.op("core", "ia_gemm_tiles", [x, w, out, M, N, Kdim, 1, 0, 0, P.STREAM], on_tiles)
+                    alts.append(P.Alt(on_tiles, out, 0, out_dtype))
+                if g.never:
+                    continue
             # a product that leaves the whole matrix: into scratch first when an activation follows
             y = program.buffer(key + ".product", T * N * out_bytes) if epilogue == "swiglu" else out
             _emit_whole(program, r.kind, x, w, y, M, N, Kdim, in_code, code, g, False)

@@ -124,6 +124,22 @@ def test_steps_of_129_to_256_rows_through_the_tiled_kernel_with_k_split(models, 
     eng.program.check_guards()
 
 
+def test_gate_and_up_on_either_side_of_the_line_between_the_tiles_and_the_library(models, monkeypatch):
+    """Configuration B with the line at 150 rows: whole prompts below and above it, the program against the parts' calls."""
+    import importlib
+    L = importlib.import_module("infernum_amd.parts.linear")
+    d, cfg, reqs, ref = models[("B", "bfloat16", "mixed")]
+    monkeypatch.setattr(L, "glu_tiles_from", lambda N, K: 150)
+    native = _engine(d, "bfloat16", PAGE["B"], 128)
+    parts = _engine(d, "bfloat16", PAGE["B"], 128, executor="parts")
+    assert {"ia_gemm_tiles", "ia_swiglu"} <= set(native.program.op_names)
+    assert any(128 < len(t) < 150 for t in reqs.values()) and any(len(t) >= 150 for t in reqs.values())
+    a, b = TT.run_steps(native, TT.trace_whole(reqs)), TT.run_steps(parts, TT.trace_whole(reqs))
+    _check(a, ref, "bfloat16", "B bfloat16 whole, gate and up on either side of 150 rows")
+    assert a.keys() == b.keys() and all(torch.equal(a[k], b[k]) for k in a)
+    native.program.check_guards()
+
+
 @pytest.mark.parametrize("name", ["A", "B", "C"])
 def test_tail_one_by_one_rotation_inside_attention_or_before_it(models, name):
     """Steps of single tokens rotate queries and keys and write the pages inside the attention kernel; with the

@@ -156,3 +156,27 @@ def test_rows_in_groups_at_the_edges_of_each_tile(counts, times, N, K_):
             assert torch.equal(out[lo:lo + n, :512], api.gemm_tiles(x[lo:lo + n].clone(), w[g])[:, :512]), g
         lo += n
     assert bool((out[lo:] == 7.0).all())
+
+
+# a matrix whose tiles fill half the compute units (few rows to the library, with more rows here), one column tile more, one of short K
+@pytest.mark.parametrize("N,K_,first", [(16384, 2048, 129), (16512, 2048, 1), (16384, 1024, 1), (10752, 5120, 257), (2816, 1536, 257)])
+def test_where_products_with_the_activation_take_it(N, K_, first):
+    """The rule against itself written plainly, and what the route returns on both sides of its line."""
+    L = importlib.import_module("infernum_amd.parts.linear")
+    api = K()
+    assert L.glu_tiles_from(N, K_) == first
+    for M in (*range(1, 700, 7), 128, 129, 256, 257, 3000):
+        tiles = math.ceil(M / 128) * math.ceil(N / 128)
+        assert (M >= first) == (K_ * (256 - tiles) < 2 ** 18 or (K_ <= 2048 and M > 128 and tiles > 64)), M
+    w = _rand(N, K_, scale=0.05, seed=8)
+    routes = L.plan(N, K_, torch.bfloat16, torch.bfloat16, "swiglu", False)
+    for M in (65, 96, 129, 257):
+        if L.route_of(routes, M).kind != "library":
+            continue
+        x = _rand(M, K_, seed=M)
+        y = L.linear(x, w, epilogue="swiglu")
+        if M >= first:
+            want = api.gemm_tiles(x, w, swiglu=True)
+        else:
+            want = api.swiglu(api.gemm_library(x, w), torch.empty((M, N // 2), dtype=torch.bfloat16, device=DEV))
+        assert torch.equal(y, want), M
