@@ -57,7 +57,7 @@ def test_products_with_the_activation(tile, M, N, K_):
 
 
 def test_the_activation_at_its_ends():
-    """Gates that saturate to either side and infinite sums give what silu(g) u gives in fp32 (0 and u g; NaN for -inf)."""
+    """Gates that saturate to either side give what silu(g) u gives in 64 bits (0 and u g)."""
     api = K()
     gates = torch.tensor([-3e4, -200.0, -90.0, -20.0, 0.0, 20.0, 200.0, 3e4], device=DEV)
     a = torch.zeros(8, 64, dtype=torch.bfloat16, device=DEV)
@@ -180,3 +180,35 @@ def test_where_products_with_the_activation_take_it(N, K_, first):
         else:
             want = api.swiglu(api.gemm_library(x, w), torch.empty((M, N // 2), dtype=torch.bfloat16, device=DEV))
         assert torch.equal(y, want), M
+
+
+def test_the_activation_where_its_sums_are_infinite_or_its_sigmoid_is_tiny():
+    """Sums of +-inf and NaN give what silu(g) u gives in fp32; a sigmoid below the smallest normal number is not lost: to -88.5 the product
+    is that of 64 bits, and further down, where exp(-g) leaves fp32, it is that or 0."""
+    api = K()
+    inf = float("inf")
+    gates = torch.tensor([inf, -inf, float("nan"), -86.0, -87.0, -87.5, -88.0, -88.5, -89.0, -90.0, -95.0, -104.0, -3e38], device=DEV)
+    n = gates.numel()
+    a = torch.zeros(n, 64, dtype=torch.bfloat16, device=DEV)
+    a[:, 0], a[:, 1] = gates.to(torch.bfloat16), 1.0
+    w = torch.zeros(32, 64, dtype=torch.bfloat16, device=DEV)
+    w[:16, 0], w[16:, 1] = 1.0, 2.0
+    w[16:, 0] = 0.0
+    out = api.gemm_tiles(a, w, swiglu=True).double()
+    g = a[:, 0].double()
+    g[:3] = gates[:3].double()
+    want = (g * torch.sigmoid(g) * 2.0)[:, None].expand(n, 16)
+    # an infinite or NaN value times the weights' zeros makes up NaN as well: the gate's own sum stays what it is only in the products' first
+    # factor, so that row 0 to 2 are NaN whatever the activation does; the rest is finite
+    assert bool(out[:3].isnan().all()) and bool(out[3:].isfinite().all())
+    assert bool(((out[3:8] - want[3:8]).abs() <= 2.0 ** -7 * want[3:8].abs()).all())
+    assert bool(((out[8:] - want[8:]).abs() <= 2.0 ** -7 * want[8:].abs()).logical_or(out[8:] == 0).all())
+    # sums that are infinite by themselves: 2 x 3e38
+    big = torch.full((4, 64), 0.0, dtype=torch.bfloat16, device=DEV)
+    big[:, 0] = big[:, 1] = torch.tensor([3e38, -3e38, 3e38, -3e38], device=DEV).to(torch.bfloat16)
+    big[:, 2] = torch.tensor([1.0, 1.0, -1.0, 0.0], device=DEV).to(torch.bfloat16)
+    w = torch.zeros(32, 64, dtype=torch.bfloat16, device=DEV)
+    w[:16, :2], w[16:, 2] = 1.0, 2.0
+    out = api.gemm_tiles(big, w, swiglu=True).float()
+    g, u = (big.float() @ w.float().t()).split(16, dim=1)
+    assert bool(g.isinf().all()) and torch.equal(torch.nan_to_num(out, nan=7.0), torch.nan_to_num(torch.nn.functional.silu(g) * u, nan=7.0))
