@@ -32,26 +32,39 @@ def _registers(text):
     return set(range(int(span.group(1)), int(span.group(2)) + 1)) if span else set()
 
 
+def _instructions(text):
+    return [(op, [x.strip() for x in args.split(",")]) for op, args in re.findall(r"^\s+([a-z]\w+) ?(.*?)$", text, re.M)]
+
+
 def test_operands_of_the_loops_come_from_lds_alone(assembly):
     kernels = re.findall(r"^(_Z\w*gemm_tiles_kernel\w+):(.*?)\.end_amdhsa_kernel", assembly, re.S | re.M)
     assert len(kernels) >= 15
     for name, body in kernels:
-        loops = [part for part in re.split(r"^\.LBB\d+_\d+:", body, flags=re.M) if "v_mfma_f32_16x16x32_bf16" in part]
-        assert len(loops) >= 2, name                    # two steps a turn, and the odd last one
-        for part in loops:
-            part = part[part.index("v_mfma"):part.rindex("v_mfma") + 200]
+        blocks = re.split(r"^(\.LBB\d+_\d+):", body, flags=re.M)
+        loops = 0
+        for label, part in zip(blocks[1::2], blocks[2::2]):
+            if "v_mfma_f32_16x16x32_bf16" not in part:
+                continue
+            found = _instructions(part)
+            matrix = [i for i, (op, _) in enumerate(found) if op == "v_mfma_f32_16x16x32_bf16"]
+            again = any(op.startswith("s_cbranch") and args[0] == label for op, args in found)
+            # a loop's body from its label to its branch, and once more from there: what its end leaves meets its beginning; the odd last
+            # step, and what stands in front of it in its block, up to its last product
+            found = found + found if again else found[:matrix[-1] + 1]
+            loops += again
             wrote = {}                                  # register -> the instruction that wrote it last
-            for op, args in re.findall(r"^\s+([vd]\w+) (.*)$", "\t" + part, re.M):
-                args = [x.strip() for x in args.split(",")]
+            for op, args in found:
                 if op == "v_mfma_f32_16x16x32_bf16":
                     assert args[0] == args[3] and args[0].startswith("a["), (name, args)
                     for r in _registers(args[1]) | _registers(args[2]):
-                        assert wrote.get(r, "ds_read_b128") == "ds_read_b128", (name, r, wrote[r])
-                    continue
-                assert "accvgpr" not in op and (op.startswith("v_") or op == "ds_read_b128"), (name, op)
-                for r in _registers(args[0]):
-                    wrote[r] = op
-            assert "scratch_" not in part[:part.rindex("v_mfma")], name
+                        assert wrote.get(r, "ds_read_b128") == "ds_read_b128", (name, label, r, wrote[r])
+                elif op.startswith(("v_", "ds_read")):
+                    assert "accvgpr" not in op, (name, label, op)
+                    for r in _registers(args[0]):
+                        wrote[r] = op
+                else:
+                    assert op.startswith(("s_", "buffer_load")) and "scratch" not in op, (name, label, op)
+        assert loops >= 1 and sum("v_mfma" in p for p in blocks[2::2]) >= 2, name       # two steps a turn, and the odd last one
 
 
 TILES = [(256, 256), (256, 224), (256, 192), (256, 160), (256, 128), (224, 256), (192, 256), (192, 192), (192, 128), (160, 256),

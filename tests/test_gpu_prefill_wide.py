@@ -186,3 +186,52 @@ def test_short_ranges_of_keys_go_to_waves_of_16_rows():
         assert torch.equal(_run(c, 8, 2, window, heads_per_workgroup=shape & ~api.PREFILL_NARROW), want)
     with pytest.raises(api.KernelError):
         _run(c, 8, 2, heads_per_workgroup=0x402)
+
+
+@pytest.mark.parametrize("nh,nkv,ps", [(4, 1, 16), (6, 2, 8), (4, 2, 64)])
+@pytest.mark.parametrize("lens,q_lens", [([1, 2, 31, 32, 33], [1, 2, 31, 32, 33]), ([95, 96, 97, 200, 161], [1, 33, 65, 64, 7]),
+                                         ([300, 449], [300, 100])])
+@pytest.mark.parametrize("chunk", [1, 16, 48, 64, 100, 300])
+def test_chunks_at_the_edges_of_tiles(nh, nkv, ps, lens, q_lens, chunk):
+    c = _case(nh, nkv, ps, lens, q_lens, seed=nh * ps + len(lens) + chunk)
+    rows, at = [], 0
+    for k, v, n, m in zip(c["k"], c["v"], c["lens"], c["q_lens"]):
+        q = c["q"][at:at + m].view(m, nh, D).double()
+        at += m
+        pos, key = torch.arange(n - m, n, device=DEV)[:, None], torch.arange(n, device=DEV)[None, :]
+        s = torch.einsum("qhd,khd->hqk", q, k.double().repeat_interleave(nh // nkv, dim=1)) * D ** -0.5
+        p = torch.softmax(s.masked_fill((key > pos) | (key < pos // chunk * chunk), -math.inf), dim=-1)
+        rows.append(torch.einsum("hqk,khd->qhd", p, v.double().repeat_interleave(nh // nkv, dim=1)).reshape(m, nh * D))
+    want = torch.cat(rows)
+    first = _run(c, nh, nkv, -chunk)
+    # as above: probabilities within 2^-9 of themselves, values of order one (a chunk of one key: of up to 4.5), one rounding to bf16
+    assert ((first.double() - want).abs() <= 1.5e-2 + 2.0 ** -8 * want.abs()).all(), (first.double() - want).abs().max().item()
+    for hpw in (1, 2, 4, K().PREFILL_NARROW | 2):
+        assert torch.equal(_run(c, nh, nkv, -chunk, heads_per_workgroup=hpw), first), hpw
+
+
+@pytest.mark.parametrize("lens,q_lens", [([1, 2, 31, 32, 33], [1, 2, 31, 32, 33]), ([95, 200, 161], [1, 64, 7]), ([300, 449], [300, 100])])
+@pytest.mark.parametrize("window", [0, 40])
+def test_sinks_and_rows_that_lie_apart(lens, q_lens, window):
+    """A sink takes its share of every row's probabilities; queries and results as column ranges of wider rows."""
+    nh, nkv, ps = 8, 2, 16
+    c = _case(nh, nkv, ps, lens, q_lens, seed=21)
+    sinks = torch.linspace(-3.0, 6.0, nh, device=DEV)
+    rows, at = [], 0
+    for k, v, n, m in zip(c["k"], c["v"], c["lens"], c["q_lens"]):
+        q = c["q"][at:at + m].view(m, nh, D).double()
+        at += m
+        pos, key = torch.arange(n - m, n, device=DEV)[:, None], torch.arange(n, device=DEV)[None, :]
+        s = torch.einsum("qhd,khd->hqk", q, k.double().repeat_interleave(nh // nkv, dim=1)) * D ** -0.5
+        s = s.masked_fill((key > pos) | ((key <= pos - window) if window else (key < 0)), -math.inf)
+        p = torch.softmax(torch.cat([s, sinks.double()[:, None, None].expand(nh, m, 1)], dim=2), dim=-1)[:, :, :-1]
+        rows.append(torch.einsum("hqk,khd->qhd", p, v.double().repeat_interleave(nh // nkv, dim=1)).reshape(m, nh * D))
+    first = _run(c, nh, nkv, window, sinks=sinks)
+    assert (first.double() - torch.cat(rows)).abs().max().item() <= 2.5e-2
+    assert torch.equal(_run(c, nh, nkv, window, sinks=sinks, heads_per_workgroup=K().PREFILL_NARROW | 4), first)
+    wide_q = torch.full((c["q"].shape[0], nh * D + 2 * nkv * D), float("nan"), dtype=torch.bfloat16, device=DEV)
+    wide_q[:, :nh * D] = c["q"]
+    wide_o = torch.full((c["q"].shape[0], nh * D + 64), 7.0, dtype=torch.bfloat16, device=DEV)
+    K().attention_prefill(wide_q[:, :nh * D], c["kp"], c["vp"], wide_o[:, :nh * D], c["starts"], c["ctx"], c["bt"], c["tiles"],
+                          c["tiles"].shape[0], nh, nkv, D, D ** -0.5, window, sinks=sinks)
+    assert torch.equal(wide_o[:, :nh * D], first) and bool((wide_o[:, nh * D:] == 7.0).all())
