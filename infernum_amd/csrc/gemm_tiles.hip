@@ -432,22 +432,54 @@ extern "C" int ia_gemm_tiles(const void* X, const void* W, void* C, int M, int N
 //   20 experts of 2,432 x 4,096, 161 rows each 243 -> 219 / 140 -> 111   32 of 1,408 x 2,048, 255 rows 165 -> 136 / 97 -> 73
 //   16 of 1,408 x 2,048, 256 rows 79 -> 71 / 53 -> 33                    8 of 2,752 x 2,048 without a gate, 500 rows 66 -> 61 / 81 -> 52
 
-// How many rows the tiles of `rows` rows multiply for groups whose sizes differ as those of a random choice do.
-static long grouped_rows(int groups, int mean, int rows) {
-  const double spread = std::sqrt((double)mean);
-  long tiles = 0;
-  for (const double d : {-1.2, -0.5, 0.0, 0.5, 1.2}) {
-    const int n = (int)(mean + d * spread);
-    tiles += ((n < 1 ? 1 : n) + rows - 1) / rows;
+// The tiles: rows of X and of W, and as template arguments.
+#define GT_GROUP_TILES(G)                                                                                                    \
+  G(96, 128, 2, 1, 2, 2) G(128, 128, 2, 2, 2, 2) G(160, 128, 3, 2, 2, 2) G(192, 128, 3, 3, 2, 2) G(128, 256, 2, 2, 4, 4)     \
+  G(192, 256, 3, 3, 4, 4) G(256, 256, 4, 4, 4, 4)
+
+// Which tile: the one with the least estimated time, in us.  A workgroup takes K / 64 steps of 0.24 a 256 x 256 tile's products, 0.47 the
+// loads of its bm + bn rows and 0.07 besides, and 10 times the square root of its area around them; two that share a compute unit take
+// 1.93 of their steps and 0.6 of the rest.  A few tiles beyond a turn of the compute units are a whole turn more, so how many there will be
+// is taken for groups whose sizes differ as those of a random choice do (mean and variance the same): sum over k of the probability that
+// a group has more than k tiles' rows.  The constants are a fit to 400 products of 4 to 128 groups of 49 to 1,024 rows on average, 1,024 to
+// 28,672 columns, K of 768 to 14,336, with ten tiles each: what it picks takes 1.9 % longer than the fastest, and 0.82 of the tiles of 128 x
+// 256 of 32 x 32 x 16 instructions (0.85 by the rule before, which lost more than 3 % to those in 43 products, up to 1.45: 32 groups of 1,408 x 2,048
+// with 80 rows, second product, 48 / 68 / 48 us by those tiles, that rule and this; 20 of 14,336 x 4,096 with 192 rows 741 / 868 / 683; 16 of
+// 2,432 x 4,096 with 90 rows 73 / 97 / 71).
+static double grouped_cost(int groups, int mean, int N, int K, int bm, int bn) {
+  double strips = 1.0;                                                       // of rows, a group
+  for (long k = 1;; ++k) {
+    const double more = 0.5 * std::erfc((k * bm + 0.5 - mean) / std::sqrt(2.0 * (mean > 0 ? mean : 1)));
+    if (more < 1e-4) break;
+    strips += more;
   }
-  return tiles * groups * rows;
+  const double tiles = strips * groups * ((N + bn - 1) / bn), area = (double)bm * bn / 65536;
+  const double one = K / GT_BK * (0.24 * area + 0.47 * (bm + bn) / 512 + 0.07), around = 10.0 * std::sqrt(area);
+  const auto least = [](double a) { return a < 1.0 ? a : 1.0; };
+  if ((bm + bn) * 256 > GT_LDS / 2) {
+    const double turns = std::floor(tiles / 256);
+    return turns < 1 ? around + one : (turns + least((tiles - 256 * turns) / 16)) * (around + one);
+  }
+  const double pair = 0.6 * around + 1.93 * one, turns = std::floor(tiles / 512), rest = tiles - 512 * turns;
+  if (rest < 1) return turns * pair;
+  return turns * pair + around + one + (rest > 256 ? (pair - around - one) * least((rest - 256) / 8) : 0.0);
 }
 
-// Which tile: of 160 x 128 and 192 x 128, two of which share a compute unit, the one that multiplies fewer rows in all (255 rows of
-// 1,408 x 2,048 136 / 140 us, 340 of 2,432 x 4,096 400 / 290, 512 of 1,408 x 2,048 262 / 220).  96 x 128 up to 90 rows (75 rows of
-// 1,408 x 2,048 90 us, 94 with 160 x 128; 100 rows of 2,432 x 4,096 233 / 164) and where 160 x 128 would not give every unit one
-// (16 of 1,408 x 2,048 with 150 rows 25 / 33), and of these 96 x 256 where that turns more tiles than units into fewer (16 of 1,408 x 2,048
-// with 75 rows 48 / 43).  Over 38 products of 49 to 1,024 rows this takes 2.6 % longer than the fastest of ten tiles.
+// The tile for a mean of `mean` rows a group: its rows * 1,024 + its columns.
+extern "C" int ia_gemm_tiles_grouped_tile(int groups, int mean, int N, int K) {
+  if (groups <= 0 || mean < 0 || N <= 0 || K <= 0) return 0;
+  double best = -1.0;
+  int tile = 0;
+#define GT_GROUP_COST(BM, BN, ...)                                                  \
+  {                                                                                 \
+    const double cost = grouped_cost(groups, mean, N, K, BM, BN);                   \
+    if (best < 0.0 || cost < best) { best = cost; tile = BM * 1024 + BN; }          \
+  }
+  GT_GROUP_TILES(GT_GROUP_COST)
+#undef GT_GROUP_COST
+  return tile;
+}
+
 extern "C" int ia_gemm_tiles_grouped(const void* X, const void* W, void* C, const int* rows_at, int groups, int among, int rows, int N, int K,
                                      hipStream_t stream) {
   if (groups <= 0 || among < groups || !rows_at) return IA_ERR_BAD_ARG;
@@ -458,16 +490,12 @@ extern "C" int ia_gemm_tiles_grouped(const void* X, const void* W, void* C, cons
   if (256ULL * K * 2 > 0xffffffffULL - GT_AHEAD) return IA_ERR_UNSUPPORTED;
   const uint16_t *x = (const uint16_t*)X, *w = (const uint16_t*)W;
   uint16_t* c = (uint16_t*)C;
-  const int mean = rows / among;
-  const long long strips = (N + 127) / 128, of_96 = (mean + 95) / 96, of_160 = (mean + 159) / 160;
-  if (mean <= 90 || groups * of_160 * strips <= 256) {
-    if (groups * of_96 * strips > 256 && groups * of_96 * ((N + 255) / 256) <= 256)
-      return launch_gemm_tiles<2, 1, 4, 4, GT_GROUPED>(x, w, c, rows, N, K, rows_at, groups, stream);
-    return launch_gemm_tiles<2, 1, 2, 2, GT_GROUPED>(x, w, c, rows, N, K, rows_at, groups, stream);
-  }
-  if (grouped_rows(groups, mean, 160) < grouped_rows(groups, mean, 192))
-    return launch_gemm_tiles<3, 2, 2, 2, GT_GROUPED>(x, w, c, rows, N, K, rows_at, groups, stream);
-  return launch_gemm_tiles<3, 3, 2, 2, GT_GROUPED>(x, w, c, rows, N, K, rows_at, groups, stream);
+  const int tile = ia_gemm_tiles_grouped_tile(groups, rows / among, N, K);
+#define GT_GROUP_ONE(BM, BN, TX0, TX1, TW0, TW1) \
+  if (tile == BM * 1024 + BN) return launch_gemm_tiles<TX0, TX1, TW0, TW1, GT_GROUPED>(x, w, c, rows, N, K, rows_at, groups, stream);
+  GT_GROUP_TILES(GT_GROUP_ONE)
+#undef GT_GROUP_ONE
+  return IA_ERR_BAD_ARG;
 }
 
 // ---- the launchers of this file as operations of a step's program (see op_call.h) ----

@@ -135,8 +135,8 @@ def test_where_whole_products_take_it(M, N, K_):
     assert api.gemm_tiles_pays(M, N, K_) == want
 
 
-# rows of the groups (and how often these repeat), columns, K; which tile they lead to: 96 x 128 as few workgroups, 96 x 256, 160 x 128,
-# 192 x 128; a tile's last row and one more, one row, none; columns that fill no tile, of two starts of the walk, off 16 bytes
+# rows of the groups (and how often these repeat), columns, K: a tile's last row and one more, one row, none; columns that fill no tile, of
+# two starts of the walk, off 16 bytes
 @pytest.mark.parametrize("counts,times,N,K_", [((96, 97, 0, 1, 95, 192), 1, 200, 64), ((3,), 1, 130, 320), ((96, 97, 0, 1, 95, 64), 6, 1032, 192),
                                                ((160, 161, 0, 1, 159, 300), 6, 1032, 320), ((192, 193, 0, 1, 191, 500), 6, 1032, 448)])
 def test_rows_in_groups_at_the_edges_of_each_tile(counts, times, N, K_):
@@ -212,3 +212,34 @@ def test_the_activation_where_its_sums_are_infinite_or_its_sigmoid_is_tiny():
     out = api.gemm_tiles(big, w, swiglu=True).float()
     g, u = (big.float() @ w.float().t()).split(16, dim=1)
     assert bool(g.isinf().all()) and torch.equal(torch.nan_to_num(out, nan=7.0), torch.nan_to_num(torch.nn.functional.silu(g) * u, nan=7.0))
+
+
+# every tile that the choice can fall on: the mean rows of so many groups that lead to it
+@pytest.mark.parametrize("tile,groups,mean,N,K_", [((96, 128), 12, 50, 200, 192), ((128, 128), 48, 97, 1034, 64), ((160, 128), 48, 128, 1032, 64),
+                                                   ((192, 128), 48, 161, 1032, 64), ((128, 256), 48, 97, 1034, 2048),
+                                                   ((192, 256), 48, 161, 1032, 2048), ((256, 256), 48, 200, 1032, 448)])
+def test_each_tile_of_rows_in_groups(tile, groups, mean, N, K_):
+    """Groups of a tile's rows, one more and one less, of one row and of none, the others such that the mean is kept."""
+    api = K()
+    bm = tile[0]
+    assert api._core().ia_gemm_tiles_grouped_tile(groups, mean, N, K_) == bm * 1024 + tile[1]
+    counts = [bm, bm + 1, 0, 1, bm - 1, 2 * bm]
+    left = mean * groups - sum(counts)
+    counts += [left // (groups - 6)] * (groups - 7)
+    counts.append(mean * groups - sum(counts))
+    assert min(counts) >= 0 and sum(counts) // groups == mean
+    x, w = _rand(sum(counts), K_, seed=5), _rand(groups, N, K_, scale=0.1, seed=6)
+    at = torch.tensor([0] + counts, device=DEV).cumsum(0).int()
+    out = torch.full((sum(counts), N), 7.0, dtype=torch.bfloat16, device=DEV)
+    api.gemm_mfma_grouped(x, w, at, out)
+    lo = 0
+    for g, n in enumerate(counts):
+        want = x[lo:lo + n].double() @ w[g].double().t()
+        # as for whole products above
+        assert bool(((out[lo:lo + n].double() - want).abs() <= 2e-5 * math.sqrt(K_) * 0.1 + 2.0 ** -8 * want.abs()).all()), g
+        if n and g < 8:                                                 # the first 512 columns begin their walk over K at 0
+            assert torch.equal(out[lo:lo + n, :512], api.gemm_tiles(x[lo:lo + n].clone(), w[g])[:, :512]), g
+        lo += n
+    rows = sum(counts) - 1                                              # the same bits, whichever tile: of the last group as if it were alone
+    alone = api.gemm_mfma_grouped(x[rows:].contiguous(), w[-1:].contiguous(), torch.tensor([0, 1], dtype=torch.int32, device=DEV))
+    assert torch.equal(alone[0], out[rows])
