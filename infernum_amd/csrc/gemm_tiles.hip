@@ -392,13 +392,15 @@ static void choose_tile(int M, int N, int K, bool glu, int& rows, int& cols) {
 // the choice of a tile gains: 2,048 x 4,096 x 14,336 208 / 184, 1,500 x 6,144 x 4,096 77 / 66, 2,300 x 2,048 x 8,192 86 / 74.  With short
 // K and more than half a turn of large tiles the library is ahead again (5,700 x 2,048 x 2,048 43 / 48, 3,737 x 3,072 x 2,048 43 / 46); with
 // long K and more than a turn it has kernels that take half as long again as their neighbours (4,096 columns, K = 14,336 at
-// 4,600 / 5,700 / 6,600 / 7,650 rows 765 / 764 / 847 / 966 us, this one 415 / 515 / 579 / 651).
+// 4,600 / 5,700 / 6,600 / 7,650 rows 765 / 764 / 847 / 966 us, this one 415 / 515 / 579 / 651), from K = 10,240 on more often than not (with K of
+// 8,192 it is ahead, 10,240 columns and 4,600 rows 494 / 548, 9,472 and 3,000 325 / 352, or behind, 9,472 and 4,096 655 / 462).  Over 403 products
+// of 400 to 8,192 rows this rule's picks take 0.92 of the library's time, 12 of them more than 3 % longer, at most 11 %.
 extern "C" int ia_gemm_tiles_pays(int M, int N, int K) {
   if (!gemm_tiles_takes(M, N, K)) return 0;
   const long large = (long)((M + 255) / 256) * ((N + 255) / 256), small = (long)((M + 127) / 128) * ((N + 127) / 128);
   const long places = (large + 255) / 256 * 256;                          // in the turns that the large tiles need
   if (small < 200 || K < 2048 || (K < 4096 && large > 140)) return 0;
-  return places * 100 >= large * (K >= 8192 && large > 256 ? 106 : 120);
+  return places * 100 >= large * (K >= 10240 && large > 256 ? 106 : 120);
 }
 
 // X [M, K], W [N, K], C [M, N] (glu: [M, N / 2], N even), bf16, contiguous, on 16 bytes.  rows, cols: the tile; 0: chosen here; rows < 0:

@@ -124,14 +124,14 @@ def test_many_rows_take_it_where_it_is_the_faster(M, N, K_, off):
 
 @pytest.mark.parametrize("M,N,K_", [(2048, 4096, 14336), (8192, 4096, 14336), (7650, 4096, 14336), (512, 4096, 14336), (1500, 6144, 4096),
                                    (300, 4096, 4096), (5700, 2048, 2048), (2300, 2048, 8192), (3000, 2048, 2048), (2048, 4096, 1984),
-                                   (2048, 4096, 4100), (70000, 4096, 32768)])
+                                   (2048, 4096, 4100), (70000, 4096, 32768), (4600, 10240, 8192), (7650, 4096, 10240)])
 def test_where_whole_products_take_it(M, N, K_):
     """The rule of sizes against itself written plainly."""
     api = K()
     large, small = math.ceil(M / 256) * math.ceil(N / 256), math.ceil(M / 128) * math.ceil(N / 128)
     empty = math.ceil(large / 256) * 256 / large
     want = (K_ % 64 == 0 and max(M, N) * K_ * 2 < 2 ** 32 - 3072 and small >= 200 and K_ >= 2048 and (K_ >= 4096 or large <= 140)
-            and empty >= (1.06 if K_ >= 8192 and large > 256 else 1.2))
+            and empty >= (1.06 if K_ >= 10240 and large > 256 else 1.2))
     assert api.gemm_tiles_pays(M, N, K_) == want
 
 
