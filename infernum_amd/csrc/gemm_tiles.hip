@@ -439,32 +439,46 @@ extern "C" int ia_gemm_tiles(const void* X, const void* W, void* C, int M, int N
   G(96, 128, 2, 1, 2, 2) G(128, 128, 2, 2, 2, 2) G(160, 128, 3, 2, 2, 2) G(192, 128, 3, 3, 2, 2) G(128, 256, 2, 2, 4, 4)     \
   G(192, 256, 3, 3, 4, 4) G(256, 256, 4, 4, 4, 4)
 
-// Which tile: the one with the least estimated time, in us.  A workgroup takes K / 64 steps of 0.24 a 256 x 256 tile's products, 0.47 the
-// loads of its bm + bn rows and 0.07 besides, and 10 times the square root of its area around them; two that share a compute unit take
-// 1.93 of their steps and 0.6 of the rest.  A few tiles beyond a turn of the compute units are a whole turn more, so how many there will be
-// is taken for groups whose sizes differ as those of a random choice do (mean and variance the same): sum over k of the probability that
-// a group has more than k tiles' rows.  The constants are a fit to 400 products of 4 to 128 groups of 49 to 1,024 rows on average, 1,024 to
-// 28,672 columns, K of 768 to 14,336, with ten tiles each: what it picks takes 1.9 % longer than the fastest, and 0.82 of the tiles of 128 x
-// 256 of 32 x 32 x 16 instructions (0.85 by the rule before, which lost more than 3 % to those in 43 products, up to 1.45: 32 groups of 1,408 x 2,048
-// with 80 rows, second product, 48 / 68 / 48 us by those tiles, that rule and this; 20 of 14,336 x 4,096 with 192 rows 741 / 868 / 683; 16 of
-// 2,432 x 4,096 with 90 rows 73 / 97 / 71).
+// Which tile: the one with the least estimated time, in us.  A workgroup takes K / 64 steps of 0.61 a 256 x 256 tile's products, 0.43 the
+// loads of its bm + bn rows and 0.1 besides, and 15.6 times the square root of its area around them; two that share a compute unit take
+// 2.03 of their steps and 0.74 of the rest.  A few tiles beyond a turn of the compute units are a whole turn more, and how many there will be
+// is not known on the host: the estimate is the mean over groups whose sizes differ as those of a random choice do and by 0.3 of their
+// mean beside that, each with as many tiles more and less as the groups' last ones scatter by.  Tiles that have a unit to themselves count 1.1
+// times: a turn of theirs that was not expected costs the most, and they cost the chip its clock (192 x 256 and 256 x 256 3 and 4 % longer over 15 ms
+// than over 12 launches; 8 groups of 404 rows of 2,752 x 2,048 and of 2,048 x 2,752 took 53 + 52 us with two of them and 59 + 59 with 160 x 128,
+// yet the pass of 2.7 ms that they are in 0.6 % longer).
+// The constants are a fit to 478 products of 4 to 128 groups of 49 to 1,024 rows on average (and those of the benchmark's designs, up to
+// 2,048), 1,024 to 28,672 columns, K of 768 to 14,336, of sizes that differ in these two ways and by 0.6 of the mean, each of ten tiles for
+// 15 ms: what it picks takes 3.9 % longer than the fastest (2 % if the sizes were known).  Against 96 x 128, 160 x 128 or 192 x 128 by the mean
+// rows it takes 0.96 of the time, more than 3 % longer in 41 of them, at most 1.25 times (by the mean / now, N x K: 16 groups of 187 rows,
+// 1,408 x 2,048 57 / 40 us; 8 of 175, 2,048 x 2,752 50 / 35; 16 of 187, 2,432 x 4,096 116 / 94; but 20 of 102, 4,096 x 2,432 100 / 118, 8 of 2,048,
+// 2,752 x 2,048 181 / 221, three tiles beyond three turns).
+static double grouped_strips(double mean, double spread, int bm) {           // of rows, a group: sum over k of how likely it has more than k
+  const double sd = std::sqrt(mean + spread * spread * mean * mean);
+  if (sd > bm) return mean / bm + 0.5;
+  const double sure = std::floor((mean - 4.0 * sd) / bm);
+  double strips = sure > 0.0 ? sure : 0.0;
+  for (double k = strips; k * bm < mean + 4.0 * sd; k += 1.0) strips += 0.5 * std::erfc((k * bm + 0.5 - mean) / (1.4142135623730951 * sd));
+  return strips;
+}
+
 static double grouped_cost(int groups, int mean, int N, int K, int bm, int bn) {
-  double strips = 1.0;                                                       // of rows, a group
-  for (long k = 1;; ++k) {
-    const double more = 0.5 * std::erfc((k * bm + 0.5 - mean) / std::sqrt(2.0 * (mean > 0 ? mean : 1)));
-    if (more < 1e-4) break;
-    strips += more;
-  }
-  const double tiles = strips * groups * ((N + bn - 1) / bn), area = (double)bm * bn / 65536;
-  const double one = K / GT_BK * (0.24 * area + 0.47 * (bm + bn) / 512 + 0.07), around = 10.0 * std::sqrt(area);
+  const double area = (double)bm * bn / 65536, around = 15.6 * std::sqrt(area);
+  const double walk = K / GT_BK * (0.613 * area + 0.431 * (bm + bn) / 512 + 0.104), one = around + walk;
+  const bool shared = (bm + bn) * 256 <= GT_LDS / 2;
+  const double pair = 0.736 * around + 2.03 * walk, cols = (N + bn - 1) / bn;
   const auto least = [](double a) { return a < 1.0 ? a : 1.0; };
-  if ((bm + bn) * 256 > GT_LDS / 2) {
-    const double turns = std::floor(tiles / 256);
-    return turns < 1 ? around + one : (turns + least((tiles - 256 * turns) / 16)) * (around + one);
+  const auto time = [&](double tiles) {
+    const double units = shared ? 512 : 256, turns = std::floor(tiles / units), rest = tiles - units * turns;
+    if (!shared) return 1.1 * one * (tiles < 256 ? 1.0 : turns + (rest > 0.0 ? 0.87 + 0.13 * least(rest / 26) : 0.0));
+    return turns * pair + (rest > 0.0 ? one : 0.0) + (rest > 256 ? (pair - one) * least((rest - 256) / 12) : 0.0);
+  };
+  double sum = 0.0;
+  for (const double spread : {0.0, 0.3}) {
+    const double tiles = grouped_strips(mean > 0 ? mean : 1, spread, bm) * groups * cols, more = cols * std::sqrt(groups * 0.125);
+    sum += time(tiles - more > 1.0 ? tiles - more : 1.0) + time(tiles) + time(tiles + more);
   }
-  const double pair = 0.6 * around + 1.93 * one, turns = std::floor(tiles / 512), rest = tiles - 512 * turns;
-  if (rest < 1) return turns * pair;
-  return turns * pair + around + one + (rest > 256 ? (pair - around - one) * least((rest - 256) / 8) : 0.0);
+  return sum;
 }
 
 // The tile for a mean of `mean` rows a group: its rows * 1,024 + its columns.

@@ -215,9 +215,9 @@ def test_the_activation_where_its_sums_are_infinite_or_its_sigmoid_is_tiny():
 
 
 # every tile that the choice can fall on: the mean rows of so many groups that lead to it
-@pytest.mark.parametrize("tile,groups,mean,N,K_", [((96, 128), 12, 50, 200, 192), ((128, 128), 48, 97, 1034, 64), ((160, 128), 48, 128, 1032, 64),
-                                                   ((192, 128), 48, 161, 1032, 64), ((128, 256), 48, 97, 1034, 2048),
-                                                   ((192, 256), 48, 161, 1032, 2048), ((256, 256), 48, 200, 1032, 448)])
+@pytest.mark.parametrize("tile,groups,mean,N,K_", [((96, 128), 12, 50, 200, 192), ((128, 128), 32, 104, 1034, 64), ((160, 128), 16, 141, 2056, 64),
+                                                   ((192, 128), 16, 176, 2056, 64), ((128, 256), 8, 623, 1034, 2752),
+                                                   ((192, 256), 8, 827, 1290, 2752), ((256, 256), 8, 884, 1546, 1024)])
 def test_each_tile_of_rows_in_groups(tile, groups, mean, N, K_):
     """Groups of a tile's rows, one more and one less, of one row and of none, the others such that the mean is kept."""
     api = K()
