@@ -11,8 +11,9 @@
 // lane (col, q) with the keys 8 q .. 8 q + 7: what the second product wants of the probabilities, and 16 contiguous bytes of a row
 // of V^T, as pages hold it.
 //
-// What bounds it: a SIMD has two such waves, whose matrix instructions take 2,176 cycles a tile, their exponentials and what goes with
-// them some 1,700, and whose reads of LDS (256 KB a tile and compute unit, half of what waves of 16 rows need) 2,048.  These have to run
+// What bounds it: with four heads a workgroup a SIMD has two such waves (LDS holds one workgroup a compute unit: one wave a SIMD with two
+// heads, every other SIMD has none with one), whose matrix instructions take 2,176 cycles a tile, their exponentials and what goes with them
+// some 1,700, and whose reads of LDS (256 KB a tile and compute unit, half of what waves of 16 rows need) 2,048.  These have to run
 // beside each other: a piece of a pair of exponentials of 32 keys' scores stands behind every product of the next 32's scores and every one of the
 // probabilities of the 32 before.  The 8B shape's heads (32 over 8), waves of 16 rows / this kernel, us: 2,048 tokens 70 / 55, 4,096
 // 191 / 148, 8,192 662 / 508 (1.08 PFLOP/s), 2,048 after 6,144 cached 293 / 226; under a window of 4,096 8,192 tokens 512 / 412.  Short ranges
