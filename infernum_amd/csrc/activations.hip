@@ -27,7 +27,7 @@ __global__ __launch_bounds__(256) void gelu_tanh_bf16x8_kernel(const uint4* __re
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const float lo = ia_activate(__uint_as_float(w[k] << 16), IA_ACT_GELU_TANH), hi = ia_activate(__uint_as_float(w[k] & 0xffff0000u), IA_ACT_GELU_TANH);
-      o[k] = (uint32_t)float_to_bf16_bits(lo) | ((uint32_t)float_to_bf16_bits(hi) << 16);
+      o[k] = two_bf16_bits(lo, hi);
     }
     out[i] = make_uint4(o[0], o[1], o[2], o[3]);
   }

@@ -584,8 +584,8 @@ __global__ __launch_bounds__(WAVES * 64, ((WAVES == 4 && IA_MAX_DIM <= 128) ? 3 
       float ov[4] = {acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
       if (BIAS && X.gate) attn_gate4(ov, X.gate + (size_t)b * X.gate_stride + (size_t)h * VD + 4 * qd + n * 16);
       uint2 wv;
-      wv.x = (uint32_t)float_to_bf16_bits(ov[0]) | ((uint32_t)float_to_bf16_bits(ov[1]) << 16);
-      wv.y = (uint32_t)float_to_bf16_bits(ov[2]) | ((uint32_t)float_to_bf16_bits(ov[3]) << 16);
+      wv.x = two_bf16_bits(ov[0], ov[1]);
+      wv.y = two_bf16_bits(ov[2], ov[3]);
       *reinterpret_cast<uint2*>(out + (size_t)b * out_row_stride + (size_t)h * VD + 4 * qd + n * 16) = wv;
     } else {
       const size_t rec = ((size_t)b * nh + h) * num_splits + split;
@@ -1047,8 +1047,8 @@ __global__ __launch_bounds__(4 * HGW * 64) void attn_prefill_kernel(
       float ov[4] = {o[c][n][0] * inv, o[c][n][1] * inv, o[c][n][2] * inv, o[c][n][3] * inv};
       if (BIAS && X.gate) attn_gate4(ov, X.gate + (size_t)(qstart + row) * X.gate_stride + ocol + n * 16);
       uint2 w;
-      w.x = (uint32_t)float_to_bf16_bits(ov[0]) | ((uint32_t)float_to_bf16_bits(ov[1]) << 16);
-      w.y = (uint32_t)float_to_bf16_bits(ov[2]) | ((uint32_t)float_to_bf16_bits(ov[3]) << 16);
+      w.x = two_bf16_bits(ov[0], ov[1]);
+      w.y = two_bf16_bits(ov[2], ov[3]);
       *reinterpret_cast<uint2*>(orow + n * 16) = w;
     }
   }

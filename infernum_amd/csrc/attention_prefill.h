@@ -422,8 +422,8 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
 #pragma unroll
     for (int n = 0; n < NSV; ++n) {
       uint2 w;
-      w.x = (uint32_t)float_to_bf16_bits(o[n][c][0] * inv) | ((uint32_t)float_to_bf16_bits(o[n][c][1] * inv) << 16);
-      w.y = (uint32_t)float_to_bf16_bits(o[n][c][2] * inv) | ((uint32_t)float_to_bf16_bits(o[n][c][3] * inv) << 16);
+      w.x = two_bf16_bits(o[n][c][0] * inv, o[n][c][1] * inv);
+      w.y = two_bf16_bits(o[n][c][2] * inv, o[n][c][3] * inv);
       *reinterpret_cast<uint2*>(orow + n * 16) = w;
     }
   }

@@ -17,12 +17,12 @@ struct bf16_t { uint16_t bits; };
 __device__ __forceinline__ float bf16_bits_to_float(uint16_t b) {
   return __uint_as_float(((uint32_t)b) << 16);
 }
-// Round to nearest, ties to even; NaN stays NaN.
-__device__ __forceinline__ uint16_t float_to_bf16_bits(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x0040u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
+// Round to nearest, ties to even; NaN stays NaN: v_cvt_pk_bf16_f32.
+__device__ __forceinline__ uint16_t float_to_bf16_bits(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
+// Two values in one instruction, the first in the lower half.
+__device__ __forceinline__ uint32_t two_bf16_bits(float a, float b) {
+  typedef __bf16 pair_t __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, (pair_t){(__bf16)a, (__bf16)b});
 }
 
 __device__ __forceinline__ float to_float(float x) { return x; }

@@ -116,8 +116,8 @@ __device__ __forceinline__ float4 load4_any(const void* p, int dtype, int i) {
 __device__ __forceinline__ void store4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
 __device__ __forceinline__ void store4(bf16_t* p, float4 v) {
   uint2 u;
-  u.x = (uint32_t)float_to_bf16_bits(v.x) | ((uint32_t)float_to_bf16_bits(v.y) << 16);
-  u.y = (uint32_t)float_to_bf16_bits(v.z) | ((uint32_t)float_to_bf16_bits(v.w) << 16);
+  u.x = two_bf16_bits(v.x, v.y);
+  u.y = two_bf16_bits(v.z, v.w);
   *reinterpret_cast<uint2*>(p) = u;
 }
 

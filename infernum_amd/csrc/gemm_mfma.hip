@@ -286,8 +286,8 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_mfma_kernel(const
           uint16_t* dstp = C + (size_t)m * NO + n;
           if (vec4 && n + 3 < NO) {
             uint2 o;
-            o.x = (uint32_t)float_to_bf16_bits(v[0]) | ((uint32_t)float_to_bf16_bits(v[1]) << 16);
-            o.y = (uint32_t)float_to_bf16_bits(v[2]) | ((uint32_t)float_to_bf16_bits(v[3]) << 16);
+            o.x = two_bf16_bits(v[0], v[1]);
+            o.y = two_bf16_bits(v[2], v[3]);
             *reinterpret_cast<uint2*>(dstp) = o;
           } else {
 #pragma unroll
@@ -313,8 +313,8 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_mfma_kernel(const
         for (int g = 0; g < 4; ++g) {
           const int n = a * 32 + 8 * g + 4 * lh;                      // 4 values from here on
           uint2 v;
-          v.x = (uint32_t)float_to_bf16_bits(acc[a][b][4 * g]) | ((uint32_t)float_to_bf16_bits(acc[a][b][4 * g + 1]) << 16);
-          v.y = (uint32_t)float_to_bf16_bits(acc[a][b][4 * g + 2]) | ((uint32_t)float_to_bf16_bits(acc[a][b][4 * g + 3]) << 16);
+          v.x = two_bf16_bits(acc[a][b][4 * g], acc[a][b][4 * g + 1]);
+          v.y = two_bf16_bits(acc[a][b][4 * g + 2], acc[a][b][4 * g + 3]);
           const int piece = (n >> 3) ^ (m & (CP - 1));
           *reinterpret_cast<uint2*>(region + (m * CP + piece) * 16 + (n & 4) * 2) = v;
         }
@@ -345,8 +345,8 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_mfma_kernel(const
         uint16_t* dstp = C + (size_t)m * N + n;
         if (vec_ok && n + 3 < N) {
           uint2 v;
-          v.x = (uint32_t)float_to_bf16_bits(acc[a][b][4 * g]) | ((uint32_t)float_to_bf16_bits(acc[a][b][4 * g + 1]) << 16);
-          v.y = (uint32_t)float_to_bf16_bits(acc[a][b][4 * g + 2]) | ((uint32_t)float_to_bf16_bits(acc[a][b][4 * g + 3]) << 16);
+          v.x = two_bf16_bits(acc[a][b][4 * g], acc[a][b][4 * g + 1]);
+          v.y = two_bf16_bits(acc[a][b][4 * g + 2], acc[a][b][4 * g + 3]);
           *reinterpret_cast<uint2*>(dstp) = v;
         } else {
 #pragma unroll

@@ -274,8 +274,8 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const uint16_t* __re
   const bool vec8 = (NO & 7) == 0;
   auto put = [&](int i, int j, const float (&v)[4]) {
     uint2 o;
-    o.x = (uint32_t)float_to_bf16_bits(v[0]) | ((uint32_t)float_to_bf16_bits(v[1]) << 16);
-    o.y = (uint32_t)float_to_bf16_bits(v[2]) | ((uint32_t)float_to_bf16_bits(v[3]) << 16);
+    o.x = two_bf16_bits(v[0], v[1]);
+    o.y = two_bf16_bits(v[2], v[3]);
     *reinterpret_cast<uint2*>(region + (j * 16 + r16) * T::OUT_ROW + (i * 16 + 4 * q4) * 2) = o;
   };
   if constexpr (GLU) {

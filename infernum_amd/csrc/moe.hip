@@ -625,8 +625,8 @@ __global__ __launch_bounds__(256) void moe_glu_kernel(const uint4* __restrict__ 
       o[k] = g * (1.0f / (1.0f + expf(-alpha * g))) * (u + shift);
     }
     uint2 r;
-    r.x = (uint32_t)float_to_bf16_bits(o[0]) | ((uint32_t)float_to_bf16_bits(o[1]) << 16);
-    r.y = (uint32_t)float_to_bf16_bits(o[2]) | ((uint32_t)float_to_bf16_bits(o[3]) << 16);
+    r.x = two_bf16_bits(o[0], o[1]);
+    r.y = two_bf16_bits(o[2], o[3]);
     y[i] = r;
   }
 }

@@ -58,8 +58,8 @@ __global__ __launch_bounds__(NB_NT) void norm_add_kernel(float* __restrict__ h, 
 __device__ __forceinline__ void nb_store4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
 __device__ __forceinline__ void nb_store4(bf16_t* p, float4 v) {
   uint2 u;
-  u.x = (uint32_t)float_to_bf16_bits(v.x) | ((uint32_t)float_to_bf16_bits(v.y) << 16);
-  u.y = (uint32_t)float_to_bf16_bits(v.z) | ((uint32_t)float_to_bf16_bits(v.w) << 16);
+  u.x = two_bf16_bits(v.x, v.y);
+  u.y = two_bf16_bits(v.z, v.w);
   *reinterpret_cast<uint2*>(p) = u;
 }
 

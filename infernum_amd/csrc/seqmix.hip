@@ -109,7 +109,7 @@ __global__ __launch_bounds__(256) void causal_conv_vec_kernel(
       a = a / (1.f + expf(-a));
       b = b / (1.f + expf(-b));
     }
-    o[e] = (uint32_t)float_to_bf16_bits(a) | ((uint32_t)float_to_bf16_bits(b) << 16);
+    o[e] = two_bf16_bits(a, b);
   }
   *(uint4*)(y + (size_t)r * y_stride + c) = make_uint4(o[0], o[1], o[2], o[3]);
 }
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(256) void causal_conv_rows_kernel(
           a = a / (1.f + expf(-a));
           b = b / (1.f + expf(-b));
         }
-        o[e] = (uint32_t)float_to_bf16_bits(a) | ((uint32_t)float_to_bf16_bits(b) << 16);
+        o[e] = two_bf16_bits(a, b);
       }
       *(uint4*)(y + (size_t)r * y_stride + c) = make_uint4(o[0], o[1], o[2], o[3]);
     }
@@ -502,7 +502,7 @@ __global__ __launch_bounds__(256) void qk_prepare_vec_kernel(
   }
   uint32_t o[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) o[e] = (uint32_t)float_to_bf16_bits(v[2 * e]) | ((uint32_t)float_to_bf16_bits(v[2 * e + 1]) << 16);
+  for (int e = 0; e < 4; ++e) o[e] = two_bf16_bits(v[2 * e], v[2 * e + 1]);
   bf16_t* dst = is_key ? k_pages + (((size_t)page * nkv + g) * page_size + off) * d + 8 * ch
                        : q_out + (size_t)t * q_stride + (size_t)hd * d + 8 * ch;
   *(uint4*)dst = make_uint4(o[0], o[1], o[2], o[3]);
@@ -637,8 +637,7 @@ __global__ __launch_bounds__(256) void qk_rows_prepare_kernel(
         uint32_t o[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          o[e] = (uint32_t)float_to_bf16_bits(__uint_as_float(u[e] << 16) * inv * wv[2 * e]) |
-                 ((uint32_t)float_to_bf16_bits(__uint_as_float(u[e] & 0xffff0000u) * inv * wv[2 * e + 1]) << 16);
+          o[e] = two_bf16_bits(__uint_as_float(u[e] << 16) * inv * wv[2 * e], __uint_as_float(u[e] & 0xffff0000u) * inv * wv[2 * e + 1]);
         const int g = part ? i / d : 0;
         T* dst = part ? k_pages + (((size_t)page * nkv + g) * page_size + off) * d + (i - g * d) : q_out + (size_t)n * q_stride + i;
         *(uint4*)dst = make_uint4(o[0], o[1], o[2], o[3]);
@@ -1228,8 +1227,8 @@ __global__ __launch_bounds__(256) void stream_add2_kernel(float* __restrict__ h,
           *reinterpret_cast<float4*>(reinterpret_cast<float*>(x) + i) = hv;
         } else {
           uint2 u;
-          u.x = (uint32_t)float_to_bf16_bits(hv.x) | ((uint32_t)float_to_bf16_bits(hv.y) << 16);
-          u.y = (uint32_t)float_to_bf16_bits(hv.z) | ((uint32_t)float_to_bf16_bits(hv.w) << 16);
+          u.x = two_bf16_bits(hv.x, hv.y);
+          u.y = two_bf16_bits(hv.z, hv.w);
           *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(x) + i) = u;
         }
       }

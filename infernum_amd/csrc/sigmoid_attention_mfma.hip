@@ -135,8 +135,8 @@ __device__ __forceinline__ float sa_gate(const uint16_t* gate, size_t at) {
 
 __device__ __forceinline__ void sa_store_bf16x4(uint16_t* at, const f32x4& x, float f) {
   uint2 u;
-  u.x = (uint32_t)float_to_bf16_bits(x[0] * f) | ((uint32_t)float_to_bf16_bits(x[1] * f) << 16);
-  u.y = (uint32_t)float_to_bf16_bits(x[2] * f) | ((uint32_t)float_to_bf16_bits(x[3] * f) << 16);
+  u.x = two_bf16_bits(x[0] * f, x[1] * f);
+  u.y = two_bf16_bits(x[2] * f, x[3] * f);
   *reinterpret_cast<uint2*>(at) = u;
 }
 

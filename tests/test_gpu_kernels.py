@@ -21,6 +21,17 @@ def _rand(*shape, dtype=torch.float32, scale=1.0, seed=0):
     return (torch.randn(*shape, generator=g) * scale).to(dtype).to(DEV)
 
 
+# every upper half with lower halves on either side of the ties: subnormal numbers, both zeros, infinities, NaN of every payload kept above
+def test_rounding_to_bf16_is_to_nearest_even_for_every_upper_half():
+    hi = torch.arange(1 << 16, dtype=torch.int64)[:, None] << 16
+    bits = (hi | torch.tensor([0, 1, 0x3fff, 0x7fff, 0x8000, 0x8001, 0xffff])).reshape(-1)
+    nan = (bits & 0x7fffffff) > 0x7f800000
+    want = torch.where(nan, bits >> 16 | 0x40, bits + 0x7fff + (bits >> 16 & 1) >> 16)
+    x = torch.where(bits >= 1 << 31, bits - (1 << 32), bits).to(torch.int32).view(torch.float32).to(DEV)
+    got = K().cast(x, torch.bfloat16).view(torch.int16).cpu().to(torch.int64) & 0xffff
+    assert torch.equal(got, want)
+
+
 # ------------------------------------------------------------------------ rows
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("H,V", [(100, 77), (4096, 1000), (1536, 333), (5120, 50), (8200, 9)])
