@@ -48,6 +48,8 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define GT_BK 64
 #define GT_ROW 128                       // bytes of a row of a step
 #define GT_LDS (160 * 1024)
+#define GT_TWO_COST 500                  // of a second launch, in units of 10 ns
+#define GT_TWO_PAYS 30                   // two launches where they are estimated to save one part in so many
 
 #if defined(__HIP_DEVICE_COMPILE__)
 typedef __attribute__((address_space(3))) void* gt_lds_ptr;
@@ -113,7 +115,7 @@ struct GemmTile {
 template <int TX0, int TX1, int TW0, int TW1, int MODE>
 __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ W,
                                                             uint16_t* __restrict__ C, int M, int N, int K, int tiles_m, int tiles_n,
-                                                            const int* __restrict__ rows_at, int groups) {
+                                                            int n_first, const int* __restrict__ rows_at, int groups) {
   using T = GemmTile<TX0, TX1, TW0, TW1, MODE>;
   constexpr bool GLU = T::GLU, GROUPED = MODE == GT_GROUPED;
   constexpr int BM = T::BM, BN = T::BN, WM = BM / 2, WN = BN / 2, STAGE = T::STAGE;
@@ -137,7 +139,7 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const uint16_t* __re
   const int group_rows = min(GROUP, tiles_m - group * GROUP);
   const int tm = group * GROUP + in_group % group_rows, tn = in_group / group_rows;
   const int m0 = GROUPED ? 0 : tm * BM;
-  const int NO = GLU ? N / 2 : N, n0 = tn * T::COLS;                          // columns of the result
+  const int NO = GLU ? N / 2 : N, n0 = n_first + tn * T::COLS;                // columns of the result
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1, r16 = lane & 15, q4 = lane >> 4;
@@ -326,8 +328,8 @@ __global__ __launch_bounds__(256, 1) void gemm_tiles_kernel(const uint16_t* __re
 }
 
 template <int TX0, int TX1, int TW0, int TW1, int MODE>
-static int launch_gemm_tiles(const uint16_t* x, const uint16_t* w, uint16_t* c, int M, int N, int K, const int* rows_at,
-                             int groups, hipStream_t stream) {
+static int launch_gemm_tiles(const uint16_t* x, const uint16_t* w, uint16_t* c, int M, int N, int K, int n_first, int n_end,
+                             const int* rows_at, int groups, hipStream_t stream) {
   using T = GemmTile<TX0, TX1, TW0, TW1, MODE>;
   static bool configured = false;
   if (!configured) {
@@ -338,9 +340,9 @@ static int launch_gemm_tiles(const uint16_t* x, const uint16_t* w, uint16_t* c, 
   }
   // grouped: a tile for every way the rows can fall into groups
   const int tiles_m = MODE == GT_GROUPED ? M / T::BM + (M < groups ? M : groups) : (M + T::BM - 1) / T::BM;
-  const int tiles_n = ((T::GLU ? N / 2 : N) + T::COLS - 1) / T::COLS;
+  const int tiles_n = (n_end - n_first + T::COLS - 1) / T::COLS;
   if ((long long)tiles_m * tiles_n > 0x7fffffffLL) return IA_ERR_UNSUPPORTED;
-  gemm_tiles_kernel<TX0, TX1, TW0, TW1, MODE><<<tiles_m * tiles_n, 256, T::LDS, stream>>>(x, w, c, M, N, K, tiles_m, tiles_n, rows_at, groups);
+  gemm_tiles_kernel<TX0, TX1, TW0, TW1, MODE><<<tiles_m * tiles_n, 256, T::LDS, stream>>>(x, w, c, M, N, K, tiles_m, tiles_n, n_first, rows_at, groups);
   IA_LAUNCH_CHECK();
   return IA_OK;
 }
@@ -372,15 +374,46 @@ static long tile_cost(int M, int NO, int K, int bm, int bn, int cols) {
   return tiles / 512 * pair + (rest > 256 ? pair : rest > 0 ? around + one : 0);
 }
 
-static void choose_tile(int M, int N, int K, bool glu, int& rows, int& cols) {
-  long best = -1;
+// A product's tiles; with two, the first `split` columns of the result in one and the others in the other.
+struct TileChoice {
+  int rows, cols, split, rows2, cols2;
+};
+
+// Large tiles fill turns of the compute units and leave a part of one.  Where that is estimated to cost more than a second launch does
+// and one part in GT_TWO_PAYS of the product, the columns of the whole turns take them, and the others, in a launch of their own, smaller
+// tiles.  One tile / two, us, M x rows of W x K, with the activation: 2,048 x 28,672 x 4,096 (3.5 turns of 256 x 256) 371 / 340, 7,680 rows
+// (13.1 turns) 1,258 / 1,223, 1,000 rows (1.8) 180 / 169, 2,925 x 11,008 x 2,048 114 / 108; plain: 4,054 x 25,664 x 4,096 627 / 593.  Of 432 products
+// of 160 to 8,192 rows it takes 13 in 100, 4.9 % faster on average.  The second launch counts 5 us although it takes some 3: below 80 us the
+// estimate is as often wrong (1,755 x 10,304 x 2,048 61 / 66, 1,776 x 11,008 x 2,048 71 / 67).
+static TileChoice choose_tiles(int M, int N, int K, bool glu) {
+  const int NO = glu ? N / 2 : N;
+  const auto best = [&](int columns, int& rows, int& cols) {
+    long least = -1;
 #define GT_COST(BM, BN, TX0, TX1, TW0, TW1)                                                                  \
-  if (!glu || TW0 == TW1) {                                                                                  \
-    const long cost = tile_cost(M, glu ? N / 2 : N, K, BM, BN, glu ? BN / 2 : BN);                           \
-    if (best < 0 || cost < best) { best = cost; rows = BM; cols = BN; }                                      \
+    if (!glu || TW0 == TW1) {                                                                                \
+      const long cost = tile_cost(M, columns, K, BM, BN, glu ? BN / 2 : BN);                                 \
+      if (least < 0 || cost < least) { least = cost; rows = BM; cols = BN; }                                 \
+    }
+    GT_TILES(GT_COST)
+#undef GT_COST
+    return least;
+  };
+  TileChoice one{0, 0, 0, 0, 0};
+  const long alone = best(NO, one.rows, one.cols);
+  long least = alone - alone / GT_TWO_PAYS;
+#define GT_COST(BM, BN, TX0, TX1, TW0, TW1)                                                                  \
+  if ((!glu || TW0 == TW1) && BM * BN >= 192 * 256) {                                                        \
+    const int wide = glu ? BN / 2 : BN, down = (M + BM - 1) / BM;                                            \
+    const int split = (int)((long)down * (NO / wide) / 256 * 256 / down) * wide;                             \
+    if (split > 0 && split < NO) {                                                                           \
+      TileChoice two{BM, BN, split, 0, 0};                                                                   \
+      const long cost = tile_cost(M, split, K, BM, BN, wide) + GT_TWO_COST + best(NO - split, two.rows2, two.cols2); \
+      if (cost < least) { least = cost; one = two; }                                                         \
+    }                                                                                                        \
   }
   GT_TILES(GT_COST)
 #undef GT_COST
+  return one;
 }
 
 // Whether this kernel or the vendor library's takes a whole product of many rows (with the activation there is a rule of its own where the
@@ -403,6 +436,19 @@ extern "C" int ia_gemm_tiles_pays(int M, int N, int K) {
   return places * 100 >= large * (K >= 10240 && large > 256 ? 106 : 120);
 }
 
+// Columns n_first to n_end - 1 of the result.
+static int gemm_tiles_columns(const uint16_t* x, const uint16_t* w, uint16_t* c, int M, int N, int K, int glu, int rows, int cols,
+                              int n_first, int n_end, hipStream_t stream) {
+#define GT_ONE(BM, BN, TX0, TX1, TW0, TW1)                                                                                            \
+  if (rows == BM && cols == BN) {                                                                                                     \
+    if (!glu) return launch_gemm_tiles<TX0, TX1, TW0, TW1, GT_PLAIN>(x, w, c, M, N, K, n_first, n_end, nullptr, 0, stream);            \
+    if constexpr (TW0 == TW1) return launch_gemm_tiles<TX0, TX1, TW0, TW1, GT_GLU>(x, w, c, M, N, K, n_first, n_end, nullptr, 0, stream); \
+  }
+  GT_TILES(GT_ONE)
+#undef GT_ONE
+  return IA_ERR_BAD_ARG;
+}
+
 // X [M, K], W [N, K], C [M, N] (glu: [M, N / 2], N even), bf16, contiguous, on 16 bytes.  rows, cols: the tile; 0: chosen here; rows < 0:
 // the same, where ia_gemm_tiles_pays (else IA_ERR_UNSUPPORTED).
 extern "C" int ia_gemm_tiles(const void* X, const void* W, void* C, int M, int N, int K, int glu, int rows, int cols, hipStream_t stream) {
@@ -412,15 +458,11 @@ extern "C" int ia_gemm_tiles(const void* X, const void* W, void* C, int M, int N
   if (rows < 0 && !glu && !ia_gemm_tiles_pays(M, N, K)) return IA_ERR_UNSUPPORTED;
   const uint16_t *x = (const uint16_t*)X, *w = (const uint16_t*)W;
   uint16_t* c = (uint16_t*)C;
-  if (rows <= 0) choose_tile(M, N, K, glu != 0, rows, cols);
-#define GT_ONE(BM, BN, TX0, TX1, TW0, TW1)                                                                        \
-  if (rows == BM && cols == BN) {                                                                                 \
-    if (!glu) return launch_gemm_tiles<TX0, TX1, TW0, TW1, GT_PLAIN>(x, w, c, M, N, K, nullptr, 0, stream);                      \
-    if constexpr (TW0 == TW1) return launch_gemm_tiles<TX0, TX1, TW0, TW1, GT_GLU>(x, w, c, M, N, K, nullptr, 0, stream);       \
-  }
-  GT_TILES(GT_ONE)
-#undef GT_ONE
-  return IA_ERR_BAD_ARG;
+  const int NO = glu ? N / 2 : N;
+  if (rows > 0) return gemm_tiles_columns(x, w, c, M, N, K, glu, rows, cols, 0, NO, stream);
+  const TileChoice t = choose_tiles(M, N, K, glu != 0);
+  const int rc = gemm_tiles_columns(x, w, c, M, N, K, glu, t.rows, t.cols, 0, t.split > 0 ? t.split : NO, stream);
+  return rc == IA_OK && t.split > 0 ? gemm_tiles_columns(x, w, c, M, N, K, glu, t.rows2, t.cols2, t.split, NO, stream) : rc;
 }
 
 // ---- rows in groups, each with a matrix of its own: the routed experts' products of many tokens ----
@@ -508,7 +550,7 @@ extern "C" int ia_gemm_tiles_grouped(const void* X, const void* W, void* C, cons
   uint16_t* c = (uint16_t*)C;
   const int tile = ia_gemm_tiles_grouped_tile(groups, rows / among, N, K);
 #define GT_GROUP_ONE(BM, BN, TX0, TX1, TW0, TW1) \
-  if (tile == BM * 1024 + BN) return launch_gemm_tiles<TX0, TX1, TW0, TW1, GT_GROUPED>(x, w, c, rows, N, K, rows_at, groups, stream);
+  if (tile == BM * 1024 + BN) return launch_gemm_tiles<TX0, TX1, TW0, TW1, GT_GROUPED>(x, w, c, rows, N, K, 0, N, rows_at, groups, stream);
   GT_GROUP_TILES(GT_GROUP_ONE)
 #undef GT_GROUP_ONE
   return IA_ERR_BAD_ARG;

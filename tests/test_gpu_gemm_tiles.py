@@ -99,6 +99,18 @@ def test_what_it_refuses():
         api.gemm_tiles(a, off)                                                          # off 16 bytes
 
 
+# columns in two launches of a tile each, the last of either in part: the same bits as one tile for all, and nothing stored twice or beyond
+@pytest.mark.parametrize("M,N,K_,swiglu", [(1125, 16392, 1024, False), (1146, 17122, 2048, True), (1121, 17634, 2048, True), (1009, 16762, 3072, False)])
+def test_columns_in_two_launches_leave_the_bits_of_one(M, N, K_, swiglu):
+    api = K()
+    a, w = _rand(M, K_, seed=21), _rand(N, K_, scale=0.1, seed=22)
+    cols = N // 2 if swiglu else N
+    out = torch.full((M + 1, cols), 7.0, dtype=torch.bfloat16, device=DEV)
+    api.gemm_tiles(a, w, out[:M], swiglu=swiglu)
+    assert torch.equal(out[:M], api.gemm_tiles(a, w, swiglu=swiglu, tile=(128, 128)))
+    assert bool((out[M:] == 7.0).all())
+
+
 @pytest.mark.parametrize("off", [False, True])
 @pytest.mark.parametrize("M,N,K_", [(300, 512, 256), (2304, 2048, 2048), (2304, 2304, 4096)])
 def test_many_rows_take_it_where_it_is_the_faster(M, N, K_, off):
