@@ -1212,6 +1212,26 @@ def test_attention_generic_by_how_rows_can_be_read(d, dv):
         assert float((outs[0][n].view(nh, dv).double() - want).abs().max()) <= (4 * d + 65) * 2.0 ** -24 * 8
 
 
+# values read four keys at a time (pages of a multiple of four keys that lie on 16 bytes, a window that begins on such a key, no kept
+# keys) and key by key: the same bits, with whatever lies behind the last key
+@pytest.mark.parametrize("dv,window", [(64, 0), (65, 0), (128, 0), (256, 0), (300, 0), (64, 8), (64, 7), (64, -20)])
+def test_attention_generic_by_how_values_can_be_read(dv, window):
+    nh, nkv, d, ps, lens, new = 4, 2, 32, 4, [65, 64, 5, 130, 66], [3, 2, 5, 1, 66]
+    case = _paged_case(nh, nkv, max(d, dv), ps, lens, new, torch.float32)
+    q = case["q"].view(case["N"], nh, -1)[:, :, :d].reshape(case["N"], nh * d).contiguous()
+    kp, vp = case["kp"][:, :, :, :d].contiguous(), case["vp"][:, :, :dv].contiguous()
+    for b, L in enumerate(lens):                       # places behind the last key hold anything
+        if L % ps:
+            vp[int(case["bt"][b, L // ps]), :, :, L % ps:] = float("nan")
+    room = torch.empty(vp.numel() + 1, device=DEV)
+    room[1:] = vp.flatten()
+    outs = []
+    for pages in (vp, room[1:].view(vp.shape)):
+        outs.append(torch.full((case["N"], nh * dv), float("nan"), device=DEV))
+        K().attention_generic(q, kp, pages, outs[-1], case["token_seq"], case["positions"], case["bt"], nh, nkv, d, d ** -0.5, window)
+    assert torch.equal(outs[0], outs[1]) and not bool(outs[0].isnan().any())
+
+
 def test_attention_generic_missing_page_poisons():
     nh, nkv, d, ps = 1, 1, 16, 4
     case = _paged_case(nh, nkv, d, ps, [20], [1], torch.float32)
