@@ -39,6 +39,7 @@
 #define DR_TB 8          // tokens whose vectors are staged together
 #define DR_WAVES 2       // waves of a workgroup: 8 columns
 #define DR_COLS (4 * DR_WAVES)
+#define DT_COLUMNS 8192  // of all states, for every column that a lane of the single tokens' kernel takes
 
 // Sum over the sixteen lanes of a row of lanes, the same bits in every lane (each step adds two numbers that the
 // other lane of the pair adds too).
@@ -343,14 +344,122 @@ __global__ __launch_bounds__(64 * DR_WAVES) void delta_scan_kernel(
   }
 }
 
+// Single tokens: every request's one row.  The same operations on every column and so the same bits; what bounds it is the state, read and
+// written once, and one trip to it: nothing is staged, a lane asks for its channels of the vectors and of CW columns of the state together
+// (16 requests of 32 heads of 128, 67 MB read and written: 14.3 us in a decoded step, with vectors of eight tokens staged in LDS by workgroups
+// of eight columns 26.0).  CW grows with the states there are, so that a compute unit has eight waves.
+template <typename T, int J, int CW>
+__global__ __launch_bounds__(256) void delta_token_kernel(const T* __restrict__ proj, int proj_stride, int r_col, int k_col, int v_col,
+                                                          const float* __restrict__ w, const float* __restrict__ a,
+                                                          const float* __restrict__ inv, float* __restrict__ state, long state_stride,
+                                                          float* __restrict__ out, const int* __restrict__ state_slots, int nh, int dim) {
+  const int hd = blockIdx.x, s = blockIdx.y, lane = threadIdx.x & 63, q = lane & 15;
+  const int c0 = (blockIdx.z * 4 + (threadIdx.x >> 6)) * (4 * CW) + (lane >> 4);          // this lane's first column
+  if (c0 - (lane >> 4) >= dim) return;
+  const size_t at = ((size_t)s * nh + hd) * dim;
+  const T* row = proj + (size_t)s * proj_stride + (size_t)hd * dim;
+  float* st = state + (size_t)state_slots[s] * state_stride + (size_t)hd * dim * dim;
+  typedef typename DrRaw<T, 4>::type raw_t;
+  float4 S4[CW][J], w4[J], a4[J];
+  raw_t k4[J], r4[J];
+  T v1[CW];
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int n = 64 * j + 4 * q, nc = n < dim ? n : 0;
+    w4[j] = *reinterpret_cast<const float4*>(w + at + nc);
+    a4[j] = *reinterpret_cast<const float4*>(a + at + nc);
+    k4[j] = *reinterpret_cast<const raw_t*>(row + k_col + nc);
+    r4[j] = *reinterpret_cast<const raw_t*>(row + r_col + nc);
+  }
+  const float scale = inv[(size_t)s * nh + hd];
+#pragma unroll
+  for (int c = 0; c < CW; ++c) {
+    const int col = min(c0 + 4 * c, dim - 1);
+    v1[c] = row[v_col + col];
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const int n = 64 * j + 4 * q;
+      S4[c][j] = *reinterpret_cast<const float4*>(st + (size_t)col * dim + (n < dim ? n : 0));
+    }
+  }
+  float u[J][4], vw[J][4], au[J][4], vk[J][4], vr[J][4];
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    float va[4];
+    dr_values(w4[j], vw[j]);
+    dr_values(a4[j], va);
+    dr_values(k4[j], vk[j]);
+    dr_values(r4[j], vr[j]);
+    const bool real = 64 * j + 4 * q < dim;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      u[j][e] = real ? vk[j][e] * scale : 0.f;
+      au[j][e] = real ? va[e] * u[j][e] : 0.f;
+      vw[j][e] = real ? vw[j][e] : 0.f;
+      vk[j][e] = real ? vk[j][e] : 0.f;
+      vr[j][e] = real ? vr[j][e] : 0.f;
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < CW; ++c) {
+    float S[J][4], d[J], o[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      dr_values(S4[c][j], S[j]);
+      if (64 * j + 4 * q >= dim) S[j][0] = S[j][1] = S[j][2] = S[j][3] = 0.f;
+      d[j] = u[j][0] * S[j][0];
+#pragma unroll
+      for (int e = 1; e < 4; ++e) d[j] = __builtin_fmaf(u[j][e], S[j][e], d[j]);
+    }
+#pragma unroll
+    for (int j = 1; j < J; ++j) d[0] += d[j];
+    const float dot = dr_sum16(d[0]), v = to_float(v1[c]);
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      o[j] = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float add = __builtin_fmaf(vk[j][e], v, -(au[j][e] * dot));
+        S[j][e] = __builtin_fmaf(vw[j][e], S[j][e], add);
+        o[j] = __builtin_fmaf(vr[j][e], S[j][e], o[j]);
+      }
+    }
+#pragma unroll
+    for (int j = 1; j < J; ++j) o[0] += o[j];
+    const float y = dr_sum16(o[0]);
+    const int col = c0 + 4 * c;
+    if (col >= dim) continue;
+    if (q == 0) out[at + col] = y;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const int n = 64 * j + 4 * q;
+      if (n < dim) *reinterpret_cast<float4*>(st + (size_t)col * dim + n) = make_float4(S[j][0], S[j][1], S[j][2], S[j][3]);
+    }
+  }
+}
+
+template <typename T, int J>
+static void launch_delta_token(const T* proj, int proj_stride, int r_col, int k_col, int v_col, const float* w, const float* a,
+                               const float* inv, float* state, long state_stride, float* out, const int* state_slots, int B, int nh,
+                               int dim, hipStream_t stream) {
+#define IA_DT(CW)                                                                                                                   \
+  delta_token_kernel<T, J, CW><<<dim3((unsigned)nh, (unsigned)B, (unsigned)((dim + 16 * CW - 1) / (16 * CW))), 256, 0, stream>>>(   \
+      proj, proj_stride, r_col, k_col, v_col, w, a, inv, state, state_stride, out, state_slots, nh, dim)
+  const long columns = (long)B * nh * dim;
+  if (J <= 2 && columns >= DT_COLUMNS * 4) IA_DT(4);
+  else if (columns >= DT_COLUMNS * 2) IA_DT(2);
+  else IA_DT(1);
+#undef IA_DT
+}
+
 // Floats a request's slot holds for one layer run.
 extern "C" long ia_delta_state_floats(int nh, int dim) { return (long)nh * dim * dim; }
 
 // proj: rows of proj_stride values (code: their type) holding r, k and v (nh dim values each from their columns); w, a
-// fp32 [N, nh, dim] and inv fp32 [N, nh] as ia_delta_prepare leaves them; out fp32 [N, nh, dim].
+// fp32 [N, nh, dim] and inv fp32 [N, nh] as ia_delta_prepare leaves them; out fp32 [N, nh, dim].  single: request s has one row, row s.
 extern "C" int ia_delta_scan(const void* proj, int code, int proj_stride, int r_col, int k_col, int v_col, const float* w,
                              const float* a, const float* inv, float* state, long state_stride, float* out,
-                             const int* seq_starts, const int* state_slots, int B, int nh, int dim, hipStream_t stream) {
+                             const int* seq_starts, const int* state_slots, int B, int nh, int dim, int single, hipStream_t stream) {
   if (B == 0) return IA_OK;
   if (!proj || !w || !a || !inv || !state || !out || !seq_starts || !state_slots || B < 0 || nh <= 0 || dim <= 0 ||
       r_col < 0 || k_col < 0 || v_col < 0 || proj_stride < r_col + nh * dim || proj_stride < k_col + nh * dim ||
@@ -363,6 +472,23 @@ extern "C" int ia_delta_scan(const void* proj, int code, int proj_stride, int r_
   const size_t el = code == IA_F32 ? 4 : 2;
   const bool fours = ((dim | proj_stride | r_col | k_col) & 3) == 0 && ((uintptr_t)proj % (4 * el)) == 0 && (state_stride & 3) == 0 &&
                      (((uintptr_t)w | (uintptr_t)a | (uintptr_t)state) & 15) == 0;
+  // the channels as the kernel of several tokens deals them out: where it has them in fours
+  if (single && fours && (dim > 96 || (dim > 32 && dim <= 64))) {
+#define IA_DT(T, JJ) launch_delta_token<T, JJ>((const T*)proj, proj_stride, r_col, k_col, v_col, w, a, inv, state, state_stride, out, state_slots, B, nh, dim, stream)
+#define IA_DT_D(T)                    \
+  do {                                \
+    if (dim <= 64) IA_DT(T, 1);       \
+    else if (dim <= 128) IA_DT(T, 2); \
+    else if (dim <= 192) IA_DT(T, 3); \
+    else IA_DT(T, 4);                 \
+  } while (0)
+    if (code == IA_F32) IA_DT_D(float);
+    else IA_DT_D(bf16_t);
+#undef IA_DT_D
+#undef IA_DT
+    IA_LAUNCH_CHECK();
+    return IA_OK;
+  }
 #define IA_DR(T, V, JJ)                                                                                                    \
   do {                                                                                                                     \
     if (fours)                                                                                                             \

@@ -1918,11 +1918,12 @@ def delta_prepare(proj: torch.Tensor, k_col: int, a_col: int, z: torch.Tensor, w
 
 def delta_scan(proj: torch.Tensor, r_col: int, k_col: int, v_col: int, w: torch.Tensor, a: torch.Tensor, inv: torch.Tensor,
                state: torch.Tensor, out: torch.Tensor, seq_starts: torch.Tensor, state_slots: torch.Tensor, nh: int,
-               dim: int) -> torch.Tensor:
+               dim: int, single: bool = False) -> torch.Tensor:
     """S_t = diag(w_t) S - (a_t * u_t)(u_t^T S) + k_t v_t^T, o_t = S_t^T r_t with u = k inv, over the rows of every
     request of the step: r, k, v from columns of ``proj``, w and a fp32 [N, nh dim], inv fp32 [N, nh], ``state``
-    [slots, >= nh dim dim] fp32 (moved on in place), ``out`` fp32 [N, nh dim]."""
+    [slots, >= nh dim dim] fp32 (moved on in place), ``out`` fp32 [N, nh dim].  ``single``: request s has one row, row s."""
     N, n, B = proj.shape[0], nh * dim, state_slots.numel()
+    _need(not single or N >= B, "delta_scan: a row for every request")
     _rows(proj, max(r_col, k_col, v_col) + n, "delta_scan")
     for t, size, what in ((w, N * n, "w"), (a, N * n, "a"), (inv, N * nh, "inv"), (out, out.shape[0] * n, "out")):
         _f32(t, size, f"delta_scan {what}")
@@ -1931,7 +1932,7 @@ def delta_scan(proj: torch.Tensor, r_col: int, k_col: int, v_col: int, w: torch.
     _i32(state_slots, B, "delta_scan state_slots")
     _ok(_core().ia_delta_scan(_p(proj), DTYPE_CODE[proj.dtype], _rows_of(proj), r_col, k_col, v_col, _p(w), _p(a), _p(inv),
                               _p(state), ctypes.c_long(stride), _p(out), _p(seq_starts), _p(state_slots), B, nh, dim,
-                              _stream()), "delta_scan")
+                              int(single), _stream()), "delta_scan")
     return out
 
 

@@ -100,7 +100,7 @@ class DeltaRule(ProjectedMixer):
         nd = ctx.num_decode
         if nd > 0:              # single tokens: the recurrence itself
             K.delta_scan(proj, self.r_col, self.k_col, self.v_col, z, a, inv, state, o, ctx.seq_starts[:nd + 1],
-                         ctx.state_slots[:nd], self.nh, self.dim)
+                         ctx.state_slots[:nd], self.nh, self.dim, single=True)
         if ctx.num_seqs > nd:   # portions of prompts: chunks of rows as matrix products
             tiles, num_tiles = ctx.row_tiles(K.PREFILL_TILE_ROWS)
             K.delta_chunked(proj, self.r_col, self.k_col, self.v_col, z, a, inv, state, o, ctx.seq_starts, ctx.state_slots,
@@ -124,7 +124,7 @@ class DeltaRule(ProjectedMixer):
         o = program.buffer("delta.o", T * self.n * 4)
         program.op("core", "ia_delta_scan", [proj, act, proj_row, self.r_col, self.k_col, self.v_col, z, a, inv, state,
                                              int(state.stride(0)), o, program.seq_starts, program.state_slots, program.ND, nh,
-                                             dim, STREAM], Guard.between(program.ND, 1))
+                                             dim, 1, STREAM], Guard.between(program.ND, 1))
         # a request holds a state slot, and a tile at least one row: so many tiles a step has at most
         most = -(-T // K.PREFILL_TILE_ROWS) + int(state.shape[0])
         records = program.buffer("delta.records", most * 4 * K.delta_chunk_floats(nh, dim) * 4)

@@ -415,6 +415,29 @@ def test_delta_rule_at_many_head_sizes(dtype, dim, heads, T):
     assert rel_err(st3, torch.where(torch.arange(7)[:, None] == slots[0], state, st.cpu()).double()) <= 2e-5
 
 
+# one, two and four columns a lane, heads that fill their channels in fours and not, columns that fill no wave; a head size and a place of
+# the columns that the kernel of several tokens keeps
+@BOTH
+@pytest.mark.parametrize("dim,heads,requests,off", [(128, 8, 1, 0), (36, 2, 3, 0), (64, 16, 9, 0), (128, 8, 17, 0), (100, 5, 70, 0), (132, 4, 33, 0),
+                                                    (256, 2, 2, 0), (200, 8, 21, 0), (96, 4, 5, 0), (128, 4, 6, 1)])
+def test_single_tokens_leave_the_bits_of_the_recurrence(dtype, dim, heads, requests, off):
+    from infernum_amd.kernels import api as K
+    n = heads * dim
+    g = torch.Generator().manual_seed(dim + requests)
+    proj = (torch.randn(requests, 3 * n + 4, generator=g) / math.sqrt(dim)).to(runtime(dtype).dtype).to(DEV)
+    w, a = (0.6 + 0.4 * torch.rand(requests, n, generator=g)).to(DEV), torch.rand(requests, n, generator=g).to(DEV)
+    inv = torch.rand(requests, heads, generator=g).to(DEV)
+    slots = torch.randperm(requests + 2, generator=g)[:requests].to(torch.int32).to(DEV)
+    state = torch.randn(requests + 2, K.delta_state_floats(heads, dim), generator=g).to(DEV)
+    starts = torch.arange(requests + 1, dtype=torch.int32, device=DEV)
+    left = []
+    for single in (False, True):
+        st, out = state.clone(), torch.full((requests, n), 7.0, device=DEV)
+        K.delta_scan(proj, off, off + n, off + 2 * n, w, a, inv, st, out, starts, slots, heads, dim, single=single)
+        left.append((st, out))
+    assert torch.equal(left[0][0], left[1][0]) and torch.equal(left[0][1], left[1][1])
+
+
 @BOTH
 def test_a_state_that_reaches_hundreds_of_tokens_back(dtype):
     """A head that hardly decays and takes nothing out carries what token 3 wrote over 600 tokens, whole and decoded."""
