@@ -427,6 +427,145 @@ static bool whole_k_pays(int M, int N, int K, int splits, bool glu) {
   return (long)M * K <= (full < 70 ? 8192 : full < 99 ? 16384 : groups < 768 ? 32768 : 65536);
 }
 
+// ---- up to 32 rows, the parts of K in one workgroup behind X in LDS ---------------------------------------------------
+// The same sums in the same order again.  A workgroup takes `groups` times 16 rows of W (GLU: of each half) with a wave for each 16 and
+// part of K, so that the matrix's rows fill one turn of the compute units; all of X goes to LDS once, straight from memory, while every
+// wave's first two chunks of W are under way, and a chunk's registers are asked for again as soon as they are free.  What bounds it: the
+// stream of W behind the launch and the first trip to memory (9,216 x 2,048, 6.2 us at the rate of a large read, at 8 / 16 / 32 rows 12.6 / 13.0 /
+// 15.0 us with the kernels above and the join, 10.8 / 11.2 / 13.4 so; 12,288 x 4,096 at 16 rows, 16.6, 25.5 and 21.8; 5,376 x 2,048 with the
+// activation at 32 rows, 3.6, 11.2 and 10.1).
+typedef __attribute__((address_space(3))) void* sk_lds_ptr;
+typedef const __attribute__((address_space(1))) void* sk_global_ptr;
+#define SK_STAGED_LDS (160 * 1024)
+#define SK_STAGED_WAVES 16
+
+template <bool GLU, int MT, typename TO>
+__global__ __launch_bounds__(SK_STAGED_WAVES * 64) void gemm_skinny_staged_kernel(const uint16_t* __restrict__ X,
+                                                                                  const uint16_t* __restrict__ W,
+                                                                                  TO* __restrict__ C, int M, int N, int K,
+                                                                                  int chunks_per_split, int splits, int groups,
+                                                                                  SkFinish finish) {
+  constexpr int NLD = SK_KC / 32;
+  extern __shared__ __attribute__((aligned(16))) char staged_lds[];
+  const int tid = threadIdx.x, lane = tid & 63, waves = blockDim.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  // strips of 16 rows of W: the groups of the first half, then those of the second
+  const int split = wave % splits, strip = wave / splits, half = GLU && strip >= groups ? 1 : 0, group = strip - half * groups;
+  const int NO = GLU ? N / 2 : N;
+  const int n0 = (blockIdx.x * groups + group) * 16;
+  const int nchunks = K / SK_KC;
+  const int c0 = split * chunks_per_split, c1 = min(nchunks, c0 + chunks_per_split), span = c1 - c0;
+  const uint16_t* wrow = W + ((size_t)min(n0 + r, NO - 1) + (size_t)half * NO) * K + q * 8;
+  const unsigned tile = (unsigned)(min(n0, NO - 1) + half * NO) / SK_BN;           // the tile of 64 rows that names the first chunk
+  const int rot = span > 1 ? (int)(((tile * 0x9E3779B1u) >> 8) % (unsigned)span) : 0;
+  const auto chunk = [&](int c) {
+    const int k = c0 + rot + min(c, span - 1);
+    return k >= c1 ? k - span : k;
+  };
+  uint4 w0[NLD], w1[NLD];
+  const auto load_w = [&](int c, uint4 (&dst)[NLD]) {
+    const uint16_t* src = wrow + chunk(c) * SK_KC;
+#pragma unroll
+    for (int j = 0; j < NLD; ++j) dst[j] = load_stream_16(src + 32 * j);
+  };
+  load_w(0, w0);
+  load_w(1, w1);
+  __builtin_amdgcn_sched_barrier(0);                   // in front of X, whose wait is for all of them
+  // rows of X with 16 bytes of padding between them, 1,024 bytes a load of a wave
+  const int stride = K * 2 + 16, pieces = K / 512;
+  for (int p = wave; p < MT * 16 * pieces; p += waves) {
+    const int row = p / pieces, at = p - row * pieces;
+    __builtin_amdgcn_global_load_lds((sk_global_ptr)(X + (size_t)min(row, M - 1) * K + at * 512 + lane * 8),
+                                     (sk_lds_ptr)(staged_lds + row * stride + at * 1024), 16, 0, 0);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  f32x4 acc[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) acc[mt] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  const auto products = [&](int c, const uint4 (&w)[NLD]) {
+    const char* x = staged_lds + r * stride + (chunk(c) * SK_KC + q * 8) * 2;
+#pragma unroll
+    for (int j = 0; j < NLD; ++j)
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const uint4 xv = *reinterpret_cast<const uint4*>(x + mt * 16 * stride + j * 64);
+        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[j]), __builtin_bit_cast(bf16x8, xv), acc[mt], 0, 0, 0);
+      }
+  };
+  for (int c = 0; c < span; c += 2) {
+    products(c, w0);
+    if (c + 2 < span) load_w(c + 2, w0);
+    if (c + 1 < span) products(c + 1, w1);
+    if (c + 3 < span) load_w(c + 3, w1);
+  }
+  __syncthreads();                                     // the parts meet in the memory of X
+  f32x4(*parts)[64] = reinterpret_cast<f32x4(*)[64]>(staged_lds);                  // [wave MT + tile of rows of X]
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) parts[wave * MT + mt][lane] = acc[mt];
+  __syncthreads();
+  for (int t = wave; t < groups * MT; t += waves) {    // a wave adds the parts of a tile of 16 x 16, in the order of their index
+    const int g = t / MT, mt = t - g * MT, m = mt * 16 + r, n = (blockIdx.x * groups + g) * 16 + 4 * q;
+    f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = {0.f, 0.f, 0.f, 0.f};
+    for (int v = 0; v < splits; ++v) {
+      a += parts[(g * splits + v) * MT + mt][lane];
+      if (GLU) b += parts[((groups + g) * splits + v) * MT + mt][lane];
+    }
+    if (m >= M) continue;
+    TO* o = C + (size_t)m * NO + n;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (n + e >= NO) continue;
+      if (GLU) store_out<TO>(o + e, a[e] / (1.0f + expf(-a[e])) * b[e]);
+      else store_finished(o + e, a[e], n + e, finish);
+    }
+  }
+}
+
+static size_t staged_lds_bytes(int M, int K) { return (size_t)((M + 15) / 16) * 16 * (K * 2 + 16); }
+
+// How many groups of 16 rows of W a workgroup of the kernel above takes of a split product whose parts are wanted joined, or 0: not that
+// kernel.  As many as fill one turn of the compute units.  Measured with cold weights over N of 2,816 to 15,360 and K of 512 to 4,096 at 1 to 32
+// rows, its time over that of the kernels above with their join: it gains where a wave has two chunks and more, so that they are under way
+// together, and
+// - three groups a workgroup (8,193 to 12,288 rows of W), or four of K up to 2,560: 0.82 to 0.99 from four rows on (9,216 x 2,048 at 1 / 4 / 8 /
+//   16 / 32 rows 0.95 / 0.90 / 0.85 / 0.87 / 0.89, 12,288 x 4,096 at 4 / 16 0.97 / 0.85; 15,360 x 4,096 at 4 / 16 1.00 / 0.96);
+// - two groups with K up to 2,560: from eight rows on (6,144 x 2,048 at 4 / 8 / 32 0.95 / 0.90 / 0.87, 8,192 x 2,048 at 8 / 12 1.01 / 0.96), while
+//   5,120 x 4,096 in six parts takes 1.13 to 1.15 and 8,192 x 3,072 0.98 to 1.09;
+// - one group with K from 2,560 on: from twelve rows on (4,096 x 2,560 / 3,072 / 4,096 at 8 1.08 / 1.05 / 0.97, at 16 0.77 / 0.87 / 0.96);
+// - with the activation one group and up to five parts, K from 1,536 on: from eight rows on (5,376 x 2,048 at 1 / 4 / 8 / 32 0.99 / 0.92 / 0.88 /
+//   0.89, 8,192 x 2,560 0.85 at 8; in six parts 5,376 x 3,072 1.06; two groups 9,472 x 2,048 1.00, x 4,096 1.05).
+// A single chunk a wave leaves it 1.0 to 1.4 (4,096 x 2,048 in eight parts 1.31 at 8 rows).
+static int staged_groups(int M, int N, int K, int splits, bool glu) {
+  if (M > 32 || K % 512 != 0 || staged_lds_bytes(M, K) > SK_STAGED_LDS) return 0;
+  const int chunks = (K / SK_KC + splits - 1) / splits, tiles = ((glu ? N / 2 : N) + 15) / 16, groups = (tiles + 255) / 256;
+  if (chunks < 2 || (glu ? 2 : 1) * groups * splits > SK_STAGED_WAVES) return 0;
+  // (a strip of the second half lies in one tile of 64 rows, whose walk over K has one start, where N is a multiple of 32)
+  if (glu) return N % 32 == 0 && groups == 1 && splits <= 5 && tiles > 128 && K >= 1536 && M >= 8 ? 1 : 0;
+  if (groups == 3 || (groups == 4 && K <= 2560)) return M >= 4 ? groups : 0;
+  if (groups == 2) return K <= 2560 && M >= (N <= 7680 ? 8 : 12) ? 2 : 0;
+  return groups == 1 && tiles > 128 && K >= 2560 && M >= 12 ? 1 : 0;
+}
+
+template <bool GLU, int MT, typename TO>
+static int launch_staged(const uint16_t* x, const uint16_t* w, TO* c, int M, int N, int K, int splits, int groups,
+                         const SkFinish& finish, hipStream_t stream) {
+  static bool allowed = false;      // more than 64 KB of LDS has to be asked for, once per kernel
+  if (!allowed) {
+    const hipError_t e = hipFuncSetAttribute((const void*)gemm_skinny_staged_kernel<GLU, MT, TO>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, SK_STAGED_LDS);
+    if (e != hipSuccess) return (int)e;
+    allowed = true;
+  }
+  const int waves = (GLU ? 2 : 1) * groups * splits, cps = (K / SK_KC + splits - 1) / splits, NO = GLU ? N / 2 : N;
+  const size_t rows = staged_lds_bytes(M, K), parts = (size_t)waves * MT * 64 * sizeof(f32x4);
+  gemm_skinny_staged_kernel<GLU, MT, TO><<<(NO + 16 * groups - 1) / (16 * groups), waves * 64, rows > parts ? rows : parts, stream>>>(
+      x, w, c, M, N, K, cps, splits, groups, finish);
+  IA_LAUNCH_CHECK();
+  return IA_OK;
+}
+
 // Shapes whose number of splits was measured (ia_gemm_skinny_set_splits, filled from a table when the library is
 // loaded): few entries, looked up per launch.
 struct KnownSplits { int N, K, splits; };
@@ -630,6 +769,15 @@ static int skinny_product(const void* X, const void* W, void* C, int out_dtype, 
     return launch_skinny<false, uint16_t, TILED>(x, w, (uint16_t*)C, nullptr, M, N, K, 1, stream);
   }
   const bool glu = epilogue == SK_EPI_SWIGLU;
+  const int groups = !TILED && C != nullptr && splits > 1 ? staged_groups(M, N, K, splits, glu) : 0;
+  if (groups > 0) {
+#define SK_STAGED(G, TO)                                                                                             \
+  (M <= 16 ? launch_staged<G, 1, TO>(x, w, (TO*)C, M, N, K, splits, groups, finish, stream)                          \
+           : launch_staged<G, 2, TO>(x, w, (TO*)C, M, N, K, splits, groups, finish, stream))
+    if (out_dtype == IA_F32) return glu ? SK_STAGED(true, float) : SK_STAGED(false, float);
+    return glu ? SK_STAGED(true, uint16_t) : SK_STAGED(false, uint16_t);
+#undef SK_STAGED
+  }
   if (!TILED && C != nullptr && splits > 1 && whole_k_pays(M, N, K, splits, glu)) {
     const int nchunks = (K + SK_KC - 1) / SK_KC, cps = (nchunks + splits - 1) / splits, NO = glu ? N / 2 : N;
     const dim3 grid((NO + 15) / 16), block((glu ? 2 : 1) * splits * 64);

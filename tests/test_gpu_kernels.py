@@ -637,6 +637,32 @@ def test_gemm_skinny_with_all_parts_in_one_workgroup_leaves_the_joined_parts_bit
         assert torch.allclose(got.double(), g / (1 + torch.exp(-g)) * u, rtol=1e-6, atol=1e-9)     # a few fp32 roundings
 
 
+# one to four groups of 16 rows of W a workgroup, of both halves too; columns that fill no group; the fewest and the most rows, a tile's last
+# and one more; two, three and four chunks a wave, an odd one at the end
+@pytest.mark.parametrize("N,K_,glu,rows", [(9216, 2048, False, (4, 15, 16, 17, 32)), (8259, 1536, False, (4, 31)), (12284, 4096, False, (4, 16)),
+                                           (13315, 1024, False, (4, 32)), (14336, 2560, False, (5, 16)), (5120, 2560, False, (8, 16)),
+                                           (8192, 2048, False, (12, 32)), (4099, 4096, False, (13,)), (4090, 2560, False, (16,)),
+                                           (5376, 2048, True, (8, 16, 17, 32)), (8160, 2560, True, (8, 16)), (7136, 1536, True, (9, 32)),
+                                           (8186, 2560, True, (8, 16))])
+def test_gemm_skinny_behind_rows_in_lds_leaves_the_joined_parts_bits(N, K_, glu, rows):
+    """Against the joined parts of 40 rows, which take the other kernels; rows behind the last are not written."""
+    api = K()
+    x, w, bias = _rand(40, K_, dtype=torch.bfloat16, seed=31), _rand(N, K_, dtype=torch.bfloat16, scale=0.05, seed=32), _rand(N, seed=33)
+    epilogue = "swiglu" if glu else None
+    assert api.gemm_skinny_splits(N, K_) > 1
+    for dtype in (torch.bfloat16, torch.float32):
+        want = api.gemm_skinny(x, w, epilogue=epilogue, out_dtype=dtype)
+        for M in rows:
+            room = torch.full((M + 1, want.shape[1]), 7.0, dtype=dtype, device=DEV)
+            api.gemm_skinny(x[:M].contiguous(), w, room[:M], epilogue=epilogue, out_dtype=dtype)
+            assert torch.equal(room[:M], want[:M]) and bool((room[M:] == 7.0).all()), (M, dtype)
+    if not glu:
+        want = api.gemm_skinny_finished(x, w, torch.empty(40, N, dtype=torch.bfloat16, device=DEV), bias, "gelu_tanh")
+        for M in rows:
+            got = api.gemm_skinny_finished(x[:M].contiguous(), w, torch.empty(M, N, dtype=torch.bfloat16, device=DEV), bias, "gelu_tanh")
+            assert torch.equal(got, want[:M]), M
+
+
 def test_gemm_skinny_takes_the_measured_number_of_parts_for_the_shapes_of_its_table():
     """The table of measured shapes is in force from the library's load on: its shapes are split as it says (the
     chunks of K dealt out evenly), others by the rule of sizes; a product of such a shape is right and its partial sums
