@@ -422,6 +422,12 @@ extern "C" int ia_gemm_mfma_split(const void* X, const void* W, float* parts, in
   // the walk goes by the tile's columns).  N x K in parts, us at 64 rows, 128 x 128 / 64 x 128: 6,144 x 4,096 in 5 14.7 / 13.6,
   // 4,096 x 14,336 in 8 25.9 / 24.9, 9,216 x 2,048 in 3 12.7 / 11.8, 2,048 x 2,048 in 8 7.4 / 6.6, 128,256 x 4,096 whole 206 / 202; at 17
   // rows 12.9 / 12.2, 26.2 / 24.4, 11.1 / 10.3, 6.3 / 5.5, 194 / 190.
+  // Where those leave half of the compute units without one, tiles of 64 x 64 give each of them half the columns and as many more units
+  // their loads; from 257 of them on a unit's second walks beside the first and the longer tiles read X less often.  64 x 128 / 64 x 64, us at
+  // 64 and 20 rows: 2,048 x 2,048 in 8 5.8 / 5.6, 5.0 / 4.8; 2,048 x 5,504 in 8 10.6 / 8.5, 9.2 / 7.7; 4,096 x 9,600 in 4 25.1 / 18.6, 22.5 / 16.9;
+  // 16,384 x 4,096 whole 37.7 / 27.1, 34.8 / 24.7; but 4,096 x 9,600 in 8 (512) 18.1 / 19.7, 8,192 x 2,048 in 4 10.6 / 11.1.
+  if (M <= 64 && (long long)((N + 63) / 64) * splits <= 256)
+    return launch_gemm_mfma<64, 64, 2, 2, 4, 1, true>((const uint16_t*)X, (const uint16_t*)W, nullptr, parts, M, N, K, splits, stream);
   if (M <= 64)
     return launch_gemm_mfma<64, 128, 2, 4, 3, 2, true>((const uint16_t*)X, (const uint16_t*)W, nullptr, parts, M, N, K, splits, stream);
   // Few columns (a router's) or few rows of them: a workgroup's walk over K is one chain of steps, each as long as its loads and its

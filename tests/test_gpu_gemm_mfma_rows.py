@@ -33,6 +33,21 @@ def test_up_to_64_rows_as_with_more(N, K_, S):
             assert torch.equal(api.gemm_mfma_swiglu(a[:M].contiguous(), w, tiled=tiled), act[:M]), M
 
 
+# as many tiles of 64 x 64 as there are compute units and one more (tiles of 64 x 128); columns that fill no tile; fewer steps of K than
+# stages, and more
+@pytest.mark.parametrize("N,K_,S", [(16380, 128, 1), (16386, 128, 1), (2040, 3200, 8), (2060, 640, 8)])
+def test_up_to_64_rows_by_how_many_tiles_there_are(N, K_, S):
+    from infernum_amd.kernels import api
+    a, w = _rand(129, K_, seed=5), _rand(N, K_, scale=0.1, seed=6)
+    of_129 = api.gemm_mfma_split(a, w, S).parts
+    want = a.double() @ w.double().t()
+    assert bool(((of_129.double().sum(0) - want).abs() <= 2e-5 * math.sqrt(K_) * 0.1).all())
+    for M in (64, 33, 17, 1):
+        parts = torch.full((S + 1, M, N), 7.0, device=DEV)
+        assert torch.equal(api.gemm_mfma_split(a[:M].contiguous(), w, S, parts[:S]).parts, of_129[:, :M]), M
+        assert bool((parts[S] == 7.0).all())
+
+
 def test_the_head_of_many_columns_from_17_rows_on():
     """An fp32 result as wide as fills the chip by the tiled kernel from 17 rows on, in the plan and in what linear gives; each row as
     near to 64 bits as by the weight-streaming kernel, and the same whatever stands beside it."""
