@@ -191,6 +191,113 @@ __global__ __launch_bounds__(256) void gemm_heads_few_kernel(const bf16_t* __res
   }
 }
 
+// The same for many rows of short K (a head's size), without LDS: a wave keeps 16 rows of x in registers and walks over its columns of the
+// head, 16 at a time, the next ones' rows of W under way (they come from the caches: a head's matrix is some tens of KB, read by every wave).
+// Bound by the reads of x and the writes of out; in tiles through LDS a step of K of 64 is a trip to memory and two barriers for 32 rows, and values
+// left one by one.  The same sums in the same order.  us, in tiles / so (at 6 TB/s): 2,047 rows of 16 heads of 224 x 64 23.8 / 9.6 (3.1), of
+// 64 x 224 with a gate 15.5 / 10.8 (3.8); 4,096 rows of 32 heads 83 / 26 (12.5) and 50 / 29 (15.2); 200 rows of 16 heads 5.4 / 3.4 and 9.3 / 3.7.
+// A wave's 32 rows share the reads of W: with short K, with a large matrix a head (1,000 rows of 128 heads of 512 x 128, 16 / 32 rows a wave 126 /
+// 75) and where 16 rows a wave fill the chip more than once (4,096 rows of 32 heads of 64 x 224 35 / 29; 2,047 of 16 10.8 / 11.6).
+#define GH_ROWS_K 256
+#define GH_ROWS_WORKGROUPS 512
+template <int KP, int MT>                                // steps of 32 of K, at most; groups of 16 rows a wave
+__global__ __launch_bounds__(256) void gemm_heads_rows_kernel(const bf16_t* __restrict__ x, int x_row, int x_head,
+                                                              const bf16_t* __restrict__ W, bf16_t* __restrict__ out, int o_row,
+                                                              int o_head, const bf16_t* __restrict__ gate, int g_row, int N, int Nout,
+                                                              int K, int tiles, bool fours) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
+  const int h = blockIdx.z, m0 = (blockIdx.y * 4 + wave) * (16 * MT);
+  if (m0 >= N) return;
+  const int first = blockIdx.x * tiles, last = min(first + tiles, (Nout + 15) / 16);
+  int row[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) row[i] = min(m0 + 16 * i + r, N - 1);
+  int kc[KP];
+  uint32_t keep[KP];                                     // pieces beyond K are read from the last place and cleared
+#pragma unroll
+  for (int j = 0; j < KP; ++j) {
+    kc[j] = min(32 * j + 8 * q, K - 8);
+    keep[j] = 32 * j + 8 * q < K ? 0xffffffffu : 0u;
+  }
+  const auto kept = [](const uint4& v, uint32_t k) { return make_uint4(v.x & k, v.y & k, v.z & k, v.w & k); };
+  uint4 xv[MT][KP], w0[KP], w1[KP];
+  uint2 g0[MT], g1[MT];
+  const auto load = [&](int t, uint4 (&w)[KP], uint2 (&g)[MT]) {
+    const bf16_t* w_row = W + ((size_t)h * Nout + min(16 * t + r, Nout - 1)) * K;
+#pragma unroll
+    for (int j = 0; j < KP; ++j) w[j] = *reinterpret_cast<const uint4*>(w_row + kc[j]);
+    if (gate) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        const bf16_t* g_at = gate + (size_t)row[i] * g_row + (size_t)h * Nout;
+        if (fours) {
+          g[i] = *reinterpret_cast<const uint2*>(g_at + min(16 * t + 4 * q, Nout - 4));
+        } else {
+          const int c = 16 * t + 4 * q, end = Nout - 1;
+          g[i].x = g_at[min(c, end)].bits | ((uint32_t)g_at[min(c + 1, end)].bits << 16);
+          g[i].y = g_at[min(c + 2, end)].bits | ((uint32_t)g_at[min(c + 3, end)].bits << 16);
+        }
+      }
+    }
+  };
+  const auto work = [&](int t, const uint4 (&w)[KP], const uint2 (&g)[MT]) {
+    tm_f32x4 acc[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) acc[i] = tm_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < KP; ++j) {
+      if (32 * j >= K) break;
+      const uint4 wt = kept(w[j], keep[j]);
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(tm_bf16x8, wt), __builtin_bit_cast(tm_bf16x8, xv[i][j]),
+                                                         acc[i], 0, 0, 0);
+    }
+    const int c = 16 * t + 4 * q;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      float y[4] = {acc[i][0], acc[i][1], acc[i][2], acc[i][3]};
+      if (gate) {
+        const float z[4] = {__uint_as_float(g[i].x << 16), __uint_as_float(g[i].x & 0xffff0000u), __uint_as_float(g[i].y << 16),
+                            __uint_as_float(g[i].y & 0xffff0000u)};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = to_float(from_float<bf16_t>(y[e])) * (1.0f / (1.0f + expf(-z[e])));
+      }
+      if (m0 + 16 * i + r >= N || c >= Nout) continue;
+      bf16_t* o_at = out + (size_t)row[i] * o_row + (size_t)h * o_head + c;
+      if (fours) {
+        *reinterpret_cast<uint2*>(o_at) = make_uint2(two_bf16_bits(y[0], y[1]), two_bf16_bits(y[2], y[3]));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (c + e < Nout) o_at[e] = from_float<bf16_t>(y[e]);
+      }
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < MT; ++i) {
+    const bf16_t* x_at = x + (size_t)row[i] * x_row + (size_t)h * x_head;
+    g0[i] = g1[i] = make_uint2(0u, 0u);
+#pragma unroll
+    for (int j = 0; j < KP; ++j) xv[i][j] = *reinterpret_cast<const uint4*>(x_at + kc[j]);
+  }
+  load(first, w0, g0);
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < KP; ++j) xv[i][j] = kept(xv[i][j], keep[j]);
+  int t = first;
+  for (; t + 1 < last; t += 2) {
+    load(t + 1, w1, g1);
+    __builtin_amdgcn_sched_barrier(0);
+    work(t, w0, g0);
+    load(min(t + 2, last - 1), w0, g0);
+    __builtin_amdgcn_sched_barrier(0);
+    work(t + 1, w1, g1);
+  }
+  if (t < last) work(t, w0, g0);
+}
+
 extern "C" int ia_gemm_heads(const void* x, int x_row, int x_head, const void* W, void* out, int o_row, int o_head,
                              const void* gate, int g_row, int dtype, int N, int H, int Nout, int K,
                              hipStream_t stream) {
@@ -209,6 +316,32 @@ extern "C" int ia_gemm_heads(const void* x, int x_row, int x_head, const void* W
       gemm_heads_few_kernel<<<dim3((Nout + 63) / 64, 1, H), 256, 0, stream>>>((const bf16_t*)x, x_row, x_head, (const bf16_t*)W,
                                                                               (bf16_t*)out, o_row, o_head, (const bf16_t*)gate,
                                                                               g_row, N, Nout, K);
+      IA_LAUNCH_CHECK();
+      return IA_OK;
+    }
+    if (K <= GH_ROWS_K) {
+      const int wide = K <= 64 || (long)Nout * K >= 32768 || (long)((N + 15) / 16) * H >= 4096 ? 2 : 1;
+      const int rows = (N + 64 * wide - 1) / (64 * wide), tiles = (Nout + 15) / 16;
+      if (rows > 65535) return IA_ERR_UNSUPPORTED;
+      // columns in so many pieces that the workgroups fill the chip
+      const long groups = (GH_ROWS_WORKGROUPS + (long)rows * H - 1) / ((long)rows * H);
+      const int per = groups >= tiles ? 1 : (int)((tiles + groups - 1) / groups);
+      const bool fours = ((Nout | o_row | o_head) & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0 &&
+                         (!gate || ((g_row & 3) == 0 && (reinterpret_cast<uintptr_t>(gate) & 7) == 0));
+      const dim3 pieces((tiles + per - 1) / per, rows, H);
+#define GH_ROWS(KP, MT)                                                                                                              \
+  gemm_heads_rows_kernel<KP, MT><<<pieces, 256, 0, stream>>>((const bf16_t*)x, x_row, x_head, (const bf16_t*)W, (bf16_t*)out, o_row, o_head, \
+                                                             (const bf16_t*)gate, g_row, N, Nout, K, per, fours)
+#define GH_ROWS_BY(MT)               \
+  do {                               \
+    if (K <= 64) GH_ROWS(2, MT);     \
+    else if (K <= 128) GH_ROWS(4, MT); \
+    else GH_ROWS(8, MT);             \
+  } while (0)
+      if (wide == 2) GH_ROWS_BY(2);
+      else GH_ROWS_BY(1);
+#undef GH_ROWS_BY
+#undef GH_ROWS
       IA_LAUNCH_CHECK();
       return IA_OK;
     }

@@ -199,6 +199,31 @@ def test_products_head_by_head_of_few_rows(N, H, J, Kd, gated):
     assert (out[:, :2] == 7.0).all() and (out[:, 2 + H * J:] == 7.0).all()
 
 
+# 16 and 32 rows a wave, the last ones of a wave's and of a workgroup's rows and one more; columns in one piece and in many, off groups of four;
+# K of a part of a step of 32 and of all of the eight.  The bits of few rows (the bound above) whatever stands beside them
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("N,H,J,Kd", [(64, 2, 64, 72), (65, 3, 37, 8), (129, 2, 224, 64), (128, 2, 130, 256), (257, 64, 20, 96), (40, 5, 300, 128),
+                                      (1030, 66, 16, 104), (100, 1, 3, 200)])
+def test_products_head_by_head_of_many_rows(N, H, J, Kd, gated):
+    from infernum_amd.kernels import api as K
+    g = torch.Generator().manual_seed(N + J)
+    x, w = torch.randn(N, H * Kd + 8, generator=g).bfloat16().cuda(), torch.randn(H, J, Kd, generator=g).bfloat16().cuda()
+    for first, lead in ((3, 2), (4, 4)):                                 # places that four values can be read and written at, and not
+        gate = torch.randn(N, H * J + 8, generator=g).bfloat16().cuda() if gated else None
+        out = torch.full((N, H * J + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+        K.gemm_heads(x, 8, Kd, w, out, lead, J, gate, first)
+        for lo in sorted({0, 16, N // 2, max(N - 5, 0)}):
+            n = min(4, N - lo)
+            few = torch.empty(n, H * J + 8, dtype=torch.bfloat16, device="cuda")
+            K.gemm_heads(x[lo:lo + n].contiguous(), 8, Kd, w, few, lead, J, gate[lo:lo + n].contiguous() if gated else None, first)
+            assert torch.equal(out[lo:lo + n, lead:lead + H * J], few[:, lead:lead + H * J]), lo
+        if not gated:
+            want = torch.einsum("nhk,hjk->nhj", x[:, 8:].double().view(N, H, Kd).cpu(), w.double().cpu()).reshape(N, H * J)
+            size = torch.einsum("nhk,hjk->nhj", x[:, 8:].double().view(N, H, Kd).cpu().abs(), w.double().cpu().abs()).reshape(N, H * J)
+            assert ((out[:, lead:lead + H * J].double().cpu() - want).abs() <= 2.0 ** -8 * want.abs() + Kd * 2.0 ** -24 * size).all()
+        assert (out[:, :lead] == 7.0).all() and (out[:, lead + H * J:] == 7.0).all()
+
+
 @BOTH
 @pytest.mark.parametrize("m,W,T", [
     (NM._mixer(3, 16, 8, 24, 24, 20), 64, 75),                       # head size 32, window inside the prompt
