@@ -1054,7 +1054,7 @@ __global__ __launch_bounds__(4 * HGW * 64) void attn_prefill_kernel(
   }
 }
 
-#if IA_ATTN_EXT == 0 && IA_HEAD_DIM == 128 && IA_VALUE_DIM == 128
+#if IA_ATTN_EXT == 0 && (IA_HEAD_DIM == 128 || IA_HEAD_DIM == 256) && IA_VALUE_DIM == IA_HEAD_DIM
 #define IA_PREFILL_WIDE 1
 #include "attention_prefill.h"
 #else
@@ -1254,7 +1254,9 @@ extern "C" int ia_attn_prefill(const void* q, int q_row_stride, const void* k_pa
       ps, num_pages, scale_log2, window, paired, sinks, stream)
     if (HGW == 1) PW_LAUNCH(1);
     if (HGW == 2) PW_LAUNCH(2);
+#if IA_HEAD_DIM <= 160
     PW_LAUNCH(4);
+#endif
 #undef PW_LAUNCH
   }
 #endif

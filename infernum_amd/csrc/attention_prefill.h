@@ -1,10 +1,11 @@
-// Prompt attention with 32 rows of a query head a wave (part of attention_mfma.hip, for a head size of 128 and two or more query heads
-// to a key/value head).
+// Prompt attention with 32 rows of a query head a wave (part of attention_mfma.hip, for a head size of 128 or 256 and two or more query
+// heads to a key/value head).
 //
 // A workgroup takes 64 rows (or, paired, 32 from each end of the request's new tokens) of up to HGW query heads of one key/value
 // head: two waves a head, 32 rows each as two tiles of 16 columns.  Keys and values come in tiles of 64 keys, by loads straight into LDS,
 // into rings of four stages: the keys of tile i + 3 and the values of tile i + 2 are asked for while tile i is worked on, half by
-// half, with one bare barrier a tile.
+// half, with one bare barrier a tile.  (Heads of 256: up to two query heads, tiles of 32 keys, each its only half, a barrier each: rings of
+// four stages fill LDS so.)
 //   S^T[key, col] = K[key, :] . Q[col, :]       v_mfma_f32_16x16x32_bf16 over 32 head dims a step
 //   O^T[dim, col] += V^T[dim, key] P^T[key, col] the same over 32 keys a step
 // Row r of the S^T tile t (of a half's two) stands for the key 8 (r / 4) + r % 4 + 4 t of the half, so that the accumulators leave
@@ -13,35 +14,38 @@
 //
 // What bounds it: with four heads a workgroup a SIMD has two such waves (LDS holds one workgroup a compute unit: one wave a SIMD with two
 // heads, every other SIMD has none with one), whose matrix instructions take 2,176 cycles a tile, their exponentials and what goes with them
-// some 1,700, and whose reads of LDS (256 KB a tile and compute unit, half of what waves of 16 rows need) 2,048.  These have to run
+// some 1,700, and whose reads of LDS (256 KB a tile and compute unit, half of what waves of 16 rows need) 1,024 where 16 lanes find 16
+// different places.  These have to run
 // beside each other: a piece of a pair of exponentials of 32 keys' scores stands behind every product of the next 32's scores and every one of the
-// probabilities of the 32 before.  The 8B shape's heads (32 over 8), waves of 16 rows / this kernel, us: 2,048 tokens 70 / 55, 4,096
-// 191 / 148, 8,192 662 / 508 (1.08 PFLOP/s), 2,048 after 6,144 cached 293 / 226; under a window of 4,096 8,192 tokens 512 / 412.  Short ranges
+// probabilities of the 32 before, and a product waits for its own two reads, not for those asked for behind them (ia_load_to_lds).  The
+// 8B shape's heads (32 over 8), waves of 16 rows / this kernel, us: 2,048 tokens 66 / 52, 4,096
+// 180 / 134, 8,192 663 / 485 (1.13 PFLOP/s), 2,048 after 6,144 cached 290 / 217; under a window of 4,096 8,192 tokens 511 / 388.  (Every read
+// waited for and keys where only 8 lanes found different places: 54, 141, 515, 227, 407.)  Heads of 256, 16 over 1: 2,047 tokens under a
+// window of 1,024 64 / 56, 3,000 tokens 156 / 115, 4,096 219 / 170; 16 over 8, 8,192 813 / 614 (0.9 PFLOP/s): one wave a SIMD, whose 66 products of
+// 32 keys take 1,056 of the 2,400 cycles that a tile takes it; 512 registers hold no more columns.  Short ranges
 // of keys are the other kernel's, by the same order of sums (a prompt of 20 tokens 5.9 / 8.9, of 257 13.9 / 15.5: a longer start, and a
 // wave's work one after the other); the line is drawn where launches are shaped.  With the products in a row and the exponentials behind them
-// 8,192 tokens took 590; with tests for a wave's first and last half inside the loop 587; with a mask in every half of a wave that has
-// rows to spare 4,016 tokens of 4 heads took 111, 80 without.
+// 8,192 tokens took 590 where this took 508; with tests for a wave's first and last half inside the loop 587; with a mask in every half of a
+// wave that has rows to spare 4,016 tokens of 4 heads took 111, 80 without.
 // Heads of 64 gained nothing (2,048 tokens 48 / 54, 8,192 438 / 418), one query head to a key/value head lost (2,000 tokens of 8 heads 53 / 67).
 //
-// In LDS the 16-byte piece c of row r (a key's values; a dim's 64 keys) lies at position c ^ s(r), s(key) = key % 4 + 4 (key / 8 % 2),
-// s(dim) = dim % 8: the 8 lanes that read together find 8 different places.
+// In LDS the 16-byte piece c of row r (a key's values; a dim's keys) lies at position c ^ s(r), s(key) = key % 4 + 4 (key / 8 % 4),
+// s(dim) = dim % 8 (of 32 keys dim / 2 % 4): the 16 lanes that read together find 16 different places.
 #pragma once
 
-#define PW_KT 64                        // keys a tile
+#define PW_KT (HD <= 128 ? 64 : 32)      // keys a tile
 #define PW_STAGES 4
 #define PW_INLINE __attribute__((always_inline))
 #define PW_BT 4096                      // block-table entries kept in LDS
 
-typedef const __attribute__((address_space(1))) void* pw_global_ptr;
-typedef __attribute__((address_space(3))) void* pw_lds_ptr;
-
+constexpr int PW_HALVES = PW_KT / 32, PW_VP = PW_KT / 8;      // 32 keys each; pieces of a dim's row of V^T
 constexpr int PW_K_BYTES = PW_KT * HD * 2, PW_V_BYTES = VD * PW_KT * 2;
 constexpr int PW_LDS = PW_STAGES * (PW_K_BYTES + PW_V_BYTES) + PW_BT * 4;
 
 typedef f32x4 pw_scores[2][2];          // of 32 keys: [tile of 16][column]
 
 template <int HGW, bool WINDOW>
-__global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
+__global__ __launch_bounds__(HGW * 128, HD <= 128 ? 2 : 1) void attn_prefill_wide_kernel(
     const uint16_t* __restrict__ q, int q_row_stride, const uint16_t* __restrict__ k_pages, const uint16_t* __restrict__ v_pages,
     uint16_t* __restrict__ out, int out_row_stride, const int* __restrict__ seq_starts, const int* __restrict__ seq_ctx,
     const int* __restrict__ block_tables, int bt_stride, const int* __restrict__ tiles, int nh, int nkv, int ps_shift, int num_pages,
@@ -53,6 +57,7 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
   extern __shared__ __attribute__((aligned(1024))) char pw_lds[];
   char* const k_lds = pw_lds;
   char* const v_lds = pw_lds + PW_STAGES * PW_K_BYTES;
+  const uint32_t k_first = ia_lds_address(k_lds), v_first = k_first + PW_STAGES * PW_K_BYTES;
   int* const s_bt = reinterpret_cast<int*>(v_lds + PW_STAGES * PW_V_BYTES);
   __shared__ int s_poison;
 
@@ -118,9 +123,11 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
     for (int i = tid; i < count; i += THREADS) s_bt[i] = bt[first + i];
   }
   // the queries are here before the first load into LDS: waiting for them behind it would wait for all of these too
-  static_assert(KS == 4, "all queries of a lane");
-  asm volatile("" : "+v"(qreg[0][0]), "+v"(qreg[0][1]), "+v"(qreg[0][2]), "+v"(qreg[0][3]), "+v"(qreg[1][0]), "+v"(qreg[1][1]),
-               "+v"(qreg[1][2]), "+v"(qreg[1][3]));
+  static_assert(KS % 4 == 0, "all queries of a lane");
+#pragma unroll
+  for (int st = 0; st < KS; st += 4)
+    asm volatile("" : "+v"(qreg[0][st]), "+v"(qreg[0][st + 1]), "+v"(qreg[0][st + 2]), "+v"(qreg[0][st + 3]), "+v"(qreg[1][st]),
+                 "+v"(qreg[1][st + 1]), "+v"(qreg[1][st + 2]), "+v"(qreg[1][st + 3]));
 #pragma unroll
   for (int c = 0; c < 2; ++c)
 #pragma unroll
@@ -129,8 +136,8 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
   const f32x4 none = {0.f, 0.f, 0.f, 0.f};
   const bf16x8_t ones = __builtin_bit_cast(bf16x8_t, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
 
-  // ---- loads.  A wave brings KG groups of eight keys, KF / KG loads each, and VF loads of 8 dims' 64 keys each, of which a lane
-  // has the same eight every time: eight keys lie in one page.  Groups beyond the range come from the page at its end (scores of theirs are
+  // ---- loads.  A wave brings KG groups of eight keys, KF / KG loads each, and VF loads of a tile's keys of VDIMS dims each, of which a
+  // lane has the same eight every time: eight keys lie in one page.  Groups beyond the range come from the page at its end (scores of theirs are
   // masked, values zeroed).
   constexpr int KG = PW_KT / 8 / NW >= 1 ? PW_KT / 8 / NW : 1, KL = KF / KG;
   static_assert(KG * KL == KF && KG * NW == PW_KT / 8, "whole groups");
@@ -138,10 +145,12 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
   const char* const k_base = reinterpret_cast<const char*>(k_pages) + (size_t)g * ps * (HD * 2);
   const char* const v_base = reinterpret_cast<const char*>(v_pages) + (size_t)g * VD * (ps * 2);
   const int k_row = lane / (HD / 8);
-  // s(key) of the rows of a load: bit 2 is the group's number's lowest bit
+  // s(key) of the rows of a load: bits 2 and 3 are the group's number's lowest
   const uint32_t k_lane_at = (uint32_t)(k_row * HD * 2 + (((lane & (HD / 8 - 1)) ^ (k_row & 3)) * 16));
-  const int v_key = 8 * ((lane & 7) ^ (lane >> 3));
-  const uint32_t v_lane_at = (uint32_t)(8 * wave * VF + (lane >> 3)) * (uint32_t)(ps * 2), v_step = (uint32_t)(16 * ps);
+  constexpr int VDIMS = 64 / PW_VP;
+  auto v_swizzle = [&](int dim) PW_INLINE { return PW_KT == 64 ? dim & 7 : (dim >> 1) & 3; };
+  const int v_key = 8 * ((lane & (PW_VP - 1)) ^ v_swizzle(lane / PW_VP));
+  const uint32_t v_lane_at = (uint32_t)(VDIMS * wave * VF + lane / PW_VP) * (uint32_t)(ps * 2), v_step = (uint32_t)(2 * VDIMS * ps);
   const int last_page = (key_hi >> ps_shift) - bt_first;
   bool bad = false;
   int k_pg[KG], v_pg;
@@ -157,12 +166,20 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
       const bool ok = (unsigned)k_pg[f] < (unsigned)num_pages;
       bad |= !ok;
       const uint32_t in_page = (uint32_t)((t * PW_KT + 8 * (wave * KG + f)) & (ps - 1)) * (HD * 2);
-      const char* src = k_base + ((uint64_t)(uint32_t)(ok ? k_pg[f] : 0) * k_page + (in_page + (k_lane_at ^ (((wave * KG + f) & 1) * 64u))));
+      const uint32_t at = k_lane_at ^ (((wave * KG + f) & 3) * 64u);
+      const char* const page = k_base + (uint64_t)(uint32_t)(ok ? k_pg[f] : 0) * k_page;
+      const char* src = page + (in_page + at);
       // a group's loads follow each other in the page and in LDS alike: the instruction's offset moves both
-      char* const dst = k_lds + slot * PW_K_BYTES + 1024 * KL * (wave * KG + f);
-      __builtin_amdgcn_global_load_lds((pw_global_ptr)src, (pw_lds_ptr)dst, 16, 0, 0);
-      if constexpr (KL > 1) __builtin_amdgcn_global_load_lds((pw_global_ptr)src, (pw_lds_ptr)dst, 16, 1024, 0);
-      static_assert(KL <= 2, "a group's loads");
+      const uint32_t dst = k_first + slot * PW_K_BYTES + 1024 * KL * (wave * KG + f);
+      ia_load_to_lds<0>(src, dst);
+      if constexpr (KL == 2) ia_load_to_lds<1024>(src, dst);
+      if constexpr (KL == 4) {                    // two keys a load: every other one's begin with key % 4 = 2
+        const char* const other = page + (in_page + (at ^ 32u));
+        ia_load_to_lds<1024>(other, dst);
+        ia_load_to_lds<2048>(src, dst);
+        ia_load_to_lds<3072>(other, dst);
+      }
+      static_assert(KL == 1 || KL == 2 || (KL == 4 && HD == 256), "a group's loads");
     }
   };
   auto load_v = [&](int t, int slot) PW_INLINE {
@@ -171,16 +188,17 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
     const uint32_t in_page = (uint32_t)((t * PW_KT + v_key) & (ps - 1)) * 2u;
     const char* src = v_base + ((uint64_t)(uint32_t)(ok ? v_pg : 0) * v_page + (v_lane_at + in_page));
 #pragma unroll
-    for (int f = 0; f < VF; ++f)
-      __builtin_amdgcn_global_load_lds((pw_global_ptr)(src + (uint64_t)(f * v_step)),
-                                       (pw_lds_ptr)(v_lds + slot * PW_V_BYTES + 1024 * (wave * VF + f)), 16, 0, 0);
+    for (int f = 0; f < VF; ++f) ia_load_to_lds<0>(src + (uint64_t)(f * v_step), v_first + slot * PW_V_BYTES + 1024 * (wave * VF + f));
   };
 
   // ---- reads: this lane's row and pieces
   const int k_lane = (8 * (j >> 2) + (j & 3)) * (HD * 2), v_lane = j * (PW_KT * 2);
-  const int piece0 = (qd ^ (j & 7)) * 16, piece1 = ((4 + qd) ^ (j & 7)) * 16;
+  const int v_piece0 = (qd ^ v_swizzle(j)) * 16, v_piece1 = ((4 + qd) ^ v_swizzle(j)) * 16;      // (of 32 keys the first alone)
+  int k_piece[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) k_piece[s] = k_lane + ((4 * s + qd) ^ j) * 16;
   auto read_k = [&](const char* half, int t, int st) PW_INLINE {        // tile t of the half's two, step st of the head dims
-    return *reinterpret_cast<const bf16x8_t*>(half + k_lane + t * (4 * HD * 2) + (st >> 1) * 128 + ((st & 1) ? piece1 : piece0));
+    return *reinterpret_cast<const bf16x8_t*>(half + k_piece[st & 3] + t * (4 * HD * 2) + (st >> 2) * 256);
   };
   // `values`: the stage of the half's tile, with this lane's place in it
   auto read_v = [&](const char* values, int n) PW_INLINE { return *reinterpret_cast<const bf16x8_t*>(values + n * (16 * PW_KT * 2)); };
@@ -257,6 +275,7 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
     constexpr int NY = NSV;                                  // turns: a read of keys and one of values, two products each
     static_assert(2 * KS == NSV, "as many reads of keys as of values");
     bf16x8_t ak[3], av[3], p[2];
+    f32x2_t e;
 #pragma unroll
     for (int y = 0; y < 2; ++y) {
       ak[y] = read_k(half, y & 1, y >> 1);
@@ -274,19 +293,19 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
         ak[(y + 2) % 3] = read_k(half, (y + 2) & 1, (y + 2) >> 1);
         av[(y + 2) % 3] = read_v(values, y + 2);
       }
-      // the turn's pairs of exponentials, a piece behind each of its four products
-      constexpr int PAIRS = 8 / NY;
-      f32x2_t e[PAIRS];
-      auto piece = [&](int stage) {
-#pragma unroll
-        for (int k = 0; k < PAIRS; ++k) {
-          const int i = y * PAIRS + k, c = i >> 2, t = (i >> 1) & 1, r = 2 * (i & 1);
-          if (stage == 0) e[k] = (f32x2_t){fmaf(cur[t][c][r], scale_log2, neg[c]), fmaf(cur[t][c][r + 1], scale_log2, neg[c])};
-          if (stage == 1) e[k][0] = __builtin_amdgcn_exp2f(e[k][0]);
-          if (stage == 2) e[k][1] = __builtin_amdgcn_exp2f(e[k][1]);
+      // the turn's pair of exponentials, a piece behind each of its four products (with twice the turns: of two turns' eight)
+      constexpr int SLOW = NY / 8;
+      static_assert(NY == 8 || NY == 16, "eight pairs of exponentials");
+      auto piece = [&](int place) {
+        const int stage = SLOW == 1 ? place : (place & 1) ? 2 * (y & 1) + (place >> 1) : 4;
+        {
+          const int i = y / SLOW, c = i >> 2, t = (i >> 1) & 1, r = 2 * (i & 1);
+          if (stage == 0) e = (f32x2_t){fmaf(cur[t][c][r], scale_log2, neg[c]), fmaf(cur[t][c][r + 1], scale_log2, neg[c])};
+          if (stage == 1) e[0] = __builtin_amdgcn_exp2f(e[0]);
+          if (stage == 2) e[1] = __builtin_amdgcn_exp2f(e[1]);
           if (stage == 3) {
-            pk[c][i & 3] = __builtin_bit_cast(uint32_t, __builtin_convertvector(e[k], bf16x2_t));
-            emax[c] = fmaxf(emax[c], fmaxf(e[k][0], e[k][1]));
+            pk[c][i & 3] = __builtin_bit_cast(uint32_t, __builtin_convertvector(e, bf16x2_t));
+            emax[c] = fmaxf(emax[c], fmaxf(e[0], e[1]));
           }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -353,8 +372,8 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
     // values of keys that no row sees are not the request's: zero them in LDS (the tiles at the ends of the range)
     const int t0 = i * PW_KT;
     if (t0 < key_lo || t0 + PW_KT - 1 > key_hi) {
-      for (int at = tid; at < VD * 8; at += THREADS) {
-        const int dim = at >> 3, key = t0 + 8 * ((at & 7) ^ (dim & 7));
+      for (int at = tid; at < VD * PW_VP; at += THREADS) {
+        const int dim = at / PW_VP, key = t0 + 8 * ((at & (PW_VP - 1)) ^ v_swizzle(dim));
         if (key >= key_lo && key + 7 <= key_hi) continue;
         uint16_t* const v = reinterpret_cast<uint16_t*>(v_lds + slot * PW_V_BYTES + at * 16);
 #pragma unroll
@@ -368,31 +387,50 @@ __global__ __launch_bounds__(HGW * 128, 2) void attn_prefill_wide_kernel(
   };
   int i = t_begin;
   if (WINDOW) {
-    for (; i < w_begin >> 1; ++i) round(i);
+    for (; i < w_begin / PW_HALVES; ++i) round(i);
   }
   const int first = i;
   if (wave_live) scores(sa, k_lds + ((i - t_begin) & 3) * PW_K_BYTES);
-  auto even = [&]() PW_INLINE {
-    const int slot = (i - t_begin) & 3;
-    const char* const here = v_lds + slot * PW_V_BYTES + v_lane;
-    part(2 * i, sa, sb, pa, pb, k_lds + slot * PW_K_BYTES + 32 * HD * 2,
-         i == first ? here + piece0 : v_lds + ((slot + 3) & 3) * PW_V_BYTES + v_lane + piece1);
-    return here;
-  };
-  for (; 2 * i < w_end; ++i) {
-    round(i);
-    const char* const here = even();
-    part(2 * i + 1, sb, sa, pb, pa, k_lds + (((i - t_begin) + 1) & 3) * PW_K_BYTES, here + piece0);
-  }
-  if (wave_live) {
-    // the last half's values: of a tile that is there until the next round
-    const bool in_first = 2 * i == w_end;
+  bool in_first;                        // the last half was a tile's first, or of tiles of one half an even one
+  const char* values;                   // the last half's: of a tile that is there until the next round
+  if constexpr (PW_HALVES == 2) {
+    auto even = [&]() PW_INLINE {
+      const int slot = (i - t_begin) & 3;
+      const char* const here = v_lds + slot * PW_V_BYTES + v_lane;
+      part(2 * i, sa, sb, pa, pb, k_lds + slot * PW_K_BYTES + 32 * HD * 2,
+           i == first ? here + v_piece0 : v_lds + ((slot + 3) & 3) * PW_V_BYTES + v_lane + v_piece1);
+      return here;
+    };
+    for (; 2 * i < w_end; ++i) {
+      round(i);
+      const char* const here = even();
+      part(2 * i + 1, sb, sa, pb, pa, k_lds + (((i - t_begin) + 1) & 3) * PW_K_BYTES, here + v_piece0);
+    }
+    in_first = 2 * i == w_end;
     if (in_first) {
       round(i);
       even();
       ++i;
     }
-    const char* const values = v_lds + ((i - 1 - t_begin) & 3) * PW_V_BYTES + v_lane + (in_first ? piece0 : piece1);
+    values = v_lds + ((i - 1 - t_begin) & 3) * PW_V_BYTES + v_lane + (in_first ? v_piece0 : v_piece1);
+  } else {
+    auto keys_of = [&](int x) PW_INLINE { return k_lds + ((x - t_begin) & 3) * PW_K_BYTES; };
+    auto values_of = [&](int x) PW_INLINE { return v_lds + ((x - t_begin) & 3) * PW_V_BYTES + v_lane + v_piece0; };
+    for (; i < w_end; i += 2) {
+      round(i);
+      part(i, sa, sb, pa, pb, keys_of(i + 1), values_of(i == first ? i : i - 1));
+      round(i + 1);
+      part(i + 1, sb, sa, pb, pa, keys_of(i + 2), values_of(i));
+    }
+    in_first = i == w_end;
+    if (in_first) {
+      round(i);
+      part(i, sa, sb, pa, pb, keys_of(i + 1), values_of(i == first ? i : i - 1));
+      ++i;
+    }
+    values = values_of(i - 1);
+  }
+  if (wave_live) {
     bf16x8_t p[2];
 #pragma unroll
     for (int c = 0; c < 2; ++c) {

@@ -227,6 +227,20 @@ __device__ __forceinline__ int ia_expert_first_chunk(int column, int K) {
   return (int)((((unsigned)(column / 512) * 0x9E3779B1u) >> 8) % chunks);
 }
 
+// Every lane's 16 bytes at src + AT, straight into LDS from lds + AT on, lane after lane (lds the same for the wave).  Written out: the
+// compiler takes the builtin for an access of memory and of LDS at once, and with one under way it waits for all reads of LDS, the newest
+// too, where it needs the oldest (prompt attention with heads of 128, two reads in flight over every product: 8,192 tokens of 32
+// heads 515 us with the builtin, 504 so; heads of 256, 8,192 tokens of 16 heads 655 / 614).  Nothing comes back in a register, and nobody
+// but the caller waits: for vmcnt before a barrier, before LDS is read and before the workgroup ends.  (One instruction has to
+// lie between the write of m0 and the load.)
+template <int AT>
+__device__ __forceinline__ void ia_load_to_lds(const char* src, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off offset:%2" ::"s"(lds), "v"(src), "n"(AT) : "memory", "m0");
+}
+__device__ __forceinline__ uint32_t ia_lds_address(const char* p) {
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p);
+}
+
 // The first key that a query at position p sees, from the mask's code: 0 all keys from 0; w > 0 a sliding
 // window, the last w keys (p - w + 1 .. p); w < 0 chunks of -w positions counted from the request's start,
 // the keys of the query's own chunk (floor(p / c) c .. p).  Never decreases with p.

@@ -1202,21 +1202,25 @@ def prefill_launch_shape(nh: int, nkv: int, d: int, q_lens: Sequence[int], ctx_l
 # A wave of 32 rows that two chunks share walks both, which all others wait for (4,096 tokens of 16 heads over 8 in chunks of 1,024 from a chunk's
 # start on 58.8 / 53.4, from 16 tokens on 60.7 / 76.5): where a request's rows do not begin on a multiple of 32 and chunks are no longer than
 # PREFILL_NARROW_CHUNK, 16 rows (183 launches under chunks: 1.3 % longer than the faster, at most 5 % longer than 16 rows).
+# Heads of 256 (two a workgroup): one prompt of 257 tokens 19.5 / 21.1, of 512 28.5 / 29.0, of 600 34.5 / 32.3; 12 of 416 56.3 / 58.8, of 512
+# 72.8 / 70.3; 20 of 130 53 / 58; a portion of 30 rows under a window of 512 31.4 / 32.5; 4,080 rows from 16 tokens on under
+# chunks of 1,024 101 / 116.
 PREFILL_NARROW_KEYS = (600, 448)
+PREFILL_NARROW_KEYS_256 = 512
 PREFILL_NARROW_CHUNK = 2048
 
 
 def prefill_shape(nh: int, nkv: int, d: int, q_lens: Sequence[int], ctx_lens: Sequence[int], window: int, device: torch.device) -> int:
-    """:func:`prefill_launch_shape`, with :data:`PREFILL_NARROW` added where waves of 16 rows are the faster (a head size of 128 with two and
-    more query heads to a key/value head has both; elsewhere it is without effect).  The bits of the result do not depend on it."""
+    """:func:`prefill_launch_shape`, with :data:`PREFILL_NARROW` added where waves of 16 rows are the faster (a head size of 128 or 256 with two
+    and more query heads to a key/value head has both; elsewhere it is without effect).  The bits of the result do not depend on it."""
     shape = prefill_launch_shape(nh, nkv, d, q_lens, ctx_lens, window, device)
-    if shape == 0 or d != 128 or nh < 2 * nkv:
+    if shape == 0 or d not in (128, 256) or nh < 2 * nkv:
         return shape
     longest = max(q + c for q, c in zip(q_lens, ctx_lens))
     if window:
         longest = min(longest, abs(window) + 64)
     shared = 0 < -window <= PREFILL_NARROW_CHUNK and any(c % 32 for c in ctx_lens)
-    narrow = shared or longest <= PREFILL_NARROW_KEYS[shape & 0xff == 4]
+    narrow = shared or longest <= (PREFILL_NARROW_KEYS_256 if d == 256 else PREFILL_NARROW_KEYS[shape & 0xff == 4])
     return shape | (PREFILL_NARROW if narrow else 0)
 
 

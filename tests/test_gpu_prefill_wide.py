@@ -15,7 +15,7 @@ def K():
     return api
 
 
-def _case(nh, nkv, ps, lens, q_lens, seed, cols=None, poison=True):
+def _case(nh, nkv, ps, lens, q_lens, seed, cols=None, poison=True, D=D):
     """Requests of lens keys whose last q_lens tokens are new, pages in a shuffled order; what no request holds is NaN."""
     g = torch.Generator(device=DEV).manual_seed(seed)
     rnd = lambda *s: torch.randn(*s, device=DEV, generator=g).to(torch.bfloat16)                     # noqa: E731
@@ -45,6 +45,7 @@ def _case(nh, nkv, ps, lens, q_lens, seed, cols=None, poison=True):
 
 def _run(c, nh, nkv, window=0, **kw):
     out = torch.full_like(c["q"], float("nan"))
+    D = c["kp"].shape[3]
     K().attention_prefill(c["q"], c["kp"], c["vp"], out, c["starts"], c["ctx"], c["bt"], c["tiles"], c["tiles"].shape[0], nh, nkv, D,
                           D ** -0.5, window, **kw)
     return out
@@ -52,6 +53,7 @@ def _run(c, nh, nkv, window=0, **kw):
 
 def _want(c, nh, nkv, window):
     rows, at = [], 0
+    D = c["kp"].shape[3]
     for k, v, n, m in zip(c["k"], c["v"], c["lens"], c["q_lens"]):
         q = c["q"][at:at + m].view(m, nh, D).double()
         at += m
@@ -235,3 +237,36 @@ def test_sinks_and_rows_that_lie_apart(lens, q_lens, window):
     K().attention_prefill(wide_q[:, :nh * D], c["kp"], c["vp"], wide_o[:, :nh * D], c["starts"], c["ctx"], c["bt"], c["tiles"],
                           c["tiles"].shape[0], nh, nkv, D, D ** -0.5, window, sinks=sinks)
     assert torch.equal(wide_o[:, :nh * D], first) and bool((wide_o[:, nh * D:] == 7.0).all())
+
+
+@pytest.mark.parametrize("nh,nkv,ps", [(4, 1, 16), (6, 2, 8), (3, 1, 64)])
+@pytest.mark.parametrize("lens,q_lens", [([1, 2, 31, 32, 33], [1, 2, 31, 32, 33]), ([63, 64, 65, 127, 129], [63, 64, 65, 127, 129]),
+                                         ([95, 96, 97, 200, 161], [1, 33, 65, 64, 7]), ([300, 449], [300, 100])])
+@pytest.mark.parametrize("window", [0, 1, 40, 100, -16, -48, -96])
+def test_heads_of_256_at_the_edges_of_tiles(nh, nkv, ps, lens, q_lens, window):
+    """A tile is one half of 32 keys there: the kernel's other loop, and the same bits from waves of 16 rows."""
+    c = _case(nh, nkv, ps, lens, q_lens, seed=nh * ps + len(lens) + window, D=256)
+    first = _run(c, nh, nkv, window, heads_per_workgroup=K().PREFILL_NARROW | 2)
+    if window >= 0:                      # as for heads of 128 above
+        assert (first.double() - _want(c, nh, nkv, window)).abs().max().item() <= 2.5e-2
+    for hpw in (0, 1, 2):
+        for paired in (False, True):
+            assert torch.equal(_run(c, nh, nkv, window, heads_per_workgroup=hpw, paired=paired), first), (hpw, paired)
+    with pytest.raises(K().KernelError):
+        _run(c, nh, nkv, window, heads_per_workgroup=4)
+    t, page = lens[-1] - 1, int(c["bt"][-1, (lens[-1] - 1) // ps])              # a value that the rows before its 16 do not meet
+    c["vp"][page, :, :, t % ps] = float("inf")
+    bad = _run(c, nh, nkv, window)
+    assert torch.equal(bad, _run(c, nh, nkv, window, heads_per_workgroup=K().PREFILL_NARROW | 2)) or not bool(bad[-1].isfinite().any())
+    blocks = -(-q_lens[-1] // 16) - 1
+    clean = [r for r in range(blocks * 16) if (lens[-1] - q_lens[-1] + r // 16 * 16 + 15) // 32 < t // 32]
+    assert torch.equal(bad[bad.shape[0] - q_lens[-1]:][clean], first[first.shape[0] - q_lens[-1]:][clean]) and not bool(bad[-1].isfinite().any())
+
+
+def test_short_ranges_of_heads_of_256_go_to_waves_of_16_rows():
+    api, dev = K(), torch.device(DEV)
+    narrow = lambda q, c, nh=16, nkv=1, w=0: bool(api.prefill_shape(nh, nkv, 256, q, c, w, dev) & api.PREFILL_NARROW)    # noqa: E731
+    line = api.PREFILL_NARROW_KEYS_256
+    assert narrow([line], [0]) and not narrow([line + 1], [0]) and narrow([30], [line - 30]) and not narrow([30], [line - 29])
+    assert narrow([64], [5000], w=line - 64) and not narrow([64], [5000], w=line - 63) and not narrow([20], [0], nh=1)
+    assert narrow([64], [5000], w=-1024) and not narrow([64], [5024], w=-1024) and not narrow([64], [5000], w=-api.PREFILL_NARROW_CHUNK - 1)
