@@ -237,6 +237,10 @@ template <int AT>
 __device__ __forceinline__ void ia_load_to_lds(const char* src, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off offset:%2" ::"s"(lds), "v"(src), "n"(AT) : "memory", "m0");
 }
+// The same from src + at, src the same for the wave.
+__device__ __forceinline__ void ia_load_to_lds(const char* src, uint32_t at, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(at), "s"(src) : "memory", "m0");
+}
 __device__ __forceinline__ uint32_t ia_lds_address(const char* p) {
   return (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p);
 }

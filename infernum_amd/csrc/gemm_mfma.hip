@@ -5,14 +5,16 @@
 // (BN / WAVES_N) of it as 32 x 32 accumulator tiles.  K is walked in steps of 64.  The BM x 64 tile of X and
 // the BN x 64 tile of W of a later step go from global memory straight into a free stage of a ring of LDS
 // buffers (global_load_lds_dwordx4: no registers and no LDS store instructions on the way) while the matrix
-// cores work on this step; one barrier a step.
+// cores work on this step; one barrier a step.  (Written out, see ia_load_to_lds: with the builtin every quarter of a step began with a
+// wait for all reads of LDS under way.  With that gone and 16 places for 16 rows, below: 28,672 x 4,096 with the activation, 64 rows 43.3
+// us before, 41.7 now, 256 rows 85.8 / 82.0; 6,144 x 4,096 in 4 parts, 64 rows 15.9 / 15.1; 2,048 rows of 4,096 x 4,096 63.2 / 58.3.)
 //
 // Both matrices have K contiguous, which is what the operands want: lane (i, h) = (lane % 32, lane / 32) of
 // an operand holds the 8 values k = 16 s + 8 h .. + 7 of row i, one 16-byte LDS read.  A load instruction
 // of a wave fills 1,024 consecutive bytes of LDS, lane by lane, which is 8 rows of 128 bytes without
-// padding; so that the reads of rows i, i + 1, .. do not all fall on the same banks, the 16-byte piece c of
-// row r lies at position c ^ (r % 8) of its row: the lane that fills position p of row r fetches piece
-// p ^ (r % 8) from global memory.
+// padding; so that the 16 rows read together fall on 16 different places of two rows' banks, the 16-byte piece c of
+// row r lies at position c ^ (r / 2 % 8) of its row: the lane that fills position p of row r fetches piece
+// p ^ (r / 2 % 8) from global memory.
 //
 // Workgroups are numbered so that the ones running together share rows of W and X in L2.
 //
@@ -34,8 +36,6 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 #define GM_BK 64
 #define GM_ROW_BYTES (GM_BK * 2)
 
-typedef const __attribute__((address_space(1))) void* gm_global_ptr;
-typedef __attribute__((address_space(3))) void* gm_lds_ptr;
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int FILL_STEPS, bool SPLIT, bool GLU = false,
           bool WT = false>
@@ -79,6 +79,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_mfma_kernel(const
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t lds_first = ia_lds_address(lds);
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
   const int li = lane & 31, lh = lane >> 5;
 
@@ -88,7 +89,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_mfma_kernel(const
 #pragma unroll
   for (int f = 0; f < FPW; ++f) {
     const int row = 8 * (f * WAVES + wave) + (lane >> 3);
-    const int piece = (lane & 7) ^ (row & 7);
+    const int piece = (lane & 7) ^ ((row >> 1) & 7);
     int r;
     if (8 * f * WAVES < BM) {
       r = min(m0 + row, M - 1);
@@ -120,10 +121,9 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_mfma_kernel(const
     return (size_t)ks * GM_ROW_BYTES;
   };
 #define GM_FILL(f, kt, buf)                                                                                  \
-  __builtin_amdgcn_global_load_lds(                                                                         \
-      (gm_global_ptr)(reinterpret_cast<const char*>((8 * (f) * WAVES < BM) ? X : W) +                       \
-                      step_offset(k_first + krot(kt), !(8 * (f) * WAVES < BM)) + src[f]),                   \
-      (gm_lds_ptr)(lds + (buf) * STAGE_BYTES + 1024 * ((f) * WAVES + wave)), 16, 0, 0)
+  ia_load_to_lds(reinterpret_cast<const char*>((8 * (f) * WAVES < BM) ? X : W) +                            \
+                     step_offset(k_first + krot(kt), !(8 * (f) * WAVES < BM)), src[f],                      \
+                 lds_first + (buf) * STAGE_BYTES + 1024 * ((f) * WAVES + wave))
 
   // W is the first operand: accumulator register r of lane (j, h) = (lane % 32, lane / 32) of tile [a][b] is
   // the product for n = 32 a + 8 (r / 4) + 4 h + r % 4 and m = 32 b + j, four neighbours in a row of C at a time
@@ -160,12 +160,12 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_mfma_kernel(const
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 2) * FPW) : "memory");
   __syncthreads();
 
-  // piece 2 s + h of row i lies at position (2 s + h) ^ (i % 8); tiles start at multiples of 32 rows
+  // piece 2 s + h of row i lies at position (2 s + h) ^ (i / 2 % 8); tiles start at multiples of 32 rows
   const int xrow = (wm * WM + li) * GM_ROW_BYTES;
   const int wrow = (BM + wn * WN + li) * GM_ROW_BYTES;
   int swz[KS];
 #pragma unroll
-  for (int s = 0; s < KS; ++s) swz[s] = ((2 * s + lh) ^ (li & 7)) * 16;
+  for (int s = 0; s < KS; ++s) swz[s] = ((2 * s + lh) ^ ((li >> 1) & 7)) * 16;
 
   // The operands of a step's first matrix instructions are read during the last quarter of the step before,
   // and the barrier stands before that quarter, so that no wave waits at a step's start:
