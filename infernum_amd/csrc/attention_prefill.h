@@ -18,10 +18,11 @@
 // different places.  These have to run
 // beside each other: a piece of a pair of exponentials of 32 keys' scores stands behind every product of the next 32's scores and every one of the
 // probabilities of the 32 before, and a product waits for its own two reads, not for those asked for behind them (ia_load_to_lds).  The
-// 8B shape's heads (32 over 8), waves of 16 rows / this kernel, us: 2,048 tokens 66 / 52, 4,096
-// 180 / 134, 8,192 663 / 485 (1.13 PFLOP/s), 2,048 after 6,144 cached 290 / 217; under a window of 4,096 8,192 tokens 511 / 388.  (Every read
+// 8B shape's heads (32 over 8), waves of 16 rows / this kernel, us: 2,048 tokens 63 / 52, 4,096
+// 164 / 134, 8,192 600 / 485 (1.13 PFLOP/s), 2,048 after 6,144 cached 271 / 217; under a window of 4,096 8,192 tokens 465 / 388.  (Every read
 // waited for and keys where only 8 lanes found different places: 54, 141, 515, 227, 407.)  Heads of 256, 16 over 1: 2,047 tokens under a
-// window of 1,024 64 / 56, 3,000 tokens 156 / 115, 4,096 219 / 170; 16 over 8, 8,192 813 / 614 (0.9 PFLOP/s): one wave a SIMD, whose 66 products of
+// window of 1,024 64 / 56, 3,000 tokens 156 / 115, 4,096 219 / 170; 16 over 8, 8,192 813 / 614 (those of 16 rows before their layout in LDS, which
+// takes a tenth off) (0.9 PFLOP/s): one wave a SIMD, whose 66 products of
 // 32 keys take 1,056 of the 2,400 cycles that a tile takes it; 512 registers hold no more columns.  Short ranges
 // of keys are the other kernel's, by the same order of sums (a prompt of 20 tokens 5.9 / 8.9, of 257 13.9 / 15.5: a longer start, and a
 // wave's work one after the other); the line is drawn where launches are shaped.  With the products in a row and the exponentials behind them
