@@ -364,7 +364,7 @@ static bool gemm_tiles_takes(int M, int N, int K) {
 // (the first loads, C); the launch takes as many turns as the tiles need with one workgroup a compute unit.  Tiles of at most 192 x 128
 // leave room for two, which together take 0.95 of two one after the other.  The constants are a fit to 80 products of 160 to 8,192 rows of
 // 768 to 28,672 columns, K of 768 to 14,336, with all fifteen tiles each: what it picks takes 1.2 % longer than the fastest on average.  (Fitted while a value's rounding took ten instructions; what
-stands around a tile has shrunk by some us since, for all tiles alike.)
+// stands around a tile has shrunk by some us since, for all tiles alike.)
 static long tile_cost(int M, int NO, int K, int bm, int bn, int cols) {
   const long tiles = (long)((M + bm - 1) / bm) * ((NO + cols - 1) / cols), steps = K / GT_BK;
   const long one = steps * (62L * bm * bn / 65536 + 56L * (bm + bn) / 512);
