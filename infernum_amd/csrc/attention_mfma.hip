@@ -660,7 +660,7 @@ static void launch_decode_reduce(const float* part_o, const float* part_ml, void
 // 16 + 4 qd .. 16 + 4 qd + 3; the values are laid into LDS in that order of keys, so the probabilities go
 // from registers to registers.
 // EIGHTS: row r of the S^T tile kt stands for the key 8 (r / 4) + r % 4 + 4 kt (the keys' rows are laid into LDS so), and lane (col, qd)
-// has the keys 8 qd .. 8 qd + 7: the order of the kernel of attention_prefill.h, whose sums these then are to the bit.  Where a launch
+// has the keys 8 qd .. 8 qd + 7: the order of the kernel of attention_prefill.h for heads of 128, whose sums these then are to the bit.  Where a launch
 // may go to either, this is the form: which one it goes to (by the width of the step's block tables, say) leaves a request's bits alone.
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 #define PF_KT (IA_MAX_DIM <= 128 ? 64 : 32)   // keys per round of the main loop (one barrier), in parts of 32
@@ -1062,9 +1062,11 @@ __global__ __launch_bounds__(4 * HGW * 64, HGW == 2 && IA_ATTN_EXT == 0 && IA_MA
 
 #if IA_ATTN_EXT == 0 && (IA_HEAD_DIM == 128 || IA_HEAD_DIM == 256) && IA_VALUE_DIM == IA_HEAD_DIM
 #define IA_PREFILL_WIDE 1
+#define IA_PREFILL_EIGHTS (IA_HEAD_DIM == 128)
 #include "attention_prefill.h"
 #else
 #define IA_PREFILL_WIDE 0
+#define IA_PREFILL_EIGHTS 0
 #endif
 
 // ------------------------------------------------------------------ C interface
@@ -1250,10 +1252,10 @@ extern "C" int ia_attn_prefill(const void* q, int q_row_stride, const void* k_pa
   if (xrc != IA_OK) return xrc;
   dim3 grid(num_tiles, nkv * HC);
   // where a wave may take 32 rows (attention_prefill.h): by the model's heads and the pages' size alone, so that all of a request's
-  // launches sum in one order; which of the two kernels a launch goes to is free then
-  const bool eights = IA_PREFILL_WIDE && G >= 2 && (ps & (ps - 1)) == 0 && ps >= 8;
+  // launches sum in one order (that of heads of 128 is another one there); which of the two kernels a launch goes to is free then
+  const bool wide = IA_PREFILL_WIDE && G >= 2 && (ps & (ps - 1)) == 0 && ps >= 8;
 #if IA_PREFILL_WIDE
-  if (eights && bt_stride <= PW_BT && !(launch_shape & IA_PREFILL_NARROW)) {
+  if (wide && bt_stride <= PW_BT && !(launch_shape & IA_PREFILL_NARROW)) {
 #define PW_LAUNCH(W)                                                                                                          \
   return (window != 0 ? launch_prefill_wide<W, true> : launch_prefill_wide<W, false>)(                                        \
       grid, q, q_row_stride, k_pages, v_pages, out, out_row_stride, seq_starts, seq_ctx, block_tables, bt_stride, tiles, nh, nkv, \
@@ -1273,7 +1275,7 @@ extern "C" int ia_attn_prefill(const void* q, int q_row_stride, const void* k_pa
       paired, sinks, X)
 #define PF_LAUNCH(C, W)                      \
   do {                                       \
-    if (eights) PF_LAUNCH_P(C, W, true, IA_PREFILL_WIDE != 0); \
+    if (wide) PF_LAUNCH_P(C, W, true, IA_PREFILL_EIGHTS != 0); \
     else if ((ps & (ps - 1)) == 0) PF_LAUNCH_P(C, W, true); \
     else PF_LAUNCH_P(C, W, false);           \
   } while (0)

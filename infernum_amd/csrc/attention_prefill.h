@@ -8,9 +8,11 @@
 // four stages fill LDS so.)
 //   S^T[key, col] = K[key, :] . Q[col, :]       v_mfma_f32_16x16x32_bf16 over 32 head dims a step
 //   O^T[dim, col] += V^T[dim, key] P^T[key, col] the same over 32 keys a step
-// Row r of the S^T tile t (of a half's two) stands for the key 8 (r / 4) + r % 4 + 4 t of the half, so that the accumulators leave
+// Heads of 128: row r of the S^T tile t (of a half's two) stands for the key 8 (r / 4) + r % 4 + 4 t of the half, so that the accumulators leave
 // lane (col, q) with the keys 8 q .. 8 q + 7: what the second product wants of the probabilities, and 16 contiguous bytes of a row
-// of V^T, as pages hold it.
+// of V^T, as pages hold it.  Heads of 256 keep the order of the kernel with 16 rows a wave, row r of tile t the key 16 t + r: a lane has the keys
+// 4 q .. 4 q + 3 and 16 + 4 q .. 16 + 4 q + 3, two reads of 8 bytes of V^T (3,000 tokens of 16 heads over 1 120 us, 116 in the order of
+// heads of 128, which is another sum of the same numbers).
 //
 // What bounds it: with four heads a workgroup a SIMD has two such waves (LDS holds one workgroup a compute unit: one wave a SIMD with two
 // heads, every other SIMD has none with one), whose matrix instructions take 2,176 cycles a tile, their exponentials and what goes with them
@@ -21,9 +23,9 @@
 // 8B shape's heads (32 over 8), waves of 16 rows / this kernel, us: 2,048 tokens 63 / 52, 4,096
 // 164 / 134, 8,192 600 / 485 (1.13 PFLOP/s), 2,048 after 6,144 cached 271 / 217; under a window of 4,096 8,192 tokens 465 / 388.  (Every read
 // waited for and keys where only 8 lanes found different places: 54, 141, 515, 227, 407.)  Heads of 256, 16 over 1: 2,047 tokens under a
-// window of 1,024 64 / 56, 3,000 tokens 156 / 115, 4,096 219 / 170; 16 over 8, 8,192 813 / 614 (those of 16 rows before their layout in LDS, which
-// takes a tenth off) (0.9 PFLOP/s): one wave a SIMD, whose 66 products of
-// 32 keys take 1,056 of the 2,400 cycles that a tile takes it; 512 registers hold no more columns.  Short ranges
+// window of 1,024 60.5 / 57, 3,000 tokens 145 / 120, 4,096 198 / 178; 16 over 8, 8,192 732 / 645 (0.85 PFLOP/s): one wave a SIMD, whose
+// 66 products of
+// 32 keys take 1,056 of the 2,500 cycles that a tile takes it; 512 registers hold no more columns.  Short ranges
 // of keys are the other kernel's, by the same order of sums (a prompt of 20 tokens 5.9 / 8.9, of 257 13.9 / 15.5: a longer start, and a
 // wave's work one after the other); the line is drawn where launches are shaped.  With the products in a row and the exponentials behind them
 // 8,192 tokens took 590 where this took 508; with tests for a wave's first and last half inside the loop 587; with a mask in every half of a
@@ -31,7 +33,8 @@
 // Heads of 64 gained nothing (2,048 tokens 48 / 54, 8,192 438 / 418), one query head to a key/value head lost (2,000 tokens of 8 heads 53 / 67).
 //
 // In LDS the 16-byte piece c of row r (a key's values; a dim's keys) lies at position c ^ s(r), s(key) = key % 4 + 4 (key / 8 % 4),
-// s(dim) = dim % 8 (of 32 keys dim / 2 % 4): the 16 lanes that read together find 16 different places.
+// s(dim) = dim % 8, for heads of 256 s(key) = key % 16, s(dim) = dim / 4 % 4: the 16 lanes that read 16 bytes together find 16 different places,
+// the 32 that read 8 bytes together 32.
 #pragma once
 
 #define PW_KT (HD <= 128 ? 64 : 32)      // keys a tile
@@ -39,6 +42,7 @@
 #define PW_INLINE __attribute__((always_inline))
 #define PW_BT 4096                      // block-table entries kept in LDS
 
+constexpr bool PW_EIGHTS = IA_PREFILL_EIGHTS;                 // the order of keys in a half, see above
 constexpr int PW_HALVES = PW_KT / 32, PW_VP = PW_KT / 8;      // 32 keys each; pieces of a dim's row of V^T
 constexpr int PW_K_BYTES = PW_KT * HD * 2, PW_V_BYTES = VD * PW_KT * 2;
 constexpr int PW_LDS = PW_STAGES * (PW_K_BYTES + PW_V_BYTES) + PW_BT * 4;
@@ -146,10 +150,11 @@ __global__ __launch_bounds__(HGW * 128, HD <= 128 ? 2 : 1) void attn_prefill_wid
   const char* const k_base = reinterpret_cast<const char*>(k_pages) + (size_t)g * ps * (HD * 2);
   const char* const v_base = reinterpret_cast<const char*>(v_pages) + (size_t)g * VD * (ps * 2);
   const int k_row = lane / (HD / 8);
-  // s(key) of the rows of a load: bits 2 and 3 are the group's number's lowest
+  // s(key) of the rows of a load: bits 2 and 3 are the group's number's lowest (heads of 256: bits 1 and 2 the load's of the group, bit 3 the
+  // group's number's lowest)
   const uint32_t k_lane_at = (uint32_t)(k_row * HD * 2 + (((lane & (HD / 8 - 1)) ^ (k_row & 3)) * 16));
   constexpr int VDIMS = 64 / PW_VP;
-  auto v_swizzle = [&](int dim) PW_INLINE { return PW_KT == 64 ? dim & 7 : (dim >> 1) & 3; };
+  auto v_swizzle = [&](int dim) PW_INLINE { return PW_KT == 64 ? dim & 7 : (dim >> 2) & 3; };
   const int v_key = 8 * ((lane & (PW_VP - 1)) ^ v_swizzle(lane / PW_VP));
   const uint32_t v_lane_at = (uint32_t)(VDIMS * wave * VF + lane / PW_VP) * (uint32_t)(ps * 2), v_step = (uint32_t)(2 * VDIMS * ps);
   const int last_page = (key_hi >> ps_shift) - bt_first;
@@ -167,20 +172,19 @@ __global__ __launch_bounds__(HGW * 128, HD <= 128 ? 2 : 1) void attn_prefill_wid
       const bool ok = (unsigned)k_pg[f] < (unsigned)num_pages;
       bad |= !ok;
       const uint32_t in_page = (uint32_t)((t * PW_KT + 8 * (wave * KG + f)) & (ps - 1)) * (HD * 2);
-      const uint32_t at = k_lane_at ^ (((wave * KG + f) & 3) * 64u);
+      const uint32_t at = k_lane_at ^ (PW_EIGHTS ? ((wave * KG + f) & 3) * 64u : ((wave * KG + f) & 1) * 128u);
       const char* const page = k_base + (uint64_t)(uint32_t)(ok ? k_pg[f] : 0) * k_page;
       const char* src = page + (in_page + at);
       // a group's loads follow each other in the page and in LDS alike: the instruction's offset moves both
       const uint32_t dst = k_first + slot * PW_K_BYTES + 1024 * KL * (wave * KG + f);
       ia_load_to_lds<0>(src, dst);
       if constexpr (KL == 2) ia_load_to_lds<1024>(src, dst);
-      if constexpr (KL == 4) {                    // two keys a load: every other one's begin with key % 4 = 2
-        const char* const other = page + (in_page + (at ^ 32u));
-        ia_load_to_lds<1024>(other, dst);
-        ia_load_to_lds<2048>(src, dst);
-        ia_load_to_lds<3072>(other, dst);
+      if constexpr (KL == 4) {                    // two keys a load, of the group's eight
+        ia_load_to_lds<1024>(page + (in_page + (at ^ 32u)), dst);
+        ia_load_to_lds<2048>(page + (in_page + (at ^ 64u)), dst);
+        ia_load_to_lds<3072>(page + (in_page + (at ^ 96u)), dst);
       }
-      static_assert(KL == 1 || KL == 2 || (KL == 4 && HD == 256), "a group's loads");
+      static_assert(PW_EIGHTS ? (HD == 128 && KL <= 2) : (HD == 256 && KL == 4), "a group's loads");
     }
   };
   auto load_v = [&](int t, int slot) PW_INLINE {
@@ -193,16 +197,26 @@ __global__ __launch_bounds__(HGW * 128, HD <= 128 ? 2 : 1) void attn_prefill_wid
   };
 
   // ---- reads: this lane's row and pieces
-  const int k_lane = (8 * (j >> 2) + (j & 3)) * (HD * 2), v_lane = j * (PW_KT * 2);
-  const int v_piece0 = (qd ^ v_swizzle(j)) * 16, v_piece1 = ((4 + qd) ^ v_swizzle(j)) * 16;      // (of 32 keys the first alone)
+  const int k_lane = (PW_EIGHTS ? 8 * (j >> 2) + (j & 3) : j) * (HD * 2), v_lane = j * (PW_KT * 2);
+  const int v_piece0 = PW_EIGHTS ? (qd ^ v_swizzle(j)) * 16 : ((qd >> 1) ^ v_swizzle(j)) * 16 + (qd & 1) * 8;
+  const int v_piece1 = ((4 + qd) ^ v_swizzle(j)) * 16;                  // (of 64 keys alone)
+  const int v_other = (v_piece0 & 32) ? -32 : 32;                       // from the lane's keys of the first 16 to those of the others
   int k_piece[4];
 #pragma unroll
   for (int s = 0; s < 4; ++s) k_piece[s] = k_lane + ((4 * s + qd) ^ j) * 16;
   auto read_k = [&](const char* half, int t, int st) PW_INLINE {        // tile t of the half's two, step st of the head dims
-    return *reinterpret_cast<const bf16x8_t*>(half + k_piece[st & 3] + t * (4 * HD * 2) + (st >> 2) * 256);
+    return *reinterpret_cast<const bf16x8_t*>(half + k_piece[st & 3] + t * ((PW_EIGHTS ? 4 : 16) * HD * 2) + (st >> 2) * 256);
   };
   // `values`: the stage of the half's tile, with this lane's place in it
-  auto read_v = [&](const char* values, int n) PW_INLINE { return *reinterpret_cast<const bf16x8_t*>(values + n * (16 * PW_KT * 2)); };
+  auto read_v = [&](const char* values, int n) PW_INLINE {
+    if constexpr (PW_EIGHTS) {
+      return *reinterpret_cast<const bf16x8_t*>(values + n * (16 * PW_KT * 2));
+    } else {
+      const uint2 a = *reinterpret_cast<const uint2*>(values + n * (16 * PW_KT * 2));
+      const uint2 b = *reinterpret_cast<const uint2*>(values + v_other + n * (16 * PW_KT * 2));
+      return __builtin_bit_cast(bf16x8_t, make_uint4(a.x, a.y, b.x, b.y));
+    }
+  };
 
   typedef uint32_t packed[2][4];        // probabilities as B operands: [column][pairs of keys]
   float emax[2];
@@ -222,7 +236,7 @@ __global__ __launch_bounds__(HGW * 128, HD <= 128 ? 2 : 1) void attn_prefill_wid
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int key = t0 + 8 * qd + 4 * t + r;
+          const int key = t0 + (PW_EIGHTS ? 8 * qd + 4 * t : 16 * t + 4 * qd) + r;
           s[t][c][r] = (key <= last && key >= first) ? s[t][c][r] : -INFINITY;
         }
     }

@@ -1202,11 +1202,11 @@ def prefill_launch_shape(nh: int, nkv: int, d: int, q_lens: Sequence[int], ctx_l
 # A wave of 32 rows that two chunks share walks both, which all others wait for (4,096 tokens of 16 heads over 8 in chunks of 1,024 from a chunk's
 # start on 58.8 / 53.4, from 16 tokens on 60.7 / 76.5): where a request's rows do not begin on a multiple of 32 and chunks are no longer than
 # PREFILL_NARROW_CHUNK, 16 rows (183 launches under chunks: 1.3 % longer than the faster, at most 5 % longer than 16 rows).
-# Heads of 256 (two a workgroup): one prompt of 257 tokens 19.5 / 21.1, of 512 28.5 / 29.0, of 600 34.5 / 32.3; 12 of 416 56.3 / 58.8, of 512
-# 72.8 / 70.3; 20 of 130 53 / 58; a portion of 30 rows under a window of 512 31.4 / 32.5; 4,080 rows from 16 tokens on under
-# chunks of 1,024 101 / 116.
+# Heads of 256 (two a workgroup): one prompt of 257 tokens 19.4 / 21.4, of 512 27.7 / 29.4, of 600 33.6 / 32.9; 12 of 416 54.9 / 59.5, of 512
+# 69.5 / 71.0, 8 of 600 37.8 / 37.5; 20 of 130 51 / 58; under a window of 512 30 rows 30.7 / 33.2, 2,048 36.5 / 39.2, of 1,024 2,047
+# 60.5 / 57.1; 4,080 rows from 16 tokens on under chunks of 1,024 95 / 118.
 PREFILL_NARROW_KEYS = (600, 448)
-PREFILL_NARROW_KEYS_256 = 512
+PREFILL_NARROW_KEYS_256 = 600
 PREFILL_NARROW_CHUNK = 2048
 
 

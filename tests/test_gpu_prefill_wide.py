@@ -263,6 +263,18 @@ def test_heads_of_256_at_the_edges_of_tiles(nh, nkv, ps, lens, q_lens, window):
     assert torch.equal(bad[bad.shape[0] - q_lens[-1]:][clean], first[first.shape[0] - q_lens[-1]:][clean]) and not bool(bad[-1].isfinite().any())
 
 
+@pytest.mark.parametrize("nh,nkv,ps", [(4, 1, 16), (6, 2, 8)])
+@pytest.mark.parametrize("lens,q_lens", [([1, 31, 33, 64, 129], [1, 31, 33, 64, 129]), ([300, 449], [300, 100])])
+@pytest.mark.parametrize("window", [0, 40, -96])
+def test_heads_of_256_sum_in_the_order_of_a_head_alone(nh, nkv, ps, lens, q_lens, window):
+    """Heads that share keys, in either kernel, leave the bits that each leaves with keys of its own (a launch that has one kernel alone)."""
+    c = _case(nh, nkv, ps, lens, q_lens, seed=nh * ps + len(lens) + window, D=256)
+    own = dict(c, kp=c["kp"].repeat_interleave(nh // nkv, dim=1).contiguous(), vp=c["vp"].repeat_interleave(nh // nkv, dim=1).contiguous())
+    want = _run(own, nh, nh, window)
+    for shape in (1, 2, K().PREFILL_NARROW | 1, K().PREFILL_NARROW | 2):
+        assert torch.equal(_run(c, nh, nkv, window, heads_per_workgroup=shape), want), shape
+
+
 def test_short_ranges_of_heads_of_256_go_to_waves_of_16_rows():
     api, dev = K(), torch.device(DEV)
     narrow = lambda q, c, nh=16, nkv=1, w=0: bool(api.prefill_shape(nh, nkv, 256, q, c, w, dev) & api.PREFILL_NARROW)    # noqa: E731
