@@ -230,6 +230,7 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_mfma_kernel(const
     buf = next_buf;
     fill_buf = (fill_buf + 1 == STAGES) ? 0 : fill_buf + 1;
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // the loads asked for past the end write LDS too, whichever way C leaves
 
   // ---- C.  A whole tile with rows of N that 16-byte stores can take goes through LDS, so that a row of the
   // wave's part leaves as consecutive 16-byte pieces (the accumulators hold 4 values of a row per lane, 32
@@ -238,7 +239,6 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_mfma_kernel(const
   if constexpr (SPLIT) {
     // the sums of this part of K, fp32, into part `part` of P [splits, M, N]: whoever reads them adds the parts in
     // the order of their index
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the loads asked for past the end write LDS too
     float* const pp = P + (size_t)part * M * N;
     const bool vec4 = (N & 3) == 0;
 #pragma unroll
@@ -301,7 +301,6 @@ __global__ __launch_bounds__(WAVES_M * WAVES_N * 64) void gemm_mfma_kernel(const
   constexpr int CP = WN / 8;                        // 16-byte pieces per row of a wave's part
   static_assert(STAGES * STAGE_BYTES >= WAVES * WM * WN * 2, "the stages must hold the tile of C");
   if (m0 + BM <= M && n0 + BN <= N && (N & 7) == 0) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // the loads asked for past the end write LDS too
     __syncthreads();
     char* region = lds + wave * (WM * WN * 2);
 #pragma unroll
