@@ -230,9 +230,15 @@ __device__ __forceinline__ int ia_expert_first_chunk(int column, int K) {
 // Every lane's 16 bytes at src + AT, straight into LDS from lds + AT on, lane after lane (lds the same for the wave).  Written out: the
 // compiler takes the builtin for an access of memory and of LDS at once, and with one under way it waits for all reads of LDS, the newest
 // too, where it needs the oldest (prompt attention with heads of 128, two reads in flight over every product: 8,192 tokens of 32
-// heads 515 us with the builtin, 504 so; heads of 256, 8,192 tokens of 16 heads 655 / 614).  Nothing comes back in a register, and nobody
-// but the caller waits: for vmcnt before a barrier, before LDS is read and before the workgroup ends.  (One instruction has to
-// lie between the write of m0 and the load.)
+// heads 515 us with the builtin, 504 so).  Nothing comes back in a register, and nobody
+// but the caller waits: for vmcnt before a barrier, before LDS is read and before the workgroup ends.
+// Two things the caller sees to, as the compiler does not look inside.  m0 is its own (it warns that m0 is not kept over such a statement): the
+// builtin, or whatever else wants m0, does not go into one kernel with these.  And where src is the same for the wave it comes from scalar
+// instructions: behind a vector instruction that writes it (v_readfirstlane) a load needs five instructions' distance, and has two here
+// (the one that has to lie between the write of m0 and the load, and that write).  The distance in every load costs split products of few
+// rows up to a seventh: 328 rows of 84 x 11,712 41.2 / 46.8 us, 278 of 612 x 8,448 in 2 17.8 / 19.7.  A test reads both from the assembly.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 template <int AT>
 __device__ __forceinline__ void ia_load_to_lds(const char* src, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off offset:%2" ::"s"(lds), "v"(src), "n"(AT) : "memory", "m0");
@@ -241,6 +247,7 @@ __device__ __forceinline__ void ia_load_to_lds(const char* src, uint32_t lds) {
 __device__ __forceinline__ void ia_load_to_lds(const char* src, uint32_t at, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(at), "s"(src) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 __device__ __forceinline__ uint32_t ia_lds_address(const char* p) {
   return (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)p);
 }

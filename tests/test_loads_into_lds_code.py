@@ -79,3 +79,51 @@ def test_no_load_is_under_way_where_a_kernel_ends(kernels):
                     under_way[to] = state
                     work.append(to)
         assert ends, name
+
+
+def test_nothing_else_of_such_a_kernel_uses_m0(kernels):
+    for name, body in kernels.items():
+        written_out = False
+        for line in body.split("\n"):
+            if "#ASMSTART" in line or "#ASMEND" in line:
+                written_out = "#ASMSTART" in line
+            code = line.split(";")[0]
+            assert written_out or not re.search(r"\bm0\b|_lds_dword|movrel|gpr_idx|sendmsg|ds_gws", code), (name, line)
+
+
+def _scalars(text):
+    """s7 or s[8:9] -> the registers' numbers."""
+    one, span = re.fullmatch(r"s(\d+)", text), re.fullmatch(r"s\[(\d+):(\d+)\]", text)
+    return {int(one.group(1))} if one else set(range(int(span.group(1)), int(span.group(2)) + 1)) if span else set()
+
+
+def test_a_scalar_address_does_not_come_from_a_vector_instruction_just_before(kernels):
+    """Five wait states between a vector instruction's write of a scalar register and a load that takes its address from it."""
+    for name, body in kernels.items():
+        blocks = _blocks(body)
+        before = {label: [] for label in blocks}
+        for label, (_, after) in blocks.items():
+            for at, to in after:
+                before[to].append((label, at))
+
+        def look(label, at, distance, wanted, seen):
+            code = blocks[label][0]
+            for line in reversed(code[:at]):
+                if distance >= 5:
+                    return
+                op, _, args = line.partition(" ")
+                if op.startswith("v_") and _scalars(args.split(",")[0].strip()) & wanted:
+                    raise AssertionError((name, label, line, wanted, distance))
+                nop = re.fullmatch(r"s_nop (\d+)", line)
+                distance += int(nop.group(1)) + 1 if nop else 1
+            for other, end in before[label]:
+                if distance < 5 and (other, distance) not in seen:
+                    seen.add((other, distance))
+                    look(other, end, distance, wanted, seen)
+
+        for label, (code, _) in blocks.items():
+            for at, line in enumerate(code):
+                if line.startswith("global_load_lds"):
+                    base = line.split(",")[1].split()[0]
+                    if base != "off":
+                        look(label, at, 0, _scalars(base), set())
