@@ -101,7 +101,8 @@ __global__ __launch_bounds__(256) void gemm_heads_kernel(const T* __restrict__ x
 }
 
 // The same on tiles of BM x 128 (tile_mfma_big): grid (tiles of 128 of Nout, tiles of BM of N, H).  With 2,048 rows
-// tiles of 32 rows took 18 and 26 us where tiles of 128 took 30 and 28 (heads of 224 x 64 and 64 x 224).
+// tiles of 32 rows take 185 us where tiles of 128 take 248 (128 heads of 224 x 512); of 48 products of K from 320 to 2,048 with 17 to 4,000
+// rows tiles of 128 gain with the longest K and thousands of rows of many heads alone (200 rows of 128 heads of 128 x 2,048 88 / 44).
 template <int BM>
 __global__ __launch_bounds__(256) void gemm_heads_big_kernel(const bf16_t* __restrict__ x, int x_row, int x_head,
                                                              const bf16_t* __restrict__ W, bf16_t* __restrict__ out,
@@ -130,20 +131,16 @@ __global__ __launch_bounds__(256) void gemm_heads_big_kernel(const bf16_t* __res
       });
 }
 
-// The same for few rows (decoding), without LDS: bound by one trip to memory.  A wave takes 16 columns of one head for up to
-// 16 rows of x and asks for eight steps of 32 values of K of both at once, none under a condition (pieces beyond K are read
+// The same for few rows (decoding) and K beyond a head's size, without LDS: bound by one trip to memory.  A wave takes 16 columns of one head for
+// up to 16 rows of x and asks for eight steps of 32 values of K of both at once, none under a condition (pieces beyond K are read
 // from the last place and cleared); the sums are those of the tiles above, step by step in the same order.  Grid (tiles of
-// 64 of Nout, 1, H).  One row, 16 heads: 224 x 64 3.9 us with the tiles and 2.4 so, 64 x 224 with
-// a gate 6.7 and 4.4, 128 x 512 with a gate 9.8 and 7.5; 16 rows 3.9 and 2.6, 6.8 and 4.0, 8.7 and 7.8.
-#define GH_FEW_ROWS 16
+// 64 of Nout, 1, H).
 // The reads of x, once for every 16 columns of W, make it lose with long rows and many workgroups.  Its time over that of the
-// tiles at 1 / 8 / 16 rows, by K and workgroups: 64 and up to 512 0.67 to 0.85; 128 x 512 0.81 / 0.85 / 0.92, 128 x 1,024 0.87 /
-// 0.95 / 1.04; 192 x 1,024 1.00 / 1.08 / 1.18; 256 x 512 0.95 / 1.02 / 1.09; 512 x 128 0.89 / 0.97 / 1.04, 512 x 256 (16 heads of
+// tiles at 1 / 8 / 16 rows, by K and workgroups: 512 x 128 0.89 / 0.97 / 1.04, 512 x 256 (16 heads of
 // 1,024) 1.03 / 1.13 / 1.16; 1,024 x 64 0.98 / 1.07 / 1.14, x 128 1.16 / 1.33 / 1.39.
+#define GH_FEW_ROWS 16
 static bool heads_few_pays(int N, int H, int Nout, int K) {
-  const long work = (long)K * H * ((Nout + 63) / 64);
-  if (K > 256) return N <= GH_FEW_ROWS && work <= (K <= 512 && N <= 8 ? 65536 : 16384);
-  return N <= GH_FEW_ROWS && work <= (N <= 4 ? 131072 : N <= 8 ? 98304 : 65536);
+  return N <= GH_FEW_ROWS && (long)K * H * ((Nout + 63) / 64) <= (K <= 512 && N <= 8 ? 65536 : 16384);
 }
 
 __global__ __launch_bounds__(256) void gemm_heads_few_kernel(const bf16_t* __restrict__ x, int x_row, int x_head,
@@ -191,22 +188,20 @@ __global__ __launch_bounds__(256) void gemm_heads_few_kernel(const bf16_t* __res
   }
 }
 
-// The same for many rows of short K (a head's size), without LDS: a wave keeps 16 rows of x in registers and walks over its columns of the
+// The same for short K (a head's size), without LDS: a wave keeps 16 rows of x in registers and walks over its columns of the
 // head, 16 at a time, the next ones' rows of W under way (they come from the caches: a head's matrix is some tens of KB, read by every wave).
 // Bound by the reads of x and the writes of out; in tiles through LDS a step of K of 64 is a trip to memory and two barriers for 32 rows, and values
-// left one by one.  The same sums in the same order.  us, in tiles / so (at 6 TB/s): 2,047 rows of 16 heads of 224 x 64 23.8 / 9.6 (3.1), of
-// 64 x 224 with a gate 15.5 / 10.8 (3.8); 4,096 rows of 32 heads 83 / 26 (12.5) and 50 / 29 (15.2); 200 rows of 16 heads 5.4 / 3.4 and 9.3 / 3.7.
-// A wave's 32 rows share the reads of W: with short K, with a large matrix a head (1,000 rows of 128 heads of 512 x 128, 16 / 32 rows a wave 126 /
-// 75) and where 16 rows a wave fill the chip more than once (4,096 rows of 32 heads of 64 x 224 35 / 29; 2,047 of 16 10.8 / 11.6).
+// left one by one.  The same sums in the same order.  us, in tiles / so (at 6 TB/s): 2,000 rows of 16 heads of 224 x 64 23.8 / 9.9 (3.0), of
+// 64 x 224 with a gate 15.9 / 9.5 (3.7), of 32 heads of 224 x 64 43.0 / 16.7 (6.1).
+// A wave may take 32 rows, which share the reads of W; a workgroup's one, two or four waves stand over the rows, so that none is without any.
 #define GH_ROWS_K 256
-#define GH_ROWS_WORKGROUPS 512
 template <int KP, int MT>                                // steps of 32 of K, at most; groups of 16 rows a wave
 __global__ __launch_bounds__(256) void gemm_heads_rows_kernel(const bf16_t* __restrict__ x, int x_row, int x_head,
                                                               const bf16_t* __restrict__ W, bf16_t* __restrict__ out, int o_row,
                                                               int o_head, const bf16_t* __restrict__ gate, int g_row, int N, int Nout,
                                                               int K, int tiles, bool fours) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, q = lane >> 4;
-  const int h = blockIdx.z, m0 = (blockIdx.y * 4 + wave) * (16 * MT);
+  const int h = blockIdx.z, m0 = (blockIdx.y * (blockDim.x >> 6) + wave) * (16 * MT);
   if (m0 >= N) return;
   const int first = blockIdx.x * tiles, last = min(first + tiles, (Nout + 15) / 16);
   int row[MT];
@@ -298,6 +293,44 @@ __global__ __launch_bounds__(256) void gemm_heads_rows_kernel(const bf16_t* __re
   if (t < last) work(t, w0, g0);
 }
 
+// How a launch of the kernel above deals out N rows and `tiles` groups of 16 columns of H heads.
+struct HeadsShape {
+  int wide, waves, rows, per;            // groups of 16 rows a wave; waves a workgroup; workgroups over the rows; groups of columns a wave
+};
+
+// The shape with the least estimated time: the trips of a wave's walk one after the other, and what all waves of the compute unit that has the
+// most of them move: their rows of x, and for every group of columns the rows of W and the result (and gate).  The numbers are a fit to
+// 763 products of 1 to 2,047 rows of 1 to 128 heads, Nout of 16 to 1,024, K of 16 to 256, each with up to 40 shapes: what it picks takes 3 %
+// longer than the fastest on average.  us, in tiles / by some 2,048 waves in workgroups of four over the rows / so: 16 rows of 128 heads of
+// 512 x 128 with a gate 7.6 / 9.5 / 5.7, 333 rows of 4 heads of 1,024 x 256 8.7 / 11.2 / 6.7, 100 rows of 16 9.0 / 10.8 / 7.5, 600 rows of 32 heads of
+// 64 x 224 9.1 / 9.8 / 6.0.  Few rows too: 1 / 2 / 16 rows of 16 heads of 64 x 224 take 3.4 / 4.7 / 3.7 in the kernel for few rows above (two
+// with a gate) and 2.5 / 2.7 / 2.6 so.  Of 1,578 products of 1 to 2,000 rows none takes more than 1.06 of its time in tiles or in that kernel,
+// 0.67 in the mean.
+static HeadsShape heads_shape(int N, int H, int tiles, int K, bool gate) {
+  HeadsShape best{0, 0, 0, 0};
+  long least = 0;
+  const int kp = K <= 64 ? 2 : K <= 128 ? 4 : 8;
+  for (int wide = 1; wide <= (N > 16 ? 2 : 1); ++wide) {
+    const int blocks = (N + 16 * wide - 1) / (16 * wide);
+    for (int waves = 1; waves <= 4 && (waves == 1 || waves < 2 * blocks); waves *= 2) {
+      const int rows = (blocks + waves - 1) / waves;
+      for (int pieces = 1, last = 0; pieces <= tiles && last != 1; ++pieces) {       // of as equal a length as can be
+        const int per = (tiles + pieces - 1) / pieces;
+        if (per == last) continue;
+        last = per;
+        const long workgroups = (long)((tiles + per - 1) / per) * rows * H;
+        const long unit = (workgroups + 255) / 256 * (waves < blocks ? waves : blocks);
+        const long cost = 32 * per + unit * (4 * wide * kp + per * (2 * kp + wide * (gate ? 2 : 1)));
+        if (least == 0 || cost < least) {
+          least = cost;
+          best = HeadsShape{wide, waves, rows, per};
+        }
+      }
+    }
+  }
+  return best;
+}
+
 extern "C" int ia_gemm_heads(const void* x, int x_row, int x_head, const void* W, void* out, int o_row, int o_head,
                              const void* gate, int g_row, int dtype, int N, int H, int Nout, int K,
                              hipStream_t stream) {
@@ -312,6 +345,29 @@ extern "C" int ia_gemm_heads(const void* x, int x_row, int x_head, const void* W
                                                               (float*)out, o_row, o_head, (const float*)gate, g_row,
                                                               N, Nout, K);
   else if (dtype == IA_BF16 && (K & 7) == 0 && tile_rows_aligned(x, x_row, x_head) && tile_rows_aligned(W, K)) {
+    if (K <= GH_ROWS_K) {
+      const int tiles = (Nout + 15) / 16;
+      const HeadsShape shape = heads_shape(N, H, tiles, K, gate != nullptr);
+      if (shape.rows > 65535) return IA_ERR_UNSUPPORTED;
+      const bool fours = ((Nout | o_row | o_head) & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0 &&
+                         (!gate || ((g_row & 3) == 0 && (reinterpret_cast<uintptr_t>(gate) & 7) == 0));
+      const dim3 pieces((tiles + shape.per - 1) / shape.per, shape.rows, H);
+#define GH_ROWS(KP, MT)                                                                                                              \
+  gemm_heads_rows_kernel<KP, MT><<<pieces, 64 * shape.waves, 0, stream>>>((const bf16_t*)x, x_row, x_head, (const bf16_t*)W, (bf16_t*)out, \
+                                                                          o_row, o_head, (const bf16_t*)gate, g_row, N, Nout, K, shape.per, fours)
+#define GH_ROWS_BY(MT)               \
+  do {                               \
+    if (K <= 64) GH_ROWS(2, MT);     \
+    else if (K <= 128) GH_ROWS(4, MT); \
+    else GH_ROWS(8, MT);             \
+  } while (0)
+      if (shape.wide == 2) GH_ROWS_BY(2);
+      else GH_ROWS_BY(1);
+#undef GH_ROWS_BY
+#undef GH_ROWS
+      IA_LAUNCH_CHECK();
+      return IA_OK;
+    }
     if (heads_few_pays(N, H, Nout, K)) {
       gemm_heads_few_kernel<<<dim3((Nout + 63) / 64, 1, H), 256, 0, stream>>>((const bf16_t*)x, x_row, x_head, (const bf16_t*)W,
                                                                               (bf16_t*)out, o_row, o_head, (const bf16_t*)gate,
@@ -319,33 +375,7 @@ extern "C" int ia_gemm_heads(const void* x, int x_row, int x_head, const void* W
       IA_LAUNCH_CHECK();
       return IA_OK;
     }
-    if (K <= GH_ROWS_K) {
-      const int wide = K <= 64 || (long)Nout * K >= 32768 || (long)((N + 15) / 16) * H >= 4096 ? 2 : 1;
-      const int rows = (N + 64 * wide - 1) / (64 * wide), tiles = (Nout + 15) / 16;
-      if (rows > 65535) return IA_ERR_UNSUPPORTED;
-      // columns in so many pieces that the workgroups fill the chip
-      const long groups = (GH_ROWS_WORKGROUPS + (long)rows * H - 1) / ((long)rows * H);
-      const int per = groups >= tiles ? 1 : (int)((tiles + groups - 1) / groups);
-      const bool fours = ((Nout | o_row | o_head) & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0 &&
-                         (!gate || ((g_row & 3) == 0 && (reinterpret_cast<uintptr_t>(gate) & 7) == 0));
-      const dim3 pieces((tiles + per - 1) / per, rows, H);
-#define GH_ROWS(KP, MT)                                                                                                              \
-  gemm_heads_rows_kernel<KP, MT><<<pieces, 256, 0, stream>>>((const bf16_t*)x, x_row, x_head, (const bf16_t*)W, (bf16_t*)out, o_row, o_head, \
-                                                             (const bf16_t*)gate, g_row, N, Nout, K, per, fours)
-#define GH_ROWS_BY(MT)               \
-  do {                               \
-    if (K <= 64) GH_ROWS(2, MT);     \
-    else if (K <= 128) GH_ROWS(4, MT); \
-    else GH_ROWS(8, MT);             \
-  } while (0)
-      if (wide == 2) GH_ROWS_BY(2);
-      else GH_ROWS_BY(1);
-#undef GH_ROWS_BY
-#undef GH_ROWS
-      IA_LAUNCH_CHECK();
-      return IA_OK;
-    }
-    const int bm = 32;      // K is short here (a head's size): many small workgroups hide each other's few steps better than few large ones
+    const int bm = 32;      // many small workgroups hide each other's steps better than few large ones
     dim3 big((Nout + TB_N - 1) / TB_N, (N + bm - 1) / bm, H);
     if (big.y > 65535u) return IA_ERR_UNSUPPORTED;
     gemm_heads_big_kernel<32><<<big, 256, 0, stream>>>((const bf16_t*)x, x_row, x_head, (const bf16_t*)W,

@@ -224,6 +224,27 @@ def test_products_head_by_head_of_many_rows(N, H, J, Kd, gated):
         assert (out[:, :lead] == 7.0).all() and (out[:, lead + H * J:] == 7.0).all()
 
 
+# one, two and four waves of a workgroup over the rows, the others over the columns: rows that leave a wave without any, columns that do; one
+# group of 16 columns a wave, some, and all 64
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("N,H,J,Kd", [(1, 16, 64, 224), (16, 3, 1030, 64), (17, 4, 17, 224), (33, 2, 200, 40), (48, 128, 100, 128), (65, 32, 130, 256),
+                                      (80, 64, 1024, 16), (333, 4, 520, 256), (515, 3, 96, 64), (2047, 16, 224, 64)])
+def test_products_head_by_head_however_the_waves_stand(N, H, J, Kd, gated):
+    from infernum_amd.kernels import api as K
+    g = torch.Generator().manual_seed(N + J)
+    x, w = torch.randn(N, H * Kd, generator=g).bfloat16().cuda(), torch.randn(H, J, Kd, generator=g).bfloat16().cuda()
+    gate = torch.randn(N, H * J, generator=g).bfloat16().cuda() if gated else None
+    out = torch.full((N + 1, H * J), 7.0, dtype=torch.bfloat16, device="cuda")
+    K.gemm_heads(x, 0, Kd, w, out[:N], 0, J, gate)
+    x64, w64 = x.double().view(N, H, Kd).transpose(0, 1).contiguous(), w.double().transpose(1, 2).contiguous()
+    want, size = torch.bmm(x64, w64).transpose(0, 1).reshape(N, H * J), torch.bmm(x64.abs(), w64.abs()).transpose(0, 1).reshape(N, H * J)
+    if gated:                            # the product is rounded to bf16 in front of the gate: twice, by at most 2^-8 of itself each time
+        s = torch.sigmoid(gate.double())
+        want, size = want * s, size * s
+    assert ((out[:N].double() - want).abs() <= (2.01 if gated else 1.0) * 2.0 ** -8 * want.abs() + Kd * 2.0 ** -23 * size).all()
+    assert (out[N:] == 7.0).all()
+
+
 @BOTH
 @pytest.mark.parametrize("m,W,T", [
     (NM._mixer(3, 16, 8, 24, 24, 20), 64, 75),                       # head size 32, window inside the prompt
