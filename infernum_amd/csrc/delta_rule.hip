@@ -446,8 +446,13 @@ static void launch_delta_token(const T* proj, int proj_stride, int r_col, int k_
   delta_token_kernel<T, J, CW><<<dim3((unsigned)nh, (unsigned)B, (unsigned)((dim + 16 * CW - 1) / (16 * CW))), 256, 0, stream>>>(   \
       proj, proj_stride, r_col, k_col, v_col, w, a, inv, state, state_stride, out, state_slots, nh, dim)
   const long columns = (long)B * nh * dim;
-  if (J <= 2 && columns >= DT_COLUMNS * 4) IA_DT(4);
-  else if (columns >= DT_COLUMNS * 2) IA_DT(2);
+  if constexpr (J <= 2) {                                // (of longer ones four do not fit beside each other)
+    if (columns >= DT_COLUMNS * 4) {
+      IA_DT(4);
+      return;
+    }
+  }
+  if (columns >= DT_COLUMNS * 2) IA_DT(2);
   else IA_DT(1);
 #undef IA_DT
 }

@@ -419,7 +419,10 @@ def test_delta_rule_at_many_head_sizes(dtype, dim, heads, T):
 # the columns that the kernel of several tokens keeps
 @BOTH
 @pytest.mark.parametrize("dim,heads,requests,off", [(128, 8, 1, 0), (36, 2, 3, 0), (64, 16, 9, 0), (128, 8, 17, 0), (100, 5, 70, 0), (132, 4, 33, 0),
-                                                    (256, 2, 2, 0), (200, 8, 21, 0), (96, 4, 5, 0), (128, 4, 6, 1)])
+                                                    (256, 2, 2, 0), (200, 8, 21, 0), (96, 4, 5, 0), (128, 4, 6, 1),
+                                                    # heads of up to 64 with two and with four columns a lane; a last wave in part beyond the head
+                                                    (64, 16, 17, 0), (64, 16, 33, 0), (36, 16, 29, 0), (36, 16, 58, 0), (44, 16, 47, 0),
+                                                    (100, 16, 21, 0), (256, 16, 9, 0)])
 def test_single_tokens_leave_the_bits_of_the_recurrence(dtype, dim, heads, requests, off):
     from infernum_amd.kernels import api as K
     n = heads * dim
