@@ -437,6 +437,11 @@ extern "C" int ia_gemm_tiles_pays(int M, int N, int K) {
   return places * 100 >= large * (K >= 10240 && large > 256 ? 106 : 120);
 }
 
+// Columns of the result that the first of a product's two launches takes (0: it is one launch).
+extern "C" int ia_gemm_tiles_split(int M, int N, int K, int glu) {
+  return gemm_tiles_takes(M, N, K) && !(glu && (N & 1)) ? choose_tiles(M, N, K, glu != 0).split : 0;
+}
+
 // Columns n_first to n_end - 1 of the result.
 static int gemm_tiles_columns(const uint16_t* x, const uint16_t* w, uint16_t* c, int M, int N, int K, int glu, int rows, int cols,
                               int n_first, int n_end, hipStream_t stream) {

@@ -105,6 +105,7 @@ def test_columns_in_two_launches_leave_the_bits_of_one(M, N, K_, swiglu):
     api = K()
     a, w = _rand(M, K_, seed=21), _rand(N, K_, scale=0.1, seed=22)
     cols = N // 2 if swiglu else N
+    assert 0 < api._core().ia_gemm_tiles_split(M, N, K_, int(swiglu)) < cols
     out = torch.full((M + 1, cols), 7.0, dtype=torch.bfloat16, device=DEV)
     api.gemm_tiles(a, w, out[:M], swiglu=swiglu)
     assert torch.equal(out[:M], api.gemm_tiles(a, w, swiglu=swiglu, tile=(128, 128)))
