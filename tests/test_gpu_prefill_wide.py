@@ -58,7 +58,8 @@ def _want(c, nh, nkv, window):
         q = c["q"][at:at + m].view(m, nh, D).double()
         at += m
         pos, key = torch.arange(n - m, n, device=DEV)[:, None], torch.arange(n, device=DEV)[None, :]
-        seen = (key <= pos) & ((key > pos - window) if window else (key >= 0))
+        first = pos - window + 1 if window > 0 else pos // -window * -window if window < 0 else 0      # < 0: chunks of -window keys
+        seen = (key <= pos) & (key >= first)
         for_heads = lambda t: t.double().repeat_interleave(nh // nkv, dim=1)                         # noqa: E731
         s = torch.einsum("qhd,khd->hqk", q, for_heads(k)) * D ** -0.5
         p = torch.softmax(s.masked_fill(~seen, -math.inf), dim=-1)
@@ -247,8 +248,8 @@ def test_heads_of_256_at_the_edges_of_tiles(nh, nkv, ps, lens, q_lens, window):
     """A tile is one half of 32 keys there: the kernel's other loop, and the same bits from waves of 16 rows."""
     c = _case(nh, nkv, ps, lens, q_lens, seed=nh * ps + len(lens) + window, D=256)
     first = _run(c, nh, nkv, window, heads_per_workgroup=K().PREFILL_NARROW | 2)
-    if window >= 0:                      # as for heads of 128 above
-        assert (first.double() - _want(c, nh, nkv, window)).abs().max().item() <= 2.5e-2
+    want = _want(c, nh, nkv, window)     # as for heads of 128 above: windows, and chunks
+    assert ((first.double() - want).abs() <= (2.5e-2 if window >= 0 else 1.5e-2 + 2.0 ** -8 * want.abs())).all()
     for hpw in (0, 1, 2):
         for paired in (False, True):
             assert torch.equal(_run(c, nh, nkv, window, heads_per_workgroup=hpw, paired=paired), first), (hpw, paired)
@@ -256,11 +257,59 @@ def test_heads_of_256_at_the_edges_of_tiles(nh, nkv, ps, lens, q_lens, window):
         _run(c, nh, nkv, window, heads_per_workgroup=4)
     t, page = lens[-1] - 1, int(c["bt"][-1, (lens[-1] - 1) // ps])              # a value that the rows before its 16 do not meet
     c["vp"][page, :, :, t % ps] = float("inf")
-    bad = _run(c, nh, nkv, window)
-    assert torch.equal(bad, _run(c, nh, nkv, window, heads_per_workgroup=K().PREFILL_NARROW | 2)) or not bool(bad[-1].isfinite().any())
+    bad, other = _run(c, nh, nkv, window), _run(c, nh, nkv, window, heads_per_workgroup=K().PREFILL_NARROW | 2)
+    finite = bad.isfinite()              # the same rows from both kernels (infinite or NaN is up to each), and the same bits elsewhere
+    assert torch.equal(finite, other.isfinite()) and torch.equal(bad[finite], other[finite])
     blocks = -(-q_lens[-1] // 16) - 1
     clean = [r for r in range(blocks * 16) if (lens[-1] - q_lens[-1] + r // 16 * 16 + 15) // 32 < t // 32]
     assert torch.equal(bad[bad.shape[0] - q_lens[-1]:][clean], first[first.shape[0] - q_lens[-1]:][clean]) and not bool(bad[-1].isfinite().any())
+
+
+@pytest.mark.parametrize("ctx,n,window", [(16, 100, 0), (1, 64, 0), (17, 97, 0), (0, 200, 40), (16, 200, 33), (5, 150, 1), (40, 130, 100),
+                                          (0, 200, -48), (30, 170, -128), (0, 257, -16)])
+def test_heads_of_256_and_a_value_that_is_not_finite(ctx, n, window):
+    """It reaches blocks of 16 rows that meet its 32 keys, the same in both kernels, and no other row."""
+    nh, nkv, ps, total = 4, 1, 16, ctx + n
+    c = _case(nh, nkv, ps, [total], [n], seed=9, D=256)
+    want = _run(c, nh, nkv, window)
+    assert bool(want.isfinite().all())
+    for t in sorted({0, 15, 31, 32, 40, 63, 64, 95, 100, ctx, total - 1}):
+        if t >= total:
+            continue
+        page = int(c["bt"][0, t // ps])
+        was = c["vp"][page, :, :, t % ps].clone()
+        c["vp"][page, :, :, t % ps] = float("inf")
+        meets = torch.zeros(n, dtype=torch.bool, device=DEV)
+        for first in range(0, n, 16):
+            lo, hi = _first_visible(ctx + first, window), ctx + min(first + 15, n - 1)
+            meets[first:first + 16] = lo // 32 <= t // 32 <= hi // 32
+        sees = torch.tensor([_first_visible(ctx + r, window) <= t <= ctx + r for r in range(n)], device=DEV)
+        for paired in (False, True):     # (a key behind the last that a workgroup's rows see is nobody's there)
+            got, other = (_run(c, nh, nkv, window, heads_per_workgroup=shape, paired=paired) for shape in (2, K().PREFILL_NARROW | 2))
+            assert torch.equal(got[~meets], want[~meets]) and not bool(got[sees].isfinite().any()), (t, paired)
+            finite = got.isfinite()
+            assert torch.equal(finite, other.isfinite()) and torch.equal(got[finite], other[finite]), (t, paired)
+        c["vp"][page, :, :, t % ps] = was
+
+
+@pytest.mark.parametrize("lens,q_lens", [([1, 2, 31, 32, 33], [1, 2, 31, 32, 33]), ([300, 449], [300, 100])])
+@pytest.mark.parametrize("window", [0, 40])
+def test_heads_of_256_with_sinks(lens, q_lens, window):
+    nh, nkv, ps = 4, 1, 16
+    c = _case(nh, nkv, ps, lens, q_lens, seed=23, D=256)
+    sinks = torch.linspace(-3.0, 6.0, nh, device=DEV)
+    first = _run(c, nh, nkv, window, sinks=sinks)
+    rows, at = [], 0                     # a sink leaves of a row what the keys' part of its denominator is
+    for k, n, m in zip(c["k"], c["lens"], c["q_lens"]):
+        q = c["q"][at:at + m].view(m, nh, 256).transpose(0, 1).double()
+        at += m
+        pos, key = torch.arange(n - m, n, device=DEV)[:, None], torch.arange(n, device=DEV)[None, :]
+        s = torch.matmul(q, k.double().permute(1, 2, 0).contiguous()) * 256 ** -0.5
+        total = s.masked_fill((key > pos) | ((key <= pos - window) if window else (key < 0)), -math.inf).logsumexp(dim=-1)
+        rows.append(torch.sigmoid(total - sinks.double()[:, None]).t().repeat_interleave(256, dim=1))
+    assert (first.double() - _want(c, nh, nkv, window) * torch.cat(rows)).abs().max().item() <= 2.5e-2
+    for shape in (1, K().PREFILL_NARROW | 2):
+        assert torch.equal(_run(c, nh, nkv, window, sinks=sinks, heads_per_workgroup=shape), first), shape
 
 
 @pytest.mark.parametrize("nh,nkv,ps", [(4, 1, 16), (6, 2, 8)])
