@@ -363,8 +363,10 @@ static bool gemm_tiles_takes(int M, int N, int K) {
 // 0.615 us a 256 x 256 tile's products and 0.56 us the loads of its BM + BN rows, and 10 us times the square root of its area around them
 // (the first loads, C); the launch takes as many turns as the tiles need with one workgroup a compute unit.  Tiles of at most 192 x 128
 // leave room for two, which together take 0.95 of two one after the other.  The constants are a fit to 80 products of 160 to 8,192 rows of
-// 768 to 28,672 columns, K of 768 to 14,336, with all fifteen tiles each: what it picks takes 1.2 % longer than the fastest on average.  (Fitted while a value's rounding took ten instructions; what
-// stands around a tile has shrunk by some us since, for all tiles alike.)
+// 768 to 28,672 columns, K of 768 to 14,336, with all fifteen tiles each: what it picks takes 1.2 % longer than the fastest on average.  They date from when a
+// value's rounding took ten instructions: since it takes one, the estimate is 17 % above what is measured below 80 us, 10 % up to 200 and right
+// beyond, for all tiles alike.  So the picks are as good: of 144 other products 0.8 % longer than the fastest, 0.7 with the constants
+// fitted to these anew.
 static long tile_cost(int M, int NO, int K, int bm, int bn, int cols) {
   const long tiles = (long)((M + bm - 1) / bm) * ((NO + cols - 1) / cols), steps = K / GT_BK;
   const long one = steps * (62L * bm * bn / 65536 + 56L * (bm + bn) / 512);
@@ -384,8 +386,9 @@ struct TileChoice {
 // and one part in GT_TWO_PAYS of the product, the columns of the whole turns take them, and the others, in a launch of their own, smaller
 // tiles.  One tile / two, us, M x rows of W x K, with the activation: 2,048 x 28,672 x 4,096 (3.5 turns of 256 x 256) 371 / 340, 7,680 rows
 // (13.1 turns) 1,258 / 1,223, 1,000 rows (1.8) 180 / 169, 2,925 x 11,008 x 2,048 114 / 108; plain: 4,054 x 25,664 x 4,096 627 / 593.  Of 432 products
-// of 160 to 8,192 rows it takes 13 in 100, 4.9 % faster on average.  The second launch counts 5 us although it takes some 3: below 80 us the
-// estimate is as often wrong (1,755 x 10,304 x 2,048 61 / 66, 1,776 x 11,008 x 2,048 71 / 67).
+// of 160 to 8,192 rows it takes 13 in 100, 4.9 % faster on average.  The second launch counts 5 us although it takes some 3: below 80 us,
+// where the estimate is high, it is as often wrong (1,755 x 10,304 x 2,048 61 / 66, 1,776 x 11,008 x 2,048 71 / 67).  Of the 144 products above
+// it takes 5: 1,559 x 22,234 x 3,904 241 / 222, 4,027 x 26,220 x 2,496 465 / 456, three within 2 % (counted 4 us, as many).
 static TileChoice choose_tiles(int M, int N, int K, bool glu) {
   const int NO = glu ? N / 2 : N;
   const auto best = [&](int columns, int& rows, int& cols) {
