@@ -314,17 +314,18 @@ static HeadsShape heads_shape(int N, int H, int tiles, int K, bool gate) {
     const int blocks = (N + 16 * wide - 1) / (16 * wide);
     for (int waves = 1; waves <= 4 && (waves == 1 || waves < 2 * blocks); waves *= 2) {
       const int rows = (blocks + waves - 1) / waves;
-      for (int pieces = 1, last = 0; pieces <= tiles && last != 1; ++pieces) {       // of as equal a length as can be
+      if (rows > 65535) continue;                        // (the launch's grid)
+      for (int pieces = 1; pieces <= tiles;) {           // of as equal a length as can be
         const int per = (tiles + pieces - 1) / pieces;
-        if (per == last) continue;
-        last = per;
-        const long workgroups = (long)((tiles + per - 1) / per) * rows * H;
+        const long workgroups = (long)pieces * rows * H;
         const long unit = (workgroups + 255) / 256 * (waves < blocks ? waves : blocks);
         const long cost = 32 * per + unit * (4 * wide * kp + per * (2 * kp + wide * (gate ? 2 : 1)));
         if (least == 0 || cost < least) {
           least = cost;
           best = HeadsShape{wide, waves, rows, per};
         }
+        if (per == 1) break;
+        pieces = (tiles + per - 2) / (per - 1);          // the fewest that are shorter
       }
     }
   }
@@ -348,7 +349,7 @@ extern "C" int ia_gemm_heads(const void* x, int x_row, int x_head, const void* W
     if (K <= GH_ROWS_K) {
       const int tiles = (Nout + 15) / 16;
       const HeadsShape shape = heads_shape(N, H, tiles, K, gate != nullptr);
-      if (shape.rows > 65535) return IA_ERR_UNSUPPORTED;
+      if (shape.waves == 0) return IA_ERR_UNSUPPORTED;
       const bool fours = ((Nout | o_row | o_head) & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0 &&
                          (!gate || ((g_row & 3) == 0 && (reinterpret_cast<uintptr_t>(gate) & 7) == 0));
       const dim3 pieces((tiles + shape.per - 1) / shape.per, shape.rows, H);

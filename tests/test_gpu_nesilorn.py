@@ -228,7 +228,8 @@ def test_products_head_by_head_of_many_rows(N, H, J, Kd, gated):
 # group of 16 columns a wave, some, and all 64
 @pytest.mark.parametrize("gated", [False, True])
 @pytest.mark.parametrize("N,H,J,Kd", [(1, 16, 64, 224), (16, 3, 1030, 64), (17, 4, 17, 224), (33, 2, 200, 40), (48, 128, 100, 128), (65, 32, 130, 256),
-                                      (80, 64, 1024, 16), (333, 4, 520, 256), (515, 3, 96, 64), (2047, 16, 224, 64)])
+                                      (80, 64, 1024, 16), (333, 4, 520, 256), (515, 3, 96, 64), (2047, 16, 224, 64),
+                                      (1100000, 1, 20, 8)])                                # more groups of 16 rows than a grid has
 def test_products_head_by_head_however_the_waves_stand(N, H, J, Kd, gated):
     from infernum_amd.kernels import api as K
     g = torch.Generator().manual_seed(N + J)
